@@ -258,6 +258,12 @@ extern "C" int ia_gemm_tiled(void* out, const void* x, const void* w, int M, int
     IA_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled: bad sizes M=%d N=%d K=%d", M, N, K);
     if (M == 0) return 0;
     const size_t elem = in_dtype == IA_F32 ? 4 : 2;
+    // The 32-bit path on the matrix cores: the same bits.  Up to 16 rows the kernel below reads the weights faster, unless
+    // they have very many rows.  (4,096 k, us, the vector units' kernels against it: 8 rows 6,144 features 42 / 66, 24,576 87 /
+    // 120, 151,936 556 / 464; 16 rows 51 / 66, 147 / 118, 901 / 479; 32 rows 99 / 45, 717 / 124; 128 rows 554 / 94, 993 / 256.)
+    if (in_dtype == IA_F32 && out_dtype == IA_F32 && K % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 &&
+        (M > GR_ROWS || N >= (M > 8 ? 64 : 256) * skinny_cus()) && (g_rows_shape == 0 || M > GR_ROWS))
+        return ia_gemm_f32(out, x, w, M, N, K, stream);
     // up to 64 rows, 16 at a time, where the tiles of 64 x 64 would be few (the weights are read once for every 16 rows:
     // at 32 rows of the 32-bit path a decode step of four layers at the sizes of an 8B model still takes a third of the time)
     if (M <= 4 * GR_ROWS && (M <= GR_ROWS || N <= 4096 * 4) && K % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) % (4 * elem)) == 0) {
@@ -277,9 +283,7 @@ extern "C" int ia_gemm_tiled(void* out, const void* x, const void* w, int M, int
     if (M > 2 * GT && N >= GB && K % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) % (4 * elem)) == 0) {
         const dim3 grid((N + GB - 1) / GB, (M + GB - 1) / GB);
         IA_CHECK(grid.y <= 65535, "gemm_tiled: %d rows exceed the grid", M);
-        if (in_dtype == IA_F32 && out_dtype == IA_F32)
-            gemm_tiled128_kernel<float, float><<<grid, 256, 0, stream>>>((float*)out, (const float*)x, (const float*)w, M, N, K);
-        else if (in_dtype == IA_BF16 && out_dtype == IA_BF16)
+        if (in_dtype == IA_BF16 && out_dtype == IA_BF16)
             gemm_tiled128_kernel<bf16_t, bf16_t><<<grid, 256, 0, stream>>>((bf16_t*)out, (const bf16_t*)x, (const bf16_t*)w, M, N, K);
         else if (in_dtype == IA_BF16 && out_dtype == IA_F32)
             gemm_tiled128_kernel<bf16_t, float><<<grid, 256, 0, stream>>>((float*)out, (const bf16_t*)x, (const bf16_t*)w, M, N, K);

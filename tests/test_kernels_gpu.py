@@ -1121,6 +1121,29 @@ def test_few_row_product_of_the_32_bit_path_with_every_block_shape(dtype):
             close(y, x[:y.shape[0]].double() @ w.double().cpu().t(), tol(dtype, 2e-6), "few rows")
 
 
+@pytest.mark.parametrize("m,n,k", [(17, 5, 4), (33, 64, 28), (161, 130, 36), (100, 259, 516), (320, 257, 132), (17, 16400, 100)])
+def test_32_bit_product_on_the_matrix_cores_has_the_bits_of_the_vector_units(m, n, k):
+    """Every shape of block that exists (10 * rows of x + rows of w, in 16 and 64), at sizes that end inside tiles and chunks: the
+    bits of the kernel for few rows, one chain of fused multiply-adds with k ascending; numbers without a leading bit, infinities
+    and NaN go the same way."""
+    from inferrs_amd import ops
+    lib = ops.library()
+    x, w = randn(m, k, dtype=torch.float32, seed=1), randn(n, k, dtype=torch.float32, seed=2)
+    x[0], x[1, 0], x[2, 1], x[3] = x[0] * 1e-38, float("inf"), float("nan"), 0.0
+    x, w = dev(x), dev(w)
+    want = torch.cat([ops.gemm_tiled(x[i:i + 8].contiguous(), w) for i in range(0, m, 8)])
+    assert float((want[4:].double() - x[4:].double() @ w.double().t()).abs().max()) <= 4e-6 * max(1.0, k ** 0.5)
+    try:
+        for shape in [0] + [10 * a + b for a in range(1, 11) for b in (1, 2)]:
+            assert lib.ia_gemm_f32_tune(shape) == 0
+            got = ops.gemm_tiled(x, w)
+            assert torch.equal(torch.isnan(got), torch.isnan(want)), shape
+            assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(want)), shape
+        assert lib.ia_gemm_f32_tune(113) != 0 and "gemm_f32_tune" in lib.ia_last_error().decode()
+    finally:
+        lib.ia_gemm_f32_tune(0)
+
+
 @pytest.mark.parametrize("m,n,k", [(130, 72, 40), (512, 4096, 1024), (2048, 6144, 4096), (300, 1000, 136), (129, 64, 33), (1024, 1024, 3072)])
 def test_vendor_gemm_called_directly_is_the_product_that_torch_gets(m, n, k):
     """The vendor's GEMM through this package's own entry point (descriptors and the library's choice of kernel kept
