@@ -77,6 +77,11 @@ int ia_gemm_f32_tune(int shape);
 int ia_gemm_rows_tune(int shape);
 int ia_gemm_skinny_bf16(void* out, const void* x, const void* w, const void* bias, int M, int N, int K,
                         int out_dtype, int dual, hipStream_t stream);
+// bfloat16 products for steps of more than 128 rows on the matrix cores, k split between blocks (gemm_wide.hip)
+int ia_gemm_wide_bf16(void* out, const void* x, const void* w, int M, int N, int K, int out_mode, int dual, hipStream_t stream);
+int ia_gemm_wide_splits(int M, int N, int K);
+int ia_gemm_wide_dual_fits(int M, int N, int K);
+int ia_gemm_wide_plan(int mt, int splits);
 // Large bfloat16 products through the vendor's library, hipBLASLt, called directly (vendor_gemm.hip).  ia_vendor_gemm_init
 // opens the library at `path` (the copy the process already holds) once; ia_vendor_gemm_bf16: out [M, N] = x [M, K] . w [N, K]^T,
 // contiguous, with `workspace_bytes` of device memory for kernels that want some.

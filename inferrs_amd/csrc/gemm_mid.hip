@@ -732,7 +732,10 @@ extern "C" int ia_add_rmsnorm_partials(void* out, void* x, const float* part, in
     const size_t mn = (size_t)rows * cols;
 #define APN_LAUNCH(S) add_rmsnorm_partials_kernel<S><<<rows, threads, 0, stream>>>(o, xs, part, splits, mn, w, eps, cols, add_one)
     if (splits == 2) APN_LAUNCH(2);
+    else if (splits == 3) APN_LAUNCH(3);
     else if (splits == 4) APN_LAUNCH(4);
+    else if (splits == 5) APN_LAUNCH(5);
+    else if (splits == 6) APN_LAUNCH(6);
     else if (splits == 8) APN_LAUNCH(8);
     else APN_LAUNCH(0);
 #undef APN_LAUNCH

@@ -1,0 +1,345 @@
+// bfloat16 products for steps of more rows than gemm_mid.hip takes (portions of prompts, several short prompts together):
+// out[M, N] = x[M, K] . w[N, K]^T, or with an activation act(x . gate^T) * (x . up^T) for w = [gate; up].
+//
+// The reference hands these products to cuBLAS like all others (`candle-core/src/cuda_backend/mod.rs:2260-2305`).
+//
+// What bounds it: the matrix pipes, once every compute unit has a share.  A few hundred rows are a few tiles of rows only,
+// and the weights of an output projection or of a feed-forward's second product a few tiles of features: k is split between
+// blocks until there is one for every unit, and the splits' 32-bit sums, [splits][M][N], are added up in their order by
+// whoever reads them (gemm_mid.hip's readers: the kernel that adds a product to the residual stream and norms it, or
+// ia_sum_partials).  A block's rows of x come in steps of 16, so that 521 rows do not pay for 768 (gw_plan below).
+//
+// A block of four waves, one a SIMD, owns 16 MT rows of x by 256 rows of w and a range of k.  A wave multiplies 64 of the
+// rows of w (four MFMA A-operands, v_mfma_f32_16x16x32_bf16) with all of the block's rows of x: MT + 4 operand reads from
+// shared memory for 4 MT products.  Stages of 64 k (whole lines of 128 bytes a row: a load of 1 KiB takes the compute unit's
+// address unit 18 cycles, in rows of 64 bytes 37) go from memory straight into shared memory (global_load_lds), two places
+// for x, which the step has just written and comes from a cache, and three for w, which comes from memory: at 128 rows a
+// stage is multiplied in 0.6 us when its operands lie in the die's L2, and in 0.85 when w comes from memory.  The walk is
+// laid out so that the matrix pipe does not wait for an operand that was asked for just before:
+//   * the operands of a step (32 k) are read while the step before it is multiplied, two reads beside each of its first
+//     groups of four products, across stages too;
+//   * the one barrier of a stage stands between its two steps: there every wave has read all of the stage (its places are
+//     free from here on) and has seen its own loads of the next stage arrive;
+//   * a stage's loads go out one beside a group: four waves that issue theirs in a row stand still until the address unit
+//     has taken them.
+// Shared memory: piece c (16 bytes) of row r lies at place c ^ ((r >> 1) & 7) of its row's 128 bytes, so that the rows which
+// one operand read takes at the same k fall on different banks.
+//
+// Measured (us, the vendor's GEMM and the kernel behind it against this one and its reader; 8B and 14B shapes): down at 200 rows
+// 56 / 38 and 226 / 61, at 456 86 / 58 and 174 / 86, at 521 107 / 64 and 186 / 93, at 1,024 127 / 101 and 260 / 160, at 2,048
+// 192 / 179 and 300 / 296; output projection at 256 25 / 23 and 49 / 26, at 1,024 46 / 44 and 63 / 62; gate|up with the activation at
+// 320 88 / 77 and 163 / 174, at 768 158 / 140 and 282 / 283.  1,200 to 1,340 TFLOP/s over a long k from 160 rows a block on, at the
+// chip's power limit (with operands of zeros a stage takes a fifth less).
+#include <type_traits>
+#include <utility>
+
+#include "common.h"
+#include "api.h"
+
+typedef __bf16 gw_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float gw_f32x4 __attribute__((ext_vector_type(4)));
+
+#define GW_BN 256                            // rows of w of a block
+#define GW_STAGE_K 64                        // k of a stage: two steps of the matrix instruction
+#define GW_ROW 128                           // bytes of a staged row
+
+struct GemmWideParams {
+    void* out;
+    const bf16_t* x;
+    const bf16_t* w;
+    int M, N, K;                             // N: output features (with the activation inside, w has 2 N rows)
+    int act;
+    int tiles_m, tiles_n, stages;            // stages: of a split (the last split may have fewer)
+};
+
+// 16 bytes a lane from memory straight into shared memory, 1 KiB a wave in lane order from `lds_at` on (the same for all
+// lanes), from `base` (the same for all lanes) + `off`.  Written out so that the compiler does not wait for it at every read
+// of shared memory: the waits stand in the code (loads come back in the order they were asked for).
+__device__ __forceinline__ void gw_load16(const char* base, uint32_t off, uint32_t lds_at) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds_at) : "memory");
+}
+
+// s_waitcnt with vmcnt(n) and lgkmcnt(0) (gfx9 encoding: vmcnt in bits 3:0 and 15:14, lgkmcnt in 11:8, expcnt left alone)
+#define GW_WAIT(n) (((n) & 15) | ((((n) >> 4) & 3) << 14) | (7 << 4))
+
+template <int... I, typename Fn>
+__device__ __forceinline__ void gw_unrolled(std::integer_sequence<int, I...>, Fn fn) {
+    (fn(std::integral_constant<int, I>()), ...);
+}
+
+enum { GW_BF16 = 0, GW_F32 = 1, GW_DUAL = 2 };          // what leaves the kernel; GW_F32: a split's sums (or whole ones)
+
+template <int MT, int OUT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void gemm_wide_kernel(const GemmWideParams p) {
+    constexpr bool DUAL = OUT == GW_DUAL;
+    constexpr int BM = 16 * MT;
+    constexpr int XL = (MT + 1) / 2, WL = 8;                 // a wave's loads of 1 KiB (8 rows) for a stage's rows of x and of w
+    constexpr int W1 = MT - XL < WL ? MT - XL : WL;          // (an odd MT: the last ones of x fetch a row again into a place nobody reads)
+    constexpr uint32_t X_STAGE = XL * 4 * 1024, W_STAGE = WL * 4 * 1024, W_AT = 2 * X_STAGE;
+    static_assert(2 * X_STAGE + 3 * W_STAGE <= 160 * 1024, "the stages fit a compute unit's shared memory");
+    static_assert(WL - W1 <= MT, "a group has room for a load");
+    constexpr int FEATS = DUAL ? GW_BN / 2 : GW_BN;          // output features of a block
+    __shared__ __attribute__((aligned(1024))) char lds[2 * X_STAGE + 3 * W_STAGE];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+
+    // Blocks go round the eight dies in turn, and each die has an L2 of its own: a die takes a contiguous range of the
+    // blocks of one range of k, rows of x fastest, so that the blocks which run together on a die share both operands.
+    const int blocks = gridDim.x, die = blockIdx.x & 7;
+    const int id = die * (blocks >> 3) + min(die, blocks & 7) + (blockIdx.x >> 3);
+    const int tiles = p.tiles_m * p.tiles_n;
+    const int split = id / tiles, tile = id - split * tiles;
+    const int m0 = (tile % p.tiles_m) * BM, n0 = (tile / p.tiles_m) * FEATS;
+    const int k_first = split * p.stages * GW_STAGE_K;
+    const int stages = min(p.stages, (p.K - k_first) / GW_STAGE_K);
+    // (blocks of different features start at different places of their range of k: rows are a power of two apart, and blocks
+    // that walk k in step ask the same memory channels at any moment)
+    const int rot = (int)((unsigned)(tile / p.tiles_m) * 5u % (unsigned)stages);
+
+    // ---- what this lane fetches: load i of the wave brings rows 8 (4 i + wave) .. + 8 of x, or of w
+    const size_t pitch = (size_t)p.K * 2;
+    const char* xbase = (const char*)p.x + (size_t)m0 * pitch + (size_t)k_first * 2;
+    const char* wbase = (const char*)p.w + (size_t)n0 * pitch + (size_t)k_first * 2;
+    uint32_t xoff[XL], woff[WL];
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+        const int row = 8 * (4 * i + wave) + (lane >> 3);
+        xoff[i] = (uint32_t)min(row, p.M - 1 - m0) * (uint32_t)pitch + ((lane & 7) ^ ((row >> 1) & 7)) * 16;     // (rows beyond the
+    }                                                                                                   // matrices are never stored)
+#pragma unroll
+    for (int i = 0; i < WL; ++i) {
+        const int row = 8 * (4 * i + wave) + (lane >> 3);
+        int at;
+        if (DUAL) {
+            const int q = row & 63, part = q >> 5;           // a wave's 64 rows: 32 of gate, then the same 32 of up
+            at = min((row >> 6) * 32 + (q & 31), p.N - 1 - n0) + part * p.N;
+        } else {
+            at = min(row, p.N - 1 - n0);
+        }
+        woff[i] = (uint32_t)at * (uint32_t)pitch + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+    // load i of stage kt of an operand into the place at `slot` (past the walk's end a stage is fetched again into a place that
+    // nobody reads any more, so that the count of loads under way is the same at every stage)
+    auto k_of = [&](int kt) __attribute__((always_inline)) {
+        const int at = (kt < stages ? kt : stages - 1) + rot;
+        return (size_t)(at < stages ? at : at - stages) * (GW_STAGE_K * 2);
+    };
+    auto fetch_x = [&](size_t k, uint32_t slot, auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (i >= 0 && i < XL) gw_load16(xbase + k, xoff[i], lds0 + slot + (uint32_t)(4 * i + wave) * 1024);
+    };
+    auto fetch_w = [&](size_t k, uint32_t slot, auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (i >= 0 && i < WL) gw_load16(wbase + k, woff[i], lds0 + W_AT + slot + (uint32_t)(4 * i + wave) * 1024);
+    };
+
+    gw_f32x4 acc[4][MT];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < MT; ++b) acc[a][b] = (gw_f32x4){0.f, 0.f, 0.f, 0.f};
+    uint4 fw[2][4], fx[2][MT];
+    // the lane's place in a tile of 16 rows, for the two steps of a stage
+    const uint32_t in_tile[2] = {(uint32_t)(r * GW_ROW + ((g ^ ((r >> 1) & 7)) * 16)),
+                                 (uint32_t)(r * GW_ROW + (((4 + g) ^ ((r >> 1) & 7)) * 16))};
+    const uint32_t w_rows = W_AT + (uint32_t)(64 * wave) * GW_ROW;
+    // read i of a step's MT + 4 operands: the rows of w first
+    auto read = [&](uint32_t xslot, uint32_t wslot, int step, auto ic) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value;
+        if constexpr (i < 4) fw[step][i] = *(const uint4*)(lds + wslot + w_rows + in_tile[step] + i * 16 * GW_ROW);
+        else if constexpr (i < MT + 4) fx[step][i - 4] = *(const uint4*)(lds + xslot + in_tile[step] + (i - 4) * 16 * GW_ROW);
+    };
+    // one step: `step`'s operands are multiplied, the other step's are read, two beside each of the first groups of four
+    // products, and `load(b)` asks for something beside group b
+    auto multiply = [&](auto step_c, uint32_t xslot, uint32_t wslot, auto load) __attribute__((always_inline)) {
+        constexpr int step = decltype(step_c)::value;
+        gw_unrolled(std::make_integer_sequence<int, MT>(), [&](auto bc) __attribute__((always_inline)) {
+            constexpr int b = decltype(bc)::value;
+            read(xslot, wslot, 1 - step, std::integral_constant<int, 2 * b>());
+            read(xslot, wslot, 1 - step, std::integral_constant<int, 2 * b + 1>());
+            load(bc);
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gw_bf16x8, fw[step][a]),
+                                                                    __builtin_bit_cast(gw_bf16x8, fx[step][b]), acc[a][b], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    constexpr auto all_x = std::make_integer_sequence<int, XL>();
+    constexpr auto all_w = std::make_integer_sequence<int, WL>();
+    // (in the order of the walk: x of a stage ahead of w of the stage behind it)
+    gw_unrolled(all_w, [&](auto i) { fetch_w(k_of(0), 0, i); });
+    gw_unrolled(all_x, [&](auto i) { fetch_x(k_of(0), 0, i); });
+    gw_unrolled(all_w, [&](auto i) { fetch_w(k_of(1), W_STAGE, i); });
+    gw_unrolled(all_x, [&](auto i) { fetch_x(k_of(1), X_STAGE, i); });
+    {
+        const size_t k = k_of(2);
+        gw_unrolled(std::make_integer_sequence<int, W1>(), [&](auto i) { fetch_w(k, 2 * W_STAGE, i); });
+    }
+    __builtin_amdgcn_s_waitcnt(GW_WAIT(WL + XL + W1));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    uint32_t xs = 0, wh = 0, wn = W_STAGE, wl = 2 * W_STAGE;     // places: this stage's x; w of this stage, the next, the one behind it
+    gw_unrolled(std::make_integer_sequence<int, MT + 4>(), [&](auto i) __attribute__((always_inline)) { read(0, 0, 0, i); });
+    size_t k_w = k_of(2);
+    for (int s = 0; s < stages; ++s) {
+        // the stage's first step; the rest of w of stage s + 2 is asked for
+        multiply(std::integral_constant<int, 0>(), xs, wh, [&](auto bc) __attribute__((always_inline)) {
+            fetch_w(k_w, wl, std::integral_constant<int, decltype(bc)::value + W1>());
+        });
+        __builtin_amdgcn_s_waitcnt(GW_WAIT(WL));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        // its second step; x of stage s + 2 and then w of stage s + 3 go into this stage's places
+        const size_t k_x = k_w;
+        k_w = k_of(s + 3);
+        multiply(std::integral_constant<int, 1>(), X_STAGE - xs, wn, [&](auto bc) __attribute__((always_inline)) {
+            constexpr int b = decltype(bc)::value;
+            if constexpr (b < XL) fetch_x(k_x, xs, bc);
+            else if constexpr (b - XL < W1) fetch_w(k_w, wh, std::integral_constant<int, b - XL>());
+        });
+        xs = X_STAGE - xs;
+        const uint32_t t = wh;
+        wh = wn; wn = wl; wl = t;
+    }
+    // (without this the compiler carries half of the accumulators through copies, 3 moves for every two products)
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < MT; ++b) asm volatile("" : "+a"(acc[a][b]));
+    __builtin_amdgcn_s_waitcnt(GW_WAIT(0));                  // (nothing may still be on its way into shared memory at the end)
+
+    // ---- results: the lane holds features 4 g .. + 4 of w tile a for row r of x tile b (N is a multiple of 4)
+#pragma unroll
+    for (int b = 0; b < MT; ++b) {
+        const int m = m0 + b * 16 + r;
+        if (m >= p.M) continue;
+#pragma unroll
+        for (int a = 0; a < (DUAL ? 2 : 4); ++a) {
+            const int n = n0 + (DUAL ? wave * 32 : wave * 64) + a * 16 + 4 * g;
+            if (n >= p.N) continue;
+            gw_f32x4 v = acc[a][b];
+            if constexpr (DUAL) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    // the products are rounded to the storage precision before the activation, as the two-kernel way rounds them
+                    const uint32_t both = pack_bf16x2(v[i], acc[a + 2][b][i]);
+                    v[i] = gate_act(__uint_as_float(both << 16), p.act) * __uint_as_float(both & 0xffff0000u);
+                }
+            }
+            if constexpr (OUT == GW_F32)
+                *(gw_f32x4*)((float*)p.out + ((size_t)split * p.M + m) * p.N + n) = v;
+            else
+                *(uint2*)((bf16_t*)p.out + (size_t)m * p.N + n) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        }
+    }
+}
+
+// How a product is shared out: rows of x a block (16 mt), ways k is split, stages of a split.
+struct WidePlan { int mt, splits, stages; double cost; };
+static WidePlan g_wide_forced = {0, 0, 0, 0.0};
+static int wide_cus() {
+    static int cus = 0;
+    if (cus == 0) {
+        int dev = 0, n = 0;
+        cus = hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+    }
+    return cus;
+}
+// A stage of 64 k, measured with every compute unit at work, rows of 16 mt (us): the memory's latency up to 8, then the matrix
+// pipes at the clock that the chip's power leaves them.
+static const double gw_stage_us[11] = {0.83, 0.89, 0.93, 1.00, 1.05, 1.16, 1.20, 1.32, 1.41, 1.55, 1.89};
+static WidePlan gw_plan(int M, int N, int K, bool dual, bool may_split) {
+    const int cus = wide_cus(), feats = dual ? GW_BN / 2 : GW_BN;
+    WidePlan best = {0, 0, 0, 1e30};
+    const long long tiles_n = (N + feats - 1) / feats;
+    const int stages = K / GW_STAGE_K;
+    for (int mt = 6; mt <= 16; ++mt) {
+        const long long tiles_m = (M + 16 * mt - 1) / (16 * mt);
+        for (int splits = 1; splits <= (may_split && !dual ? 8 : 1); ++splits) {
+            const int each = (stages + splits - 1) / splits;
+            if (splits > 1 && each < 8) break;
+            if ((splits - 1) * each >= stages) continue;
+            const long long rounds = (tiles_m * tiles_n * splits + cus - 1) / cus;
+            // in us: a block's stages, its start and its end, and the splits' sums on their way out and back in
+            const double cost = (double)rounds * (each * gw_stage_us[mt - 6] + 3.0) + (splits > 1 ? 1.0 + 0.42e-6 * splits * M * N * 4.0 : 0.0);
+            if (cost < best.cost) best = {mt, splits, each, cost};
+        }
+    }
+    return best;
+}
+
+// (a plan for measurements and tests: blocks of 16 mt rows, k split `splits` ways; 0, 0: the plan's own)
+extern "C" int ia_gemm_wide_plan(int mt, int splits) {
+    IA_CHECK((mt == 0 && splits == 0) || (mt >= 6 && mt <= 16 && splits >= 1 && splits <= 8),
+             "gemm_wide_plan: no blocks of %d rows with %d splits of k", 16 * mt, splits);
+    g_wide_forced = {mt, splits, 0, 0.0};
+    return 0;
+}
+
+static WidePlan wide_plan(int M, int N, int K, bool dual, bool may_split) {
+    WidePlan p = gw_plan(M, N, K, dual, may_split);
+    if (g_wide_forced.mt) {
+        p.mt = g_wide_forced.mt;
+        int splits = may_split && !dual ? g_wide_forced.splits : 1;
+        const int stages = K / GW_STAGE_K;
+        if (splits > stages) splits = stages;
+        p.stages = (stages + splits - 1) / splits;
+        p.splits = (stages + p.stages - 1) / p.stages;
+    }
+    return p;
+}
+
+// The ways k is split where the result may stay split (ia_gemm_wide_bf16 with out_mode 2).
+extern "C" int ia_gemm_wide_splits(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
+    return wide_plan(M, N, K, false, true).splits;
+}
+
+// Whether a [gate; up] of N features each goes here instead of to the vendor's GEMM and the activation's kernel: where this
+// kernel's own time comes within a tenth of 1.22 PFLOP/s (or of 4 TB/s over the operands) and what the second kernel takes.
+// Measured over the six dense shapes and 130 to 1,024 rows: 0.90 to 1.5 of the two kernels' time, 1.1 on average; beyond that the
+// vendor's blocks of 256 x 256 are as fast or faster (8B shape, 2,048 rows: 316 against 353 us).
+extern "C" int ia_gemm_wide_dual_fits(int M, int N, int K) {
+    if (M <= 0 || M > 1024 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4 || ((long long)N + GW_BN) * K * 2 >= (1LL << 32)) return 0;
+    const double flops = 4.0 * M * N * K / 1.22e9, bytes = (2.0 * N + M) * K * 2.0 / 4.0e6;
+    return gw_plan(M, N, K, true, false).cost <= 1.1 * ((flops > bytes ? flops : bytes) + 8.0 + M * (double)N * 6.0 / 5.0e6);
+}
+
+// out_mode 0: out [M, N] bfloat16; 1: float; 2: [splits][M][N] float with splits = ia_gemm_wide_splits(M, N, K).  dual (an
+// activation, IA_ACT_*): w = [gate; up] of N rows each (mode 0 only).  K a multiple of 64, operands 16-byte aligned.
+extern "C" int ia_gemm_wide_bf16(void* out, const void* x, const void* w, int M, int N, int K, int out_mode, int dual,
+                                 hipStream_t stream) {
+    IA_CHECK(M > 0 && N > 0 && K > 0 && K % GW_STAGE_K == 0 && N % 4 == 0, "gemm_wide: bad sizes M=%d N=%d K=%d (K a multiple of %d, N of 4)",
+             M, N, K, GW_STAGE_K);
+    IA_CHECK(out_mode >= 0 && out_mode <= 2 && (!dual || out_mode == 0), "gemm_wide: output mode %d%s", out_mode,
+             dual ? " does not go with the activation inside" : " is unknown");
+    IA_CHECK(dual >= 0 && dual <= IA_ACT_LAST, "gemm_wide: unknown activation %d", dual);
+    IA_CHECK((((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0, "gemm_wide: operands must be 16-byte aligned");
+    // (a lane's offset from its block's first row is 32 bits wide)
+    IA_CHECK(((dual ? (long long)N : 0) + GW_BN) * K * 2 < (1LL << 32), "gemm_wide: N=%d rows of K=%d are too far apart", N, K);
+    const WidePlan plan = wide_plan(M, N, K, dual != 0, out_mode == 2);
+    const int feats = dual ? GW_BN / 2 : GW_BN;
+    GemmWideParams p;
+    p.out = out; p.x = (const bf16_t*)x; p.w = (const bf16_t*)w;
+    p.M = M; p.N = N; p.K = K; p.act = dual;
+    p.tiles_m = (M + 16 * plan.mt - 1) / (16 * plan.mt);
+    p.tiles_n = (N + feats - 1) / feats;
+    p.stages = plan.stages;
+    const long long blocks = (long long)p.tiles_m * p.tiles_n * plan.splits;
+    IA_CHECK(plan.mt >= 6 && plan.stages > 0 && blocks < (1LL << 31), "gemm_wide: %lld blocks", blocks);
+    switch (plan.mt) {
+#define GW_CASE(MT) \
+    case MT: if (dual) gemm_wide_kernel<MT, GW_DUAL><<<(unsigned)blocks, 256, 0, stream>>>(p); \
+             else if (out_mode == 0) gemm_wide_kernel<MT, GW_BF16><<<(unsigned)blocks, 256, 0, stream>>>(p); \
+             else gemm_wide_kernel<MT, GW_F32><<<(unsigned)blocks, 256, 0, stream>>>(p); break;
+    GW_CASE(6) GW_CASE(7) GW_CASE(8) GW_CASE(9) GW_CASE(10) GW_CASE(11) GW_CASE(12) GW_CASE(13) GW_CASE(14) GW_CASE(15) GW_CASE(16)
+#undef GW_CASE
+    }
+    IA_LAUNCH_CHECK("gemm_wide");
+    return 0;
+}

@@ -76,7 +76,7 @@ class _Timed:
         fn = getattr(self._lib, name)
         if KernelTimer.active is None or not name.startswith("ia_") or name.endswith(("_workspace", "_blocks", "_block_rows",
                                                                                       "_error", "_version", "_capacity", "_top",
-                                                                                      "_splits", "_tune", "_target", "_counters", "_fills", "_plan", "_plans")):
+                                                                                      "_splits", "_tune", "_target", "_counters", "_fills", "_fits", "_plan", "_plans")):
             return fn
         timer = KernelTimer.active
         return lambda *args: timer.call(name[3:], fn, *args)
@@ -1046,6 +1046,40 @@ def gemm_mid_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = tor
     return out
 
 
+# ---- products of 129 to 2,048 rows ---------------------------------------------------------------
+# Steps with prompt portions: gemm_wide.hip splits k between blocks where the vendor's GEMM leaves the chip half empty (its
+# header has the figures, and the rule for [gate; up]).
+WIDE_MAX_ROWS = 2048
+
+
+def wide_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether gemm_wide.hip takes x . w^T (beyond the rows of gemm_mid.hip, up to `WIDE_MAX_ROWS`)."""
+    return (MID_PRODUCTS == "own" and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and MID_MAX_ROWS < x.shape[0] <= WIDE_MAX_ROWS and x.shape[1] % 64 == 0 and w.shape[1] == x.shape[1]
+            and w.shape[0] % 4 == 0 and x.is_contiguous() and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
+def gemm_wide_bf16(x: torch.Tensor, w: torch.Tensor, dual: bool = False, partial: bool = False, activation: str = "silu"):
+    """x [m, k] . w[n, k]^T in bfloat16 (k a multiple of 64, n of 4); `dual` and `partial` as `gemm_mid_bf16` has them."""
+    _dev(x, w)
+    m, k = x.shape
+    rows, k2 = w.shape
+    if (k2 != k or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or m < 1 or k % 64 or rows % (8 if dual else 4)
+            or (dual and partial) or not (x.is_contiguous() and w.is_contiguous())):
+        raise KernelError(f"gemm_wide: x {tuple(x.shape)} {x.dtype} does not fit w {tuple(w.shape)} {w.dtype}")
+    n = rows // 2 if dual else rows
+    lib = library()
+    if partial:
+        splits = lib.ia_gemm_wide_splits(m, n, k)
+        if splits > 1:
+            parts = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+            _check(lib.ia_gemm_wide_bf16(_p(parts), _p(x), _p(w), m, n, k, 2, 0, _stream()))
+            return Partials(parts)
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    _check(lib.ia_gemm_wide_bf16(_p(out), _p(x), _p(w), m, n, k, 0, activation_code(activation) if dual else 0, _stream()))
+    return out
+
+
 def linear_partials(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None):
     """x . w^T for a reader that takes `Partials` (the norm that adds the product to the stream): split along k where the
     weight has few rows.  None when the product of 17 to 64 rows does not take these operands (a bias among them: the
@@ -1054,6 +1088,8 @@ def linear_partials(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tenso
     # product of another width follows it)
     if bias is None and isinstance(x, torch.Tensor) and x.shape[0] >= MID_MIN_ROWS and mid_fits(x, w, few_rows=True):
         return gemm_mid_bf16(x, w, partial=True)
+    if bias is None and isinstance(x, torch.Tensor) and wide_fits(x, w):
+        return gemm_wide_bf16(x, w, partial=True)
     return None
 
 
@@ -1243,6 +1279,9 @@ def gated_linear(x, w_gate_up: torch.Tensor, activation: str = "silu",
         if (even and mid_fits(x, w_gate_up)
                 and w_gate_up.numel() * w_gate_up.element_size() <= MID_DUAL_MAX_BYTES):
             return gemm_mid_bf16(x, w_gate_up, dual=True, activation=activation)
+        if (w_gate_up.shape[0] % 8 == 0 and wide_fits(x, w_gate_up)
+                and library().ia_gemm_wide_dual_fits(x.shape[0], w_gate_up.shape[0] // 2, x.shape[1])):
+            return gemm_wide_bf16(x, w_gate_up, dual=True, activation=activation)
         if even and x.dtype == torch.bfloat16 and skinny_fits(x, w_gate_up) and _own_large(x, w_gate_up):
             return gemm_mfma_bf16(x, w_gate_up, dual=True, activation=activation)
     # (a [gate; up] beyond MID_DUAL_MAX_BYTES at 17 to 64 rows: the vendor's GEMM, not the plain product of gemm_mid.hip)

@@ -1121,6 +1121,47 @@ def test_few_row_product_of_the_32_bit_path_with_every_block_shape(dtype):
             close(y, x[:y.shape[0]].double() @ w.double().cpu().t(), tol(dtype, 2e-6), "few rows")
 
 
+@pytest.mark.parametrize("m,n,k", [(129, 260, 64), (130, 4, 192), (160, 516, 640), (257, 1024, 128), (521, 256, 1088), (1000, 300, 2048)])
+def test_wide_product_in_every_block_shape(m, n, k):
+    """Blocks of every number of rows and k split every way that exists, at sizes that end inside tiles of rows, of features and
+    inside a share of k: the exact product within its storage's rounding, 32-bit sums that do not depend on the blocks' rows,
+    and the activation inside, rounded between the two as two kernels would round."""
+    from inferrs_amd import ops
+    lib = ops.library()
+    x, w = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.05)
+    gu = randn(2 * n, k, dtype=torch.bfloat16, seed=3, scale=0.05)
+    want = x.double() @ w.double().t()
+    gate, up = (x.double() @ gu.double().t()).split(n, dim=1)
+    dx, dw, dgu = dev(x), dev(w), dev(gu)
+    sums = {}
+    try:
+        for mt, splits in [(0, 0)] + [(a, b) for a in range(6, 17) for b in range(1, 9)]:
+            assert lib.ia_gemm_wide_plan(mt, splits) == 0
+            if splits <= 1:
+                close(ops.gemm_wide_bf16(dx, dw), want, 2 ** -8, ("stored", mt))
+                for name, act in (("silu", torch.nn.functional.silu), ("gelu_tanh", lambda z: torch.nn.functional.gelu(z, approximate="tanh"))):
+                    # (gate, up, and what they give: three roundings of 2^-9)
+                    close(ops.gemm_wide_bf16(dx, dgu, dual=True, activation=name), act(gate) * up, 3 * 2 ** -8, (name, mt))
+            parts = ops.gemm_wide_bf16(dx, dw, partial=True)
+            if not isinstance(parts, ops.Partials):
+                continue
+            close(parts.parts.sum(0), want, 4e-6, ("partial sums", mt, splits))
+            close(parts.materialize(), want, 2 ** -8, ("added up", mt, splits))
+            ways = parts.parts.shape[0]
+            assert torch.equal(parts.parts, sums.setdefault(ways, parts.parts)), (mt, splits)
+        assert lib.ia_gemm_wide_plan(5, 1) != 0 and "gemm_wide_plan" in lib.ia_last_error().decode()
+    finally:
+        lib.ia_gemm_wide_plan(0, 0)
+    # its readers with every number of splits: the sum added to a stream and normed
+    stream, norm_w = randn(m, n, dtype=torch.bfloat16, seed=5), randn(n, dtype=torch.float32, seed=6)
+    for ways, parts in sums.items():
+        ours, theirs = dev(stream), dev(stream)
+        got = ops.add_rmsnorm_partials(ours, ops.Partials(parts), dev(norm_w), 1e-6)
+        # (the same sums; the two kernels add a row's squares up in different orders, 1e-7, which can move a rounding of 2^-8)
+        close(got, ops.add_rmsnorm(theirs, ops.Partials(parts).materialize(), dev(norm_w), 1e-6), 2 ** -8, ways)
+        assert torch.equal(ours, theirs), ways
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 5, 4), (33, 64, 28), (161, 130, 36), (100, 259, 516), (320, 257, 132), (17, 16400, 100)])
 def test_32_bit_product_on_the_matrix_cores_has_the_bits_of_the_vector_units(m, n, k):
     """Every shape of block that exists (10 * rows of x + rows of w, in 16 and 64), at sizes that end inside tiles and chunks: the
