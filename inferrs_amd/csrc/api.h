@@ -65,6 +65,11 @@ int ia_attention_generic(void* out, const void* q, const void* k_cache, const vo
                          const float* sinks, int keep_first, float softcap, hipStream_t stream);
 long long ia_attention_generic_workspace(int n, int nq, int nkv, int d, int dv, int max_kv_len);
 
+// ia_qk_rope_kv on projections still split along their k, [splits][n][(nq + 2 nkv) d] 32-bit sums (bfloat16 caches)
+int ia_qk_rope_kv_partials(void* q_out, void* k_cache, void* v_cache, const float* parts, int splits, const float* q_norm_w,
+                           const float* k_norm_w, const float* cos_t, const float* sin_t, const int* slots, int n, int nq, int nkv,
+                           int d, int page_size, float eps, int add_one, hipStream_t stream);
+int ia_qk_rope_kv_partials_fits(int n, int d, int rot, int interleaved, int page_size);
 int ia_gemm_tiled(void* out, const void* x, const void* w, int M, int N, int K, int in_dtype,
                   int out_dtype, hipStream_t stream);
 // (what ia_gemm_tiled runs for many rows of the 32-bit path: K a multiple of 4, x and w 16-byte aligned; `shape`

@@ -328,9 +328,43 @@ extern "C" int ia_qk_rope_kv_strided(void* q_out, void* k_cache, void* v_cache, 
 #define QKV_THREADS 256
 #define QKV_GROUP 8
 
+// A step's projections as the kernels below read them, eight features at a time: stored rows, or a product still split along
+// its k, 32-bit sums [splits][..] that are added up in their order and rounded here, as a kernel that stores them would.
+struct StoredRows {
+    const bf16_t* rows;
+    __device__ __forceinline__ uint4 eight(size_t at) const { return *(const uint4*)(rows + at); }
+};
+template <int SPLITS>                    // 0: any number
+struct SplitRows {
+    const float* parts;
+    int splits;
+    size_t apart;                        // floats from a split to the next
+    __device__ __forceinline__ uint4 eight(size_t at) const {
+        float4 a = *(const float4*)(parts + at), b = *(const float4*)(parts + at + 4);
+        auto add = [&](const float4& c, const float4& d) {
+            a.x += c.x; a.y += c.y; a.z += c.z; a.w += c.w;
+            b.x += d.x; b.y += d.y; b.z += d.z; b.w += d.w;
+        };
+        if constexpr (SPLITS > 0) {
+            float4 c[SPLITS - 1], d[SPLITS - 1];
+#pragma unroll
+            for (int k = 0; k < SPLITS - 1; ++k) {
+                c[k] = *(const float4*)(parts + (k + 1) * apart + at);
+                d[k] = *(const float4*)(parts + (k + 1) * apart + at + 4);
+            }
+#pragma unroll
+            for (int k = 0; k < SPLITS - 1; ++k) add(c[k], d[k]);
+        } else {
+            for (int k = 1; k < splits; ++k) add(*(const float4*)(parts + k * apart + at), *(const float4*)(parts + k * apart + at + 4));
+        }
+        return make_uint4(pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w));
+    }
+};
+
 // The values of eight neighbouring tokens, for as many heads as the block's threads cover (see below).
+template <typename Rows>
 __device__ __forceinline__ void values_in_groups(uint16_t* tile /* [head of the block][token of the group][d] */,
-                                                 bf16_t* __restrict__ v_cache, const bf16_t* __restrict__ qkv,
+                                                 bf16_t* __restrict__ v_cache, const Rows qkv,
                                                  const int* __restrict__ slots, int vb, int n, int nq, int nkv,
                                                  int d, int page_size) {
     const int tpu = d / 8;
@@ -343,7 +377,7 @@ __device__ __forceinline__ void values_in_groups(uint16_t* tile /* [head of the 
         const int hl = u / QKV_GROUP, ti = u - hl * QKV_GROUP;
         if (tok0 + ti < n && head0 + hl < nkv)
             *(uint4*)(tile + (size_t)u * d + t * 8) =
-                *(const uint4*)(qkv + ((size_t)(tok0 + ti) * (nq + 2 * nkv) + nq + nkv + head0 + hl) * d + t * 8);
+                qkv.eight(((size_t)(tok0 + ti) * (nq + 2 * nkv) + nq + nkv + head0 + hl) * d + t * 8);
     }
     int slot[QKV_GROUP];
     bool together = tok0 + QKV_GROUP <= n;
@@ -398,7 +432,7 @@ __global__ __launch_bounds__(QKV_THREADS) void qk_rope_kv_bf16_vec_kernel(
     const int units_per_block = QKV_THREADS / tpu;
     const int u = threadIdx.x / tpu, t = threadIdx.x - u * tpu;
     if (v_from >= 0 && (int)blockIdx.x >= v_from) {
-        values_in_groups((uint16_t*)rows, v_cache, qkv, slots, (int)blockIdx.x - v_from, n, nq, nkv, d, page_size);
+        values_in_groups((uint16_t*)rows, v_cache, StoredRows{qkv}, slots, (int)blockIdx.x - v_from, n, nq, nkv, d, page_size);
         return;
     }
     const int heads = slots ? (v_from >= 0 ? nq + nkv : nq + 2 * nkv) : nq;
@@ -508,11 +542,12 @@ __global__ __launch_bounds__(QKV_THREADS) void qk_rope_kv_bf16_vec_kernel(
 // rows are all asked for before the first is used, and the sum of squares and the rotation partners
 // go from lane to lane without shared memory.  The sum runs in the order of the kernel above, so
 // that both give the same bits.
-#define QKV_HEADS 8
-template <int TPU>
+// QKV_HEADS: 8; 2 in steps of few tokens, where threads of eight heads would leave most of the chip without a block (117 tokens
+// of 24 heads: 44 blocks; 8.3 -> 5.6 us).
+template <int TPU, int QKV_HEADS, typename Rows>
 __global__ __launch_bounds__(QKV_THREADS) void qk_rope_kv_bf16_rows_kernel(
     bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache,
-    const bf16_t* __restrict__ qkv, const float* __restrict__ q_norm_w, const float* __restrict__ k_norm_w,
+    const Rows qkv, const float* __restrict__ q_norm_w, const float* __restrict__ k_norm_w,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t, const int* __restrict__ slots,
     int n, int nq, int nkv, int page_size, float eps, int add_one, int v_from) {
     constexpr int D = TPU * 8, HALF = D / 2;
@@ -529,11 +564,11 @@ __global__ __launch_bounds__(QKV_THREADS) void qk_rope_kv_bf16_rows_kernel(
     const int hn = nq + nkv - h0 < QKV_HEADS ? nq + nkv - h0 : QKV_HEADS;
     const int e0 = t * 8;
     const bool first = e0 < HALF;
-    const bf16_t* src = qkv + ((size_t)tok * (nq + 2 * nkv) + h0) * D + e0;
+    const size_t src = ((size_t)tok * (nq + 2 * nkv) + h0) * D + e0;
     uint4 raw[QKV_HEADS];
 #pragma unroll
     for (int i = 0; i < QKV_HEADS; ++i)
-        if (i < hn) raw[i] = *(const uint4*)(src + (size_t)i * D);
+        if (i < hn) raw[i] = qkv.eight(src + (size_t)i * D);
     const size_t at = (size_t)tok * HALF + (first ? e0 : e0 - HALF);
     const float4 c0 = *(const float4*)(cos_t + at), c1 = *(const float4*)(cos_t + at + 4);
     const float4 s0 = *(const float4*)(sin_t + at), s1 = *(const float4*)(sin_t + at + 4);
@@ -592,16 +627,23 @@ __global__ __launch_bounds__(QKV_THREADS) void qk_rope_kv_bf16_rows_kernel(
     }
 }
 
-template <int TPU>
-static void launch_rows(bf16_t* q_out, bf16_t* k_cache, bf16_t* v_cache, const bf16_t* qkv, const float* q_norm_w,
+template <int TPU, typename Rows>
+static void launch_rows(bf16_t* q_out, bf16_t* k_cache, bf16_t* v_cache, const Rows qkv, const float* q_norm_w,
                         const float* k_norm_w, const float* cos_t, const float* sin_t, const int* slots, int n,
                         int nq, int nkv, int page_size, float eps, int add_one, long long v_blocks,
                         hipStream_t stream) {
-    const long long chunks = (nq + nkv + QKV_HEADS - 1) / QKV_HEADS;
-    const long long qk_blocks = ((long long)n * chunks + QKV_THREADS / TPU - 1) / (QKV_THREADS / TPU);
-    qk_rope_kv_bf16_rows_kernel<TPU><<<(unsigned)(qk_blocks + v_blocks), QKV_THREADS, 0, stream>>>(
-        q_out, k_cache, v_cache, qkv, q_norm_w, k_norm_w, cos_t, sin_t, slots, n, nq, nkv, page_size, eps, add_one,
-        (int)qk_blocks);
+    auto blocks = [&](int heads) {
+        const long long chunks = (nq + nkv + heads - 1) / heads;
+        return ((long long)n * chunks + QKV_THREADS / TPU - 1) / (QKV_THREADS / TPU);
+    };
+    const bool few = blocks(8) < 512;
+    const long long qk_blocks = blocks(few ? 2 : 8);
+    if (few)
+        qk_rope_kv_bf16_rows_kernel<TPU, 2, Rows><<<(unsigned)(qk_blocks + v_blocks), QKV_THREADS, 0, stream>>>(
+            q_out, k_cache, v_cache, qkv, q_norm_w, k_norm_w, cos_t, sin_t, slots, n, nq, nkv, page_size, eps, add_one, (int)qk_blocks);
+    else
+        qk_rope_kv_bf16_rows_kernel<TPU, 8, Rows><<<(unsigned)(qk_blocks + v_blocks), QKV_THREADS, 0, stream>>>(
+            q_out, k_cache, v_cache, qkv, q_norm_w, k_norm_w, cos_t, sin_t, slots, n, nq, nkv, page_size, eps, add_one, (int)qk_blocks);
 }
 
 static int g_group_values = 1, g_rows = 1;
@@ -642,7 +684,7 @@ extern "C" int ia_qk_rope_kv(void* q_out, void* k_cache, void* v_cache, const vo
         const int tpu = d / 8;
         if (grouped && g_rows && cos_t != nullptr && rot == d && !interleaved && tpu >= 2 && tpu <= 64 &&
             (tpu & (tpu - 1)) == 0) {
-#define ROWS_CASE(T) case T: launch_rows<T>((bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache, (const bf16_t*)qkv, \
+#define ROWS_CASE(T) case T: launch_rows<T>((bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache, StoredRows{(const bf16_t*)qkv}, \
                      q_norm_w, k_norm_w, cos_t, sin_t, slots, n, nq, nkv, page_size, eps, add_one, v_blocks, stream); break;
             switch (tpu) { ROWS_CASE(2) ROWS_CASE(4) ROWS_CASE(8) ROWS_CASE(16) ROWS_CASE(32) ROWS_CASE(64) }
 #undef ROWS_CASE
@@ -667,5 +709,38 @@ extern "C" int ia_qk_rope_kv(void* q_out, void* k_cache, void* v_cache, const vo
     else
         IA_CHECK(false, "qk_rope_kv: unknown dtype %d", dtype);
     IA_LAUNCH_CHECK("qk_rope_kv");
+    return 0;
+}
+
+// Whether ia_qk_rope_kv_partials takes a step: the sizes that its kernel is made for (whole heads rotated in halves, pages of whole groups).
+extern "C" int ia_qk_rope_kv_partials_fits(int n, int d, int rot, int interleaved, int page_size) {
+    const int tpu = d / 8;
+    return n >= 2 * QKV_GROUP && d % 8 == 0 && rot == d && !interleaved && page_size > 0 && page_size % QKV_GROUP == 0 && tpu >= 2 &&
+           tpu <= QKV_THREADS / QKV_GROUP && (tpu & (tpu - 1)) == 0;
+}
+
+// ia_qk_rope_kv on projections that are still split along their k: parts [splits][n][(nq + 2 nkv) d] float, added up in their order
+// and rounded to bfloat16 on the way in, the same bits as from the stored product.  bfloat16 caches, a rotation, slots.
+extern "C" int ia_qk_rope_kv_partials(void* q_out, void* k_cache, void* v_cache, const float* parts, int splits,
+                                      const float* q_norm_w, const float* k_norm_w, const float* cos_t, const float* sin_t,
+                                      const int* slots, int n, int nq, int nkv, int d, int page_size, float eps, int add_one,
+                                      hipStream_t stream) {
+    IA_CHECK(nq > 0 && nkv > 0 && splits >= 1, "qk_rope_kv_partials: bad sizes nq=%d nkv=%d splits=%d", nq, nkv, splits);
+    IA_CHECK(ia_qk_rope_kv_partials_fits(n, d, d, 0, page_size), "qk_rope_kv_partials: n=%d, heads of %d, pages of %d are not taken", n, d, page_size);
+    IA_CHECK(q_out && k_cache && v_cache && parts && cos_t && sin_t && slots, "qk_rope_kv_partials: an array is missing");
+    const uintptr_t ptrs = (uintptr_t)q_out | (uintptr_t)parts | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)q_norm_w |
+                           (uintptr_t)k_norm_w | (uintptr_t)cos_t | (uintptr_t)sin_t;
+    IA_CHECK((ptrs & 15) == 0, "qk_rope_kv_partials: arrays must be 16-byte aligned");
+    const int tpu = d / 8, hpb = QKV_THREADS / tpu / QKV_GROUP;
+    const long long v_blocks = (long long)((n + QKV_GROUP - 1) / QKV_GROUP) * ((nkv + hpb - 1) / hpb);
+    IA_CHECK((long long)n * (nq + nkv) < (1ll << 30), "qk_rope_kv_partials: %d tokens are too many for one launch", n);
+    const size_t apart = (size_t)n * (nq + 2 * nkv) * d;
+#define PARTS_LAUNCH(T, S) launch_rows<T>((bf16_t*)q_out, (bf16_t*)k_cache, (bf16_t*)v_cache, SplitRows<S>{parts, splits, apart}, \
+                     q_norm_w, k_norm_w, cos_t, sin_t, slots, n, nq, nkv, page_size, eps, add_one, v_blocks, stream)
+#define PARTS_CASE(T) case T: if (splits == 2) PARTS_LAUNCH(T, 2); else if (splits == 4) PARTS_LAUNCH(T, 4); else PARTS_LAUNCH(T, 0); break;
+    switch (tpu) { PARTS_CASE(2) PARTS_CASE(4) PARTS_CASE(8) PARTS_CASE(16) PARTS_CASE(32) }
+#undef PARTS_CASE
+#undef PARTS_LAUNCH
+    IA_LAUNCH_CHECK("qk_rope_kv_partials");
     return 0;
 }

@@ -317,7 +317,16 @@ def qk_rope_kv(qkv: torch.Tensor, nq: int, nkv: int, d: int, *,
                rot: int, interleaved: bool, k_cache: Optional[torch.Tensor],
                v_cache: Optional[torch.Tensor], slots: Optional[torch.Tensor],
                page_size: int) -> torch.Tensor:
-    """Norm and rotate q and k, write k and v at `slots` of the cache; returns q [n, nq, d]."""
+    """Norm and rotate q and k, write k and v at `slots` of the cache; returns q [n, nq, d].  `qkv` may be a product still split
+    along its k (`Partials`), where the step's sizes are taken that way and there is a rotation and a cache to write."""
+    parts = None
+    if isinstance(qkv, Partials):
+        splits, n, width = qkv.parts.shape
+        if (cos is None or slots is None or k_cache is None or k_cache.dtype != torch.bfloat16 or width != (nq + 2 * nkv) * d
+                or not qk_rope_kv_partials_fits(n, d, rot, interleaved, page_size)):
+            qkv = qkv.materialize()
+        else:
+            parts, qkv = qkv.parts, qkv.parts[0]
     _dev(qkv, q_norm_w, k_norm_w, cos, sin, k_cache, v_cache, slots)
     _f32(q_norm_w, "q_norm weight"); _f32(k_norm_w, "k_norm weight"); _f32(cos, "cos"); _f32(sin, "sin")
     n = qkv.shape[0]
@@ -335,13 +344,23 @@ def qk_rope_kv(qkv: torch.Tensor, nq: int, nkv: int, d: int, *,
             raise KernelError("qk_rope_kv: slots given without a cache")
         if slots.numel() != n:
             raise KernelError(f"qk_rope_kv: {slots.numel()} slots for {n} tokens")
-        _check_cache(k_cache, v_cache, nkv, page_size, d, qkv.dtype, "qk_rope_kv")
-    q_out = torch.empty((n, nq, d), dtype=qkv.dtype, device=qkv.device)
+        _check_cache(k_cache, v_cache, nkv, page_size, d, qkv.dtype if parts is None else torch.bfloat16, "qk_rope_kv")
+    q_out = torch.empty((n, nq, d), dtype=qkv.dtype if parts is None else torch.bfloat16, device=qkv.device)
+    if parts is not None:
+        _check(library().ia_qk_rope_kv_partials(
+            _p(q_out), _p(k_cache), _p(v_cache), _p(parts), parts.shape[0], _p(q_norm_w), _p(k_norm_w), _p(cos), _p(sin), _p(slots),
+            n, nq, nkv, d, page_size, ctypes.c_float(eps), int(add_one), _stream()))
+        return q_out
     _check(library().ia_qk_rope_kv(
         _p(q_out), _p(k_cache if slots is not None else None), _p(v_cache if slots is not None else None),
         _p(qkv), _p(q_norm_w), _p(k_norm_w), _p(cos), _p(sin), _p(slots), n, nq, nkv, d, rot,
         int(interleaved), page_size, ctypes.c_float(eps), int(add_one), _dt(qkv), _stream()))
     return q_out
+
+
+def qk_rope_kv_partials_fits(n: int, d: int, rot: int, interleaved: bool, page_size: int) -> bool:
+    """Whether `qk_rope_kv` reads projections that are still split along their k (`Partials`) in a step of `n` tokens."""
+    return bool(library().ia_qk_rope_kv_partials_fits(n, d, rot, int(interleaved), page_size))
 
 
 def qk_rope_kv_strided(proj: torch.Tensor, nq: int, nkv: int, d: int, dv: int, *, q_off: int, k_off: Optional[int],
@@ -1080,15 +1099,16 @@ def gemm_wide_bf16(x: torch.Tensor, w: torch.Tensor, dual: bool = False, partial
     return out
 
 
-def linear_partials(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None):
+def linear_partials(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, own_rows: bool = False):
     """x . w^T for a reader that takes `Partials` (the norm that adds the product to the stream): split along k where the
     weight has few rows.  None when the product of 17 to 64 rows does not take these operands (a bias among them: the
     caller then forms the whole product, and `linear` adds the bias)."""
     # (whoever asks is in a step whose products go to gemm_mid.hip: the rule has been asked with the stream's width, and a
     # product of another width follows it)
-    if bias is None and isinstance(x, torch.Tensor) and x.shape[0] >= MID_MIN_ROWS and mid_fits(x, w, few_rows=True):
+    # (`own_rows`: outside such a step, the width of the rows themselves decides)
+    if bias is None and isinstance(x, torch.Tensor) and x.shape[0] >= MID_MIN_ROWS and mid_fits(x, w, few_rows=not own_rows):
         return gemm_mid_bf16(x, w, partial=True)
-    if bias is None and isinstance(x, torch.Tensor) and wide_fits(x, w):
+    if bias is None and isinstance(x, torch.Tensor) and wide_fits(x, w) and (not own_rows or x.shape[0] <= 1024):
         return gemm_wide_bf16(x, w, partial=True)
     return None
 

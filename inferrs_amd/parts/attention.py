@@ -268,7 +268,13 @@ class Attention(Mixer):
             return self._forward_general(ctx, h, cache)
         s = self.spec
         group = ctx.groups[cache.group]
-        qkv = self.qkv(h)
+        # (steps with prompt portions: the product may stay split along k for the kernel that reads it next)
+        qkv = None
+        if (ctx.max_q_len > 1 and cache.writable and not hasattr(h, "materialize")
+                and ops.qk_rope_kv_partials_fits(h.shape[0], s.head_dim, self.position.rot_dim, self.position.interleaved, group.page_size)):
+            qkv = ops.linear_partials(h, self.qkv.weight, self.qkv.bias, own_rows=True)
+        if qkv is None:
+            qkv = self.qkv(h)
         table = ctx.position_table(self.position)
         cos, sin = table if table is not None else (None, None)
         if ctx.max_q_len == 1 and ops.attention_decode_fused_fits(qkv.dtype, s.head_dim, group.page_size,

@@ -197,6 +197,30 @@ def test_qk_rope_kv_values_of_a_prompt_portion(nq, nkv, d, page, layout):
     assert torch.equal(q, q_1) and torch.equal(kc_d, kc_1) and torch.equal(vc_d, vc_1)
 
 
+@pytest.mark.parametrize("n,nq,nkv,d,page", [(16, 5, 5, 64, 8), (117, 16, 8, 128, 16), (61, 2, 1, 256, 24), (19, 3, 3, 16, 16), (1900, 32, 8, 128, 16),
+                                             (10, 4, 2, 128, 16), (33, 4, 2, 48, 8)])
+@pytest.mark.parametrize("splits", [2, 3, 4, 8])
+def test_qk_rope_kv_of_a_product_still_split(n, nq, nkv, d, page, splits):
+    """Projections as the sums of splits of k: queries and caches with the bits of the stored product, in steps that the kernel
+    for it takes (few tokens and many) and in those that it leaves to the kernel that stores the product first."""
+    from inferrs_amd import ops
+    g = torch.Generator().manual_seed(5)
+    pages = n // page + 3
+    slots = dev((torch.arange(n) + page + 3).to(torch.int32))
+    width = (nq + 2 * nkv) * d
+    split = ops.Partials(dev(randn(splits, n, width, dtype=torch.float32, seed=n + splits)))
+    norms = [dev(randn(d, dtype=torch.float32, seed=s)) for s in (23, 24)]
+    cos, sin = dev(torch.rand(n, d // 2, generator=g)), dev(torch.rand(n, d // 2, generator=g))
+    got = []
+    for rows in (split, split.materialize()):
+        kc, vc = (torch.zeros(shape, dtype=torch.bfloat16, device="cuda") for shape in ((pages, nkv, page, d), (pages, nkv, d, page)))
+        q = ops.qk_rope_kv(rows, nq, nkv, d, q_norm_w=norms[0], k_norm_w=norms[1], eps=1e-6, add_one=False, cos=cos, sin=sin, rot=d,
+                           interleaved=False, k_cache=kc, v_cache=vc, slots=slots, page_size=page)
+        got.append((q, kc, vc))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 def ref_attention(q, kc, vc, positions, token_seq, table, window, scale):
     n, nq, d = q.shape
     nkv, page = kc.shape[1], kc.shape[2]
