@@ -603,7 +603,7 @@ __global__ __launch_bounds__(256) void linear_carry_mfma_kernel(const ScanArgs a
 #define LL_V_LD 36
 
 template <typename T>
-__global__ __launch_bounds__(256) void linear_local_mfma_kernel(const ScanArgs a, int ld_s) {
+__global__ __launch_bounds__(256) void linear_local_mfma_kernel(const ScanArgs a, int ld_s, int cols) {
     extern __shared__ __attribute__((aligned(16))) float ll_shared[];
     // (The scores take the place of the queries where a row of queries is long enough for a row of scores: a wave
     // writes the scores of its 16 tokens after it has read those tokens' queries, and nobody else reads them.  Two
@@ -646,7 +646,7 @@ __global__ __launch_bounds__(256) void linear_local_mfma_kernel(const ScanArgs a
         }
         const float g_last = __shfl(g, LC_TOKENS - 1, IA_WAVE);
         g_s[tt] = g; b_s[tt] = b; w_s[tt] = expf(g_last - g) * b;
-        if (tt == 0) a.chunk_a[(long long)blockIdx.z * a.H + h] = expf(g_last);
+        if (tt == 0 && blockIdx.x == 0) a.chunk_a[(long long)blockIdx.z * a.H + h] = expf(g_last);
     }
     __syncthreads();
     // ---- the weighted scores ------------------------------------------------------------------------------------
@@ -675,7 +675,8 @@ __global__ __launch_bounds__(256) void linear_local_mfma_kernel(const ScanArgs a
     const float skip = a.skip != nullptr ? a.skip[h] : 0.f;
     float* const u_out = a.chunk_s + ((long long)blockIdx.z * a.H + h) * vt * a.dim;
     const int row_tiles = (a.dim + 15) / 16;
-    for (int j0 = 0; j0 < vt; j0 += 32) {
+    const int j_end = min(vt, ((int)blockIdx.x + 1) * cols);
+    for (int j0 = blockIdx.x * cols; j0 < j_end; j0 += 32) {
         __syncthreads();                                   // (the scores are written; the columns before are used up)
         {
             const int j = j0 + (threadIdx.x & 31);
@@ -779,6 +780,15 @@ extern "C" long long ia_linear_scan_workspace(int n_seqs, int max_q_len, int chu
 // chunk 0: every request's tokens are walked from its state row.  chunk > 0: portions are cut into chunks of that many
 // tokens that run side by side; `workspace` holds ia_linear_scan_workspace(...) floats and max_q_len is an upper bound
 // of the tokens a request brings.
+static int linear_cus() {
+    static int cus = 0;
+    if (cus == 0) {
+        int dev = 0, n = 0;
+        cus = hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+    }
+    return cus;
+}
+
 extern "C" int ia_linear_scan(float* out, float* den, float* state, long long row_floats, long long s_off,
                               const void* q, long long q_ld, int q_off, int q_heads,
                               const void* k, long long k_ld, int k_off, int k_heads,
@@ -857,7 +867,14 @@ extern "C" int ia_linear_scan(float* out, float* den, float* state, long long ro
     const bool cores = g_carry_mfma && dim <= LC_MAX_DIM && chunk <= LC_TOKENS;
     if (cores) {
         const int ld_s = (dim + 3) / 4 * 4 + 4;
-        const dim3 lgrid(1, (unsigned)H, (unsigned)(n_seqs * a.max_chunks));
+        // Columns a block: all of them, or fewer (in steps of 32), each share with scores of its own, until the step has two
+        // blocks for every compute unit (24 chunks of 8 heads with values of 256 and a normaliser: nine steps of columns in 192
+        // blocks 74.5 us, three blocks a chunk and head 41; 16 heads of 128 in 384 blocks 37.9, in 768 31).
+        const int steps = (vt + 31) / 32;
+        int shares = 1;
+        while (shares < steps && (long long)shares * H * n_seqs * a.max_chunks < 2 * linear_cus()) ++shares;
+        const int cols = (steps + shares - 1) / shares * 32;
+        const dim3 lgrid((unsigned)((vt + cols - 1) / cols), (unsigned)H, (unsigned)(n_seqs * a.max_chunks));
         const int lshm = (int)((2 * LC_TOKENS * ld_s + LC_TOKENS * ((ld_s >= LL_P_LD ? 0 : LL_P_LD) + LL_V_LD) + 3 * LC_TOKENS) * sizeof(float));
         static int asked_f32 = 0, asked_bf16 = 0;          // shared memory beyond 64 KiB has to be asked for, once per instantiation
         int& asked = dtype == IA_F32 ? asked_f32 : asked_bf16;
@@ -868,8 +885,8 @@ extern "C" int ia_linear_scan(float* out, float* den, float* state, long long ro
             IA_CHECK(e == hipSuccess, "linear_scan: cannot ask for %d bytes of shared memory: %s", 112 * 1024, hipGetErrorString(e));
             asked = 112 * 1024;
         }
-        if (dtype == IA_F32) linear_local_mfma_kernel<float><<<lgrid, 256, lshm, stream>>>(a, ld_s);
-        else linear_local_mfma_kernel<bf16_t><<<lgrid, 256, lshm, stream>>>(a, ld_s);
+        if (dtype == IA_F32) linear_local_mfma_kernel<float><<<lgrid, 256, lshm, stream>>>(a, ld_s, cols);
+        else linear_local_mfma_kernel<bf16_t><<<lgrid, 256, lshm, stream>>>(a, ld_s, cols);
     } else {
         LS_LAUNCH(LS_LOCAL, grid);
     }

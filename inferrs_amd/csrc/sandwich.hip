@@ -45,6 +45,86 @@ __global__ __launch_bounds__(1024) void sandwich_step_kernel(
         st(h + (long long)r * W + c, sw_row[c] * rs2 * (w_pre != nullptr ? w_pre[c] : 1.f));
 }
 
+// The same for widths of a multiple of eight: a thread owns eight neighbouring features, which stay in registers between the two
+// norms, and moves them 16 bytes at a time.  Bound by the memory: 14 bytes a feature for a bfloat16 output and rows (1,500 rows of
+// 2,048: 17.0 -> 9.6 us; one feature a thread asked for 2 and 4 bytes at a time and read the row back from shared memory twice).
+__device__ __forceinline__ void sw_load8(const float* p, float (&v)[8]) {
+    const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+__device__ __forceinline__ void sw_load8(const bf16_t* p, float (&v)[8]) {
+    const uint4 q = *(const uint4*)p;
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[2 * j] = __uint_as_float(w[j] << 16);
+        v[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
+    }
+}
+__device__ __forceinline__ void sw_store8(float* p, const float (&v)[8]) {
+    *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
+    *(float4*)(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+}
+__device__ __forceinline__ void sw_store8(bf16_t* p, const float (&v)[8]) {
+    *(uint4*)p = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+}
+
+template <typename TY, typename TH>
+__global__ __launch_bounds__(1024) void sandwich_step8_kernel(
+    float* __restrict__ x, const TY* __restrict__ y1, float s1, const TY* __restrict__ y2, float s2,
+    const float* __restrict__ w_post, const TY* __restrict__ e_rows, const float* __restrict__ e_vec,
+    const float* __restrict__ w_pre, float eps_post, float eps, TH* __restrict__ h, const int* __restrict__ rows, int W) {
+    __shared__ float scratch[16];
+    const int r = blockIdx.x, c = threadIdx.x * 8;
+    const bool in = c < W;
+    const int row = rows != nullptr ? rows[r] : r;
+    const long long at = (long long)row * W + c;
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, t[8];
+    if (in) sw_load8(x + at, v);
+    if (y1 != nullptr) {
+        float sq = 0.f;
+        if (in) {
+            sw_load8(y1 + at, y);
+            if (y2 != nullptr) sw_load8(y2 + at, t);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                y[j] *= s1;
+                if (y2 != nullptr) y[j] = fmaf(s2, t[j], y[j]);
+                sq = fmaf(y[j], y[j], sq);
+            }
+        }
+        const float rs = 1.0f / sqrtf(block_sum(sq, scratch) / (float)W + eps_post);
+        if (in) {
+            sw_load8(w_post + c, t);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] += y[j] * rs * t[j];
+        }
+    }
+    float sq = 0.f;
+    if (in) {
+        if (e_rows != nullptr) {
+            sw_load8(e_rows + at, t);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] += t[j];
+        }
+        if (e_vec != nullptr) {
+            sw_load8(e_vec + c, t);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] += t[j];
+        }
+        if (rows == nullptr && (y1 != nullptr || e_rows != nullptr || e_vec != nullptr)) sw_store8(x + at, v);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sq = fmaf(v[j], v[j], sq);
+    }
+    if (h == nullptr) return;
+    const float rs2 = 1.0f / sqrtf(block_sum(sq, scratch) / (float)W + eps);
+    if (!in) return;
+    if (w_pre != nullptr) sw_load8(w_pre + c, t);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = v[j] * rs2 * (w_pre != nullptr ? t[j] : 1.f);
+    sw_store8(h + (long long)r * W + c, v);
+}
+
 // y_dtype: precision of y1, y2 and e_rows; h_dtype: of h.  0 float32, 1 bfloat16.
 extern "C" int ia_sandwich_step(float* x, const void* y1, float s1, const void* y2, float s2, const float* w_post,
                                 const void* e_rows, const float* e_vec, const float* w_pre, float eps_post, float eps, void* h,
@@ -54,6 +134,20 @@ extern "C" int ia_sandwich_step(float* x, const void* y1, float s1, const void* 
     IA_CHECK(y1 != nullptr || y2 == nullptr, "sandwich_step: a second output goes with a first");
     IA_CHECK(y1 == nullptr || w_post != nullptr, "sandwich_step: an output to add needs the weight of the norm behind it");
     if (n == 0) return 0;
+    if (W % 8 == 0 && W <= 8192 && (((uintptr_t)x | (uintptr_t)y1 | (uintptr_t)y2 | (uintptr_t)w_post | (uintptr_t)e_rows |
+                                     (uintptr_t)e_vec | (uintptr_t)w_pre | (uintptr_t)h) & 15) == 0) {
+        const int threads8 = (W / 8 + IA_WAVE - 1) / IA_WAVE * IA_WAVE;
+#define IA_LAUNCH8(TY, TH)                                                                                        \
+    sandwich_step8_kernel<TY, TH><<<n, threads8, 0, stream>>>(x, (const TY*)y1, s1, (const TY*)y2, s2, w_post,      \
+                                                              (const TY*)e_rows, e_vec, w_pre, eps_post, eps, (TH*)h, rows, W)
+        if (y_dtype == IA_F32 && h_dtype == IA_F32) { IA_LAUNCH8(float, float); }
+        else if (y_dtype == IA_F32) { IA_LAUNCH8(float, bf16_t); }
+        else if (h_dtype == IA_F32) { IA_LAUNCH8(bf16_t, float); }
+        else { IA_LAUNCH8(bf16_t, bf16_t); }
+#undef IA_LAUNCH8
+        IA_LAUNCH_CHECK("sandwich_step");
+        return 0;
+    }
     const int threads = W >= 4096 ? 1024 : W >= 1024 ? 512 : 256;
     const size_t shm = (size_t)W * sizeof(float);
 #define IA_LAUNCH(TY, TH)                                                                                         \
