@@ -334,15 +334,24 @@ class Engine:
         extra = self._pad_rows(len(triples), 1) if len(singles) == len(triples) else 0
         if extra:
             triples = list(triples) + [(_PAD, [0], [0])] * extra
-        longest = self.cache.max_length(singles) + 1 if singles else 0
+        longest = longest_single = self.cache.max_length(singles) + 1 if singles else 0
+        longest_multi = 0
         for t in triples:
             if len(t[1]) > 1:
-                longest = max(longest, self.cache.length(t[0]) + len(t[1]))
+                longest_multi = max(longest_multi, self.cache.length(t[0]) + len(t[1]))
+        longest = max(longest, longest_multi)
         pad_pages = self._bucket_pages(longest)
         self._drop_stale_graphs()
         ctx = self.builder.build(triples, pad_pages=pad_pages)
         self._drop_stale_graphs()                       # (the buffer may have moved in this very build)
         key = (ctx.n_seqs, ctx.n_tokens, ctx.n_single, int(ctx.want_rows.shape[0]), ctx.max_q_len, pad_pages)
+        if 0 < ctx.n_single < ctx.n_seqs:
+            # (portions beside single tokens: each run's launches follow from its own longest context, in buckets of their own.
+            # 512 tokens behind 1,500 beside contexts of 3,100: bounded by those, the portion's keys were split in two at 2,048,
+            # the second half empty, 82 us a layer at 40 query heads against 48)
+            bounds = self._bucket_pages(longest_single), self._bucket_pages(longest_multi)
+            ctx.max_kv_single, ctx.max_kv_multi = (pages * self.page_size for pages in bounds)
+            key += bounds
         entry = self._graphs.get(key)
         if entry is not None:
             self._graphs.move_to_end(key)

@@ -498,10 +498,21 @@ def attention_split(n_seqs: int, nkv: int, g: int, max_q_len: int, max_kv_len: i
             # walks are short, and where the blocks are few the kernel halves them instead (a portion of 512 tokens at
             # a context of 2,048, 32 query heads: 29.7 us whole in blocks of 64 columns against 36.8 in two splits)
             return 1, -(-max_kv_len // 64) * 64
+        # Full rounds of the compute units times a share's keys, in microseconds: a key takes a block of 128 columns 0.0183 alone
+        # on its unit and 0.02 on a full chip, one of 64 columns (which the kernel takes for few blocks that are not split)
+        # 0.0138; partial sums and their merge about 13 and 1 a split.  Measured, whole and in 2, 3 and 4 splits: 40 query heads,
+        # 512 tokens at 7,512 keys 138, 155, 117, 136; 300 tokens at 7,300 91, 79, 105, 90; 256 tokens at 12,256 144, 119, 90, 129;
+        # 32 query heads, 512 tokens at 8,012 117, 103, 130, 110; 256 tokens at 3,256 43, 43, 37, 33.
         items = n_seqs * nkv * -(-cols // ATTN_TILE_COLS)
-        splits = 1
-        while items * splits < ATTN_TILE_BLOCKS and max_kv_len >= 2 * splits * ATTN_TILE_MIN_CHUNK and splits < 128:
-            splits *= 2
+        whole = 4.0 + 0.0138 * max_kv_len if 2 * items <= ATTN_TILE_BLOCKS else 8.0 + 0.0183 * max_kv_len * -(-items // ATTN_TILE_BLOCKS)
+        best, splits = whole, 1
+        for ways in range(2, 17):
+            chunk = -(-(-(-max_kv_len // ways)) // 64) * 64
+            if chunk < ATTN_TILE_MIN_CHUNK:
+                break
+            cost = 21.0 + ways + 0.02 * chunk * -(-items * ways // ATTN_TILE_BLOCKS)
+            if cost < best:
+                best, splits = cost, ways
         chunk = -(-max_kv_len // splits)
         return splits, -(-chunk // 64) * 64
     col_blocks = 1 if cols <= 16 else -(-cols // 32)
@@ -1072,8 +1083,9 @@ WIDE_MAX_ROWS = 2048
 
 
 def wide_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether gemm_wide.hip takes x . w^T (beyond the rows of gemm_mid.hip, up to `WIDE_MAX_ROWS`)."""
-    return (MID_PRODUCTS == "own" and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+    """Whether gemm_wide.hip takes x . w^T (beyond the rows of gemm_mid.hip, up to `WIDE_MAX_ROWS`); not where the switches ask
+    for the vendor's GEMM or for the tiled kernel of gemm_mfma.hip throughout."""
+    return (MID_PRODUCTS == "own" and LARGE_PRODUCTS == "library" and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and MID_MAX_ROWS < x.shape[0] <= WIDE_MAX_ROWS and x.shape[1] % 64 == 0 and w.shape[1] == x.shape[1]
             and w.shape[0] % 4 == 0 and x.is_contiguous() and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
