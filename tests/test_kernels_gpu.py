@@ -411,6 +411,21 @@ def test_attention_mfma_prompt_portions_head_size_128(nq, nkv, page, window, len
         close(outs[0], want, 2 ** -7, f"blocks of 64 columns, splits={splits}")
 
 
+@pytest.mark.parametrize("splits", [5, 7, 11, 16])
+def test_attention_mfma_portion_in_any_number_of_splits(splits):
+    """Portions late in their contexts with the keys in other numbers of shares than powers of two: shares that end inside a
+    request's keys, that lie behind its newest token, and a last share of the whole step that is nearly empty."""
+    from inferrs_amd import ops
+    dtype, d, nq, nkv, page = torch.bfloat16, 128, 8, 2, 16
+    lens, q_lens = [1030, 210], [70, 33]
+    q, kc, vc, positions, token_seq, table = attention_case(dtype, nq, nkv, d, page, lens, q_lens, 23, needle=True)
+    cu = torch.tensor([0, 70, 103], dtype=torch.int32)
+    scale = 1.0 / math.sqrt(d)
+    got = ops.attention_mfma(dev(q), dev(kc), dev(vc), dev(positions), dev(cu), dev(table), max_q_len=70, max_kv_len=1030,
+                             window=None, scale=scale, splits=splits)
+    close(got, ref_attention_dense(q, kc, vc, positions, token_seq, table, None, scale), 2 ** -7, splits)
+
+
 def test_attention_mfma_prompt_that_half_fills_the_chip():
     """Between one and two blocks a compute unit the second half of the blocks walks its tiles in the other
     order; with 47 tiles a row of the grid that half does not begin at a row's start."""
@@ -838,6 +853,19 @@ def test_mid_product(m, n, k):
         close(split.materialize(), want, 2 ** -8, "sum of the splits")
     else:
         assert ops.library().ia_gemm_mid_splits(n, k) == 1 or (m * n) % 4
+
+
+@pytest.mark.parametrize("m", [17, 64, 65, 128])
+@pytest.mark.parametrize("n", [131056, 131072, 131077])
+def test_mid_product_of_a_logits_head(m, n):
+    """Around the number of features from which the blocks have eight waves (131,057 and more on 256 compute units), rows of
+    both pipelines, features that fill no block."""
+    from inferrs_amd import ops
+    k = 384
+    x, w = dev(randn(m, k, dtype=torch.bfloat16, seed=m)), dev(randn(n, k, dtype=torch.bfloat16, seed=n, scale=0.05))
+    want = x.float().cpu() @ w.float().cpu().t()
+    close(ops.gemm_mid_bf16(x, w, torch.float32), want, 2e-6 * math.sqrt(k), "a head's logits")
+    close(ops.gemm_mid_bf16(x, w), want, 2 ** -8, "a head's logits, stored in 16 bits")
 
 
 def test_mid_product_splits_depend_on_the_weight_alone():

@@ -322,6 +322,40 @@ def test_captured_mixed_steps_equal_eager_ones(tiny, dtype):
     assert err <= (1e-5 if dtype == "float32" else 3e-2), err
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_captured_mixed_steps_whose_runs_lie_in_different_buckets(tiny, dtype):
+    """A request decodes through buckets of 64 tokens while portions beside it come from other buckets, shorter and longer than
+    its own: a captured step holds its launches' bounds, so a step of the same sizes in another pair of buckets is another
+    graph.  Twice over the same way, so that every pair is met eagerly and replayed; the logits are those without graphs."""
+    from inferrs_amd.engine import Engine, Entry
+    folder, cfg, params = tiny["B"]
+    vocab = TINY["B"]["vocab_size"]
+    portion, portions, rounds = 24, 6, 4
+    single = random_tokens(90 + rounds * portions, vocab, 700)
+    prompt = random_tokens(portion * portions, vocab, 701)
+    outs = {}
+    for graphs in (True, False):
+        eng = Engine.from_folder(folder, dtype=dtype, page_size=8, num_pages=60, max_seqs=4, use_graphs=graphs)
+        eng.GRAPH_HOST_SHARE, eng.GRAPH_BUCKET_TOKENS = 0.0, 64
+        eng.step([Entry("a", single[:90], [])])
+        at, rows = 90, []
+        for k in range(rounds):
+            for j in range(portions):
+                rows.append(eng.step([Entry("a", [single[at]], [0]), Entry(f"p{k}", prompt[j * portion:(j + 1) * portion], [portion - 1])]).clone())
+                torch.cuda.synchronize()
+                at += 1
+            eng.end_request(f"p{k}")
+        eng.cache.check_invariants()
+        assert not graphs or eng.graph_replays >= 6
+        outs[graphs] = torch.stack(rows)
+    scale = float(outs[False].abs().max())
+    assert float((outs[True] - outs[False]).abs().max()) / scale <= (1e-6 if dtype == "float32" else 2e-2)
+    for column, toks, places in ((0, single, list(range(90, at))), (1, prompt, [portion * (j + 1) - 1 for j in range(portions)] * rounds)):
+        ref = pm.forward(cfg, params, toks)
+        err = float((outs[True][:, column].cpu().double() - ref[places]).abs().max() / ref.abs().max())
+        assert err <= (1e-5 if dtype == "float32" else 3e-2), (column, err)
+
+
 def test_a_shape_whose_step_the_gpu_bounds_stays_eager(tiny):
     """The capture of a step other than a decode step is decided by a measurement: with a share that no host can
     reach the shape is marked eager at its third step and never captured, and its logits are the same."""
