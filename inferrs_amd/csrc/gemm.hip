@@ -1,10 +1,10 @@
 // Matrix products y[m, n] = sum_k x[m, k] * w[n, k] for weights stored [out, in] as the
 // checkpoints hold them (the reference's Linear is x . W^T, candle-nn/src/linear.rs:64-72).
 //
-//   * ia_gemm_tiled: plain 64x64 tiles through shared memory, fused multiply-adds in 32-bit
+//   * ia_gemm_tiled: plain tiles through shared memory, fused multiply-adds in 32-bit
 //     with k ascending for every output, whatever the number of rows: a row's result does
 //     not depend on what else is in the batch.  It is the matrix product of the true 32-bit
-//     path and takes bfloat16 inputs of any size as the fallback of the kernel below.
+//     path (a decode step's rows here, more on the matrix cores with the same bits, gemm_f32.hip) and takes bfloat16 inputs of any size as the fallback of the kernel below.
 //   * ia_gemm_skinny_bf16: few rows (decode batches, logits of a few positions) against a
 //     large weight matrix.  The product is bound by reading the weights once, so each wave
 //     streams 16 weight rows in 16-byte pieces straight into MFMA 16x16x32 operands and
@@ -76,7 +76,7 @@ __device__ __forceinline__ float4 gr_load4(const bf16_t* p) {
                        bf16_bits_to_f32((uint16_t)v.y), bf16_bits_to_f32((uint16_t)(v.y >> 16)));
 }
 
-// The same sums in tiles of 128 x 128 for many rows (prompts of the 32-bit path): a thread owns 8 x 8 outputs (rows
+// The same sums in tiles of 128 x 128 for many rows of bfloat16 that no kernel of the matrix cores takes: a thread owns 8 x 8 outputs (rows
 // 4 ty .. + 4 and 64 + 4 ty .. + 4, features likewise with tx), so that every value read from shared memory meets eight
 // fused multiply-adds instead of four; k ascending for every output as above, hence the same bits.  K a multiple of 4.
 #define GB 128
@@ -260,12 +260,11 @@ extern "C" int ia_gemm_tiled(void* out, const void* x, const void* w, int M, int
     const size_t elem = in_dtype == IA_F32 ? 4 : 2;
     // The 32-bit path on the matrix cores: the same bits.  Up to 16 rows the kernel below reads the weights faster, unless
     // they have very many rows.  (4,096 k, us, the vector units' kernels against it: 8 rows 6,144 features 42 / 66, 24,576 87 /
-    // 120, 151,936 556 / 464; 16 rows 51 / 66, 147 / 118, 901 / 479; 32 rows 99 / 45, 717 / 124; 128 rows 554 / 94, 993 / 256.)
+    // 120, 151,936 556 / 464; 16 rows 51 / 66, 147 / 118, 901 / 479; 32 rows 99 / 46, 717 / 133; 128 rows 554 / 104, 993 / 238.)
     if (in_dtype == IA_F32 && out_dtype == IA_F32 && K % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 &&
         (M > GR_ROWS || N >= (M > 8 ? 64 : 256) * skinny_cus()) && (g_rows_shape == 0 || M > GR_ROWS))
         return ia_gemm_f32(out, x, w, M, N, K, stream);
-    // up to 64 rows, 16 at a time, where the tiles of 64 x 64 would be few (the weights are read once for every 16 rows:
-    // at 32 rows of the 32-bit path a decode step of four layers at the sizes of an 8B model still takes a third of the time)
+    // up to 64 rows, 16 at a time, where the tiles of 64 x 64 would be few (the weights are read once for every 16 rows)
     if (M <= 4 * GR_ROWS && (M <= GR_ROWS || N <= 4096 * 4) && K % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) % (4 * elem)) == 0) {
         const size_t out_elem = out_dtype == IA_F32 ? 4 : 2;
         for (int m0 = 0; m0 < M; m0 += GR_ROWS) {

@@ -869,7 +869,7 @@ extern "C" int ia_linear_scan(float* out, float* den, float* state, long long ro
         const int ld_s = (dim + 3) / 4 * 4 + 4;
         // Columns a block: all of them, or fewer (in steps of 32), each share with scores of its own, until the step has two
         // blocks for every compute unit (24 chunks of 8 heads with values of 256 and a normaliser: nine steps of columns in 192
-        // blocks 74.5 us, three blocks a chunk and head 41; 16 heads of 128 in 384 blocks 37.9, in 768 31).
+        // blocks 74 us, shared out 71; 16 heads of 128 in 384 blocks 38, in 768 29).
         const int steps = (vt + 31) / 32;
         int shares = 1;
         while (shares < steps && (long long)shares * H * n_seqs * a.max_chunks < 2 * linear_cus()) ++shares;

@@ -47,7 +47,7 @@ __global__ __launch_bounds__(1024) void sandwich_step_kernel(
 
 // The same for widths of a multiple of eight: a thread owns eight neighbouring features, which stay in registers between the two
 // norms, and moves them 16 bytes at a time.  Bound by the memory: 14 bytes a feature for a bfloat16 output and rows (1,500 rows of
-// 2,048: 17.0 -> 9.6 us; one feature a thread asked for 2 and 4 bytes at a time and read the row back from shared memory twice).
+// 2,048: 17.0 -> 9.8 us; one feature a thread asked for 2 and 4 bytes at a time and read the row back from shared memory twice).
 __device__ __forceinline__ void sw_load8(const float* p, float (&v)[8]) {
     const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;

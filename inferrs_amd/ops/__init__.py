@@ -480,7 +480,7 @@ def attention_mfma_fits(dtype: torch.dtype, d: int, page_size: int, dv: Optional
 
 
 ATTN_TILE_COLS = 128           # head size 128, prompt portions: columns a block of four waves
-ATTN_TILE_BLOCKS = 256         # blocks wanted (one a compute unit: eight waves) before the keys stop being split
+ATTN_TILE_BLOCKS = 256         # compute units: a block's eight waves fill one
 ATTN_TILE_MIN_CHUNK = 512      # fewest keys a block's share is worth (eight stages of 64)
 ATTN_TILE_WHOLE_UP_TO = 2048   # contexts up to this length are not split
 
@@ -704,7 +704,7 @@ def attention_decode_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: to
 
 # ---- matrix products --------------------------------------------------------------------------
 
-# Beyond this many rows (one tile of MFMA columns) the vendor's GEMM reads the weights faster.  Up to 16 rows the
+# Beyond this many rows (one tile of MFMA columns) other kernels read the weights faster.  Up to 16 rows the
 # skinny products also take over the sums and norms of the residual stream; a decode step at a context of 2,048
 # and the sizes of an 8 B model takes 5.02 ms with 12 requests, 5.20 with 13 and 5.22 with 16 (5.54 and 5.44 with
 # the vendor's GEMM and norm kernels of their own from 13 rows on; at the 14B shape 9.7 against 10.9 ms at 14 rows).
@@ -1143,7 +1143,7 @@ def add_rmsnorm_partials(x: torch.Tensor, delta: Partials, w: torch.Tensor, eps:
 
 def linear(x, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None, mid: bool = True,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x [m, k] . w[n, k]^T (+ bias [n], in the precision of w).  32-bit: the tiled kernel (true 32-bit, fixed
+    """x [m, k] . w[n, k]^T (+ bias [n], in the precision of w).  32-bit: `gemm_tiled` (true 32-bit, fixed
     order).  bfloat16: the skinny MFMA kernel for up to SKINNY_MAX_ROWS rows, the vendor's GEMM beyond that (the
     reference uses cuBLAS for all of them).  A 32-bit result of bfloat16 operands (logits) comes straight from
     the skinny kernel's accumulators for those few rows; beyond that it is the vendor's bfloat16
