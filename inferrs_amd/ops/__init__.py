@@ -498,19 +498,24 @@ def attention_split(n_seqs: int, nkv: int, g: int, max_q_len: int, max_kv_len: i
             # walks are short, and where the blocks are few the kernel halves them instead (a portion of 512 tokens at
             # a context of 2,048, 32 query heads: 29.7 us whole in blocks of 64 columns against 36.8 in two splits)
             return 1, -(-max_kv_len // 64) * 64
-        # Full rounds of the compute units times a share's keys, in microseconds: a key takes a block of 128 columns 0.0183 alone
-        # on its unit and 0.02 on a full chip, one of 64 columns (which the kernel takes for few blocks that are not split)
-        # 0.0138; partial sums and their merge about 13 and 1 a split.  Measured, whole and in 2, 3 and 4 splits: 40 query heads,
-        # 512 tokens at 7,512 keys 138, 155, 117, 136; 300 tokens at 7,300 91, 79, 105, 90; 256 tokens at 12,256 144, 119, 90, 129;
-        # 32 query heads, 512 tokens at 8,012 117, 103, 130, 110; 256 tokens at 3,256 43, 43, 37, 33.
+        # In microseconds: whole, a key takes a block of 64 columns (which the kernel takes for few blocks that are not split)
+        # 0.0119 and one of 128 0.0172 a round of the compute units; in shares 0.0175, and a round's worth of partial sums 10.3 to
+        # write, read and merge; 2.5 % from the measurements in the mean.  Whole against 2, 3 and 4 shares, 40 query heads: 512 tokens
+        # at 6,000 keys 113, 128, 99 and 115, at 16,384 293, 304, 221 and 246; 1,024 tokens at 3,000 keys 98, 117, 117 and 128 (their
+        # early blocks walk less than the context: `max_q_len` / 2); 32 query heads, 256 tokens at 4,096 57, 56, 74 and 64; five query heads a
+        # key head, 32 tokens at 2,304 34, 32, 26 and 25.  Against powers of two up to one block a compute unit: 1.16 times as fast
+        # in the mean of 142 sizes at which the two differ, 0.95 (1.6 us) to 1.49.
         items = n_seqs * nkv * -(-cols // ATTN_TILE_COLS)
-        whole = 4.0 + 0.0138 * max_kv_len if 2 * items <= ATTN_TILE_BLOCKS else 8.0 + 0.0183 * max_kv_len * -(-items // ATTN_TILE_BLOCKS)
-        best, splits = whole, 1
-        for ways in range(2, 17):
+        if 2 * items <= ATTN_TILE_BLOCKS:
+            best = 6.0 + 0.0119 * max_kv_len
+        else:
+            best = 15.0 + 0.0172 * (max_kv_len - max_q_len // 2) * -(-items // ATTN_TILE_BLOCKS)
+        splits = 1
+        for ways in range(2, 129):
             chunk = -(-(-(-max_kv_len // ways)) // 64) * 64
             if chunk < ATTN_TILE_MIN_CHUNK:
                 break
-            cost = 21.0 + ways + 0.02 * chunk * -(-items * ways // ATTN_TILE_BLOCKS)
+            cost = 10.2 + 0.18 * ways + 10.3 * items * ways / ATTN_TILE_BLOCKS + 0.0175 * chunk * -(-items * ways // ATTN_TILE_BLOCKS)
             if cost < best:
                 best, splits = cost, ways
         chunk = -(-max_kv_len // splits)
