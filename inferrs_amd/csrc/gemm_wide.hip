@@ -300,6 +300,27 @@ extern "C" int ia_gemm_wide_splits(int M, int N, int K) {
     return wide_plan(M, N, K, false, true).splits;
 }
 
+// The share of full rounds of the compute units that blocks of 256 x 256, the vendor's largest, would make of a product.
+static double vendor_fill(int M, int N) {
+    const long long tiles = (long long)((M + 255) / 256) * ((N + 255) / 256), cus = wide_cus();
+    return (double)tiles / (double)((tiles + cus - 1) / cus * cus);
+}
+
+// Whether a product whose result may stay split goes here instead of to the vendor's GEMM, for the reader that adds it to the
+// residual stream and norms it.  Both sides measured with their readers in captured graphs (between single launches the vendor's
+// side waits for the host, which a graph does not) at 129 to 2,048 rows: the products of six dense shapes (27 counts of rows) and a
+// grid of 512 to 8,192 features by 512 to 16,384 k (20 counts).  The kernel gains by what the split gives, so it needs a long k
+// and enough features; short products are a few microseconds of fixed costs and the sums' way out and back in on top (us, the
+// vendor's side / this: 0.6B shape, 512 rows, o 14 / 17, down 17 / 20; 1.7B shape o 18 / 22, down 33 / 29; 4B shape, 144 rows, o 20 / 21;
+// 8B shape, 521 rows, o 42 / 35, down 109 / 66).  Where this rule says yes, no point of either set is below 0.97 of the vendor's
+// speed; 1.25 times as fast in the mean of the dense shapes' points.  Unsplit: where the vendor's blocks leave half of the chip
+// empty (14B shape, down at 1,536 rows, 367 / 243).
+extern "C" int ia_gemm_wide_norm_fits(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
+    if (gw_plan(M, N, K, false, true).splits == 1) return K >= 8192 && vendor_fill(M, N) < 0.5;
+    return K >= 4096 && N >= 1024 && (long long)K * (N < 3072 ? N : 3072) >= (M <= 256 ? 3072 : 2048) * 4096LL;
+}
+
 // Whether a [gate; up] of N features each goes here instead of to the vendor's GEMM and the activation's kernel: where this
 // kernel's own time comes within a tenth of 1.22 PFLOP/s (or of 4 TB/s over the operands) and what the second kernel takes.
 // Measured over the six dense shapes and 130 to 1,024 rows: 0.90 to 1.5 of the two kernels' time, 1.1 on average; beyond that the

@@ -1125,7 +1125,8 @@ def linear_partials(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tenso
     # (`own_rows`: outside such a step, the width of the rows themselves decides)
     if bias is None and isinstance(x, torch.Tensor) and x.shape[0] >= MID_MIN_ROWS and mid_fits(x, w, few_rows=not own_rows):
         return gemm_mid_bf16(x, w, partial=True)
-    if bias is None and isinstance(x, torch.Tensor) and wide_fits(x, w) and (not own_rows or x.shape[0] <= 1024):
+    if bias is None and isinstance(x, torch.Tensor) and wide_fits(x, w) and (
+            x.shape[0] <= 1024 if own_rows else library().ia_gemm_wide_norm_fits(x.shape[0], w.shape[0], x.shape[1])):
         return gemm_wide_bf16(x, w, partial=True)
     return None
 

@@ -1214,6 +1214,19 @@ def test_wide_product_in_every_block_shape(m, n, k):
         assert torch.equal(ours, theirs), ways
 
 
+@pytest.mark.parametrize("m,n,k,split", [(512, 1024, 2048, None), (512, 1024, 3072, None), (160, 2560, 4096, None), (521, 4096, 4096, True),
+                                         (160, 4096, 12288, True), (1536, 5120, 17408, False)])
+def test_product_ahead_of_the_streams_norm_takes_the_measured_route(m, n, k, split):
+    """`linear_partials` names the wide kernel's result, split or whole, where that was measured faster, and None where the vendor's
+    GEMM was (the caller then forms the whole product)."""
+    from inferrs_amd import ops
+    x, w = dev(randn(m, k, dtype=torch.bfloat16, seed=1)), dev(randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.05))
+    got = ops.linear_partials(x, w)
+    assert (got is None) == (split is None) and (split is None or isinstance(got, ops.Partials) == split)
+    if got is not None:
+        close(got.materialize() if split else got, x.double().cpu() @ w.double().cpu().t(), 2 ** -8, (m, n, k))
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 5, 4), (33, 64, 28), (161, 130, 36), (100, 259, 516), (320, 257, 132), (17, 16400, 100)])
 def test_32_bit_product_on_the_matrix_cores_has_the_bits_of_the_vector_units(m, n, k):
     """Every shape of block that exists (10 * rows of x + rows of w, in 16 and 64), at sizes that end inside tiles and chunks: the

@@ -51,3 +51,18 @@ def test_prompt_split_covers_the_context(d):
             assert chunk % 64 == 0, "the tiled kernel walks stages of 64 keys"
             if 2 * q > kv:
                 assert splits == 1, "portions that span most of their context keep their keys together"
+
+
+# Output features and k of the products of dense layers: width, feed-forward and query heads (of 128, beside 8 key heads).
+DENSE = {"0.6B": (1024, 3072, 16), "1.7B": (2048, 6144, 16), "4B": (2560, 9728, 32), "8B": (4096, 12288, 32), "14B": (5120, 17408, 40),
+         "32B": (5120, 25600, 64)}
+
+
+@pytest.mark.parametrize("shape,product,rows,own", [
+    # where both kernels were timed in captured graphs, the product with its reader, on either side of the rule
+    ("0.6B", "o", 512, False), ("0.6B", "down", 512, False), ("1.7B", "o", 384, False), ("1.7B", "down", 512, True), ("4B", "o", 144, False),
+    ("4B", "o", 420, True), ("8B", "o", 521, True), ("8B", "down", 200, True), ("14B", "down", 129, True), ("14B", "down", 1536, True),
+    ("32B", "o", 1024, True)])
+def test_products_behind_which_the_stream_is_normed_go_where_they_are_faster(shape, product, rows, own):
+    width, ff, heads = DENSE[shape]
+    assert bool(ops.library().ia_gemm_wide_norm_fits(rows, width, heads * 128 if product == "o" else ff)) == own
