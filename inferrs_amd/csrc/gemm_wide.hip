@@ -321,6 +321,17 @@ extern "C" int ia_gemm_wide_norm_fits(int M, int N, int K) {
     return K >= 4096 && N >= 1024 && (long long)K * (N < 3072 ? N : 3072) >= (M <= 256 ? 3072 : 2048) * 4096LL;
 }
 
+// The same for the kernel that norms and turns queries and keys and writes the cache (129 to 1,024 rows; six dense shapes, and 1,536
+// to 12,288 features by 512 to 8,192 k).  That reader takes the splits at the price of a stored product, and a product of q|k|v has
+// many features, so that the split gives less than above: unsplit, or over a short k, the vendor's GEMM is as fast or faster (us, the
+// vendor's side / this: 0.6B shape, 512 rows 17 / 20; 1.7B shape, 256 rows 18 / 24; 4B shape, 640 rows 38 / 39; 8B shape, 256 rows
+// 45 / 31, 456 rows 40 / 42; 14B shape, 521 rows 72 / 54).  Where this rule says yes, no point of the two sets is below 0.97 of the
+// vendor's speed (of 179 other sizes two, 0.95 and 0.96), 1.2 times as fast in the mean.
+extern "C" int ia_gemm_wide_rope_fits(int M, int N, int K) {
+    if (M <= 0 || M > 1024 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
+    return K >= 4096 && (K >= 5120 || M <= 384) && (long long)N * K >= 4096LL * 5120 && gw_plan(M, N, K, false, true).splits > 1;
+}
+
 // Whether a [gate; up] of N features each goes here instead of to the vendor's GEMM and the activation's kernel: where this
 // kernel's own time comes within a tenth of 1.22 PFLOP/s (or of 4 TB/s over the operands) and what the second kernel takes.
 // Measured over the six dense shapes and 130 to 1,024 rows: 0.90 to 1.5 of the two kernels' time, 1.1 on average; beyond that the

@@ -1117,17 +1117,18 @@ def gemm_wide_bf16(x: torch.Tensor, w: torch.Tensor, dual: bool = False, partial
 
 
 def linear_partials(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, own_rows: bool = False):
-    """x . w^T for a reader that takes `Partials` (the norm that adds the product to the stream): split along k where the
-    weight has few rows.  None when the product of 17 to 64 rows does not take these operands (a bias among them: the
-    caller then forms the whole product, and `linear` adds the bias)."""
-    # (whoever asks is in a step whose products go to gemm_mid.hip: the rule has been asked with the stream's width, and a
-    # product of another width follows it)
-    # (`own_rows`: outside such a step, the width of the rows themselves decides)
+    """x . w^T for a reader that takes `Partials`, split along k where the weight has few rows: the norm that adds the product to
+    the stream, or (`own_rows`) the kernel that norms and turns queries and keys.  None where `linear` is faster, or where
+    neither gemm_mid.hip (up to `MID_MAX_ROWS` rows) nor gemm_wide.hip (up to `WIDE_MAX_ROWS`) takes these operands, a bias among
+    them: the caller then forms the whole product, and `linear` adds the bias."""
+    # (up to MID_MAX_ROWS rows: who asks ahead of the norm is in a step whose products go to gemm_mid.hip, the rule has been asked with
+    # the stream's width, and a product of another width follows it; with `own_rows` the width of the rows themselves decides)
     if bias is None and isinstance(x, torch.Tensor) and x.shape[0] >= MID_MIN_ROWS and mid_fits(x, w, few_rows=not own_rows):
         return gemm_mid_bf16(x, w, partial=True)
-    if bias is None and isinstance(x, torch.Tensor) and wide_fits(x, w) and (
-            x.shape[0] <= 1024 if own_rows else library().ia_gemm_wide_norm_fits(x.shape[0], w.shape[0], x.shape[1])):
-        return gemm_wide_bf16(x, w, partial=True)
+    if bias is None and isinstance(x, torch.Tensor) and wide_fits(x, w):
+        lib = library()
+        if (lib.ia_gemm_wide_rope_fits if own_rows else lib.ia_gemm_wide_norm_fits)(x.shape[0], w.shape[0], x.shape[1]):
+            return gemm_wide_bf16(x, w, partial=True)
     return None
 
 

@@ -1227,6 +1227,18 @@ def test_product_ahead_of_the_streams_norm_takes_the_measured_route(m, n, k, spl
         close(got.materialize() if split else got, x.double().cpu() @ w.double().cpu().t(), 2 ** -8, (m, n, k))
 
 
+@pytest.mark.parametrize("m,n,k,split", [(512, 4096, 1024, False), (256, 4096, 2048, False), (456, 6144, 4096, False), (256, 6144, 4096, True),
+                                         (521, 7168, 5120, True), (100, 4096, 1024, True)])
+def test_product_ahead_of_the_rotation_takes_the_measured_route(m, n, k, split):
+    """Queries, keys and values: split where that was measured faster, else None (the vendor's GEMM)."""
+    from inferrs_amd import ops
+    x, w = dev(randn(m, k, dtype=torch.bfloat16, seed=1)), dev(randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.05))
+    got = ops.linear_partials(x, w, own_rows=True)
+    assert (got is not None) == split
+    if split and m > ops.MID_MAX_ROWS:
+        close(got.materialize(), x.double().cpu() @ w.double().cpu().t(), 2 ** -8, (m, n, k))
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 5, 4), (33, 64, 28), (161, 130, 36), (100, 259, 516), (320, 257, 132), (17, 16400, 100)])
 def test_32_bit_product_on_the_matrix_cores_has_the_bits_of_the_vector_units(m, n, k):
     """Every shape of block that exists (10 * rows of x + rows of w, in 16 and 64), at sizes that end inside tiles and chunks: the

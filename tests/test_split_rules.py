@@ -66,3 +66,10 @@ DENSE = {"0.6B": (1024, 3072, 16), "1.7B": (2048, 6144, 16), "4B": (2560, 9728, 
 def test_products_behind_which_the_stream_is_normed_go_where_they_are_faster(shape, product, rows, own):
     width, ff, heads = DENSE[shape]
     assert bool(ops.library().ia_gemm_wide_norm_fits(rows, width, heads * 128 if product == "o" else ff)) == own
+
+
+@pytest.mark.parametrize("shape,rows,own", [("0.6B", 512, False), ("1.7B", 256, False), ("4B", 320, False), ("4B", 640, False), ("8B", 160, True),
+                                            ("8B", 256, True), ("8B", 456, False), ("14B", 521, True), ("14B", 900, False), ("32B", 456, True)])
+def test_products_of_queries_and_keys_go_where_they_are_faster(shape, rows, own):
+    width, _, heads = DENSE[shape]
+    assert bool(ops.library().ia_gemm_wide_rope_fits(rows, (heads + 16) * 128, width)) == own
