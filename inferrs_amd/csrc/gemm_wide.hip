@@ -332,14 +332,21 @@ extern "C" int ia_gemm_wide_rope_fits(int M, int N, int K) {
     return K >= 4096 && (K >= 5120 || M <= 384) && (long long)N * K >= 4096LL * 5120 && gw_plan(M, N, K, false, true).splits > 1;
 }
 
-// Whether a [gate; up] of N features each goes here instead of to the vendor's GEMM and the activation's kernel: where this
-// kernel's own time comes within a tenth of 1.22 PFLOP/s (or of 4 TB/s over the operands) and what the second kernel takes.
-// Measured over the six dense shapes and 130 to 1,024 rows: 0.90 to 1.5 of the two kernels' time, 1.1 on average; beyond that the
-// vendor's blocks of 256 x 256 are as fast or faster (8B shape, 2,048 rows: 316 against 353 us).
+// Whether a [gate; up] of N features each goes here instead of to the vendor's GEMM and the activation's kernel.  The product cannot
+// be split, so the kernel gains where its own blocks fill their rounds (its time within 0.9 of 1.22 PFLOP/s, or of 4 TB/s over the
+// operands, and what the second kernel takes; all of it for a short k under few features) and the vendor's blocks of 256 x 256 do
+// not, or, with many rows and features, where the vendor's last round is half empty.  Measured in captured graphs at 129 to 1,024 rows, the six dense shapes and 1,024 to
+// 25,600 features by 512 to 8,192 k, and 400 other sizes: where this rule says yes no point is below 0.97 of the two kernels'
+// speed, 1.2 times as fast in the mean (us, the two kernels / this: 1.7B shape, 512 rows 36 / 35; 8B shape, 320 rows 81 / 77, 456 rows
+// 101 / 108, 512 rows 102 / 124; 14B shape, 160 rows 107 / 115, 521 rows 201 / 208, 900 rows 404 / 300; 4B shape, 768 rows 82 / 102,
+// 900 rows 114 / 107).
 extern "C" int ia_gemm_wide_dual_fits(int M, int N, int K) {
-    if (M <= 0 || M > 1024 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4 || ((long long)N + GW_BN) * K * 2 >= (1LL << 32)) return 0;
+    if (M < 300 || M > 1024 || N < 2048 || K <= 0 || K % GW_STAGE_K || N % 4 || ((long long)N + GW_BN) * K * 2 >= (1LL << 32)) return 0;
+    const double theirs = vendor_fill(M, 2 * N);
+    if (M >= 800 && N >= 8192 && theirs <= 0.72) return 1;
     const double flops = 4.0 * M * N * K / 1.22e9, bytes = (2.0 * N + M) * K * 2.0 / 4.0e6;
-    return gw_plan(M, N, K, true, false).cost <= 1.1 * ((flops > bytes ? flops : bytes) + 8.0 + M * (double)N * 6.0 / 5.0e6);
+    const double limit = M >= 512 && K <= 2048 && N <= 6144 ? 1.0 : theirs <= 0.6 ? 0.9 : 0.0;
+    return gw_plan(M, N, K, true, false).cost <= limit * ((flops > bytes ? flops : bytes) + 8.0 + M * (double)N * 6.0 / 5.0e6);
 }
 
 // out_mode 0: out [M, N] bfloat16; 1: float; 2: [splits][M][N] float with splits = ia_gemm_wide_splits(M, N, K).  dual (an

@@ -1239,6 +1239,21 @@ def test_product_ahead_of_the_rotation_takes_the_measured_route(m, n, k, split):
         close(got.materialize(), x.double().cpu() @ w.double().cpu().t(), 2 ** -8, (m, n, k))
 
 
+@pytest.mark.parametrize("m,n,k", [(512, 12288, 4096), (700, 3072, 1024), (900, 9728, 2560)])
+def test_gate_and_up_on_either_route(m, n, k):
+    """Both sides of the rule give the product with its activation: a route that the vendor's GEMM takes, and two of the wide kernel."""
+    from inferrs_amd import ops
+    x, w = dev(randn(m, k, dtype=torch.bfloat16, seed=1)), dev(randn(2 * n, k, dtype=torch.bfloat16, seed=2, scale=0.05))
+    own = n != 12288
+    assert bool(ops.library().ia_gemm_wide_dual_fits(m, n, k)) == own
+    got = ops.gated_linear(x, w)
+    if own:
+        assert torch.equal(got, ops.gemm_wide_bf16(x, w, dual=True))
+    rows = slice(m - 40, m)                                    # (the tile that ends inside the matrix)
+    gate, up = (x[rows].float().cpu() @ w.float().cpu().t()).split(n, dim=1)
+    close(got[rows], torch.nn.functional.silu(gate) * up, 3 * 2 ** -8, (m, n, k))
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 5, 4), (33, 64, 28), (161, 130, 36), (100, 259, 516), (320, 257, 132), (17, 16400, 100)])
 def test_32_bit_product_on_the_matrix_cores_has_the_bits_of_the_vector_units(m, n, k):
     """Every shape of block that exists (10 * rows of x + rows of w, in 16 and 64), at sizes that end inside tiles and chunks: the

@@ -73,3 +73,17 @@ def test_products_behind_which_the_stream_is_normed_go_where_they_are_faster(sha
 def test_products_of_queries_and_keys_go_where_they_are_faster(shape, rows, own):
     width, _, heads = DENSE[shape]
     assert bool(ops.library().ia_gemm_wide_rope_fits(rows, (heads + 16) * 128, width)) == own
+
+
+@pytest.mark.parametrize("shape,rows,own", [("0.6B", 129, False), ("0.6B", 700, True), ("4B", 160, False), ("4B", 768, False), ("4B", 900, True), ("8B", 129, False), ("8B", 456, False),
+                                            ("8B", 512, False), ("14B", 200, False), ("14B", 521, False), ("14B", 832, True), ("14B", 1024, True)])
+def test_gate_and_up_go_where_they_are_faster(shape, rows, own):
+    width, ff, _ = DENSE[shape]
+    assert bool(ops.library().ia_gemm_wide_dual_fits(rows, ff, width)) == own
+
+
+def test_the_wide_kernels_rules_refuse_what_the_kernel_does_not_take():
+    lib = ops.library()
+    for fits in (lib.ia_gemm_wide_norm_fits, lib.ia_gemm_wide_rope_fits, lib.ia_gemm_wide_dual_fits):
+        for m, n, k in ((0, 4096, 8192), (512, 0, 8192), (512, 4096, 0), (900, 8192, 8200), (900, 8194, 8192), (-5, -4, -64)):
+            assert fits(m, n, k) == 0
