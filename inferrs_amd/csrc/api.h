@@ -72,10 +72,12 @@ int ia_qk_rope_kv_partials(void* q_out, void* k_cache, void* v_cache, const floa
 int ia_qk_rope_kv_partials_fits(int n, int d, int rot, int interleaved, int page_size);
 int ia_gemm_tiled(void* out, const void* x, const void* w, int M, int N, int K, int in_dtype,
                   int out_dtype, hipStream_t stream);
-// (what ia_gemm_tiled runs for many rows of the 32-bit path: K a multiple of 4, x and w 16-byte aligned; `shape`
+// (what ia_gemm_tiled runs for more than a few rows of the 32-bit path: K a multiple of 4, x and w 16-byte aligned; `shape`
 // forces a block of 16 * (shape / 10) rows of x by 64 * (shape % 10) of w, 0: the kernel's own rule)
 int ia_gemm_f32(void* out, const void* x, const void* w, int M, int N, int K, hipStream_t stream);
 int ia_gemm_f32_tune(int shape);
+// (whether ia_gemm_tiled runs it, for 32-bit operands and results that are 16-byte aligned)
+int ia_gemm_f32_fits(int M, int N, int K);
 // bias: bfloat16 [N] ([2 N] with dual), or null
 // (ia_gemm_tiled at up to 64 rows: the shape of its kernel for few rows, 100 * output features + staged rows a wave:
 // 816, 808, 416 or 1608; 0: the kernel's own rule)

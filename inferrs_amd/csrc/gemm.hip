@@ -252,17 +252,25 @@ static void launch_rows(void* o, const void* xi, const void* w, int rows, int N,
     }
 }
 
+// Whether a 32-bit product goes to the matrix cores (gemm_f32.hip).  Up to 16 rows the kernel above reads the weights faster,
+// or as fast; at 9 to 16 rows it reads every weight for twice the arithmetic, and from 64 features a compute unit on the matrix
+// cores are faster.  Weights not in a cache, in graphs, us, the kernel above / the matrix cores: 8 rows, 4,096 k, 24,576 features 90 / 128,
+// 128,256 398 / 445, 151,936 470 / 474, 1,024 k, 151,936 135 / 145; 16 rows, 4,096 k, 16,384 features 118 / 59, 24,576 147 / 127, 151,936
+// 790 / 474.  (Weights that a cache holds, 4,096 k: 16 rows, 6,144 features 51 / 66; 32 rows 99 / 46, 24,576 717 / 133; 128 rows 554 /
+// 104, 993 / 238.)
+extern "C" int ia_gemm_f32_fits(int M, int N, int K) {
+    return M > 8 && N > 0 && K > 0 && K % 4 == 0 && (M > GR_ROWS || N >= 64 * skinny_cus());
+}
+
 // in_dtype: storage of x and w; out_dtype: storage of the result.
 extern "C" int ia_gemm_tiled(void* out, const void* x, const void* w, int M, int N, int K,
                              int in_dtype, int out_dtype, hipStream_t stream) {
     IA_CHECK(M >= 0 && N > 0 && K > 0, "gemm_tiled: bad sizes M=%d N=%d K=%d", M, N, K);
     if (M == 0) return 0;
     const size_t elem = in_dtype == IA_F32 ? 4 : 2;
-    // The 32-bit path on the matrix cores: the same bits.  Up to 16 rows the kernel below reads the weights faster, unless
-    // they have very many rows.  (4,096 k, us, the vector units' kernels against it: 8 rows 6,144 features 42 / 66, 24,576 87 /
-    // 120, 151,936 556 / 464; 16 rows 51 / 66, 147 / 118, 901 / 479; 32 rows 99 / 46, 717 / 133; 128 rows 554 / 104, 993 / 238.)
-    if (in_dtype == IA_F32 && out_dtype == IA_F32 && K % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 &&
-        (M > GR_ROWS || N >= (M > 8 ? 64 : 256) * skinny_cus()) && (g_rows_shape == 0 || M > GR_ROWS))
+    // the 32-bit path on the matrix cores: the same bits
+    if (in_dtype == IA_F32 && out_dtype == IA_F32 && ia_gemm_f32_fits(M, N, K) && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 &&
+        (g_rows_shape == 0 || M > GR_ROWS))
         return ia_gemm_f32(out, x, w, M, N, K, stream);
     // up to 64 rows, 16 at a time, where the tiles of 64 x 64 would be few (the weights are read once for every 16 rows)
     if (M <= 4 * GR_ROWS && (M <= GR_ROWS || N <= 4096 * 4) && K % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) % (4 * elem)) == 0) {

@@ -87,3 +87,10 @@ def test_the_wide_kernels_rules_refuse_what_the_kernel_does_not_take():
     for fits in (lib.ia_gemm_wide_norm_fits, lib.ia_gemm_wide_rope_fits, lib.ia_gemm_wide_dual_fits):
         for m, n, k in ((0, 4096, 8192), (512, 0, 8192), (512, 4096, 0), (900, 8192, 8200), (900, 8194, 8192), (-5, -4, -64)):
             assert fits(m, n, k) == 0
+
+
+def test_32_bit_products_of_up_to_8_rows_stay_on_the_vector_units():
+    fits = ops.library().ia_gemm_f32_fits
+    for n, k in ((6144, 4096), (24576, 4096), (65536, 2048), (128256, 4096), (151936, 1024), (151936, 4096), (262144, 2560)):
+        assert not any(fits(m, n, k) for m in range(0, 9))
+        assert all(fits(m, n, k) == (n >= 16384) for m in range(9, 17)) and fits(17, n, k) and not fits(17, n, k + 2)
