@@ -301,6 +301,8 @@ int ia_linear_scan(float* out, float* den, float* state, long long row_floats, l
                    const int* cu_tokens, const int* state_slots, int n_seqs, int H, int dim, int vdim,
                    float q_scale, float k_scale, int act, int chunk, int max_q_len, float* workspace, int dtype,
                    hipStream_t stream);
+// (value columns a block takes of `units` (chunk, head) pairs with vt columns, a rule of ia_linear_scan's)
+int ia_linear_scan_columns(long long units, int vt, int dim);
 long long ia_linear_scan_workspace(int n_seqs, int max_q_len, int chunk, int H, int dim, int vdim, int normaliser);
 // 1 (the default): what a chunk's start contributes is formed on the matrix cores in true 32-bit (keys up to 128, chunks up
 // to 64 tokens); 0: on the vector units

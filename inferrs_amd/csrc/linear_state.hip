@@ -777,9 +777,6 @@ extern "C" long long ia_linear_scan_workspace(int n_seqs, int max_q_len, int chu
     return (long long)n_seqs * max_chunks * ((long long)H * (vdim + (normaliser ? 1 : 0)) * dim + H);
 }
 
-// chunk 0: every request's tokens are walked from its state row.  chunk > 0: portions are cut into chunks of that many
-// tokens that run side by side; `workspace` holds ia_linear_scan_workspace(...) floats and max_q_len is an upper bound
-// of the tokens a request brings.
 static int linear_cus() {
     static int cus = 0;
     if (cus == 0) {
@@ -789,6 +786,29 @@ static int linear_cus() {
     return cus;
 }
 
+// Shared memory of a block of linear_local_mfma_kernel.
+static int linear_local_bytes(int dim) {
+    const int ld_s = (dim + 3) / 4 * 4 + 4;
+    return (int)((2 * LC_TOKENS * ld_s + LC_TOKENS * ((ld_s >= LL_P_LD ? 0 : LL_P_LD) + LL_V_LD) + 3 * LC_TOKENS) * sizeof(float));
+}
+
+// Columns of a block of linear_local_mfma_kernel for `units` (chunk, head) pairs with vt columns: all of them, or fewer (in steps of
+// 32), each share with scores of its own, as long as every block is on the chip at once (shared memory and, at four, registers).
+// A share more than that is a second round.  The three kernels in graphs, us, whole columns / shared out so / up to two blocks a compute
+// unit whatever fits: 64 heads of 128 x 64, 300 tokens 51 / 51 / 61; 16 of 128 x 256, 700 tokens 100 / 81 / 97, 1,500 tokens 140 / 141 /
+// 151; 16 of 64 x 128, 1,500 tokens 65 / 58 / 58; 8 of 128 x 256 with a normaliser, 1,500 tokens 113 / 97 / 110; 99 sizes 1.15 times as
+// fast as whole columns, none slower than 0.99.
+extern "C" int ia_linear_scan_columns(long long units, int vt, int dim) {
+    const int steps = (vt + 31) / 32, on_a_unit = 160 * 1024 / linear_local_bytes(dim);
+    const long long at_once = (long long)linear_cus() * (on_a_unit < 1 ? 1 : on_a_unit > 4 ? 4 : on_a_unit);
+    int shares = 1;
+    while (shares < steps && (shares + 1) * units <= at_once) ++shares;
+    return (steps + shares - 1) / shares * 32;
+}
+
+// chunk 0: every request's tokens are walked from its state row.  chunk > 0: portions are cut into chunks of that many
+// tokens that run side by side; `workspace` holds ia_linear_scan_workspace(...) floats and max_q_len is an upper bound
+// of the tokens a request brings.
 extern "C" int ia_linear_scan(float* out, float* den, float* state, long long row_floats, long long s_off,
                               const void* q, long long q_ld, int q_off, int q_heads,
                               const void* k, long long k_ld, int k_off, int k_heads,
@@ -867,15 +887,9 @@ extern "C" int ia_linear_scan(float* out, float* den, float* state, long long ro
     const bool cores = g_carry_mfma && dim <= LC_MAX_DIM && chunk <= LC_TOKENS;
     if (cores) {
         const int ld_s = (dim + 3) / 4 * 4 + 4;
-        // Columns a block: all of them, or fewer (in steps of 32), each share with scores of its own, until the step has two
-        // blocks for every compute unit (24 chunks of 8 heads with values of 256 and a normaliser: nine steps of columns in 192
-        // blocks 74 us, shared out 71; 16 heads of 128 in 384 blocks 38, in 768 29).
-        const int steps = (vt + 31) / 32;
-        int shares = 1;
-        while (shares < steps && (long long)shares * H * n_seqs * a.max_chunks < 2 * linear_cus()) ++shares;
-        const int cols = (steps + shares - 1) / shares * 32;
+        const int cols = ia_linear_scan_columns((long long)H * n_seqs * a.max_chunks, vt, dim);
         const dim3 lgrid((unsigned)((vt + cols - 1) / cols), (unsigned)H, (unsigned)(n_seqs * a.max_chunks));
-        const int lshm = (int)((2 * LC_TOKENS * ld_s + LC_TOKENS * ((ld_s >= LL_P_LD ? 0 : LL_P_LD) + LL_V_LD) + 3 * LC_TOKENS) * sizeof(float));
+        const int lshm = linear_local_bytes(dim);
         static int asked_f32 = 0, asked_bf16 = 0;          // shared memory beyond 64 KiB has to be asked for, once per instantiation
         int& asked = dtype == IA_F32 ? asked_f32 : asked_bf16;
         if (lshm > asked) {

@@ -101,3 +101,16 @@ def test_a_logits_head_has_blocks_of_eight_waves_over_a_long_k_only(n, k, eight)
     """(`fills`: whether the plan's blocks are three stages deep, as those of eight waves are and the general ones are not)"""
     lib = ops.library()
     assert bool(lib.ia_gemm_mid_fills(n, k, 0)) == eight and lib.ia_gemm_mid_splits(n, k) == 1
+
+
+def test_a_chunks_columns_are_shared_out_within_one_round_of_the_chip():
+    """A chunk's block brings keys and queries of 64 tokens into shared memory: a compute unit holds two such blocks at 128 entries a
+    key, three at 64, four (by their registers) at 32."""
+    columns = ops.library().ia_linear_scan_columns
+    for dim, at_once in ((128, 512), (96, 512), (64, 768), (32, 1024), (16, 1024)):
+        for units, vt in itertools.product((1, 5, 100, 192, 255, 256, 257, 288, 320, 352, 384, 512, 513, 4000), (1, 32, 33, 64, 128, 161, 257)):
+            cols = columns(units, vt, dim)
+            shares = -(-vt // cols)
+            assert cols >= 32 and cols % 32 == 0 and (shares == 1 or shares * units <= at_once), (dim, units, vt, cols)
+    # (64 heads x 5 chunks, 32 x 11: two shares each would be a second round; 8 heads x 24 chunks: two shares, not three)
+    assert columns(320, 64, 128) == 64 and columns(352, 64, 128) == 64 and columns(192, 257, 128) == 160 and columns(384, 128, 64) == 64
