@@ -239,6 +239,19 @@ class Engine:
         bucket_pages = max(1, self.GRAPH_BUCKET_TOKENS // self.page_size)
         return -(-(-(-longest // self.page_size)) // bucket_pages) * bucket_pages
 
+    @staticmethod
+    def _run_bound(longest: int, bucket_tokens: int, widest: int, least: int = 1) -> int:
+        """The tokens that bound one run's launches in a step of portions beside single tokens whose longer run is bounded by
+        `widest`: the run's bucket (`least` buckets or more), beyond eight buckets rounded up to one of four sizes between powers of
+        two.  Every pair of bounds is a graph of its own, met twice before it is captured: a prompt of 40,960 tokens beside contexts as
+        long meets 16, not 40, of the `MAX_GRAPHS` that decode steps share.  (ms a prompt, one bound for both runs / a bound a run:
+        0.6B shape, portions of 256 of 8,192 tokens beside 8 contexts of 9,000 164 / 154 with 1 / 7 graphs, of 24,576 beside 4 of 30,000
+        695 / 610; 12 layers of the 8B shape 136 / 128 and 545 / 476.  The captures fall to the first prompt: 0.6B shape, portions of 128
+        of 4,096 beside 4 contexts of 3,000, 112 / 128, from then on 102 / 100.)"""
+        buckets = max(least, -(-longest // bucket_tokens))
+        step = 1 << max(0, (buckets - 1).bit_length() - 3)
+        return min(-(-buckets // step) * step * bucket_tokens, widest)
+
     def chain_ready(self, seq_ids: Sequence[Hashable], steps: int) -> bool:
         """Whether `decode_chain` can run these requests for `steps` steps: their shape has a
         captured graph whose context bucket holds them to the end."""
@@ -346,12 +359,15 @@ class Engine:
         self._drop_stale_graphs()                       # (the buffer may have moved in this very build)
         key = (ctx.n_seqs, ctx.n_tokens, ctx.n_single, int(ctx.want_rows.shape[0]), ctx.max_q_len, pad_pages)
         if 0 < ctx.n_single < ctx.n_seqs:
-            # (portions beside single tokens: each run's launches follow from its own longest context, in buckets of their own.
-            # 512 tokens behind 1,500 beside contexts of 3,100: bounded by those, the portion's keys were split in two at 2,048,
-            # the second half empty, 82 us a layer at 40 query heads against 48)
-            bounds = self._bucket_pages(longest_single), self._bucket_pages(longest_multi)
-            ctx.max_kv_single, ctx.max_kv_multi = (pages * self.page_size for pages in bounds)
-            key += bounds
+            # (portions beside single tokens: each run's launches follow from its own longest context.  512 tokens behind 1,500
+            # beside contexts of 3,100: bounded by those, the portion's keys were split in two at 2,048, the second half empty,
+            # 82 us a layer at 40 query heads against 48)
+            widest = pad_pages * self.page_size
+            bucket = max(1, self.GRAPH_BUCKET_TOKENS // self.page_size) * self.page_size
+            # (a portion's keys are not split at up to 2,048: its first two buckets have the same launches)
+            ctx.max_kv_single = self._run_bound(longest_single, bucket, widest)
+            ctx.max_kv_multi = self._run_bound(longest_multi, bucket, widest, least=2)
+            key += (ctx.max_kv_single, ctx.max_kv_multi)
         entry = self._graphs.get(key)
         if entry is not None:
             self._graphs.move_to_end(key)

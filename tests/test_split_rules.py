@@ -114,3 +114,20 @@ def test_a_chunks_columns_are_shared_out_within_one_round_of_the_chip():
             assert cols >= 32 and cols % 32 == 0 and (shares == 1 or shares * units <= at_once), (dim, units, vt, cols)
     # (64 heads x 5 chunks, 32 x 11: two shares each would be a second round; 8 heads x 24 chunks: two shares, not three)
     assert columns(320, 64, 128) == 64 and columns(352, 64, 128) == 64 and columns(192, 257, 128) == 160 and columns(384, 128, 64) == 64
+
+
+def test_bounds_of_mixed_steps_are_few_and_close():
+    """A step of portions beside single tokens is captured once a pair of bounds: what bounds a run covers it, exceeds its bucket by a
+    quarter at most (from eight buckets on), never exceeds the longer run's, and takes few values over a long prompt."""
+    from inferrs_amd.engine import Engine
+    bucket, widest = Engine.GRAPH_BUCKET_TOKENS, 40 * Engine.GRAPH_BUCKET_TOKENS
+    for least, most in ((1, 17), (2, 16)):
+        bounds = [Engine._run_bound(n, bucket, widest, least) for n in range(1, widest + 1)]
+        for n, b in enumerate(bounds, 1):
+            buckets = max(least, -(-n // bucket))
+            assert n <= b <= widest and b % bucket == 0 and b // bucket <= buckets * 1.25
+            assert buckets > 8 or b == buckets * bucket
+        assert bounds == sorted(bounds) and len(set(bounds)) <= most
+    assert Engine._run_bound(100, 1024, 1024, 2) == 1024 and Engine._run_bound(9000, 1024, 9 * 1024) == 9 * 1024
+    # a portion of up to 2,048 tokens of context beside anything: one graph
+    assert len({Engine._run_bound(n, bucket, widest, 2) for n in range(1, 2049)}) == 1
