@@ -322,8 +322,11 @@ def qk_rope_kv(qkv: torch.Tensor, nq: int, nkv: int, d: int, *,
     parts = None
     if isinstance(qkv, Partials):
         splits, n, width = qkv.parts.shape
+        # (that kernel reads everything in 16-byte pieces; arrays that begin elsewhere go with the stored product)
+        arrays = (q_norm_w, k_norm_w, cos, sin, k_cache, v_cache, qkv.parts)
         if (cos is None or slots is None or k_cache is None or k_cache.dtype != torch.bfloat16 or width != (nq + 2 * nkv) * d
-                or not qk_rope_kv_partials_fits(n, d, rot, interleaved, page_size)):
+                or not qk_rope_kv_partials_fits(n, d, rot, interleaved, page_size)
+                or any(t is not None and t.data_ptr() % 16 for t in arrays)):
             qkv = qkv.materialize()
         else:
             parts, qkv = qkv.parts, qkv.parts[0]

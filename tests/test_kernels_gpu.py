@@ -221,6 +221,30 @@ def test_qk_rope_kv_of_a_product_still_split(n, nq, nkv, d, page, splits):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("which", ["q_norm_w", "k_norm_w", "cos", "sin"])
+def test_qk_rope_kv_of_a_split_product_beside_unaligned_arrays(which):
+    """A norm's weight or a rotation's table that does not begin at a multiple of 16 bytes: taken, as beside a stored product."""
+    from inferrs_amd import ops
+    n, nq, nkv, d, page = 40, 4, 2, 128, 16
+    g = torch.Generator().manual_seed(7)
+    split = ops.Partials(dev(randn(2, n, (nq + 2 * nkv) * d, dtype=torch.float32, seed=9)))
+    arrays = {"q_norm_w": randn(d, dtype=torch.float32, seed=1), "k_norm_w": randn(d, dtype=torch.float32, seed=2),
+              "cos": torch.rand(n, d // 2, generator=g), "sin": torch.rand(n, d // 2, generator=g)}
+    arrays = {k: dev(v) for k, v in arrays.items()}
+    off = torch.empty(arrays[which].numel() + 1, device="cuda")
+    off[1:] = arrays[which].view(-1)
+    arrays[which] = off[1:].view(arrays[which].shape)
+    slots = dev(torch.arange(n, dtype=torch.int32))
+    got = []
+    for rows in (split, split.materialize()):
+        kc, vc = (torch.zeros(shape, dtype=torch.bfloat16, device="cuda") for shape in ((4, nkv, page, d), (4, nkv, d, page)))
+        q = ops.qk_rope_kv(rows, nq, nkv, d, eps=1e-6, add_one=False, rot=d, interleaved=False, k_cache=kc, v_cache=vc, slots=slots,
+                           page_size=page, **arrays)
+        got.append((q, kc, vc))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 def ref_attention(q, kc, vc, positions, token_seq, table, window, scale):
     n, nq, d = q.shape
     nkv, page = kc.shape[1], kc.shape[2]
