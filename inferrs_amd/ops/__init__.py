@@ -1143,7 +1143,7 @@ def add_rmsnorm_partials(x: torch.Tensor, delta: Partials, w: torch.Tensor, eps:
     splits, rows, cols = parts.shape
     if x.dtype != torch.bfloat16 or tuple(x.shape) != (rows, cols) or w.numel() != cols:
         raise KernelError(f"add_rmsnorm_partials: x {tuple(x.shape)} {x.dtype} does not fit the product {tuple(parts.shape)}")
-    if cols % 4 or cols > 8192:
+    if cols % 4 or cols > 8192 or (x.data_ptr() | parts.data_ptr() | w.data_ptr()) % 16:
         return add_rmsnorm(x, delta.materialize(), w, eps, add_one)
     out = torch.empty_like(x)
     _check(library().ia_add_rmsnorm_partials(_p(out), _p(x), _p(parts), splits, _p(w), ctypes.c_float(eps), rows, cols,

@@ -245,6 +245,19 @@ def test_qk_rope_kv_of_a_split_product_beside_unaligned_arrays(which):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("which", ["stream", "weight"])
+def test_a_split_product_added_to_an_unaligned_stream_or_beside_an_unaligned_weight(which):
+    """Rows or a norm's weight that do not begin at a multiple of 16 bytes: taken, as beside a stored product."""
+    from inferrs_amd import ops
+    m, n = 150, 256
+    parts = ops.Partials(dev(randn(3, m, n, dtype=torch.float32, seed=1)))
+    w, x = dev(randn(n + 1, dtype=torch.float32, seed=2)), dev(randn(m * n + 1, dtype=torch.bfloat16, seed=3))
+    w = w[1:] if which == "weight" else w[:n]
+    rows = [(x.clone()[1:] if which == "stream" else x.clone()[:-1]).view(m, n) for _ in range(2)]
+    got = ops.add_rmsnorm_partials(rows[0], parts, w, 1e-6)
+    assert torch.equal(got, ops.add_rmsnorm(rows[1], parts.materialize(), w, 1e-6)) and torch.equal(*rows)
+
+
 def ref_attention(q, kc, vc, positions, token_seq, table, window, scale):
     n, nq, d = q.shape
     nkv, page = kc.shape[1], kc.shape[2]
