@@ -308,44 +308,46 @@ static double vendor_fill(int M, int N) {
 
 // Whether a product whose result may stay split goes here instead of to the vendor's GEMM, for the reader that adds it to the
 // residual stream and norms it.  Both sides measured with their readers in captured graphs (between single launches the vendor's
-// side waits for the host, which a graph does not) at 129 to 2,048 rows: the products of six dense shapes (27 counts of rows) and a
-// grid of 512 to 8,192 features by 512 to 16,384 k (20 counts).  The kernel gains by what the split gives, so it needs a long k
-// and enough features; short products are a few microseconds of fixed costs and the sums' way out and back in on top (us, the
-// vendor's side / this: 0.6B shape, 512 rows, o 14 / 17, down 17 / 20; 1.7B shape o 18 / 22, down 33 / 29; 4B shape, 144 rows, o 20 / 21;
-// 8B shape, 521 rows, o 42 / 35, down 109 / 66).  Where this rule says yes, no point of either set is below 0.97 of the vendor's
-// speed; 1.25 times as fast in the mean of the dense shapes' points.  Unsplit: where the vendor's blocks leave half of the chip
-// empty (14B shape, down at 1,536 rows, 367 / 243).
+// side waits for the host, which a graph does not) at 129 to 2,048 rows: the products of six dense shapes (27 counts of rows), a
+// grid of 512 to 8,192 features by 512 to 16,384 k (20 counts), and 458 sizes drawn where the rule says yes.  The kernel gains by what
+// the split gives, so it needs a long k and enough features; short products are a few microseconds of fixed costs and the sums' way
+// out and back in on top (us, the vendor's side / this: 0.6B shape, 512 rows, o 14 / 17, down 17 / 20; 1.7B shape o 18 / 22, down 33 /
+// 29; 4B shape, 144 rows, o 20 / 21; 8B shape, 521 rows, o 42 / 35, down 109 / 66).  Unsplit: where the vendor's blocks leave a third
+// of the chip empty (14B shape, down at 1,536 rows, 367 / 243).  Of the 1,729 points where this rule says yes four are below 0.97 of
+// the vendor's speed, 0.90 to 0.96, all of them unsplit; 1.26 times as fast over all of the dense shapes' points.
 extern "C" int ia_gemm_wide_norm_fits(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
-    if (gw_plan(M, N, K, false, true).splits == 1) return K >= 8192 && vendor_fill(M, N) < 0.5;
-    return K >= 4096 && N >= 1024 && (long long)K * (N < 3072 ? N : 3072) >= (M <= 256 ? 3072 : 2048) * 4096LL;
+    if (gw_plan(M, N, K, false, true).splits == 1) return K >= 8192 && vendor_fill(M, N) < 0.63;
+    return K >= 4096 && N >= 1024 && (long long)K * (N < 3072 ? N : 3072) >= (M <= 192 ? 3072 : M <= 256 ? 2560 : 2048) * 4096LL;
 }
 
-// The same for the kernel that norms and turns queries and keys and writes the cache (129 to 1,024 rows; six dense shapes, and 1,536
-// to 12,288 features by 512 to 8,192 k).  That reader takes the splits at the price of a stored product, and a product of q|k|v has
-// many features, so that the split gives less than above: unsplit, or over a short k, the vendor's GEMM is as fast or faster (us, the
-// vendor's side / this: 0.6B shape, 512 rows 17 / 20; 1.7B shape, 256 rows 18 / 24; 4B shape, 640 rows 38 / 39; 8B shape, 256 rows
-// 45 / 31, 456 rows 40 / 42; 14B shape, 521 rows 72 / 54).  Where this rule says yes, no point of the two sets is below 0.97 of the
-// vendor's speed (of 179 other sizes two, 0.95 and 0.96), 1.2 times as fast in the mean.
+// The same for the kernel that norms and turns queries and keys and writes the cache (129 to 1,024 rows; six dense shapes, 1,536 to
+// 12,288 features by 512 to 8,192 k, and 239 drawn sizes).  That reader takes the splits at the price of a stored product, and a
+// product of q|k|v has many features, so that the split gives less than above: unsplit, or over a short k, the vendor's GEMM is as
+// fast or faster (us, the vendor's side / this: 0.6B shape, 512 rows 17 / 20; 1.7B shape, 256 rows 18 / 24; 4B shape, 640 rows 38 / 39;
+// 8B shape, 256 rows 45 / 31, 456 rows 40 / 42, 700 rows 58 / 49; 14B shape, 521 rows 72 / 54).  Of the 599 points where this rule says
+// yes two are below 0.97 of the vendor's speed (0.95 and 0.96), 1.2 times as fast in the mean.  (The vendor's GEMM is slow at exactly
+// 224 and 256 rows, 4B shape 36 / 28, and not between: a rule for those two counts would be one for nothing else.)
 extern "C" int ia_gemm_wide_rope_fits(int M, int N, int K) {
     if (M <= 0 || M > 1024 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
-    return K >= 4096 && (K >= 5120 || M <= 384) && (long long)N * K >= 4096LL * 5120 && gw_plan(M, N, K, false, true).splits > 1;
+    return K >= 4096 && (K >= 5120 || M <= 384 || M >= 500) && (long long)N * K >= 4096LL * 5120 &&
+           gw_plan(M, N, K, false, true).splits > 1;
 }
 
 // Whether a [gate; up] of N features each goes here instead of to the vendor's GEMM and the activation's kernel.  The product cannot
 // be split, so the kernel gains where its own blocks fill their rounds (its time within 0.9 of 1.22 PFLOP/s, or of 4 TB/s over the
-// operands, and what the second kernel takes; all of it for a short k under few features) and the vendor's blocks of 256 x 256 do
-// not, or, with many rows and features, where the vendor's last round is half empty.  Measured in captured graphs at 129 to 1,024 rows, the six dense shapes and 1,024 to
-// 25,600 features by 512 to 8,192 k, and 400 other sizes: where this rule says yes no point is below 0.97 of the two kernels'
-// speed, 1.2 times as fast in the mean (us, the two kernels / this: 1.7B shape, 512 rows 36 / 35; 8B shape, 320 rows 81 / 77, 456 rows
-// 101 / 108, 512 rows 102 / 124; 14B shape, 160 rows 107 / 115, 521 rows 201 / 208, 900 rows 404 / 300; 4B shape, 768 rows 82 / 102,
-// 900 rows 114 / 107).
+// operands, and what the second kernel takes; within 1.05 of it for a short k under few features, or many rows and features) and the
+// vendor's blocks of 256 x 256 do not, or, from 800 rows, where the vendor's last round is half empty.  Measured in captured graphs at
+// 129 to 1,024 rows, the six dense shapes, 1,024 to 25,600 features by 512 to 8,192 k, and 805 sizes drawn where the rule says yes: of
+// 1,056 points where it does one is below 0.97 of the two kernels' speed (0.96), 1.2 times as fast in the mean (us, the two kernels /
+// this: 1.7B shape, 512 rows 36 / 35; 8B shape, 320 rows 81 / 77, 456 rows 101 / 108, 512 rows 102 / 124, 700 rows 165 / 135; 14B shape,
+// 160 rows 107 / 115, 521 rows 201 / 208, 900 rows 404 / 300; 4B shape, 768 rows 82 / 102, 900 rows 114 / 107).
 extern "C" int ia_gemm_wide_dual_fits(int M, int N, int K) {
     if (M < 300 || M > 1024 || N < 2048 || K <= 0 || K % GW_STAGE_K || N % 4 || ((long long)N + GW_BN) * K * 2 >= (1LL << 32)) return 0;
     const double theirs = vendor_fill(M, 2 * N);
     if (M >= 800 && N >= 8192 && theirs <= 0.72) return 1;
     const double flops = 4.0 * M * N * K / 1.22e9, bytes = (2.0 * N + M) * K * 2.0 / 4.0e6;
-    const double limit = M >= 512 && K <= 2048 && N <= 6144 ? 1.0 : theirs <= 0.6 ? 0.9 : 0.0;
+    const double limit = theirs > 0.6 ? 0.0 : (M >= 400 && K <= 2048 && N <= 6144) || (M >= 640 && N >= 8192) ? 1.05 : 0.9;
     return gw_plan(M, N, K, true, false).cost <= limit * ((flops > bytes ? flops : bytes) + 8.0 + M * (double)N * 6.0 / 5.0e6);
 }
 
