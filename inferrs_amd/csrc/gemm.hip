@@ -272,7 +272,8 @@ extern "C" int ia_gemm_tiled(void* out, const void* x, const void* w, int M, int
     if (in_dtype == IA_F32 && out_dtype == IA_F32 && ia_gemm_f32_fits(M, N, K) && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 &&
         (g_rows_shape == 0 || M > GR_ROWS))
         return ia_gemm_f32(out, x, w, M, N, K, stream);
-    // up to 64 rows, 16 at a time, where the tiles of 64 x 64 would be few (the weights are read once for every 16 rows)
+    // up to 16 rows, or up to 64 of bfloat16, 16 at a time, where the tiles of 64 x 64 would be few (the weights are read once for
+    // every 16 rows)
     if (M <= 4 * GR_ROWS && (M <= GR_ROWS || N <= 4096 * 4) && K % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) % (4 * elem)) == 0) {
         const size_t out_elem = out_dtype == IA_F32 ? 4 : 2;
         for (int m0 = 0; m0 < M; m0 += GR_ROWS) {

@@ -147,7 +147,6 @@ extern "C" int ia_gemm_f32_tune(int shape) {
 // x and w 16-byte aligned, K a multiple of 4.
 extern "C" int ia_gemm_f32(void* out, const void* x, const void* w, int M, int N, int K, hipStream_t stream) {
     IA_CHECK(M > 0 && N > 0 && K > 0 && K % 4 == 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
-    IA_CHECK((M + 127LL) / 128 <= 65535, "gemm_f32: %d rows exceed the grid", M);
     IA_CHECK((((uintptr_t)x | (uintptr_t)w) & 15) == 0, "gemm_f32: x and w must be 16-byte aligned");
     static int cus = 0;
     if (cus == 0) {
@@ -158,7 +157,7 @@ extern "C" int ia_gemm_f32(void* out, const void* x, const void* w, int M, int N
     // times the instructions a block has for a step of four k, and a little a turn; a block that is alone on its unit waits for
     // memory besides (32 rows, 4,096 features: 1 x 1 tiles 47 us, 2 x 1 62, 3 x 1 73, 4 x 1 95).  Measured at 555 rows and 4,096 features:
     // 9 x 1 tiles in one turn 192 us, 5 x 1 in two 191, 3 x 1 in three 188, 10 x 1 in one 204; at 24,576 features 9 x 2 in three
-    // turns 918, 7 x 2 in four 942, 9 x 1 in six 969; 130 rows and 24,576 features: 5 x 1 in three turns 297, 3 x 2 in six 330.
+    // turns 918, 7 x 2 in four 942, 9 x 1 in six 969; 130 rows and 24,576 features: 5 x 1 in three turns 297, 3 x 2 in three 330.
     int best_m = 8, best_n = 2;
     double best = 1e30;
     for (int nr = 1; nr <= 2; ++nr)
@@ -170,6 +169,8 @@ extern "C" int ia_gemm_f32(void* out, const void* x, const void* w, int M, int N
             if (cost < best && blocks < (1LL << 31)) best = cost, best_m = mt, best_n = nr;
         }
     if (g_f32_shape) best_m = g_f32_shape / 10, best_n = g_f32_shape % 10;
+    const long long blocks = (long long)((M + 16LL * best_m - 1) / (16 * best_m)) * ((N + 64LL * best_n - 1) / (64 * best_n));
+    IA_CHECK(blocks < (1LL << 31), "gemm_f32: %d rows by %d features are %lld blocks, too many for one launch", M, N, blocks);
     float* o = (float*)out;
     const float *xi = (const float*)x, *wi = (const float*)w;
     switch (best_m * 10 + best_n) {

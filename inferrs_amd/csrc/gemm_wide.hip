@@ -25,11 +25,12 @@
 // Shared memory: piece c (16 bytes) of row r lies at place c ^ ((r >> 1) & 7) of its row's 128 bytes, so that the rows which
 // one operand read takes at the same k fall on different banks.
 //
-// Measured (us, the vendor's GEMM and the kernel behind it against this one and its reader; 8B and 14B shapes): down at 200 rows
-// 56 / 38 and 226 / 61, at 456 86 / 58 and 174 / 86, at 521 107 / 64 and 186 / 93, at 1,024 127 / 101 and 260 / 160, at 2,048
-// 192 / 179 and 300 / 296; output projection at 256 25 / 23 and 49 / 26, at 1,024 46 / 44 and 63 / 62; gate|up with the activation at
-// 320 88 / 77 and 163 / 174, at 768 158 / 140 and 282 / 283.  1,200 to 1,340 TFLOP/s over a long k from 160 rows a block on, at the
-// chip's power limit (with operands of zeros a stage takes a fifth less).
+// Measured in captured graphs (us, the vendor's GEMM and the kernel behind it / this one and its reader; 8B and 14B shapes): down at
+// 200 rows 54 / 42 and 230 / 64, at 456 88 / 59 and 173 / 87, at 521 109 / 66 and 184 / 93, at 1,024 132 / 103 and 257 / 160, at 2,048
+// 196 / 184 and 301 / 300; output projection at 256 28 / 25 and 56 / 33, at 1,024 51 / 48 and 76 / 67; gate|up with the activation, 8B
+// shape, at 320 81 / 77, at 700 165 / 135, 14B shape at 900 404 / 300.  A stage's rate over a long k is 1,270 to 1,340 TFLOP/s with
+// 160 to 240 rows a block and 1,140 with 256, at the chip's power limit (with operands of zeros a stage takes a fifth less).
+
 #include <type_traits>
 #include <utility>
 
@@ -67,7 +68,7 @@ __device__ __forceinline__ void gw_unrolled(std::integer_sequence<int, I...>, Fn
     (fn(std::integral_constant<int, I>()), ...);
 }
 
-enum { GW_BF16 = 0, GW_F32 = 1, GW_DUAL = 2 };          // what leaves the kernel; GW_F32: a split's sums (or whole ones)
+enum { GW_BF16 = 0, GW_F32 = 1, GW_DUAL = 2 };          // what leaves the kernel; GW_F32: a split's sums
 
 template <int MT, int OUT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
@@ -351,13 +352,13 @@ extern "C" int ia_gemm_wide_dual_fits(int M, int N, int K) {
     return gw_plan(M, N, K, true, false).cost <= limit * ((flops > bytes ? flops : bytes) + 8.0 + M * (double)N * 6.0 / 5.0e6);
 }
 
-// out_mode 0: out [M, N] bfloat16; 1: float; 2: [splits][M][N] float with splits = ia_gemm_wide_splits(M, N, K).  dual (an
-// activation, IA_ACT_*): w = [gate; up] of N rows each (mode 0 only).  K a multiple of 64, operands 16-byte aligned.
+// out_mode 0: out [M, N] bfloat16; 2: [splits][M][N] float with splits = ia_gemm_wide_splits(M, N, K).  dual (an activation,
+// IA_ACT_*): w = [gate; up] of N rows each (mode 0 only).  K a multiple of 64, operands 16-byte aligned.
 extern "C" int ia_gemm_wide_bf16(void* out, const void* x, const void* w, int M, int N, int K, int out_mode, int dual,
                                  hipStream_t stream) {
     IA_CHECK(M > 0 && N > 0 && K > 0 && K % GW_STAGE_K == 0 && N % 4 == 0, "gemm_wide: bad sizes M=%d N=%d K=%d (K a multiple of %d, N of 4)",
              M, N, K, GW_STAGE_K);
-    IA_CHECK(out_mode >= 0 && out_mode <= 2 && (!dual || out_mode == 0), "gemm_wide: output mode %d%s", out_mode,
+    IA_CHECK((out_mode == 0 || out_mode == 2) && (!dual || out_mode == 0), "gemm_wide: output mode %d%s", out_mode,
              dual ? " does not go with the activation inside" : " is unknown");
     IA_CHECK(dual >= 0 && dual <= IA_ACT_LAST, "gemm_wide: unknown activation %d", dual);
     IA_CHECK((((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0, "gemm_wide: operands must be 16-byte aligned");

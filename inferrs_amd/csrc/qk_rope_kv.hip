@@ -543,7 +543,7 @@ __global__ __launch_bounds__(QKV_THREADS) void qk_rope_kv_bf16_vec_kernel(
 // go from lane to lane without shared memory.  The sum runs in the order of the kernel above, so
 // that both give the same bits.
 // QKV_HEADS: 8; 2 in steps of few tokens, where threads of eight heads would leave most of the chip without a block (117 tokens
-// of 24 heads: 44 blocks; 8.3 -> 5.2 us, the two splits of their product added up on the way).
+// of 24 heads: 22 blocks of queries and keys; 8.3 -> 5.2 us, the two splits of their product added up on the way).
 template <int TPU, int QKV_HEADS, typename Rows>
 __global__ __launch_bounds__(QKV_THREADS) void qk_rope_kv_bf16_rows_kernel(
     bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache,

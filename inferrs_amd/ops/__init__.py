@@ -1086,7 +1086,7 @@ def gemm_mid_bf16(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype = tor
 
 # ---- products of 129 to 2,048 rows ---------------------------------------------------------------
 # Steps with prompt portions: gemm_wide.hip splits k between blocks where the vendor's GEMM leaves the chip half empty (its
-# header has the figures, and the rule for [gate; up]).
+# header has the figures; which product goes there is asked of ia_gemm_wide_norm_fits, _rope_fits and _dual_fits).
 WIDE_MAX_ROWS = 2048
 
 
@@ -1155,7 +1155,7 @@ def linear(x, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None, mid: boo
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [m, k] . w[n, k]^T (+ bias [n], in the precision of w).  32-bit: `gemm_tiled` (true 32-bit, fixed
     order).  bfloat16: the skinny MFMA kernel for up to SKINNY_MAX_ROWS rows, the vendor's GEMM beyond that (the
-    reference uses cuBLAS for all of them).  A 32-bit result of bfloat16 operands (logits) comes straight from
+    reference uses cuBLAS for all of them; products that `linear_partials` or `gated_linear` send to gemm_wide.hip do not come here).  A 32-bit result of bfloat16 operands (logits) comes straight from
     the skinny kernel's accumulators for those few rows; beyond that it is the vendor's bfloat16
     result widened, which is what the reference does for every row (its logits are computed in
     the model's precision and cast for sampling, `inferrs/src/sampler.rs:182`).  From `mid_from_rows(k)` rows on (and up to
