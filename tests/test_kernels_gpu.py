@@ -1216,10 +1216,10 @@ def test_few_row_product_of_the_32_bit_path_with_every_block_shape(dtype):
             close(y, x[:y.shape[0]].double() @ w.double().cpu().t(), tol(dtype, 2e-6), "few rows")
 
 
-@pytest.mark.parametrize("m,n,k", [(129, 260, 64), (130, 4, 192), (160, 516, 640), (257, 1024, 128), (521, 256, 1088), (1000, 300, 2048)])
+@pytest.mark.parametrize("m,n,k", [(129, 260, 64), (130, 4, 192), (160, 516, 640), (257, 1024, 128), (521, 256, 1088), (1000, 300, 2048), (2047, 1540, 640)])
 def test_wide_product_in_every_block_shape(m, n, k):
     """Blocks of every number of rows and k split every way that exists, at sizes that end inside tiles of rows, of features and
-    inside a share of k: the exact product within its storage's rounding, 32-bit sums that do not depend on the blocks' rows,
+    inside a share of k, and (2,047 rows) in more than one round of blocks: the exact product within its storage's rounding, 32-bit sums that do not depend on the blocks' rows,
     and the activation inside, rounded between the two as two kernels would round."""
     from inferrs_amd import ops
     lib = ops.library()
@@ -1297,11 +1297,11 @@ def test_gate_and_up_on_either_route(m, n, k):
     close(got[rows], torch.nn.functional.silu(gate) * up, 3 * 2 ** -8, (m, n, k))
 
 
-@pytest.mark.parametrize("m,n,k", [(17, 5, 4), (33, 64, 28), (161, 130, 36), (100, 259, 516), (320, 257, 132), (17, 16400, 100)])
+@pytest.mark.parametrize("m,n,k", [(17, 5, 4), (33, 64, 28), (161, 130, 36), (100, 259, 516), (320, 257, 132), (17, 16400, 100), (33, 33000, 36)])
 def test_32_bit_product_on_the_matrix_cores_has_the_bits_of_the_vector_units(m, n, k):
-    """Every shape of block that exists (10 * rows of x + rows of w, in 16 and 64), at sizes that end inside tiles and chunks: the
-    bits of the kernel for few rows, one chain of fused multiply-adds with k ascending; numbers without a leading bit, infinities
-    and NaN go the same way."""
+    """Every shape of block that exists (10 * rows of x + rows of w, in 16 and 64), at sizes that end inside tiles and chunks, in grids
+    of up to a block a compute unit and (33,000 features) of more, whose chunks are shorter: the bits of the kernel for few rows, one
+    chain of fused multiply-adds with k ascending; numbers without a leading bit, infinities and NaN go the same way."""
     from inferrs_amd import ops
     lib = ops.library()
     x, w = randn(m, k, dtype=torch.float32, seed=1), randn(n, k, dtype=torch.float32, seed=2)
@@ -1318,6 +1318,23 @@ def test_32_bit_product_on_the_matrix_cores_has_the_bits_of_the_vector_units(m, 
         assert lib.ia_gemm_f32_tune(113) != 0 and "gemm_f32_tune" in lib.ia_last_error().decode()
     finally:
         lib.ia_gemm_f32_tune(0)
+
+
+@pytest.mark.parametrize("m", [1, 7, 8, 9, 12, 16])
+@pytest.mark.parametrize("n", [16383, 16384, 65535, 65536])
+def test_32_bit_products_of_few_rows_have_the_same_bits_on_either_route(m, n):
+    """Around the rows and features (64 a compute unit) from which a product goes to the matrix cores: the bits of the kernel for few
+    rows, asked for by its shape, as the rule would have it there."""
+    from inferrs_amd import ops
+    lib, k = ops.library(), 68
+    x, w = dev(randn(m, k, dtype=torch.float32, seed=m)), dev(randn(n, k, dtype=torch.float32, seed=n))
+    got = ops.gemm_tiled(x, w)
+    try:
+        lib.ia_gemm_rows_tune(816)
+        assert torch.equal(got, ops.gemm_tiled(x, w))
+    finally:
+        lib.ia_gemm_rows_tune(0)
+    close(got, x.double().cpu() @ w.double().cpu().t(), 2e-6, (m, n))
 
 
 @pytest.mark.parametrize("m,n,k", [(130, 72, 40), (512, 4096, 1024), (2048, 6144, 4096), (300, 1000, 136), (129, 64, 33), (1024, 1024, 3072)])
