@@ -30,7 +30,6 @@
 // 196 / 184 and 301 / 300; output projection at 256 28 / 25 and 56 / 33, at 1,024 51 / 48 and 76 / 67; gate|up with the activation, 8B
 // shape, at 320 81 / 77, at 700 165 / 135, 14B shape at 900 404 / 300.  A stage's rate over a long k is 1,270 to 1,340 TFLOP/s with
 // 160 to 240 rows a block and 1,140 with 256, at the chip's power limit (with operands of zeros a stage takes a fifth less).
-
 #include <type_traits>
 #include <utility>
 
@@ -301,55 +300,64 @@ extern "C" int ia_gemm_wide_splits(int M, int N, int K) {
     return wide_plan(M, N, K, false, true).splits;
 }
 
+// The rules below say where this kernel goes ahead of the vendor's GEMM.  They were measured in whole steps: prompts of 130 to 2,048
+// tokens of six dense shapes (width 1,024 to 5,120) replayed from graphs, with each product on either kernel, side by side in one
+// process.  (A graph of the product and its reader alone is no measure: its operands lie in caches that a step's other kernels have
+// turned over, and it put [gate; up] of the 8B shape at 176 to 360 rows on the wrong side by 2 to 3 % of the layer.)
+
 // The share of full rounds of the compute units that blocks of 256 x 256, the vendor's largest, would make of a product.
 static double vendor_fill(int M, int N) {
     const long long tiles = (long long)((M + 255) / 256) * ((N + 255) / 256), cus = wide_cus();
     return (double)tiles / (double)((tiles + cus - 1) / cus * cus);
 }
 
+// Whether a step of M rows of a stream of `width` features is one that the host bounds where it is met eagerly, as every length of a
+// prompt is the first times: a call of the vendor's GEMM costs the host 14 us and one of this package's kernels 6.5, and these products
+// take the GPU little more.  They stay here even where a replayed step would have the vendor's GEMM a little ahead.  us a layer, eager /
+// replayed, the products by the rules for wide steps and by this one: 0.6B shape (width 1,024), 300 tokens 156 / 92 and 125 / 86,
+// 512 tokens 155 / 97 and 105 / 100, 1.7B shape (2,048), 400 tokens 156 / 127 and 128 / 123, 640 tokens 158 / 149 and 149 / 146, 4B shape
+// (2,560), 130 tokens 165 / 151 and 153 / 143.  Beyond it the GPU is the bound either way (1.7B shape, 1,024 tokens 191 / 186 and 197 /
+// 195; 4B shape, 512 tokens 207 / 198 and 206 / 200).
+static bool host_bound(int M, int width) { return width <= 2048 ? M < 1024 : width <= 3072 && (long long)M * width < (1LL << 20); }
+
 // Whether a product whose result may stay split goes here instead of to the vendor's GEMM, for the reader that adds it to the
-// residual stream and norms it.  Both sides measured with their readers in captured graphs (between single launches the vendor's
-// side waits for the host, which a graph does not) at 129 to 2,048 rows: the products of six dense shapes (27 counts of rows), a
-// grid of 512 to 8,192 features by 512 to 16,384 k (20 counts), and 458 sizes drawn where the rule says yes.  The kernel gains by what
-// the split gives, so it needs a long k and enough features; short products are a few microseconds of fixed costs and the sums' way
-// out and back in on top (us, the vendor's side / this: 0.6B shape, 512 rows, o 14 / 17, down 17 / 20; 1.7B shape o 18 / 22, down 33 /
-// 29; 4B shape, 144 rows, o 20 / 21; 8B shape, 521 rows, o 42 / 35, down 109 / 66).  Unsplit: where the vendor's blocks leave a third
-// of the chip empty (14B shape, down at 1,536 rows, 367 / 243).  Of the 1,729 points where this rule says yes four are below 0.97 of
-// the vendor's speed, 0.90 to 0.96, all of them unsplit; 1.26 times as fast over all of the dense shapes' points.
+// residual stream and norms it.  The kernel gains by what the split gives, so it needs a long k and enough features; short products are
+// a few microseconds of fixed costs and the sums' way out and back in on top (us a layer by the vendor's GEMM and by this one: 14B
+// shape, down at 200 rows 534 / 366, at 521 625 / 541, o at 256 572 / 546; 1.7B shape, 1,024 rows, down 197 / 192, o 197 / 200).
+// Unsplit: where the vendor's blocks leave a third of the chip empty (14B shape, down at 1,536 rows, 1,249 / 1,130).
 extern "C" int ia_gemm_wide_norm_fits(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
+    if (host_bound(M, N)) return 1;
     if (gw_plan(M, N, K, false, true).splits == 1) return K >= 8192 && vendor_fill(M, N) < 0.63;
     return K >= 4096 && N >= 1024 && (long long)K * (N < 3072 ? N : 3072) >= (M <= 192 ? 3072 : M <= 256 ? 2560 : 2048) * 4096LL;
 }
 
-// The same for the kernel that norms and turns queries and keys and writes the cache (129 to 1,024 rows; six dense shapes, 1,536 to
-// 12,288 features by 512 to 8,192 k, and 239 drawn sizes).  That reader takes the splits at the price of a stored product, and a
-// product of q|k|v has many features, so that the split gives less than above: unsplit, or over a short k, the vendor's GEMM is as
-// fast or faster (us, the vendor's side / this: 0.6B shape, 512 rows 17 / 20; 1.7B shape, 256 rows 18 / 24; 4B shape, 640 rows 38 / 39;
-// 8B shape, 256 rows 45 / 31, 456 rows 40 / 42, 700 rows 58 / 49; 14B shape, 521 rows 72 / 54).  Of the 599 points where this rule says
-// yes two are below 0.97 of the vendor's speed (0.95 and 0.96), 1.2 times as fast in the mean.  (The vendor's GEMM is slow at exactly
-// 224 and 256 rows, 4B shape 36 / 28, and not between: a rule for those two counts would be one for nothing else.)
+// The same for the kernel that norms and turns queries and keys and writes the cache, up to 1,024 rows.  A product of q|k|v has many
+// features, so that the split gives less than above: over a short k the vendor's GEMM is as fast or faster (us a layer: 4B shape, 456
+// rows 241 / 244, 850 rows 332 / 336), over a long one this kernel, split or not (8B shape, 130 rows 251 / 236, 700 rows 436 / 420, 900
+// 484 / 475; 14B shape, 521 rows 625 / 605; 32B shape, 900 rows 1,105 / 1,085; of 46 points one, 14B shape at 768 rows, is slower, 740 / 742).
 extern "C" int ia_gemm_wide_rope_fits(int M, int N, int K) {
     if (M <= 0 || M > 1024 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
-    return K >= 4096 && (K >= 5120 || M <= 384 || M >= 500) && (long long)N * K >= 4096LL * 5120 &&
-           gw_plan(M, N, K, false, true).splits > 1;
+    return host_bound(M, K) || (K >= 4096 && (long long)N * K >= 4096LL * 5120);
 }
 
-// Whether a [gate; up] of N features each goes here instead of to the vendor's GEMM and the activation's kernel.  The product cannot
-// be split, so the kernel gains where its own blocks fill their rounds (its time within 0.9 of 1.22 PFLOP/s, or of 4 TB/s over the
-// operands, and what the second kernel takes; within 1.05 of it for a short k under few features, or many rows and features) and the
-// vendor's blocks of 256 x 256 do not, or, from 800 rows, where the vendor's last round is half empty.  Measured in captured graphs at
-// 129 to 1,024 rows, the six dense shapes, 1,024 to 25,600 features by 512 to 8,192 k, and 805 sizes drawn where the rule says yes: of
-// 1,056 points where it does one is below 0.97 of the two kernels' speed (0.96), 1.2 times as fast in the mean (us, the two kernels /
-// this: 1.7B shape, 512 rows 36 / 35; 8B shape, 320 rows 81 / 77, 456 rows 101 / 108, 512 rows 102 / 124, 700 rows 165 / 135; 14B shape,
-// 160 rows 107 / 115, 521 rows 201 / 208, 900 rows 404 / 300; 4B shape, 768 rows 82 / 102, 900 rows 114 / 107).
+// Whether a [gate; up] of N features each goes here instead of to the vendor's GEMM and the activation's kernel, up to 1,024 rows.  The
+// product cannot be split.  This kernel's own time has to come within a tenth of 1.22 PFLOP/s (or of 4 TB/s over the operands) and what
+// the second kernel takes; not where its blocks leave two fifths of their rounds empty (14B shape, 130 to 200 rows: 454 / 461, 468 / 474,
+// 534 / 544 us a layer) nor where the vendor's are nearly all work (4B shape, 768 rows, 287 / 298).  Elsewhere 8B shape, 200 rows 250 /
+// 243, 700 rows 436 / 412, 14B shape, 900 rows 934 / 831, 32B shape, 1,024 rows 1,222 / 1,167; where the rule says yes, at worst 0.985 of
+// the step's speed.
 extern "C" int ia_gemm_wide_dual_fits(int M, int N, int K) {
-    if (M < 300 || M > 1024 || N < 2048 || K <= 0 || K % GW_STAGE_K || N % 4 || ((long long)N + GW_BN) * K * 2 >= (1LL << 32)) return 0;
-    const double theirs = vendor_fill(M, 2 * N);
-    if (M >= 800 && N >= 8192 && theirs <= 0.72) return 1;
+    if (M <= 0 || M > 1024 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4 || ((long long)N + GW_BN) * K * 2 >= (1LL << 32)) return 0;
+    const WidePlan plan = gw_plan(M, N, K, true, false);
+    if (!host_bound(M, K)) {
+        const long long cus = wide_cus(), tiles_m = (M + 16 * plan.mt - 1) / (16 * plan.mt), tiles_n = (N + GW_BN / 2 - 1) / (GW_BN / 2);
+        const long long ours = (tiles_m * tiles_n + cus - 1) / cus * cus;                  // (blocks that this kernel's rounds have room for)
+        const long long theirs = ((M + 255) / 256 * ((2LL * N + 255) / 256) + cus - 1) / cus * cus;
+        if (N < 2048 || tiles_m * tiles_n < 0.6 * ours || 2.0 * M * N >= 0.85 * 65536.0 * theirs) return 0;
+    }
     const double flops = 4.0 * M * N * K / 1.22e9, bytes = (2.0 * N + M) * K * 2.0 / 4.0e6;
-    const double limit = theirs > 0.6 ? 0.0 : (M >= 400 && K <= 2048 && N <= 6144) || (M >= 640 && N >= 8192) ? 1.05 : 0.9;
-    return gw_plan(M, N, K, true, false).cost <= limit * ((flops > bytes ? flops : bytes) + 8.0 + M * (double)N * 6.0 / 5.0e6);
+    return plan.cost <= 1.1 * ((flops > bytes ? flops : bytes) + 8.0 + M * (double)N * 6.0 / 5.0e6);
 }
 
 // out_mode 0: out [M, N] bfloat16; 2: [splits][M][N] float with splits = ia_gemm_wide_splits(M, N, K).  dual (an activation,

@@ -1257,7 +1257,7 @@ def test_wide_product_in_every_block_shape(m, n, k):
         assert torch.equal(ours, theirs), ways
 
 
-@pytest.mark.parametrize("m,n,k,split", [(512, 1024, 2048, None), (512, 1024, 3072, None), (160, 2560, 4096, None), (521, 4096, 4096, True),
+@pytest.mark.parametrize("m,n,k,split", [(512, 1024, 2048, True), (1024, 1024, 2048, None), (160, 2560, 4096, True), (521, 4096, 4096, True),
                                          (160, 4096, 12288, True), (1536, 5120, 17408, False)])
 def test_product_ahead_of_the_streams_norm_takes_the_measured_route(m, n, k, split):
     """`linear_partials` names the wide kernel's result, split or whole, where that was measured faster, and None where the vendor's
@@ -1270,16 +1270,16 @@ def test_product_ahead_of_the_streams_norm_takes_the_measured_route(m, n, k, spl
         close(got.materialize() if split else got, x.double().cpu() @ w.double().cpu().t(), 2 ** -8, (m, n, k))
 
 
-@pytest.mark.parametrize("m,n,k,split", [(512, 4096, 1024, False), (256, 4096, 2048, False), (456, 6144, 4096, False), (256, 6144, 4096, True),
+@pytest.mark.parametrize("m,n,k,split", [(512, 4096, 1024, False), (1024, 4096, 1024, None), (640, 6144, 2560, None), (456, 6144, 4096, True),
                                          (521, 7168, 5120, True), (100, 4096, 1024, True)])
 def test_product_ahead_of_the_rotation_takes_the_measured_route(m, n, k, split):
-    """Queries, keys and values: split where that was measured faster, else None (the vendor's GEMM)."""
+    """Queries, keys and values: the package's kernel, split or whole, where that was measured faster, else None (the vendor's GEMM)."""
     from inferrs_amd import ops
     x, w = dev(randn(m, k, dtype=torch.bfloat16, seed=1)), dev(randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.05))
     got = ops.linear_partials(x, w, own_rows=True)
-    assert (got is not None) == split
-    if split and m > ops.MID_MAX_ROWS:
-        close(got.materialize(), x.double().cpu() @ w.double().cpu().t(), 2 ** -8, (m, n, k))
+    assert (got is None) == (split is None) and (split is None or isinstance(got, ops.Partials) == split)
+    if got is not None:
+        close(got.materialize() if split else got, x.double().cpu() @ w.double().cpu().t(), 2 ** -8, (m, n, k))
 
 
 @pytest.mark.parametrize("m,n,k", [(512, 12288, 4096), (700, 3072, 1024), (900, 9728, 2560)])

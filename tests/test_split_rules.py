@@ -59,24 +59,29 @@ DENSE = {"0.6B": (1024, 3072, 16), "1.7B": (2048, 6144, 16), "4B": (2560, 9728, 
 
 
 @pytest.mark.parametrize("shape,product,rows,own", [
-    # where both kernels were timed in captured graphs, the product with its reader, on either side of the rule
-    ("0.6B", "o", 512, False), ("0.6B", "down", 512, False), ("1.7B", "o", 384, False), ("1.7B", "down", 512, True), ("4B", "o", 144, False),
-    ("4B", "o", 200, True), ("8B", "down", 2048, True), ("4B", "o", 420, True), ("8B", "o", 521, True), ("8B", "down", 200, True), ("14B", "down", 129, True), ("14B", "down", 1536, True),
-    ("32B", "o", 1024, True)])
+    # where whole steps were timed with the product on either kernel, on either side of the rule; narrow steps, which the host bounds
+    # wherever they are met eagerly, stay with the kernel whose call costs less
+    ("0.6B", "o", 512, True), ("0.6B", "down", 1000, True), ("0.6B", "o", 1024, False), ("0.6B", "down", 1024, False),
+    ("1.7B", "o", 384, True), ("1.7B", "down", 900, True), ("1.7B", "o", 1024, False), ("1.7B", "down", 1024, True),
+    ("4B", "o", 144, True), ("4B", "o", 420, True), ("8B", "down", 2048, True), ("8B", "o", 521, True), ("8B", "down", 200, True),
+    ("14B", "down", 129, True), ("14B", "down", 1536, True), ("32B", "o", 1024, True)])
 def test_products_behind_which_the_stream_is_normed_go_where_they_are_faster(shape, product, rows, own):
     width, ff, heads = DENSE[shape]
     assert bool(ops.library().ia_gemm_wide_norm_fits(rows, width, heads * 128 if product == "o" else ff)) == own
 
 
-@pytest.mark.parametrize("shape,rows,own", [("0.6B", 512, False), ("1.7B", 256, False), ("4B", 320, False), ("4B", 640, False), ("8B", 160, True),
-                                            ("8B", 256, True), ("8B", 456, False), ("8B", 700, True), ("14B", 521, True), ("14B", 900, False), ("32B", 456, True)])
+@pytest.mark.parametrize("shape,rows,own", [("0.6B", 512, True), ("0.6B", 1024, False), ("1.7B", 900, True), ("1.7B", 1024, False), ("4B", 409, True),
+                                            ("4B", 410, False), ("4B", 640, False), ("8B", 160, True), ("8B", 456, True), ("8B", 1024, True),
+                                            ("8B", 1025, False), ("14B", 521, True), ("14B", 900, True), ("32B", 456, True)])
 def test_products_of_queries_and_keys_go_where_they_are_faster(shape, rows, own):
     width, _, heads = DENSE[shape]
     assert bool(ops.library().ia_gemm_wide_rope_fits(rows, (heads + 16) * 128, width)) == own
 
 
-@pytest.mark.parametrize("shape,rows,own", [("0.6B", 129, False), ("0.6B", 700, True), ("4B", 160, False), ("4B", 768, False), ("4B", 900, True), ("8B", 129, False), ("8B", 456, False),
-                                            ("8B", 512, False), ("8B", 700, True), ("1.7B", 456, True), ("14B", 200, False), ("14B", 521, False), ("14B", 832, True), ("14B", 1024, True)])
+@pytest.mark.parametrize("shape,rows,own", [("0.6B", 512, True), ("0.6B", 700, True), ("1.7B", 456, True), ("4B", 160, True), ("4B", 580, True),
+                                            ("4B", 768, False), ("4B", 900, True), ("8B", 200, True), ("8B", 320, True), ("8B", 456, False),
+                                            ("8B", 512, False), ("8B", 700, True), ("14B", 130, False), ("14B", 200, False), ("14B", 521, False),
+                                            ("14B", 832, True), ("14B", 1024, True), ("14B", 1025, False), ("32B", 1024, True)])
 def test_gate_and_up_go_where_they_are_faster(shape, rows, own):
     width, ff, _ = DENSE[shape]
     assert bool(ops.library().ia_gemm_wide_dual_fits(rows, ff, width)) == own
