@@ -9,6 +9,7 @@ as the door to the vendor's GEMM library (the reference uses cuBLAS there,
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Dict, Optional, Tuple
 
@@ -361,6 +362,7 @@ def qk_rope_kv(qkv: torch.Tensor, nq: int, nkv: int, d: int, *,
     return q_out
 
 
+@functools.lru_cache(maxsize=4096)
 def qk_rope_kv_partials_fits(n: int, d: int, rot: int, interleaved: bool, page_size: int) -> bool:
     """Whether `qk_rope_kv` reads projections that are still split along their k (`Partials`) in a step of `n` tokens."""
     return bool(library().ia_qk_rope_kv_partials_fits(n, d, rot, int(interleaved), page_size))
@@ -1119,6 +1121,14 @@ def gemm_wide_bf16(x: torch.Tensor, w: torch.Tensor, dual: bool = False, partial
     return out
 
 
+@functools.lru_cache(maxsize=4096)
+def _wide_pays(reader: str, m: int, n: int, k: int) -> bool:
+    """gemm_wide.hip's rule for `m` rows, `n` features and k ahead of a reader ("norm", "rope", or "dual": [gate; up] of n features
+    each).  A rule follows from these sizes alone and is asked three times a layer, so its answers are kept: a step that the host
+    bounds waits for each (0.7 to 0.9 us through ctypes; a product that stays with the vendor's GEMM 4.6 us of asking -> 0.6)."""
+    return m <= WIDE_MAX_ROWS and bool(getattr(library(), f"ia_gemm_wide_{reader}_fits")(m, n, k))
+
+
 def linear_partials(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, own_rows: bool = False):
     """x . w^T for a reader that takes `Partials`, split along k where the weight has few rows: the norm that adds the product to
     the stream, or (`own_rows`) the kernel that norms and turns queries and keys.  None where `linear` is faster, or where
@@ -1126,12 +1136,14 @@ def linear_partials(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tenso
     them: the caller then forms the whole product, and `linear` adds the bias."""
     # (up to MID_MAX_ROWS rows: who asks ahead of the norm is in a step whose products go to gemm_mid.hip, the rule has been asked with
     # the stream's width, and a product of another width follows it; with `own_rows` the width of the rows themselves decides)
-    if bias is None and isinstance(x, torch.Tensor) and x.shape[0] >= MID_MIN_ROWS and mid_fits(x, w, few_rows=not own_rows):
-        return gemm_mid_bf16(x, w, partial=True)
-    if bias is None and isinstance(x, torch.Tensor) and wide_fits(x, w):
-        lib = library()
-        if (lib.ia_gemm_wide_rope_fits if own_rows else lib.ia_gemm_wide_norm_fits)(x.shape[0], w.shape[0], x.shape[1]):
-            return gemm_wide_bf16(x, w, partial=True)
+    if bias is not None or not isinstance(x, torch.Tensor):
+        return None
+    m, k = x.shape
+    if m <= MID_MAX_ROWS:
+        if m >= MID_MIN_ROWS and mid_fits(x, w, few_rows=not own_rows):
+            return gemm_mid_bf16(x, w, partial=True)
+    elif _wide_pays("rope" if own_rows else "norm", m, w.shape[0], k) and wide_fits(x, w):
+        return gemm_wide_bf16(x, w, partial=True)
     return None
 
 
@@ -1321,8 +1333,8 @@ def gated_linear(x, w_gate_up: torch.Tensor, activation: str = "silu",
         if (even and mid_fits(x, w_gate_up)
                 and w_gate_up.numel() * w_gate_up.element_size() <= MID_DUAL_MAX_BYTES):
             return gemm_mid_bf16(x, w_gate_up, dual=True, activation=activation)
-        if (w_gate_up.shape[0] % 8 == 0 and wide_fits(x, w_gate_up)
-                and library().ia_gemm_wide_dual_fits(x.shape[0], w_gate_up.shape[0] // 2, x.shape[1])):
+        if (x.shape[0] > MID_MAX_ROWS and w_gate_up.shape[0] % 8 == 0
+                and _wide_pays("dual", x.shape[0], w_gate_up.shape[0] // 2, x.shape[1]) and wide_fits(x, w_gate_up)):
             return gemm_wide_bf16(x, w_gate_up, dual=True, activation=activation)
         if even and x.dtype == torch.bfloat16 and skinny_fits(x, w_gate_up) and _own_large(x, w_gate_up):
             return gemm_mfma_bf16(x, w_gate_up, dual=True, activation=activation)
