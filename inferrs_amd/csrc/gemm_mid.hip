@@ -456,12 +456,12 @@ static MidPlan mid_plan(int N, int K, bool dual) {
     }
     if (best.waves != 0 && best_fill >= 0.9) return best;
     // Four rounds and more of blocks of eight waves (a logits head): the rows of x are fetched half as often as by blocks of
-    // four, and three stages hide the memory better than a second block.  From 2,560 k on: below, 96 rows are slower and few rows no
-    // faster.  Five vocabularies of 131,072 to 262,144, weights not in a cache, the time of blocks of four / eight waves in the mean:
-    // 5,120 k 24 rows 1.05, 64 rows 1.08, 128 rows 1.21, 4,096 k 1.02, 1.08, 1.21, 2,560 k 1.04, 1.05, 1.24; 2,048 k 0.98, 1.01, 1.13
-    // and 96 rows 0.96 to 1.03; 1,024 k 1.03, 1.04, 1.16 and 96 rows 0.91 to 1.01 (151,936 features of 4,096 k, us: 24 rows 250 / 238,
-    // 64 rows 271 / 247, 128 rows 352 / 287).
-    if (!dual && K >= 2560 && tiles >= 4 * 8 * cus) return {8, 1, 3};
+    // four, and three stages hide the memory better than a second block.  The head alone, five vocabularies of 131,072 to 262,144, the
+    // time of blocks of four / eight waves in the mean: 5,120 k 24 rows 1.05, 64 rows 1.08, 128 rows 1.21, 4,096 k 1.02, 1.08, 1.21,
+    // 2,560 k 1.04, 1.05, 1.24.  Over a short k inside decode steps of two layers, the step by four / by eight: 1,024 k, 151,936 features,
+    // 20 rows 197 / 195 us, 64 rows 235 / 233, 96 rows 249 / 255, 128 rows 308 / 289, 2,048 k 278 / 278, 322 / 320, 351 / 347, 408 / 383;
+    // over four vocabularies 1.05 to 1.08 at 112 and 128 rows, up to 96 rows 0.96 (200,064 features of 1,024 k at 80 and 96) to 1.02.
+    if (!dual && tiles >= 4 * 8 * cus) return {8, 1, 3};
     MidPlan wide = {4, 1, 2};
     if (!dual) {
         const int blocks = (N + 63) / 64;

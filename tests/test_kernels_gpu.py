@@ -895,16 +895,16 @@ def test_mid_product(m, n, k):
 @pytest.mark.parametrize("m", [17, 64, 65, 128])
 @pytest.mark.parametrize("n", [131056, 131072, 131077])
 def test_mid_product_of_a_logits_head(m, n):
-    """Around the number of features from which the blocks of a long k have eight waves (131,057 and more on 256 compute units), rows
-    of both pipelines, features that fill no block: in the blocks that a short k has, and in blocks of eight waves."""
+    """Around the number of features from which the blocks have eight waves (131,057 and more on 256 compute units), rows of both
+    pipelines, features that fill no block: in the rule's blocks, and in blocks of four and of eight waves."""
     from inferrs_amd import ops
     k = 384
     x, w = dev(randn(m, k, dtype=torch.bfloat16, seed=m)), dev(randn(n, k, dtype=torch.bfloat16, seed=n, scale=0.05))
     want = x.float().cpu() @ w.float().cpu().t()
     lib = ops.library()
     try:
-        for waves in (0, 8):
-            assert lib.ia_gemm_mid_plan(waves, 1 if waves else 0, 3 if waves else 0) == 0
+        for waves, splits, stages in ((0, 0, 0), (4, 1, 2), (8, 1, 3)):
+            assert lib.ia_gemm_mid_plan(waves, splits, stages) == 0
             close(ops.gemm_mid_bf16(x, w, torch.float32), want, 2e-6 * math.sqrt(k), ("a head's logits", waves))
             close(ops.gemm_mid_bf16(x, w), want, 2 ** -8, ("a head's logits, stored in 16 bits", waves))
     finally:
