@@ -1165,14 +1165,15 @@ def add_rmsnorm_partials(x: torch.Tensor, delta: Partials, w: torch.Tensor, eps:
 
 def linear(x, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None, mid: bool = True,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x [m, k] . w[n, k]^T (+ bias [n], in the precision of w).  32-bit: `gemm_tiled` (true 32-bit, fixed
-    order).  bfloat16: the skinny MFMA kernel for up to SKINNY_MAX_ROWS rows, the vendor's GEMM beyond that (the
-    reference uses cuBLAS for all of them; products that `linear_partials` or `gated_linear` send to gemm_wide.hip do not come here).  A 32-bit result of bfloat16 operands (logits) comes straight from
-    the skinny kernel's accumulators for those few rows; beyond that it is the vendor's bfloat16
-    result widened, which is what the reference does for every row (its logits are computed in
-    the model's precision and cast for sampling, `inferrs/src/sampler.rs:182`).  From `mid_from_rows(k)` rows on (and up to
-    `MID_MAX_ROWS`) a bfloat16 result comes from gemm_mid.hip; `mid=False`: from the skinny product or the vendor's GEMM.  The skinny kernel adds a bias to its sums before it rounds them; behind every
-    other product a kernel of its own adds it to the stored rows."""
+    """x [m, k] . w[n, k]^T (+ bias [n], in the precision of w).  32-bit: `gemm_tiled` (true 32-bit, fixed order).
+    bfloat16: the skinny MFMA kernel for up to SKINNY_MAX_ROWS rows, the vendor's GEMM beyond that (the reference uses
+    cuBLAS for all of them; products that `linear_partials` or `gated_linear` send to gemm_wide.hip do not come here).
+    A 32-bit result of bfloat16 operands (logits) comes straight from the skinny kernel's accumulators for those few
+    rows; beyond that it is the vendor's bfloat16 result widened, which is what the reference does for every row (its
+    logits are computed in the model's precision and cast for sampling, `inferrs/src/sampler.rs:182`).  From
+    `mid_from_rows(k)` rows on (and up to `MID_MAX_ROWS`) a bfloat16 result comes from gemm_mid.hip; `mid=False`: from
+    the skinny product or the vendor's GEMM.  The skinny kernel adds a bias to its sums before it rounds them; behind
+    every other product a kernel of its own adds it to the stored rows."""
     out_dtype = out_dtype or x.dtype
     if bias is not None and (bias.dtype != w.dtype or bias.numel() != w.shape[0]):
         raise KernelError(f"linear: a bias of {bias.numel()} {bias.dtype} entries for a weight {tuple(w.shape)} {w.dtype}")

@@ -324,8 +324,8 @@ def test_captured_mixed_steps_equal_eager_ones(tiny, dtype):
 
 @pytest.mark.parametrize("dtype,bucket", [("float32", 64), ("bfloat16", 64), ("bfloat16", 32), ("bfloat16", 8)])
 def test_captured_mixed_steps_whose_runs_lie_in_different_buckets(tiny, dtype, bucket):
-    """A request decodes through buckets of 64 tokens (or fewer, so that bounds lie further apart than buckets) while portions beside it come from other buckets, shorter and longer than
-    its own: a captured step holds its launches' bounds, so a step of the same sizes in another pair of buckets is another
+    """A request decodes through buckets of 64 tokens (or fewer, so that bounds lie further apart than buckets) while portions
+    beside it come from other buckets, shorter and longer than its own: a captured step holds its launches' bounds, so a step of the same sizes in another pair of buckets is another
     graph.  Twice over the same way, so that every pair is met eagerly and replayed; the logits are those without graphs."""
     from inferrs_amd.engine import Engine, Entry
     folder, cfg, params = tiny["B"]
