@@ -335,7 +335,7 @@ extern "C" int ia_gemm_wide_norm_fits(int M, int N, int K) {
 // The same for the kernel that norms and turns queries and keys and writes the cache, up to 1,024 rows.  A product of q|k|v has many
 // features, so that the split gives less than above: over a short k the vendor's GEMM is as fast or faster (us a layer: 4B shape, 456
 // rows 241 / 244, 850 rows 332 / 336), over a long one this kernel, split or not (8B shape, 130 rows 251 / 236, 700 rows 436 / 420, 900
-// 484 / 475; 14B shape, 521 rows 625 / 605; 32B shape, 900 rows 1,105 / 1,085; of 46 points one, 14B shape at 768 rows, is slower, 740 / 742).
+// 484 / 475; 14B shape, 521 rows 625 / 605; 32B shape, 900 rows 1,105 / 1,085; of 69 points three are slower, by up to 0.4 %).
 extern "C" int ia_gemm_wide_rope_fits(int M, int N, int K) {
     if (M <= 0 || M > 1024 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
     return host_bound(M, K) || (K >= 4096 && (long long)N * K >= 4096LL * 5120);
@@ -345,8 +345,9 @@ extern "C" int ia_gemm_wide_rope_fits(int M, int N, int K) {
 // product cannot be split.  This kernel's own time has to come within a tenth of 1.22 PFLOP/s (or of 4 TB/s over the operands) and what
 // the second kernel takes; not where its blocks leave two fifths of their rounds empty (14B shape, 130 to 200 rows: 454 / 461, 468 / 474,
 // 534 / 544 us a layer) nor where the vendor's are nearly all work (4B shape, 768 rows, 287 / 298).  Elsewhere 8B shape, 200 rows 250 /
-// 243, 700 rows 436 / 412, 14B shape, 900 rows 934 / 831, 32B shape, 1,024 rows 1,222 / 1,167; where the rule says yes, at worst 0.985 of
-// the step's speed.
+// 243, 700 rows 436 / 412, 14B shape, 900 rows 934 / 831, 32B shape, 1,024 rows 1,222 / 1,167; of the 63 points of wide shapes where the
+// rule says yes ten are slower by more than half a percent, 1.2 at most.  It still refuses some that would gain (14B shape, 580 rows
+// 692 / 662, 32B shape, 400 rows 803 / 773).
 extern "C" int ia_gemm_wide_dual_fits(int M, int N, int K) {
     if (M <= 0 || M > 1024 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4 || ((long long)N + GW_BN) * K * 2 >= (1LL << 32)) return 0;
     const WidePlan plan = gw_plan(M, N, K, true, false);
