@@ -162,10 +162,13 @@ int ia_penalize(float* logits, int rows, int vocab, const int* window, int w, co
 int ia_window_push(int* window, int rows, int w, const int* caps, const int* tokens, hipStream_t stream);
 long long ia_sample_workspace(int rows, int vocab);
 int ia_sample_max_top(void);
+int ia_sample_narrow_top(void);                       // rows with a top_k of up to this many take the shorter way
 // n_top, lp_out [rows, 1 + max_top], lp_ids [rows, max_top]: all null, or the log-probabilities asked for per row
 int ia_sample(int* out, const float* logits, void* workspace, int rows, int vocab,
               const float* temperature, const int* top_k, const float* top_p, const float* min_p,
-              const float* u, const int* n_top, float* lp_out, int* lp_ids, hipStream_t stream);
+              const float* u, const int* n_top, float* lp_out, int* lp_ids, const int* window, int w,
+              const float* rep, const float* freq, const float* pres, const int* bias_ids, const float* bias_vals,
+              int nb, int narrow_only, hipStream_t stream);
 
 // ---- several residual streams a token (streams.hip) ------------------------------------------------------------
 // streams: 32-bit [n, S, W].  One call adds a sub-layer's output into the streams (x_t <- sum_s mix[s][t] x_s +

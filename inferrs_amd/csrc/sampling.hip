@@ -208,50 +208,87 @@ extern "C" int ia_argmax_static(int* out, const float* logits, int rows, int voc
 // ---- penalties ------------------------------------------------------------------------------
 // window [rows, w]: the last tokens of prompt and output, -1 where a row has fewer.
 // bias_ids / bias_vals [rows, nb]: -1 ends a row's list.
-__global__ void penalize_kernel(float* __restrict__ logits, int vocab, const int* __restrict__ window, int w,
-                                const float* __restrict__ rep, const float* __restrict__ freq,
-                                const float* __restrict__ pres, const int* __restrict__ bias_ids,
-                                const float* __restrict__ bias_vals, int nb) {
-    const int rowi = blockIdx.x;
-    float* row = logits + (size_t)rowi * vocab;
-    for (int j = threadIdx.x; j < nb; j += blockDim.x) {
-        const int id = bias_ids[(size_t)rowi * nb + j];
-        if (id >= 0 && id < vocab) atomicAdd(row + id, bias_vals[(size_t)rowi * nb + j]);
-    }
-    __syncthreads();
-    const int* win = window + (size_t)rowi * w;
-    const float rp = rep[rowi], fp = freq[rowi], pp = pres[rowi];
-    // one thread per distinct token: the one holding its first occurrence
+struct Penalties {
+    const int* window;
+    int w;
+    const float *rep, *freq, *pres;
+    const int* bias_ids;
+    const float* bias_vals;
+    int nb;
+    __host__ __device__ bool any() const { return w > 0 || nb > 0; }
+};
+
+#define PENALTY_STAGED 1024                         // entries of a window that a block keeps in shared memory
+
+// one thread per distinct token of the window: the one holding its first occurrence
+__device__ __forceinline__ void penalize_window(float* z, int lo, int n, const int* held, int w, float rp, float fp, float pp) {
     for (int j = threadIdx.x; j < w; j += blockDim.x) {
-        const int id = win[j];
-        if (id < 0 || id >= vocab) continue;
-        bool first = true;
-        int count = 0;
+        const int id = held[j];
+        if (id < lo || id - lo >= n) continue;
+        int before = 0, count = 0;
+#pragma unroll 8
         for (int i = 0; i < w; ++i) {
-            if (win[i] == id) {
-                if (i < j) { first = false; break; }
-                ++count;
-            }
+            const int same = held[i] == id ? 1 : 0;
+            before += i < j ? same : 0;
+            count += same;
         }
-        if (!first) continue;
-        float v = row[id];
+        if (before > 0) continue;
+        float v = z[id - lo];
         if (rp != 1.0f && rp != 0.0f) v = v >= 0.f ? v / rp : v * rp;
         if (fp != 0.0f || pp != 0.0f) {
             v -= fp * (float)count;
             v -= pp;
         }
-        row[id] = v;
+        z[id - lo] = v;
     }
+}
+
+// A row's window into shared memory (PENALTY_STAGED words at `s_win`); a barrier has to follow.
+__device__ __forceinline__ void stage_window(const Penalties& p, int rowi, int* s_win) {
+    if (p.w <= PENALTY_STAGED)
+        for (int j = threadIdx.x; j < p.w; j += blockDim.x) s_win[j] = p.window[(size_t)rowi * p.w + j];
+}
+
+// A row's bias and penalties on the logits of its tokens lo .. lo + n, which lie at z[0 .. n) (shared or global memory).
+// All threads of the block call it, with every z and the staged window written behind a barrier; it ends with one.
+__device__ __forceinline__ void penalize_range(float* z, int lo, int n, const Penalties& p, int rowi, const int* s_win) {
+    const int w = p.w;
+    const float rp = w > 0 ? p.rep[rowi] : 1.f, fp = w > 0 ? p.freq[rowi] : 0.f, pp = w > 0 ? p.pres[rowi] : 0.f;
+    if (p.nb > 0) {
+        for (int j = threadIdx.x; j < p.nb; j += blockDim.x) {
+            const int id = p.bias_ids[(size_t)rowi * p.nb + j];
+            if (id >= lo && id - lo < n) atomicAdd(z + (id - lo), p.bias_vals[(size_t)rowi * p.nb + j]);
+        }
+        __syncthreads();
+    }
+    if (w > PENALTY_STAGED) penalize_window(z, lo, n, p.window + (size_t)rowi * w, w, rp, fp, pp);
+    else penalize_window(z, lo, n, s_win, w, rp, fp, pp);
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(256) void penalize_kernel(float* __restrict__ logits, int vocab, const Penalties p) {
+    __shared__ int s_win[PENALTY_STAGED];
+    stage_window(p, blockIdx.x, s_win);
+    __syncthreads();
+    penalize_range(logits + (size_t)blockIdx.x * vocab, 0, vocab, p, blockIdx.x, s_win);
+}
+
+static int check_penalties(const char* who, const Penalties& p) {
+    IA_CHECK(p.w >= 0 && p.nb >= 0, "%s: bad sizes window=%d bias=%d", who, p.w, p.nb);
+    IA_CHECK(p.w == 0 || (p.window != nullptr && p.rep != nullptr && p.freq != nullptr && p.pres != nullptr),
+             "%s: a window of %d tokens without its arrays", who, p.w);
+    IA_CHECK(p.nb == 0 || (p.bias_ids != nullptr && p.bias_vals != nullptr), "%s: %d bias entries without their arrays", who, p.nb);
+    return 0;
 }
 
 extern "C" int ia_penalize(float* logits, int rows, int vocab, const int* window, int w, const float* rep,
                            const float* freq, const float* pres, const int* bias_ids, const float* bias_vals,
                            int nb, hipStream_t stream) {
-    IA_CHECK(rows >= 0 && vocab > 0 && w >= 0 && nb >= 0, "penalize: bad sizes rows=%d vocab=%d window=%d bias=%d", rows, vocab, w, nb);
-    IA_CHECK(w == 0 || window != nullptr, "penalize: a window of %d tokens without its array", w);
-    IA_CHECK(nb == 0 || (bias_ids != nullptr && bias_vals != nullptr), "penalize: %d bias entries without their arrays", nb);
-    if (rows == 0 || (w == 0 && nb == 0)) return 0;
-    penalize_kernel<<<rows, 256, 0, stream>>>(logits, vocab, window, w, rep, freq, pres, bias_ids, bias_vals, nb);
+    IA_CHECK(rows >= 0 && vocab > 0, "penalize: bad sizes rows=%d vocab=%d", rows, vocab);
+    const Penalties p = {window, w, rep, freq, pres, bias_ids, bias_vals, nb};
+    if (const int bad = check_penalties("penalize", p)) return bad;
+    if (rows == 0 || !p.any()) return 0;
+    penalize_kernel<<<rows, 256, 0, stream>>>(logits, vocab, p);
     IA_LAUNCH_CHECK("penalize");
     return 0;
 }
@@ -526,7 +563,8 @@ __device__ Cut top_k_cut(const uint32_t* __restrict__ keys, int n, int k, int* s
 
 // The reference's steps on the first k entries of a row's ordered list.  `keys` [n] holds the row's candidates in
 // the order of their tokens' indices (every stretch of the row has left its own first k there, so the row's first
-// k are among them), `token_of` [n] their tokens, `probs` the whole row's probabilities by token.
+// k are among them), `token_of` [n] their tokens (null: a candidate's place is its token), `probs` the whole row's
+// probabilities by token.
 // `open`: the row has no top_k; k tokens are only the beginning of its list, whose weight is `total`.  The steps
 // then succeed if top_p or min_p end the list within these k, or else the walk ends there; if not, nothing is
 // written and false comes back (the caller goes the long way).
@@ -567,11 +605,14 @@ __device__ bool sample_top_k(int* __restrict__ out, const uint32_t* __restrict__
         }
     __syncthreads();
     __shared__ float cprob[SAMPLE_FAST_K];
-    for (int i = threadIdx.x; i < n; i += blockDim.x) cprob[i] = probs[token_of[(int)~(uint32_t)(cand[i] & 0xffffffffull)]];
+    auto index_of = [&](int i) {
+        const int place = (int)~(uint32_t)(cand[i] & 0xffffffffull);
+        return token_of != nullptr ? token_of[place] : place;
+    };
+    for (int i = threadIdx.x; i < n; i += blockDim.x) cprob[i] = probs[index_of(i)];
     __syncthreads();
     if (threadIdx.x == 0) {
         // ---- the reference's steps 7 to 12 on its sorted list
-        auto index_of = [&](int i) { return token_of[(int)~(uint32_t)(cand[i] & 0xffffffffull)]; };
         bool ended = !open, done = true;                    // ended: the list's end lies within these n tokens
         int len = n;
         if (tp < 1.0f) {
@@ -644,11 +685,19 @@ __device__ bool sample_top_k(int* __restrict__ out, const uint32_t* __restrict__
 //     first k entries of the ordered list (k: the row's top_k, or SAMPLE_FAST_K for a row without one), written
 //     in the order of their tokens at a place that follows from k and the stretches' lengths alone;
 //   then one block a row (sample_kernel) picks the row's first k among those candidates and walks them.
-// A row's words: keys [vocab], probabilities [vocab], the candidates' keys and tokens [stretches * SAMPLE_FAST_K]
-// each, and the stretches' maxima, sums and sums of probabilities [stretches] each.
+// Rows with a top_k of up to SAMPLE_NARROW_K ("narrow" ones; the reference's default is 50) need no second pass: the
+// first leaves those of its stretch's logits that can be among the row's first k (see narrow_candidates), the last
+// block works out their probabilities alone.  24 rows of 151,936 logits with the default parameters: 86 us of kernels,
+// of them the second pass 36 (16 bytes written a logit, three histograms of keys that mostly fall into one bin) and the
+// last 28 (three more of them and one thread's walk through shared memory), before; 30 now, 16 and 13.
+// Bias and penalties are applied where a stretch's logits are read; the caller's logits stay as they are.
+// A row's words: keys [vocab], probabilities [vocab], the candidates' keys (narrow rows: their logits over the
+// temperature) and tokens [stretches * SAMPLE_FAST_K] each, and the stretches' maxima, sums and sums of probabilities
+// (narrow rows: numbers of candidates) [stretches] each.
 #define SAMPLE_STRETCH 4096
 #define SAMPLE_STAGED 8192              // candidates of a row that its last block keeps in shared memory
 #define SAMPLE_MAX_STRETCHES 1024       // the stretches' sums meet in a block's shared memory: 4 M tokens a row
+#define SAMPLE_NARROW_K 64
 struct RowLayout {
     int vocab, stretches, stretch;      // stretch: tokens a stretch (the last one may be shorter), a multiple of 4
     long long words;                    // of a row
@@ -669,6 +718,7 @@ struct RowLayout {
     __device__ float* part_max(uint32_t* ws, int row) const { return (float*)(cand_tokens(ws, row) + (size_t)stretches * SAMPLE_FAST_K); }
     __device__ float* part_sum(uint32_t* ws, int row) const { return part_max(ws, row) + stretches; }
     __device__ float* part_total(uint32_t* ws, int row) const { return part_sum(ws, row) + stretches; }
+    __device__ int* part_count(uint32_t* ws, int row) const { return (int*)part_total(ws, row); }
 };
 
 static RowLayout row_layout(int vocab) {
@@ -691,72 +741,191 @@ __device__ __forceinline__ bool row_temperature(const float* temperature, const 
     return true;
 }
 
+// Lane i's value, i the same for all lanes: no trip through shared memory.
+__device__ __forceinline__ float lane_value(float v, int i) { return __uint_as_float((uint32_t)__builtin_amdgcn_readlane(__float_as_int(v), i)); }
+
 // The row's maximum, the sum of exp(z / temperature - maximum) and (with `with_total`) the sum of the probabilities
 // from the stretches' (a stretch of nothing but -inf adds nothing to the sum); every block that asks gets the same bits.
-// `s_parts`: 3 * stretches floats of shared memory.  All threads of the block call it.
+// All threads of the block call it; the first wave does the work, a stretch a lane, and adds up in order through scalar
+// registers (every thread adding them up out of shared memory kept its reads busy for 2 us of the last block's time).
 struct RowSums { float mx, sum, total; };
-__device__ RowSums row_sums(const RowLayout& l, uint32_t* ws, int rowi, bool with_total, float* s_parts) {
-    const float* parts = l.part_max(ws, rowi);               // maxima, sums, totals: one after the other
-    const int n = (with_total ? 3 : 2) * l.stretches;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s_parts[i] = parts[i];
+__device__ RowSums row_sums(const RowLayout& l, uint32_t* ws, int rowi, bool with_total) {
+    __shared__ RowSums s_sums;
+    if (threadIdx.x < IA_WAVE) {
+        const float *maxima = l.part_max(ws, rowi), *sums = l.part_sum(ws, rowi), *totals = l.part_total(ws, rowi);
+        const int lane = threadIdx.x;
+        RowSums r;
+        r.mx = -INFINITY;
+        float first_m = -INFINITY, first_s = 0.f, first_t = 0.f;      // (the first 64 stretches' are read once)
+        if (lane < l.stretches) {
+            first_m = maxima[lane];
+            first_s = sums[lane];
+            if (with_total) first_t = totals[lane];
+        }
+        for (int b = lane; b < l.stretches; b += IA_WAVE) r.mx = fmaxf(r.mx, b == lane ? first_m : maxima[b]);
+        r.mx = wave_max(r.mx);
+        r.sum = r.total = 0.f;
+        for (int b0 = 0; b0 < l.stretches; b0 += IA_WAVE) {
+            const int b = b0 + lane;
+            float m = first_m, a = first_s, t = first_t;
+            if (b0 > 0) {
+                m = b < l.stretches ? maxima[b] : -INFINITY;
+                a = b < l.stretches ? sums[b] : 0.f;
+                t = with_total && b < l.stretches ? totals[b] : 0.f;
+            }
+            const float e = m > -INFINITY ? expf(m - r.mx) : 0.f;
+            const unsigned long long counts = __ballot(m > -INFINITY);
+            const int here = l.stretches - b0 < IA_WAVE ? l.stretches - b0 : IA_WAVE;
+            for (int i = 0; i < here; ++i) {
+                if ((counts >> i) & 1) r.sum = fmaf(lane_value(a, i), lane_value(e, i), r.sum);
+                if (with_total) r.total += lane_value(t, i);
+            }
+        }
+        if (lane == 0) s_sums = r;
+    }
     __syncthreads();
-    RowSums r;
-    r.mx = -INFINITY;
-    for (int b = 0; b < l.stretches; ++b) r.mx = fmaxf(r.mx, s_parts[b]);
-    r.sum = 0.f;
-    for (int b = 0; b < l.stretches; ++b)
-        if (s_parts[b] > -INFINITY) r.sum += s_parts[l.stretches + b] * expf(s_parts[b] - r.mx);
-    r.total = 0.f;
-    if (with_total)
-        for (int b = 0; b < l.stretches; ++b) r.total += s_parts[2 * l.stretches + b];
-    __syncthreads();
-    return r;
+    return s_sums;
 }
 
+// A stretch's logits into shared memory, with the row's bias and penalties.  All threads of the block call it; it ends with a barrier.
+__device__ __forceinline__ void load_stretch(float* s_z, const float* __restrict__ logits, const RowLayout& l, int rowi, int b,
+                                             const Penalties& pen, int* s_win) {
+    const int lo = b * l.stretch, n = l.length(b);
+    const float* row = logits + (size_t)rowi * l.vocab + lo;
+    stage_window(pen, rowi, s_win);
+    if (((uintptr_t)row & 15) == 0) {
+        // all of a thread's pieces of four under way together
+        constexpr int PER = SAMPLE_STRETCH / 4 / 256;
+        float4 v[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int c = (j * 256 + (int)threadIdx.x) * 4;
+            v[j] = c + 4 <= n ? *(const float4*)(row + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int c = (j * 256 + (int)threadIdx.x) * 4;
+            if (c + 4 <= n) *(float4*)(s_z + c) = v[j];
+        }
+        const int rest = (n & ~3) + (int)threadIdx.x;
+        if (rest < n) s_z[rest] = row[rest];
+    } else {
+        constexpr int PER = SAMPLE_STRETCH / 256;
+        float v[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int c = j * 256 + (int)threadIdx.x;
+            v[j] = c < n ? row[c] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int c = j * 256 + (int)threadIdx.x;
+            if (c < n) s_z[c] = v[j];
+        }
+    }
+    __syncthreads();
+    if (pen.any()) penalize_range(s_z, lo, n, pen, rowi, s_win);
+}
+
+__device__ __forceinline__ bool is_narrow(int k, int vocab, int fast) { return fast == 1 && k > 0 && k < vocab && k <= SAMPLE_NARROW_K; }
+
+// Those of a stretch's logits that can be among the row's first k tokens, k <= SAMPLE_NARROW_K, ordered by their
+// rounded probabilities p = exp(y - the row's maximum) / the row's sum and by index where these are equal; y, the logits over the
+// temperature.  Of the 128 pairs of threads k hold a maximum of at least Y, the k-th largest of these
+// maxima.  A y under Y by NARROW_MARGIN has k tokens of its stretch strictly before it as long as its p is no denormal: the
+// difference y - maximum is off by 4e-6 at most (up to 128 away; p vanishes beyond 104), the exponential by two units in
+// the last place and the quotient by half of one, 3e-7 of p together, so that p's of tokens 2e-5 apart cannot meet.  (The
+// margin is twice that, for the rounding of Y - margin; where y is so large that the margin is below its spacing, tokens under Y
+// are a whole unit in the last place of y below it.)  A y of NARROW_DEPTH under the stretch's maximum has a p under
+// NARROW_FLOOR.  The last block takes no token whose p is under the floor from these candidates (sample_narrow), so
+// both may be left out.  SAMPLE_FAST_K places; a stretch with more candidates (equal logits in great number) says so by its count.
+#define NARROW_MARGIN 4e-5f
+#define NARROW_DEPTH 88.0f              // exp(-88) = 6e-39, a sixteenth of a hundredth of the floor
+#define NARROW_FLOOR 1e-36f
+
+// Bound by the trip to the memory, a logit's division and exponential, and the barriers between its phases; several blocks a
+// compute unit hide each other's.
 __global__ __launch_bounds__(256) void sample_partials_kernel(const float* __restrict__ logits, uint32_t* __restrict__ workspace,
                                                               const RowLayout l, const float* __restrict__ temperature,
-                                                              const int* __restrict__ n_top) {
-    __shared__ float scratch[32];
-    const int rowi = blockIdx.y, b = blockIdx.x;
+                                                              const int* __restrict__ top_k, const int* __restrict__ n_top,
+                                                              const Penalties pen, int fast) {
+    __shared__ __attribute__((aligned(16))) float s_z[SAMPLE_STRETCH];
+    __shared__ int s_win[PENALTY_STAGED];
+    __shared__ __attribute__((aligned(16))) uint32_t s_group[128];
+    __shared__ float s_max[256 / IA_WAVE], s_sum[256 / IA_WAVE];
+    __shared__ uint32_t s_kth;
+    __shared__ int s_n;
+    constexpr int PER = SAMPLE_STRETCH / 256;
+    const int rowi = blockIdx.y, b = blockIdx.x, t = threadIdx.x, wave = t / IA_WAVE;
+    const int k = top_k[rowi];
     float temp;
     if (!row_temperature(temperature, n_top, rowi, temp)) return;
-    const float* row = logits + (size_t)rowi * l.vocab + (size_t)b * l.stretch;
+    const bool narrow = is_narrow(k, l.vocab, fast);
     const int n = l.length(b);
-    // temperature, and the softmax's two sums (sampler.rs:232-249); four loads under way
-    float mx = -INFINITY;
-    for (int c0 = threadIdx.x; c0 < n; c0 += 4 * blockDim.x) {
-        float z[4];
+    if (t == 0) { s_kth = 0u; s_n = 0; }
+    load_stretch(s_z, logits, l, rowi, b, pen, s_win);
+    // temperature, and the softmax's two sums (sampler.rs:232-249)
+    float y[PER], mx = -INFINITY;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int c = c0 + j * (int)blockDim.x;
-            z[j] = c < n ? row[c] : -INFINITY;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (c0 + j * (int)blockDim.x < n) mx = fmaxf(mx, z[j] / temp);
+    for (int j = 0; j < PER; ++j) {
+        const int c = t + j * 256;
+        y[j] = c < n ? s_z[c] / temp : -INFINITY;
+        mx = fmaxf(mx, y[j]);
     }
+    // (the keys of the pairs' maxima; a NaN is no maximum, and a row that holds one is not settled by candidates)
+    const uint32_t mine = order_key(fmaxf(mx, __shfl_xor(mx, 1, IA_WAVE)));
+    if ((t & 1) == 0) s_group[t >> 1] = mine;
     mx = wave_max(mx);
-    if ((threadIdx.x & (IA_WAVE - 1)) == 0) scratch[16 + threadIdx.x / IA_WAVE] = mx;
+    if ((t & (IA_WAVE - 1)) == 0) s_max[wave] = mx;
     __syncthreads();
-    for (int w = 0; w < (int)(blockDim.x / IA_WAVE); ++w) mx = fmaxf(mx, scratch[16 + w]);
+    for (int w = 0; w < 256 / IA_WAVE; ++w) mx = fmaxf(mx, s_max[w]);
     float sum = 0.f;
-    if (mx > -INFINITY)
-        for (int c0 = threadIdx.x; c0 < n; c0 += 4 * blockDim.x) {
-            float z[4];
+    if (mx > -INFINITY) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int c = c0 + j * (int)blockDim.x;
-                z[j] = c < n ? row[c] : 0.f;
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (c0 + j * (int)blockDim.x < n) sum += expf(z[j] / temp - mx);
-        }
-    sum = block_sum(sum, scratch);
-    if (threadIdx.x == 0) {
-        l.part_max(workspace, rowi)[b] = mx;
-        l.part_sum(workspace, rowi)[b] = sum;
+        for (int j = 0; j < PER; ++j)
+            if (t + j * 256 < n) sum += expf(y[j] - mx);
     }
+    sum = wave_sum(sum);
+    if ((t & (IA_WAVE - 1)) == 0) s_sum[wave] = sum;
+    if (narrow) {
+        // a pair's rank among the pairs, half of the comparisons each
+        int before = 0;
+#pragma unroll
+        for (int i = 0; i < 64; i += 4) {
+            const int at = (t & 1) * 64 + i;
+            const uint4 g = *(const uint4*)(s_group + at);
+            const uint32_t e[4] = {g.x, g.y, g.z, g.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) before += (e[q] > mine || (e[q] == mine && at + q < (t >> 1))) ? 1 : 0;
+        }
+        before += __shfl_xor(before, 1, IA_WAVE);
+        if (before == k - 1 && (t & 1) == 0) s_kth = mine;
+    }
+    __syncthreads();
+    if (t == 0) {
+        float total = 0.f;
+        for (int w = 0; w < 256 / IA_WAVE; ++w) total += s_sum[w];
+        l.part_max(workspace, rowi)[b] = mx;
+        l.part_sum(workspace, rowi)[b] = total;
+    }
+    if (!narrow) return;
+    uint32_t* cand_y = l.cand_keys(workspace, rowi) + (size_t)b * SAMPLE_FAST_K;
+    int* cand_token = l.cand_tokens(workspace, rowi) + (size_t)b * SAMPLE_FAST_K;
+    const uint32_t kth = s_kth;
+    const float least = fmaxf(__uint_as_float((kth & 0x80000000u) ? kth & 0x7fffffffu : ~kth) - NARROW_MARGIN, mx - NARROW_DEPTH);
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int c = t + j * 256;
+        if (c < n && y[j] >= least && y[j] > -INFINITY) {
+            const int slot = atomicAdd(&s_n, 1);
+            if (slot < SAMPLE_FAST_K) {
+                cand_y[slot] = __float_as_uint(y[j]);
+                cand_token[slot] = b * l.stretch + c;
+            }
+        }
+    }
+    __syncthreads();
+    if (t == 0) l.part_count(workspace, rowi)[b] = s_n;
 }
 
 // How many entries of a row's ordered list are picked out before the reference's steps run on them: the row's
@@ -771,20 +940,22 @@ __device__ __forceinline__ int picked_out(int k, int vocab, int fast_top_k) {
 #define STRETCH_THREADS 256
 __global__ __launch_bounds__(STRETCH_THREADS) void sample_stretch_kernel(
     const float* __restrict__ logits, uint32_t* __restrict__ workspace, const RowLayout l,
-    const float* __restrict__ temperature, const int* __restrict__ top_k, const int* __restrict__ n_top, int fast_top_k) {
+    const float* __restrict__ temperature, const int* __restrict__ top_k, const int* __restrict__ n_top, const Penalties pen,
+    int fast_top_k) {
     __shared__ float scratch[32];
     __shared__ int s_counts[STRETCH_THREADS];
     __shared__ int s_waves[STRETCH_THREADS / IA_WAVE];
-    __shared__ uint32_t s_keys[SAMPLE_STRETCH];             // the stretch's keys: the choice below reads them several times
-    __shared__ float s_parts[2 * SAMPLE_MAX_STRETCHES];
+    __shared__ __attribute__((aligned(16))) uint32_t s_keys[SAMPLE_STRETCH];   // the stretch's logits, then its keys: the choice below reads them several times
+    __shared__ int s_win[PENALTY_STAGED];
     const int rowi = blockIdx.y, b = blockIdx.x;
     float temp;
     if (!row_temperature(temperature, n_top, rowi, temp)) return;
+    if (is_narrow(top_k[rowi], l.vocab, fast_top_k)) return;
     const int lo = b * l.stretch, n = l.length(b);
-    const float* row = logits + (size_t)rowi * l.vocab + lo;
+    load_stretch((float*)s_keys, logits, l, rowi, b, pen, s_win);
     uint32_t* keys = l.keys(workspace, rowi) + lo;
     float* probs = l.probs(workspace, rowi) + lo;
-    const RowSums rs = row_sums(l, workspace, rowi, false, s_parts);
+    const RowSums rs = row_sums(l, workspace, rowi, false);
     // The list is ordered by the probabilities themselves, as the reference sorts them: logits whose
     // probabilities round to the same number (or vanish together) are ties, taken in index order.
     float t = 0.f;
@@ -793,7 +964,7 @@ __global__ __launch_bounds__(STRETCH_THREADS) void sample_stretch_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int c = c0 + j * (int)blockDim.x;
-            z[j] = c < n ? row[c] : 0.f;
+            z[j] = c < n ? __uint_as_float(s_keys[c]) : 0.f;
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -851,6 +1022,155 @@ __global__ __launch_bounds__(STRETCH_THREADS) void sample_stretch_kernel(
     }
 }
 
+// The reference's steps (sampler.rs:251-335) on a narrow row: the candidates' probabilities, the first k of them in order
+// and the walk, with the sums in the reference's order.  False, and nothing that counts is written, where the candidates
+// do not settle the row: a stretch had more than its places, there is a NaN or no number to start from, or the draw (or
+// an entry that is reported) lies among probabilities under the floor, whose order and ties the candidates do not hold.
+// A block of 1,024 threads; all of them call it.
+// One block a row, so the time is a chain: one trip to the memory (a wave takes the stretches wave, wave + 16, ...; the first
+// 128 candidates of three of them are asked for before their number is known, the places exist), five barriers, and the
+// reference's running sums over up to 64 values, which go lane by lane through a scalar register (through shared memory a step
+// took 100 cycles).
+__device__ bool sample_narrow(int* __restrict__ out, const RowLayout& l, uint32_t* __restrict__ ws, int rowi, int k,
+                              float tp, float mp, float u, int want_top, float* __restrict__ lp_out, int* __restrict__ lp_ids) {
+    __shared__ unsigned long long s_list[SAMPLE_FAST_K];    // (key, ~token): larger is earlier in the list
+    __shared__ unsigned long long s_first[SAMPLE_NARROW_K];
+    __shared__ __attribute__((aligned(16))) uint32_t s_group[128];
+    __shared__ uint32_t s_kth;
+    __shared__ int s_n, s_over, s_settled;
+    const int t = threadIdx.x, lane = t & (IA_WAVE - 1), wave = t / IA_WAVE;
+    const uint32_t* cand_y = l.cand_keys(ws, rowi);
+    const int* cand_token = l.cand_tokens(ws, rowi);
+    const int* counts = l.part_count(ws, rowi);
+    if (t == 0) { s_n = 0; s_over = 0; s_kth = 0u; s_settled = 0; }
+    constexpr int KEEP = 3, WAVES = SAMPLE_THREADS / IA_WAVE;
+    uint32_t key[KEEP][2];
+    int token[KEEP][2], held[KEEP];
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) {
+        const int b = wave + i * WAVES;
+        const int from = b < l.stretches ? b : 0;
+        held[i] = b < l.stretches ? counts[from] : 0;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            key[i][h] = cand_y[(size_t)from * SAMPLE_FAST_K + h * IA_WAVE + lane];
+            token[i][h] = cand_token[(size_t)from * SAMPLE_FAST_K + h * IA_WAVE + lane];
+        }
+    }
+    const RowSums rs = row_sums(l, ws, rowi, false);
+    auto probability = [&](uint32_t y) {
+        const float e = expf(__uint_as_float(y) - rs.mx);
+        return rs.sum > 0.f ? e / rs.sum : e;
+    };
+    uint32_t mine = 0u;
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            key[i][h] = h * IA_WAVE + lane < held[i] ? order_key(probability(key[i][h])) : 0u;
+            mine = key[i][h] > mine ? key[i][h] : mine;
+        }
+    // the k-th largest of 128 groups' maxima: at least k candidates are no smaller
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+        const uint32_t other = (uint32_t)__shfl_xor((int)mine, o, IA_WAVE);
+        mine = other > mine ? other : mine;
+    }
+    if ((t & 7) == 0) s_group[t >> 3] = mine;
+    __syncthreads();
+    int before = 0;
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+        const int at = (t & 7) * 16 + i;
+        const uint4 g = *(const uint4*)(s_group + at);
+        const uint32_t e[4] = {g.x, g.y, g.z, g.w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) before += (e[q] > mine || (e[q] == mine && at + q < (t >> 3))) ? 1 : 0;
+    }
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) before += __shfl_xor(before, o, IA_WAVE);
+    if (before == k - 1 && (t & 7) == 0) s_kth = mine;
+    __syncthreads();
+    const uint32_t kth = s_kth;
+    auto take = [&](uint32_t ky, int tok) {
+        if (ky == 0u || ky < kth) return;
+        const int slot = atomicAdd(&s_n, 1);
+        if (slot < SAMPLE_FAST_K) s_list[slot] = ((unsigned long long)ky << 32) | (uint32_t)~(uint32_t)tok;
+    };
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) take(key[i][h], token[i][h]);
+    // what the registers did not hold: candidates beyond 128 of a stretch, stretches beyond 48
+    for (int b = wave, i = 0; b < l.stretches; b += WAVES, ++i) {
+        const int all = counts[b], end = all < SAMPLE_FAST_K ? all : SAMPLE_FAST_K;
+        if (all > SAMPLE_FAST_K && lane == 0) s_over = 1;
+        for (int at = (i < KEEP ? 2 * IA_WAVE : 0) + lane; at < end; at += IA_WAVE)
+            take(order_key(probability(cand_y[(size_t)b * SAMPLE_FAST_K + at])), cand_token[(size_t)b * SAMPLE_FAST_K + at]);
+    }
+    __syncthreads();
+    const int found = s_n;
+    if (s_over || found > SAMPLE_FAST_K || found == 0 || !(rs.mx > -INFINITY && rs.mx < INFINITY) || !(rs.sum > 0.f && rs.sum < INFINITY))
+        return false;
+    // an entry's place is the number of larger ones (no two are equal: a token has one entry)
+    if (t < found) {
+        const unsigned long long e = s_list[t];
+        int place = 0;
+#pragma unroll 8
+        for (int i = 0; i < found; ++i) place += s_list[i] > e ? 1 : 0;
+        if (place < k) s_first[place] = e;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const int n = found < k ? found : k;
+        const unsigned long long e = lane < n ? s_first[lane] : 0ull;
+        const float p = lane < n ? __uint_as_float((uint32_t)(e >> 32) & 0x7fffffffu) : 0.f;     // (a probability's sign bit is 0)
+        const int id = (int)~(uint32_t)(e & 0xffffffffull);
+        int len = n;
+        float filtered = 0.f;
+        for (int i = 0; i < n; ++i) {
+            filtered += lane_value(p, i);
+            if (tp < 1.0f && filtered >= tp) { len = i + 1; break; }
+        }
+        if (mp > 0.0f) {
+            const unsigned long long under = __ballot(lane < len && !(p >= lane_value(p, 0) * mp));
+            const int cut = under ? __ffsll((long long)under) - 1 : len;
+            if (cut > 0 && cut < len) {
+                len = cut;
+                filtered = 0.f;
+                for (int i = 0; i < len; ++i) filtered += lane_value(p, i);
+            }
+        }
+        const float norm = p / filtered;
+        float rng = u;
+        int at = -1;
+        for (int i = 0; i < len; ++i) {
+            const float step = lane_value(norm, i);
+            if (rng < step) { at = i; break; }
+            rng -= step;
+        }
+        // (a list that ends before its k-th token for want of candidates ends in tokens under the floor)
+        bool settled = filtered > 0.f && (at >= 0 || n == k);
+        if (at < 0) at = len - 1;
+        const int shown = want_top < SAMPLE_MAX_TOP ? want_top : SAMPLE_MAX_TOP;
+        settled = settled && lane_value(p, at) >= NARROW_FLOOR;
+        if (shown > 0) settled = settled && (len >= shown || n == k || len < n) && lane_value(p, (shown < len ? shown : len) - 1) >= NARROW_FLOOR;
+        if (settled) {
+            if (want_top >= 0) {
+                if (lane < shown && lane < len) {
+                    lp_ids[(size_t)rowi * SAMPLE_MAX_TOP + lane] = id;
+                    lp_out[(size_t)rowi * (1 + SAMPLE_MAX_TOP) + 1 + lane] = p > 0.f ? logf(norm) : -INFINITY;
+                }
+                if (lane == at) lp_out[(size_t)rowi * (1 + SAMPLE_MAX_TOP)] = p > 0.f ? logf(norm) : -INFINITY;
+            }
+            if (lane == at) out[rowi] = id;
+            if (lane == 0) s_settled = 1;
+        }
+    }
+    __syncthreads();
+    return s_settled != 0;
+}
+
 // n_top (may be null): per row -1 = no log-probabilities, else how many of the list's first entries are
 // reported besides the drawn token's (sampler.rs:285-352).  lp_out [rows, 1 + SAMPLE_MAX_TOP]: the drawn
 // token's log-probability within the kept list, then the entries'; lp_ids [rows, SAMPLE_MAX_TOP]: their ids (-1: none).
@@ -858,7 +1178,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     int* __restrict__ out, const float* __restrict__ logits, uint32_t* __restrict__ workspace, const RowLayout l,
     const float* __restrict__ temperature, const int* __restrict__ top_k, const float* __restrict__ top_p,
     const float* __restrict__ min_p, const float* __restrict__ u, const int* __restrict__ n_top,
-    float* __restrict__ lp_out, int* __restrict__ lp_ids, int fast_top_k) {
+    float* __restrict__ lp_out, int* __restrict__ lp_ids, const Penalties pen, int fast_top_k, int narrow_only) {
     __shared__ float scratch[32];
     __shared__ int s_counts[SAMPLE_THREADS];
     __shared__ float sv[16];
@@ -871,18 +1191,51 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         lp_ids[(size_t)rowi * SAMPLE_MAX_TOP + threadIdx.x] = -1;
         lp_out[(size_t)rowi * (1 + SAMPLE_MAX_TOP) + 1 + threadIdx.x] = -INFINITY;
     }
+    uint32_t* keys = l.keys(workspace, rowi);
+    float* probs = l.probs(workspace, rowi);
+    __shared__ int s_win[PENALTY_STAGED];
+    // The row's logits with its bias and penalties, in the keys' place.
+    auto touched_row = [&]() {
+        float* z = (float*)keys;
+        stage_window(pen, rowi, s_win);
+        for (int c = threadIdx.x; c < vocab; c += blockDim.x) z[c] = row[c];
+        __syncthreads();
+        if (pen.any()) penalize_range(z, 0, vocab, pen, rowi, s_win);
+        return z;
+    };
+    // (all of a row's parameters are asked for at once: one after the other each is a trip to the memory)
+    const int k = top_k[rowi];
+    const float tp = top_p[rowi], mp = min_p[rowi], draw = u[rowi];
     float temp;
     if (!row_temperature(temperature, n_top, rowi, temp)) {
-        argmax_row(row, vocab, sv, si, out + rowi);
+        int touched = 0;
+        for (int i = threadIdx.x; i < pen.w; i += blockDim.x) touched |= pen.window[(size_t)rowi * pen.w + i] >= 0;
+        for (int i = threadIdx.x; i < pen.nb; i += blockDim.x) touched |= pen.bias_ids[(size_t)rowi * pen.nb + i] >= 0;
+        argmax_row(__syncthreads_or(touched) ? touched_row() : row, vocab, sv, si, out + rowi);
         return;
     }
-    const uint32_t* keys = l.keys(workspace, rowi);
-    const float* probs = l.probs(workspace, rowi);
-    __shared__ float s_parts[3 * SAMPLE_MAX_STRETCHES];
-    const RowSums rs = row_sums(l, workspace, rowi, true, s_parts);
-    const float sum = rs.sum, total = rs.total;             // total: the weight of the whole list
+    const bool narrow = is_narrow(k, vocab, fast_top_k);
+    if (narrow && sample_narrow(out, l, workspace, rowi, k, tp, mp, draw, want_top, lp_out, lp_ids)) return;
+    const bool listed = !narrow && !narrow_only;            // the second pass has been over the row
+    __syncthreads();
+    const RowSums rs = row_sums(l, workspace, rowi, listed);
+    const float sum = rs.sum;
+    float total = rs.total;                                 // the weight of the whole list
+    if (!listed) {
+        // what the second pass leaves, by this block alone
+        const float* z = touched_row();
+        total = 0.f;
+        for (int c = threadIdx.x; c < vocab; c += blockDim.x) {
+            const float e = expf(z[c] / temp - rs.mx);
+            const float pr = sum > 0.f ? e / sum : e;
+            probs[c] = pr;
+            keys[c] = order_key(pr);
+            total += pr;
+        }
+        total = block_sum(total, scratch);
+        __syncthreads();
+    }
 
-    const int k = top_k[rowi];
     const int picked = picked_out(k, vocab, fast_top_k);
     if (picked > 0) {
         // the list's first entries: the row's top_k, or, without one, 1,024 tokens, which hold the nucleus, the min_p
@@ -890,27 +1243,25 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         const bool open = !(k > 0 && k < vocab);
         // (few candidates are read from shared memory: the choice among them reads them several times)
         __shared__ uint32_t s_cand[SAMPLE_STAGED];
-        const int n_cand = l.candidates(picked);
-        const uint32_t* cand_keys = l.cand_keys(workspace, rowi);
+        const int n_cand = listed ? l.candidates(picked) : vocab;
+        const uint32_t* cand_keys = listed ? l.cand_keys(workspace, rowi) : keys;
         if (n_cand <= SAMPLE_STAGED) {
             for (int i = threadIdx.x; i < n_cand; i += blockDim.x) s_cand[i] = cand_keys[i];
             __syncthreads();
             cand_keys = s_cand;
         }
-        if (sample_top_k(out, cand_keys, l.cand_tokens(workspace, rowi), probs, n_cand, rowi,
-                         picked, open, total, top_p[rowi], min_p[rowi], u[rowi], want_top, lp_out, lp_ids, s_counts))
+        if (sample_top_k(out, cand_keys, listed ? l.cand_tokens(workspace, rowi) : nullptr, probs, n_cand, rowi,
+                         picked, open, total, tp, mp, draw, want_top, lp_out, lp_ids, s_counts))
             return;
     }
     // how long the kept prefix is (sampler.rs:256-283)
     int keep = vocab;
     if (k > 0 && k < keep) keep = k;
-    const float tp = top_p[rowi];
     if (tp < 1.0f) {
         const Prefix p = shortest_prefix(keys, probs, vocab, tp, false, false, scratch);
         const int n = p.above + p.take;
         if (n < keep) keep = n;
     }
-    const float mp = min_p[rowi];
     if (mp > 0.0f) {
         const float thr = (sum > 0.f ? 1.0f / sum : 1.0f) * mp;       // the largest probability is exp(0) / sum
         float n = 0.f;
@@ -945,11 +1296,11 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     // the walk (sampler.rs:323-335): the first place where the running sum of p / filtered exceeds u
     int token;
     if (!(filtered > 0.f)) {
-        argmax_row(row, vocab, sv, si, out + rowi);
+        argmax_row(pen.any() ? touched_row() : row, vocab, sv, si, out + rowi);
         if (want_top >= 0 && threadIdx.x == 0) lp_out[(size_t)rowi * (1 + SAMPLE_MAX_TOP)] = -INFINITY;
         return;
     }
-    const Prefix hit = shortest_prefix(keys, probs, vocab, u[rowi] * filtered, false, true, scratch);
+    const Prefix hit = shortest_prefix(keys, probs, vocab, draw * filtered, false, true, scratch);
     if (keep < vocab && (hit.ties == 0 || hit.above + hit.take > keep)) {
         token = nth_with_key(keys, vocab, kept.key, kept.take, s_counts);          // the last kept token
     } else if (hit.ties == 0) {
@@ -1002,29 +1353,40 @@ extern "C" long long ia_sample_workspace(int rows, int vocab) {
 }
 
 static int g_sample_fast = 1;
-// Measurement and test switch: 0 sends rows with a top_k through the bisections as well.
+// Measurement and test switch: 0 sends rows with a top_k through the bisections as well, 2 narrow ones the way of other rows
+// with a top_k.
 extern "C" void ia_sample_tune(int fast_top_k) { g_sample_fast = fast_top_k; }
 
 extern "C" int ia_sample_max_top(void) { return SAMPLE_MAX_TOP; }
+extern "C" int ia_sample_narrow_top(void) { return SAMPLE_NARROW_K; }
 
-// n_top, lp_out, lp_ids: all null, or all given (see sample_kernel).
+// n_top, lp_out, lp_ids: all null, or all given (see sample_kernel).  window .. nb: bias and penalties as in ia_penalize
+// (w = nb = 0: none), on the way; the logits stay as they are.  `narrow_only`: the caller knows that every row has a top_k of
+// 1 .. ia_sample_narrow_top() below vocab or is a greedy one, so that the second pass has nothing to do (a row of another kind is
+// still drawn rightly, by one block).
 extern "C" int ia_sample(int* out, const float* logits, void* workspace, int rows, int vocab,
                          const float* temperature, const int* top_k, const float* top_p, const float* min_p,
-                         const float* u, const int* n_top, float* lp_out, int* lp_ids, hipStream_t stream) {
+                         const float* u, const int* n_top, float* lp_out, int* lp_ids, const int* window, int w,
+                         const float* rep, const float* freq, const float* pres, const int* bias_ids, const float* bias_vals,
+                         int nb, int narrow_only, hipStream_t stream) {
     IA_CHECK(rows >= 0 && vocab > 0, "sample: bad sizes rows=%d vocab=%d", rows, vocab);
     IA_CHECK(workspace != nullptr || rows == 0, "sample: needs a workspace of ia_sample_workspace(rows, vocab) words");
     IA_CHECK((n_top == nullptr) == (lp_out == nullptr) && (n_top == nullptr) == (lp_ids == nullptr),
              "sample: the arrays of the log-probabilities come together");
     IA_CHECK(rows <= 65535, "sample: at most 65535 rows a call, not %d", rows);
     IA_CHECK(vocab <= SAMPLE_STRETCH * SAMPLE_MAX_STRETCHES, "sample: at most %d tokens a row, not %d", SAMPLE_STRETCH * SAMPLE_MAX_STRETCHES, vocab);
+    const Penalties pen = {window, w, rep, freq, pres, bias_ids, bias_vals, nb};
+    if (const int bad = check_penalties("sample", pen)) return bad;
     if (rows == 0) return 0;
     const RowLayout l = row_layout(vocab);
     const dim3 grid((unsigned)l.stretches, (unsigned)rows);
-    sample_partials_kernel<<<grid, 256, 0, stream>>>(logits, (uint32_t*)workspace, l, temperature, n_top);
-    sample_stretch_kernel<<<grid, STRETCH_THREADS, 0, stream>>>(logits, (uint32_t*)workspace, l, temperature, top_k, n_top,
-                                                               g_sample_fast);
+    const int fast = g_sample_fast;
+    sample_partials_kernel<<<grid, 256, 0, stream>>>(logits, (uint32_t*)workspace, l, temperature, top_k, n_top, pen, fast);
+    if (fast != 1) narrow_only = 0;
+    if (!narrow_only)
+        sample_stretch_kernel<<<grid, STRETCH_THREADS, 0, stream>>>(logits, (uint32_t*)workspace, l, temperature, top_k, n_top, pen, fast);
     sample_kernel<<<rows, SAMPLE_THREADS, 0, stream>>>(out, logits, (uint32_t*)workspace, l, temperature,
-                                                       top_k, top_p, min_p, u, n_top, lp_out, lp_ids, g_sample_fast);
+                                                       top_k, top_p, min_p, u, n_top, lp_out, lp_ids, pen, fast, narrow_only);
     IA_LAUNCH_CHECK("sample");
     return 0;
 }

@@ -1233,31 +1233,40 @@ def argmax(logits: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Te
     return out
 
 
-def penalize(logits: torch.Tensor, window: Optional[torch.Tensor], repetition: torch.Tensor,
-             frequency: torch.Tensor, presence: torch.Tensor, bias_ids: Optional[torch.Tensor] = None,
-             bias_vals: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """In place on float32 logits [rows, vocab]: logit bias, then repetition, frequency and presence
-    penalties over each row's `window` of earlier tokens (int32 [rows, w], -1 = none)."""
-    _dev(logits, window, repetition, frequency, presence, bias_ids, bias_vals)
-    _f32(logits, "logits"); _f32(repetition, "repetition"); _f32(frequency, "frequency"); _f32(presence, "presence")
-    rows, vocab = logits.shape
+def _penalty_args(who: str, rows: int, window: Optional[torch.Tensor], repetition: Optional[torch.Tensor],
+                  frequency: Optional[torch.Tensor], presence: Optional[torch.Tensor], bias_ids: Optional[torch.Tensor] = None,
+                  bias_vals: Optional[torch.Tensor] = None) -> tuple:
+    """Bias and penalties of `rows` rows, checked, as the entry points take them."""
+    _dev(window, repetition, frequency, presence, bias_ids, bias_vals)
+    _f32(repetition, "repetition"); _f32(frequency, "frequency"); _f32(presence, "presence")
     w = 0 if window is None else window.shape[1]
     nb = 0 if bias_ids is None else bias_ids.shape[1]
     if window is not None:
         _i32(window, "window")
         if window.shape[0] != rows:
-            raise KernelError("penalize: one window row per row of logits")
+            raise KernelError(f"{who}: one window row per row of logits")
     if (bias_ids is None) != (bias_vals is None):
-        raise KernelError("penalize: bias ids and values come together")
+        raise KernelError(f"{who}: bias ids and values come together")
     if bias_ids is not None:
         _i32(bias_ids, "bias_ids"); _f32(bias_vals, "bias_vals")
         if bias_ids.shape != bias_vals.shape or bias_ids.shape[0] != rows:
-            raise KernelError("penalize: bias arrays must be [rows, entries]")
+            raise KernelError(f"{who}: bias arrays must be [rows, entries]")
     for t in (repetition, frequency, presence):
         if t.numel() != rows:
-            raise KernelError("penalize: one penalty value per row of logits")
-    _check(library().ia_penalize(_p(logits), rows, vocab, _p(window), w, _p(repetition), _p(frequency),
-                                 _p(presence), _p(bias_ids), _p(bias_vals), nb, _stream()))
+            raise KernelError(f"{who}: one penalty value per row of logits")
+    return _p(window), w, _p(repetition), _p(frequency), _p(presence), _p(bias_ids), _p(bias_vals), nb
+
+
+def penalize(logits: torch.Tensor, window: Optional[torch.Tensor], repetition: torch.Tensor,
+             frequency: torch.Tensor, presence: torch.Tensor, bias_ids: Optional[torch.Tensor] = None,
+             bias_vals: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """In place on float32 logits [rows, vocab]: logit bias, then repetition, frequency and presence
+    penalties over each row's `window` of earlier tokens (int32 [rows, w], -1 = none)."""
+    _dev(logits)
+    _f32(logits, "logits")
+    rows, vocab = logits.shape
+    args = _penalty_args("penalize", rows, window, repetition, frequency, presence, bias_ids, bias_vals)
+    _check(library().ia_penalize(_p(logits), rows, vocab, *args, _stream()))
     return logits
 
 
@@ -1273,22 +1282,40 @@ def window_push(window: torch.Tensor, caps: torch.Tensor, tokens: torch.Tensor) 
     return window
 
 
+_NO_PENALTIES = (None, 0, None, None, None, None, None, 0)
+
+
+def sample_narrow_top() -> int:
+    """Rows with a top_k of up to this many, below the vocabulary, are drawn from a few candidates of every stretch of the row."""
+    return library().ia_sample_narrow_top()
+
+
 def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor,
-           min_p: torch.Tensor, u: torch.Tensor, n_top: Optional[torch.Tensor] = None):
+           min_p: torch.Tensor, u: torch.Tensor, n_top: Optional[torch.Tensor] = None, *,
+           penalties: Optional[tuple] = None, narrow_only: bool = False, out: Optional[torch.Tensor] = None):
     """One token per row of float32 logits: greedy where temperature < 1e-5, else temperature,
     top-k, top-p, min-p and the walk to the row's random number u in [0, 1).  With `n_top` (int32
     per row: -1 none, else 0..20) also returns the log-probabilities within the kept list, float32
     [rows, 1 + 20] (the drawn token's, then the list's first entries'), and those entries' ids, int32
-    [rows, 20] (-1: no entry): the result is then (tokens, log-probabilities, ids)."""
-    _dev(logits, temperature, top_k, top_p, min_p, u, n_top)
+    [rows, 20] (-1: no entry): the result is then (tokens, log-probabilities, ids).
+    `penalties`: what `penalize` takes behind the logits, applied on the way (the logits stay as they are).
+    `narrow_only`: the caller knows that every row is greedy or has a top_k in 1 .. `sample_narrow_top()` below the
+    vocabulary, and saves a launch.  `out`: where the tokens go (int32 [rows])."""
+    _dev(logits, temperature, top_k, top_p, min_p, u, n_top, out)
     _f32(logits, "logits"); _f32(temperature, "temperature"); _f32(top_p, "top_p"); _f32(min_p, "min_p"); _f32(u, "u")
     _i32(top_k, "top_k")
     rows, vocab = logits.shape
     for t in (temperature, top_k, top_p, min_p, u) + ((n_top,) if n_top is not None else ()):
         if t.numel() != rows:
             raise KernelError("sample: one parameter value per row of logits")
+    pen = _NO_PENALTIES if penalties is None else _penalty_args("sample", rows, *penalties)
     lib = library()
-    out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
+    if out is None:
+        out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
+    else:
+        _i32(out, "out")
+        if out.numel() != rows:
+            raise KernelError("sample: one place per row of logits")
     ws = torch.empty((lib.ia_sample_workspace(rows, vocab),), dtype=torch.int32, device=logits.device)
     lp = ids = None
     if n_top is not None:
@@ -1297,7 +1324,7 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
         lp = torch.empty((rows, 1 + most), dtype=torch.float32, device=logits.device)
         ids = torch.empty((rows, most), dtype=torch.int32, device=logits.device)
     _check(lib.ia_sample(_p(out), _p(logits), _p(ws), rows, vocab, _p(temperature), _p(top_k), _p(top_p),
-                         _p(min_p), _p(u), _p(n_top), _p(lp), _p(ids), _stream()))
+                         _p(min_p), _p(u), _p(n_top), _p(lp), _p(ids), *pen, int(narrow_only), _stream()))
     return out if n_top is None else (out, lp, ids)
 
 

@@ -62,7 +62,7 @@ class Sampler:
         if all(p.is_plain_greedy for p in params):
             return ops.argmax(logits).cpu().tolist(), [None] * rows
 
-        # penalties and bias, on a copy only if something is changed
+        # penalties and bias, which the draw applies on the way (the logits stay as they are)
         width = max((min(p.repeat_last_n, len(prev)) if p.has_penalty else 0) for p, prev in zip(params, previous))
         n_bias = max(len(p.logit_bias) for p in params)
         window = rep = freq = pres = bias_ids = bias_vals = None
@@ -92,15 +92,18 @@ class Sampler:
                         for p, prev, seed in zip(params, previous, seeds)], dtype=np.float32)
         n_top = np.asarray([p.top_logprobs if p.logprobs else -1 for p in params], dtype=np.int32)
         penalized = window is not None
+        narrow = all_narrow(int(top_k.min()), int(top_k.max()), logits.shape[1])
         window, rep, freq, pres, bias_ids, bias_vals, temperature, top_k, top_p, min_p, u, n_top = self._upload(
             window if width else None, rep, freq, pres, bias_ids, bias_vals, temperature, top_k, top_p, min_p, u, n_top)
+        penalties = None
         if penalized:
-            logits = logits.clone()
-            ops.penalize(logits, window, rep, freq, pres, bias_ids, bias_vals)
+            penalties = (window, rep, freq, pres, bias_ids, bias_vals)
+            if not logits.is_contiguous():
+                logits = logits.clone()
         if not any(p.logprobs for p in params):
-            out = ops.sample(logits, temperature, top_k, top_p, min_p, u)
+            out = ops.sample(logits, temperature, top_k, top_p, min_p, u, penalties=penalties, narrow_only=narrow)
             return out.cpu().tolist(), [None] * rows
-        out, lp, ids = ops.sample(logits, temperature, top_k, top_p, min_p, u, n_top)
+        out, lp, ids = ops.sample(logits, temperature, top_k, top_p, min_p, u, n_top, penalties=penalties, narrow_only=narrow)
         tokens, lp, ids = out.cpu().tolist(), lp.cpu().tolist(), ids.cpu().tolist()
         infos = []
         for i, p in enumerate(params):
@@ -110,6 +113,11 @@ class Sampler:
             top = tuple((t, v) for t, v in zip(ids[i], lp[i][1:]) if t >= 0)[:p.top_logprobs]
             infos.append(TokenLogprob(tokens[i], lp[i][0], top))
         return tokens, infos
+
+
+def all_narrow(least: int, most: int, vocab: int) -> bool:
+    """Rows whose top_k lies in `least` .. `most` all go `ops.sample`'s shortest way."""
+    return 0 < least and most <= min(ops.sample_narrow_top(), vocab - 1)
 
 
 class ChainDraw:
@@ -150,6 +158,7 @@ class ChainDraw:
         top_k = np.asarray([p.top_k for p in params], dtype=np.int32)
         top_p = np.asarray([p.top_p for p in params], dtype=np.float32)
         min_p = np.asarray([p.min_p for p in params], dtype=np.float32)
+        self.least_k, self.most_k = int(top_k.min()), int(top_k.max())
         # the step of a draw is the number of tokens before it (`sampler.rs:323-325`)
         u = np.asarray([[rand_f32(seed, len(prev) + i) if p.draw_temperature(len(prev)) >= SAMPLING_EPS else 0.0
                          for p, prev, seed in zip(params, previous, seeds)] for i in range(steps)],
@@ -159,14 +168,12 @@ class ChainDraw:
                                                             pres, temperature, top_k, top_p, min_p, u)
 
     def pick(self, logits: torch.Tensor, step: int, out: torch.Tensor) -> None:
-        """The tokens of the run's `step`-th step from its logits, into `out` (int32 [rows], on the device).
-        The penalties are applied to `logits` in place: inside a run they are the captured step's own output buffer,
-        which the next step overwrites and nobody else reads."""
+        """The tokens of the run's `step`-th step from its logits, into `out` (int32 [rows], on the device)."""
         if self.greedy:
             ops.argmax(logits, out=out)
             return
-        if self.penalized:
-            ops.penalize(logits, self.window, self.rep, self.freq, self.pres, self.bias_ids, self.bias_vals)
-        out.copy_(ops.sample(logits, self.temperature, self.top_k, self.top_p, self.min_p, self.u[step]))
+        penalties = (self.window, self.rep, self.freq, self.pres, self.bias_ids, self.bias_vals) if self.penalized else None
+        ops.sample(logits, self.temperature, self.top_k, self.top_p, self.min_p, self.u[step], penalties=penalties,
+                   narrow_only=all_narrow(self.least_k, self.most_k, logits.shape[1]), out=out)
         if self.window is not None:
             ops.window_push(self.window, self.caps, out)

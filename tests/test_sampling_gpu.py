@@ -128,6 +128,71 @@ def test_rows_with_a_top_k_take_the_same_tokens_on_both_paths(vocab, top_k):
     assert torch.equal(torch.isfinite(lp_f), finite) and float((lp_f[finite] - lp_s[finite]).abs().max()) < 1e-4
 
 
+def _narrow_logits(kind, rows, vocab, g):
+    z = torch.randn(rows, vocab, generator=g) * 2.5
+    if kind == "masked":                               # few tokens allowed, the others at -inf or the type's lowest value
+        z[:, torch.rand(vocab, generator=g) < 0.98] = -math.inf
+        z[1::2] = z[1::2].clamp_min(torch.finfo(torch.float32).min)
+    elif kind == "coarse":
+        z = z.to(torch.bfloat16).float()
+    elif kind == "flat":                               # more equal logits than a stretch has places for candidates
+        z[::2] = 0.25
+        z[1::2, vocab // 2:] = 9.0
+    elif kind == "peaked":
+        z[:, vocab // 3] = 400.0
+    elif kind == "numbers":                            # rows without a number to start from, with infinities, with a NaN
+        z[0] = -math.inf
+        z[1, 5] = math.inf
+        z[2, 7] = math.nan
+        z[3] = math.nan
+    return z
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["plain", "masked", "coarse", "flat", "peaked", "numbers"])
+@pytest.mark.parametrize("vocab,top_k", [(65, 64), (67, 1), (4096, 50), (4097, 64), (10001, 50), (151936, 50), (151937, 2), (70000, 63)])
+def test_narrow_rows_draw_what_other_rows_with_a_top_k_draw(kind, vocab, top_k):
+    """Rows with a top_k of up to 64 are drawn from candidates that a stretch's logits leave behind, with the penalties on
+    the way; switched off, their first top_k tokens are found among the keys of all tokens of a penalised copy.  The sums are
+    the same in the same order, so tokens, log-probabilities and ids are equal, not only close."""
+    from inferrs_amd import ops
+    g = torch.Generator().manual_seed(vocab + top_k)
+    rows, w = 8, 70 if vocab != 10001 else 1100         # (a window within and beyond what a block keeps in shared memory)
+    z = _narrow_logits(kind, rows, vocab, g)
+    window = torch.randint(0, max(2, vocab // 50), (rows, w), generator=g, dtype=torch.int32)
+    window[1, 3:] = -1
+    rep, freq, pres = torch.linspace(0.9, 1.4, rows), torch.linspace(0.0, 0.3, rows), torch.full((rows,), 0.1)
+    ids = torch.tensor([[3, vocab - 1, vocab + 5], [2, -1, -1]] * (rows // 2), dtype=torch.int32)
+    vals = torch.tensor([[0.5, 4.0, 1.0], [-1.0, 0.0, 0.0]] * (rows // 2))
+    temperature = torch.tensor([0.7, 1.5, 0.05, 1.0, 1e-5, 3.0, 0.7, 0.0])
+    top_p, min_p = torch.tensor([0.9, 1.0] * (rows // 2)), torch.tensor([0.0, 0.0, 0.05, 0.0] * (rows // 4))
+    k, n_top = torch.full((rows,), top_k, dtype=torch.int32), torch.tensor([5, -1, 0, 20] * (rows // 4), dtype=torch.int32)
+    pen = [t.to("cuda") for t in (window, rep, freq, pres, ids, vals)]
+    z, temperature, k, top_p, min_p, n_top = (t.to("cuda") for t in (z, temperature, k, top_p, min_p, n_top))
+    touched = ops.penalize(z.clone(), *pen)
+    aside = torch.cat([torch.zeros(1, device="cuda"), z.flatten()])[1:].view(rows, vocab)      # rows that start anywhere
+    for u in (torch.zeros(rows), torch.rand(rows, generator=g), torch.full((rows,), 1.0)):
+        u = u.to("cuda")
+        ops.library().ia_sample_tune(2)
+        try:
+            want = ops.sample(touched, temperature, k, top_p, min_p, u, n_top)
+        finally:
+            ops.library().ia_sample_tune(1)
+        for logits, more in ((z, {}), (z, {"narrow_only": True}), (aside, {"narrow_only": True})):
+            got = ops.sample(logits, temperature, k, top_p, min_p, u, n_top, penalties=pen, **more)
+            assert torch.equal(got[0], want[0]), (kind, got[0].tolist(), want[0].tolist())
+            for i in range(rows):
+                if int(n_top[i]) >= 0 and float(temperature[i]) > 0:
+                    assert torch.equal(got[2][i], want[2][i]) and torch.equal(got[1][i].nan_to_num(7.0), want[1][i].nan_to_num(7.0)), (kind, i)
+    # rows of another kind are drawn rightly whatever the caller claims
+    k[::2] = torch.tensor([0, 65, 200, vocab], dtype=torch.int32, device="cuda")
+    u = torch.rand(rows, generator=g).to("cuda")
+    got = ops.sample(z, temperature, k, top_p, min_p, u, penalties=pen, narrow_only=True)
+    want = ops.sample(touched, temperature, k, top_p, min_p, u)
+    if kind != "numbers":                              # (the whole list's weight is added up in another order there)
+        assert int((got == want).sum()) >= rows - 1, (got.tolist(), want.tolist())
+
+
 @pytest.mark.gpu
 def test_mixed_rows_do_not_influence_each_other():
     from inferrs_amd.sampling import Sampler
