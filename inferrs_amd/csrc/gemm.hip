@@ -319,7 +319,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define SK_KSTEP 32     // k per MFMA
-#define SK_MAX_WAVES 16
+#define SK_MAX_WAVES 8      // of a block: sixteen of half the k each left two waves a SIMD the registers for one short chunk
 
 // Operand layout of v_mfma_f32_16x16x32_bf16: lane l supplies row (l % 16) of A and column
 // (l % 16) of B, each with the eight k values (l / 16) * 8 .. + 8; lane l receives
@@ -368,7 +368,7 @@ struct SkinnyStream {
     const bf16_t* bias;         // [N] ([2 N] with DUAL), added to every row's sums before anything is rounded; or null
 };
 
-// STAGE: 0, or the k steps of a staged chunk (8 or 16).
+// STAGE: 0, or the k steps of a staged chunk (8).
 template <int MT, int RT, bool DUAL, int STAGE>
 __global__ __launch_bounds__(SK_MAX_WAVES * IA_WAVE) void gemm_skinny_kernel(
     void* __restrict__ out, int out_f32, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
@@ -723,6 +723,256 @@ __global__ __launch_bounds__(SK_MAX_WAVES * IA_WAVE) void gemm_skinny_kernel(
         }
 }
 
+// The same product for up to 16 rows of x and weights that one or two rounds of blocks cover (q|k|v, o and down of every model,
+// [gate; up] of small ones).  Such a kernel is short: a chip that does nothing else takes 1.6 us a kernel inside a graph, 3.3 to read 8 MB
+// and 7 to read 32, and what a product spends beside that is its own chain of waits.  So the weight's first chunk (C steps of k a
+// wave) is asked for at once, and everything that does not need it is done while it is on its way: x goes straight into the wave's
+// corner of shared memory (no register, no wait a row), the rows' sums of squares become scales.  Behind the product the tiles of all
+// waves are read together, and a thread finishes one feature of one row (four of them one after the other, all in one wave, were 0.4 us
+// of code that no cache holds yet).  A range longer than a chunk: BURST_AHEAD asks for the next chunk of both operands, x through
+// registers, before it multiplies this one (one block a compute unit has the registers), BURST_CHUNKS leaves that to the other block
+// on the unit.  The order of every sum is that of gemm_skinny_kernel: the same bits.
+// Measured inside graphs, us, a layer's four products one behind another, before and now: 0.6B shape, 1 row 24.3 -> 18.5, 8 rows 26.8 -> 20.6;
+// 1.7B shape, 1 row 35.2 -> 31.0, 8 rows 39.7 -> 35.2; 4B shape, 1 row 57.1 -> 50; 8B shape, 1 row 78.2 -> 75.8, 8 rows 84.0 -> 82.5
+// (q|k|v 11.7 -> 10.0 at one row, the bare read of its 50 MB 9.9); 14B shape, 1 row 129.4 -> 124.4.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+enum { BURST_WHOLE = 0, BURST_AHEAD = 1, BURST_CHUNKS = 2 };
+template <int NA, int XR, int C, int MODE>
+__global__ __launch_bounds__(SK_MAX_WAVES * IA_WAVE) __attribute__((amdgpu_waves_per_eu(MODE == BURST_AHEAD ? 2 : 4))) void gemm_burst_kernel(
+    void* __restrict__ out, int out_f32, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+    int M, int N, int K, int kper, int rpb, int rot_mul, const SkinnyStream st) {
+    constexpr bool MORE = MODE != BURST_WHOLE;
+    constexpr int PIECES = C * 4;                           // 16-byte pieces of a row's chunk
+    constexpr int PITCH = PIECES * 16;                      // bytes of a staged row
+    constexpr int ROWS_A_LOAD = IA_WAVE / PIECES;           // rows of x that one load instruction brings
+    constexpr int XL = (XR + ROWS_A_LOAD - 1) / ROWS_A_LOAD;
+    extern __shared__ f32x4 red[];                          // [waves][NA][64], then [waves][rows of x, a whole number of loads]
+    __shared__ float scale_row[16];
+    const int lane = threadIdx.x & (IA_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / IA_WAVE);
+    const int waves = blockDim.x / IA_WAVE;
+    const int n0 = blockIdx.x * rpb;
+    const int r = lane & 15, g = lane >> 4;
+    const int ks0 = wave * kper;
+    const int len = min(kper, K / SK_KSTEP - ks0);          // (K is a multiple of 32, and no wave is without a step)
+    // (as in gemm_skinny_kernel)
+    const int rot = MORE && len > 16 ? (int)((blockIdx.x * (unsigned)rot_mul) % (unsigned)len) / 16 * 16 : 0;
+    auto step_of = [&](int i) {                             // the k step that is multiplied i-th; the last one beyond the end
+        int at = min(i, len - 1) + rot;
+        if (MORE) at = at >= len ? at - len : at;
+        return ks0 + at;
+    };
+    const int j = r < rpb ? r : rpb - 1;
+    const bf16_t* const wrow = w + (size_t)(n0 + j < N ? n0 + j : N - 1) * K + g * 8;
+    const size_t up = (size_t)N * K;
+
+    struct Chunk { u32x4 a[C][NA]; };
+    auto ask_w = [&](Chunk& c, int first) __attribute__((always_inline)) {
+        if (MORE) {
+#pragma unroll
+            for (int i = 0; i < C; ++i)
+#pragma unroll
+                for (int q = 0; q < NA; ++q) c.a[i][q] = *(const u32x4*)(wrow + q * up + step_of(first + i) * SK_KSTEP);
+        } else {
+            // (a range shorter than the chunk: groups of four steps beyond it are left out)
+            const bf16_t* p = wrow + ks0 * SK_KSTEP;
+#pragma unroll
+            for (int i = 0; i < C; i += 4)
+                if (i < len)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+#pragma unroll
+                        for (int q = 0; q < NA; ++q) c.a[i + b][q] = *(const u32x4*)(p + q * up + min(i + b, len - 1) * SK_KSTEP);
+        }
+    };
+    // A wave's piece of x: a row's 16-byte pieces lie exchanged by the row's number, so that the operand reads, 16 rows at once,
+    // meet no bank twice.  Lane l of a load brings what belongs at its place.
+    const int x_loads = (M + ROWS_A_LOAD - 1) / ROWS_A_LOAD;
+    const int sub = lane / PIECES, place = lane % PIECES;
+    char* const stage = (char*)(red + waves * NA * IA_WAVE) + wave * (x_loads * IA_WAVE * 16);
+    auto x_from = [&](int l, int first) __attribute__((always_inline)) {
+        const int row = l * ROWS_A_LOAD + sub, piece = place ^ (row & 7);
+        return x + (size_t)min(row, M - 1) * K + (size_t)step_of(first + piece / 4) * SK_KSTEP + piece % 4 * 8;
+    };
+    u32x4 xp[MODE == BURST_AHEAD ? XL : 1];
+    auto ask_x = [&](int first) __attribute__((always_inline)) {
+        if constexpr (MODE == BURST_AHEAD) {
+#pragma unroll
+            for (int l = 0; l < XL; ++l)
+                if (l < x_loads) xp[l] = *(const u32x4*)x_from(l, first);
+        } else {
+            for (int l = 0; l < x_loads; ++l)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)x_from(l, first),
+                                                 (__attribute__((address_space(3))) void*)(stage + l * IA_WAVE * 16), 16, 0, 0);
+        }
+    };
+    auto put_x = [&]() __attribute__((always_inline)) {
+        if constexpr (MODE == BURST_AHEAD)
+#pragma unroll
+            for (int l = 0; l < XL; ++l)
+                if (l < x_loads) *(u32x4*)(stage + (l * IA_WAVE + lane) * 16) = xp[l];
+    };
+
+    // what the start and the end need of the stream (see gemm_skinny_kernel): a row's sums of squares a wave
+    constexpr int SS_ROWS = 2, SS_VEC = 2;
+    float4 ss_mine[SS_ROWS][SS_VEC];
+    const bool scaled = st.sums_in != nullptr;
+    const bool ss_wide = scaled && (st.n_sums & 3) == 0 && st.n_sums <= 4 * IA_WAVE * SS_VEC;
+    if (ss_wide) {
+#pragma unroll
+        for (int i = 0; i < SS_ROWS; ++i) {
+            const int m = wave + i * waves;
+            if (m < M)
+#pragma unroll
+                for (int v = 0; v < SS_VEC; ++v) {
+                    const int at = 4 * (lane + v * IA_WAVE);
+                    ss_mine[i][v] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (at < st.n_sums) ss_mine[i][v] = *(const float4*)(st.sums_in + (size_t)m * st.n_sums + at);
+                }
+        }
+    }
+    Chunk c0;
+    ask_x(0);
+    ask_w(c0, 0);
+    // Behind the sum a thread owns one feature of one row: lane l of wave v feature l % 16 of row 4 v + l / 16.
+    const int f = lane & 15;
+    const bool mine_in = f < rpb && n0 + f < N;
+    float old = 0.f, next_w = 0.f;
+    if constexpr (NA == 1) {
+        const int m = 4 * wave + (lane >> 4);
+        if (st.resid != nullptr && mine_in && m < M) {
+            old = ld(st.resid + (size_t)m * N + n0 + f);
+            if (st.scaled_out != nullptr) next_w = st.next_w[n0 + f];
+        }
+    }
+    if (scaled) {
+        for (int i = 0, m = wave; m < M; ++i, m += waves) {
+            float ss = 0.f;
+            if (ss_wide && i < SS_ROWS) {
+                const float4 (&v)[SS_VEC] = i == 0 ? ss_mine[0] : ss_mine[1];
+                ss = ((v[0].x + v[0].y) + v[0].z) + v[0].w;
+#pragma unroll
+                for (int b = 1; b < SS_VEC; ++b) ss += ((v[b].x + v[b].y) + v[b].z) + v[b].w;
+            } else {
+                for (int b = lane; b < st.n_sums; b += IA_WAVE) ss += st.sums_in[(size_t)m * st.n_sums + b];
+            }
+            ss = wave_sum(ss);
+            if (lane == 0) scale_row[m] = 1.0f / sqrtf(ss / (float)K + st.eps);
+        }
+    }
+    f32x4 acc[NA];
+#pragma unroll
+    for (int q = 0; q < NA; ++q) acc[q] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int rr = r < M ? r : 0;
+    const char* const mine[2] = {stage + rr * PITCH + (g ^ (rr & 7)) * 16, stage + rr * PITCH + ((4 + g) ^ (rr & 7)) * 16};
+    // One wave's own corner: its shared-memory operations run in program order.
+    auto own_corner = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    auto multiply = [&](const Chunk& c, int first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < C; i += 4) {
+            if (first + i >= len) break;
+            u32x4 b[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) b[v] = *(const u32x4*)(mine[v & 1] + (i + v) / 2 * 128);
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (first + i + v < len)
+#pragma unroll
+                    for (int q = 0; q < NA; ++q)
+                        acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, c.a[i + v][q]),
+                                                                         __builtin_bit_cast(bf16x8, b[v]), acc[q], 0, 0, 0);
+        }
+    };
+    if constexpr (MODE == BURST_WHOLE) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // (x is in shared memory, the weight in registers)
+        own_corner();
+        multiply(c0, 0);
+    } else if constexpr (MODE == BURST_CHUNKS) {
+        for (int first = 0; first < len; first += C) {
+            if (first > 0) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the last chunk's operands have been read)
+                ask_x(first);
+                ask_w(c0, first);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            own_corner();
+            multiply(c0, first);
+            own_corner();
+        }
+    } else {
+        Chunk c1;
+        for (int first = 0; first < len; first += 2 * C) {
+            put_x();
+            own_corner();
+            if (first + C < len) { ask_x(first + C); ask_w(c1, first + C); }
+            multiply(c0, first);
+            own_corner();
+            if (first + C >= len) break;
+            put_x();
+            own_corner();
+            if (first + 2 * C < len) { ask_x(first + 2 * C); ask_w(c0, first + 2 * C); }
+            multiply(c1, first + C);
+            own_corner();
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NA; ++q) red[(wave * NA + q) * IA_WAVE + lane] = acc[q];
+    __syncthreads();
+    const float* const tiles = (const float*)red;           // [waves][NA][feature / 4][row][feature % 4]
+    for (int m0 = 4 * wave; m0 < M; m0 += 4 * waves) {
+        const int m = m0 + (lane >> 4);
+        const bool in = mine_in && m < M;
+        float part[NA][SK_MAX_WAVES], s[NA];
+#pragma unroll
+        for (int v = 0; v < SK_MAX_WAVES; ++v)
+#pragma unroll
+            for (int q = 0; q < NA; ++q)
+                part[q][v] = tiles[((min(v, waves - 1) * NA + q) * IA_WAVE + f / 4 * 16 + (m & 15)) * 4 + f % 4];
+        const float scale = scaled ? scale_row[m & 15] : 1.f;
+#pragma unroll
+        for (int q = 0; q < NA; ++q) {
+            s[q] = part[q][0];
+#pragma unroll
+            for (int v = 1; v < SK_MAX_WAVES; ++v) s[q] = v < waves ? s[q] + part[q][v] : s[q];
+            if (scaled) s[q] *= scale;
+            if (st.bias != nullptr && in) s[q] += ld(st.bias + (size_t)q * N + n0 + f);
+        }
+        const size_t at = (size_t)m * N + n0 + f;
+        if (NA == 1 && st.resid != nullptr) {
+            // (all lanes stay for the row's sum of squares: four neighbours one after the other, then pairs, as in gemm_skinny_kernel)
+            float sq = 0.f;
+            if (in) {
+                if (m0 != 4 * wave) {
+                    old = ld(st.resid + at);
+                    if (st.scaled_out != nullptr) next_w = st.next_w[n0 + f];
+                }
+                const float h = round_to(st.resid, round_to(st.resid, s[0]) + old);
+                ::st(st.resid + at, h);
+                sq = h * h;
+                if (st.scaled_out != nullptr) ::st(st.scaled_out + at, h * (st.add_one ? 1.0f + next_w : next_w));
+            }
+            float four = __shfl(sq, lane & ~3) + __shfl(sq, (lane & ~3) + 1);
+            four += __shfl(sq, (lane & ~3) + 2);
+            four += __shfl(sq, lane | 3);
+            four += __shfl_xor(four, 4, IA_WAVE);
+            four += __shfl_xor(four, 8, IA_WAVE);
+            if (f == 0 && m < M) st.sums_out[(size_t)m * gridDim.x + blockIdx.x] = four;
+            continue;
+        }
+        if (!in) continue;
+        float v = s[0];
+        if constexpr (NA == 2)
+            // the products are rounded to the storage precision before the activation, as the two-kernel path rounds them
+            v = gate_act(round_to((const bf16_t*)nullptr, s[0]), st.act) * round_to((const bf16_t*)nullptr, s[1]);
+        if (out_f32) ((float*)out)[at] = v;
+        else ::st((bf16_t*)out + at, v);
+    }
+}
+
 // Tuning knobs (ia_gemm_skinny_tune): waves wanted on the chip before k stops being split,
 // fewest k steps worth a wave, and the stagger of the blocks' starting points.
 static int g_target_waves = 2048, g_min_ksteps = 8, g_rot_mul = 5, g_min_waves = 8, g_stage = 1;
@@ -780,8 +1030,11 @@ static void skinny_split(int N, int K, int rt, int tiles_per_wave, int* waves_ou
     // 2 x 12,288 x 4,096 at 8 rows 40.1 -> 38.8 us, at 16 rows 49.4 -> 42.8 (5,120 wide it does not: 72.4 -> 74.4 us).
     const int half = (g_min_waves + 1) / 2;
     const int min_waves = (rt == 2 || (skinny_tall(groups) && ksteps % (SK_CHUNK * half) == 0)) ? half : g_min_waves;
+    // A weight that one or two rounds of blocks cover is worth a wave for half as many steps (a k of 1,024, eight waves a block instead of
+    // four: q|k|v of the 0.6B shape 3.8 -> 3.4 us, [gate; up] 5.2 -> 4.6).
+    const int fewest = skinny_tall(groups) ? g_min_ksteps : (g_min_ksteps + 1) / 2;
     int waves = 1;
-    while (waves * 2 <= SK_MAX_WAVES && waves * 2 <= most && ksteps / (waves * 2) >= g_min_ksteps &&
+    while (waves * 2 <= SK_MAX_WAVES && waves * 2 <= most && ksteps / (waves * 2) >= fewest &&
            (groups * waves < g_target_waves || waves < min_waves))
         waves *= 2;
     int kper = (ksteps + waves - 1) / waves;
@@ -804,7 +1057,7 @@ static void skinny_split(int N, int K, int rt, int tiles_per_wave, int* waves_ou
 }
 
 #define SK_STAGE_LDS_MOST (80 * 1024)         // two blocks a compute unit
-#define SK_STAGE16_LDS_MOST (160 * 1024)     // one block a compute unit: all of its shared memory
+#define SK_SHARED_A_UNIT (160 * 1024)        // a compute unit's shared memory
 #define SK_SCALES_RESERVE 256                // the rows' sums of squares: static shared memory beside the launch's own area
 
 // Shared memory beyond 64 KiB has to be asked for, once per instantiation.
@@ -820,6 +1073,42 @@ static int skinny_ask_shared(int bytes) {
     return 0;
 }
 
+// Shared memory of a block of gemm_burst_kernel: the waves' tiles and their pieces of x.
+static size_t burst_shared(int waves, int na, int rows, int c) {
+    const int rows_a_load = IA_WAVE / (4 * c), loads = (rows + rows_a_load - 1) / rows_a_load;
+    return (size_t)waves * IA_WAVE * 16 * (na + loads);
+}
+
+template <int NA, int XR, int C, int MODE>
+static int launch_burst(unsigned grid, int waves, void* out, int out_f32, const bf16_t* x, const bf16_t* w, int M, int N, int K,
+                        int kper, int rpb, const SkinnyStream& st, hipStream_t stream) {
+    const size_t bytes = burst_shared(waves, NA, M, C);
+    static bool asked = false;
+    if (!asked && bytes > 65536 - SK_SCALES_RESERVE) {
+        const hipError_t e = hipFuncSetAttribute((const void*)gemm_burst_kernel<NA, XR, C, MODE>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, SK_SHARED_A_UNIT - SK_SCALES_RESERVE);
+        IA_CHECK(e == hipSuccess, "gemm_skinny: cannot ask for %zu bytes of shared memory: %s", bytes, hipGetErrorString(e));
+        asked = true;
+    }
+    gemm_burst_kernel<NA, XR, C, MODE><<<grid, waves * IA_WAVE, bytes, stream>>>(out, out_f32, x, w, M, N, K, kper, rpb, g_rot_mul, st);
+    return 0;
+}
+
+template <int NA>
+static int launch_burst_rows(unsigned grid, int waves, void* out, int out_f32, const bf16_t* x, const bf16_t* w, int M, int N, int K,
+                             int kper, int rpb, const SkinnyStream& st, hipStream_t stream) {
+    constexpr int LONG = NA == 1 ? 16 : 8;
+#define SK_BURST(XR, C, MODE) return launch_burst<NA, XR, C, MODE>(grid, waves, out, out_f32, x, w, M, N, K, kper, rpb, st, stream)
+    if (kper <= 8) SK_BURST(1, 8, BURST_WHOLE);
+    if (kper <= LONG) SK_BURST(1, LONG, BURST_WHOLE);
+    // (more than 8 rows of x beside two chunks of the weight do not fit a wave's registers: 4,096 x 12,288, 16 rows, 23.5 us as it was,
+    // 27.7 asked for ahead)
+    if ((int)grid > skinny_cus() || M > 8) SK_BURST(1, LONG, BURST_CHUNKS);
+    if (M <= 2) SK_BURST(2, LONG, BURST_AHEAD);
+    SK_BURST(8, LONG, BURST_AHEAD);
+#undef SK_BURST
+}
+
 template <int MT, int RT, bool DUAL>
 static int launch_skinny(void* out, int out_f32, const bf16_t* x, const bf16_t* w, int M, int N, int K,
                          int m_base, const SkinnyStream& st, hipStream_t stream) {
@@ -832,7 +1121,6 @@ static int launch_skinny(void* out, int out_f32, const bf16_t* x, const bf16_t* 
     if constexpr (MT == 1) {
         const int rows = M - m_base < 16 ? M - m_base : 16;
         const size_t staged8 = tiles + (size_t)waves * rows * (8 * 2 * SK_KSTEP + SK_STAGE_PAD);
-        const size_t staged16 = tiles + (size_t)waves * rows * (16 * 2 * SK_KSTEP + SK_STAGE_PAD);
         int stage = 0;
         if (g_stage && rows >= 1 && skinny_tall((int)grid)) {
             // Staging pays where blocks stream for long: with at least three blocks for every compute unit (also with
@@ -842,29 +1130,23 @@ static int launch_skinny(void* out, int out_f32, const bf16_t* x, const bf16_t* 
             // 5.44 without staging; seven waves, a width of 5,120: all 16).  Measured at 8 rows: gate|up 46 -> 40 us,
             // logits head 261 -> 224 us; at 14 rows a decode step of the 14B shape 10.9 -> 9.7 ms.
             if (kper >= 8 && staged8 <= SK_STAGE_LDS_MOST - SK_SCALES_RESERVE) stage = 8;
-        } else if (g_stage && rows >= 1 && !DUAL && RT == 1) {
-            // A weight that one or two rounds of blocks cover (o, down, qkv) is read in one burst, and what counts
-            // is how much a wave has in flight: chunks of 16 steps, as much as without staging, and up to
-            // all of a compute unit's shared memory for its block.  Measured at 8 rows: down 25.6 -> 22.3 us,
-            // o 11.5 -> 9.9, qkv 16.8 -> 14.2; at 16 rows 30.4 -> 24.5, 12.9 -> 10.6, 19.1 -> 16.8.  (From 9 rows on
-            // the area leaves room for one block of qkv's 384 on a compute unit, and they go in two rounds;
-            // chunks of 8, which keep it one round, were no faster: 15.8 against 16.4 us at 10 rows, 17.4
-            // against 16.7 at 16.)
-            if (kper % 16 == 0 && staged16 <= SK_STAGE16_LDS_MOST - SK_SCALES_RESERVE) stage = 16;
+        }
+        if constexpr (RT == 1) {
+            // A weight that one or two rounds of blocks cover is read in one burst (gemm_burst_kernel).  Not [gate; up] in more
+            // blocks than the chip has units where a wave's range is longer than its chunk of 8 (2 x 9,728 x 2,560, ranges of 10, one row:
+            // 23.4 us by the general kernel, whose blocks hold half the registers, 25.5 in chunks) or where the rows leave shared memory
+            // for one block a unit (2 x 6,144 x 2,048, 16 rows: 16.3 and 18.6 us).
+            const bool one_a_unit = 2 * (burst_shared(waves, 2, rows, 8) + SK_SCALES_RESERVE) > SK_SHARED_A_UNIT;
+            const bool general = DUAL && (int)grid > skinny_cus() && (kper > 8 || one_a_unit);
+            if (g_stage && rows >= 1 && m_base == 0 && K % SK_KSTEP == 0 && !skinny_tall((int)grid) && !general &&
+                (K / SK_KSTEP + kper - 1) / kper == waves)
+                return launch_burst_rows<DUAL ? 2 : 1>(grid, waves, out, out_f32, x, w, M, N, K, kper, rpb, st, stream);
         }
         if (stage == 8) {
             if (skinny_ask_shared<MT, RT, DUAL, 8>(SK_STAGE_LDS_MOST - SK_SCALES_RESERVE)) return 1;
             gemm_skinny_kernel<MT, RT, DUAL, 8><<<grid, waves * IA_WAVE, staged8, stream>>>(
                 out, out_f32, x, w, M, N, K, kper, rpb, m_base, g_rot_mul, st);
             return 0;
-        }
-        if constexpr (!DUAL && RT == 1) {
-            if (stage == 16) {
-                if (skinny_ask_shared<MT, RT, DUAL, 16>(SK_STAGE16_LDS_MOST - SK_SCALES_RESERVE)) return 1;
-                gemm_skinny_kernel<MT, RT, DUAL, 16><<<grid, waves * IA_WAVE, staged16, stream>>>(
-                    out, out_f32, x, w, M, N, K, kper, rpb, m_base, g_rot_mul, st);
-                return 0;
-            }
         }
     }
     gemm_skinny_kernel<MT, RT, DUAL, 0><<<grid, waves * IA_WAVE, waves > 1 ? tiles : 0, stream>>>(

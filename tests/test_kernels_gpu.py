@@ -711,6 +711,39 @@ def test_skinny_variants_for_one_round_weights_agree_bit_for_bit():
                            part), (lo, hi)
 
 
+@pytest.mark.parametrize("n,k,blocks", [
+    (1024, 1024, 64), (1024, 3072, 128),            # ranges of 4 and 12 steps a wave
+    (1000, 4096, 37), (77, 544, 5),                 # whole chunks of 16; fewer features than the last block holds, a short last wave
+    (4096, 12288, 256), (2560, 9728, 2),            # longer ranges, a block a compute unit; their last chunk not full
+    (5120, 5120, 320), (4096 + 48, 7168, 600)])     # more blocks than compute units; more sums than the start of the kernel takes
+def test_burst_products_have_the_bits_of_the_general_kernel(n, k, blocks):
+    from inferrs_amd import ops
+    lib = ops.library()
+    w, gain = dev(randn(n, k, dtype=torch.bfloat16, seed=n)), dev(randn(n, dtype=torch.float32, seed=4))
+    for m in (1, 2, 3, 8, 9, 16):
+        x, stream = dev(randn(m, k, dtype=torch.bfloat16, seed=k + m)), randn(m, n, dtype=torch.bfloat16, seed=5)
+        sums = dev(randn(m, blocks, dtype=torch.float32, seed=6).abs() * k / blocks)
+        bias = dev(randn(n, dtype=torch.bfloat16, seed=7))
+
+        def products():
+            resid, scaled = dev(stream), torch.empty((m, n), dtype=torch.bfloat16, device="cuda")
+            left = torch.empty((m, lib.ia_gemm_skinny_blocks(n)), dtype=torch.float32, device="cuda")
+            ops._stream_product(x, w, n, torch.bfloat16, False, resid=resid, sums_out=left, scaled_out=scaled, next_w=gain, bias=bias)
+            out = [resid, scaled, left, ops._stream_product(x, w, n, torch.bfloat16, False, sums_in=sums, eps=1e-6, bias=bias),
+                   ops.gemm_skinny_bf16(x, w, torch.float32)]
+            if n % 2 == 0:
+                out.append(ops._stream_product(x, w, n // 2, torch.bfloat16, True, sums_in=sums, eps=1e-6))
+            return [o.cpu() for o in out]
+
+        try:
+            lib.ia_gemm_skinny_tune(2048, 8, 5, 8, 0)
+            want = products()
+        finally:
+            lib.ia_gemm_skinny_tune(2048, 8, 5, 8, 1)
+        for what, (a, b) in enumerate(zip(products(), want)):
+            assert torch.equal(a, b), (m, what)
+
+
 @pytest.mark.parametrize("dual", [False, True])
 def test_skinny_variants_for_tall_weights_agree_bit_for_bit(dual):
     # a weight with three blocks a compute unit and more takes the variant that stages the activations through
