@@ -86,6 +86,9 @@ struct AttnParams {
     const float* sinks;         // with sink: null, or [nq] values s_h a query head (natural logarithm, not scaled): the term is 2^(s_h log2 e - m)
     int mask_chunk;             // > 0: a query sees the keys of its own chunk of this many positions only, up to itself
     int keep_first;             // > 0: it sees the first so many positions besides (forms 1 and 2)
+    uint32_t page_magic;        // decode kernel: pos / page is umulhi(2 (pos / 16), page_magic) >> page_shift
+    int page_shift;
+    int teams_log2;             // decode kernel: log2 of the blocks that share a (request, key/value head)
     float cap_in;               // form 2: a raw score s stands for tanh(s * scale / cap); this is 2 log2(e) scale / cap, and scale_log2 is cap * log2(e)
 };
 
@@ -472,17 +475,16 @@ __device__ __forceinline__ float column_sum(float x) {
 //    last block reads past the caches after it has seen the full count.  The counters are zero
 //    between calls (the last block puts its counter back), so calls that share them must not overlap.
 // The sum over the splits runs in the order of the splits whoever comes last: the result is the same every time.
-// Measured (head size 128, 32 query and 8 key/value heads, context 8,192, time stamps inside the kernel): a wave
-// knows its token's position 0.8 us after it starts, has asked for the rows and the first keys at 2.5, has its rows
-// formed at 4.6 and its two steps done at 6.6 (batch 1, 64 keys a wave); the block's waves have met at 7.0, the
-// partial result is out at 7.5, the count back at 9.3 and the last block has merged at 13 to 16 us.  A fence of
-// device scope in place of the write-through stores cost 100 us a layer at batch 8 (it writes back and empties
-// the whole L2 of the die, once a block).  The kernel needs a SIMD's whole register file for a wave (two sets of
-// operands, and more in the rows' forming), so a compute unit holds one block: the step's split keeps its waves
-// within one round of the chip.  Against the kernel above with a merge kernel behind it, a layer, each at its
-// best split: batch 8 52.4 against 56.5 us, batch 3 26.0 against 29.0, batch 16 98.8 against 103, batch 32 189
-// against 195, batch 64 358 against 366; batch 8 at a context of 2,048 20.9 against 24.4, batch 64 at 1,024 49.0
-// against 56.7; batch 1 17 to 18 us both ways.
+// A wave is mostly alone on its SIMD, so every instruction it executes is four cycles of the step (returning from the kernel early, 16 query
+// and 8 key/value heads, 700 keys, 64 a wave: rows and first keys are there 1.0 us after the start, rows formed 2.0 later, two steps done
+// 3.5 later, a team merged 0.9 later, the hand-over 2.5).  So rows are formed by all lanes, numbers of pages come without divisions,
+// the edges of a walk are handled once, ahead of its first and last step, and not in every copy of a step, results that meet are
+// asked for together, and lanes exchange sums without a trip through shared memory; and nothing is held that can be read again, so
+// that (head sizes up to 128) two waves share a SIMD.  us a layer, before and now: 16 query heads, batch 1, 200 keys 10.6 -> 7.9,
+// 1,000 11.6 -> 9.0, 8,000 16.8 -> 14.0; 32 query heads, batch 4 at 2,000 15.2 -> 12.6, batch 8 at 700 13.7 -> 11.3, at
+// 8,192 52.9 -> 51.2, batch 64 at 1,500 73.9 -> 72.0; 64 query heads, batch 2 at 1,500 15.2 -> 11.9.  Of the context at 8,192, batch 8, the
+// bytes alone take 42.  A fence of device scope in place of the write-through stores cost 100 us a layer at batch 8 (it writes
+// back and empties the whole L2 of the die, once a block).
 // Partial results that blocks on other compute units read within the same kernel: written through to memory and
 // read past the caches that are not coherent between the chip's dies (32-bit accesses of device scope, no order
 // of their own), so that no cache has to be written back or emptied as a whole.
@@ -493,13 +495,31 @@ __device__ __forceinline__ float get_across(const float* at) {
     return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The sum over `LANES` neighbouring lanes (8, 16 or 32, aligned), in all of them, in the vector units' own lane exchanges.
+template <int LANES>
+__device__ __forceinline__ float row_sum(float x) {
+#define ROW_STEP(CTRL) x += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), CTRL, 0xf, 0xf, true))
+    ROW_STEP(0xb1);                                         // lane ^ 1
+    ROW_STEP(0x4e);                                         // lane ^ 2
+    ROW_STEP(0x141);                                        // the other four of eight
+    if constexpr (LANES >= 16) ROW_STEP(0x140);             // the other eight of sixteen
+#undef ROW_STEP
+    if constexpr (LANES >= 32) {
+        auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    }
+    return x;
+}
+
 struct DecodeOperands {
     uint4 k[2][KS];             // as Operands above
     uint4 v[DB];
 };
 
+#define DECODE_TEAM 4           // waves of a block at most
+
 template <bool ENABLED = (HD % 64 == 0 && HDV == HD)>
-__global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnParams p, int* counters, int team) {
+__global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_per_eu(HD <= 128 ? 2 : 1))) void attn_decode_kernel(const AttnParams p, int* counters, int team) {
     if constexpr (ENABLED) {
         extern __shared__ __align__(16) float team_mem[];       // [team][columns][HD] partial outputs, then [team][columns][2]
         __shared__ int s_last;
@@ -508,12 +528,17 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
         const int lane = threadIdx.x & (IA_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / IA_WAVE);
         const int r = lane & 15, G = lane >> 4;
         const int g = p.nq / p.nkv;
-        const int teams = p.splits / team;
-        const int kvh = blockIdx.y / teams, tm = blockIdx.y - kvh * teams;
+        const int teams = 1 << p.teams_log2;
+        const int kvh = blockIdx.y >> p.teams_log2, tm = blockIdx.y & (teams - 1);
         const int split = tm * team + wave;
         const int seq = p.seq_begin + blockIdx.z;
         const int col0 = blockIdx.x * 16;
         const int n_cols = g - col0 < 16 ? g - col0 : 16;       // this block's columns (the grid has no empty block)
+        // (a division by a number known at run time only is some thirty instructions one after the other, and the walk's start
+        // would wait for six of them)
+        auto page_of = [&](int pos) __attribute__((always_inline)) {
+            return (int)(__umulhi((uint32_t)pos >> 3 & ~1u, p.page_magic) >> p.page_shift);
+        };
         // What a wave needs before it can ask for its first keys is a chain of small reads, each a trip to the
         // memory: the token's position, then the pages' numbers.  A decode step's token is known without a read
         // (request seq_begin + i owns token token_begin + i), and where no window moves the walk's start the first
@@ -525,7 +550,7 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
         int early[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int idx = (c_lo + 16 * i) / p.page;
+            const int idx = page_of(c_lo + 16 * i);
             early[i] = bt[idx < p.max_pages ? idx : p.max_pages - 1];
         }
         const int kv_start = p.positions[t0];
@@ -539,56 +564,49 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
         lo &= ~31;
 
         // ---- loads, in the order in which their results are needed ------------------------------------
-        // The rows of the projections' output that this wave norms and rotates (its query heads' rows and the new
-        // key's: every wave asks for it, one wave uses it), the norms' weights and the angles, then the first
-        // step's keys and values: the rows are formed while those are on their way, and the second step's are asked
-        // for after that (a wave can have 63 loads outstanding: all at once would stall the issue of the last ones
-        // until the first come back).
+        // The rows of the projections' output that this wave norms and rotates (its query heads' rows, and behind them the new
+        // key's), the norms' weights and the angles, then the first step's keys and values: the rows are formed while those are
+        // on their way, and the second step's are asked for after that (a wave can have 63 loads outstanding: all at once
+        // would stall the issue of the last ones until the first come back).
+        // The rows are shared out over all lanes: a lane has four features of a row and the four that they are turned with, HD / 2
+        // further on, a pass takes ROWS rows, and they meet the matrix operand's layout in the wave's own shared memory.  (With a
+        // column's features in the four lanes that need them, 32 a lane, two rows took 2 of the 7 us that a wave has.)
         const int qkv_row = (p.nq + 2 * p.nkv) * HD;
         const bf16_t* token_row = p.qkv + (size_t)t0 * qkv_row;
-        uint4 qraw[KS], kraw[KS];
-        uint32_t vnew[DB];
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            qraw[ks] = *(const uint4*)(token_row + (size_t)head * HD + ks * 32 + G * 8);
-            kraw[ks] = *(const uint4*)(token_row + (size_t)(p.nq + kvh) * HD + ks * 32 + G * 8);
-        }
-        // the norms' weights and the token's angles for this lane's features (a feature's rotation partner, HD / 2
-        // further on, lies in the same lane)
-        constexpr int HK = KS / 2 > 0 ? KS / 2 : 1;      // (head sizes without this kernel still parse it)
-        float4 qw[KS][2], kw[KS][2], cs[HK][2], sn[HK][2];
-        if (p.q_norm_w != nullptr) {
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    qw[ks][h] = *(const float4*)(p.q_norm_w + ks * 32 + G * 8 + 4 * h);
-                    kw[ks][h] = *(const float4*)(p.k_norm_w + ks * 32 + G * 8 + 4 * h);
-                }
-        }
+        constexpr int ROW_LANES = HD <= 64 ? 8 : HD <= 128 ? 16 : 32, ROWS = IA_WAVE / ROW_LANES, ROW_USED = HD / 8;
+        const int ri = lane % ROW_LANES < ROW_USED ? lane % ROW_LANES : ROW_USED - 1, rsub = lane / ROW_LANES;
+        struct RowPart { uint2 lo, hi; float4 wlo, whi; };
+        auto ask_rows = [&](RowPart& part, int pass) __attribute__((always_inline)) {
+            const int t = pass * ROWS + rsub;
+            const bf16_t* from = token_row + (size_t)(t < n_cols ? kvh * g + col0 + t : p.nq + kvh) * HD + 4 * ri;
+            part.lo = *(const uint2*)from;
+            part.hi = *(const uint2*)(from + HD / 2);
+            if (p.q_norm_w != nullptr) {
+                const float* w = (t < n_cols ? p.q_norm_w : p.k_norm_w) + 4 * ri;
+                part.wlo = *(const float4*)w;
+                part.whi = *(const float4*)(w + HD / 2);
+            }
+        };
+        RowPart rows0, rows1;
+        ask_rows(rows0, 0);
+        float4 cs = make_float4(1.f, 1.f, 1.f, 1.f), sn = make_float4(0.f, 0.f, 0.f, 0.f);
         if (p.cos_t != nullptr) {
-#pragma unroll
-            for (int ks = 0; ks < KS / 2; ++ks)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const size_t a0 = (size_t)t0 * (HD / 2) + ks * 32 + G * 8 + 4 * h;
-                    cs[ks][h] = *(const float4*)(p.cos_t + a0);
-                    sn[ks][h] = *(const float4*)(p.sin_t + a0);
-                }
+            cs = *(const float4*)(p.cos_t + (size_t)t0 * (HD / 2) + 4 * ri);
+            sn = *(const float4*)(p.sin_t + (size_t)t0 * (HD / 2) + 4 * ri);
         }
-
+        if (n_cols + 1 > ROWS) ask_rows(rows1, 1);
 
         // A step's 32 keys are two groups of 16 slots, each inside one page (page sizes are multiples of 16).
         // Slots past the request's length are read like any others as long as their page is the request's (their
         // scores are masked and their values zeroed in the step); pages past its last are not asked for.
-        const int last_idx = (kv_total - 1) / p.page;
+        const int last_idx = page_of(kv_total - 1);
         const bool k_second = r >= 8, v_second = G >= 2;
         const uint32_t k_lane[2] = {(uint32_t)((((8 * (r >> 2) + (r & 3)) & 15) * HD + G * 8) * 2),
                                     (uint32_t)((((8 * (r >> 2) + 4 + (r & 3)) & 15) * HD + G * 8) * 2)};
         const uint32_t v_lane = (uint32_t)((r * p.page + 8 * (G & 1)) * 2);
         const size_t v_stride = (size_t)16 * p.page * 2;
         auto load_pages = [&](DecodeOperands& op, int k0, int page_a, int page_b) __attribute__((always_inline)) {
-            const int off_a = k0 % p.page, off_b = (k0 + 16) % p.page;
+            const int off_a = k0 - page_of(k0) * p.page, off_b = k0 + 16 - page_of(k0 + 16) * p.page;
             const char* ka = (const char*)(p.k_cache + (((size_t)page_a * p.nkv + kvh) * p.page + off_a) * HD);
             const char* kb = (const char*)(p.k_cache + (((size_t)page_b * p.nkv + kvh) * p.page + off_b) * HD);
             const char* va = (const char*)(p.v_cache + ((size_t)page_a * p.nkv + kvh) * HD * p.page + off_a);
@@ -603,82 +621,113 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
             for (int db = 0; db < DB; ++db) op.v[db] = *(const uint4*)(vbase + db * v_stride);
         };
         auto load_step = [&](DecodeOperands& op, int k0) __attribute__((always_inline)) {
-            int idx_a = k0 / p.page, idx_b = (k0 + 16) / p.page;
+            int idx_a = page_of(k0), idx_b = page_of(k0 + 16);
             idx_a = idx_a < last_idx ? idx_a : last_idx;
             idx_b = idx_b < last_idx ? idx_b : last_idx;
             load_pages(op, k0, bt[idx_a], bt[idx_b]);
         };
         // the first two steps, with the pages read ahead where the walk starts at the split's own start
         auto load_early = [&](DecodeOperands& op, int k0, int i) __attribute__((always_inline)) {
-            if (lo == c_lo && (k0 + 16) / p.page <= last_idx) load_pages(op, k0, early[2 * i], early[2 * i + 1]);
+            if (lo == c_lo && page_of(k0 + 16) <= last_idx) load_pages(op, k0, early[2 * i], early[2 * i + 1]);
             else load_step(op, k0);
         };
         const int n_steps = lo < hi ? (hi - lo + 31) / 32 : 0;
         DecodeOperands opa, opb;
         load_early(opa, lo, 0);
 
-        // One head's row, normed and rotated as the separate kernel does it (32-bit throughout, one rounding at
-        // the end): lane (., G) holds the features ks * 32 + G * 8 .. + 8 of the row, and a feature's rotation
-        // partner, HD / 2 further on, lies in the same lane.
-        auto normed_rotated = [&](const uint4 (&raw)[KS], const float4 (&nw)[KS][2], uint4 (&packed)[KS]) __attribute__((always_inline)) {
-            float f[KS][8];
-            float ss = 0.f;
+        const bool has_new = p.slots != nullptr && hi == kv_total && lo < hi;
+        const int slot = has_new ? p.slots[t0] : 0;
+        uint32_t vnew[DB];
+        if (has_new) {
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const uint32_t w[4] = {raw[ks].x, raw[ks].y, raw[ks].z, raw[ks].w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    f[ks][2 * j] = __uint_as_float(w[j] << 16);
-                    f[ks][2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
-                }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) ss += f[ks][j] * f[ks][j];
-            }
-            if (p.q_norm_w != nullptr) {
-                ss += __shfl_xor(ss, 16, IA_WAVE);
-                ss += __shfl_xor(ss, 32, IA_WAVE);
-                const float scale = 1.0f / sqrtf(ss / (float)HD + p.norm_eps);
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks) {
-                    const float gw[8] = {nw[ks][0].x, nw[ks][0].y, nw[ks][0].z, nw[ks][0].w,
-                                         nw[ks][1].x, nw[ks][1].y, nw[ks][1].z, nw[ks][1].w};
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) f[ks][j] = scale * f[ks][j] * (p.norm_add_one ? 1.0f + gw[j] : gw[j]);
-                }
-            }
-            if (p.cos_t != nullptr) {
-#pragma unroll
-                for (int ks = 0; ks < KS / 2; ++ks) {
-                    const float c[8] = {cs[ks][0].x, cs[ks][0].y, cs[ks][0].z, cs[ks][0].w,
-                                        cs[ks][1].x, cs[ks][1].y, cs[ks][1].z, cs[ks][1].w};
-                    const float sv[8] = {sn[ks][0].x, sn[ks][0].y, sn[ks][0].z, sn[ks][0].w,
-                                         sn[ks][1].x, sn[ks][1].y, sn[ks][1].z, sn[ks][1].w};
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const float a = f[ks][j], b = f[ks + KS / 2][j];
-                        f[ks][j] = a * c[j] - b * sv[j];
-                        f[ks + KS / 2][j] = a * sv[j] + b * c[j];
-                    }
-                }
-            }
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-                packed[ks] = make_uint4(pack_bf16x2(f[ks][0], f[ks][1]), pack_bf16x2(f[ks][2], f[ks][3]),
-                                        pack_bf16x2(f[ks][4], f[ks][5]), pack_bf16x2(f[ks][6], f[ks][7]));
-        };
-        uint4 qreg[KS], knew[KS];
-        normed_rotated(qraw, qw, qreg);
-        normed_rotated(kraw, kw, knew);
+            for (int db = 0; db < DB; ++db) vnew[db] = token_row[(size_t)(p.nq + p.nkv + kvh) * HD + db * 16 + r].bits;
+        }
         if (n_steps >= 2) load_early(opb, lo + 32, 1);
 
-        const bool has_new = p.slots != nullptr && hi == kv_total && lo < hi;
+        // Rows, normed and rotated as the separate kernel does it (32-bit throughout, one rounding at the end).  A row's 16-byte
+        // pieces lie exchanged by its number, so that operand reads of several rows meet no bank twice.  They fit where the wave's
+        // partial outputs will lie.
+        char* const row_mem = (char*)(team_mem + (size_t)wave * n_cols * HD);
+        auto form_rows = [&](const RowPart& part, int pass) __attribute__((always_inline)) {
+            const int t = pass * ROWS + rsub;
+            float a[4] = {__uint_as_float(part.lo.x << 16), __uint_as_float(part.lo.x & 0xffff0000u),
+                          __uint_as_float(part.lo.y << 16), __uint_as_float(part.lo.y & 0xffff0000u)};
+            float b[4] = {__uint_as_float(part.hi.x << 16), __uint_as_float(part.hi.x & 0xffff0000u),
+                          __uint_as_float(part.hi.y << 16), __uint_as_float(part.hi.y & 0xffff0000u)};
+            if (p.q_norm_w != nullptr) {
+                float ss = 0.f;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) ss += a[j] * a[j];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) ss += b[j] * b[j];
+                if (ROW_USED != ROW_LANES) ss = lane % ROW_LANES < ROW_USED ? ss : 0.f;
+                ss = row_sum<ROW_LANES>(ss);
+                const float scale = 1.0f / sqrtf(ss / (float)HD + p.norm_eps), one = p.norm_add_one ? 1.0f : 0.0f;
+                const float wa[4] = {part.wlo.x, part.wlo.y, part.wlo.z, part.wlo.w}, wb[4] = {part.whi.x, part.whi.y, part.whi.z, part.whi.w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) { a[j] = scale * a[j] * (wa[j] + one); b[j] = scale * b[j] * (wb[j] + one); }
+            }
+            if (p.cos_t != nullptr) {
+                const float c[4] = {cs.x, cs.y, cs.z, cs.w}, sv[4] = {sn.x, sn.y, sn.z, sn.w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float x = a[j], y = b[j];
+                    a[j] = x * c[j] - y * sv[j];
+                    b[j] = x * sv[j] + y * c[j];
+                }
+            }
+            if (t <= n_cols && lane % ROW_LANES < ROW_USED) {
+                char* const at = row_mem + t * (HD * 2) + (ri & 1) * 8;
+                *(uint2*)(at + ((ri / 2) ^ (t & 7)) * 16) = make_uint2(pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]));
+                *(uint2*)(at + ((HD / 16 + ri / 2) ^ (t & 7)) * 16) = make_uint2(pack_bf16x2(b[0], b[1]), pack_bf16x2(b[2], b[3]));
+            }
+        };
+        const int passes = (n_cols + (has_new ? 1 : 0) + ROWS - 1) / ROWS;
+        form_rows(rows0, 0);
+        if (passes > 1) form_rows(rows1, 1);
+        for (int pass = 2; pass < passes; ++pass) {
+            ask_rows(rows0, pass);
+            form_rows(rows0, pass);
+        }
+        // (the wave's own memory: its shared-memory operations run in program order)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        uint4 qreg[KS];
+        {
+            const int t = cvalid ? r : n_cols - 1;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) qreg[ks] = *(const uint4*)(row_mem + t * (HD * 2) + ((ks * 4 + G) ^ (t & 7)) * 16);
+        }
+        // the new key's features ks * 32 + G * 8 .. + 8
+        auto new_key = [&](int ks) __attribute__((always_inline)) {
+            return *(const uint4*)(row_mem + n_cols * (HD * 2) + ((ks * 4 + G) ^ (n_cols & 7)) * 16);
+        };
 
         f32x4 acc[DB];
         float m = -INFINITY, l = 0.f;
 #pragma unroll
         for (int db = 0; db < DB; ++db) acc[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-        auto compute_step = [&](DecodeOperands& op, int k0) __attribute__((always_inline)) {
+        // What only the walk's first step needs: keys below the window.
+        auto first_edge = [&](DecodeOperands& op, int k0) __attribute__((always_inline)) {
+            if (k0 < window_floor) {
+                // keys below the window may lie in pages that the request has given back: as above
+                const int first_good = window_floor - (k0 + 8 * G);
+                if (first_good > 0) {
+#pragma unroll
+                    for (int db = 0; db < DB; ++db) {
+                        uint32_t w[4] = {op.v[db].x, op.v[db].y, op.v[db].z, op.v[db].w};
+#pragma unroll
+                        for (int j = 0; j < 8; ++j)
+                            if (j < first_good) w[j >> 1] &= (j & 1) ? 0x0000ffffu : 0xffff0000u;
+                        op.v[db] = make_uint4(w[0], w[1], w[2], w[3]);
+                    }
+                }
+            }
+        };
+        // What only its last step needs: the end of the request's keys, and the new one.
+        auto last_edge = [&](DecodeOperands& op, int k0) __attribute__((always_inline)) {
             if (k0 + 32 > kv_total) {
                 // slots beyond the request's length hold anything at all: zero those values so that a probability
                 // of zero times their content stays zero
@@ -694,20 +743,6 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
                     }
                 }
             }
-            if (k0 < window_floor) {
-                // keys below the window may lie in pages that the request has given back: as above
-                const int first_good = window_floor - (k0 + 8 * G);
-                if (first_good > 0) {
-#pragma unroll
-                    for (int db = 0; db < DB; ++db) {
-                        uint32_t w[4] = {op.v[db].x, op.v[db].y, op.v[db].z, op.v[db].w};
-#pragma unroll
-                        for (int j = 0; j < 8; ++j)
-                            if (j < first_good) w[j >> 1] &= (j & 1) ? 0x0000ffffu : 0xffff0000u;
-                        op.v[db] = make_uint4(w[0], w[1], w[2], w[3]);
-                    }
-                }
-            }
             if (has_new && k0 + 32 >= kv_total) {
                 // (values chosen, never addresses: the operands stay in registers)
                 const int kk = kv_total - 1 - k0;
@@ -715,10 +750,11 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
                 const bool first = mine && ((kk >> 2) & 1) == 0, second = mine && ((kk >> 2) & 1) == 1;
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
-                    op.k[0][ks].x = first ? knew[ks].x : op.k[0][ks].x; op.k[0][ks].y = first ? knew[ks].y : op.k[0][ks].y;
-                    op.k[0][ks].z = first ? knew[ks].z : op.k[0][ks].z; op.k[0][ks].w = first ? knew[ks].w : op.k[0][ks].w;
-                    op.k[1][ks].x = second ? knew[ks].x : op.k[1][ks].x; op.k[1][ks].y = second ? knew[ks].y : op.k[1][ks].y;
-                    op.k[1][ks].z = second ? knew[ks].z : op.k[1][ks].z; op.k[1][ks].w = second ? knew[ks].w : op.k[1][ks].w;
+                    const uint4 key = new_key(ks);
+                    op.k[0][ks].x = first ? key.x : op.k[0][ks].x; op.k[0][ks].y = first ? key.y : op.k[0][ks].y;
+                    op.k[0][ks].z = first ? key.z : op.k[0][ks].z; op.k[0][ks].w = first ? key.w : op.k[0][ks].w;
+                    op.k[1][ks].x = second ? key.x : op.k[1][ks].x; op.k[1][ks].y = second ? key.y : op.k[1][ks].y;
+                    op.k[1][ks].z = second ? key.z : op.k[1][ks].z; op.k[1][ks].w = second ? key.w : op.k[1][ks].w;
                 }
                 const int j = kk & 7;
                 const bool vmine = G == (kk >> 3);
@@ -732,6 +768,8 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
                     op.v[db].w = vmine && (j >> 1) == 3 ? (op.v[db].w & keep) | put : op.v[db].w;
                 }
             }
+        };
+        auto compute_step = [&](DecodeOperands& op, int k0) __attribute__((always_inline)) {
             f32x4 s[2];
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
@@ -755,9 +793,7 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
                 }
             }
             float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
-            mx = fmaxf(mx, __shfl_xor(mx, 16, IA_WAVE));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, IA_WAVE));
-            const float m_new = fmaxf(m, mx * p.scale_log2);
+            const float m_new = fmaxf(m, column_max(mx) * p.scale_log2);
             const float m_use = m_new == -INFINITY ? 0.f : m_new;
             const float alpha = __builtin_amdgcn_exp2f(m - m_use);
             float pr[8], psum = 0.f;
@@ -786,11 +822,12 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
                     __builtin_bit_cast(bf16x8, op.v[db]), __builtin_bit_cast(bf16x8, pb), acc[db], 0, 0, 0);
         };
 
-        // The walk: two steps' operands are under way at any time.  Inside the loop every step has a step two
-        // further on, so its loads are unconditional (the compiler counts what is outstanding and waits for the
-        // older set only); the last one to three steps follow it.  opa holds step k0, opb step k0 + 32.
+        // The walk: two steps' operands are under way at any time.  Inside the loop the loads are unconditional (the compiler counts
+        // what is outstanding and waits for the older set only; behind the walk's last step they fetch the request's last page once
+        // more, which is in a cache); the last one or two steps follow it.  opa holds step k0, opb step k0 + 32.
         int k0 = lo, left = n_steps;
-        while (left > 3) {
+        if (left > 0) first_edge(opa, k0);
+        while (left > 2) {
             compute_step(opa, k0);
             load_step(opa, k0 + 64);
             compute_step(opb, k0 + 32);
@@ -798,22 +835,12 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
             k0 += 64;
             left -= 2;
         }
-        if (left == 3) {
-            compute_step(opa, k0);
-            load_step(opa, k0 + 64);
-            compute_step(opb, k0 + 32);
-            k0 += 64;
-            left = 1;
-        }
-        // (the new value's features, for the wave that ends with the new key: asked for here, where they are needed)
-        if (has_new) {
-#pragma unroll
-            for (int db = 0; db < DB; ++db) vnew[db] = token_row[(size_t)(p.nq + p.nkv + kvh) * HD + db * 16 + r].bits;
-        }
         if (left == 2) {
             compute_step(opa, k0);
+            last_edge(opb, k0 + 32);
             compute_step(opb, k0 + 32);
         } else if (left == 1) {
+            last_edge(opa, k0);
             compute_step(opa, k0);
         }
 
@@ -822,13 +849,12 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
         // brought, and now writes them to the cache for the steps to come.  (After the walk: with no store before
         // them, the block table's reads go through the scalar cache.)
         if (has_new) {
-            const int slot = p.slots[t0];
             const int page = slot / p.page, off = slot - page * p.page;
             const int kk = (kv_total - 1) & 31;
             if (r == (((kk >> 3) << 2) | (kk & 3))) {
                 bf16_t* krow = p.k_cache_w + (((size_t)page * p.nkv + kvh) * p.page + off) * HD + G * 8;
 #pragma unroll
-                for (int ks = 0; ks < KS; ++ks) *(uint4*)(krow + ks * 32) = knew[ks];
+                for (int ks = 0; ks < KS; ++ks) *(uint4*)(krow + ks * 32) = new_key(ks);
             }
             if (G == (kk >> 3)) {
                 bf16_t* vdst = p.v_cache_w + (((size_t)page * p.nkv + kvh) * HD + r) * p.page + off;
@@ -837,9 +863,7 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
             }
         }
 
-        float lt = l;
-        lt += __shfl_xor(lt, 16, IA_WAVE);
-        lt += __shfl_xor(lt, 32, IA_WAVE);
+        const float lt = column_sum(l);
         const size_t row0 = (size_t)t0 * p.nq + kvh * g + col0;        // the block's first (token, head) row
         if (p.splits == 1) {
             if (!cvalid) return;
@@ -871,17 +895,23 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
         const int pieces = n_cols * (HD / 4);                           // 16-byte pieces of the block's result
         for (int e = threadIdx.x; e < pieces; e += blockDim.x) {
             const int col = e / (HD / 4), piece = e - col * (HD / 4);
-            float mx = -INFINITY;
-            for (int w = 0; w < team; ++w) mx = fmaxf(mx, team_ml[(w * n_cols + col) * 2]);
-            f32x4 o = (f32x4){0.f, 0.f, 0.f, 0.f};
-            float total = 0.f;
-            for (int w = 0; w < team; ++w) {
-                const float mw = team_ml[(w * n_cols + col) * 2];
-                const float wt = mw == -INFINITY ? 0.f : exp2f(mw - mx);      // a split that held no key of this row
-                const f32x4 v = *(const f32x4*)(team_o + ((size_t)w * n_cols + col) * HD + piece * 4);
-                o[0] = fmaf(v[0], wt, o[0]); o[1] = fmaf(v[1], wt, o[1]);
-                o[2] = fmaf(v[2], wt, o[2]); o[3] = fmaf(v[3], wt, o[3]);
-                total = fmaf(team_ml[(w * n_cols + col) * 2 + 1], wt, total);
+            // (all of the team's results are asked for together)
+            float mw[DECODE_TEAM], lw[DECODE_TEAM], mx = -INFINITY, total = 0.f;
+            f32x4 v[DECODE_TEAM], o = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < DECODE_TEAM; ++w) {
+                const int at = (w < team ? w : 0) * n_cols + col;
+                mw[w] = team_ml[at * 2];
+                lw[w] = team_ml[at * 2 + 1];
+                v[w] = *(const f32x4*)(team_o + (size_t)at * HD + piece * 4);
+                mx = fmaxf(mx, mw[w]);
+            }
+#pragma unroll
+            for (int w = 0; w < DECODE_TEAM; ++w) {
+                const float wt = w >= team || mw[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw[w] - mx);      // (a split that held no key of this row)
+                o[0] = fmaf(v[w][0], wt, o[0]); o[1] = fmaf(v[w][1], wt, o[1]);
+                o[2] = fmaf(v[w][2], wt, o[2]); o[3] = fmaf(v[w][3], wt, o[3]);
+                total = fmaf(lw[w], wt, total);
             }
             if (teams == 1) {
                 const float inv = 1.0f / (p.sink ? total + sink_term(p.sinks, (int)((row0 + col) % p.nq), mx) : total);
@@ -934,17 +964,36 @@ __global__ __launch_bounds__(4 * IA_WAVE) void attn_decode_kernel(const AttnPara
             if (active) {
                 const float* ml = p.part_ml + (row0 + col) * teams * 2;
                 const float* po = p.part_o + (row0 + col) * teams * HD + piece * 4;
-#pragma unroll 8
-                for (int t = grp; t < teams; t += groups) {
-                    const float2 mt = make_float2(get_across(ml + 2 * t), get_across(ml + 2 * t + 1));
-                    const float* pv = po + (size_t)t * HD;
-                    const f32x4 v = (f32x4){get_across(pv), get_across(pv + 1), get_across(pv + 2), get_across(pv + 3)};
-                    const float m_new = fmaxf(mx, mt.x);
-                    const float back = m_new == -INFINITY ? 0.f : exp2f(mx - m_new);        // rescales what is summed so far
-                    const float wt = mt.x == -INFINITY ? 0.f : exp2f(mt.x - m_new);
-                    o[0] = fmaf(v[0], wt, o[0] * back); o[1] = fmaf(v[1], wt, o[1] * back);
-                    o[2] = fmaf(v[2], wt, o[2] * back); o[3] = fmaf(v[3], wt, o[3] * back);
-                    total = fmaf(mt.y, wt, total * back);
+                // (eight blocks' results at a time, their loads under way together and one change of the maximum for all)
+                constexpr int AT_ONCE = 8;
+                for (int t1 = grp; t1 < teams; t1 += AT_ONCE * groups) {
+                    float mt[AT_ONCE], lt_[AT_ONCE], m_new = mx;
+                    f32x4 v[AT_ONCE];
+#pragma unroll
+                    for (int i = 0; i < AT_ONCE; ++i) {
+                        const int t = t1 + i * groups;
+                        mt[i] = -INFINITY;
+                        lt_[i] = 0.f;
+                        v[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                        if (t < teams) {
+                            const float* pv = po + (size_t)t * HD;
+                            mt[i] = get_across(ml + 2 * t);
+                            lt_[i] = get_across(ml + 2 * t + 1);
+                            v[i] = (f32x4){get_across(pv), get_across(pv + 1), get_across(pv + 2), get_across(pv + 3)};
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < AT_ONCE; ++i) m_new = fmaxf(m_new, mt[i]);
+                    const float back = m_new == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mx - m_new);       // rescales what is summed so far
+                    o[0] *= back; o[1] *= back; o[2] *= back; o[3] *= back;
+                    total *= back;
+#pragma unroll
+                    for (int i = 0; i < AT_ONCE; ++i) {
+                        const float wt = mt[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mt[i] - m_new);
+                        o[0] = fmaf(v[i][0], wt, o[0]); o[1] = fmaf(v[i][1], wt, o[1]);
+                        o[2] = fmaf(v[i][2], wt, o[2]); o[3] = fmaf(v[i][3], wt, o[3]);
+                        total = fmaf(lt_[i], wt, total);
+                    }
                     mx = m_new;
                 }
             }
@@ -1614,7 +1663,7 @@ static size_t decode_team_bytes(int team, int g) {
     return (waves > groups ? waves : groups) * sizeof(float);
 }
 static int decode_team(int splits, int g) {
-    const int team = decode_team_bytes(4, g) <= 65536 ? 4 : 2;
+    const int team = decode_team_bytes(DECODE_TEAM, g) <= 65536 ? DECODE_TEAM : 2;
     return splits >= team ? team : splits;
 }
 
@@ -1674,7 +1723,7 @@ static int attention_launch(void* out, float* workspace, const void* q, const vo
     IA_CHECK(mask_chunk >= 0 && (sinks == nullptr || sink), "attention_mfma: mask_chunk %d must be >= 0 (0 = none), and sink values go with a sink", mask_chunk);
     p.sinks = sinks; p.mask_chunk = mask_chunk;
     IA_CHECK(keep_first >= 0 && softcap >= 0.f, "attention_mfma: keep_first %d and softcap %g must be >= 0 (0 = none)", keep_first, (double)softcap);
-    p.keep_first = keep_first; p.cap_in = 0.f;
+    p.keep_first = keep_first; p.cap_in = 0.f; p.page_magic = 0; p.page_shift = 0; p.teams_log2 = 0;
     if (softcap > 0.f) {
         p.cap_in = scale / softcap * (2.0f * 1.4426950408889634f);
         p.scale_log2 = softcap * 1.4426950408889634f;
@@ -1708,7 +1757,13 @@ static int attention_launch(void* out, float* workspace, const void* q, const vo
         IA_CHECK((long long)nkv * teams <= 65535, "attention_mfma: grid too large (nkv*blocks=%d)", nkv * teams);
         p.part_ml = workspace ? workspace + (size_t)n * nq * teams * HD : nullptr;
         const dim3 fgrid((unsigned)col_blocks, nkv * teams, n_seqs);
-        const size_t shared = team > 1 ? decode_team_bytes(team, g) : 0;
+        const size_t shared = decode_team_bytes(team, g);
+        p.teams_log2 = __builtin_ctz((unsigned)teams);
+        // With d = page / 16 and 2^(s - 1) < d <= 2^s, M = 2^(31 + s) / d rounded up fits 32 bits and exceeds the quotient by less than
+        // 2^s / d parts of 2^-(31 + s): q M >> (31 + s) is q / d for every q = pos / 16 below 2^27, hence for every position.
+        const uint32_t d16 = (uint32_t)page_size / 16;
+        p.page_shift = d16 > 1 ? 32 - __builtin_clz(d16 - 1) : 0;
+        p.page_magic = (uint32_t)(((1ULL << (31 + p.page_shift)) + d16 - 1) / d16);
         attn_decode_kernel<><<<fgrid, team * IA_WAVE, shared, stream>>>(p, fused->counters, team);
         IA_LAUNCH_CHECK("attention_decode");
         return 0;

@@ -545,11 +545,11 @@ def decode_split(n_seqs: int, nkv: int, g: int, max_kv_len: int) -> Tuple[int, i
     (request x kv head x 16 query heads x split) within one round of the chip and a wave's share at 64 keys
     or more; beyond 32 splits (eight blocks to merge) only where a share would exceed 128 keys.  Measured at head
     size 128, 32 query and 8 kv heads, context 8,192 (microseconds a layer): batch 1
-    18.0 with 64 splits against 20.0 with 128, batch 3 27.6 with 32 against 34.1 with 64, batch 8 52.4 with 16
-    against 55.5 with 32, batch 64 358 with 2 against 375 with 4.  Shares of 64 keys against 128, the kernel called
-    back to back in a graph: batch 1 at a context of 1,024 11.3 against 13.0, of 2,048 12.4 against 13.7; batch 4
-    at 2,048 14.3 against 15.9; batch 8 at 1,024 13.3 against 14.6; at a context of 512 four splits are as good as
-    any (10.8), and 64 splits of 64 keys at 4,096 lose to 32 of 128 (batch 2: 17.0 against 16.0)."""
+    17.8 with 64 splits against 21.3 with 32, batch 4 31.1 with 32 against 36.6 with 16, batch 8 51.2 with 16
+    against 56.5 with 32, batch 64 at 1,500 72.0 with 2 against 71.2 with 4 and 82 with 8.  Shares of 64 keys against 128:
+    batch 1 at 2,048 9.3 against 11.8; batch 4 12.6 against 14.1; batch 8 17.6 against 21.1; and 64 splits of 64 keys at 4,096 lose
+    to 32 of 128 (batch 2, an earlier kernel: 17.0 against 16.0).  Shares of 32 keys at a bound of 1,024 are worth 0.2 to 1.0 us to one
+    to four requests (16 query heads, batch 1, 700 keys 8.0 against 8.7) and lose at eight (12.6 against 11.3): not taken."""
     items = n_seqs * nkv * -(-g // 16)
     min_chunk = DECODE_MIN_CHUNK if max_kv_len > 512 else 128
     splits = 1

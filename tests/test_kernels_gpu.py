@@ -842,6 +842,35 @@ def test_attention_decode_fused_is_the_three_kernels_in_one(nq, nkv, d, page, wi
         assert counters is None or int(counters.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("nq,nkv,d,page,window", [
+    (3, 1, 128, 16, None), (8, 2, 128, 112, 40), (7, 1, 128, 16, None), (8, 1, 128, 32, 95),    # the new key in the first pass over
+    (16, 1, 128, 16, None), (17, 1, 64, 48, None), (5, 1, 192, 16, 33), (2, 1, 256, 80, None)])  # the rows, the second, a third, a last of its own
+def test_attention_decode_rows_and_walks_of_every_length(nq, nkv, d, page, window):
+    from inferrs_amd import ops
+    lens = [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 223]          # one to seven steps of 32 keys, their last one full or not
+    q, kc, vc, positions, token_seq, table = attention_case(torch.bfloat16, nq, nkv, d, page, lens, [1] * len(lens), 29)
+    n, scale = len(lens), 1.0 / math.sqrt(d)
+    qkv = dev(randn(n, (nq + 2 * nkv) * d, dtype=torch.bfloat16, seed=5))
+    qw, kw = dev(1 + 0.3 * randn(d, dtype=torch.float32, seed=6)), dev(1 + 0.3 * randn(d, dtype=torch.float32, seed=7))
+    ang = positions.float()[:, None] / 10000.0 ** (torch.arange(0, d, 2, dtype=torch.float32) / d)
+    cos, sin = dev(torch.cos(ang)), dev(torch.sin(ang))
+    slots = dev(torch.tensor([int(table[s, (l - 1) // page]) * page + (l - 1) % page for s, l in enumerate(lens)], dtype=torch.int32))
+    cu, table, positions = dev(torch.arange(n + 1, dtype=torch.int32)), dev(table), dev(positions)
+    k1, v1 = dev(kc), dev(vc)
+    q1 = ops.qk_rope_kv(qkv, nq, nkv, d, q_norm_w=qw, k_norm_w=kw, eps=1e-5, add_one=True, cos=cos, sin=sin, rot=d, interleaved=False,
+                        k_cache=k1, v_cache=v1, slots=slots, page_size=page)
+    want = ops.attention_generic(q1, k1, v1, positions, dev(token_seq), table, window=window, scale=scale).float().cpu()
+    for splits in (1, 2, 8):
+        k2, v2 = dev(kc), dev(vc)
+        got = ops.attention_decode_fused(qkv, k2, v2, positions, cu, table, nq=nq, nkv=nkv, d=d, slots=slots, q_norm_w=qw, k_norm_w=kw,
+                                         eps=1e-5, add_one=True, cos=cos, sin=sin, max_kv_len=max(lens), window=window, scale=scale,
+                                         splits=splits).float().cpu()
+        close(got, want, 2 ** -7, f"splits={splits}")
+        assert torch.equal(v2, v1)
+        dk = (k2.float() - k1.float()).abs()                # (the same but for a last bit: the sum of squares in another order)
+        assert float(dk.max()) <= 2 ** -7 * float(k1.float().abs().max()) and float((dk > 0).float().mean()) < 1e-3
+
+
 def test_attention_decode_merge_is_the_same_every_time():
     """The blocks of a (request, key/value head) finish in any order and the last one merges: the sum runs in the
     order of the splits, so twenty calls give the same bits, and so does a call captured in a graph and replayed."""
