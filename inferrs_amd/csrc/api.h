@@ -130,6 +130,8 @@ int ia_gemm_mid_tune(int kc, int ns);
 // (how a block's waves share its products, for measurements and tests: 0 the kernel's own rule, 1 a tile of weight rows a
 // wave over all rows of the step, 2 two tiles a wave over half of the rows wherever the shape allows; the same bits)
 int ia_gemm_mid_blocking(int how);
+// (tiles of 16 rows a block takes at most, 1 to 8, for measurements and tests; 0: the kernel's own rule; the same bits)
+int ia_gemm_mid_rows(int tiles);
 // (a fixed shape of the blocks for measurements and tests: waves a block, 2 to 8 (0: the kernel's own rule), ways k is split
 // and stages, 2 or 3 (2: four waves only); the caller's partial sums must have as many splits); a shape that has no
 // kernel is an error and changes nothing

@@ -21,8 +21,8 @@
 // rows) in lane order, and the lane picks the piece it fetches accordingly.
 //
 // How many waves a block has and how k is split follow from the weight's shape (mid_plan below): the chip should get a block
-// for every compute unit and no more, three stages deep; a weight that no such shape fits takes four waves a block, two
-// stages and several blocks a unit.
+// for every compute unit and no more, three stages deep; a weight of more blocks than that takes four waves a block, two
+// stages and several blocks a unit.  A small weight's blocks take the step's rows in groups (mid_row_tiles).
 //
 // The weights went straight from memory into the A-operands before (a load of 16 rows x 64 bytes a lane group): such a
 // load holds the compute unit's address unit for about 86 cycles, a load of 1 KiB in whole rows for about 32, and by its
@@ -58,7 +58,7 @@ enum { MID_OUT_BF16 = 0, MID_OUT_F32 = 1, MID_OUT_PARTIAL = 2 };
 // shared memory (swap_up, in a stage's place) to the waves that hold the gate rows' sums of the same features.
 template <int MT, bool DUAL, int TILES>
 __device__ __forceinline__ void mid_finish(gmid_f32x4 (&acc)[MT], gmid_f32x4* swap_up, void* out, int out_mode,
-                                           int M, int N, int lane, int r, int g, int tile, int part, int n_first, int split,
+                                           int M, int rows, int N, int lane, int r, int g, int tile, int part, int n_first, int split,
                                            int act) {
     constexpr int FEATURE_TILES = DUAL ? TILES / 2 : TILES;
     if (DUAL) __syncthreads();                                            // everybody is done with the stages
@@ -73,7 +73,7 @@ __device__ __forceinline__ void mid_finish(gmid_f32x4 (&acc)[MT], gmid_f32x4* sw
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             const int m = mt * 16 + r;
-            if (m >= M) continue;
+            if (m >= rows) continue;
             const gmid_f32x4 up = swap_up[(tile * MT + mt) * IA_WAVE + lane];
             float v[4];
 #pragma unroll
@@ -97,7 +97,7 @@ __device__ __forceinline__ void mid_finish(gmid_f32x4 (&acc)[MT], gmid_f32x4* sw
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         const int m = mt * 16 + r;
-        if (m >= M) continue;
+        if (m >= rows) continue;
         if (out_mode == MID_OUT_BF16) {
             bf16_t* o = (bf16_t*)out + (size_t)m * N + nb;
             if (nb + 3 < N && (N & 3) == 0) {
@@ -125,11 +125,11 @@ __device__ __forceinline__ void mid_finish(gmid_f32x4 (&acc)[MT], gmid_f32x4* sw
 // exchanged; otherwise the features n_first .. + 32.  The arithmetic is mid_finish's.
 template <int MH, bool DUAL>
 __device__ __forceinline__ void mid_finish_paired(gmid_f32x4 (&acc0)[MH], gmid_f32x4 (&acc1)[MH], void* out, int out_mode,
-                                                  int M, int N, int r, int g, int mt_first, int n_first, int split, int act) {
+                                                  int M, int rows, int N, int r, int g, int mt_first, int n_first, int split, int act) {
 #pragma unroll
     for (int mt = 0; mt < MH; ++mt) {
         const int m = (mt_first + mt) * 16 + r;
-        if (m >= M) continue;
+        if (m >= rows) continue;
         if (DUAL) {
             const int nb = n_first + 4 * g;
             float v[4];
@@ -216,6 +216,10 @@ __global__ __launch_bounds__(W * IA_WAVE) void gemm_mid_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / IA_WAVE);
     const int r = lane & 15, g = lane >> 4;
     const int tile = wave;
+    // the block's rows: 16 MT of the step's from m_first on (gridDim.z groups of them, see launch_mid)
+    const int m_first = blockIdx.z * X_ROWS, rows = M - m_first < X_ROWS ? M - m_first : X_ROWS;
+    x += (size_t)m_first * K;
+    out = (char*)out + (size_t)m_first * N * (out_mode == MID_OUT_BF16 ? 2 : 4);
     const int split = blockIdx.y;
     const int k_begin = split * k_per_block;
     const int k_len = K - k_begin < k_per_block ? K - k_begin : k_per_block;
@@ -264,7 +268,7 @@ __global__ __launch_bounds__(W * IA_WAVE) void gemm_mid_kernel(
         const int piece = (lane % PIECES) ^ swizzle(row);
         const bf16_t* base;
         if (row < X_ROWS || row >= ROWS) {
-            base = x + (size_t)(row < M ? row : 0) * K;                   // (rows beyond the step read row 0: never stored)
+            base = x + (size_t)(row < rows ? row : 0) * K;                 // (rows beyond the step read row 0: never stored)
         } else {
             const int wr = row - X_ROWS, t = wr / 16;                          // weight row of the block: tile t, row wr % 16
             const int pt = DUAL ? t / FEATURE_TILES : 0;
@@ -390,9 +394,9 @@ __global__ __launch_bounds__(W * IA_WAVE) void gemm_mid_kernel(
     }
     if constexpr (PAIRED) {
         const int n_pair = blockIdx.x * (16 * FEATURE_TILES) + (DUAL ? 16 : 32) * pair;
-        mid_finish_paired<MH, DUAL>(acc, acc1, out, out_mode, M, N, r, g, mt_first, n_pair, split, act);
+        mid_finish_paired<MH, DUAL>(acc, acc1, out, out_mode, M, rows, N, r, g, mt_first, n_pair, split, act);
     } else {
-        mid_finish<MT, DUAL, TILES>(acc, (gmid_f32x4*)mid_s1, out, out_mode, M, N, lane, r, g, tile, part, n_first, split, act);
+        mid_finish<MT, DUAL, TILES>(acc, (gmid_f32x4*)mid_s1, out, out_mode, M, rows, N, lane, r, g, tile, part, n_first, split, act);
     }
 }
 
@@ -416,16 +420,16 @@ static int mid_cus() {
     return cus;
 }
 
-struct MidPlan { int waves, splits, stages; };
+struct MidPlan { int waves, splits, stages; double fill; };     // fill: see mid_plan
 // a plan for measurements and tests: waves (0: the rule), splits, stages
-static MidPlan g_mid_forced = {0, 0, 0};
+static MidPlan g_mid_forced = {0, 0, 0, 0.0};
 #define MID_MAX_WAVES 8
 extern "C" int ia_gemm_mid_plan(int waves, int splits, int stages) {
     IA_CHECK(waves == 0 || (waves >= 2 && waves <= MID_MAX_WAVES && splits >= 1 && splits <= 16 && (splits & (splits - 1)) == 0
                             && (stages == 3 || (waves == 4 && stages == 2))),
              "gemm_mid_plan: no block of %d waves with %d splits of k, %d stages deep (2 to 8 waves, 2^k splits up to 16, "
              "3 stages, or 4 waves with 2; 0 waves: the plan's own)", waves, splits, stages);
-    g_mid_forced = {waves, splits, stages};
+    g_mid_forced = {waves, splits, stages, stages == 3 ? 1.0 : 0.0};
     return 0;
 }
 
@@ -434,7 +438,7 @@ static MidPlan mid_plan(int N, int K, bool dual) {
     const int tiles = (N + 15) / 16;                       // of a part
     const int chunks = K / MID_CHUNK_MIN_K;
     if (g_mid_forced.waves > 0) return g_mid_forced;
-    MidPlan best = {0, 0, 0};
+    MidPlan best = {0, 0, 0, 0.0};
     double best_fill = 0.0;
     bool best_long = false;
     for (int t = 1; t <= (dual ? MID_MAX_WAVES / 2 : MID_MAX_WAVES); ++t) {
@@ -445,24 +449,31 @@ static MidPlan mid_plan(int N, int K, bool dual) {
             if ((long long)blocks * splits > cus) break;
             // the share of the chip's compute units that get a block, times the share of a block's tiles that are real
             const double fill = (double)blocks * splits / cus * ((double)tiles / ((double)blocks * t));
+            // (blocks of two waves under an activation: only where they fill the chip.  2 x 3,072 x 1,024, 117 rows in groups: 10.1 us, 8.9 by
+            // blocks of four)
+            if (dual && t == 1 && fill < 0.9) continue;
             const bool is_long = chunks / splits >= 8;
             const bool better = fill > best_fill + 0.02 || (fill > best_fill - 0.02 && (is_long || !best_long));
             if (best.waves == 0 || better) {
-                best = {dual ? 2 * t : t, splits, 3};
+                best = {dual ? 2 * t : t, splits, 3, fill};
                 best_fill = fill > best_fill ? fill : best_fill;
                 best_long = is_long;
             }
         }
     }
-    if (best.waves != 0 && best_fill >= 0.9) return best;
+    // A weight that one round of blocks covers: three stages deep also where some units get no block (0.3 of the chip is the smallest
+    // share that was measured).  (Blocks of four waves two stages
+    // deep, several a unit, had taken those weights: 2 x 9,728 x 2,560, 0.79 of the chip, 24 rows 27.7 -> 22.0 us, 64 rows 33.4 -> 25.2, 117 rows
+    // 51.5 -> 34.5; 2 x 6,144 x 2,048, 0.75, 18.0 -> 13.2, 19.8 -> 15.1, 20.7 -> 20.3; 2,560 x 9,728, 0.84, 18.8 -> 12.8, 20.8 -> 17.1, 22.0 -> 22.6.)
+    if (best.waves != 0 && best_fill >= 0.3) return best;
     // Four rounds and more of blocks of eight waves (a logits head): the rows of x are fetched half as often as by blocks of
     // four, and three stages hide the memory better than a second block.  The head alone, five vocabularies of 131,072 to 262,144, the
     // time of blocks of four / eight waves in the mean: 5,120 k 24 rows 1.05, 64 rows 1.08, 128 rows 1.21, 4,096 k 1.02, 1.08, 1.21,
     // 2,560 k 1.04, 1.05, 1.24.  Over a short k inside decode steps of two layers, the step by four / by eight: 1,024 k, 151,936 features,
     // 20 rows 197 / 195 us, 64 rows 235 / 233, 96 rows 249 / 255, 128 rows 308 / 289, 2,048 k 278 / 278, 322 / 320, 351 / 347, 408 / 383;
     // over four vocabularies 1.05 to 1.08 at 112 and 128 rows, up to 96 rows 0.96 (200,064 features of 1,024 k at 80 and 96) to 1.02.
-    if (!dual && tiles >= 4 * 8 * cus) return {8, 1, 3};
-    MidPlan wide = {4, 1, 2};
+    if (!dual && tiles >= 4 * 8 * cus) return {8, 1, 3, 1.0};
+    MidPlan wide = {4, 1, 2, 0.0};
     if (!dual) {
         const int blocks = (N + 63) / 64;
         while (blocks * wide.splits < cus && wide.splits < 16 && chunks % (2 * wide.splits) == 0 && chunks / (2 * wide.splits) >= 4)
@@ -474,7 +485,7 @@ static MidPlan mid_plan(int N, int K, bool dual) {
 // Whether the weight's blocks fill the chip evenly, one a compute unit, three stages deep (dual: [gate; up] of N features).
 extern "C" int ia_gemm_mid_fills(int N, int K, int dual) {
     if (N <= 0 || K <= 0 || K % MID_CHUNK_MIN_K) return 0;
-    return mid_plan(N, K, dual != 0).stages == 3;
+    return mid_plan(N, K, dual != 0).fill >= 0.9;
 }
 
 extern "C" int ia_gemm_mid_splits(int N, int K) {
@@ -510,13 +521,13 @@ static int launch_mid(void* out, int out_mode, const bf16_t* x, const bf16_t* w,
     MidPlan plan = mid_plan(N, K, DUAL);
     if (out_mode != MID_OUT_PARTIAL && !DUAL && plan.splits != 1) {
         // a stored product cannot be split: four waves a block over all of k
-        plan = {4, 1, 2};
+        plan = {4, 1, 2, 0.0};
     }
-    if (g_mid_kc != 0 && MT <= 4) plan = {4, DUAL || out_mode != MID_OUT_PARTIAL ? 1 : plan.splits, g_mid_ns};
+    if (g_mid_kc != 0 && MT <= 4) plan = {4, DUAL || out_mode != MID_OUT_PARTIAL ? 1 : plan.splits, g_mid_ns, 0.0};
     const int kc = g_mid_kc != 0 ? g_mid_kc : 4;
     IA_CHECK(plan.splits == splits, "gemm_mid: the plan's %d splits against the caller's %d", plan.splits, splits);
     const int features = 16 * plan.waves / (DUAL ? 2 : 1);            // output features of a block
-    const dim3 grid((N + features - 1) / features, splits);
+    const dim3 grid((N + features - 1) / features, splits, (M + 16 * MT - 1) / (16 * MT));
     // every block's share of k is whole chunks (a share that is not would lose its tail and start off the loads' alignment)
     IA_CHECK(splits >= 1 && K % (splits * MID_CHUNK_MIN_K) == 0, "gemm_mid: K=%d does not split %d ways in multiples of %d",
              K, splits, MID_CHUNK_MIN_K);
@@ -582,6 +593,35 @@ static int launch_mid(void* out, int out_mode, const bf16_t* x, const bf16_t* w,
     return 0;
 }
 
+// ia_gemm_mid_rows(tiles): the tiles of 16 rows that a block takes, at most (0: the rule below; for measurements and tests).
+static int g_mid_rows = 0;
+extern "C" int ia_gemm_mid_rows(int tiles) {
+    IA_CHECK(tiles >= 0 && tiles <= 8, "gemm_mid_rows: 1 to 8 tiles of 16 rows (0: the rule), got %d", tiles);
+    g_mid_rows = tiles;
+    return 0;
+}
+
+// Tiles of 16 rows that a block takes: all of the step's where the weight's blocks give most of the chip's compute units one.  A
+// smaller weight leaves units idle while its blocks bring every row of x for themselves and wait out each stage alone; its rows
+// are shared out in as many groups as give the units a block each, two of a weight of up to 16 MiB, which the caches hold
+// for the groups' blocks.  The bits are the same: each sum's order follows from the weight's shape.
+// us, all rows a block / in groups, at 24, 64 and 117 rows: 2 x 3,072 x 1,024 (96 blocks, two stages) 10.0 / 6.6, 12.2 / 7.5, 13.0 / 9.3;
+// 1,024 x 2,048 (128 blocks) 4.0 / 3.2, 4.9 / 3.6, 6.7 / 4.5; 1,024 x 3,072 4.5 / 3.7, 5.6 / 4.1, 8.0 / 5.2; 4,096 x 1,024 (256 blocks, two
+// groups) 4.6 / 4.0, 5.6 / 5.2, 7.8 / 7.2; not taken at 21 MB, 2,560 x 4,096 (256 blocks) 7.3 / 8.9, 9.0 / 11.1, nor at 50 MB, 2 x 6,144 x 2,048
+// (192 blocks) 13.2 / 14.3, 15.1 / 17.3.
+static int mid_row_tiles(int M, int N, int K, bool dual, int splits) {
+    const int mt = (M + 15) / 16;
+    if (g_mid_rows) return g_mid_rows < mt ? g_mid_rows : mt;
+    MidPlan plan = mid_plan(N, K, dual);
+    if (plan.splits != splits) plan = {4, 1, 2, 0.0};
+    const int features = 16 * plan.waves / (dual ? 2 : 1);
+    const long long blocks = (long long)((N + features - 1) / features) * splits;
+    const long long bytes = (long long)(dual ? 2 : 1) * N * K * 2;
+    const long long fit = (bytes <= (16LL << 20) ? 2 : 1) * mid_cus() / blocks;
+    const int groups = fit < mt ? (int)fit : mt;
+    return groups > 1 ? (mt + groups - 1) / groups : mt;
+}
+
 // out_mode 0: out [M, N] bfloat16; 1: out [M, N] float; 2: out [splits][M][N] float with splits =
 // ia_gemm_mid_splits(N, K), to be added up by the reader.  dual (an activation, IA_ACT_*): w = [gate; up] of N rows each, out = act(x . gate^T)
 // * (x . up^T) in bfloat16 (mode 0 only).  M in 1..128, K a multiple of 128.
@@ -600,7 +640,7 @@ extern "C" int ia_gemm_mid_bf16_scaled(void* out, const void* x, const void* w, 
     const int splits = out_mode == MID_OUT_PARTIAL && !dual ? mid_plan(N, K, false).splits : 1;
     const bf16_t* xb = (const bf16_t*)x;
     const bf16_t* wb = (const bf16_t*)w;
-    const int mt = (M + 15) / 16;
+    const int mt = mid_row_tiles(M, N, K, dual != 0, splits);
     int rc = 0;
     if (dual) {
         if (mt == 1) rc = launch_mid<1, true>(out, out_mode, xb, wb, M, N, K, 1, sums_in, n_sums, eps, dual, stream);

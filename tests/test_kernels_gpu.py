@@ -711,6 +711,36 @@ def test_skinny_variants_for_one_round_weights_agree_bit_for_bit():
                            part), (lo, hi)
 
 
+@pytest.mark.parametrize("n,k,dual", [(3072, 1024, True), (1024, 3072, False), (1000, 512, False), (9728, 2560, True), (2560, 9728, False)])
+def test_mid_products_of_rows_in_groups_have_the_same_bits(n, k, dual):
+    # groups of 1 to 8 tiles of rows a block, the last one not full, and the rule's own choice
+    from inferrs_amd import ops
+    lib = ops.library()
+    w = dev(randn((2 if dual else 1) * n, k, dtype=torch.bfloat16, seed=n, scale=0.05))
+    for m in (17, 33, 64, 65, 100, 128):
+        x = dev(randn(m, k, dtype=torch.bfloat16, seed=m))
+
+        def product(partial):
+            got = ops.gemm_mid_bf16(x, w, dual=dual, partial=partial)
+            return got.parts if isinstance(got, ops.Partials) else got
+
+        try:
+            lib.ia_gemm_mid_rows(8)
+            want = [product(False), product(not dual)]
+            exact = x.double() @ w.double().t()
+            if dual:
+                g = exact[:, :n].to(torch.bfloat16).double()
+                exact = g / (1 + torch.exp(-g)) * exact[:, n:].to(torch.bfloat16).double()
+            close(want[0], exact, 2 ** -6, f"{m} rows")
+            for tiles in (1, 2, 3, 5, 0):
+                lib.ia_gemm_mid_rows(tiles)
+                for a, b in zip((product(False), product(not dual)), want):
+                    assert torch.equal(a, b), (m, tiles)
+        finally:
+            lib.ia_gemm_mid_rows(0)
+    assert lib.ia_gemm_mid_rows(9) != 0 and b"gemm_mid_rows" in lib.ia_last_error()
+
+
 @pytest.mark.parametrize("n,k,blocks", [
     (1024, 1024, 64), (1024, 3072, 128),            # ranges of 4 and 12 steps a wave
     (1000, 4096, 37), (77, 544, 5),                 # whole chunks of 16; fewer features than the last block holds, a short last wave
