@@ -1005,14 +1005,16 @@ MID_MIN_ROWS = 5              # fewest rows for which a split product is worth t
 
 def mid_from_rows(width: int) -> int:
     """Rows of a step from which the products of a model of this width (the residual stream's) run on gemm_mid.hip.
-    Measured, decode steps at a context of 2,048 (ms a step, skinny products against gemm_mid.hip): width 4,096 (8B
-    shape) 6 rows 4.72 / 4.89, 8 rows 3.99 / 4.00, 9 rows 4.27 / 4.22, 12 rows 4.40 / 4.34, 16 rows 4.69 / 4.56; width
-    5,120, where the skinny product's blocks are no whole tiles and its waves' shares of k are uneven (14B shape): 4 rows
-    6.50 / 6.52, 6 rows 6.85 / 6.71, 8 rows 7.13 / 6.94, 12 rows 8.12 / 7.39, 16 rows 9.49 / 7.78 (32B shape: 8 rows 15.09 /
-    14.26, 16 rows 19.10 / 15.42)."""
+    Measured, decode steps at a context of 700, the step's time on gemm_mid.hip over that with the skinny products: width 1,024
+    (0.6B shape) 8 rows 1.18, 12 rows 1.15, 16 rows 1.11; 2,048 (1.7B) 8 rows 1.06, 12 rows 1.02, 16 rows 0.97; 4,096 (8B) 8 rows 1.04,
+    10 rows 1.01, 12 rows 1.00, 16 rows 0.99.  A width that is no power of two leaves the skinny product's waves uneven shares of k and
+    blocks that are no whole tiles: 2,560 (4B) 5 rows 1.00, 6 rows 0.98, 10 rows 0.93, 16 rows 0.89; 5,120 (14B) 5 rows 1.03, 6 rows 1.00,
+    8 rows 0.99, 16 rows 0.89.  (Narrower powers of two were not measured and stay at 9.)"""
     if MID_FROM_ROWS is not None:
         return MID_FROM_ROWS
-    return 9 if width & (width - 1) == 0 else MID_MIN_ROWS
+    if width & (width - 1) == 0:
+        return 9 if width < 1024 else 17 if width < 2048 else 13
+    return MID_MIN_ROWS if width < 4096 else 6
 # [gate; up] weights beyond this many bytes go to the vendor's GEMM and the SiLU kernel also at 17 to 64 rows.  Measured at 32
 # rows (kernel after kernel, launch gaps included): 2 x 12,288 x 4,096 (201 MB) 49 us here against 49 + 5 us there,
 # 2 x 25,600 x 5,120 (524 MB) 125 us here against 96 + 5 us there; the plain products are faster here at every size
