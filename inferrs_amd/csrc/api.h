@@ -64,6 +64,12 @@ int ia_attention_generic(void* out, const void* q, const void* k_cache, const vo
                          float scale, int dtype, float* workspace, int max_kv_len, int sink, int mask_chunk,
                          const float* sinks, int keep_first, float softcap, hipStream_t stream);
 long long ia_attention_generic_workspace(int n, int nq, int nkv, int d, int dv, int max_kv_len);
+// The same for portions of prompts in 32 bits (requests of several tokens, neighbours in the step), where it fits: the same bits
+int ia_attention_portions_f32_fits(int n, int nq, int nkv, int d, int dv, int page_size, int max_kv_len);
+int ia_attention_portions_f32(void* out, const void* q, const void* k_cache, const void* v_cache, const int* positions,
+                              const int* token_seq, const int* block_table, int n, int max_pages, int nq, int nkv, int d,
+                              int page_size, int window, float scale, int max_kv_len, int sink, int mask_chunk,
+                              const float* sinks, int keep_first, float softcap, hipStream_t stream);
 
 // ia_qk_rope_kv on projections still split along their k, [splits][n][(nq + 2 nkv) d] 32-bit sums (bfloat16 caches)
 int ia_qk_rope_kv_partials(void* q_out, void* k_cache, void* v_cache, const float* parts, int splits, const float* q_norm_w,

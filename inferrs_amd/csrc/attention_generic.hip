@@ -500,3 +500,256 @@ extern "C" int ia_attention_generic(void* out, const void* q, const void* k_cach
     }
     return 0;
 }
+
+// ---- portions of prompts in 32 bits, on the matrix cores ---------------------------------------------------------
+// What the kernel above does with a wave a token and key/value head, 16 (token, query head) columns a wave at a time:
+// v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one after the other, a fused multiply-add each, so that a
+// score with its dimensions ascending and an output with its keys ascending are the chains of that kernel, and with the same
+// running maxima, sums (the butterfly's tree of additions) and segments the results are the same bits (tested).
+//
+// What bounds it: at 555 tokens the longest walk, nine tiles one after the other; a tile costs a wave 8,192 cycles of matrix
+// products.  The kernel above brings every key and value once a token: 8B shape, 555 tokens, 309 us a layer by it, 104
+// by this one.  A block of four waves owns 64 columns of a key/value head and shares a tile of 64 keys and values in shared
+// memory, two blocks a compute unit; blocks of the latest tokens, whose walks are longest, start first.
+//
+// Row i of a product's tile of 16 keys is key 4 (i % 4) + i / 4 of them: lane (column r, group G) then holds the probabilities of the
+// keys 4 s + G, which is where the second product's operand of step s wants them.  Columns of one wave see different keys: a key
+// that a column does not see has the probability 0 there, and that product leaves its sums as they are unless the value is
+// no number or infinite.  A tile with such a value is added up on the vector units, each column with its own keys.
+typedef float ag_f32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ float ag_pair_sum(float x, bool half) {
+    const uint32_t u = __float_as_uint(x);
+    if (half) {
+        auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    }
+    auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+
+template <int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attn_portions_f32_kernel(
+    float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
+    const int* __restrict__ positions, const int* __restrict__ token_seq, const int* __restrict__ block_table,
+    int n, int max_pages, int nq, int nkv, int page_size, int window, float scale, int sink, int mask_chunk,
+    const float* __restrict__ sinks, int keep_first, float softcap) {
+    constexpr int KP = D + 4, VP = AG_TILE + 4, DT = D / 16;
+    __shared__ __attribute__((aligned(16))) float sk[AG_TILE * KP];     // [key][dim]
+    __shared__ __attribute__((aligned(16))) float sv[D * VP];           // [dim][key]
+    __shared__ int s_bad;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, G = lane >> 4;
+    const int g = nq / nkv, kvh = blockIdx.y;
+    const int first_col = (gridDim.x - 1 - blockIdx.x) * 64;
+    const int tok_first = first_col / g, tok_last = min((first_col + 63) / g, n - 1);
+    const int col = first_col + 16 * wave + r;
+    const int tok = min(col / g, n - 1), head = kvh * g + col % g;
+    const bool col_in = col < n * g;
+    const int pos = positions[tok];
+    const AgWalk wk = ag_walk(pos, window, mask_chunk, keep_first);
+    auto seen = [&](int key) __attribute__((always_inline)) { return key <= pos && (key >= wk.lo || key < wk.keep); };
+    float qf[D / 4];
+#pragma unroll
+    for (int i = 0; i < D / 4; ++i) qf[i] = q[((size_t)tok * nq + head) * D + 4 * i + G];
+
+    // Tokens of one request at a time (lane i: the block's i-th token).
+    const int my_tok = min(tok_first + lane, tok_last);
+    const int my_seq = token_seq[my_tok], my_pos = positions[my_tok];
+    const AgWalk my_walk = ag_walk(my_pos, window, mask_chunk, keep_first);
+    for (int run = tok_first, run_end; run <= tok_last; run = run_end) {
+        const int seq = __shfl(my_seq, run - tok_first);
+        const unsigned long long others = __ballot(my_seq != seq || tok_first + lane > tok_last) >> (run - tok_first);
+        run_end = others ? run + __ffsll(others) - 1 : tok_last + 1;
+        const bool mine = tok_first + lane >= run && tok_first + lane < run_end;
+        const int max_pos = (int)wave_max(mine ? (float)my_pos : -1.f);             // (positions are exact in 32-bit floats)
+        const int min_lo = -(int)wave_max(mine ? -(float)my_walk.lo : -16777216.f);
+        const int max_keep = (int)wave_max(mine ? (float)my_walk.keep : 0.f);
+        const int* bt = block_table + (size_t)seq * max_pages;
+        auto key_in = [&](int key) __attribute__((always_inline)) { return key <= max_pos && (key >= min_lo || key < max_keep); };
+        const bool in = col_in && tok >= run && tok < run_end;
+
+        float m = -INFINITY, l = 0.f, big_m = -INFINITY, big_l = 0.f;
+        bool any_in_seg = false;
+        ag_f32x4 o[DT], big_o[DT];
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[t] = big_o[t] = (ag_f32x4){0.f, 0.f, 0.f, 0.f};
+        auto end_segment = [&]() __attribute__((always_inline)) {
+            float m_out, a, b;
+            ag_merge_scales(big_m, m, m_out, a, b);
+            if (any_in_seg) {
+                big_l = ag_merge_value(big_l, a, l, b);
+                big_m = m_out;
+            }
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    big_o[t][i] = any_in_seg ? ag_merge_value(big_o[t][i], a, o[t][i], b) : big_o[t][i];
+                    o[t][i] = 0.f;
+                }
+            m = -INFINITY;
+            l = 0.f;
+            any_in_seg = false;
+        };
+        const int tile_last = max_pos / AG_TILE;
+        int seg = -1;
+        for (int tile = max_keep > 0 ? 0 : min_lo / AG_TILE; tile <= tile_last; ++tile) {
+            const int j0 = tile * AG_TILE;
+            if (j0 + AG_TILE - 1 < min_lo && j0 >= max_keep) continue;
+            if (seg >= 0 && tile / AG_SEG_TILES != seg) end_segment();
+            seg = tile / AG_SEG_TILES;
+            // ---- the tile into shared memory: keys and values that no column of this request sees as zeros ------------------
+            const int j4 = (j0 + lane) & ~3;
+            const bool near_in = key_in(j4) || key_in(j4 + 1) || key_in(j4 + 2) || key_in(j4 + 3);      // (four keys share a page)
+            const int my_page = near_in ? bt[(j0 + lane) / page_size] : 0, my_off = (j0 + lane) % page_size;
+            float4 piece[D / 16];
+#pragma unroll
+            for (int i = 0; i < D / 16; ++i) {
+                const int p = tid + 256 * i, key = p / (D / 4), e = p % (D / 4) * 4;
+                const int page = __shfl(my_page, key), off = __shfl(my_off, key);
+                piece[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (key_in(j0 + key)) piece[i] = *(const float4*)(k_cache + (((size_t)page * nkv + kvh) * page_size + off) * D + e);
+            }
+            __syncthreads();                                                    // (the last tile has been read)
+            if (tid == 0) s_bad = 0;
+#pragma unroll
+            for (int i = 0; i < D / 16; ++i) {
+                const int p = tid + 256 * i;
+                *(float4*)(sk + p / (D / 4) * KP + p % (D / 4) * 4) = piece[i];
+            }
+            bool bad = false;
+            {
+                const int k4 = tid % 16 * 4, page = __shfl(my_page, k4), off = __shfl(my_off, k4);
+                const bool in0 = key_in(j0 + k4), in1 = key_in(j0 + k4 + 1), in2 = key_in(j0 + k4 + 2), in3 = key_in(j0 + k4 + 3);
+#pragma unroll
+                for (int i = 0; i < D / 16; ++i) {
+                    const int e = tid / 16 + 16 * i;
+                    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (in0 || in1 || in2 || in3) v = *(const float4*)(v_cache + (((size_t)page * nkv + kvh) * D + e) * page_size + off);
+                    v.x = in0 ? v.x : 0.f; v.y = in1 ? v.y : 0.f; v.z = in2 ? v.z : 0.f; v.w = in3 ? v.w : 0.f;
+                    piece[i] = v;
+                }
+#pragma unroll
+                for (int i = 0; i < D / 16; ++i) {
+                    const uint32_t top = 0x7f800000u;
+                    bad |= (__float_as_uint(piece[i].x) & top) == top || (__float_as_uint(piece[i].y) & top) == top ||
+                           (__float_as_uint(piece[i].z) & top) == top || (__float_as_uint(piece[i].w) & top) == top;
+                    *(float4*)(sv + (tid / 16 + 16 * i) * VP + k4) = piece[i];
+                }
+            }
+            __syncthreads();
+            if (bad) s_bad = 1;
+            __syncthreads();
+            const bool active = in && j0 <= pos && (j0 + AG_TILE - 1 >= wk.lo || j0 < wk.keep);
+            if (!__any(active)) continue;
+            // ---- scores ----------------------------------------------------------------------------------------------------
+            ag_f32x4 s[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) s[t] = (ag_f32x4){0.f, 0.f, 0.f, 0.f};
+            const float* const ka = sk + (4 * (r & 3) + (r >> 2)) * KP + G;
+#pragma unroll
+            for (int e = 0; e < D / 4; ++e)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[16 * t * KP + 4 * e], qf[e], s[t], 0, 0, 0);
+            // ---- running maximum and sum: lane (r, G) has the keys 16 t + 4 i + G -----------------------------------------------
+            float p[4][4], mx = -INFINITY;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float sc = s[t][i] * scale;
+                    if (softcap > 0.f) sc = softcap * tanhf(sc / softcap);
+                    p[t][i] = active && seen(j0 + 16 * t + 4 * i + G) ? sc : -INFINITY;
+                    mx = fmaxf(mx, p[t][i]);
+                }
+            mx = fmaxf(mx, __shfl_xor(mx, 16, IA_WAVE));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, IA_WAVE));
+            const float m_new = fmaxf(m, mx);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    p[t][i] = active && seen(j0 + 16 * t + 4 * i + G) ? expf(p[t][i] - m_new) : 0.f;
+            // the additions of a butterfly over the 64 keys, 32 apart first: the tiles, then i, then the lane groups
+            float four[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) four[i] = (p[0][i] + p[2][i]) + (p[1][i] + p[3][i]);
+            float sum = (four[0] + four[2]) + (four[1] + four[3]);
+            sum = ag_pair_sum(sum, true);
+            sum = ag_pair_sum(sum, false);
+            float alpha = 1.f;
+            if (active) {
+                alpha = expf(m - m_new);
+                l = fmaf(l, alpha, sum);
+                m = m_new;
+                any_in_seg = true;
+            }
+#pragma unroll
+            for (int t = 0; t < DT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[t][i] *= alpha;
+            // ---- outputs ---------------------------------------------------------------------------------------------------
+            if (!s_bad) {
+                const float* const va = sv + r * VP + G;
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int d = 0; d < DT; ++d)
+                            o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[16 * d * VP + 16 * t + 4 * i], p[t][i], o[d], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        for (int b = 0; b < 4; ++b) {
+                            const int key = 16 * t + 4 * i + b;
+                            const float pk = __shfl(p[t][i], 16 * b + r);
+                            const bool ok = active && seen(j0 + key);
+#pragma unroll
+                            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                                for (int c = 0; c < 4; ++c)
+                                    o[d][c] = ok ? fmaf(pk, sv[(16 * d + 4 * G + c) * VP + key], o[d][c]) : o[d][c];
+                        }
+            }
+        }
+        if (seg >= 0) end_segment();
+        if (in) {
+            const float inv = 1.0f / (sink ? big_l + expf((sinks != nullptr ? sinks[head] : 0.f) - big_m) : big_l);
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+                *(ag_f32x4*)(out + ((size_t)tok * nq + head) * D + 16 * d + 4 * G) =
+                    (ag_f32x4){big_o[d][0] * inv, big_o[d][1] * inv, big_o[d][2] * inv, big_o[d][3] * inv};
+        }
+    }
+}
+
+// Whether portions of prompts (requests of several tokens each, 32-bit) take attn_portions_f32_kernel: its sizes, and columns
+// for a block.  Steps of few tokens at long contexts stay with a wave a segment (their walks would be long ones in few blocks).
+extern "C" int ia_attention_portions_f32_fits(int n, int nq, int nkv, int d, int dv, int page_size, int max_kv_len) {
+    return n > 0 && nkv > 0 && nq % nkv == 0 && (d == 64 || d == 128) && dv == d && page_size % 4 == 0 && nkv <= 65535 &&
+           (long long)n * (nq / nkv) >= 64 && (long long)n * (nq / nkv) < (1LL << 30) && max_kv_len <= (1 << 24) &&
+           ia_attention_generic_workspace(n, nq, nkv, d, dv, max_kv_len) == 0;
+}
+
+extern "C" int ia_attention_portions_f32(void* out, const void* q, const void* k_cache, const void* v_cache, const int* positions,
+                                         const int* token_seq, const int* block_table, int n, int max_pages, int nq, int nkv, int d,
+                                         int page_size, int window, float scale, int max_kv_len, int sink, int mask_chunk,
+                                         const float* sinks, int keep_first, float softcap, hipStream_t stream) {
+    IA_CHECK(ia_attention_portions_f32_fits(n, nq, nkv, d, d, page_size, max_kv_len), "attention: no kernel for portions of %d tokens, "
+             "%d and %d heads of %d, pages of %d", n, nq, nkv, d, page_size);
+    IA_CHECK((((uintptr_t)out | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0, "attention: arrays must be 16-byte aligned");
+    IA_CHECK(max_pages > 0 && window >= 0 && mask_chunk >= 0 && keep_first >= 0 && softcap >= 0.f && (sinks == nullptr || sink),
+             "attention: bad arguments max_pages=%d window=%d mask_chunk=%d keep_first=%d", max_pages, window, mask_chunk, keep_first);
+    const dim3 grid((unsigned)(((long long)n * (nq / nkv) + 63) / 64), nkv);
+#define AG_PORTIONS(D) attn_portions_f32_kernel<D><<<grid, 256, 0, stream>>>((float*)out, (const float*)q, (const float*)k_cache, \
+        (const float*)v_cache, positions, token_seq, block_table, n, max_pages, nq, nkv, page_size, window, scale, sink, mask_chunk, \
+        sinks, keep_first, softcap)
+    if (d == 64) AG_PORTIONS(64);
+    else AG_PORTIONS(128);
+#undef AG_PORTIONS
+    IA_LAUNCH_CHECK("attention_portions_f32");
+    return 0;
+}

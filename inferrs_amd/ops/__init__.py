@@ -429,7 +429,7 @@ def attention_generic(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
                       *, window: Optional[int], scale: float, max_kv_len: Optional[int] = None,
                       split: Optional[bool] = None, sink: bool = False, mask_chunk: Optional[int] = None,
                       sinks: Optional[torch.Tensor] = None, keep_first: int = 0,
-                      softcap: Optional[float] = None) -> torch.Tensor:
+                      softcap: Optional[float] = None, portions: bool = False) -> torch.Tensor:
     """q [n, nq, d] against the paged cache (values may have a width of their own: v_cache [pages, nkv, dv, page_size],
     the result is [n, nq, dv]); token i sees the keys at positions <= positions[i]
     (and > positions[i] - window) of row token_seq[i] of the table.  Any head size up to 512, any
@@ -439,7 +439,9 @@ def attention_generic(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     `sink`: the softmax's denominator holds one more term, exp(0): a key of score 0 that has no value; `sinks` [nq]
     (32-bit): the term is exp(sinks[h]) for query head h instead (not scaled).  `mask_chunk`: a token sees the keys of its
     own chunk of that many positions only (chunks counted from position 0 of the sequence), up to itself.  `keep_first`: it
-    sees the first so many positions besides.  `softcap`: a score becomes softcap * tanh(score / softcap)."""
+    sees the first so many positions besides.  `softcap`: a score becomes softcap * tanh(score / softcap).  `portions`: the tokens
+    are portions of prompts, several neighbours of each request, which 32-bit heads of 64 and 128 take on the matrix cores (the
+    same bits; single tokens of many requests would be slow there)."""
     _dev(q, k_cache, v_cache, positions, token_seq, block_table, sinks)
     sink = _check_sinks(sinks, sink, q.shape[1])
     _i32(positions, "positions"); _i32(token_seq, "token_seq"); _i32(block_table, "block_table")
@@ -453,6 +455,13 @@ def attention_generic(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
     max_kv_len = capacity if max_kv_len is None else min(int(max_kv_len), capacity)
     out = torch.empty((n, nq, dv), dtype=q.dtype, device=q.device)
     lib = library()
+    if (portions and not split and q.dtype == torch.float32 and (out.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0
+            and lib.ia_attention_portions_f32_fits(n, nq, nkv, d, dv, page_size, max_kv_len)):
+        _check(lib.ia_attention_portions_f32(
+            _p(out), _p(q), _p(k_cache), _p(v_cache), _p(positions), _p(token_seq), _p(block_table), n, block_table.shape[1], nq, nkv, d,
+            page_size, int(window or 0), ctypes.c_float(scale), max_kv_len, int(bool(sink)), int(mask_chunk or 0), _p(sinks),
+            int(keep_first), ctypes.c_float(softcap or 0.0), _stream()))
+        return out
     ws_floats = lib.ia_attention_generic_workspace(n, nq, nkv, d, dv, max_kv_len) if split is not False else 0
     if split and not ws_floats:
         raise KernelError("attention: a step of this many tokens, or of so few keys, is not split")

@@ -901,6 +901,46 @@ def test_attention_decode_rows_and_walks_of_every_length(nq, nkv, d, page, windo
         assert float(dk.max()) <= 2 ** -7 * float(k1.float().abs().max()) and float((dk > 0).float().mean()) < 1e-3
 
 
+@pytest.mark.parametrize("nq,nkv,d,page,lens,news,extra", [
+    (8, 2, 128, 16, [200], [200], {}), (4, 4, 64, 12, [130, 65], [130, 65], {}), (32, 2, 128, 16, [61, 40, 3], [61, 40, 3], {}),
+    (5, 1, 128, 16, [700, 90], [640, 20], dict(window=70)), (6, 2, 64, 20, [1100], [1090], dict(mask_chunk=96, sink=True)),
+    (8, 2, 128, 16, [600, 64], [600, 30], dict(window=100, keep_first=5, softcap=3.0)), (4, 2, 128, 16, [300], [290], dict(scale=4.0))])
+def test_attention_portions_in_32_bits_have_the_bits_of_the_plain_kernel(nq, nkv, d, page, lens, news, extra):
+    import ctypes
+    from inferrs_amd import ops
+    extra = dict(extra)
+    q, kc, vc, positions, token_seq, table = attention_case(torch.float32, nq, nkv, d, page, lens, news, 31)
+    scale, window = extra.pop("scale", 1.0 / math.sqrt(d)), extra.pop("window", None)
+    if extra.get("sink"):
+        extra["sinks"] = dev(randn(nq, dtype=torch.float32, seed=3))
+    n = q.shape[0]
+    args = [dev(q), dev(kc), dev(vc), dev(positions), dev(token_seq), dev(table)]
+    kw = dict(window=window, scale=scale, max_kv_len=max(lens), split=False, **extra)
+    lib = ops.library()
+
+    def portions():
+        out = torch.empty_like(args[0])
+        ops._check(lib.ia_attention_portions_f32(
+            *(ops._p(t) for t in (out, *args)), n, table.shape[1], nq, nkv, d, page, int(window or 0), ctypes.c_float(scale), 512,
+            int(bool(extra.get("sink"))), int(extra.get("mask_chunk", 0)), ops._p(extra.get("sinks")), int(extra.get("keep_first", 0)),
+            ctypes.c_float(extra.get("softcap", 0.0)), ops._stream()))
+        return out.cpu()
+
+    want = ops.attention_generic(*args, **kw).cpu()
+    assert torch.equal(portions(), want)
+    if max(lens) <= 512:
+        with ops.KernelTimer() as timer:
+            got = ops.attention_generic(*args, portions=True, **kw)
+        assert torch.equal(got.cpu(), want) and set(timer.summary()) == {"attention_portions_f32"}
+    # a value that is no number reaches the tokens that see it and no others
+    last = int(torch.nonzero(positions == lens[0] - 1)[0])
+    args[2][int(table[0, (lens[0] - 1) // page]), :, 3, (lens[0] - 1) % page] = float("inf")
+    want = ops.attention_generic(*args, **kw).cpu()
+    got = portions()
+    assert not torch.isfinite(want[last, :, 3]).any() and int(torch.isfinite(want).all(-1).all(-1).sum()) == n - 1
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
+
+
 def test_attention_decode_merge_is_the_same_every_time():
     """The blocks of a (request, key/value head) finish in any order and the last one merges: the sum runs in the
     order of the splits, so twenty calls give the same bits, and so does a call captured in a graph and replayed."""
