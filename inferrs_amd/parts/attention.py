@@ -232,7 +232,7 @@ class Attention(Mixer):
         return ops.attention_generic(q, cache.k, cache.v, ctx.positions, ctx.token_seq, group.block_table,
                                      window=s.window, scale=s.softmax_scale, max_kv_len=ctx.max_kv_len, sink=s.sink,
                                      mask_chunk=s.mask_chunk, keep_first=s.keep_first, softcap=s.softcap,
-                                     portions=ctx.n_single == 0)
+                                     portions=ctx.n_single == 0 and ctx.n_tokens >= 8 * ctx.n_seqs)
 
     def load_notes(self, page_size: int):
         """What the log should say once when a model with this part is set up: a decode step that cannot take the
@@ -312,5 +312,5 @@ class Attention(Mixer):
         else:
             a = ops.attention_generic(q, cache.k, cache.v, ctx.positions, ctx.token_seq, group.block_table,
                                       window=s.window, scale=s.softmax_scale, max_kv_len=ctx.max_kv_len, sink=s.sink,
-                                      portions=ctx.n_single == 0)
+                                      portions=ctx.n_single == 0 and ctx.n_tokens >= 8 * ctx.n_seqs)
         return self._project(ctx, a.view(a.shape[0], s.n_heads * s.head_dim))
