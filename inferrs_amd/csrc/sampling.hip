@@ -1058,16 +1058,19 @@ __device__ bool sample_narrow(int* __restrict__ out, const RowLayout& l, uint32_
         }
     }
     const RowSums rs = row_sums(l, ws, rowi, false);
-    auto probability = [&](uint32_t y) {
+    // A candidate's key; 0 for one under the floor, which settles nothing (a token far above all others leaves thousands of
+    // those behind, more than there are places: 50 of each stretch whose probabilities are all 0).
+    auto key_of = [&](uint32_t y) {
         const float e = expf(__uint_as_float(y) - rs.mx);
-        return rs.sum > 0.f ? e / rs.sum : e;
+        const float p = rs.sum > 0.f ? e / rs.sum : e;
+        return p >= NARROW_FLOOR ? order_key(p) : 0u;
     };
     uint32_t mine = 0u;
 #pragma unroll
     for (int i = 0; i < KEEP; ++i)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            key[i][h] = h * IA_WAVE + lane < held[i] ? order_key(probability(key[i][h])) : 0u;
+            key[i][h] = h * IA_WAVE + lane < held[i] ? key_of(key[i][h]) : 0u;
             mine = key[i][h] > mine ? key[i][h] : mine;
         }
     // the k-th largest of 128 groups' maxima: at least k candidates are no smaller
@@ -1106,7 +1109,7 @@ __device__ bool sample_narrow(int* __restrict__ out, const RowLayout& l, uint32_
         const int all = counts[b], end = all < SAMPLE_FAST_K ? all : SAMPLE_FAST_K;
         if (all > SAMPLE_FAST_K && lane == 0) s_over = 1;
         for (int at = (i < KEEP ? 2 * IA_WAVE : 0) + lane; at < end; at += IA_WAVE)
-            take(order_key(probability(cand_y[(size_t)b * SAMPLE_FAST_K + at])), cand_token[(size_t)b * SAMPLE_FAST_K + at]);
+            take(key_of(cand_y[(size_t)b * SAMPLE_FAST_K + at]), cand_token[(size_t)b * SAMPLE_FAST_K + at]);
     }
     __syncthreads();
     const int found = s_n;

@@ -193,6 +193,64 @@ def test_narrow_rows_draw_what_other_rows_with_a_top_k_draw(kind, vocab, top_k):
         assert int((got == want).sum()) >= rows - 1, (got.tolist(), want.tolist())
 
 
+def _draw_and_way(args, vocab, pen, narrow_only):
+    """`ops.sample` with a workspace of the test's own: the result, and the way each row went, by what it left there."""
+    from inferrs_amd import ops
+    lib, rows, filler = ops.library(), args[0].shape[0], 0x55555555
+    stretches = -(-vocab // 4096)
+    words = lib.ia_sample_workspace(rows, vocab) // rows
+    ws = torch.full((rows, words), filler, dtype=torch.int32, device="cuda")
+    out = torch.empty(rows, dtype=torch.int32, device="cuda")
+    lp, ids = torch.empty(rows, 21, device="cuda"), torch.empty(rows, 20, dtype=torch.int32, device="cuda")
+    logits, temperature, top_k, top_p, min_p, u, n_top = args
+    ops._check(lib.ia_sample(*(ops._p(t) for t in (out, logits, ws)), rows, vocab,
+                             *(ops._p(t) for t in (temperature, top_k, top_p, min_p, u, n_top, lp, ids)),
+                             *ops._penalty_args("test", rows, *pen), int(narrow_only), ops._stream()))
+    # a row's keys, and its stretches' sums of probabilities behind keys, probabilities, candidates, maxima and sums
+    totals = ws[:, 2 * vocab + 2 * stretches * 1024 + 2 * stretches:][:, :stretches].contiguous().view(torch.float32)
+    ways = []
+    for i in range(rows):
+        if bool((ws[i, :vocab] == filler).all()):
+            ways.append("candidates")
+        else:
+            ways.append("second pass" if abs(float(totals[i].sum()) - 1.0) < 1e-3 else "one block")
+    return (out, lp, ids), ways
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vocab", [4096, 32769, 151936])
+@pytest.mark.parametrize("kw,way", [
+    (dict(top_logprobs=0, logit_bias={7: 100.0}), "candidates"),                    # one token far above all others: the candidates of
+    (dict(temperature=1.0, top_p=0.5, top_logprobs=1, logit_bias={7: 200.0}), "candidates"),      # most stretches have a probability of 0
+    (dict(temperature=0.02, top_logprobs=0), "candidates"),
+    (dict(temperature=0.02, top_p=1.0, top_k=64, top_logprobs=1), "candidates")])
+def test_narrow_rows_are_not_left_to_one_block(vocab, kw, way, monkeypatch):
+    """Rows that the candidates can settle are drawn from those, not by the one block that works out a whole row; what they
+    report is that of the other way to the bit."""
+    from inferrs_amd import ops
+    from inferrs_amd.sampling import Sampler
+    rows = 4
+    g = torch.Generator().manual_seed(vocab)
+    z = (torch.randn(rows, vocab, generator=g) * 2.5).to("cuda")
+    params = [SamplingParams(logprobs=True, seed=i, **kw) for i in range(rows)]
+    asked = []
+    whole = ops.sample
+    monkeypatch.setattr(ops, "sample", lambda *a, **k: asked.append((a, k)) or whole(*a, **k))
+    previous = [torch.randint(0, vocab, (80,), generator=g).tolist() for _ in range(rows)]
+    tokens, infos = Sampler("cuda:0").sample_with_logprobs(z, params, previous, list(range(rows)))
+    (args, more), = asked
+    assert more["narrow_only"] == (way == "candidates")
+    got, ways = _draw_and_way(args, vocab, more["penalties"], more["narrow_only"])
+    assert ways == [way] * rows
+    assert got[0].tolist() == tokens and [len(i.top_logprobs) for i in infos] == [int((r >= 0).sum()) for r in got[2]]
+    ops.library().ia_sample_tune(2)
+    try:
+        want = whole(*args, **more)
+    finally:
+        ops.library().ia_sample_tune(1)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.gpu
 def test_mixed_rows_do_not_influence_each_other():
     from inferrs_amd.sampling import Sampler
