@@ -170,7 +170,9 @@ int ia_penalize(float* logits, int rows, int vocab, const int* window, int w, co
 int ia_window_push(int* window, int rows, int w, const int* caps, const int* tokens, hipStream_t stream);
 long long ia_sample_workspace(int rows, int vocab);
 int ia_sample_max_top(void);
-int ia_sample_narrow_top(void);                       // rows with a top_k of up to this many take the shorter way
+int ia_sample_narrow_top(void);                       // rows with a top_k of up to this many take the shorter way,
+// but for those whose reported entries reach beyond what that way holds: whether a row with these parameters takes it
+int ia_sample_is_narrow(int top_k, int vocab, float temperature, float top_p, float min_p, int n_top, int biased);
 // n_top, lp_out [rows, 1 + max_top], lp_ids [rows, max_top]: all null, or the log-probabilities asked for per row
 int ia_sample(int* out, const float* logits, void* workspace, int rows, int vocab,
               const float* temperature, const int* top_k, const float* top_p, const float* min_p,

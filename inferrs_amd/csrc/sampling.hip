@@ -685,8 +685,8 @@ __device__ bool sample_top_k(int* __restrict__ out, const uint32_t* __restrict__
 //     first k entries of the ordered list (k: the row's top_k, or SAMPLE_FAST_K for a row without one), written
 //     in the order of their tokens at a place that follows from k and the stretches' lengths alone;
 //   then one block a row (sample_kernel) picks the row's first k among those candidates and walks them.
-// Rows with a top_k of up to SAMPLE_NARROW_K ("narrow" ones; the reference's default is 50) need no second pass: the
-// first leaves those of its stretch's logits that can be among the row's first k (see narrow_candidates), the last
+// Rows with a top_k of up to SAMPLE_NARROW_K ("narrow" ones, see is_narrow; the reference's default is 50) need no second pass: the
+// first leaves those of its stretch's logits that can be among the row's first k (see NARROW_MARGIN), the last
 // block works out their probabilities alone.  24 rows of 151,936 logits with the default parameters: 86 us of kernels,
 // of them the second pass 36 (16 bytes written a logit, three histograms of keys that mostly fall into one bin) and the
 // last 28 (three more of them and one thread's walk through shared memory), before; 30 now, 16 and 13.
@@ -827,7 +827,31 @@ __device__ __forceinline__ void load_stretch(float* s_z, const float* __restrict
     if (pen.any()) penalize_range(s_z, lo, n, pen, rowi, s_win);
 }
 
-__device__ __forceinline__ bool is_narrow(int k, int vocab, int fast) { return fast == 1 && k > 0 && k < vocab && k <= SAMPLE_NARROW_K; }
+// What decides whether a row is a narrow one: a top_k of up to SAMPLE_NARROW_K, and candidates that hold what it reports.  A row that
+// reports entries (two and more; the first is always a candidate) of a list that neither top_p nor min_p ends reports tokens far
+// under its maximum, down to those whose probability is 0 (by index then), and the candidates end at NARROW_FLOOR, 83 under it.
+// At NARROW_COOL these are 20 between the logits, more than a model's first entries are apart; below it, and where a bias may set
+// a token apart from all others, such rows stay with the second pass.  Whole draws of 24 rows of 151,936 with entries and no
+// top_p, us, candidates and one block a row for what they do not settle / second pass: temperature 0 877 / 356, a bias of 100
+// 887 / 362; temperature 0.1 with logits close enough to be settled 243 / 310.
+#define NARROW_COOL 0.25f
+__host__ __device__ __forceinline__ bool is_narrow(int k, int vocab, float temp, float tp, float mp, int want_top, bool biased) {
+    const bool open = want_top > 1 && !(tp < 1.0f) && !(mp > 0.0f);
+    return k > 0 && k < vocab && k <= SAMPLE_NARROW_K && !(open && (biased || temp < NARROW_COOL));
+}
+
+// A row's parameters as the passes read them.
+struct RowParams {
+    const float* temperature;
+    const int* top_k;
+    const float *top_p, *min_p;
+    const int* n_top;
+};
+// (a row's list of biases starts with its first token or holds none)
+__device__ __forceinline__ bool row_is_narrow(const RowParams& r, const Penalties& p, int rowi, int vocab, int fast) {
+    return fast == 1 && is_narrow(r.top_k[rowi], vocab, r.temperature[rowi], r.top_p[rowi], r.min_p[rowi], r.n_top != nullptr ? r.n_top[rowi] : -1,
+                                  p.nb > 0 && p.bias_ids[(size_t)rowi * p.nb] >= 0);
+}
 
 // Those of a stretch's logits that can be among the row's first k tokens, k <= SAMPLE_NARROW_K, ordered by their
 // rounded probabilities p = exp(y - the row's maximum) / the row's sum and by index where these are equal; y, the logits over the
@@ -840,15 +864,14 @@ __device__ __forceinline__ bool is_narrow(int k, int vocab, int fast) { return f
 // NARROW_FLOOR.  The last block takes no token whose p is under the floor from these candidates (sample_narrow), so
 // both may be left out.  SAMPLE_FAST_K places; a stretch with more candidates (equal logits in great number) says so by its count.
 #define NARROW_MARGIN 4e-5f
-#define NARROW_DEPTH 88.0f              // exp(-88) = 6e-39, a sixteenth of a hundredth of the floor
+#define NARROW_DEPTH 88.0f              // exp(-88) = 6e-39, under a hundredth of the floor
 #define NARROW_FLOOR 1e-36f
 
 // Bound by the trip to the memory, a logit's division and exponential, and the barriers between its phases; several blocks a
 // compute unit hide each other's.
 __global__ __launch_bounds__(256) void sample_partials_kernel(const float* __restrict__ logits, uint32_t* __restrict__ workspace,
-                                                              const RowLayout l, const float* __restrict__ temperature,
-                                                              const int* __restrict__ top_k, const int* __restrict__ n_top,
-                                                              const Penalties pen, int fast) {
+                                                              const RowLayout l, const RowParams params, const Penalties pen,
+                                                              int fast) {
     __shared__ __attribute__((aligned(16))) float s_z[SAMPLE_STRETCH];
     __shared__ int s_win[PENALTY_STAGED];
     __shared__ __attribute__((aligned(16))) uint32_t s_group[128];
@@ -857,10 +880,10 @@ __global__ __launch_bounds__(256) void sample_partials_kernel(const float* __res
     __shared__ int s_n;
     constexpr int PER = SAMPLE_STRETCH / 256;
     const int rowi = blockIdx.y, b = blockIdx.x, t = threadIdx.x, wave = t / IA_WAVE;
-    const int k = top_k[rowi];
+    const int k = params.top_k[rowi];
+    const bool narrow = row_is_narrow(params, pen, rowi, l.vocab, fast);
     float temp;
-    if (!row_temperature(temperature, n_top, rowi, temp)) return;
-    const bool narrow = is_narrow(k, l.vocab, fast);
+    if (!row_temperature(params.temperature, params.n_top, rowi, temp)) return;
     const int n = l.length(b);
     if (t == 0) { s_kth = 0u; s_n = 0; }
     load_stretch(s_z, logits, l, rowi, b, pen, s_win);
@@ -939,8 +962,7 @@ __device__ __forceinline__ int picked_out(int k, int vocab, int fast_top_k) {
 
 #define STRETCH_THREADS 256
 __global__ __launch_bounds__(STRETCH_THREADS) void sample_stretch_kernel(
-    const float* __restrict__ logits, uint32_t* __restrict__ workspace, const RowLayout l,
-    const float* __restrict__ temperature, const int* __restrict__ top_k, const int* __restrict__ n_top, const Penalties pen,
+    const float* __restrict__ logits, uint32_t* __restrict__ workspace, const RowLayout l, const RowParams params, const Penalties pen,
     int fast_top_k) {
     __shared__ float scratch[32];
     __shared__ int s_counts[STRETCH_THREADS];
@@ -949,8 +971,8 @@ __global__ __launch_bounds__(STRETCH_THREADS) void sample_stretch_kernel(
     __shared__ int s_win[PENALTY_STAGED];
     const int rowi = blockIdx.y, b = blockIdx.x;
     float temp;
-    if (!row_temperature(temperature, n_top, rowi, temp)) return;
-    if (is_narrow(top_k[rowi], l.vocab, fast_top_k)) return;
+    if (!row_temperature(params.temperature, params.n_top, rowi, temp)) return;
+    if (row_is_narrow(params, pen, rowi, l.vocab, fast_top_k)) return;
     const int lo = b * l.stretch, n = l.length(b);
     load_stretch((float*)s_keys, logits, l, rowi, b, pen, s_win);
     uint32_t* keys = l.keys(workspace, rowi) + lo;
@@ -982,7 +1004,7 @@ __global__ __launch_bounds__(STRETCH_THREADS) void sample_stretch_kernel(
     }
     t = block_sum(t, scratch);
     if (threadIdx.x == 0) l.part_total(workspace, rowi)[b] = t;
-    const int k = picked_out(top_k[rowi], l.vocab, fast_top_k);
+    const int k = picked_out(params.top_k[rowi], l.vocab, fast_top_k);
     if (k == 0) return;
     __syncthreads();
     // ---- the stretch's own first k, in the order of their tokens
@@ -1025,7 +1047,8 @@ __global__ __launch_bounds__(STRETCH_THREADS) void sample_stretch_kernel(
 // The reference's steps (sampler.rs:251-335) on a narrow row: the candidates' probabilities, the first k of them in order
 // and the walk, with the sums in the reference's order.  False, and nothing that counts is written, where the candidates
 // do not settle the row: a stretch had more than its places, there is a NaN or no number to start from, or the draw (or
-// an entry that is reported) lies among probabilities under the floor, whose order and ties the candidates do not hold.
+// an entry that is reported) lies among probabilities under the floor, whose order and ties the candidates do not hold.  (A list
+// that top_p or min_p ends before that holds none of these, however few candidates there are: at temperature 0 it is mostly one.)
 // A block of 1,024 threads; all of them call it.
 // One block a row, so the time is a chain: one trip to the memory (a wave takes the stretches wave, wave + 16, ...; the first
 // 128 candidates of three of them are asked for before their number is known, the places exist), five barriers, and the
@@ -1130,14 +1153,18 @@ __device__ bool sample_narrow(int* __restrict__ out, const RowLayout& l, uint32_
         const float p = lane < n ? __uint_as_float((uint32_t)(e >> 32) & 0x7fffffffu) : 0.f;     // (a probability's sign bit is 0)
         const int id = (int)~(uint32_t)(e & 0xffffffffull);
         int len = n;
+        bool ended = n == k;                                // the list ends within the candidates
         float filtered = 0.f;
         for (int i = 0; i < n; ++i) {
             filtered += lane_value(p, i);
-            if (tp < 1.0f && filtered >= tp) { len = i + 1; break; }
+            if (tp < 1.0f && filtered >= tp) { len = i + 1; ended = true; break; }
         }
         if (mp > 0.0f) {
-            const unsigned long long under = __ballot(lane < len && !(p >= lane_value(p, 0) * mp));
+            const float least = lane_value(p, 0) * mp;
+            const unsigned long long under = __ballot(lane < len && !(p >= least));
             const int cut = under ? __ffsll((long long)under) - 1 : len;
+            // (tokens that are no candidates are under the floor: a threshold above it leaves them out)
+            if (cut > 0) ended = ended || cut < len || least >= NARROW_FLOOR;
             if (cut > 0 && cut < len) {
                 len = cut;
                 filtered = 0.f;
@@ -1152,12 +1179,12 @@ __device__ bool sample_narrow(int* __restrict__ out, const RowLayout& l, uint32_
             if (rng < step) { at = i; break; }
             rng -= step;
         }
-        // (a list that ends before its k-th token for want of candidates ends in tokens under the floor)
-        bool settled = filtered > 0.f && (at >= 0 || n == k);
+        // (a list that ends before its k-th token only for want of candidates goes on in tokens under the floor)
+        bool settled = filtered > 0.f && (at >= 0 || ended);
         if (at < 0) at = len - 1;
         const int shown = want_top < SAMPLE_MAX_TOP ? want_top : SAMPLE_MAX_TOP;
         settled = settled && lane_value(p, at) >= NARROW_FLOOR;
-        if (shown > 0) settled = settled && (len >= shown || n == k || len < n) && lane_value(p, (shown < len ? shown : len) - 1) >= NARROW_FLOOR;
+        if (shown > 0) settled = settled && (len >= shown || ended) && lane_value(p, (shown < len ? shown : len) - 1) >= NARROW_FLOOR;
         if (settled) {
             if (want_top >= 0) {
                 if (lane < shown && lane < len) {
@@ -1179,9 +1206,8 @@ __device__ bool sample_narrow(int* __restrict__ out, const RowLayout& l, uint32_
 // token's log-probability within the kept list, then the entries'; lp_ids [rows, SAMPLE_MAX_TOP]: their ids (-1: none).
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     int* __restrict__ out, const float* __restrict__ logits, uint32_t* __restrict__ workspace, const RowLayout l,
-    const float* __restrict__ temperature, const int* __restrict__ top_k, const float* __restrict__ top_p,
-    const float* __restrict__ min_p, const float* __restrict__ u, const int* __restrict__ n_top,
-    float* __restrict__ lp_out, int* __restrict__ lp_ids, const Penalties pen, int fast_top_k, int narrow_only) {
+    const RowParams params, const float* __restrict__ u, float* __restrict__ lp_out, int* __restrict__ lp_ids, const Penalties pen,
+    int fast_top_k, int narrow_only) {
     __shared__ float scratch[32];
     __shared__ int s_counts[SAMPLE_THREADS];
     __shared__ float sv[16];
@@ -1189,7 +1215,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     const int rowi = blockIdx.x;
     const int vocab = l.vocab;
     const float* row = logits + (size_t)rowi * vocab;
-    const int want_top = n_top != nullptr ? n_top[rowi] : -1;
+    const int want_top = params.n_top != nullptr ? params.n_top[rowi] : -1;
     if (want_top >= 0 && threadIdx.x < SAMPLE_MAX_TOP) {
         lp_ids[(size_t)rowi * SAMPLE_MAX_TOP + threadIdx.x] = -1;
         lp_out[(size_t)rowi * (1 + SAMPLE_MAX_TOP) + 1 + threadIdx.x] = -INFINITY;
@@ -1207,17 +1233,17 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         return z;
     };
     // (all of a row's parameters are asked for at once: one after the other each is a trip to the memory)
-    const int k = top_k[rowi];
-    const float tp = top_p[rowi], mp = min_p[rowi], draw = u[rowi];
+    const int k = params.top_k[rowi];
+    const float tp = params.top_p[rowi], mp = params.min_p[rowi], draw = u[rowi];
+    const bool narrow = row_is_narrow(params, pen, rowi, vocab, fast_top_k);
     float temp;
-    if (!row_temperature(temperature, n_top, rowi, temp)) {
+    if (!row_temperature(params.temperature, params.n_top, rowi, temp)) {
         int touched = 0;
         for (int i = threadIdx.x; i < pen.w; i += blockDim.x) touched |= pen.window[(size_t)rowi * pen.w + i] >= 0;
         for (int i = threadIdx.x; i < pen.nb; i += blockDim.x) touched |= pen.bias_ids[(size_t)rowi * pen.nb + i] >= 0;
         argmax_row(__syncthreads_or(touched) ? touched_row() : row, vocab, sv, si, out + rowi);
         return;
     }
-    const bool narrow = is_narrow(k, vocab, fast_top_k);
     if (narrow && sample_narrow(out, l, workspace, rowi, k, tp, mp, draw, want_top, lp_out, lp_ids)) return;
     const bool listed = !narrow && !narrow_only;            // the second pass has been over the row
     __syncthreads();
@@ -1362,11 +1388,15 @@ extern "C" void ia_sample_tune(int fast_top_k) { g_sample_fast = fast_top_k; }
 
 extern "C" int ia_sample_max_top(void) { return SAMPLE_MAX_TOP; }
 extern "C" int ia_sample_narrow_top(void) { return SAMPLE_NARROW_K; }
+// Whether a row with these parameters needs no second pass (n_top: as in ia_sample; biased: it has a logit bias).
+extern "C" int ia_sample_is_narrow(int top_k, int vocab, float temperature, float top_p, float min_p, int n_top, int biased) {
+    return is_narrow(top_k, vocab, temperature, top_p, min_p, n_top, biased != 0);
+}
 
 // n_top, lp_out, lp_ids: all null, or all given (see sample_kernel).  window .. nb: bias and penalties as in ia_penalize
-// (w = nb = 0: none), on the way; the logits stay as they are.  `narrow_only`: the caller knows that every row has a top_k of
-// 1 .. ia_sample_narrow_top() below vocab or is a greedy one, so that the second pass has nothing to do (a row of another kind is
-// still drawn rightly, by one block).
+// (w = nb = 0: none), on the way; the logits stay as they are.  `narrow_only`: the caller knows that every row is a narrow one
+// (ia_sample_is_narrow) or a greedy one, so that the second pass has nothing to do (a row of another kind is still drawn rightly, by
+// one block).
 extern "C" int ia_sample(int* out, const float* logits, void* workspace, int rows, int vocab,
                          const float* temperature, const int* top_k, const float* top_p, const float* min_p,
                          const float* u, const int* n_top, float* lp_out, int* lp_ids, const int* window, int w,
@@ -1384,12 +1414,13 @@ extern "C" int ia_sample(int* out, const float* logits, void* workspace, int row
     const RowLayout l = row_layout(vocab);
     const dim3 grid((unsigned)l.stretches, (unsigned)rows);
     const int fast = g_sample_fast;
-    sample_partials_kernel<<<grid, 256, 0, stream>>>(logits, (uint32_t*)workspace, l, temperature, top_k, n_top, pen, fast);
+    const RowParams params = {temperature, top_k, top_p, min_p, n_top};
+    sample_partials_kernel<<<grid, 256, 0, stream>>>(logits, (uint32_t*)workspace, l, params, pen, fast);
     if (fast != 1) narrow_only = 0;
     if (!narrow_only)
-        sample_stretch_kernel<<<grid, STRETCH_THREADS, 0, stream>>>(logits, (uint32_t*)workspace, l, temperature, top_k, n_top, pen, fast);
-    sample_kernel<<<rows, SAMPLE_THREADS, 0, stream>>>(out, logits, (uint32_t*)workspace, l, temperature,
-                                                       top_k, top_p, min_p, u, n_top, lp_out, lp_ids, pen, fast, narrow_only);
+        sample_stretch_kernel<<<grid, STRETCH_THREADS, 0, stream>>>(logits, (uint32_t*)workspace, l, params, pen, fast);
+    sample_kernel<<<rows, SAMPLE_THREADS, 0, stream>>>(out, logits, (uint32_t*)workspace, l, params, u, lp_out, lp_ids, pen, fast,
+                                                       narrow_only);
     IA_LAUNCH_CHECK("sample");
     return 0;
 }

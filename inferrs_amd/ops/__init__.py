@@ -1297,8 +1297,18 @@ _NO_PENALTIES = (None, 0, None, None, None, None, None, 0)
 
 
 def sample_narrow_top() -> int:
-    """Rows with a top_k of up to this many, below the vocabulary, are drawn from a few candidates of every stretch of the row."""
+    """Rows with a top_k of up to this many, below the vocabulary, are drawn from a few candidates of every stretch of the row,
+    but for those that `sample_is_narrow` leaves out."""
     return library().ia_sample_narrow_top()
+
+
+def sample_is_narrow(top_k: int, vocab: int, temperature: float, top_p: float, min_p: float, n_top: int = -1,
+                     biased: bool = False) -> bool:
+    """Whether `sample` draws a row with these parameters from a few candidates of every stretch (`narrow_only`): a top_k in 1 ..
+    `sample_narrow_top()`, unless the row reports two entries and more of a list that neither top_p nor min_p ends, at a low
+    temperature or with a logit bias: those entries lie beyond the candidates."""
+    return bool(library().ia_sample_is_narrow(top_k, vocab, ctypes.c_float(temperature), ctypes.c_float(top_p),
+                                              ctypes.c_float(min_p), n_top, int(biased)))
 
 
 def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor,
@@ -1310,8 +1320,7 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
     [rows, 1 + 20] (the drawn token's, then the list's first entries'), and those entries' ids, int32
     [rows, 20] (-1: no entry): the result is then (tokens, log-probabilities, ids).
     `penalties`: what `penalize` takes behind the logits, applied on the way (the logits stay as they are).
-    `narrow_only`: the caller knows that every row is greedy or has a top_k in 1 .. `sample_narrow_top()` below the
-    vocabulary, and saves a launch.  `out`: where the tokens go (int32 [rows])."""
+    `narrow_only`: the caller knows that every row is greedy or one that `sample_is_narrow`, and saves a launch.  `out`: where the tokens go (int32 [rows])."""
     _dev(logits, temperature, top_k, top_p, min_p, u, n_top, out)
     _f32(logits, "logits"); _f32(temperature, "temperature"); _f32(top_p, "top_p"); _f32(min_p, "min_p"); _f32(u, "u")
     _i32(top_k, "top_k")

@@ -93,6 +93,11 @@ class Sampler:
         n_top = np.asarray([p.top_logprobs if p.logprobs else -1 for p in params], dtype=np.int32)
         penalized = window is not None
         narrow = all_narrow(int(top_k.min()), int(top_k.max()), logits.shape[1])
+        # (rows that report entries of a list which top_p or min_p may not end, to within what 32 bits round: one call for all)
+        open_rows = [p for p in params if p.top_logprobs > 1 and p.top_p > 0.999 and p.min_p < 1e-6]
+        if narrow and open_rows:
+            narrow = ops.sample_is_narrow(open_rows[0].top_k, logits.shape[1], min(p.temperature for p in open_rows), 1.0, 0.0, 2,
+                                          any(p.logit_bias for p in open_rows))
         window, rep, freq, pres, bias_ids, bias_vals, temperature, top_k, top_p, min_p, u, n_top = self._upload(
             window if width else None, rep, freq, pres, bias_ids, bias_vals, temperature, top_k, top_p, min_p, u, n_top)
         penalties = None
@@ -116,7 +121,8 @@ class Sampler:
 
 
 def all_narrow(least: int, most: int, vocab: int) -> bool:
-    """Rows whose top_k lies in `least` .. `most` all go `ops.sample`'s shortest way."""
+    """Rows whose top_k lies in `least` .. `most` all go `ops.sample`'s shortest way, where they report no more than the token drawn
+    and the first entry."""
     return 0 < least and most <= min(ops.sample_narrow_top(), vocab - 1)
 
 

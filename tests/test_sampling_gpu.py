@@ -223,10 +223,20 @@ def _draw_and_way(args, vocab, pen, narrow_only):
     (dict(top_logprobs=0, logit_bias={7: 100.0}), "candidates"),                    # one token far above all others: the candidates of
     (dict(temperature=1.0, top_p=0.5, top_logprobs=1, logit_bias={7: 200.0}), "candidates"),      # most stretches have a probability of 0
     (dict(temperature=0.02, top_logprobs=0), "candidates"),
-    (dict(temperature=0.02, top_p=1.0, top_k=64, top_logprobs=1), "candidates")])
+    (dict(temperature=0.02, top_p=1.0, top_k=64, top_logprobs=1), "candidates"),
+    (dict(temperature=0.0, top_logprobs=5), "candidates"),                          # one candidate a stretch, top_p ends the list at the first
+    (dict(temperature=0.0, top_logprobs=20), "candidates"),
+    (dict(temperature=0.0, top_logprobs=5, top_p=1.0, min_p=0.05), "candidates"),   # min_p ends it
+    (dict(temperature=0.0, top_logprobs=1, top_p=1.0), "candidates"),
+    (dict(temperature=0.0, top_logprobs=2, top_p=1.0), "second pass"),              # nothing does: tokens of probability 0 are reported
+    (dict(temperature=0.2, top_logprobs=20, top_p=1.0), "second pass"),
+    (dict(temperature=0.5, top_logprobs=20, top_p=1.0), "candidates"),
+    (dict(temperature=1.0, top_logprobs=5, top_p=1.0, logit_bias={7: 200.0}), "second pass"),
+    (dict(temperature=1.0, top_logprobs=5, logit_bias={7: 200.0}), "candidates")])
 def test_narrow_rows_are_not_left_to_one_block(vocab, kw, way, monkeypatch):
-    """Rows that the candidates can settle are drawn from those, not by the one block that works out a whole row; what they
-    report is that of the other way to the bit."""
+    """Rows that the candidates can settle are drawn from those, rows that report what lies beyond them keep the second pass over many
+    blocks, and the sampler asks for it where a row needs it: the one block that works out a whole row is left for what nobody can
+    foresee.  What the rows report is the same to the bit."""
     from inferrs_amd import ops
     from inferrs_amd.sampling import Sampler
     rows = 4
