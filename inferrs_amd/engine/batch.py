@@ -66,9 +66,12 @@ class StepContext:
 
     def position_table(self, position_part) -> Optional[Any]:
         """The position part's table for this step's tokens, built once per distinct spec."""
-        key = position_part.spec
+        return self.once(position_part.spec, lambda: position_part.table(self.positions))
+
+    def once(self, key, make) -> Any:
+        """What `make` gives for this step, asked for by many layers and worked out for the first."""
         if key not in self._tables:
-            self._tables[key] = position_part.table(self.positions)
+            self._tables[key] = make()
         return self._tables[key]
 
 

@@ -232,7 +232,16 @@ class Attention(Mixer):
         return ops.attention_generic(q, cache.k, cache.v, ctx.positions, ctx.token_seq, group.block_table,
                                      window=s.window, scale=s.softmax_scale, max_kv_len=ctx.max_kv_len, sink=s.sink,
                                      mask_chunk=s.mask_chunk, keep_first=s.keep_first, softcap=s.softcap,
-                                     portions=ctx.n_single == 0 and ctx.n_tokens >= 8 * ctx.n_seqs)
+                                     portions=Attention.portions_pay(s, ctx, q))
+
+    @staticmethod
+    def portions_pay(s: AttentionSpec, ctx, q) -> bool:
+        """Whether the step's portions of prompts take the 32-bit kernel of the matrix cores (the same bits either way; a captured
+        step keeps the choice made for the portions it was captured with)."""
+        if q.dtype != torch.float32 or ctx.n_single != 0:
+            return False
+        sizes = (s.n_heads, s.n_kv_heads, s.head_dim, min(s.window or 1 << 30, s.mask_chunk or 1 << 30))
+        return ctx.once(("portions", *sizes), lambda: ops.attention_portions_pay(ctx.q_lens, ctx.kv_starts, *sizes))
 
     def load_notes(self, page_size: int):
         """What the log should say once when a model with this part is set up: a decode step that cannot take the
@@ -312,5 +321,5 @@ class Attention(Mixer):
         else:
             a = ops.attention_generic(q, cache.k, cache.v, ctx.positions, ctx.token_seq, group.block_table,
                                       window=s.window, scale=s.softmax_scale, max_kv_len=ctx.max_kv_len, sink=s.sink,
-                                      portions=ctx.n_single == 0 and ctx.n_tokens >= 8 * ctx.n_seqs)
+                                      portions=self.portions_pay(s, ctx, q))
         return self._project(ctx, a.view(a.shape[0], s.n_heads * s.head_dim))

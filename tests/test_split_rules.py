@@ -136,3 +136,29 @@ def test_bounds_of_mixed_steps_are_few_and_close():
     assert Engine._run_bound(100, 1024, 1024, 2) == 1024 and Engine._run_bound(9000, 1024, 9 * 1024) == 9 * 1024
     # a portion of up to 2,048 tokens of context beside anything: one graph
     assert len({Engine._run_bound(n, bucket, widest, 2) for n in range(1, 2049)}) == 1
+
+
+@pytest.mark.parametrize("heads,q_lens,kv_starts,span,plain,portions", [
+    ((32, 8, 128), [555], [0], None, 309, 104), ((8, 8, 64), [144], [0], None, 26.3, 24.6), ((16, 2, 64), [17], [0], None, 16.8, 14.7),
+    ((32, 8, 128), [16] * 16, [484] * 16, None, 339, 82), ((8, 8, 64), [64] * 16, [7936] * 16, None, 5956, 839),
+    ((32, 4, 128), [2] * 64 + [500], [498] * 64 + [0], None, 405, 297), ((64, 8, 128), [5] * 73, [4700] * 73, None, 1859, 1079),
+    ((8, 8, 64), [9] * 30, [4200] * 30, 19, 20.9, 66.6), ((16, 8, 128), [2] * 64 + [500], [3998] * 64 + [0], None, 1513, 9095),
+    ((8, 8, 64), [3] * 32 + [512], [1997] * 32 + [2000], None, 886, 4331), ((16, 8, 128), [8] * 16, [492] * 16, None, 156, 281),
+    ((8, 8, 64), [8] * 64, [7992] * 64, None, 2992, 6235), ((32, 8, 128), [2] * 16 + [200], [498] * 16 + [0], None, 170, 564),
+    ((8, 8, 64), [16] * 16, [1984] * 16, None, 318, 757)])
+def test_portions_in_32_bits_take_the_faster_kernel_at_the_measured_points(heads, q_lens, kv_starts, span, plain, portions):
+    """The choice between the two 32-bit kernels as a layer makes it, against both measured times (us)."""
+    from types import SimpleNamespace
+
+    import torch
+    from inferrs_amd.engine.batch import StepContext
+    from inferrs_amd.parts.attention import Attention
+    nq, nkv, d = heads
+    spec = SimpleNamespace(n_heads=nq, n_kv_heads=nkv, head_dim=d, window=span, mask_chunk=None)
+    ctx = SimpleNamespace(n_single=0, n_seqs=len(q_lens), n_tokens=sum(q_lens), q_lens=q_lens, kv_starts=kv_starts, _tables={})
+    ctx.once = lambda key, make: StepContext.once(ctx, key, make)
+    q = torch.empty(0)
+    assert Attention.portions_pay(spec, ctx, q) == (portions < plain)
+    assert Attention.portions_pay(spec, ctx, q) == (portions < plain) and len(ctx._tables) == 1
+    ctx.n_single = 1
+    assert not Attention.portions_pay(spec, ctx, q) and not Attention.portions_pay(spec, SimpleNamespace(n_single=0), q.bfloat16())
