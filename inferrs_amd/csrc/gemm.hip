@@ -731,7 +731,8 @@ __global__ __launch_bounds__(SK_MAX_WAVES * IA_WAVE) void gemm_skinny_kernel(
 // waves are read together, and a thread finishes one feature of one row (four of them one after the other, all in one wave, were 0.4 us
 // of code that no cache holds yet).  A range longer than a chunk: BURST_AHEAD asks for the next chunk of both operands, x through
 // registers, before it multiplies this one (one block a compute unit has the registers), BURST_CHUNKS leaves that to the other block
-// on the unit.  The order of every sum is that of gemm_skinny_kernel: the same bits.
+// on the unit.  The order of every sum is that of gemm_skinny_kernel with k shared out alike: the same bits as that kernel's at the same
+// waves a block (skinny_split gives a k of 1,024 eight here, four in taller weights, and no weight sixteen).
 // Measured inside graphs, us, a layer's four products one behind another, before and now: 0.6B shape, 1 row 24.3 -> 18.5, 8 rows 26.8 -> 20.6;
 // 1.7B shape, 1 row 35.2 -> 31.0, 8 rows 39.7 -> 35.2; 4B shape, 1 row 57.1 -> 50; 8B shape, 1 row 78.2 -> 75.8, 8 rows 84.0 -> 82.5
 // (q|k|v 11.7 -> 10.0 at one row, the bare read of its 50 MB 9.9); 14B shape, 1 row 129.4 -> 124.4.

@@ -405,10 +405,11 @@ __global__ __launch_bounds__(W * IA_WAVE) void gemm_mid_kernel(
 //   splits ways k is split between blocks (gridDim.y); the splits' sums are added up by the reader
 //   stages of the pipeline
 // Wanted: a block for every compute unit and no more, three stages deep (a block a unit: what it has under way is all that
-// hides the memory's latency; two rounds of blocks would leave the second half empty).  Among the ways that fill nine
-// tenths of the chip, the one with the most waves a block wins (the rows of x are fetched once a block) as long as a block
-// keeps eight chunks of k.  A weight that no way fits (a logits head: thousands of blocks) takes four waves a block two stages
-// deep, several blocks a unit, k split until there is a block for every unit.
+// hides the memory's latency; two rounds of blocks would leave the second half empty).  Among the ways that one round holds the
+// one that fills the chip best wins; of ways that fill it alike, the one with the most waves a block (the rows of x are fetched once
+// a block) as long as a block keeps eight chunks of k.  A weight whose best way leaves less than 0.3 of the chip at work, or of
+// which one round holds none, takes four waves a block two stages deep, several blocks a unit, k split until there is a block for
+// every unit; one of four rounds and more of blocks of eight waves (a logits head) takes those, three stages deep.
 static int mid_cus() {
     static int cus = 0;
     if (cus == 0) {

@@ -696,7 +696,7 @@ __device__ bool sample_top_k(int* __restrict__ out, const uint32_t* __restrict__
 // (narrow rows: numbers of candidates) [stretches] each.
 #define SAMPLE_STRETCH 4096
 #define SAMPLE_STAGED 8192              // candidates of a row that its last block keeps in shared memory
-#define SAMPLE_MAX_STRETCHES 1024       // the stretches' sums meet in a block's shared memory: 4 M tokens a row
+#define SAMPLE_MAX_STRETCHES 1024       // 4 M tokens a row
 #define SAMPLE_NARROW_K 64
 struct RowLayout {
     int vocab, stretches, stretch;      // stretch: tokens a stretch (the last one may be shorter), a multiple of 4

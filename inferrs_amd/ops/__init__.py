@@ -588,7 +588,7 @@ def attention_split(n_seqs: int, nkv: int, g: int, max_q_len: int, max_kv_len: i
     return splits, chunk
 
 
-DECODE_WAVES = 1024            # the decode kernel holds a wave a SIMD: as many waves as the chip has SIMDs, no more
+DECODE_WAVES = 1024            # as many waves as the chip has SIMDs (head sizes up to 128 have room for two on each, see below)
 DECODE_MIN_CHUNK = 64          # fewest keys a wave's share is worth (two steps of 32); 128 up to a context of 512
 DECODE_MANY_SPLITS = 32        # more splits than these only where a split would still hold more than 128 keys
 
@@ -598,8 +598,11 @@ def decode_split(n_seqs: int, nkv: int, g: int, max_kv_len: int) -> Tuple[int, i
     (request x kv head x 16 query heads x split) within one round of the chip and a wave's share at 64 keys
     or more; beyond 32 splits (eight blocks to merge) only where a share would exceed 128 keys.  Measured at head
     size 128, 32 query and 8 kv heads, context 8,192 (microseconds a layer): batch 1
-    17.8 with 64 splits against 21.3 with 32, batch 4 31.1 with 32 against 36.6 with 16, batch 8 51.2 with 16
-    against 56.5 with 32, batch 64 at 1,500 72.0 with 2 against 71.2 with 4 and 82 with 8.  Shares of 64 keys against 128:
+    17.8 with 64 splits against 21.3 with 32, batch 4 31.3 with 32 against 36.7 with 16.  A SIMD has the registers for two waves up to a
+    head size of 128, and twice the waves, two rounds' worth side by side, are slower up to 32 requests (batch 4 37.3, batch 8 56.2
+    against 51.3 and at 2,000 18.4 against 17.4, batch 16 at 1,500 25.6 against 24.8, batch 32 at 1,500 43.2 against 37.8): more partial
+    results to hand over, and one wave's loads keep a SIMD's share of the memory busy; at 64 requests they are 1 to 5 % faster (700 keys
+    36.0 against 37.2, 1,500 71.1 and 72.0, 4,000 177.6 and 187.3): not taken.  Shares of 64 keys against 128:
     batch 1 at 2,048 9.3 against 11.8; batch 4 12.6 against 14.1; batch 8 17.6 against 21.1; and 64 splits of 64 keys at 4,096 lose
     to 32 of 128 (batch 2, an earlier kernel: 17.0 against 16.0).  Shares of 32 keys at a bound of 1,024 are worth 0.2 to 1.0 us to one
     to four requests (16 query heads, batch 1, 700 keys 8.0 against 8.7) and lose at eight (12.6 against 11.3): not taken."""
