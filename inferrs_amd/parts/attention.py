@@ -241,6 +241,8 @@ class Attention(Mixer):
         if q.dtype != torch.float32 or ctx.n_single != 0:
             return False
         sizes = (s.n_heads, s.n_kv_heads, s.head_dim, min(s.window or 1 << 30, s.mask_chunk or 1 << 30))
+        if ctx.n_seqs == 1:
+            return ops.attention_portions_pay([ctx.n_tokens], [ctx.max_kv_len - ctx.n_tokens], *sizes)
         return ctx.once(("portions", *sizes), lambda: ops.attention_portions_pay(ctx.q_lens, ctx.kv_starts, *sizes))
 
     def load_notes(self, page_size: int):

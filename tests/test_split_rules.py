@@ -155,10 +155,11 @@ def test_portions_in_32_bits_take_the_faster_kernel_at_the_measured_points(heads
     from inferrs_amd.parts.attention import Attention
     nq, nkv, d = heads
     spec = SimpleNamespace(n_heads=nq, n_kv_heads=nkv, head_dim=d, window=span, mask_chunk=None)
-    ctx = SimpleNamespace(n_single=0, n_seqs=len(q_lens), n_tokens=sum(q_lens), q_lens=q_lens, kv_starts=kv_starts, _tables={})
+    ctx = SimpleNamespace(n_single=0, n_seqs=len(q_lens), n_tokens=sum(q_lens), q_lens=q_lens, kv_starts=kv_starts, _tables={},
+                          max_kv_len=max(a + b for a, b in zip(q_lens, kv_starts)))
     ctx.once = lambda key, make: StepContext.once(ctx, key, make)
     q = torch.empty(0)
     assert Attention.portions_pay(spec, ctx, q) == (portions < plain)
-    assert Attention.portions_pay(spec, ctx, q) == (portions < plain) and len(ctx._tables) == 1
+    assert Attention.portions_pay(spec, ctx, q) == (portions < plain) and len(ctx._tables) == (len(q_lens) > 1)
     ctx.n_single = 1
     assert not Attention.portions_pay(spec, ctx, q) and not Attention.portions_pay(spec, SimpleNamespace(n_single=0), q.bfloat16())
