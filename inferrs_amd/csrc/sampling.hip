@@ -219,6 +219,7 @@ struct Penalties {
 };
 
 #define PENALTY_STAGED 1024                         // entries of a window that a block keeps in shared memory
+#define SAMPLE_STRETCH 4096                         // tokens of a row that a block draws among (see RowLayout)
 
 // one thread per distinct token of the window: the one holding its first occurrence
 __device__ __forceinline__ void penalize_window(float* z, int lo, int n, const int* held, int w, float rp, float fp, float pp) {
@@ -250,8 +251,9 @@ __device__ __forceinline__ void stage_window(const Penalties& p, int rowi, int* 
 }
 
 // A row's bias and penalties on the logits of its tokens lo .. lo + n, which lie at z[0 .. n) (shared or global memory).
-// All threads of the block call it, with every z and the staged window written behind a barrier; it ends with one.
-__device__ __forceinline__ void penalize_range(float* z, int lo, int n, const Penalties& p, int rowi, const int* s_win) {
+// All threads of the block call it, with every z and the staged window written behind a barrier; it ends with one.  `s_win`: see
+// stage_window, PENALTY_STAGED words also where the window is longer.
+__device__ __forceinline__ void penalize_range(float* z, int lo, int n, const Penalties& p, int rowi, int* s_win) {
     const int w = p.w;
     const float rp = w > 0 ? p.rep[rowi] : 1.f, fp = w > 0 ? p.freq[rowi] : 0.f, pp = w > 0 ? p.pres[rowi] : 0.f;
     if (p.nb > 0) {
@@ -261,8 +263,32 @@ __device__ __forceinline__ void penalize_range(float* z, int lo, int n, const Pe
         }
         __syncthreads();
     }
-    if (w > PENALTY_STAGED) penalize_window(z, lo, n, p.window + (size_t)rowi * w, w, rp, fp, pp);
-    else penalize_window(z, lo, n, s_win, w, rp, fp, pp);
+    const int* held = s_win;
+    int m = w;
+    if (w > PENALTY_STAGED) {
+        // A long window: its entries among the stretch's tokens, in any order, where these fit (each entry searched the whole window in
+        // memory: whole draws with the last 4,000 tokens, us, 128 rows of 262,144 21,615 -> 7,932, 24 rows of 151,936 4,612 -> 1,557).  A
+        // whole row's do not fit.
+        __shared__ int s_held;
+        const int* const all = p.window + (size_t)rowi * w;
+        held = all;
+        if (n <= SAMPLE_STRETCH) {
+            if (threadIdx.x == 0) s_held = 0;
+            __syncthreads();
+            for (int j = threadIdx.x; j < w; j += blockDim.x) {
+                const int id = all[j];
+                if (id < lo || id - lo >= n) continue;
+                const int slot = atomicAdd(&s_held, 1);
+                if (slot < PENALTY_STAGED) s_win[slot] = id;
+            }
+            __syncthreads();
+            if (s_held <= PENALTY_STAGED) {
+                held = s_win;
+                m = s_held;
+            }
+        }
+    }
+    penalize_window(z, lo, n, held, m, rp, fp, pp);
     __syncthreads();
 }
 
@@ -694,7 +720,6 @@ __device__ bool sample_top_k(int* __restrict__ out, const uint32_t* __restrict__
 // A row's words: keys [vocab], probabilities [vocab], the candidates' keys (narrow rows: their logits over the
 // temperature) and tokens [stretches * SAMPLE_FAST_K] each, and the stretches' maxima, sums and sums of probabilities
 // (narrow rows: numbers of candidates) [stretches] each.
-#define SAMPLE_STRETCH 4096
 #define SAMPLE_STAGED 8192              // candidates of a row that its last block keeps in shared memory
 #define SAMPLE_MAX_STRETCHES 1024       // 4 M tokens a row
 #define SAMPLE_NARROW_K 64

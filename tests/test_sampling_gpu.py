@@ -207,6 +207,39 @@ def test_narrow_rows_draw_what_other_rows_with_a_top_k_draw(kind, vocab, top_k):
             assert before - off <= float(u[i]) <= before + float(p[mine]) + off, (kind, i, mine, before, float(u[i]))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("vocab,w", [(10001, 1025), (10001, 2500), (4097, 3000), (151936, 4000)])
+def test_long_windows_penalise_as_one_block_does(vocab, w):
+    """Windows beyond what a block keeps in shared memory: a stretch's block takes the entries among its own tokens, or all of them
+    where these are too many; the draws are those from a copy that one block a row has penalised."""
+    from inferrs_amd import ops
+    g = torch.Generator().manual_seed(vocab + w)
+    rows = 6
+    z = (torch.randn(rows, vocab, generator=g) * 2.5).to("cuda")
+    window = torch.randint(0, vocab, (rows, w), generator=g, dtype=torch.int32)
+    window[0, 5::2] = window[0, 4]                     # one token half of the time: too many entries in its stretch
+    window[1, w // 2:] = -1
+    window[2] = z[2].topk(40).indices.cpu().int()[torch.randint(0, 40, (w,), generator=g)]
+    window[3, ::3] = vocab - 1
+    window[4, ::7] = vocab + 3                          # (no token of the vocabulary)
+    pen = [t.to("cuda") for t in (window, torch.linspace(0.9, 1.4, rows), torch.linspace(0.0, 0.01, rows), torch.full((rows,), 0.1))]
+    touched = ops.penalize(z.clone(), *pen)
+    exact = z.double().cpu()
+    for i in range(rows):
+        ids, counts = window[i][(window[i] >= 0) & (window[i] < vocab)].long().unique(return_counts=True)
+        v = exact[i, ids]
+        exact[i, ids] = torch.where(v >= 0, v / float(pen[1][i]), v * float(pen[1][i])) - float(pen[2][i]) * counts - float(pen[3][i])
+    assert float((touched.cpu().double() - exact).abs().max()) < 1e-4       # (counts up to w at 0.01 each: values of up to 40, rounded thrice)
+    temperature, u = torch.full((rows,), 1.5, device="cuda"), torch.rand(rows, generator=g).to("cuda")
+    top_p, min_p = torch.full((rows,), 0.95, device="cuda"), torch.zeros(rows, device="cuda")
+    n_top = torch.full((rows,), 20, dtype=torch.int32, device="cuda")
+    for k in (50, 200):
+        top_k = torch.full((rows,), k, dtype=torch.int32, device="cuda")
+        got = ops.sample(z, temperature, top_k, top_p, min_p, u, n_top, penalties=pen)
+        want = ops.sample(touched, temperature, top_k, top_p, min_p, u, n_top)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), k
+
+
 def _draw_and_way(args, vocab, pen, narrow_only):
     """`ops.sample` with a workspace of the test's own: the result, and the way each row went, by what it left there."""
     from inferrs_amd import ops
