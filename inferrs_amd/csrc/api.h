@@ -138,6 +138,8 @@ int ia_gemm_mid_tune(int kc, int ns);
 int ia_gemm_mid_blocking(int how);
 // (tiles of 16 rows a block takes at most, 1 to 8, for measurements and tests; 0: the kernel's own rule; the same bits)
 int ia_gemm_mid_rows(int tiles);
+// (the tiles that the rule gives a block of a product of M rows)
+int ia_gemm_mid_row_tiles(int M, int N, int K, int dual, int splits);
 // (a fixed shape of the blocks for measurements and tests: waves a block, 2 to 8 (0: the kernel's own rule), ways k is split
 // and stages, 2 or 3 (2: four waves only); the caller's partial sums must have as many splits); a shape that has no
 // kernel is an error and changes nothing

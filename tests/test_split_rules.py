@@ -163,3 +163,14 @@ def test_portions_in_32_bits_take_the_faster_kernel_at_the_measured_points(heads
     assert Attention.portions_pay(spec, ctx, q) == (portions < plain) and len(ctx._tables) == (len(q_lens) > 1)
     ctx.n_single = 1
     assert not Attention.portions_pay(spec, ctx, q) and not Attention.portions_pay(spec, SimpleNamespace(n_single=0), q.bfloat16())
+
+
+@pytest.mark.parametrize("rows,n,k,dual,splits,tiles", [
+    (24, 3072, 1024, 1, 1, 1), (117, 3072, 1024, 1, 1, 2), (64, 1024, 2048, 0, 4, 1), (117, 4096, 1024, 0, 2, 4),    # groups: two blocks a unit
+    (103, 5120, 1024, 0, 2, 7), (107, 5120, 1536, 0, 2, 7), (84, 6144, 640, 1, 1, 6), (89, 8192, 512, 1, 1, 6),      # which these have no room for
+    (64, 2560, 4096, 0, 8, 4), (117, 6144, 2048, 1, 1, 8), (16, 1024, 1024, 0, 2, 1)])
+def test_rows_of_the_mid_products_are_grouped_within_one_round_of_the_chip(rows, n, k, dual, splits, tiles):
+    """Tiles of 16 rows a block at measured points (256 compute units, which is what the rule takes without a GPU too)."""
+    lib = ops.library()
+    assert dual or lib.ia_gemm_mid_splits(n, k) == splits
+    assert lib.ia_gemm_mid_row_tiles(rows, n, k, dual, splits) == tiles
