@@ -407,8 +407,8 @@ __global__ __launch_bounds__(W * IA_WAVE) void gemm_mid_kernel(
 // Wanted: a block for every compute unit and no more, three stages deep (a block a unit: what it has under way is all that
 // hides the memory's latency; two rounds of blocks would leave the second half empty).  Among the ways that one round holds the
 // one that fills the chip best wins; of ways that fill it alike, the one with the most waves a block (the rows of x are fetched once
-// a block) as long as a block keeps eight chunks of k.  A weight whose best way leaves less than 0.3 of the chip at work, or of
-// which one round holds none, takes four waves a block two stages deep, several blocks a unit, k split until there is a block for
+// a block) as long as a block keeps eight chunks of k.  A weight whose best way leaves less than 0.3 of the chip at work (or less than 0.9
+// and is the slower one, see mid_plan), or of which one round holds none, takes four waves a block two stages deep, several blocks a unit, k split until there is a block for
 // every unit; one of four rounds and more of blocks of eight waves (a logits head) takes those, three stages deep.
 static int mid_cus() {
     static int cus = 0;
@@ -466,7 +466,17 @@ static MidPlan mid_plan(int N, int K, bool dual) {
     // share that was measured).  (Blocks of four waves two stages
     // deep, several a unit, had taken those weights: 2 x 9,728 x 2,560, 0.79 of the chip, 24 rows 27.7 -> 22.0 us, 64 rows 33.4 -> 25.2, 117 rows
     // 51.5 -> 34.5; 2 x 6,144 x 2,048, 0.75, 18.0 -> 13.2, 19.8 -> 15.1, 20.7 -> 20.3; 2,560 x 9,728, 0.84, 18.8 -> 12.8, 20.8 -> 17.1, 22.0 -> 22.6.)
-    if (best.waves != 0 && best_fill >= 0.3) return best;
+    // Not where the two stages would have split k more often (3,200 x 2,048 to 3,072 and the like: a block's chain twice as long, 0.84 to 0.97
+    // of their speed over 8 points), nor for three waves over whole k (9,728 and 10,240 features of up to 1,152 k: no pairs of tiles, 0.91
+    // to 1.04, 0.96 in the mean of 16; three waves with splits 0.96 to 1.35).
+    MidPlan wide = {4, 1, 2, 0.0};
+    if (!dual) {
+        const int blocks = (N + 63) / 64;
+        while (blocks * wide.splits < cus && wide.splits < 16 && chunks % (2 * wide.splits) == 0 && chunks / (2 * wide.splits) >= 4)
+            wide.splits *= 2;
+    }
+    const bool worse = best_fill < 0.9 && (best.splits < wide.splits || (best.waves == 3 && best.splits == 1));
+    if (best.waves != 0 && best_fill >= 0.3 && !worse) return best;
     // Four rounds and more of blocks of eight waves (a logits head): the rows of x are fetched half as often as by blocks of
     // four, and three stages hide the memory better than a second block.  The head alone, five vocabularies of 131,072 to 262,144, the
     // time of blocks of four / eight waves in the mean: 5,120 k 24 rows 1.05, 64 rows 1.08, 128 rows 1.21, 4,096 k 1.02, 1.08, 1.21,
@@ -474,12 +484,6 @@ static MidPlan mid_plan(int N, int K, bool dual) {
     // 20 rows 197 / 195 us, 64 rows 235 / 233, 96 rows 249 / 255, 128 rows 308 / 289, 2,048 k 278 / 278, 322 / 320, 351 / 347, 408 / 383;
     // over four vocabularies 1.05 to 1.08 at 112 and 128 rows, up to 96 rows 0.96 (200,064 features of 1,024 k at 80 and 96) to 1.02.
     if (!dual && tiles >= 4 * 8 * cus) return {8, 1, 3, 1.0};
-    MidPlan wide = {4, 1, 2, 0.0};
-    if (!dual) {
-        const int blocks = (N + 63) / 64;
-        while (blocks * wide.splits < cus && wide.splits < 16 && chunks % (2 * wide.splits) == 0 && chunks / (2 * wide.splits) >= 4)
-            wide.splits *= 2;
-    }
     return wide;
 }
 

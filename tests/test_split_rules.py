@@ -176,3 +176,9 @@ def test_rows_of_the_mid_products_are_grouped_within_one_round_of_the_chip(rows,
     lib = ops.library()
     assert dual or splits == 1 or lib.ia_gemm_mid_splits(n, k) == splits
     assert lib.ia_gemm_mid_row_tiles(rows, n, k, dual, splits) == tiles
+
+
+@pytest.mark.parametrize("n,k,splits", [(3200, 2048, 4), (3200, 3072, 4), (9728, 512, 1), (10240, 1152, 1),      # two stages are faster
+                                        (3072, 1024, 2), (2560, 9728, 4), (1024, 3072, 4), (5120, 1536, 2), (3200, 3328, 2)])
+def test_plans_of_small_weights_split_k_as_often_as_two_stages_would(n, k, splits):
+    assert ops.library().ia_gemm_mid_splits(n, k) == splits
