@@ -42,15 +42,14 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define HD IA_HEAD_DIM
 // The values' width where it is not the keys' (IA_VALUE_DIM, a multiple of 16 up to 256): the kernel of single waves
-// and the merges of split keys take it; the decode kernel and the tile kernel are for values as wide as keys.
+// the merges of split keys and the decode kernel take any, the tile kernel the widths below.
 #ifndef IA_VALUE_DIM
 #define IA_VALUE_DIM IA_HEAD_DIM
 #endif
 static_assert(IA_VALUE_DIM % 16 == 0 && IA_VALUE_DIM >= 16 && IA_VALUE_DIM <= 256, "value size");
 #define HDV IA_VALUE_DIM
 #define HDMAX (HD > HDV ? HD : HDV)
-#define DBV (HDV / 16)          // 16-dim blocks of the output
-#define DB (HD / 16)            // the same in the kernels for values as wide as keys
+#define DBV (HDV / 16)          // 16-dim blocks of the values
 // The tile kernel (prompt portions, keys of 128) takes values of 32 to 128 in steps of 32: a load of 1 KiB brings 32 features
 // of 16 keys, and the groups' exchange at its end fits the stages up to the keys' own width.
 #define TILE_FITS (HD == 128 && HDV % 32 == 0 && HDV <= 128)
@@ -74,10 +73,14 @@ struct AttnParams {
     // The decode kernel, with the per-head norm, the rotation and the cache write inside: q is not
     // read from `q` but formed from the projections' output, and the wave that walks a request's
     // newest key forms that key and value, uses them and writes them to the cache.
-    const bf16_t* qkv;          // [n, (nq + 2 nkv) * d]: q heads, then k heads, then v heads
+    const bf16_t* qkv;          // [n, row_ld]: q heads at q_off, k heads at k_off, v heads at v_off of a token's row
+    int row_ld, q_off, k_off, v_off;
+    int rot;                    // features of a head that rotate, halves paired (a multiple of 8)
+    const bf16_t* gate;         // null, or where a token's gate values begin in its row: the output is times their sigmoid
+    int gate_ld, gate_per_head; // pitch of the rows; 1: a value a query head, 0: a value a feature
     const float* q_norm_w;      // [d], or null: no norm
     const float* k_norm_w;
-    const float* cos_t;         // [n, d / 2], or null: no rotation
+    const float* cos_t;         // [n, rot / 2], or null: no rotation
     const float* sin_t;
     const int* slots;           // [n] cache slot of each token, or null: this layer writes no cache
     float norm_eps;
@@ -88,7 +91,7 @@ struct AttnParams {
     int keep_first;             // > 0: it sees the first so many positions besides (forms 1 and 2)
     uint32_t page_magic;        // decode kernel: pos / page is umulhi(2 (pos / 16), page_magic) >> page_shift
     int page_shift;
-    int teams_log2;             // decode kernel: log2 of the blocks that share a (request, key/value head)
+    int teams, col_blocks;      // decode kernel: blocks that share the keys of a (request, key/value head, block of 16 query heads), and those blocks of heads
     float cap_in;               // form 2: a raw score s stands for tanh(s * scale / cap); this is 2 log2(e) scale / cap, and scale_log2 is cap * log2(e)
 };
 
@@ -475,6 +478,12 @@ __device__ __forceinline__ float column_sum(float x) {
 //    last block reads past the caches after it has seen the full count.  The counters are zero
 //    between calls (the last block puts its counter back), so calls that share them must not overlap.
 // The sum over the splits runs in the order of the splits whoever comes last: the result is the same every time.
+// Rows of any layout come in: query, key and value heads at places of their own, values narrower or wider than keys, the first `rot`
+// features of a head turned, a gate's values behind them (the output is times their sigmoid before it is rounded), no keys at all
+// (a layer that reads another's cache; queries that a kernel before has formed).  16 query heads of 128 beside values of 64 and a gate,
+// 8 requests at 2,000 keys, window 1,024: four kernels of 5.3, 7.8, 4.5 and 4.0 us (norm and rotation, attention, merge, gate), 10.2 in
+// this one, a step of six such layers 657 -> 600 us; the single tokens of a step that also brings a portion, 40 query heads, 9 requests at 3,100
+// keys: 28.6 + 4.8 us by the kernel of single waves and its merge, 27.1 here beside nothing else.
 // A wave is mostly alone on its SIMD, so every instruction it executes is four cycles of the step (returning from the kernel early, 16 query
 // and 8 key/value heads, 700 keys, 64 a wave: rows and first keys are there 1.0 us after the start, rows formed 2.0 later, two steps done
 // 3.5 later, a team merged 0.9 later, the hand-over 2.5).  So rows are formed by all lanes, numbers of pages come without divisions,
@@ -511,28 +520,35 @@ __device__ __forceinline__ float row_sum(float x) {
     return x;
 }
 
+// 32-bit words of shared memory of a wave with `cols` columns: its rows and the new key, and behind its walk its partial outputs in
+// the same place (a wave may be at its outputs while another still reads its rows: the places of two waves have nothing in common).
+__host__ __device__ constexpr int decode_wave_words(int cols) {
+    return cols * HDV > (cols + 1) * HD / 2 ? cols * HDV : (cols + 1) * HD / 2;
+}
+
 struct DecodeOperands {
     uint4 k[2][KS];             // as Operands above
-    uint4 v[DB];
+    uint4 v[DBV];
 };
 
 #define DECODE_TEAM 4           // waves of a block at most
 
-template <bool ENABLED = (HD % 64 == 0 && HDV == HD)>
-__global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_per_eu(HD <= 128 ? 2 : 1))) void attn_decode_kernel(const AttnParams p, int* counters, int team) {
+template <bool ENABLED = (HD % 64 == 0)>
+__global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_per_eu(HDMAX <= 128 ? 2 : 1))) void attn_decode_kernel(const AttnParams p, int* counters, int team) {
     if constexpr (ENABLED) {
-        extern __shared__ __align__(16) float team_mem[];       // [team][columns][HD] partial outputs, then [team][columns][2]
+        extern __shared__ __align__(16) float team_mem[];       // [team][words of a wave], then [team][columns][2]
         __shared__ int s_last;
         // (the wave's number through a scalar register: what follows from it, the split's range and the pages' numbers,
         // is then the same for all lanes by construction, and the block table is read through the scalar cache)
         const int lane = threadIdx.x & (IA_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / IA_WAVE);
         const int r = lane & 15, G = lane >> 4;
         const int g = p.nq / p.nkv;
-        const int teams = 1 << p.teams_log2;
-        const int kvh = blockIdx.y >> p.teams_log2, tm = blockIdx.y & (teams - 1);
+        const int teams = p.teams;
+        const int cb = p.col_blocks > 1 ? (int)blockIdx.x / teams : 0;
+        const int kvh = blockIdx.y, tm = (int)blockIdx.x - cb * teams;
         const int split = tm * team + wave;
         const int seq = p.seq_begin + blockIdx.z;
-        const int col0 = blockIdx.x * 16;
+        const int col0 = cb * 16;
         const int n_cols = g - col0 < 16 ? g - col0 : 16;       // this block's columns (the grid has no empty block)
         // (a division by a number known at run time only is some thirty instructions one after the other, and the walk's start
         // would wait for six of them)
@@ -568,31 +584,32 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
         // key's), the norms' weights and the angles, then the first step's keys and values: the rows are formed while those are
         // on their way, and the second step's are asked for after that (a wave can have 63 loads outstanding: all at once
         // would stall the issue of the last ones until the first come back).
-        // The rows are shared out over all lanes: a lane has four features of a row and the four that they are turned with, HD / 2
-        // further on, a pass takes ROWS rows, and they meet the matrix operand's layout in the wave's own shared memory.  (With a
+        // The rows are shared out over all lanes: a lane has four features of a row and the four that they are turned with, rot / 2
+        // further on (behind the features that rotate: the next four), a pass takes ROWS rows, and they meet the matrix operand's layout in the wave's own shared memory.  (With a
         // column's features in the four lanes that need them, 32 a lane, two rows took 2 of the 7 us that a wave has.)
-        const int qkv_row = (p.nq + 2 * p.nkv) * HD;
-        const bf16_t* token_row = p.qkv + (size_t)t0 * qkv_row;
+        const bf16_t* token_row = p.qkv + (size_t)t0 * p.row_ld;
         constexpr int ROW_LANES = HD <= 64 ? 8 : HD <= 128 ? 16 : 32, ROWS = IA_WAVE / ROW_LANES, ROW_USED = HD / 8;
         const int ri = lane % ROW_LANES < ROW_USED ? lane % ROW_LANES : ROW_USED - 1, rsub = lane / ROW_LANES;
+        const bool rotates = 8 * ri < p.rot;
+        const int fa = rotates ? 4 * ri : 8 * ri, fb = rotates ? 4 * ri + p.rot / 2 : 8 * ri + 4;       // (the first rot / 8 lanes hold the rotated part)
         struct RowPart { uint2 lo, hi; float4 wlo, whi; };
         auto ask_rows = [&](RowPart& part, int pass) __attribute__((always_inline)) {
             const int t = pass * ROWS + rsub;
-            const bf16_t* from = token_row + (size_t)(t < n_cols ? kvh * g + col0 + t : p.nq + kvh) * HD + 4 * ri;
-            part.lo = *(const uint2*)from;
-            part.hi = *(const uint2*)(from + HD / 2);
+            const bf16_t* from = token_row + (t < n_cols ? p.q_off + (kvh * g + col0 + t) * HD : p.k_off + kvh * HD);
+            part.lo = *(const uint2*)(from + fa);
+            part.hi = *(const uint2*)(from + fb);
             if (p.q_norm_w != nullptr) {
-                const float* w = (t < n_cols ? p.q_norm_w : p.k_norm_w) + 4 * ri;
-                part.wlo = *(const float4*)w;
-                part.whi = *(const float4*)(w + HD / 2);
+                const float* w = t < n_cols ? p.q_norm_w : p.k_norm_w;
+                part.wlo = *(const float4*)(w + fa);
+                part.whi = *(const float4*)(w + fb);
             }
         };
         RowPart rows0, rows1;
         ask_rows(rows0, 0);
         float4 cs = make_float4(1.f, 1.f, 1.f, 1.f), sn = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (p.cos_t != nullptr) {
-            cs = *(const float4*)(p.cos_t + (size_t)t0 * (HD / 2) + 4 * ri);
-            sn = *(const float4*)(p.sin_t + (size_t)t0 * (HD / 2) + 4 * ri);
+        if (p.cos_t != nullptr && rotates) {
+            cs = *(const float4*)(p.cos_t + (size_t)t0 * (p.rot / 2) + 4 * ri);
+            sn = *(const float4*)(p.sin_t + (size_t)t0 * (p.rot / 2) + 4 * ri);
         }
         if (n_cols + 1 > ROWS) ask_rows(rows1, 1);
 
@@ -609,8 +626,8 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
             const int off_a = k0 - page_of(k0) * p.page, off_b = k0 + 16 - page_of(k0 + 16) * p.page;
             const char* ka = (const char*)(p.k_cache + (((size_t)page_a * p.nkv + kvh) * p.page + off_a) * HD);
             const char* kb = (const char*)(p.k_cache + (((size_t)page_b * p.nkv + kvh) * p.page + off_b) * HD);
-            const char* va = (const char*)(p.v_cache + ((size_t)page_a * p.nkv + kvh) * HD * p.page + off_a);
-            const char* vb = (const char*)(p.v_cache + ((size_t)page_b * p.nkv + kvh) * HD * p.page + off_b);
+            const char* va = (const char*)(p.v_cache + ((size_t)page_a * p.nkv + kvh) * HDV * p.page + off_a);
+            const char* vb = (const char*)(p.v_cache + ((size_t)page_b * p.nkv + kvh) * HDV * p.page + off_b);
             const char* kbase = k_second ? kb : ka;
             const char* vbase = (v_second ? vb : va) + v_lane;
 #pragma unroll
@@ -618,7 +635,7 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) op.k[t][ks] = *(const uint4*)(kbase + k_lane[t] + ks * 64);
 #pragma unroll
-            for (int db = 0; db < DB; ++db) op.v[db] = *(const uint4*)(vbase + db * v_stride);
+            for (int db = 0; db < DBV; ++db) op.v[db] = *(const uint4*)(vbase + db * v_stride);
         };
         auto load_step = [&](DecodeOperands& op, int k0) __attribute__((always_inline)) {
             int idx_a = page_of(k0), idx_b = page_of(k0 + 16);
@@ -637,17 +654,17 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
 
         const bool has_new = p.slots != nullptr && hi == kv_total && lo < hi;
         const int slot = has_new ? p.slots[t0] : 0;
-        uint32_t vnew[DB];
+        uint32_t vnew[DBV];
         if (has_new) {
 #pragma unroll
-            for (int db = 0; db < DB; ++db) vnew[db] = token_row[(size_t)(p.nq + p.nkv + kvh) * HD + db * 16 + r].bits;
+            for (int db = 0; db < DBV; ++db) vnew[db] = token_row[p.v_off + kvh * HDV + db * 16 + r].bits;
         }
         if (n_steps >= 2) load_early(opb, lo + 32, 1);
 
         // Rows, normed and rotated as the separate kernel does it (32-bit throughout, one rounding at the end).  A row's 16-byte
         // pieces lie exchanged by its number, so that operand reads of several rows meet no bank twice.  They fit where the wave's
         // partial outputs will lie.
-        char* const row_mem = (char*)(team_mem + (size_t)wave * n_cols * HD);
+        char* const row_mem = (char*)(team_mem + (size_t)wave * decode_wave_words(n_cols));
         auto form_rows = [&](const RowPart& part, int pass) __attribute__((always_inline)) {
             const int t = pass * ROWS + rsub;
             float a[4] = {__uint_as_float(part.lo.x << 16), __uint_as_float(part.lo.x & 0xffff0000u),
@@ -667,7 +684,7 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
 #pragma unroll
                 for (int j = 0; j < 4; ++j) { a[j] = scale * a[j] * (wa[j] + one); b[j] = scale * b[j] * (wb[j] + one); }
             }
-            if (p.cos_t != nullptr) {
+            if (p.cos_t != nullptr && rotates) {
                 const float c[4] = {cs.x, cs.y, cs.z, cs.w}, sv[4] = {sn.x, sn.y, sn.z, sn.w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
@@ -677,9 +694,9 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
                 }
             }
             if (t <= n_cols && lane % ROW_LANES < ROW_USED) {
-                char* const at = row_mem + t * (HD * 2) + (ri & 1) * 8;
-                *(uint2*)(at + ((ri / 2) ^ (t & 7)) * 16) = make_uint2(pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]));
-                *(uint2*)(at + ((HD / 16 + ri / 2) ^ (t & 7)) * 16) = make_uint2(pack_bf16x2(b[0], b[1]), pack_bf16x2(b[2], b[3]));
+                char* const at = row_mem + t * (HD * 2);
+                *(uint2*)(at + ((fa >> 3) ^ (t & 7)) * 16 + (fa & 4) * 2) = make_uint2(pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]));
+                *(uint2*)(at + ((fb >> 3) ^ (t & 7)) * 16 + (fb & 4) * 2) = make_uint2(pack_bf16x2(b[0], b[1]), pack_bf16x2(b[2], b[3]));
             }
         };
         const int passes = (n_cols + (has_new ? 1 : 0) + ROWS - 1) / ROWS;
@@ -704,10 +721,10 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
             return *(const uint4*)(row_mem + n_cols * (HD * 2) + ((ks * 4 + G) ^ (n_cols & 7)) * 16);
         };
 
-        f32x4 acc[DB];
+        f32x4 acc[DBV];
         float m = -INFINITY, l = 0.f;
 #pragma unroll
-        for (int db = 0; db < DB; ++db) acc[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int db = 0; db < DBV; ++db) acc[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
         // What only the walk's first step needs: keys below the window.
         auto first_edge = [&](DecodeOperands& op, int k0) __attribute__((always_inline)) {
@@ -716,7 +733,7 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
                 const int first_good = window_floor - (k0 + 8 * G);
                 if (first_good > 0) {
 #pragma unroll
-                    for (int db = 0; db < DB; ++db) {
+                    for (int db = 0; db < DBV; ++db) {
                         uint32_t w[4] = {op.v[db].x, op.v[db].y, op.v[db].z, op.v[db].w};
 #pragma unroll
                         for (int j = 0; j < 8; ++j)
@@ -734,7 +751,7 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
                 const int first_bad = kv_total - (k0 + 8 * G);
                 if (first_bad < 8) {
 #pragma unroll
-                    for (int db = 0; db < DB; ++db) {
+                    for (int db = 0; db < DBV; ++db) {
                         uint32_t w[4] = {op.v[db].x, op.v[db].y, op.v[db].z, op.v[db].w};
 #pragma unroll
                         for (int j = 0; j < 8; ++j)
@@ -760,7 +777,7 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
                 const bool vmine = G == (kk >> 3);
                 const uint32_t keep = (j & 1) ? 0x0000ffffu : 0xffff0000u;
 #pragma unroll
-                for (int db = 0; db < DB; ++db) {
+                for (int db = 0; db < DBV; ++db) {
                     const uint32_t put = (j & 1) ? vnew[db] << 16 : vnew[db];
                     op.v[db].x = vmine && (j >> 1) == 0 ? (op.v[db].x & keep) | put : op.v[db].x;
                     op.v[db].y = vmine && (j >> 1) == 1 ? (op.v[db].y & keep) | put : op.v[db].y;
@@ -811,13 +828,13 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
             pb.w = pack_bf16x2(pr[6], pr[7]);
             if (__any(alpha != 1.0f)) {
 #pragma unroll
-                for (int db = 0; db < DB; ++db) {
+                for (int db = 0; db < DBV; ++db) {
                     acc[db][0] *= alpha; acc[db][1] *= alpha;
                     acc[db][2] *= alpha; acc[db][3] *= alpha;
                 }
             }
 #pragma unroll
-            for (int db = 0; db < DB; ++db)
+            for (int db = 0; db < DBV; ++db)
                 acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                     __builtin_bit_cast(bf16x8, op.v[db]), __builtin_bit_cast(bf16x8, pb), acc[db], 0, 0, 0);
         };
@@ -857,53 +874,75 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
                 for (int ks = 0; ks < KS; ++ks) *(uint4*)(krow + ks * 32) = new_key(ks);
             }
             if (G == (kk >> 3)) {
-                bf16_t* vdst = p.v_cache_w + (((size_t)page * p.nkv + kvh) * HD + r) * p.page + off;
+                bf16_t* vdst = p.v_cache_w + (((size_t)page * p.nkv + kvh) * HDV + r) * p.page + off;
 #pragma unroll
-                for (int db = 0; db < DB; ++db) vdst[(size_t)db * 16 * p.page].bits = (uint16_t)vnew[db];
+                for (int db = 0; db < DBV; ++db) vdst[(size_t)db * 16 * p.page].bits = (uint16_t)vnew[db];
             }
         }
 
         const float lt = column_sum(l);
         const size_t row0 = (size_t)t0 * p.nq + kvh * g + col0;        // the block's first (token, head) row
+        // A piece of four features of the output: divided by the row's sum, times the sigmoid of the gate's values.
+        auto ask_gate = [&](int col, int feature) __attribute__((always_inline)) {
+            const bf16_t* from = p.gate + (size_t)t0 * p.gate_ld;
+            const int at = kvh * g + col0 + col;
+            if (p.gate_per_head) {
+                const uint32_t one = from[at].bits * 0x10001u;
+                return make_uint2(one, one);
+            }
+            return *(const uint2*)(from + (size_t)at * HDV + feature);
+        };
+        auto put_out = [&](int col, int feature, const f32x4& o, float inv, const uint2& gate) __attribute__((always_inline)) {
+            float v[4] = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
+            if (p.gate != nullptr) {
+                const float z[4] = {__uint_as_float(gate.x << 16), __uint_as_float(gate.x & 0xffff0000u),
+                                    __uint_as_float(gate.y << 16), __uint_as_float(gate.y & 0xffff0000u)};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[j] = v[j] / (1.0f + expf(-z[j]));
+            }
+            *(uint2*)(p.out + (row0 + col) * HDV + feature) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        };
         if (p.splits == 1) {
             if (!cvalid) return;
             const float inv = 1.0f / (p.sink ? lt + sink_term(p.sinks, head, m) : lt);
-            bf16_t* o = p.out + (row0 + r) * HD + 4 * G;
+            uint2 gate[DBV];
+            if (p.gate != nullptr) {
 #pragma unroll
-            for (int db = 0; db < DB; ++db) {
-                uint2 w;
-                w.x = pack_bf16x2(acc[db][0] * inv, acc[db][1] * inv);
-                w.y = pack_bf16x2(acc[db][2] * inv, acc[db][3] * inv);
-                *(uint2*)(o + 16 * db) = w;
+                for (int db = 0; db < DBV; ++db) gate[db] = ask_gate(r, 16 * db + 4 * G);
             }
+#pragma unroll
+            for (int db = 0; db < DBV; ++db) put_out(r, 16 * db + 4 * G, acc[db], inv, gate[db]);
             return;
         }
 
         // ---- the block's waves add up: lane (col, G) holds dims 16 db + 4 G + i of its column --------
-        float* team_o = team_mem;                                       // [team][n_cols][HD]
-        float* team_ml = team_mem + (size_t)team * n_cols * HD;         // [team][n_cols][2]
+        const int words = decode_wave_words(n_cols);
+        float* team_o = team_mem;                                       // [team][words], of each [n_cols][HDV]
+        float* team_ml = team_mem + (size_t)team * words;               // [team][n_cols][2]
         if (cvalid) {
-            float* o = team_o + ((size_t)wave * n_cols + r) * HD + 4 * G;
+            float* o = team_o + (size_t)wave * words + r * HDV + 4 * G;
 #pragma unroll
-            for (int db = 0; db < DB; ++db) *(f32x4*)(o + 16 * db) = acc[db];
+            for (int db = 0; db < DBV; ++db) *(f32x4*)(o + 16 * db) = acc[db];
             if (G == 0) {
                 team_ml[(wave * n_cols + r) * 2] = m;
                 team_ml[(wave * n_cols + r) * 2 + 1] = lt;
             }
         }
         __syncthreads();
-        const int pieces = n_cols * (HD / 4);                           // 16-byte pieces of the block's result
+        const int pieces = n_cols * (HDV / 4);                           // 16-byte pieces of the block's result
         for (int e = threadIdx.x; e < pieces; e += blockDim.x) {
-            const int col = e / (HD / 4), piece = e - col * (HD / 4);
+            const int col = e / (HDV / 4), piece = e - col * (HDV / 4);
             // (all of the team's results are asked for together)
             float mw[DECODE_TEAM], lw[DECODE_TEAM], mx = -INFINITY, total = 0.f;
+            uint2 gate = make_uint2(0, 0);
+            if (teams == 1 && p.gate != nullptr) gate = ask_gate(col, piece * 4);
             f32x4 v[DECODE_TEAM], o = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int w = 0; w < DECODE_TEAM; ++w) {
-                const int at = (w < team ? w : 0) * n_cols + col;
+                const int of = w < team ? w : 0, at = of * n_cols + col;
                 mw[w] = team_ml[at * 2];
                 lw[w] = team_ml[at * 2 + 1];
-                v[w] = *(const f32x4*)(team_o + (size_t)at * HD + piece * 4);
+                v[w] = *(const f32x4*)(team_o + (size_t)of * words + col * HDV + piece * 4);
                 mx = fmaxf(mx, mw[w]);
             }
 #pragma unroll
@@ -915,12 +954,9 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
             }
             if (teams == 1) {
                 const float inv = 1.0f / (p.sink ? total + sink_term(p.sinks, (int)((row0 + col) % p.nq), mx) : total);
-                uint2 w;
-                w.x = pack_bf16x2(o[0] * inv, o[1] * inv);
-                w.y = pack_bf16x2(o[2] * inv, o[3] * inv);
-                *(uint2*)(p.out + (row0 + col) * HD + piece * 4) = w;
+                put_out(col, piece * 4, o, inv, gate);
             } else {
-                float* po = p.part_o + ((row0 + col) * teams + tm) * HD + piece * 4;
+                float* po = p.part_o + ((row0 + col) * teams + tm) * HDV + piece * 4;
                 put_across(po, o[0]); put_across(po + 1, o[1]); put_across(po + 2, o[2]); put_across(po + 3, o[3]);
                 if (piece == 0) {
                     float* ml = p.part_ml + ((row0 + col) * teams + tm) * 2;
@@ -932,7 +968,7 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
         if (teams == 1) return;
 
         // ---- the last block of this (request, key/value head, column block) merges the blocks' results --------
-        int* counter = counters + ((size_t)blockIdx.z * p.nkv + kvh) * gridDim.x + blockIdx.x;
+        int* counter = counters + ((size_t)blockIdx.z * p.nkv + kvh) * p.col_blocks + cb;
         // The hand-over.  Writer: a wave's vector-memory counter counts a store down when the memory has taken it
         // (the stores above are written through, so that is the point where every die reads it), and
         // `s_waitcnt vmcnt(0)` holds the wave until all of its stores are there; then the barrier, so that this
@@ -960,10 +996,12 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
             const bool active = grp < groups && e < pieces;
             float mx = -INFINITY, total = 0.f;
             f32x4 o = (f32x4){0.f, 0.f, 0.f, 0.f};
-            const int col = active ? e / (HD / 4) : 0, piece = active ? e - col * (HD / 4) : 0;
+            const int col = active ? e / (HDV / 4) : 0, piece = active ? e - col * (HDV / 4) : 0;
+            uint2 gate = make_uint2(0, 0);
             if (active) {
+                if (grp == 0 && p.gate != nullptr) gate = ask_gate(col, piece * 4);
                 const float* ml = p.part_ml + (row0 + col) * teams * 2;
-                const float* po = p.part_o + (row0 + col) * teams * HD + piece * 4;
+                const float* po = p.part_o + (row0 + col) * teams * HDV + piece * 4;
                 // (eight blocks' results at a time, their loads under way together and one change of the maximum for all)
                 constexpr int AT_ONCE = 8;
                 for (int t1 = grp; t1 < teams; t1 += AT_ONCE * groups) {
@@ -976,7 +1014,7 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
                         lt_[i] = 0.f;
                         v[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
                         if (t < teams) {
-                            const float* pv = po + (size_t)t * HD;
+                            const float* pv = po + (size_t)t * HDV;
                             mt[i] = get_across(ml + 2 * t);
                             lt_[i] = get_across(ml + 2 * t + 1);
                             v[i] = (f32x4){get_across(pv), get_across(pv + 1), get_across(pv + 2), get_across(pv + 3)};
@@ -1018,10 +1056,7 @@ __global__ __launch_bounds__(DECODE_TEAM * IA_WAVE) __attribute__((amdgpu_waves_
                 continue;
             }
             const float inv = 1.0f / (p.sink ? total + sink_term(p.sinks, (int)((row0 + col) % p.nq), mx) : total);
-            uint2 w;
-            w.x = pack_bf16x2(o[0] * inv, o[1] * inv);
-            w.y = pack_bf16x2(o[2] * inv, o[3] * inv);
-            *(uint2*)(p.out + (row0 + col) * HD + piece * 4) = w;
+            put_out(col, piece * 4, o, inv, gate);
         }
         if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);     // zero again for the next call
     }
@@ -1653,18 +1688,23 @@ extern "C" long long ia_attention_mfma_workspace(int n, int nq, int splits) {
 struct FusedArgs {
     const void* qkv; const float* q_norm_w; const float* k_norm_w; const float* cos_t; const float* sin_t;
     const int* slots; float eps; int add_one;
+    int row_ld, q_off, k_off, v_off, rot;
+    const void* gate; int gate_ld, gate_per_head;
     int* counters; int n_counters;
 };
 
-// Neighbouring splits that one block of the decode kernel takes (a wave each): four, or two where the waves'
-// results for g query heads of a key/value head would not fit 64 KiB of shared memory.
+// Neighbouring splits that one block of the decode kernel takes (a wave each): up to four, or two where the waves'
+// results for g query heads of a key/value head would not fit 64 KiB of shared memory; every block takes as many.
 static size_t decode_team_bytes(int team, int g) {
-    const size_t waves = (size_t)team * (g < 16 ? g : 16) * (HD + 2), groups = (size_t)team * IA_WAVE * 6;   // (see the kernel's end)
+    const int cols = g < 16 ? g : 16;
+    const size_t waves = (size_t)team * (decode_wave_words(cols) + 2 * cols), groups = (size_t)team * IA_WAVE * 6;   // (see the kernel's end)
     return (waves > groups ? waves : groups) * sizeof(float);
 }
 static int decode_team(int splits, int g) {
     const int team = decode_team_bytes(DECODE_TEAM, g) <= 65536 ? DECODE_TEAM : 2;
-    return splits >= team ? team : splits;
+    int t = splits < team ? splits : team;
+    while (splits % t) --t;
+    return t;
 }
 
 // Floats of workspace that a decode step of `splits` key splits needs (one partial result a block), and the
@@ -1672,7 +1712,7 @@ static int decode_team(int splits, int g) {
 extern "C" long long ia_attention_decode_workspace(int n, int nq, int nkv, int splits) {
     if (n <= 0 || nq <= 0 || nkv <= 0 || splits <= 0) return 0;
     const int teams = splits / decode_team(splits, nq / nkv);
-    return teams > 1 ? (long long)n * nq * teams * (HD + 2) : 0;
+    return teams > 1 ? (long long)n * nq * teams * (HDV + 2) : 0;
 }
 extern "C" long long ia_attention_decode_counters(int n, int nq, int nkv, int splits) {
     if (n <= 0 || nq <= 0 || nkv <= 0 || splits <= 0) return 0;
@@ -1712,7 +1752,8 @@ static int attention_launch(void* out, float* workspace, const void* q, const vo
     p.k_cache_w = (bf16_t*)k_cache;
     p.v_cache_w = (bf16_t*)v_cache;
     p.qkv = nullptr; p.q_norm_w = p.k_norm_w = p.cos_t = p.sin_t = nullptr; p.slots = nullptr;
-    p.norm_eps = 0.f; p.norm_add_one = 0;
+    p.norm_eps = 0.f; p.norm_add_one = 0; p.row_ld = p.q_off = p.k_off = p.v_off = p.rot = 0;
+    p.gate = nullptr; p.gate_ld = p.gate_per_head = 0;
     p.block_table = block_table;
     p.cu_tokens = cu_tokens;
     p.positions = positions;
@@ -1723,7 +1764,7 @@ static int attention_launch(void* out, float* workspace, const void* q, const vo
     IA_CHECK(mask_chunk >= 0 && (sinks == nullptr || sink), "attention_mfma: mask_chunk %d must be >= 0 (0 = none), and sink values go with a sink", mask_chunk);
     p.sinks = sinks; p.mask_chunk = mask_chunk;
     IA_CHECK(keep_first >= 0 && softcap >= 0.f, "attention_mfma: keep_first %d and softcap %g must be >= 0 (0 = none)", keep_first, (double)softcap);
-    p.keep_first = keep_first; p.cap_in = 0.f; p.page_magic = 0; p.page_shift = 0; p.teams_log2 = 0;
+    p.keep_first = keep_first; p.cap_in = 0.f; p.page_magic = 0; p.page_shift = 0; p.teams = p.col_blocks = 1;
     if (softcap > 0.f) {
         p.cap_in = scale / softcap * (2.0f * 1.4426950408889634f);
         p.scale_log2 = softcap * 1.4426950408889634f;
@@ -1739,14 +1780,15 @@ static int attention_launch(void* out, float* workspace, const void* q, const vo
     const dim3 grid((unsigned)(p.pair ? (col_blocks + 1) / 2 : col_blocks), nkv * splits, n_seqs);
     if (fused != nullptr) {
         IA_CHECK(form == FORM_PLAIN, "attention_mfma: the fused form takes no kept first positions and no capped scores");
-        IA_CHECK(HD % 64 == 0 && HDV == HD && max_q_len == 1, "attention_mfma: the fused form takes single tokens, head sizes in "
-                 "steps of 64 and values as wide as keys (head size %d, %d tokens a request)", HD, max_q_len);
+        IA_CHECK(HD % 64 == 0 && max_q_len == 1, "attention_mfma: the fused form takes single tokens and head sizes in "
+                 "steps of 64 (head size %d, %d tokens a request)", HD, max_q_len);
         p.qkv = (const bf16_t*)fused->qkv;
         p.q_norm_w = fused->q_norm_w; p.k_norm_w = fused->k_norm_w;
         p.cos_t = fused->cos_t; p.sin_t = fused->sin_t; p.slots = fused->slots;
         p.norm_eps = fused->eps; p.norm_add_one = fused->add_one;
+        p.row_ld = fused->row_ld; p.q_off = fused->q_off; p.k_off = fused->k_off; p.v_off = fused->v_off; p.rot = fused->rot;
+        p.gate = (const bf16_t*)fused->gate; p.gate_ld = fused->gate_ld; p.gate_per_head = fused->gate_per_head;
         // 16 columns a wave, whatever the number of query heads of a key/value head
-        IA_CHECK(splits == 1 || (splits & (splits - 1)) == 0, "attention_mfma: the decode kernel splits the keys 2^k ways, not %d", splits);
         const int team = decode_team(splits, g), teams = splits / team;
         const int col_blocks = (g + 15) / 16;
         IA_CHECK(teams == 1 || workspace != nullptr, "attention_mfma: the decode kernel needs a workspace for %d blocks a request "
@@ -1754,11 +1796,11 @@ static int attention_launch(void* out, float* workspace, const void* q, const vo
         IA_CHECK(teams == 1 || (fused->counters != nullptr && (long long)n_seqs * nkv * col_blocks <= fused->n_counters),
                  "attention_mfma: the decode kernel needs %lld zeroed counters, got %d", (long long)n_seqs * nkv * col_blocks,
                  fused->counters ? fused->n_counters : 0);
-        IA_CHECK((long long)nkv * teams <= 65535, "attention_mfma: grid too large (nkv*blocks=%d)", nkv * teams);
-        p.part_ml = workspace ? workspace + (size_t)n * nq * teams * HD : nullptr;
-        const dim3 fgrid((unsigned)col_blocks, nkv * teams, n_seqs);
+        p.part_ml = workspace ? workspace + (size_t)n * nq * teams * HDV : nullptr;
+        const dim3 fgrid((unsigned)(col_blocks * teams), nkv, n_seqs);
         const size_t shared = decode_team_bytes(team, g);
-        p.teams_log2 = __builtin_ctz((unsigned)teams);
+        p.teams = teams;
+        p.col_blocks = col_blocks;
         // With d = page / 16 and 2^(s - 1) < d <= 2^s, M = 2^(31 + s) / d rounded up fits 32 bits and exceeds the quotient by less than
         // 2^s / d parts of 2^-(31 + s): q M >> (31 + s) is q / d for every q = pos / 16 below 2^27, hence for every position.
         const uint32_t d16 = (uint32_t)page_size / 16;
@@ -1833,28 +1875,46 @@ extern "C" int ia_attention_mfma(void* out, float* workspace, const void* q, con
 }
 
 // Whether this head size has the fused decode form.
-extern "C" int ia_attention_mfma_has_fused(void) { return HD % 64 == 0 && HDV == HD ? 1 : 0; }
+extern "C" int ia_attention_mfma_has_fused(void) { return HD % 64 == 0 ? 1 : 0; }
 
 // Decode steps, one token a request: the per-head norm of q and k (weights may be null: none), the rotation
-// by each token's angles (cos, sin [n, d / 2], whole heads, halves paired; may be null: none) and the write
-// of the new key and value at `slots` (may be null: nothing is written and the cache is only read) happen
-// inside the attention kernel.  `qkv` [n, (nq + 2 nkv) * d] is the projections' output.
+// by each token's angles (cos, sin [n, rot / 2], the first `rot` features of a head, halves paired; may be null: none) and the
+// write of the new key and value at `slots` (may be null: nothing is written and the cache is only read) happen
+// inside the attention kernel.  `qkv` [n, row_ld] is the projections' output: query heads at q_off of a row, key heads at k_off,
+// value heads at v_off (without `slots` the last two are not used).  `gate` (may be null) points at the first token's gate values,
+// rows gate_ld apart, a value a feature of the joined heads or (gate_per_head) a head: the output is times their sigmoid.
 extern "C" int ia_attention_mfma_decode_fused(void* out, float* workspace, const void* qkv, void* k_cache,
                                               void* v_cache, const int* block_table, const int* cu_tokens,
                                               const int* positions, const int* slots, const float* q_norm_w,
                                               const float* k_norm_w, const float* cos_t, const float* sin_t,
-                                              float eps, int add_one, int n, int seq_begin, int n_seqs,
+                                              float eps, int add_one, int row_ld, int q_off, int k_off, int v_off, int rot,
+                                              const void* gate, int gate_ld, int gate_per_head, int n, int seq_begin, int n_seqs,
                                               int token_begin, int n_tokens, int max_kv_len, int max_pages,
                                               int nq, int nkv, int d, int page_size, int window, float scale,
-                                              int splits, int chunk, int sink, int* counters, int n_counters,
+                                              int splits, int chunk, int sink, int mask_chunk, int* counters, int n_counters,
                                               hipStream_t stream) {
-    IA_CHECK(qkv != nullptr && (q_norm_w == nullptr) == (k_norm_w == nullptr) && (cos_t == nullptr) == (sin_t == nullptr),
-             "attention_mfma_decode_fused: qkv is needed; norm weights and angle tables come in pairs");
+    IA_CHECK(qkv != nullptr && (cos_t == nullptr) == (sin_t == nullptr) && (k_norm_w == nullptr || q_norm_w != nullptr) &&
+             (slots == nullptr || (q_norm_w == nullptr) == (k_norm_w == nullptr)),
+             "attention_mfma_decode_fused: qkv is needed; norm weights (where keys are written) and angle tables come in pairs");
     IA_CHECK((((uintptr_t)qkv | (uintptr_t)q_norm_w | (uintptr_t)k_norm_w | (uintptr_t)cos_t | (uintptr_t)sin_t) & 15) == 0,
              "attention_mfma_decode_fused: arrays must be 16-byte aligned");
     IA_CHECK(n_seqs == n_tokens, "attention_mfma_decode_fused: one token a request (%d requests, %d tokens)", n_seqs, n_tokens);
-    const FusedArgs fused = {qkv, q_norm_w, k_norm_w, cos_t, sin_t, slots, eps, add_one, counters, n_counters};
+    IA_CHECK(rot >= 0 && rot <= HD && rot % 8 == 0 && (cos_t == nullptr || rot > 0), "attention_mfma_decode_fused: rotation of %d features of "
+             "%d (steps of 8)", rot, HD);
+    IA_CHECK(row_ld % 4 == 0 && q_off % 4 == 0 && q_off >= 0 && nkv > 0 && q_off + (long long)nq * HD <= row_ld,
+             "attention_mfma_decode_fused: %d query heads at %d of rows of %d", nq, q_off, row_ld);
+    if (slots == nullptr) {                                  // (the row of a new key is asked for and not used: any row will do)
+        k_off = q_off; v_off = 0;
+        k_norm_w = q_norm_w;
+    }
+    IA_CHECK(k_off % 4 == 0 && k_off >= 0 && v_off >= 0 && k_off + (long long)nkv * HD <= row_ld &&
+             (slots == nullptr || v_off + (long long)nkv * HDV <= row_ld),
+             "attention_mfma_decode_fused: %d key heads at %d and value heads at %d of rows of %d", nkv, k_off, v_off, row_ld);
+    IA_CHECK(gate == nullptr || (gate_ld >= (gate_per_head ? nq : nq * HDV) && (gate_per_head || (gate_ld % 4 == 0 && ((uintptr_t)gate & 7) == 0))),
+             "attention_mfma_decode_fused: gate values of %d heads in rows %d apart (pieces of four are read at once)", nq, gate_ld);
+    const FusedArgs fused = {qkv, q_norm_w, k_norm_w, cos_t, sin_t, slots, eps, add_one, row_ld, q_off, k_off, v_off, rot,
+                             gate, gate_ld, gate_per_head, counters, n_counters};
     return attention_launch(out, workspace, nullptr, k_cache, v_cache, block_table, cu_tokens, positions, n, seq_begin,
                             n_seqs, token_begin, n_tokens, 1, max_kv_len, max_pages, nq, nkv, d, page_size,
-                            window, scale, splits, chunk, sink, 0, nullptr, 0, 0.f, &fused, stream);
+                            window, scale, splits, chunk, sink, mask_chunk, nullptr, 0, 0.f, &fused, stream);
 }

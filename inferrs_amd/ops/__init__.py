@@ -617,6 +617,27 @@ def decode_split(n_seqs: int, nkv: int, g: int, max_kv_len: int) -> Tuple[int, i
     return splits, -(-chunk // 32) * 32
 
 
+@functools.lru_cache(maxsize=4096)
+def decode_shares(n_seqs: int, nkv: int, g: int, max_kv_len: int) -> Tuple[int, int]:
+    """(splits, keys per split) that a decode step takes: `decode_split`'s, but for three counts beside its powers of two that were
+    faster (us, 8 key/value heads, 16 to 64 query heads): twelve for eight where that still is one round of the chip (9 requests at
+    2,048 keys 17.3 -> 14.9, at 8,192 43.5 -> 36.2); one block of three waves for one of four (24 requests at 1,024 keys 16.2 ->
+    15.3, at 2,048 26.7 -> 24.6); and 48 for 32 at one or two
+    requests of 3,072 to 4,095 keys (11.9 -> 10.6).  Of 480 points longer than 512 keys that these rules decide or leave, none is slower
+    than 0.945 of the former's speed."""
+    splits, chunk = decode_split(n_seqs, nkv, g, max_kv_len)
+    items = n_seqs * nkv * -(-g // 16)
+    if splits == 4 and max_kv_len > 512:
+        splits = 3
+    elif splits == 8 and items * 12 <= DECODE_WAVES and max_kv_len >= 12 * DECODE_MIN_CHUNK:
+        splits = 12
+    elif splits == 32 and items <= 16 and 48 * DECODE_MIN_CHUNK <= max_kv_len < 4096:
+        splits = 48
+    else:
+        return splits, chunk
+    return splits, -(-(-(-max_kv_len // splits)) // 32) * 32
+
+
 def attention_mfma(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
                    cu_tokens: torch.Tensor, block_table: torch.Tensor, *, max_q_len: int, max_kv_len: int,
                    window: Optional[int], scale: float, splits: Optional[int] = None,
@@ -696,12 +717,19 @@ def _decode_counters(device: torch.device, needed: int) -> Optional[torch.Tensor
     return have
 
 
+@functools.lru_cache(maxsize=4096)
+def _decode_sizes(target: str, n: int, nq: int, nkv: int, splits: int) -> Tuple[int, int]:
+    """(floats of workspace, counters) of a decode step."""
+    lib = _raw_library(target)
+    return lib.ia_attention_decode_workspace(n, nq, nkv, splits), lib.ia_attention_decode_counters(n, nq, nkv, splits)
+
+
 def attention_decode_fused_fits(dtype: torch.dtype, d: int, page_size: int, rot: int, interleaved: bool,
-                                has_rotation: bool) -> bool:
-    """Whether decode steps can take `attention_decode_fused`: what the matrix-core kernel takes, head sizes
-    in steps of 64, and a rotation (if any) of whole heads with halves paired."""
-    return (attention_mfma_fits(dtype, d, page_size) and d % 64 == 0
-            and (not has_rotation or (rot == d and not interleaved)))
+                                has_rotation: bool, dv: Optional[int] = None) -> bool:
+    """Whether decode steps can take `attention_decode_fused`: what the matrix-core kernel takes, keys' widths
+    in steps of 64, and a rotation (if any) of the first features of a head in steps of 8, halves paired."""
+    return (attention_mfma_fits(dtype, d, page_size, dv) and d % 64 == 0
+            and (not has_rotation or (rot % 8 == 0 and 0 < rot <= d and not interleaved)))
 
 
 def attention_decode_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
@@ -711,21 +739,37 @@ def attention_decode_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: to
                            cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], max_kv_len: int,
                            window: Optional[int], scale: float, splits: Optional[int] = None,
                            seqs: Optional[Tuple[int, int]] = None, out: Optional[torch.Tensor] = None,
-                           sink: bool = False) -> torch.Tensor:
+                           sink: bool = False, mask_chunk: Optional[int] = None, dv: Optional[int] = None,
+                           offsets: Optional[Tuple[int, Optional[int], Optional[int]]] = None, rot: Optional[int] = None,
+                           gate_off: Optional[int] = None, gate_per_head: bool = False) -> torch.Tensor:
     """Decode steps (one token a request) in one kernel: per-head norm of q and k, rotation, the write
     of the new key and value at `slots` (None: the cache is only read) and the attention over the pages.
-    `qkv` [n, (nq + 2 nkv) * d] is the projections' output; request s owns token s.  Returns [n, nq, d]."""
+    `qkv` [n, (nq + 2 nkv) * d] is the projections' output; request s owns token s.  Returns [n, nq, d].
+    Rows of other layouts: values of width `dv`, `offsets` = where the query, key and value heads begin in a row (the last two
+    are None where nothing is written), `rot` = the first features of a head that rotate, and `gate_off` = where a row's gate values
+    begin (one a feature of the joined heads, or `gate_per_head`): the output is times their sigmoid."""
     _dev(qkv, k_cache, v_cache, positions, cu_tokens, block_table, slots, q_norm_w, k_norm_w, cos, sin, out)
     _i32(positions, "positions"); _i32(cu_tokens, "cu_tokens"); _i32(block_table, "block_table")
     _f32(q_norm_w, "q_norm weight"); _f32(k_norm_w, "k_norm weight"); _f32(cos, "cos"); _f32(sin, "sin")
     n = qkv.shape[0]
     page_size = k_cache.shape[2]
-    _check_cache(k_cache, v_cache, nkv, page_size, d, qkv.dtype, "attention_decode_fused")
-    if not attention_decode_fused_fits(qkv.dtype, d, page_size, d, False, cos is not None):
+    dv, rot = d if dv is None else dv, d if rot is None else rot
+    _check_cache(k_cache, v_cache, nkv, page_size, d, qkv.dtype, "attention_decode_fused", dv)
+    if not attention_decode_fused_fits(qkv.dtype, d, page_size, rot, False, cos is not None, dv):
         raise KernelError(f"attention_decode_fused: takes bfloat16, head sizes in steps of 64 and page sizes in "
                           f"steps of 16; got {qkv.dtype}, head size {d}, page size {page_size}")
-    if qkv.dim() != 2 or qkv.shape[1] != (nq + 2 * nkv) * d or nq % nkv:
-        raise KernelError(f"attention_decode_fused: qkv has shape {tuple(qkv.shape)}, expected [n, {(nq + 2 * nkv) * d}]")
+    if offsets is None:
+        offsets = (0, nq * d, (nq + nkv) * d)
+        if qkv.dim() != 2 or qkv.shape[1] != (nq + nkv) * d + nkv * dv or nq % nkv:
+            raise KernelError(f"attention_decode_fused: qkv has shape {tuple(qkv.shape)}, expected [n, {(nq + nkv) * d + nkv * dv}]")
+    ld_ = qkv.shape[-1]
+    q_off, k_off, v_off = offsets
+    if (qkv.dim() != 2 or nq % nkv or ld_ % 4 or q_off % 4 or q_off < 0 or q_off + nq * d > ld_
+            or (slots is not None and (k_off is None or v_off is None or k_off % 4 or k_off < 0 or k_off + nkv * d > ld_
+                                       or v_off < 0 or v_off + nkv * dv > ld_))):
+        raise KernelError(f"attention_decode_fused: heads at {offsets} of rows {tuple(qkv.shape)}")
+    if gate_off is not None and (gate_off < 0 or gate_off + nq * (1 if gate_per_head else dv) > ld_ or (not gate_per_head and gate_off % 4)):
+        raise KernelError(f"attention_decode_fused: gate values at {gate_off} of rows {tuple(qkv.shape)}")
     all_seqs = cu_tokens.numel() - 1
     seq_begin, n_seqs = seqs if seqs is not None else (0, all_seqs)
     if (positions.numel() != n or block_table.dim() != 2 or block_table.shape[0] < all_seqs or seq_begin < 0
@@ -736,35 +780,34 @@ def attention_decode_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: to
     for w, name in ((q_norm_w, "q_norm"), (k_norm_w, "k_norm")):
         if w is not None and w.numel() != d:
             raise KernelError(f"attention_decode_fused: {name} weight has {w.numel()} entries, head_dim is {d}")
-    if (q_norm_w is None) != (k_norm_w is None) or (cos is None) != (sin is None):
+    if (slots is not None and (q_norm_w is None) != (k_norm_w is None)) or (cos is None) != (sin is None):
         raise KernelError("attention_decode_fused: norm weights and angle tables come in pairs")
-    if cos is not None and (cos.shape != (n, d // 2) or sin.shape != cos.shape):
-        raise KernelError(f"attention_decode_fused: rotary tables must be [{n}, {d // 2}]")
+    if cos is not None and (cos.shape != (n, rot // 2) or sin.shape != cos.shape):
+        raise KernelError(f"attention_decode_fused: rotary tables must be [{n}, {rot // 2}]")
     if slots is not None:
         _i32(slots, "slots")
         if slots.numel() != n:
             raise KernelError(f"attention_decode_fused: {slots.numel()} slots for {n} tokens")
     if out is None:
-        out = torch.empty((n, nq, d), dtype=qkv.dtype, device=qkv.device)
-    elif tuple(out.shape) != (n, nq, d) or out.dtype != qkv.dtype:
-        raise KernelError("attention_decode_fused: `out` must be [n, nq, d] in the dtype of qkv")
+        out = torch.empty((n, nq, dv), dtype=qkv.dtype, device=qkv.device)
+    elif tuple(out.shape) != (n, nq, dv) or out.dtype != qkv.dtype:
+        raise KernelError("attention_decode_fused: `out` must be [n, nq, the values' width] in the dtype of qkv")
     if splits is None:
-        splits, chunk = decode_split(n_seqs, nkv, nq // nkv, max_kv_len)
+        splits, chunk = decode_shares(n_seqs, nkv, nq // nkv, max_kv_len)
     else:
         chunk = -(-(-(-max_kv_len // splits)) // 32) * 32
-    if splits & (splits - 1):
-        raise KernelError(f"attention_decode_fused: the keys are split 2^k ways, not {splits}")
-    target = _build.attn_target(d)
+    target = _build.attn_target(d, dv)
     lib = library(target)
-    ws_floats = lib.ia_attention_decode_workspace(n, nq, nkv, splits)
+    ws_floats, n_counters = _decode_sizes(target, n, nq, nkv, splits)
     ws = torch.empty((ws_floats,), dtype=torch.float32, device=qkv.device) if ws_floats else None
-    counters = _decode_counters(qkv.device, lib.ia_attention_decode_counters(n, nq, nkv, splits))
+    counters = _decode_counters(qkv.device, n_counters)
     _check(lib.ia_attention_mfma_decode_fused(
         _p(out), _p(ws), _p(qkv), _p(k_cache), _p(v_cache), _p(block_table), _p(cu_tokens), _p(positions), _p(slots),
-        _p(q_norm_w), _p(k_norm_w), _p(cos), _p(sin), ctypes.c_float(eps), int(add_one), n, seq_begin, n_seqs,
-        seq_begin, n_seqs, max_kv_len, block_table.shape[1], nq, nkv, d, page_size, int(window or 0),
-        ctypes.c_float(scale), splits, chunk, int(bool(sink)), _p(counters), counters.numel() if counters is not None else 0,
-        _stream()), target)
+        _p(q_norm_w), _p(k_norm_w), _p(cos), _p(sin), eps, int(add_one), ld_, q_off, k_off or 0, v_off or 0,
+        rot if cos is not None else 0, _p(qkv) + 2 * gate_off if gate_off is not None else None, ld_, int(gate_per_head), n, seq_begin,
+        n_seqs, seq_begin, n_seqs, max_kv_len, block_table.shape[1], nq, nkv, d, page_size, int(window or 0),
+        scale, splits, chunk, int(bool(sink)), int(mask_chunk or 0), _p(counters),
+        counters.numel() if counters is not None else 0, _stream()), target)
     return out
 
 

@@ -187,6 +187,17 @@ class Attention(Mixer):
         table = ctx.position_table(self.position)
         cos, sin = table if table is not None else (None, None)
         writes = cache.writable and s.own_kv
+        if (ctx.max_q_len == 1 and s.v_mix is None and not s.keep_first and s.softcap is None
+                and ops.attention_decode_fused_fits(proj.dtype, d, group.page_size, self.position.rot_dim, self.position.interleaved,
+                                                    cos is not None, dv)):
+            # decode steps: norm, rotation, cache write, attention and gate in one kernel
+            a = ops.attention_decode_fused(
+                proj, cache.k, cache.v, ctx.positions, ctx.cu_tokens, group.block_table, nq=H, nkv=G, d=d, dv=dv,
+                offsets=(self.q_off, self.k_off, self.v_off), slots=group.slots if writes else None, q_norm_w=self.q_norm_w,
+                k_norm_w=self.k_norm_w, eps=self.norm_eps, add_one=self.norm_add_one, cos=cos, sin=sin, rot=self.position.rot_dim,
+                max_kv_len=ctx.max_kv_len, window=s.window, scale=s.softmax_scale, sink=s.sink, mask_chunk=s.mask_chunk,
+                gate_off=self.g_off, gate_per_head=bool(s.gate and s.gate_per_head))
+            return self._project(ctx, a.view(a.shape[0], H * dv))
         v_with = None
         if s.v_mix is not None:
             values = proj[:, self.v_off:self.v_off + G * dv]
@@ -201,38 +212,40 @@ class Attention(Mixer):
             q_norm_w=self.q_norm_w, k_norm_w=self.k_norm_w, eps=self.norm_eps, add_one=self.norm_add_one, cos=cos, sin=sin,
             rot=self.position.rot_dim, interleaved=self.position.interleaved, k_cache=cache.k, v_cache=cache.v,
             slots=group.slots if writes else None, page_size=group.page_size, v_with=v_with, v_mix=self.v_mix)
-        a = self._attend(ctx, q, cache, group)
+        a = self.attend(s, ctx, q, cache, group)
         joined = a.view(a.shape[0], H * dv)
         if s.gate:
             ops.sigmoid_gate(joined, proj, self.g_off, group=dv if s.gate_per_head else 1)
         return self._project(ctx, joined)
 
-    def _attend(self, ctx, q, cache, group):
-        return self.attend(self.spec, ctx, q, cache, group)
-
     @staticmethod
     def attend(s: AttentionSpec, ctx, q, cache, group):
         """The paged attention of the step's queries: the matrix cores where they take the sizes, else the plain kernel."""
-        if ops.attention_mfma_fits(q.dtype, s.head_dim, group.page_size, s.value_dim):
-            common = dict(window=s.window, scale=s.softmax_scale, sink=s.sink, mask_chunk=s.mask_chunk,
-                          keep_first=s.keep_first, softcap=s.softcap)
-            if 0 < ctx.n_single < ctx.n_seqs:
-                # single tokens (decode) and portions of prompts want different launches: the first
-                # split their long key ranges between waves, the second have columns enough
-                a = ops.attention_mfma(q, cache.k, cache.v, ctx.positions, ctx.cu_tokens, group.block_table,
-                                       max_q_len=1, max_kv_len=ctx.max_kv_single, seqs=(0, ctx.n_single),
-                                       tokens=(0, ctx.n_single), **common)
-                ops.attention_mfma(q, cache.k, cache.v, ctx.positions, ctx.cu_tokens, group.block_table,
-                                   max_q_len=ctx.max_q_len, max_kv_len=ctx.max_kv_multi,
-                                   seqs=(ctx.n_single, ctx.n_seqs - ctx.n_single),
-                                   tokens=(ctx.n_single, ctx.n_tokens - ctx.n_single), out=a, **common)
-                return a
-            return ops.attention_mfma(q, cache.k, cache.v, ctx.positions, ctx.cu_tokens, group.block_table,
-                                      max_q_len=ctx.max_q_len, max_kv_len=ctx.max_kv_len, **common)
-        return ops.attention_generic(q, cache.k, cache.v, ctx.positions, ctx.token_seq, group.block_table,
-                                     window=s.window, scale=s.softmax_scale, max_kv_len=ctx.max_kv_len, sink=s.sink,
-                                     mask_chunk=s.mask_chunk, keep_first=s.keep_first, softcap=s.softcap,
-                                     portions=Attention.portions_pay(s, ctx, q))
+        if not ops.attention_mfma_fits(q.dtype, s.head_dim, group.page_size, s.value_dim):
+            return ops.attention_generic(q, cache.k, cache.v, ctx.positions, ctx.token_seq, group.block_table,
+                                         window=s.window, scale=s.softmax_scale, max_kv_len=ctx.max_kv_len, sink=s.sink,
+                                         mask_chunk=s.mask_chunk, keep_first=s.keep_first, softcap=s.softcap,
+                                         portions=Attention.portions_pay(s, ctx, q))
+        # Single tokens (decode) and portions of prompts want different launches: the first split their long key ranges between
+        # waves, the second have columns enough.
+        n, singles = q.shape[0], ctx.n_single
+        of = (cache.k, cache.v, ctx.positions, ctx.cu_tokens, group.block_table)
+        common = dict(window=s.window, scale=s.softmax_scale, sink=s.sink, mask_chunk=s.mask_chunk)
+        special = dict(keep_first=s.keep_first, softcap=s.softcap)
+        a = None
+        if singles > 0:
+            max_kv = ctx.max_kv_single if singles < ctx.n_seqs else ctx.max_kv_len
+            if not s.keep_first and s.softcap is None and ops.attention_decode_fused_fits(
+                    q.dtype, s.head_dim, group.page_size, 0, False, False, s.value_dim):
+                a = ops.attention_decode_fused(q.view(n, -1), *of, nq=q.shape[1], nkv=cache.k.shape[1], d=s.head_dim,
+                                               dv=s.value_dim, offsets=(0, None, None), slots=None, q_norm_w=None, k_norm_w=None,
+                                               eps=0.0, add_one=False, cos=None, sin=None, max_kv_len=max_kv, seqs=(0, singles), **common)
+            else:
+                a = ops.attention_mfma(q, *of, max_q_len=1, max_kv_len=max_kv, seqs=(0, singles), tokens=(0, singles), **common, **special)
+        if singles < ctx.n_seqs:
+            a = ops.attention_mfma(q, *of, max_q_len=ctx.max_q_len, max_kv_len=ctx.max_kv_multi if singles else ctx.max_kv_len,
+                                   seqs=(singles, ctx.n_seqs - singles), tokens=(singles, ctx.n_tokens - singles), out=a, **common, **special)
+        return a
 
     @staticmethod
     def portions_pay(s: AttentionSpec, ctx, q) -> bool:
@@ -259,7 +272,7 @@ class Attention(Mixer):
         s = self.spec
         return [f"attention with head size {s.head_dim}, page size {page_size}, rotation of {self.position.rot_dim} features "
                 f"({'interleaved' if self.position.interleaved else 'halves'}): decode steps do not take the fused kernel "
-                "(head sizes in steps of 64, page sizes in steps of 16, whole heads rotated in halves); norm and "
+                "(head sizes in steps of 64, page sizes in steps of 16, rotations in halves and steps of 8 features); norm and "
                 "rotation, the cache write and the attention run as kernels of their own"]
 
     def _project(self, ctx, a: torch.Tensor):
@@ -297,7 +310,8 @@ class Attention(Mixer):
                 qkv, cache.k, cache.v, ctx.positions, ctx.cu_tokens, group.block_table, nq=s.n_heads,
                 nkv=s.n_kv_heads, d=s.head_dim, slots=group.slots if cache.writable else None,
                 q_norm_w=self.q_norm_w, k_norm_w=self.k_norm_w, eps=self.norm_eps, add_one=self.norm_add_one,
-                cos=cos, sin=sin, max_kv_len=ctx.max_kv_len, window=s.window, scale=s.softmax_scale, sink=s.sink)
+                cos=cos, sin=sin, rot=self.position.rot_dim, max_kv_len=ctx.max_kv_len, window=s.window, scale=s.softmax_scale,
+                sink=s.sink)
             return self._project(ctx, a.view(a.shape[0], s.n_heads * s.head_dim))
         q = ops.qk_rope_kv(
             qkv, s.n_heads, s.n_kv_heads, s.head_dim,
@@ -305,23 +319,5 @@ class Attention(Mixer):
             cos=cos, sin=sin, rot=self.position.rot_dim, interleaved=self.position.interleaved,
             k_cache=cache.k, v_cache=cache.v, slots=group.slots if cache.writable else None,
             page_size=group.page_size)
-        if ops.attention_mfma_fits(q.dtype, s.head_dim, group.page_size):
-            common = dict(window=s.window, scale=s.softmax_scale, sink=s.sink)
-            if 0 < ctx.n_single < ctx.n_seqs:
-                # single tokens (decode) and portions of prompts want different launches: the first
-                # split their long key ranges between waves, the second have columns enough
-                a = ops.attention_mfma(q, cache.k, cache.v, ctx.positions, ctx.cu_tokens, group.block_table,
-                                       max_q_len=1, max_kv_len=ctx.max_kv_single, seqs=(0, ctx.n_single),
-                                       tokens=(0, ctx.n_single), **common)
-                ops.attention_mfma(q, cache.k, cache.v, ctx.positions, ctx.cu_tokens, group.block_table,
-                                   max_q_len=ctx.max_q_len, max_kv_len=ctx.max_kv_multi,
-                                   seqs=(ctx.n_single, ctx.n_seqs - ctx.n_single),
-                                   tokens=(ctx.n_single, ctx.n_tokens - ctx.n_single), out=a, **common)
-            else:
-                a = ops.attention_mfma(q, cache.k, cache.v, ctx.positions, ctx.cu_tokens, group.block_table,
-                                       max_q_len=ctx.max_q_len, max_kv_len=ctx.max_kv_len, **common)
-        else:
-            a = ops.attention_generic(q, cache.k, cache.v, ctx.positions, ctx.token_seq, group.block_table,
-                                      window=s.window, scale=s.softmax_scale, max_kv_len=ctx.max_kv_len, sink=s.sink,
-                                      portions=self.portions_pay(s, ctx, q))
+        a = self.attend(s, ctx, q, cache, group)
         return self._project(ctx, a.view(a.shape[0], s.n_heads * s.head_dim))

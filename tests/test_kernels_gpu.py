@@ -872,6 +872,65 @@ def test_attention_decode_fused_is_the_three_kernels_in_one(nq, nkv, d, page, wi
         assert counters is None or int(counters.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("nq,nkv,d,dv_,page,window,mask_chunk,rot,gate,own", [
+    (16, 4, 128, 64, 16, 40, None, 64, "feature", True),       # values narrower than keys, half of a head rotating
+    (16, 4, 128, 64, 16, 300, None, 64, "feature", False),     # a layer that reads another's cache: rows [q | g]
+    (6, 2, 64, 16, 32, None, None, 24, "head", True), (5, 1, 64, 256, 16, None, 100, 8, None, True),
+    (17, 1, 128, 128, 48, 95, None, 120, "head", True), (4, 2, 192, 192, 16, None, None, 0, "feature", True),
+    (3, 3, 256, 256, 16, None, 33, 256, "head", False), (2, 2, 128, 64, 16, None, None, 128, None, True)])
+def test_attention_decode_takes_rows_of_any_layout(nq, nkv, d, dv_, page, window, mask_chunk, rot, gate, own):
+    """Values of another width than keys, part of a head rotating, rows with a gate in them or without keys, chunks for a mask:
+    against the kernels of norm and rotation, attention and gate one after the other.  The gate's kernel rounds the joined heads
+    before it multiplies them, hence a bound of two roundings to bfloat16 of the largest value."""
+    from inferrs_amd import ops
+    dtype = torch.bfloat16
+    lens = [300, 17, 1000, 33, 64, 1]
+    q, kc, vc, positions, token_seq, table = attention_case(dtype, nq, nkv, d, page, lens, [1] * len(lens), 29)
+    vc = randn(kc.shape[0], nkv, dv_, page, dtype=dtype, seed=9)
+    n, at = len(lens), nq * d
+    offsets = (0, at, at + nkv * d) if own else (0, None, None)
+    at += nkv * (d + dv_) if own else 0
+    g_off = at if gate else None
+    width = at + (0 if gate is None else nq * (dv_ if gate == "feature" else 1))
+    width += -width % 8
+    proj = dev(randn(n, width, dtype=dtype, seed=5))
+    qw, kw = (dev(1 + 0.3 * randn(d, dtype=torch.float32, seed=s)) for s in (6, 7))
+    cos = sin = None
+    if rot:
+        ang = positions.float()[:, None] * (1.0 / (10000.0 ** (torch.arange(0, rot, 2, dtype=torch.float32) / rot)))[None, :]
+        cos, sin = dev(torch.cos(ang)), dev(torch.sin(ang))
+    slots = dev(torch.tensor([int(table[s, (l - 1) // page]) * page + (l - 1) % page for s, l in enumerate(lens)], dtype=torch.int32))
+    cu, scale = dev(torch.arange(n + 1, dtype=torch.int32)), 1.0 / math.sqrt(d)
+    positions, table = dev(positions), dev(table)
+    k1, v1 = dev(kc), dev(vc)
+    q1 = ops.qk_rope_kv_strided(proj, nq, nkv, d, dv_, q_off=0, k_off=offsets[1], v_off=offsets[2], q_norm_w=qw, k_norm_w=kw if own else None,
+                                eps=1e-5, add_one=False, cos=cos, sin=sin, rot=rot, interleaved=False, k_cache=k1, v_cache=v1,
+                                slots=slots if own else None, page_size=page)
+    for splits in (None, 1, 4, 32):
+        want = ops.attention_mfma(q1, k1, v1, positions, cu, table, max_q_len=1, max_kv_len=max(lens), window=window, scale=scale,
+                                  splits=splits, mask_chunk=mask_chunk).view(n, nq * dv_)
+        if gate:
+            ops.sigmoid_gate(want, proj, g_off, group=1 if gate == "feature" else dv_)
+        k2, v2 = dev(kc), dev(vc)
+        got = ops.attention_decode_fused(proj, k2, v2, positions, cu, table, nq=nq, nkv=nkv, d=d, dv=dv_, offsets=offsets, rot=rot,
+                                         slots=slots if own else None, q_norm_w=qw, k_norm_w=kw if own else None, eps=1e-5, add_one=False,
+                                         cos=cos, sin=sin, max_kv_len=max(lens), window=window, scale=scale, splits=splits,
+                                         mask_chunk=mask_chunk, gate_off=g_off, gate_per_head=gate == "head")
+        close(got.view(n, -1).float().cpu(), want.float().cpu(), 2 ** -7, f"rows of any layout, splits={splits}")
+        assert torch.equal(v2, v1)
+        dk = (k2.float() - k1.float()).abs()
+        assert float(dk.max()) <= 2 ** -7 * float(k1.float().abs().max()) and float((dk > 0).float().mean()) < 1e-3
+        # queries that are formed already, a run of the step's tokens
+        some = ops.attention_decode_fused(q1.view(n, -1), k1, v1, positions, cu, table, nq=nq, nkv=nkv, d=d, dv=dv_, offsets=(0, None, None),
+                                          slots=None, q_norm_w=None, k_norm_w=None, eps=0.0, add_one=False, cos=None, sin=None,
+                                          max_kv_len=max(lens[:3]), seqs=(0, 3), window=window, scale=scale, mask_chunk=mask_chunk)
+        want = ops.attention_mfma(q1, k1, v1, positions, cu, table, max_q_len=1, max_kv_len=max(lens), window=window, scale=scale,
+                                  mask_chunk=mask_chunk)
+        close(some[:3].float().cpu(), want[:3].float().cpu(), 2 ** -7, "formed queries")
+        counters = ops._DECODE_COUNTERS.get(torch.cuda.current_device())
+        assert counters is None or int(counters.abs().sum()) == 0
+
+
 @pytest.mark.parametrize("nq,nkv,d,page,window", [
     (3, 1, 128, 16, None), (8, 2, 128, 112, 40), (7, 1, 128, 16, None), (8, 1, 128, 32, 95),    # the new key in the first pass over
     (16, 1, 128, 16, None), (17, 1, 64, 48, None), (5, 1, 192, 16, 33), (2, 1, 256, 80, None)])  # the rows, the second, a third, a last of its own

@@ -182,3 +182,18 @@ def test_rows_of_the_mid_products_are_grouped_within_one_round_of_the_chip(rows,
                                         (3072, 1024, 2), (2560, 9728, 4), (1024, 3072, 4), (5120, 1536, 2), (3200, 3328, 2)])
 def test_plans_of_small_weights_split_k_as_often_as_two_stages_would(n, k, splits):
     assert ops.library().ia_gemm_mid_splits(n, k) == splits
+
+
+@pytest.mark.parametrize("g", [1, 2, 5, 8, 16, 20])
+def test_decode_shares_are_whole_blocks_that_cover_the_context(g):
+    """What a decode step takes in place of `decode_split`'s counts: as many waves as one round of the chip holds, blocks of equally
+    many waves (up to four, so that more than four shares come in fours), shares of two steps of 32 keys or more."""
+    others = set()
+    for n_seqs, nkv, kv in itertools.product(range(1, 65), (1, 2, 4, 8), (31, 512, 513, 1024, 2048, 3072, 4095, 4096, 8192, 40960)):
+        base, (splits, chunk) = ops.decode_split(n_seqs, nkv, g, kv), ops.decode_shares(n_seqs, nkv, g, kv)
+        assert chunk % 32 == 0 and splits * chunk >= kv and 1 <= splits <= 128
+        assert splits <= 4 or splits % 4 == 0
+        if (splits, chunk) != base:
+            others.add(splits)
+            assert chunk >= 64 and n_seqs * nkv * -(-g // 16) * splits <= ops.DECODE_WAVES
+    assert others == {3, 12, 48}
