@@ -72,17 +72,34 @@ __host__ __device__ __forceinline__ int ia_key_floor(int pos, int window, int ma
 
 // ---- reductions -----------------------------------------------------------------------------
 // Butterfly over the 64 lanes: every lane ends with the same value, and the order of the
-// additions is fixed by the lane numbers alone.
+// additions is fixed by the lane numbers alone: lanes 32 apart, then 16, 8, 4, 2, 1.  The lanes
+// exchange through the vector units (swaps of halves and of rows of 16, turns inside a row; behind
+// the step of 8 lanes a turn by 4 brings what the lane 4 apart holds), six steps of about ten
+// cycles where six trips through shared memory took about a hundred each.  All lanes of the wave
+// take part.
+template <int CTRL>
+__device__ __forceinline__ float wave_lane(float v) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+
+template <typename OP>
+__device__ __forceinline__ float wave_all(float v, OP op) {
+    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    v = op(v, wave_lane<0x128>(v));                 // turned by 8
+    v = op(v, wave_lane<0x124>(v));                 // turned by 4
+    v = op(v, wave_lane<0x4e>(v));                  // lane ^ 2
+    return op(v, wave_lane<0xb1>(v));               // lane ^ 1
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = IA_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, IA_WAVE);
-    return v;
+    return wave_all(v, [](float x, float y) { return x + y; });
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = IA_WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, IA_WAVE));
-    return v;
+    return wave_all(v, [](float x, float y) { return fmaxf(x, y); });
 }
 
 // Sum over a block of up to 1024 threads; `scratch` holds 16 floats of shared memory.
@@ -94,8 +111,12 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
     __syncthreads();
     if (lane == 0) scratch[wave] = v;
     __syncthreads();
-    float total = 0.f;
-    for (int w = 0; w < nwaves; ++w) total += scratch[w];
+    // (all sixteen are asked for together, whatever lies behind the last wave's)
+    float part[16], total = 0.f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) part[w] = scratch[w];
+#pragma unroll
+    for (int w = 0; w < 16; ++w) total += w < nwaves ? part[w] : 0.f;
     return total;
 }
 
