@@ -240,7 +240,8 @@ int ia_route(int* sel, float* weight, const void* h, const void* router, int n, 
 // 16 tokens in one block, with the plan
 int ia_route_logits(int* sel, float* weight, const float* logits, long long ld, int off, int n, int E, int top, float scale,
                     int score_fn, int renorm, const float* choice_bias, int gates, float* gate_out, int group_count, int group_keep,
-                    int* order, int* tile_expert, int* tile_first, int* tile_rows, int* meta, int plan_E, int tile, hipStream_t stream);
+                    int* order, int* tile_expert, int* tile_first, int* tile_rows, int* meta, int plan_E, int tile,
+                    void* act, int inter, float limit, float alpha, hipStream_t stream);
 int ia_route_plans(int n, int W, int rows, int dtype, const void* h, const void* router);    // 1: ia_route makes this step's plan itself
 int ia_route_tiles(int pairs, int E);
 int ia_route_plan(int* order, int* tile_expert, int* tile_first, int* tile_rows, int* meta, const int* sel,

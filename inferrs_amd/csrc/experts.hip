@@ -34,6 +34,26 @@ __device__ __forceinline__ void load8(const bf16_t* p, float (&v)[8]) {
     }
 }
 
+// The largest of a wave's keys and its place: of equal ones the lowest, `key[q]` of lane l being place 64 q + l; place 0x7fffffff where
+// no key is above minus infinity.  One maximum over the wave and a vote, where exchanging pairs of a key and a place took two or
+// three trips through shared memory a step.
+template <int Q>
+__device__ __forceinline__ float wave_best(const float (&key)[Q], int& place) {
+    float best = -INFINITY;
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+        if (key[q] > best) best = key[q];
+    best = wave_max(best);
+    place = 0x7fffffff;
+#pragma unroll
+    for (int q = Q - 1; q >= 0; --q) {
+        const unsigned long long at = __ballot(key[q] == best);
+        if (at != 0ull) place = q * IA_WAVE + __builtin_ctzll(at);
+    }
+    if (__builtin_amdgcn_readfirstlane(__float_as_uint(best)) == 0xff800000u) place = 0x7fffffff;
+    return best;
+}
+
 // One wave: a token's choice and weights from its logits (of E rows of the router's matrix, the last `gates` of which take no
 // part in it).  Q: registers of logits a lane (E - gates up to 64 Q).
 template <int Q>
@@ -81,18 +101,11 @@ __device__ __forceinline__ void route_pick(int* __restrict__ sel, float* __restr
         }
         int in = 0;         // bit q: the group in register q stays
         for (int k = 0; k < group_keep; ++k) {
-            float best = -INFINITY;
-            int best_g = 0x7fffffff;
+            int best_g;
+            wave_best<Q>(worth, best_g);
 #pragma unroll
             for (int q = 0; q < Q; ++q)
-                if (!((in >> q) & 1) && worth[q] > best) { best = worth[q]; best_g = q * IA_WAVE + lane; }
-#pragma unroll
-            for (int o = IA_WAVE / 2; o > 0; o >>= 1) {
-                const float ob = __shfl_xor(best, o, IA_WAVE);
-                const int og = __shfl_xor(best_g, o, IA_WAVE);
-                if (ob > best || (ob == best && og < best_g)) { best = ob; best_g = og; }
-            }
-            if (best_g % IA_WAVE == lane) in |= 1 << (best_g / IA_WAVE);
+                if (best_g == q * IA_WAVE + lane) { in |= 1 << q; worth[q] = -INFINITY; }
         }
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
@@ -114,37 +127,23 @@ __device__ __forceinline__ void route_pick(int* __restrict__ sel, float* __restr
             key[q] = e < E && z[q] > -INFINITY ? sc[q] + choice_bias[e] : -INFINITY;
         }
         for (int k = 0; k < top; ++k) {
-            float best = -INFINITY, best_s = 0.f;
-            int best_e = 0x7fffffff;
+            int best_e;
+            wave_best<Q>(key, best_e);
+            float best_s = 0.f;
 #pragma unroll
-            for (int q = 0; q < Q; ++q)
-                if (key[q] > best) { best = key[q]; best_e = q * IA_WAVE + lane; best_s = sc[q]; }
-#pragma unroll
-            for (int o = IA_WAVE / 2; o > 0; o >>= 1) {
-                const float ob = __shfl_xor(best, o, IA_WAVE), os = __shfl_xor(best_s, o, IA_WAVE);
-                const int oe = __shfl_xor(best_e, o, IA_WAVE);
-                if (ob > best || (ob == best && oe < best_e)) { best = ob; best_e = oe; best_s = os; }
-            }
-#pragma unroll
-            for (int q = 0; q < Q; ++q)
+            for (int q = 0; q < Q; ++q) {
+                const float of = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sc[q]), best_e & (IA_WAVE - 1)));
+                if (best_e / IA_WAVE == q) best_s = of;
                 if (best_e == q * IA_WAVE + lane) key[q] = -INFINITY;
+            }
             total += best_s;
             if (lane == k) { mine = best_s; mine_e = best_e; }
         }
     } else
     for (int k = 0; k < top; ++k) {
-        // every lane's best, then the wave's: the largest logit, of equal ones the lower index
-        float best = -INFINITY;
-        int best_e = 0x7fffffff;
-#pragma unroll
-        for (int q = 0; q < Q; ++q)
-            if (z[q] > best) { best = z[q]; best_e = q * IA_WAVE + lane; }
-#pragma unroll
-        for (int o = IA_WAVE / 2; o > 0; o >>= 1) {
-            const float ob = __shfl_xor(best, o, IA_WAVE);
-            const int oe = __shfl_xor(best_e, o, IA_WAVE);
-            if (ob > best || (ob == best && oe < best_e)) { best = ob; best_e = oe; }
-        }
+        // the largest logit, of equal ones the lower index
+        int best_e;
+        const float best = wave_best<Q>(z, best_e);
 #pragma unroll
         for (int q = 0; q < Q; ++q)
             if (best_e == q * IA_WAVE + lane) z[q] = -INFINITY;
@@ -220,6 +219,18 @@ __global__ __launch_bounds__(64 * WAVES) void route_kernel(int* __restrict__ sel
     route_pick<IA_MAX_EXPERTS / IA_WAVE>(sel, weight, logits, t, lane, E, top, scale, score_fn, renorm, choice_bias, gates, gate_out, group_count, group_keep);
 }
 
+// The sum over a wave's lanes up to this one: inside rows of 16 by shifts, then a row's total to the row behind it and the first
+// half's to the second.
+__device__ __forceinline__ int wave_running_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
 // The whole block.  `order` [pairs]: the pairs grouped by expert; tiles: expert, first place in `order`, rows; meta[0]: tiles.
 // sel may lie in shared memory.
 struct RoutePlan {
@@ -241,15 +252,10 @@ __device__ __forceinline__ void route_plan_block(const RoutePlan& p, const int* 
         for (int e0 = 0; e0 < E; e0 += IA_WAVE) {
             const int e = e0 + (int)threadIdx.x;
             const int mine = e < E ? count[e] : 0, mine_t = (mine + tile - 1) / tile;
-            int sum = mine, sum_t = mine_t;
-#pragma unroll
-            for (int o = 1; o < IA_WAVE; o <<= 1) {
-                const int u = __shfl_up(sum, o, IA_WAVE), v = __shfl_up(sum_t, o, IA_WAVE);
-                if ((int)threadIdx.x >= o) { sum += u; sum_t += v; }
-            }
+            const int sum = wave_running_sum(mine), sum_t = wave_running_sum(mine_t);
             if (e < E) { first[e] = at + sum - mine; tile0[e] = tiles + sum_t - mine_t; }
-            at += __shfl(sum, IA_WAVE - 1, IA_WAVE);
-            tiles += __shfl(sum_t, IA_WAVE - 1, IA_WAVE);
+            at += __builtin_amdgcn_readlane(sum, IA_WAVE - 1);
+            tiles += __builtin_amdgcn_readlane(sum_t, IA_WAVE - 1);
         }
         if (threadIdx.x == 0) meta[0] = tiles;
     }
@@ -288,6 +294,8 @@ __global__ __launch_bounds__(64 * IA_RM_WAVES) void route_mfma_kernel(int* __res
     extern __shared__ float rm_part[];             // [waves][tokens][16 NT]
     __shared__ float logits[IA_RM_TOKENS][16 * NT];
     __shared__ int chosen[IA_RM_TOKENS * IA_MAX_TOP];
+    __shared__ float bias[16 * NT];                // (here before the logits are: the picking does not wait for it)
+    if (choice_bias != nullptr && (int)threadIdx.x < E - gates) bias[threadIdx.x] = choice_bias[threadIdx.x];
     const int t0 = blockIdx.x * IA_RM_TOKENS, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, G = lane >> 4;
     const bf16_t* row = h + (long long)(t0 + r16 < n ? t0 + r16 : n - 1) * W;
@@ -298,16 +306,29 @@ __global__ __launch_bounds__(64 * IA_RM_WAVES) void route_mfma_kernel(int* __res
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[j] = (tm_f32x4){0.f, 0.f, 0.f, 0.f};
     const int steps = (W + 31) / 32;
-#pragma unroll 4
-    for (int st = wave; st < steps; st += IA_RM_WAVES) {
-        const int c = 32 * st + 8 * G;
-        const bool in = c < W;                     // (widths in steps of 8: a piece lies inside or outside as a whole)
-        const tm_u32x4 zero = {0u, 0u, 0u, 0u};
-        const tm_u32x4 x = in ? *reinterpret_cast<const tm_u32x4*>(row + c) : zero;
+    // (four steps' operands are asked for before any is used, from addresses that are always inside a row: one trip to the memory
+    // for widths up to 2,048, where a branch a step had made it four; 36 outputs of 2,048 features, 8 tokens: 12.2 -> 10.6 us; 13.9
+    // before the picking exchanged through the vector units)
+    for (int st0 = wave; st0 < steps; st0 += 4 * IA_RM_WAVES) {
+        tm_u32x4 x[4], b[4][NT];
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            const tm_u32x4 b = in ? *reinterpret_cast<const tm_u32x4*>(w[j] + c) : zero;
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(tm_bf16x8, x), __builtin_bit_cast(tm_bf16x8, b), acc[j], 0, 0, 0);
+        for (int i = 0; i < 4; ++i) {
+            const int c = 32 * (st0 + i * IA_RM_WAVES) + 8 * G, at = c < W ? c : 0;
+            x[i] = *reinterpret_cast<const tm_u32x4*>(row + at);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) b[i][j] = *reinterpret_cast<const tm_u32x4*>(w[j] + at);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool in = 32 * (st0 + i * IA_RM_WAVES) + 8 * G < W;      // (widths in steps of 8: a piece lies inside or outside as a whole)
+            const tm_u32x4 zero = {0u, 0u, 0u, 0u};
+            const tm_u32x4 xi = in ? x[i] : zero;
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const tm_u32x4 bi = in ? b[i][j] : zero;
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(tm_bf16x8, xi), __builtin_bit_cast(tm_bf16x8, bi), acc[j], 0, 0, 0);
+            }
         }
     }
 #pragma unroll
@@ -323,21 +344,49 @@ __global__ __launch_bounds__(64 * IA_RM_WAVES) void route_mfma_kernel(int* __res
     }
     __syncthreads();
     if (t0 + wave < n)
-        route_pick<1>(sel, weight, logits[wave], t0 + wave, lane, E, top, scale, score_fn, renorm, choice_bias, gates, gate_out, group_count, group_keep,
+        route_pick<1>(sel, weight, logits[wave], t0 + wave, lane, E, top, scale, score_fn, renorm, choice_bias != nullptr ? bias : nullptr, gates, gate_out, group_count, group_keep,
                       chosen + wave * top);
     if (plan.order == nullptr) return;             // (the same for all threads; the grid is one block otherwise)
     __syncthreads();
     route_plan_block(plan, chosen, n * top);
 }
 
+// An expert's activation over its two sums.  Clamped: g' * sigmoid(alpha g') * (u' + 1), g' = min(g, limit), u' = clamp(u,
+// -limit, limit); plain (IA_EXPERT_SILU): silu(g) * u.  The choice is the same for all lanes of a launch.
+enum { IA_EXPERT_CLAMPED = 0, IA_EXPERT_SILU = 1 };
+__device__ __forceinline__ float expert_act(float g, float u, float limit, float alpha, int form) {
+    if (form == IA_EXPERT_SILU) return g / (1.0f + expf(-g)) * u;
+    const float gv = fminf(g, limit), uv = fminf(fmaxf(u, -limit), limit);
+    return gv / (1.0f + expf(-alpha * gv)) * (uv + 1.0f);
+}
+
 // The choice from logits that another product has left in 32-bit rows, for steps of up to 16 tokens: a wave a token, then the
 // plan.  (A router's matrix read by one compute unit takes as long as the unit's share of the memory's rate lets it; as rows
-// of a large product beside it, it is spread over the chip.)
+// of a large product beside it, it is spread over the chip.)  Where that product is a shared expert's [gate; up], its sums stand in
+// front of the logits in the same rows, and the blocks behind the first form the activation from them (`act` [n, inter], unrounded
+// sums in): 36 outputs beside 2 x 3,072 features of 2,048, 8 tokens: 10.6 + 8.1 + 4.6 us by the router's own product, [gate; up] and
+// the activation's kernel, 8.2 + 5.2 so.
+struct RouteGate {
+    bf16_t* act;                                   // null: no activation
+    const float* rows;                             // [n, ld]: gate, up, ..
+    int inter;
+    float limit, alpha;
+};
 __global__ __launch_bounds__(64 * IA_RM_WAVES) void route_logits_kernel(int* __restrict__ sel, float* __restrict__ weight,
                                                                         const float* __restrict__ logits, long long ld, int n, int E,
                                                                         int top, float scale, int score_fn, int renorm,
                                                                         const float* __restrict__ choice_bias, int gates,
-                                                                        float* __restrict__ gate_out, int group_count, int group_keep, const RoutePlan plan) {
+                                                                        float* __restrict__ gate_out, int group_count, int group_keep, const RoutePlan plan,
+                                                                        const RouteGate gu) {
+    if (blockIdx.x > 0) {
+        const int pieces = gu.inter / 4, i = ((int)blockIdx.x - 1) * blockDim.x + threadIdx.x;
+        if (i >= n * pieces) return;
+        const int t = i / pieces, c = (i - t * pieces) * 4;
+        const float4 g = *(const float4*)(gu.rows + t * ld + c), u = *(const float4*)(gu.rows + t * ld + gu.inter + c);
+        auto form = [&](float a, float b) { return expert_act(a, b, gu.limit, gu.alpha, IA_EXPERT_CLAMPED); };
+        *(uint2*)(gu.act + (size_t)t * gu.inter + c) = make_uint2(pack_bf16x2(form(g.x, u.x), form(g.y, u.y)), pack_bf16x2(form(g.z, u.z), form(g.w, u.w)));
+        return;
+    }
     __shared__ int chosen[IA_RM_TOKENS * IA_MAX_TOP];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (wave < n) {
@@ -350,15 +399,6 @@ __global__ __launch_bounds__(64 * IA_RM_WAVES) void route_logits_kernel(int* __r
     }
     __syncthreads();
     route_plan_block(plan, chosen, n * top);
-}
-
-// An expert's activation over its two sums.  Clamped: g' * sigmoid(alpha g') * (u' + 1), g' = min(g, limit), u' = clamp(u,
-// -limit, limit); plain (IA_EXPERT_SILU): silu(g) * u.  The choice is the same for all lanes of a launch.
-enum { IA_EXPERT_CLAMPED = 0, IA_EXPERT_SILU = 1 };
-__device__ __forceinline__ float expert_act(float g, float u, float limit, float alpha, int form) {
-    if (form == IA_EXPERT_SILU) return g / (1.0f + expf(-g)) * u;
-    const float gv = fminf(g, limit), uv = fminf(fmaxf(u, -limit), limit);
-    return gv / (1.0f + expf(-alpha * gv)) * (uv + 1.0f);
 }
 
 // act[place][j] = expert_act(gate_j . x, up_j . x);
@@ -567,7 +607,8 @@ extern "C" int ia_route(int* sel, float* weight, const void* h, const void* rout
 extern "C" int ia_route_logits(int* sel, float* weight, const float* logits, long long ld, int off, int n, int E, int top, float scale,
                                int score_fn, int renorm, const float* choice_bias, int gates, float* gate_out, int group_count,
                                int group_keep, int* order, int* tile_expert, int* tile_first, int* tile_rows, int* meta, int plan_E,
-                               int tile, hipStream_t stream) {
+                               int tile, void* act, int inter, float limit, float alpha, hipStream_t stream) {
+    // act: null, or [n, inter] bfloat16: the clamped activation of the first 2 inter columns of the rows (gate, then up)
     IA_CHECK(route_groups_fit(E, top, group_count, group_keep), "route_logits: %d of %d groups of %d outputs, top %d", group_keep, group_count, E, top);
     IA_CHECK(n >= 0 && n <= IA_RM_TOKENS && E >= 1 && gates >= 0 && E + gates <= IA_MAX_EXPERTS && top >= 1 && top <= E && top <= IA_MAX_TOP &&
              off >= 0 && off + E + gates <= ld && (gates == 0 || gate_out != nullptr) && order != nullptr,
@@ -577,8 +618,12 @@ extern "C" int ia_route_logits(int* sel, float* weight, const float* logits, lon
     RoutePlan plan;
     plan.order = order; plan.tile_expert = tile_expert; plan.tile_first = tile_first; plan.tile_rows = tile_rows; plan.meta = meta;
     plan.E = plan_E; plan.tile = tile;
-    route_logits_kernel<<<1, 64 * IA_RM_WAVES, 0, stream>>>(sel, weight, logits + off, ld, n, E + gates, top, scale, score_fn, renorm,
-                                                            choice_bias, gates, gate_out, group_count, group_keep, plan);
+    IA_CHECK(act == nullptr || (inter > 0 && inter % 4 == 0 && ld % 4 == 0 && 2ll * inter <= ld && limit > 0.f && (((uintptr_t)logits) & 15) == 0 && (((uintptr_t)act) & 7) == 0),
+             "route_logits: an activation of %d features from rows of %lld (steps of 4, aligned)", inter, ld);
+    const RouteGate gu = {(bf16_t*)act, logits, inter, limit, alpha};
+    const long long pieces = act != nullptr ? (long long)n * (inter / 4) : 0;
+    route_logits_kernel<<<(unsigned)(1 + (pieces + 64 * IA_RM_WAVES - 1) / (64 * IA_RM_WAVES)), 64 * IA_RM_WAVES, 0, stream>>>(
+        sel, weight, logits + off, ld, n, E + gates, top, scale, score_fn, renorm, choice_bias, gates, gate_out, group_count, group_keep, plan, gu);
     IA_LAUNCH_CHECK("route_logits");
     return 0;
 }

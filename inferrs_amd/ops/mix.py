@@ -290,10 +290,12 @@ ROUTE_LOGITS_ROWS = 16        # rows of a step whose router's logits may come wi
 
 
 def route_logits(rows: torch.Tensor, off: int, experts: int, top: int, scale: float, score: str, renormalize: bool,
-                 choice_bias: Optional[torch.Tensor], gates: int, plan: ExpertPlan, groups: Optional[Tuple[int, int]] = None):
+                 choice_bias: Optional[torch.Tensor], gates: int, plan: ExpertPlan, groups: Optional[Tuple[int, int]] = None,
+                 gated: Optional[Tuple[int, float, float]] = None):
     """`route` from logits that a product beside the router's matrix has left: 32-bit rows [n, ..] (up to `ROUTE_LOGITS_ROWS`),
     the experts' logits from column `off` on, those of the `gates` behind them.  The plan is made as well.  Returns
-    (experts, weights, gates or None)."""
+    (experts, weights, gates or None).  `gated` (features, limit, slope): the rows begin with the sums of a [gate; up] of so many
+    features, whose clamped activation (`clamped_gate_mul`'s formula on the 32-bit sums) comes back as a fourth result, bfloat16."""
     _dev(rows, choice_bias); _f32(rows, "logits"); _f32(choice_bias, "choice_bias")
     n, ld = rows.shape
     if n > ROUTE_LOGITS_ROWS or off < 0 or off + experts + gates > ld or plan.pairs != n * top or score not in SCORE_FUNCTIONS:
@@ -302,11 +304,15 @@ def route_logits(rows: torch.Tensor, off: int, experts: int, top: int, scale: fl
     sel = torch.empty((n, top), dtype=torch.int32, device=rows.device)
     weight = torch.empty((n, top), dtype=torch.float32, device=rows.device)
     gate_out = torch.empty((n, gates), dtype=torch.float32, device=rows.device) if gates else None
+    inter, limit, slope = gated if gated is not None else (0, 0.0, 0.0)
+    if gated is not None and (not rows.is_contiguous() or inter < 1 or 2 * inter > off):
+        raise KernelError(f"route_logits: an activation of {inter} features in front of logits at {off}")
+    act = torch.empty((n, inter), dtype=torch.bfloat16, device=rows.device) if gated is not None else None
     _check(library().ia_route_logits(_p(sel), _p(weight), _p(rows), ld, off, n, experts, top, ctypes.c_float(scale), SCORE_FUNCTIONS[score],
                                      int(renormalize), _p(choice_bias), gates, _p(gate_out), count, keep, *(_p(x) for x in plan.parts), plan.experts,
-                                     plan.tile, _stream()))
+                                     plan.tile, _p(act), inter, limit, slope, _stream()))
     plan.done = True
-    return sel, weight, gate_out
+    return (sel, weight, gate_out) if gated is None else (sel, weight, gate_out, act)
 
 
 def tile_weights(w: torch.Tensor) -> torch.Tensor:

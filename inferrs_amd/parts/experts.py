@@ -102,6 +102,15 @@ class RoutedExperts(FeedForward):
             self.shared = part_class("ffn", spec.shared)(
                 spec.shared, {k[len("shared."):]: v for k, v in tensors.items() if k.startswith("shared.") and k != "shared.sg"},
                 dtype, device)
+        # a shared expert's [gate; up] with the router's rows behind it: steps of a few rows form both in one product with 32-bit
+        # results (padded with rows of zeros: the result's rows then start at multiples of 16 bytes)
+        self.beside = None
+        if isinstance(self.shared, ClampedMlp) and dtype == torch.bfloat16 and self.shared.gate_up.bias is None and spec.shared.intermediate % 4 == 0:
+            first = self.shared.gate_up.weight
+            pad = -(first.shape[0] + self.router.shape[0]) % 8
+            self.beside = torch.cat([first, self.router, torch.zeros((pad, first.shape[1]), dtype=dtype, device=first.device)], dim=0)
+            self.shared.gate_up.weight = self.beside[:first.shape[0]]
+            self.router = self.beside[first.shape[0]:first.shape[0] + self.router.shape[0]]
         E = spec.experts
         gate_up = torch.stack([torch.cat([to_compute(tensors[f"e{e}.gate"], dtype, device),
                                           to_compute(tensors[f"e{e}.up"], dtype, device)], dim=0) for e in range(E)])
@@ -117,13 +126,17 @@ class RoutedExperts(FeedForward):
         s = self.spec
         if hasattr(h, "materialize"):
             h = h.materialize()
-        gate = None
+        gate = act = None
         plan = ops.mix.ExpertPlan(h.shape[0], s.top, s.experts, self.tiled, h.device)
         logits = getattr(ctx, "router_logits", None)
         if logits is not None:                       # (a block has laid the router's matrix beside one of its own)
             ctx.router_logits = None
             sel, weights, gate = ops.mix.route_logits(logits[0], logits[1], s.experts + s.identity, s.top, s.scale, s.score, s.renormalize,
                                                       self.correction, int(s.shared_gate), plan, groups=s.groups)
+        elif self.beside is not None and h.shape[0] <= min(ops.mix.ROUTE_LOGITS_ROWS, ops.SKINNY_MAX_ROWS) and ops.skinny_fits(h, self.beside):
+            sel, weights, gate, act = ops.mix.route_logits(
+                ops.linear(h, self.beside, torch.float32), 2 * s.shared.intermediate, s.experts + s.identity, s.top, s.scale, s.score, s.renormalize,
+                self.correction, int(s.shared_gate), plan, groups=s.groups, gated=(s.shared.intermediate, s.shared.limit, s.shared.alpha))
         elif s.shared_gate:
             sel, weights, gate = ops.route(h, self.router, s.top, s.scale, s.score, s.renormalize, self.correction, gates=1, plan=plan,
                                            groups=s.groups)
@@ -132,7 +145,9 @@ class RoutedExperts(FeedForward):
         rows = ops.experts_forward(h, sel, self.gate_up, self.down, s.limit, s.alpha,
                                    ff=s.intermediate if self.tiled else None,
                                    in_weight=weights if s.weight_on_input else None, activation=s.activation, plan=plan)
-        extra = self.shared.forward(ctx, h) if self.shared is not None else None
+        extra = None
+        if self.shared is not None:
+            extra = self.shared.forward(ctx, h) if act is None else self.shared.project(ctx, act)
         if s.weight_on_input:
             weights = None
         if s.identity == 0 and extra is None and weights is not None:
@@ -161,7 +176,9 @@ class ClampedMlp(FeedForward):
     def forward(self, ctx, h):
         if hasattr(h, "materialize"):
             h = h.materialize()
-        act = ops.clamped_gate_mul(self.gate_up(h), self.spec.limit, self.spec.alpha)
+        return self.project(ctx, ops.clamped_gate_mul(self.gate_up(h), self.spec.limit, self.spec.alpha))
+
+    def project(self, ctx, act):
         if getattr(ctx, "partial_sums", False):
             split = ops.linear_partials(act, self.down.weight, self.down.bias)
             if split is not None:

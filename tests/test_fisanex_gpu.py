@@ -555,3 +555,33 @@ def test_trace_runner_program(models, tmp_path):
     assert [l for l in p.stdout.splitlines() if l.startswith("done")] == [f"done {i}" for i in range(len(trace.lines))]
     err, where = worst(trace.read(out_dir, cfg["vocab"]), ref, some)
     assert err <= TOL_F32, (err, where)
+
+
+@pytest.mark.parametrize("n,inter,E,gates", [(1, 4, 5, 0), (3, 68, 36, 0), (16, 3072, 64, 1), (7, 1000, 200, 3)])
+def test_choice_beside_a_gated_product(n, inter, E, gates):
+    """`route_logits` over rows [gate | up | logits | gates]: the choice of rows without the first part, equal logits among them (the
+    lower index wins), and the clamped activation of the unrounded sums: 32-bit arithmetic and one rounding to bfloat16."""
+    import torch
+    from inferrs_amd import ops
+    top, limit, slope = min(4, E), 1.3, 1.702
+    gen = torch.Generator().manual_seed(n + E)
+    pad = -(2 * inter + E + gates) % 8
+    rows = torch.randn((n, 2 * inter + E + gates + pad), generator=gen)
+    rows[:, 2 * inter:2 * inter + E] = torch.randint(-3, 4, (n, E), generator=gen).float()       # many equal logits
+    bias = torch.randint(0, 2, (E,), generator=gen).float() * 0.25
+    for choice_bias in (None, bias):
+        plans = [ops.mix.ExpertPlan(n, top, E, False, "cuda") for _ in range(2)]
+        b = None if choice_bias is None else choice_bias.cuda()
+        alone = rows[:, 2 * inter:].contiguous().cuda()
+        want = ops.mix.route_logits(alone, 0, E, top, 1.5, "softmax", False, b, gates, plans[0])
+        got = ops.mix.route_logits(rows.cuda(), 2 * inter, E, top, 1.5, "softmax", False, b, gates, plans[1], gated=(inter, limit, slope))
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        assert gates == 0 or torch.equal(got[2], want[2])
+        z = rows[:, 2 * inter:2 * inter + E].double()
+        key = torch.softmax(z, dim=1) + (0 if choice_bias is None else bias.double())
+        order = torch.argsort(key, dim=1, descending=True, stable=True)[:, :top]
+        if choice_bias is None:                                     # (sums of a score and a bias may tie in 32 bits only)
+            assert torch.equal(got[0].cpu().long(), order)
+        g, u = rows[:, :inter].double().clamp(max=limit), rows[:, inter:2 * inter].double().clamp(-limit, limit)
+        act = g * torch.sigmoid(slope * g) * (u + 1)
+        assert float((got[3].cpu().double() - act).abs().max()) <= 2 ** -8 * float(act.abs().max()) * 1.01
