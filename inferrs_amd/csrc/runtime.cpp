@@ -395,6 +395,26 @@ extern "C" {
 const char* iar_last_error(void) { return g_error; }
 int iar_abi_version(void) { return IAR_ABI_VERSION; }
 
+// ---- random numbers of draws ------------------------------------------------------------------
+// A function of (seed, step) alone (the reference's, inferrs/src/sampler.rs:370-397): splitmix64 of the seed, mixed with the
+// step, one xorshift round, the high 32 bits of a multiply as a 32-bit float, over 2^32.
+void iar_rand_f32(int n, const uint64_t* seeds, const int64_t* steps, float* out) {
+    const uint64_t golden = 0x9E3779B97F4A7C15ull;
+    auto mix = [](uint64_t x) {
+        x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+        x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
+        return x ^ (x >> 31);
+    };
+    for (int i = 0; i < n; ++i) {
+        uint64_t x = mix(mix(seeds[i] + golden) + ((uint64_t)steps[i] + 1) * golden);
+        if (x == 0) x = 0x1234567890ABCDEFull;
+        x ^= x << 13;
+        x ^= x >> 7;
+        x ^= x << 17;
+        out[i] = (float)((x * 0x2545F4914F6CDD1Dull) >> 32) / 4294967296.0f;
+    }
+}
+
 // ---- cache manager --------------------------------------------------------------------------
 void* iar_cache_create(int page_size, int max_seqs, int n_groups, const int* windows, const int* keep_first, const int* num_pages) {
     if (page_size < 1) { fail(IAR_ERROR, "page_size must be >= 1, got %d", page_size); return nullptr; }

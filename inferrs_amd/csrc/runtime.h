@@ -66,6 +66,7 @@ int iar_cache_check_invariants(void* cache);
 int iar_build_step(void* cache, int n_entries, const int64_t* keys, const int* q_lens, const int* tokens,
                    const int* want_counts, const int* want, int pad_pages, int advance, int32_t* out,
                    long long capacity, int* meta, int* order_out);
+void iar_rand_f32(int n, const uint64_t* seeds, const int64_t* steps, float* out);
 long long iar_step_words(void* cache, int n_entries, const int64_t* keys, const int* q_lens, int n_want,
                          int pad_pages, int advance);
 

@@ -1438,6 +1438,35 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
     return out if n_top is None else (out, lp, ids)
 
 
+def sample_packed(logits: torch.Tensor, words: torch.Tensor, width: int, n_bias: int, *, penalized: bool,
+                  narrow_only: bool) -> torch.Tensor:
+    """`sample` of rows whose parameters lie one behind another in `words` (32-bit words on the device; an array a parameter, a row's
+    entries together): with `penalized` the windows [rows, width] (none for a width of 0), the repetition, frequency and presence
+    penalties, the biases' ids and values [rows, n_bias]; then temperature, top_k, top_p, min_p and u."""
+    _dev(logits, words); _f32(logits, "logits"); _i32(words, "words")
+    rows, vocab = logits.shape
+    if words.numel() < rows * ((width + 3 + 2 * n_bias if penalized else 0) + 5):
+        raise KernelError(f"sample_packed: {words.numel()} words for {rows} rows, windows of {width} and {n_bias} biases")
+    at, step = _p(words), 4 * rows
+    pen = _NO_PENALTIES
+    if penalized:
+        rep = at + width * step
+        ids = rep + 3 * step
+        pen = (at if width else None, width, rep, rep + step, rep + 2 * step, ids if n_bias else None,
+               ids + n_bias * step if n_bias else None, n_bias)
+        at = ids + 2 * n_bias * step
+    out = torch.empty((rows,), dtype=torch.int32, device=logits.device)
+    ws = torch.empty((_sample_workspace(rows, vocab),), dtype=torch.int32, device=logits.device)
+    _check(library().ia_sample(_p(out), _p(logits), _p(ws), rows, vocab, at, at + step, at + 2 * step, at + 3 * step, at + 4 * step,
+                               None, None, None, *pen, int(narrow_only), _stream()))
+    return out
+
+
+@functools.lru_cache(maxsize=256)
+def _sample_workspace(rows: int, vocab: int) -> int:
+    return _raw_library().ia_sample_workspace(rows, vocab)
+
+
 def _mid_dual_fits(x: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
     """[gate; up] at up to 16 rows on gemm_mid.hip: where the weight makes a block for every compute unit."""
     return (w_gate_up.shape[0] % 2 == 0 and mid_fits(x, w_gate_up, few_rows=True)

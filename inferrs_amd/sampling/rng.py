@@ -4,6 +4,10 @@ from __future__ import annotations
 
 import os
 import struct
+from array import array
+from typing import Sequence
+
+from ..native import runtime
 
 _M64 = (1 << 64) - 1
 _GOLDEN = 0x9E3779B97F4A7C15
@@ -28,6 +32,12 @@ def rand_f32(seed: int, step: int) -> float:
     hi = ((x * 0x2545F4914F6CDD1D) & _M64) >> 32
     as_f32 = struct.unpack("<f", struct.pack("<f", float(hi)))[0]       # u64 -> f32 rounds to nearest
     return struct.unpack("<f", struct.pack("<f", as_f32 / 4294967296.0))[0]
+
+
+def rand_f32_many(seeds: Sequence[int], steps: Sequence[int], out: int) -> None:
+    """`rand_f32` of every pair, as 32-bit floats to the address `out`."""
+    s, t = array("Q", [seed & _M64 for seed in seeds]), array("q", steps)
+    runtime().iar_rand_f32(len(s), s.buffer_info()[0], t.buffer_info()[0], out)
 
 
 def fresh_seed() -> int:

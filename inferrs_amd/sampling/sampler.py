@@ -4,6 +4,8 @@ presence penalties over the last `repeat_last_n` tokens, temperature, softmax, t
 min-p, and the walk to a random number that depends on the request's seed and step only."""
 from __future__ import annotations
 
+from array import array
+from struct import pack
 from typing import List, Optional, Sequence
 
 import numpy as np
@@ -11,7 +13,7 @@ import torch
 
 from .. import ops
 from .params import SAMPLING_EPS, SamplingParams, TokenLogprob
-from .rng import rand_f32
+from .rng import rand_f32, rand_f32_many
 
 
 class Sampler:
@@ -39,6 +41,54 @@ class Sampler:
             at += a.size
         return out
 
+    def _pack(self, params: Sequence[SamplingParams], previous: Sequence[Sequence[int]], seeds: Sequence[int]):
+        """What a draw takes beside the logits, laid out as `ops.sample_packed` reads it, on its way to the device: (words, the
+        windows' width, biases a row, whether there are penalties or biases).  A field at a time over all rows and one array of the
+        interpreter's for each kind of number: 24 rows with windows of 64 had taken 110 us as NumPy rows and a random number each."""
+        rows, lens = len(params), [len(prev) for prev in previous]
+        last = [p.repeat_last_n for p in params]
+        rep, freq, pres = ([p.repetition_penalty for p in params], [p.frequency_penalty for p in params],
+                           [p.presence_penalty for p in params])
+        # (rows without a penalty, and those with no token yet, have no window)
+        takes = [min(k, n) if k > 0 and n > 0 and (r != 1.0 or f != 0.0 or q != 0.0) else 0
+                 for k, n, r, f, q in zip(last, lens, rep, freq, pres)]
+        width, n_bias = max(takes), max([len(p.logit_bias) for p in params])
+        penalized = bool(width or n_bias)
+        whole, real = [], []                                    # the arrays in front: 32-bit numbers, and what follows them
+        if penalized:
+            for prev, take in zip(previous, takes):
+                if take:
+                    whole += prev[-take:]
+                if take < width:
+                    whole += [-1] * (width - take)
+            real += [r if take else 1.0 for r, take in zip(rep, takes)]
+            real += [f if take else 0.0 for f, take in zip(freq, takes)]
+            real += [q if take else 0.0 for q, take in zip(pres, takes)]
+        # (packing arguments is twice as fast as an array out of a list, which takes numbers beyond 32 bits as infinities)
+        parts = [pack(f"{len(whole)}i", *whole), array("f", real).tobytes()]
+        if n_bias:
+            pairs = [sorted(p.logit_bias.items()) for p in params]
+            pairs = [row + [(-1, 0.0)] * (n_bias - len(row)) for row in pairs]
+            parts.append(pack(f"{rows * n_bias}i", *[int(t) for row in pairs for t, _ in row]))
+            parts.append(array("f", [v for row in pairs for _, v in row]).tobytes())
+        temperature = [p.temperature for p in params]
+        if min(temperature) < SAMPLING_EPS:
+            temperature = [p.draw_temperature(n) for p, n in zip(params, lens)]
+        parts += [array("f", temperature).tobytes(), pack(f"{rows}i", *[p.top_k for p in params]),
+                  array("f", [p.top_p for p in params] + [p.min_p for p in params]).tobytes()]
+        front = b"".join(parts)
+        at = len(front)
+        host = torch.empty(at // 4 + 2 * rows, dtype=torch.int32, pin_memory=self.device.type == "cuda")
+        view = memoryview(host.numpy()).cast("B")
+        view[:at] = front
+        # the step of a draw is the number of tokens before it (`sampler.rs:323-325`); rows of temperature 0 draw nothing
+        rand_f32_many(seeds, lens, host.data_ptr() + at)
+        for i, t in enumerate(temperature):
+            if t < SAMPLING_EPS:
+                view[at + 4 * i:at + 4 * i + 4] = b"\0\0\0\0"
+        view[at + 4 * rows:] = pack(f"{rows}i", *[p.top_logprobs if p.logprobs else -1 for p in params])
+        return host.to(self.device, non_blocking=True), width, n_bias, penalized
+
     def begin_chain(self, params: Sequence[SamplingParams], previous: Sequence[Sequence[int]],
                     seeds: Sequence[int], steps: int) -> "ChainDraw":
         """The draws of the next `steps` decode steps of these requests, prepared for the device."""
@@ -62,52 +112,29 @@ class Sampler:
         if all(p.is_plain_greedy for p in params):
             return ops.argmax(logits).cpu().tolist(), [None] * rows
 
-        # penalties and bias, which the draw applies on the way (the logits stay as they are)
-        width = max((min(p.repeat_last_n, len(prev)) if p.has_penalty else 0) for p, prev in zip(params, previous))
-        n_bias = max(len(p.logit_bias) for p in params)
-        window = rep = freq = pres = bias_ids = bias_vals = None
-        if width or n_bias:
-            window = np.full((rows, max(width, 1)), -1, dtype=np.int32)
-            rep = np.ones(rows, dtype=np.float32)
-            freq = np.zeros(rows, dtype=np.float32)
-            pres = np.zeros(rows, dtype=np.float32)
-            for i, (p, prev) in enumerate(zip(params, previous)):
-                if p.has_penalty and prev:
-                    tail = list(prev[-p.repeat_last_n:])
-                    window[i, :len(tail)] = tail
-                    rep[i], freq[i], pres[i] = p.repetition_penalty, p.frequency_penalty, p.presence_penalty
-            if n_bias:
-                bias_ids = np.full((rows, n_bias), -1, dtype=np.int32)
-                bias_vals = np.zeros((rows, n_bias), dtype=np.float32)
-                for i, p in enumerate(params):
-                    for j, (tid, b) in enumerate(sorted(p.logit_bias.items())):
-                        bias_ids[i, j], bias_vals[i, j] = int(tid), float(b)
-
-        temperature = np.asarray([p.draw_temperature(len(prev)) for p, prev in zip(params, previous)], dtype=np.float32)
-        top_k = np.asarray([p.top_k for p in params], dtype=np.int32)
-        top_p = np.asarray([p.top_p for p in params], dtype=np.float32)
-        min_p = np.asarray([p.min_p for p in params], dtype=np.float32)
-        # the step of a draw is the number of tokens before it (`sampler.rs:323-325`)
-        u = np.asarray([rand_f32(seed, len(prev)) if p.draw_temperature(len(prev)) >= SAMPLING_EPS else 0.0
-                        for p, prev, seed in zip(params, previous, seeds)], dtype=np.float32)
-        n_top = np.asarray([p.top_logprobs if p.logprobs else -1 for p in params], dtype=np.int32)
-        penalized = window is not None
-        narrow = all_narrow(int(top_k.min()), int(top_k.max()), logits.shape[1])
+        words, width, n_bias, penalized = self._pack(params, previous, seeds)
+        top_k = [p.top_k for p in params]
+        reports = any([p.logprobs for p in params])
+        narrow = all_narrow(min(top_k), max(top_k), logits.shape[1])
         # (rows that report entries of a list which top_p or min_p may not end, to within what 32 bits round: one call for all)
-        open_rows = [p for p in params if p.top_logprobs > 1 and p.top_p > 0.999 and p.min_p < 1e-6]
+        open_rows = [p for p in params if p.top_logprobs > 1 and p.top_p > 0.999 and p.min_p < 1e-6] if reports else ()
         if narrow and open_rows:
             narrow = ops.sample_is_narrow(open_rows[0].top_k, logits.shape[1], min(p.temperature for p in open_rows), 1.0, 0.0, 2,
                                           any(p.logit_bias for p in open_rows))
-        window, rep, freq, pres, bias_ids, bias_vals, temperature, top_k, top_p, min_p, u, n_top = self._upload(
-            window if width else None, rep, freq, pres, bias_ids, bias_vals, temperature, top_k, top_p, min_p, u, n_top)
+        if not logits.is_contiguous():
+            logits = logits.clone()
+        # (penalties and bias are applied on the way: the logits stay as they are)
+        if not reports:
+            out = ops.sample_packed(logits, words, width, n_bias, penalized=penalized, narrow_only=narrow)
+            return out.cpu().tolist(), [None] * rows
+        sizes = ([rows * width] + [rows] * 3 + [rows * n_bias] * 2 if penalized else []) + [rows] * 6
+        *pen, temperature, top_k, top_p, min_p, u, n_top = words.split(sizes)
         penalties = None
         if penalized:
-            penalties = (window, rep, freq, pres, bias_ids, bias_vals)
-            if not logits.is_contiguous():
-                logits = logits.clone()
-        if not any(p.logprobs for p in params):
-            out = ops.sample(logits, temperature, top_k, top_p, min_p, u, penalties=penalties, narrow_only=narrow)
-            return out.cpu().tolist(), [None] * rows
+            window, rep, freq, pres, bias_ids, bias_vals = pen
+            penalties = (window.view(rows, width) if width else None, *(t.view(torch.float32) for t in (rep, freq, pres)),
+                         *((bias_ids.view(rows, n_bias), bias_vals.view(torch.float32).view(rows, n_bias)) if n_bias else (None, None)))
+        temperature, top_p, min_p, u = (t.view(torch.float32) for t in (temperature, top_p, min_p, u))
         out, lp, ids = ops.sample(logits, temperature, top_k, top_p, min_p, u, n_top, penalties=penalties, narrow_only=narrow)
         tokens, lp, ids = out.cpu().tolist(), lp.cpu().tolist(), ids.cpu().tolist()
         infos = []
