@@ -102,6 +102,11 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(float* __restrict__ out, 
                 __syncthreads();
                 read(sh[buf ^ 1], 0, 0);
             }
+            // (the compiler sinks the reads behind the step's products to save registers; a step of one instruction in a wave
+            // that is alone on its SIMD is then the reads' latency: 4,096 x 4,096, 64 rows 48.0 -> 37.2 us.  Larger tiles, and several
+            // blocks a unit, lose 2 to 6 % by it, and by a second chunk on its way 5 to 15 %: there neither the shared memory's
+            // latency nor the memory's sets the pace.)
+            if constexpr (MT * NR == 1 && GF_K == 128) __builtin_amdgcn_sched_barrier(0);
             multiply(j & 1);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -155,7 +160,7 @@ extern "C" int ia_gemm_f32(void* out, const void* x, const void* w, int M, int N
     }
     // A compute unit's time is what its blocks multiply one after the other or side by side: full turns of the compute units
     // times the instructions a block has for a step of four k, and a little a turn; a block that is alone on its unit waits for
-    // memory besides (32 rows, 4,096 features: 1 x 1 tiles 47 us, 2 x 1 62, 3 x 1 73, 4 x 1 95).  Measured at 555 rows and 4,096 features:
+    // memory besides (32 rows, 4,096 features: 1 x 1 tiles 36 us, 2 x 1 60, 3 x 1 77, 4 x 1 95; 100 rows: 1 x 1 tiles in two turns 73, 2 x 1 in one 63).  Measured at 555 rows and 4,096 features:
     // 9 x 1 tiles in one turn 192 us, 5 x 1 in two 191, 3 x 1 in three 188, 10 x 1 in one 204; at 24,576 features 9 x 2 in three
     // turns 918, 7 x 2 in four 942, 9 x 1 in six 969; 130 rows and 24,576 features: 5 x 1 in three turns 297, 3 x 2 in three 330.
     int best_m = 8, best_n = 2;
@@ -164,8 +169,10 @@ extern "C" int ia_gemm_f32(void* out, const void* x, const void* w, int M, int N
         for (int mt = 10; mt >= 1; --mt) {
             const long long blocks = (long long)((M + 16 * mt - 1) / (16 * mt)) * ((N + 64 * nr - 1) / (64 * nr));
             const double work = mt * nr;
-            const double alone = 0.65 * work + 1.55 > 1.03 * work ? 0.65 * work + 1.55 : 1.03 * work;
-            const double cost = blocks <= cus ? alone : (double)((blocks + cus - 1) / cus) * (work + 0.3);
+            // (two turns of the smallest blocks are no cheaper than two blocks alone)
+            const long long turns = (blocks + cus - 1) / cus;
+            const double alone = mt * nr == 1 ? 1.65 : 0.65 * work + 1.55 > 1.03 * work ? 0.65 * work + 1.55 : 1.03 * work;
+            const double cost = turns == 1 ? alone : (double)turns * (work + (mt * nr == 1 && turns == 2 ? 0.5 : 0.3));
             if (cost < best && blocks < (1LL << 31)) best = cost, best_m = mt, best_n = nr;
         }
     if (g_f32_shape) best_m = g_f32_shape / 10, best_n = g_f32_shape % 10;
