@@ -743,6 +743,268 @@ __global__ __launch_bounds__(256) void linear_local_mfma_kernel(const ScanArgs a
     }
 }
 
+// ---- chunks of bfloat16 rows on the bfloat16 matrix cores ----------------------------------------------------------------
+// q, k and v are bfloat16 values, so every product q.k is exact there and only its sums are 32-bit, as they were.  What is 32-bit
+// on one side (weighted scores, weighted values, the matrix a chunk starts from) goes in as three bfloat16 numbers that add up to
+// it exactly (eight bits of its 24 each): three products on an instruction that multiplies sixteen times as much a cycle as the
+// 32-bit one.  Errors against 64 bits, 20 sizes: 0.52 to 1.02 of the 32-bit kernels', 0.87 in the mean.  The walk over a chunk comes in two kernels with
+// `chunk_states_kernel` between them: the chunk's own matrix U alone, and then every output at once, from the chunk's tokens and from
+// the matrix it starts from, so that outputs are written once and not read again.  What bounded the 32-bit kernels: their instruction
+// (a third of the time) and one operand read of 4 bytes a lane for each of its steps.  us, the three kernels, before and now (1,500
+// tokens): 64 heads of 128 x 64 152 -> 73, 8 of 128 x 256 with a normaliser 98 -> 47, 16 of 64 x 128 58 -> 35; 300 tokens 56 -> 33, 41 -> 24, 28 -> 18.
+#define LX_LD 72                        // bfloat16 values of a staged row of 64 tokens: 16 rows' 16-byte pieces fall on different banks
+typedef __bf16 ls_bf16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ ls_f32x4 lx_mfma(const uint4& x, const uint4& y, const ls_f32x4& acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(ls_bf16x8, x), __builtin_bit_cast(ls_bf16x8, y), acc, 0, 0, 0);
+}
+// x = part 0 + part 1 + part 2 exactly, each in the upper half of its word: the leading eight bits, those behind them, the rest
+__device__ __forceinline__ void lx_split(float x, uint32_t (&part)[3]) {
+    part[0] = __float_as_uint(x) & 0xffff0000u;
+    const float rest = x - __uint_as_float(part[0]);
+    part[1] = __float_as_uint(rest) & 0xffff0000u;
+    part[2] = __float_as_uint(rest - __uint_as_float(part[1]));
+}
+// eight values -> the three operands that add up to them
+__device__ __forceinline__ void lx_split8(const float (&x)[8], uint4 (&part)[3]) {
+    uint32_t w[3][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t a[3], b[3];
+        lx_split(x[2 * i], a);
+        lx_split(x[2 * i + 1], b);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) w[p][i] = (a[p] >> 16) | (b[p] & 0xffff0000u);
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p) part[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
+}
+// A wave's lanes as the chunk's 64 tokens: the sums of the decays' logarithms up to each (g), the input scales (b) and, where `run`
+// is asked for, the products of the decays.
+__device__ __forceinline__ void lx_gates(const ScanArgs& a, int h, int first, int nt, int tt, float& g, float& b, float* run) {
+    g = 0.f;
+    b = 0.f;
+    float r = 1.f;
+    if (tt < nt) {
+        const float an = a.log_a[a.a_per_token ? (long long)(first + tt) * a.H + h : h];
+        g = fmaxf(a.a_per_token ? an : logf(an), -1e4f);
+        r = a.a_per_token ? expf(an) : an;
+        b = a.b != nullptr ? a.b[(long long)(first + tt) * a.H + h] : 1.f;
+    }
+#pragma unroll
+    for (int o = 1; o < LC_TOKENS; o <<= 1) {
+        const float before = __shfl_up(g, o, IA_WAVE);
+        if (tt >= o) g += before;
+    }
+    if (run == nullptr) return;
+#pragma unroll
+    for (int o = 1; o < LC_TOKENS; o <<= 1) {
+        const float before = __shfl_up(r, o, IA_WAVE);
+        if (tt >= o) r *= before;
+    }
+    *run = r;
+}
+
+// U = sum_s exp(G_last - G_s) b_s k_s v_s^T over a chunk, for 64 columns of v: keys and weighted values lie feature by feature in shared
+// memory (a lane brings 16 bytes of its token and lays them down a feature each), a wave owns every fourth 16 rows of U.
+template <int KS>
+__global__ __launch_bounds__(256) void linear_chunk_matrix_kernel(const ScanArgs a) {
+    __shared__ __attribute__((aligned(16))) uint16_t k_t[32 * KS][LX_LD];
+    __shared__ __attribute__((aligned(16))) uint16_t v_t[3][64][LX_LD];
+    __shared__ float w_s[LC_TOKENS];
+    const int h = blockIdx.y, j0 = blockIdx.x * 64;
+    const int seq = blockIdx.z / a.max_chunks, c = blockIdx.z - seq * a.max_chunks;
+    const int first = a.cu_tokens[seq] + c * a.chunk, end = a.cu_tokens[seq + 1];
+    if (first >= end) return;                              // (the whole block)
+    const int nt = end - first < a.chunk ? end - first : a.chunk;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, g4 = lane >> 4;
+    const int vt = a.vdim + (a.den != nullptr ? 1 : 0);
+    const long long token = first + (lane < nt ? lane : nt - 1);
+    const bf16_t* k = (const bf16_t*)a.k + a.k_off + (long long)(h / (a.H / a.k_heads)) * a.dim + token * a.k_ld;
+    const bf16_t* v = (const bf16_t*)a.v + a.v_off + (long long)h * a.vdim + j0 + token * a.v_ld;
+    uint4 kp[KS], vp[2];
+#pragma unroll
+    for (int i = 0; i < KS; ++i) kp[i] = *(const uint4*)(k + (wave + 4 * i) * 8);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) vp[i] = *(const uint4*)(v + (wave + 4 * i) * 8);
+    float g, b;
+    lx_gates(a, h, first, nt, lane, g, b, nullptr);
+    const float g_last = __shfl(g, LC_TOKENS - 1, IA_WAVE);
+    const float w = lane < nt ? expf(g_last - g) * b * a.k_scale : 0.f;      // (tokens that the chunk does not have weigh nothing)
+    if (wave == 0) w_s[lane] = w;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.chunk_a[(long long)blockIdx.z * a.H + h] = expf(g_last);
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+        const uint32_t word[4] = {kp[i].x, kp[i].y, kp[i].z, kp[i].w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) k_t[(wave + 4 * i) * 8 + j][lane] = lane < nt ? (uint16_t)(word[j >> 1] >> (16 * (j & 1))) : (uint16_t)0;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t word[4] = {vp[i].x, vp[i].y, vp[i].z, vp[i].w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            uint32_t part[3];
+            lx_split(lane < nt ? __uint_as_float(j & 1 ? word[j >> 1] & 0xffff0000u : word[j >> 1] << 16) * w : 0.f, part);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) v_t[p][(wave + 4 * i) * 8 + j][lane] = (uint16_t)(part[p] >> 16);
+        }
+    }
+    __syncthreads();
+    float* const u_out = a.chunk_s + ((long long)blockIdx.z * a.H + h) * vt * a.dim;
+#pragma unroll
+    for (int mt = wave; mt < 2 * KS; mt += 4) {
+        uint4 kf[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) kf[u] = *(const uint4*)&k_t[16 * mt + r16][32 * u + 8 * g4];
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct) {
+            ls_f32x4 acc = (ls_f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int p = 2; p >= 0; --p)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) acc = lx_mfma(kf[u], *(const uint4*)&v_t[p][16 * ct + r16][32 * u + 8 * g4], acc);
+            *(ls_f32x4*)(u_out + (long long)(j0 + 16 * ct + r16) * a.dim + 16 * mt + 4 * g4) = acc;
+        }
+    }
+    if (a.den != nullptr && blockIdx.x == 0 && (int)threadIdx.x < a.dim) {   // the column of ones
+        float sum = 0.f;
+        for (int t = 0; t < LC_TOKENS; ++t) sum = fmaf(__uint_as_float((uint32_t)k_t[threadIdx.x][t] << 16), w_s[t], sum);
+        u_out[(long long)a.vdim * a.dim + threadIdx.x] = sum;
+    }
+}
+
+// out_t = sum_(s <= t) (q_t . k_s) exp(G_t - G_s) b_s v_s + (prod_(s <= t) a_s) S^T q_t (+ skip v_t) for 64 columns of v, S the matrix that the
+// chunk starts from.  A wave scores 16 tokens (as columns, with the keys' rows exchanged so that a lane ends up with eight scores of
+// neighbouring keys: one operand's piece) and leaves their weighted scores in shared memory; then it owns 16 columns of v for all tokens.
+template <int KS>
+__global__ __launch_bounds__(256) void linear_chunk_outputs_kernel(const ScanArgs a) {
+    __shared__ __attribute__((aligned(16))) uint16_t q_s[LC_TOKENS][32 * KS + 8];
+    __shared__ __attribute__((aligned(16))) uint16_t p_s[3][LC_TOKENS][LX_LD];
+    __shared__ __attribute__((aligned(16))) uint16_t v_t[64][LX_LD];
+    __shared__ float g_s[LC_TOKENS], b_s[LC_TOKENS], run_s[LC_TOKENS];
+    const int h = blockIdx.y, j0 = blockIdx.x * 64;
+    const int seq = blockIdx.z / a.max_chunks, c = blockIdx.z - seq * a.max_chunks;
+    const int first = a.cu_tokens[seq] + c * a.chunk, end = a.cu_tokens[seq + 1];
+    if (first >= end) return;                              // (the whole block)
+    const int nt = end - first < a.chunk ? end - first : a.chunk;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, g4 = lane >> 4;
+    const int vt = a.vdim + (a.den != nullptr ? 1 : 0);
+    auto row = [&](int t) { return (long long)first + (t < nt ? t : nt - 1); };     // (of a token that the chunk does not have: the last one's, masked)
+    const bf16_t* q = (const bf16_t*)a.q + a.q_off + (long long)(h / (a.H / a.q_heads)) * a.dim + 8 * g4;
+    const bf16_t* k = (const bf16_t*)a.k + a.k_off + (long long)(h / (a.H / a.k_heads)) * a.dim + 8 * g4;
+    const bf16_t* v = (const bf16_t*)a.v + a.v_off + (long long)h * a.vdim + j0;
+    const float* start = a.chunk_s + ((long long)blockIdx.z * a.H + h) * vt * a.dim;
+    // ---- everything that comes from memory is asked for first
+    const int t_mine = 16 * wave + r16;
+    uint4 qf[KS], kf[2][2][KS], vp[2];
+    float4 sf[KS][2];
+    const bool both = wave >= 2;                           // (the first 32 tokens' queries see the first 32 keys only)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *(const uint4*)(q + row(t_mine) * a.q_ld + 32 * ks);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                if (u == 0 || both) kf[u][tt][ks] = *(const uint4*)(k + row(32 * u + 8 * (r16 >> 2) + 4 * tt + (r16 & 3)) * a.k_ld + 32 * ks);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) vp[i] = *(const uint4*)(v + row(lane) * a.v_ld + (wave + 4 * i) * 8);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) sf[ks][i] = *(const float4*)(start + (long long)(j0 + t_mine) * a.dim + 32 * ks + 8 * g4 + 4 * i);
+    float g, b, run;
+    lx_gates(a, h, first, nt, lane, g, b, &run);
+    if (wave == 0) { g_s[lane] = g; b_s[lane] = b * a.k_scale * a.q_scale; run_s[lane] = run * a.q_scale; }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) *(uint4*)&q_s[t_mine][32 * ks + 8 * g4] = qf[ks];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t word[4] = {vp[i].x, vp[i].y, vp[i].z, vp[i].w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v_t[(wave + 4 * i) * 8 + j][lane] = lane < nt ? (uint16_t)(word[j >> 1] >> (16 * (j & 1))) : (uint16_t)0;
+    }
+    __syncthreads();
+    // ---- weighted scores: lane (token 16 wave + r16) holds keys 32 u + 8 g4 + 4 tt + i
+    const float g_mine = g_s[t_mine];
+    float ones = 0.f;                                      // what the column of ones gives
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        if (u == 1 && !both) break;
+        float score[8];
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            ls_f32x4 acc = (ls_f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) acc = lx_mfma(kf[u][tt][ks], qf[ks], acc);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int at = 32 * u + 8 * g4 + 4 * tt + i;
+                score[4 * tt + i] = at <= t_mine && at < nt ? acc[i] * expf(g_mine - g_s[at]) * b_s[at] : 0.f;
+                ones += score[4 * tt + i];
+            }
+        }
+        uint4 part[3];
+        lx_split8(score, part);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *(uint4*)&p_s[p][t_mine][32 * u + 8 * g4] = part[p];
+    }
+    if (a.den != nullptr && blockIdx.x == 0) {
+        const float* s_ones = start + (long long)a.vdim * a.dim + 8 * g4;
+        float carried = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const uint32_t word[4] = {qf[ks].x, qf[ks].y, qf[ks].z, qf[ks].w};
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                carried = fmaf(__uint_as_float(j & 1 ? word[j >> 1] & 0xffff0000u : word[j >> 1] << 16), s_ones[32 * ks + j], carried);
+        }
+        ones = fmaf(run_s[t_mine], carried, ones);
+        ones += __shfl_xor(ones, 16, IA_WAVE);
+        ones += __shfl_xor(ones, 32, IA_WAVE);
+        if (g4 == 0 && t_mine < nt) a.den[((long long)first + t_mine) * a.H + h] = ones;
+    }
+    uint4 s_part[KS][3];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        const float x[8] = {sf[ks][0].x, sf[ks][0].y, sf[ks][0].z, sf[ks][0].w, sf[ks][1].x, sf[ks][1].y, sf[ks][1].z, sf[ks][1].w};
+        lx_split8(x, s_part[ks]);
+    }
+    __syncthreads();
+    // ---- columns 16 wave .. of v: lane holds columns 16 wave + 4 g4 + i of token 16 tile + r16
+    uint4 vf[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) vf[u] = *(const uint4*)&v_t[16 * wave + r16][32 * u + 8 * g4];
+    const float skip = a.skip != nullptr ? a.skip[h] : 0.f;
+#pragma unroll
+    for (int tile = 0; tile < 4; ++tile) {
+        if (16 * tile >= nt) break;                        // (the same for all threads)
+        const int t = 16 * tile + r16;
+        ls_f32x4 own = (ls_f32x4){0.f, 0.f, 0.f, 0.f}, carried = own;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const uint4 qt = *(const uint4*)&q_s[t][32 * ks + 8 * g4];
+#pragma unroll
+            for (int p = 2; p >= 0; --p) carried = lx_mfma(s_part[ks][p], qt, carried);
+        }
+#pragma unroll
+        for (int u = 0; u < (tile >= 2 ? 2 : 1); ++u)
+#pragma unroll
+            for (int p = 2; p >= 0; --p) own = lx_mfma(vf[u], *(const uint4*)&p_s[p][t][32 * u + 8 * g4], own);
+        if (t >= nt) continue;
+        const float r = run_s[t];
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            o[i] = fmaf(r, carried[i], own[i]);
+            if (a.skip != nullptr) o[i] = fmaf(skip, __uint_as_float((uint32_t)v_t[16 * wave + 4 * g4 + i][t] << 16), o[i]);
+        }
+        *(float4*)(a.out + (((long long)first + t) * a.H + h) * a.vdim + j0 + 16 * wave + 4 * g4) = make_float4(o[0], o[1], o[2], o[3]);
+    }
+}
+
 // A request's chunks in order, one thread an entry of the heads' matrices: the workspace's U_c becomes the matrix that
 // chunk c starts from, the state row takes the matrix behind the last chunk.
 __global__ void chunk_states_kernel(float* __restrict__ chunk_s, const float* __restrict__ chunk_a, float* __restrict__ state,
@@ -767,7 +1029,7 @@ __global__ void chunk_states_kernel(float* __restrict__ chunk_s, const float* __
     *srow = S;
 }
 
-// (tests switch the matrix cores' form of CARRY off to compare it with the vector units')
+// (tests switch the matrix cores' forms off to compare them with the vector units': 0; 2: the 32-bit ones only)
 static int g_carry_mfma = 1;
 extern "C" void ia_linear_scan_tune(int carry_mfma) { g_carry_mfma = carry_mfma; }
 
@@ -885,7 +1147,22 @@ extern "C" int ia_linear_scan(float* out, float* den, float* state, long long ro
     const int per_head = vt * dim;
     const dim3 sgrid((unsigned)(((long long)H * per_head + 255) / 256), (unsigned)n_seqs);
     const bool cores = g_carry_mfma && dim <= LC_MAX_DIM && chunk <= LC_TOKENS;
-    if (cores) {
+    // bfloat16 rows as they are, in whole steps of the bfloat16 instruction and of 64 columns, read 16 bytes at a time
+    const bool split = cores && g_carry_mfma != 2 && dtype == IA_BF16 && act == IA_ACT_NONE && dim % 32 == 0 && vdim % 64 == 0 && a.q_vec && a.k_vec && a.wide &&
+                       v_off % 8 == 0 && v_ld % 8 == 0 && (((uintptr_t)v | (uintptr_t)out) & 15) == 0;
+    const dim3 xgrid((unsigned)(vdim / 64), (unsigned)H, (unsigned)(n_seqs * a.max_chunks));
+#define LX_LAUNCH(KERNEL)                                                             \
+    do {                                                                              \
+        switch (dim / 32) {                                                           \
+            case 1: KERNEL<1><<<xgrid, 256, 0, stream>>>(a); break;                   \
+            case 2: KERNEL<2><<<xgrid, 256, 0, stream>>>(a); break;                   \
+            case 3: KERNEL<3><<<xgrid, 256, 0, stream>>>(a); break;                   \
+            default: KERNEL<4><<<xgrid, 256, 0, stream>>>(a); break;                  \
+        }                                                                             \
+    } while (0)
+    if (split) {
+        LX_LAUNCH(linear_chunk_matrix_kernel);
+    } else if (cores) {
         const int ld_s = (dim + 3) / 4 * 4 + 4;
         const int cols = ia_linear_scan_columns((long long)H * n_seqs * a.max_chunks, vt, dim);
         const dim3 lgrid((unsigned)((vt + cols - 1) / cols), (unsigned)H, (unsigned)(n_seqs * a.max_chunks));
@@ -906,7 +1183,9 @@ extern "C" int ia_linear_scan(float* out, float* den, float* state, long long ro
     }
     chunk_states_kernel<<<sgrid, 256, 0, stream>>>(a.chunk_s, a.chunk_a, state, row_floats, s_off, cu_tokens, state_slots, per_head,
                                                    H, chunk, a.max_chunks);
-    if (cores) {
+    if (split) {
+        LX_LAUNCH(linear_chunk_outputs_kernel);
+    } else if (cores) {
         const int ld_s = (dim + 3) / 4 * 4 + 4;
         const dim3 cgrid((unsigned)((vt + LC_COLS - 1) / LC_COLS), (unsigned)H, (unsigned)(n_seqs * a.max_chunks));
         const size_t cshm = (size_t)((LC_TOKENS + LC_COLS) * ld_s + LC_TOKENS) * sizeof(float);
@@ -915,6 +1194,7 @@ extern "C" int ia_linear_scan(float* out, float* den, float* state, long long ro
     } else {
         LS_LAUNCH(LS_CARRY, grid);
     }
+#undef LX_LAUNCH
 #undef LS_LAUNCH
 #undef LS_LAUNCH_P
     IA_LAUNCH_CHECK("linear_scan (chunks)");

@@ -148,8 +148,9 @@ def linear_scan(*, q: torch.Tensor, q_off: int, q_heads: int, k: torch.Tensor, k
     `max_q_len`: an upper bound of the tokens a request brings (0: unknown, the step's tokens).  `chunk`: 0 walks every
     request's tokens in order; a number cuts portions into chunks of that many tokens that run side by side (three
     kernels: each chunk from nothing, the chunks' matrices in order, what each chunk's start contributes; for keys of
-    up to 128 entries and chunks of up to 64 tokens the first and the third are products on the matrix cores in true
-    32-bit), which differs from the walk by rounding; None: chunks of `SCAN_CHUNK` for steps with a portion of more than `SCAN_CHUNKS_FROM` tokens."""
+    up to 128 entries and chunks of up to 64 tokens the first and the third are products on the matrix cores, in true
+    32-bit or, of bfloat16 rows, in bfloat16 numbers that add up to the 32-bit ones), which differs from the walk by rounding; None: chunks
+    of `SCAN_CHUNK` for steps with a portion of more than `SCAN_CHUNKS_FROM` tokens, or fewer where bfloat16 rows go in such numbers."""
     _dev(q, k, v, state, cu_tokens, state_slots, log_a, decay, b, skip)
     _f32(log_a, "log_a"); _f32(decay, "decay"); _f32(b, "b"); _f32(skip, "skip")
     _i32(cu_tokens, "cu_tokens"); _i32(state_slots, "state_slots")
@@ -171,7 +172,13 @@ def linear_scan(*, q: torch.Tensor, q_off: int, q_heads: int, k: torch.Tensor, k
     n_seqs = state_slots.numel()
     longest = int(max_q_len) or n
     if chunk is None:
-        chunk = SCAN_CHUNK if longest > SCAN_CHUNKS_FROM else 0
+        least = SCAN_CHUNKS_FROM
+        if (q.dtype == torch.bfloat16 and act == 0 and dim % 32 == 0 and dim <= 128 and vdim % 64 == 0
+                and (q_off | k_off | v_off | q.shape[1] | k.shape[1] | v.shape[1]) % 8 == 0 and (s_off | row) % 4 == 0):
+            # (chunks of such rows are the bfloat16 matrix cores': one request of 32 tokens 17.7 us by chunks, 19.6 by the walk, 100 tokens
+            # 22 and 51; a request more costs a chunk's matrices: 4 of 32 tokens 27.1 and 27.6, 8 of 16 35 and 26)
+            least = min(least, 32 + 6 * (n_seqs - 1))
+        chunk = SCAN_CHUNK if longest > least else 0
         while chunk and n_seqs * -(-longest // chunk) * heads * (vdim + 1) * dim > SCAN_WORKSPACE_FLOATS:
             chunk *= 2
     lib = library()

@@ -349,6 +349,51 @@ def test_scan_in_chunks_is_the_walk(H, qh, dim, vdim, normaliser, dtype):
                 assert float((got - want).abs().max()) <= 2e-5 * scale, (chunk, matrix_cores, float((got - want).abs().max()) / scale)
 
 
+@pytest.mark.parametrize("H,qh,dim,vdim,normaliser", [(4, 2, 32, 64, True), (2, 1, 64, 128, False), (3, 3, 96, 64, True), (2, 1, 128, 256, False)])
+def test_chunks_of_bfloat16_numbers_that_add_up(H, qh, dim, vdim, normaliser):
+    """Chunks on the bfloat16 matrix cores, 32-bit values as three bfloat16 numbers each: portions that end inside a tile of 16 tokens, a
+    group of 32 and a chunk of 64 and at their edges, beside single tokens, against the recurrence in 64 bits: no further off than
+    the kernels of the 32-bit instruction (a sum in another order: a quarter is allowed)."""
+    from inferrs_amd import ops
+    g = torch.Generator().manual_seed(dim)
+    lens = [64, 1, 128, 17, 33, 47, 65, 79, 16]
+    n, vt = sum(lens), vdim + int(normaliser)
+    q, k, v = (torch.randn(n, w, generator=g).bfloat16() for w in (qh * dim + 8, qh * dim + 16, H * vdim))
+    log_a = -torch.rand(n, H, generator=g) * torch.tensor([0.01, 0.2, 2.0, 0.5])[:H]
+    log_a[40] = -20.0                                      # a token that forgets (nearly) everything
+    b, skip = torch.rand(n, H, generator=g), torch.randn(H, generator=g)
+    start = torch.randn(len(lens) + 1, H * vt * dim + 8, generator=g)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    slots = torch.tensor([3, 0, 1, 2, 4, 5, 6, 7, 9], dtype=torch.int32)
+    Q, K = (x[:, 8:8 + qh * dim].double().view(n, qh, dim).repeat_interleave(H // qh, 1) for x in (q, k))
+    V = torch.cat([v.double().view(n, H, vdim), torch.ones(n, H, 1, dtype=torch.float64)], dim=2)[:, :, :vt]
+    want = torch.zeros(n, H, vt, dtype=torch.float64)
+    final = start.double().clone()
+    for s in range(len(lens)):
+        S = final[slots[s], 8:].view(H, vt, dim)
+        for t in range(int(cu[s]), int(cu[s + 1])):
+            S.mul_(log_a[t].double().exp()[:, None, None]).add_(b[t].double()[:, None, None] * V[t][:, :, None] * (K[t] * 0.7)[:, None, :])
+            want[t] = (S * (Q[t] * 0.3)[:, None, :]).sum(-1)
+    want[:, :, :vdim] += skip.double()[:, None] * V[:, :, :vdim]
+    errors = []
+    for way in (1, 2):
+        state = dev(start.clone())
+        ops.library().ia_linear_scan_tune(way)
+        try:
+            out = ops.linear_scan(q=dev(q), q_off=8, q_heads=qh, k=dev(k), k_off=8, k_heads=qh, v=dev(v), v_off=0, heads=H, dim=dim, vdim=vdim,
+                                  state=state, s_off=8, cu_tokens=dev(cu), state_slots=dev(slots), skip=dev(skip), q_scale=0.3, k_scale=0.7,
+                                  normaliser=normaliser, max_q_len=max(lens), chunk=64, log_a=dev(log_a), b=dev(b))
+        finally:
+            ops.library().ia_linear_scan_tune(1)
+        outs = out if normaliser else (out, None)
+        got = outs[0].cpu().double().view(n, H, vdim)
+        e = [float((got - want[:, :, :vdim]).norm() / want[:, :, :vdim].norm()), float((state.cpu().double() - final).norm() / final.norm())]
+        if normaliser:
+            e.append(float((outs[1].cpu().double() - want[:, :, vdim]).norm() / want[:, :, vdim].norm()))
+        errors.append(e)
+    assert all(new <= 1.25 * old and new < 1e-5 for new, old in zip(*errors)), errors
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_gates_of_long_portions_are_the_walk(dtype):
     from inferrs_amd import ops
