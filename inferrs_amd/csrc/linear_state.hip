@@ -71,6 +71,19 @@ __global__ void conv_act8_kernel(bf16_t* __restrict__ out, const bf16_t* __restr
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] = 0.f;
     }
+    if (k == 4 && t - 3 >= first) {
+        // (four taps, every input in this step: all are asked for before the first is used; 1,500 tokens of 4,352 channels 16.1 -> 13.9 us)
+        float v[4][8], tp[4][8];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            ls_unpack8(x + (long long)(t - 3 + j) * x_ld + x_off + c, v[j]);
+            ls_unpack8(taps + (long long)j * C + c, tp[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[e] = fmaf(tp[j][e], v[j][e], acc[e]);
+    } else
     for (int j = 0; j < k; ++j) {
         const int src = t - (k - 1 - j);
         float v[8], tp[8];
@@ -205,37 +218,72 @@ __global__ __launch_bounds__(EG_THREADS) void exp_gates_block_kernel(
     const int hi = lo + per < last ? lo + per : last;
     float* mp = state + (long long)state_slots[seq] * row_floats + m_off + h;
     const float bi = bias_i[h], bf = bias_f[h];
-    // the run's gates (parked where the results go) and its pair
+    // the run's gates and its pair.  Runs of up to EG_HELD tokens are held in registers, their loads under way together; of
+    // longer ones the gates are parked where the results go (1,500 tokens, all parked: 20.5 us; held 15.2).
+    constexpr int EG_HELD = 8;
+    const bool held = per <= EG_HELD;                            // (the same for all threads)
+    float kept_i[EG_HELD], kept_f[EG_HELD];
     float sum_f = 0.f, top = -INFINITY;
-    for (int t = lo; t < hi; ++t) {
-        const float gi = cap * tanhf((ld(proj + (long long)t * p_ld + i_off + h) + bi) / cap);
-        const float zf = cap * tanhf((ld(proj + (long long)t * p_ld + f_off + h) + bf) / cap);
-        const float gf = -ls_softplus(-zf);
-        log_a[(long long)t * H + h] = gf;
-        b[(long long)t * H + h] = gi;
+    auto gate = [&](float ri, float rf, float& gi, float& gf) {
+        gi = cap * tanhf((ri + bi) / cap);
+        const float zf = cap * tanhf((rf + bf) / cap);
+        gf = -ls_softplus(-zf);
         sum_f += gf;
         top = fmaxf(top + gf, gi);
+    };
+    if (held) {
+#pragma unroll
+        for (int j = 0; j < EG_HELD; ++j) {
+            const int t = lo + j < last ? lo + j : last - 1;     // (behind the run's end: read and not used)
+            kept_i[j] = ld(proj + (long long)t * p_ld + i_off + h);
+            kept_f[j] = ld(proj + (long long)t * p_ld + f_off + h);
+        }
+#pragma unroll
+        for (int j = 0; j < EG_HELD; ++j)
+            if (lo + j < hi) gate(kept_i[j], kept_f[j], kept_i[j], kept_f[j]);
+    } else {
+        for (int t = lo; t < hi; ++t) {
+            float gi, gf;
+            gate(ld(proj + (long long)t * p_ld + i_off + h), ld(proj + (long long)t * p_ld + f_off + h), gi, gf);
+            log_a[(long long)t * H + h] = gf;
+            b[(long long)t * H + h] = gi;
+        }
     }
     sf[threadIdx.x] = sum_f; si[threadIdx.x] = top;
     __syncthreads();
     if (threadIdx.x == 0) {
+        // (sixteen pairs are read at once)
         float m = *mp;
-        for (int i = 0; i < EG_THREADS; ++i) {
-            start[i] = m;
-            m = fmaxf(m + sf[i], si[i]);                         // (an empty run is the pair (0, -inf): m stays)
+        for (int i0 = 0; i0 < EG_THREADS; i0 += 16) {
+            float f[16], g[16], from[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) { f[i] = sf[i0 + i]; g[i] = si[i0 + i]; }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                from[i] = m;
+                m = fmaxf(m + f[i], g[i]);                       // (an empty run is the pair (0, -inf): m stays)
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) start[i0 + i] = from[i];
         }
         *mp = m;
     }
     __syncthreads();
     float m = start[threadIdx.x];
-    for (int t = lo; t < hi; ++t) {
-        const float gf = log_a[(long long)t * H + h], gi = b[(long long)t * H + h];
+    auto put = [&](int t, float gi, float gf) {
         const float m_new = fmaxf(gf + m, gi);
         log_a[(long long)t * H + h] = gf + m - m_new;
         b[(long long)t * H + h] = expf(gi - m_new);
         floor_[(long long)t * H + h] = expf(-m_new);
         m = m_new;
+    };
+    if (held) {
+#pragma unroll
+        for (int j = 0; j < EG_HELD; ++j)
+            if (lo + j < hi) put(lo + j, kept_i[j], kept_f[j]);
+        return;
     }
+    for (int t = lo; t < hi; ++t) put(t, b[(long long)t * H + h], log_a[(long long)t * H + h]);
 }
 
 // max_q_len: an upper bound of the tokens a request brings (steps with long portions take a block a (request, head))
@@ -1281,6 +1329,79 @@ __global__ __launch_bounds__(1024) void group_norm_gate_block_kernel(
     }
 }
 
+// The same where everything comes in pieces of eight features (16-byte accesses): `lanes` threads a (token, group) with ITERS pieces
+// each, a part of a wave up to 64 of them and a whole block beyond.  Every value is read and gated once and stays in registers for
+// the second pass, where the kernels above read and gate it again.  us at 1,500 tokens, before and now: a group of 4,096 gated first
+// 28.3 -> 14.9, 16 groups of 128 and 8 of 256 with a normaliser 13.2 and 16.8 -> 9.4 in the mean.
+__device__ __forceinline__ void gn_load8(const float* p, float (&v)[8]) {
+    const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+__device__ __forceinline__ void gn_load8(const bf16_t* p, float (&v)[8]) { ls_unpack8(p, v); }
+__device__ __forceinline__ void gn_store8(float* p, const float (&v)[8]) {
+    *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
+    *(float4*)(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+}
+__device__ __forceinline__ void gn_store8(bf16_t* p, const float (&v)[8]) {
+    *(uint4*)p = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+}
+template <typename T, int ITERS>
+__global__ __launch_bounds__(512) void group_norm_gate_vec_kernel(
+    T* __restrict__ out, const float* __restrict__ o, const float* __restrict__ den, const float* __restrict__ floor_,
+    int head, const T* __restrict__ gate, long long g_ld, int g_off, int act, int gate_first,
+    const float* __restrict__ w, int w_from, float eps, int inner, int group, long long units, int lanes) {
+    __shared__ float scratch[16];
+    const int per_block = blockDim.x / lanes, of = threadIdx.x / lanes, lane = threadIdx.x - of * lanes;
+    const long long unit = (long long)blockIdx.x * per_block + of;
+    const bool in = unit < units;                          // (nobody returns ahead of the sums)
+    const int per_row = inner / group;
+    const long long t = in ? unit / per_row : 0;
+    const int c0 = in ? (int)(unit - t * per_row) * group : 0;
+    const int H = inner / head;
+    float y[ITERS][8], z[ITERS][8], wv[ITERS][8], over[ITERS];
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        const int e = (lane + it * lanes) * 8, c = c0 + e;
+        over[it] = 1.f;
+        if (!in || e >= group) continue;
+        gn_load8(o + t * inner + c, y[it]);
+        if (gate != nullptr) gn_load8(gate + t * g_ld + g_off + c, z[it]);
+        if (w != nullptr) gn_load8(w + (w_from ? e : c), wv[it]);
+        if (den != nullptr) {
+            const long long at = t * H + c / head;         // (heads of a multiple of eight features)
+            over[it] = fmaxf(fabsf(den[at]), floor_[at]) + 1e-6f;
+        }
+    }
+    float sq = 0.f;
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        if (!in || (lane + it * lanes) * 8 >= group) continue;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (den != nullptr) y[it][i] = y[it][i] / over[it];
+            if (gate != nullptr) z[it][i] = ls_gate(z[it][i], act);
+            if (gate != nullptr && gate_first) y[it][i] *= z[it][i];
+            sq = fmaf(y[it][i], y[it][i], sq);
+        }
+    }
+    if (lanes > IA_WAVE) sq = block_sum(sq, scratch);
+    else
+        for (int s = lanes / 2; s > 0; s >>= 1) sq += __shfl_xor(sq, s, IA_WAVE);
+    const float rs = 1.0f / sqrtf(sq / (float)group + eps);
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        const int e = (lane + it * lanes) * 8, c = c0 + e;
+        if (!in || e >= group) continue;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            y[it][i] *= rs;
+            if (w != nullptr) y[it][i] *= wv[it][i];
+            if (gate != nullptr && !gate_first) y[it][i] *= z[it][i];
+        }
+        gn_store8(out + t * inner + c, y[it]);
+    }
+}
+
 extern "C" int ia_group_norm_gate(void* out, const float* o, const float* den, const float* floor_, int head,
                                   const void* gate, long long g_ld, int g_off, int act, int gate_first, const float* w,
                                   int w_count, float eps, int n, int inner, int group, int dtype, hipStream_t stream) {
@@ -1295,6 +1416,22 @@ extern "C" int ia_group_norm_gate(void* out, const float* o, const float* den, c
     if (n == 0) return 0;
     const long long units = (long long)n * (inner / group);
     IA_CHECK(units < 2147483647LL, "group_norm_gate: %d tokens x %d groups exceed the grid", n, inner / group);
+    if (group % 8 == 0 && inner % 8 == 0 && head % 8 == 0 && (gate == nullptr || (g_ld % 8 == 0 && g_off % 8 == 0)) && group <= 8192 &&
+        (((uintptr_t)out | (uintptr_t)o | (uintptr_t)gate | (uintptr_t)w) & 15) == 0) {
+        // threads a group: enough for its pieces, a power of two inside a wave; two pieces each in blocks (of up to 512 threads)
+        int lanes = 1;
+        while (lanes < 64 && lanes * 8 < group) lanes *= 2;
+        if (group > 512) lanes = (group / 8 + 127) / 128 * 64;
+        const int threads = lanes > 64 ? lanes : 256;
+        const unsigned blocks = (unsigned)((units + threads / lanes - 1) / (threads / lanes));
+#define GN_LAUNCH(T, ITERS) group_norm_gate_vec_kernel<T, ITERS><<<blocks, threads, 0, stream>>>((T*)out, o, den, floor_, head, (const T*)gate, g_ld, \
+                                                                          g_off, act, gate_first, w, w_from, eps, inner, group, units, lanes)
+        if (dtype == IA_F32) { if (lanes * 8 >= group) GN_LAUNCH(float, 1); else GN_LAUNCH(float, 2); }
+        else { if (lanes * 8 >= group) GN_LAUNCH(bf16_t, 1); else GN_LAUNCH(bf16_t, 2); }
+#undef GN_LAUNCH
+        IA_LAUNCH_CHECK("group_norm_gate (pieces)");
+        return 0;
+    }
     if (group > 256) {
         // (four features a thread where the group is wide enough: steps of few tokens have few blocks, and a block's
         // walk over its group is what they wait for)

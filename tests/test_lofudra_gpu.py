@@ -599,3 +599,37 @@ def test_trace_runner_program(models, tmp_path):
     assert [l for l in p.stdout.splitlines() if l.startswith("done")] == [f"done {i}" for i in range(len(trace.lines))]
     err, where = worst(trace.read(out_dir, cfg["vocab"]), ref, some)
     assert err <= TOL_F32, (err, where)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("group,groups,head,gate_first,normaliser", [
+    (8, 3, 8, False, False), (64, 5, 64, True, False), (200, 3, 40, False, True), (256, 8, 256, False, True), (264, 2, 8, True, True),
+    (512, 2, 64, True, False), (520, 1, 104, False, False), (1032, 3, 24, True, False), (4096, 1, 64, True, False), (8192, 1, 128, False, False)])
+def test_group_norm_in_pieces(group, groups, head, gate_first, normaliser, dtype):
+    """Groups of one piece of eight features up to the widest that goes in pieces, against 64 bits; 32-bit sums of at most 8,192
+    squares, an exponential and a few products: 1e-5 of the largest value in 32-bit, one rounding in bfloat16."""
+    from inferrs_amd import ops
+    g = torch.Generator().manual_seed(group)
+    n, inner = 7, group * groups
+    o = torch.randn(n, inner, generator=g)
+    gate = torch.randn(n, inner + 24, generator=g).to(dtype)
+    den, floor = torch.randn(n, inner // head, generator=g), torch.rand(n, inner // head, generator=g) + 0.1
+    for w in (None, torch.randn(group, generator=g), torch.randn(inner, generator=g)):
+        y = o.double()
+        if normaliser:
+            y = y / (torch.maximum(den.abs(), floor).double() + 1e-6).repeat_interleave(head, 1)
+        z = gate[:, 16:16 + inner].double()
+        z = z * torch.sigmoid(z)
+        if gate_first:
+            y = y * z
+        y = y.view(n, groups, group)
+        y = (y / torch.sqrt(y.pow(2).mean(-1, keepdim=True) + 1e-5)).reshape(n, inner)
+        if w is not None:
+            y = y * (w if w.numel() == inner else w.repeat(groups)).double()
+        if not gate_first:
+            y = y * z
+        got = ops.group_norm_gate(dev(o), group=group, head=head, eps=1e-5, out_dtype=dtype, weight=None if w is None else dev(w), gate=dev(gate),
+                                  gate_off=16, act=ops.state.ACT_SILU, gate_first=gate_first, den=dev(den) if normaliser else None,
+                                  floor=dev(floor) if normaliser else None).cpu().double()
+        bound = 1e-5 * float(y.abs().max()) + (2 ** -8 * y.abs() if dtype == torch.bfloat16 else 0)
+        assert bool(((got - y).abs() <= bound).all()), float((got - y).abs().max())
