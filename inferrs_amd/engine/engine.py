@@ -46,6 +46,7 @@ _PAD = ("inferrs_amd", "rows that fill a decode step")
 
 class Engine:
     GRAPH_BUCKET_TOKENS = 1024      # a captured step serves context lengths up to a multiple of this
+    GRAPH_SHORT_TOKENS = 512        # portions whose contexts are no longer than this are bounded by it
     GRAPH_MAX_TOKENS = 1024         # steps of more tokens run eagerly: their kernels outlast the host, and a graph would hold their buffers
     MAX_GRAPHS = 48                 # captured graphs kept (the one replayed longest ago goes first)
     MAX_SHAPES_SEEN = 512           # shapes remembered as seen, with what was measured of them
@@ -367,7 +368,14 @@ class Engine:
             # (a portion's keys are not split at up to 2,048: its first two buckets have the same launches)
             ctx.max_kv_single = self._run_bound(longest_single, bucket, widest)
             ctx.max_kv_multi = self._run_bound(longest_multi, bucket, widest, least=2)
+            if longest_multi <= self.GRAPH_SHORT_TOKENS:
+                ctx.max_kv_multi = min(self.GRAPH_SHORT_TOKENS, widest)
             key += (ctx.max_kv_single, ctx.max_kv_multi)
+        elif ctx.n_single == 0 and longest <= self.GRAPH_SHORT_TOKENS < pad_pages * self.page_size:
+            # (few tokens behind a short context are not worth a split of their keys, which a bucket's bound would have: 40 tokens of
+            # two query heads a key head 7.6 us a layer whole, 15.8 split for 1,024)
+            ctx.max_kv_len = self.GRAPH_SHORT_TOKENS
+            key += (ctx.max_kv_len,)
         entry = self._graphs.get(key)
         if entry is not None:
             self._graphs.move_to_end(key)

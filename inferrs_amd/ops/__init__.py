@@ -541,6 +541,7 @@ ATTN_TILE_COLS = 128           # head size 128, prompt portions: columns a block
 ATTN_TILE_BLOCKS = 256         # compute units: a block's eight waves fill one
 ATTN_TILE_MIN_CHUNK = 512      # fewest keys a block's share is worth (eight stages of 64)
 ATTN_TILE_WHOLE_UP_TO = 2048   # contexts up to this length are not split
+ATTN_TILE_FEW_UP_TO = 512     # fewer columns than a block has: keys that one walk takes whole
 
 
 def attention_split(n_seqs: int, nkv: int, g: int, max_q_len: int, max_kv_len: int, d: int = 0) -> Tuple[int, int]:
@@ -578,6 +579,10 @@ def attention_split(n_seqs: int, nkv: int, g: int, max_q_len: int, max_kv_len: i
                 best, splits = cost, ways
         chunk = -(-max_kv_len // splits)
         return splits, -(-chunk // 64) * 64
+    if d == 128 and cols > 16 and max_kv_len <= ATTN_TILE_FEW_UP_TO and n_seqs * nkv * -(-cols // 64) <= ATTN_TILE_BLOCKS:
+        # few columns in one round of blocks that share their keys: whole (40 tokens behind 100, two query heads a key head, 12.8 us
+        # in two splits of single waves, 7.6 whole; 20 tokens behind 450 12.1 in four, 10.5 whole; 177 sizes 1.06 to 2.39 times as fast)
+        return 1, -(-max_kv_len // 64) * 64
     col_blocks = 1 if cols <= 16 else -(-cols // 32)
     items = n_seqs * nkv * col_blocks
     splits = 1

@@ -872,6 +872,27 @@ def test_attention_decode_fused_is_the_three_kernels_in_one(nq, nkv, d, page, wi
         assert counters is None or int(counters.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("nq,nkv,qs,window", [(16, 8, [9, 60, 1, 17], None), (32, 8, [31, 5, 20], 40), (17, 1, [1, 7], None), (4, 4, [63, 17, 64], 100)])
+def test_portions_of_few_columns_share_their_keys(nq, nkv, qs, window):
+    """Portions of 17 to 127 columns a key head and shorter ones beside them, behind contexts up to where the rule keeps keys whole, in
+    blocks of four waves against the kernel of single waves (the same keys in the same tiles of 32, sums in another order)."""
+    from inferrs_amd import ops
+    d, page = 128, 16
+    lens = [q + c for q, c in zip(qs, (0, 130, 448, 65))]
+    q, kc, vc, positions, token_seq, table = attention_case(torch.bfloat16, nq, nkv, d, page, lens, qs, 31)
+    cu = torch.tensor([0] + torch.tensor(qs).cumsum(0).tolist(), dtype=torch.int32)
+    assert ops.attention_split(len(qs), nkv, nq // nkv, max(qs), max(lens), d)[0] == 1
+    lib, outs = ops.library("attn_d128"), []
+    for tiles in (1, 0):
+        lib.ia_attention_mfma_tiles(tiles)
+        try:
+            outs.append(ops.attention_mfma(dev(q), dev(kc), dev(vc), dev(positions), dev(cu), dev(table), max_q_len=max(qs),
+                                           max_kv_len=max(lens), window=window, scale=d ** -0.5).float().cpu())
+        finally:
+            lib.ia_attention_mfma_tiles(1)
+    close(outs[0], outs[1], 2 ** -7, "few columns")
+
+
 @pytest.mark.parametrize("nq,nkv,d,dv_,page,window,mask_chunk,rot,gate,own", [
     (16, 4, 128, 64, 16, 40, None, 64, "feature", True),       # values narrower than keys, half of a head rotating
     (16, 4, 128, 64, 16, 300, None, 64, "feature", False),     # a layer that reads another's cache: rows [q | g]
