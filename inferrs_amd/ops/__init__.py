@@ -624,23 +624,30 @@ def decode_split(n_seqs: int, nkv: int, g: int, max_kv_len: int) -> Tuple[int, i
 
 @functools.lru_cache(maxsize=4096)
 def decode_shares(n_seqs: int, nkv: int, g: int, max_kv_len: int) -> Tuple[int, int]:
-    """(splits, keys per split) that a decode step takes: `decode_split`'s, but for three counts beside its powers of two that were
-    faster (us, 8 key/value heads, 16 to 64 query heads): twelve for eight where that still is one round of the chip (9 requests at
-    2,048 keys 17.3 -> 14.9, at 8,192 43.5 -> 36.2); one block of three waves for one of four (24 requests at 1,024 keys 16.2 ->
-    15.3, at 2,048 26.7 -> 24.6); and 48 for 32 at one or two
-    requests of 3,072 to 4,095 keys (11.9 -> 10.6).  Of 480 points longer than 512 keys that these rules decide or leave, none is slower
-    than 0.945 of the former's speed."""
+    """(splits, keys per split) that a decode step takes: `decode_split`'s, but for other counts where they were faster over contexts of
+    8 to 97 % of the bound up to 1,024 keys and 55 to 97 % of longer ones (a step's bound is a bucket's, and batches of more than eight hold
+    contexts from a third of the longest; in the mean over 8 key/value heads of 2 and 4 query heads and 4 of 4):
+    a round's worth of waves that eight splits leave idle goes to twelve (9 and 10 requests of 8 key heads at 2,048 keys 1.11, 3,072 1.18,
+    8,192 1.21); up to 1,024 keys four splits meet in one block where eight are handed over between two (10 to 16 requests 1.09 to 1.15);
+    blocks of three waves for four where nearly the whole round is taken, at 3,072 keys and more (28 and 32 requests 1.01 to 1.04); one or two
+    requests of 3,072 to 4,096 keys take 48 and 64 splits for 32 (1.05 to 1.13, 1.02 to 1.11), three or four of 3,072 to 4,095 or 8,192 and
+    more 28 (1.10 to 1.15, 1.10)."""
     splits, chunk = decode_split(n_seqs, nkv, g, max_kv_len)
     items = n_seqs * nkv * -(-g // 16)
-    if splits == 4 and max_kv_len > 512:
-        splits = 3
-    elif splits == 8 and items * 12 <= DECODE_WAVES and max_kv_len >= 12 * DECODE_MIN_CHUNK:
-        splits = 12
-    elif splits == 32 and items <= 16 and 48 * DECODE_MIN_CHUNK <= max_kv_len < 4096:
-        splits = 48
-    else:
+    other = splits
+    if splits == 8 and 512 < max_kv_len <= 1024:
+        other = 4
+    elif splits == 8 and items * 12 <= DECODE_WAVES and max_kv_len >= 2048:
+        other = 12
+    elif splits == 4 and items >= 224 and max_kv_len >= 3072:
+        other = 3
+    elif splits == 32 and items <= 16 and 3072 <= max_kv_len <= 4096:
+        other = 64 if max_kv_len == 4096 else 48
+    elif splits == 32 and 16 < items <= 36 and (3072 <= max_kv_len < 4096 or max_kv_len >= 8192):
+        other = 28
+    if other == splits:
         return splits, chunk
-    return splits, -(-(-(-max_kv_len // splits)) // 32) * 32
+    return other, -(-(-(-max_kv_len // other)) // 32) * 32
 
 
 def attention_mfma(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
