@@ -795,11 +795,11 @@ __global__ __launch_bounds__(256) void linear_local_mfma_kernel(const ScanArgs a
 // q, k and v are bfloat16 values, so every product q.k is exact there and only its sums are 32-bit, as they were.  What is 32-bit
 // on one side (weighted scores, weighted values, the matrix a chunk starts from) goes in as three bfloat16 numbers that add up to
 // it exactly (eight bits of its 24 each): three products on an instruction that multiplies sixteen times as much a cycle as the
-// 32-bit one.  Errors against 64 bits, 20 sizes: 0.52 to 1.02 of the 32-bit kernels', 0.87 in the mean.  The walk over a chunk comes in two kernels with
+// 32-bit one.  Errors against 64 bits, 20 sizes: 0.47 to 1.15 of the 32-bit kernels', 0.86 in the mean.  The walk over a chunk comes in two kernels with
 // `chunk_states_kernel` between them: the chunk's own matrix U alone, and then every output at once, from the chunk's tokens and from
 // the matrix it starts from, so that outputs are written once and not read again.  What bounded the 32-bit kernels: their instruction
 // (a third of the time) and one operand read of 4 bytes a lane for each of its steps.  us, the three kernels, before and now (1,500
-// tokens): 64 heads of 128 x 64 152 -> 73, 8 of 128 x 256 with a normaliser 98 -> 47, 16 of 64 x 128 58 -> 35; 300 tokens 56 -> 33, 41 -> 24, 28 -> 18.
+// tokens): 64 heads of 128 x 64 152 -> 74, 8 of 128 x 256 with a normaliser 98 -> 47, 16 of 64 x 128 58 -> 35; 300 tokens 56 -> 33, 41 -> 24, 28 -> 18.
 #define LX_LD 72                        // bfloat16 values of a staged row of 64 tokens: 16 rows' 16-byte pieces fall on different banks
 typedef __bf16 ls_bf16x8 __attribute__((ext_vector_type(8)));
 
@@ -809,7 +809,8 @@ __device__ __forceinline__ ls_f32x4 lx_mfma(const uint4& x, const uint4& y, cons
 // x = part 0 + part 1 + part 2 exactly, each in the upper half of its word: the leading eight bits, those behind them, the rest
 __device__ __forceinline__ void lx_split(float x, uint32_t (&part)[3]) {
     part[0] = __float_as_uint(x) & 0xffff0000u;
-    const float rest = x - __uint_as_float(part[0]);
+    // (an infinity less itself is no number: the smaller of that and a bound above every rest keeps the products infinite)
+    const float rest = fminf(x - __uint_as_float(part[0]), 0x1p120f);
     part[1] = __float_as_uint(rest) & 0xffff0000u;
     part[2] = __float_as_uint(rest - __uint_as_float(part[1]));
 }

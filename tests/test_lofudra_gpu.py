@@ -394,6 +394,37 @@ def test_chunks_of_bfloat16_numbers_that_add_up(H, qh, dim, vdim, normaliser):
     assert all(new <= 1.25 * old and new < 1e-5 for new, old in zip(*errors)), errors
 
 
+@pytest.mark.parametrize("where", ["state", "values", "nan"])
+def test_chunks_keep_infinities(where):
+    """One infinite entry of the state, one infinite value, one entry that is no number: the chunks on the bfloat16 matrix cores give finite
+    numbers, infinities and no numbers in the same places as those of the 32-bit instruction."""
+    from inferrs_amd import ops
+    g = torch.Generator().manual_seed(5)
+    H, dim, vdim, n = 2, 64, 64, 150
+    q, k, v = (torch.randn(n, H * w, generator=g).bfloat16() for w in (dim, dim, vdim))
+    start = torch.randn(1, H * vdim * dim, generator=g)
+    if where == "values":
+        v[70, 3] = -float("inf")
+    else:
+        start[0, 5 * dim + 9] = float("inf") if where == "state" else float("nan")
+    got = []
+    for way in (1, 2):
+        state = dev(start.clone())
+        ops.library().ia_linear_scan_tune(way)
+        try:
+            out = ops.linear_scan(q=dev(q), q_off=0, q_heads=H, k=dev(k), k_off=0, k_heads=H, v=dev(v), v_off=0, heads=H, dim=dim, vdim=vdim,
+                                  state=state, s_off=0, cu_tokens=dev(torch.tensor([0, n], dtype=torch.int32)),
+                                  state_slots=dev(torch.zeros(1, dtype=torch.int32)), skip=dev(torch.zeros(H)), q_scale=0.3, k_scale=0.7,
+                                  normaliser=False, max_q_len=n, chunk=64, log_a=dev(torch.full((n, H), -0.01)), b=dev(torch.ones(n, H)))
+        finally:
+            ops.library().ia_linear_scan_tune(1)
+        got.append((out.float().cpu(), state.cpu()))
+    for new, old in zip(*got):
+        assert bool((new.isfinite() == old.isfinite()).all()) and bool((new.isnan() == old.isnan()).all())
+        assert bool((new[new.isinf()] == old[old.isinf()]).all())
+    assert where == "nan" or got[0][1].isinf().any()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_gates_of_long_portions_are_the_walk(dtype):
     from inferrs_amd import ops
