@@ -46,7 +46,7 @@ _PAD = ("inferrs_amd", "rows that fill a decode step")
 
 class Engine:
     GRAPH_BUCKET_TOKENS = 1024      # a captured step serves context lengths up to a multiple of this
-    GRAPH_SHORT_TOKENS = 512        # portions whose contexts are no longer than this are bounded by it
+    GRAPH_SHORT_TOKENS = 512        # portions of few columns whose contexts are no longer than this are bounded by it
     GRAPH_MAX_TOKENS = 1024         # steps of more tokens run eagerly: their kernels outlast the host, and a graph would hold their buffers
     MAX_GRAPHS = 48                 # captured graphs kept (the one replayed longest ago goes first)
     MAX_SHAPES_SEEN = 512           # shapes remembered as seen, with what was measured of them
@@ -86,6 +86,7 @@ class Engine:
         # Decode steps (one token a request) and steps of few tokens are bound by their launches: each distinct
         # shape is captured into a HIP graph the second time it is seen and replayed from then on.
         self.use_graphs = use_graphs and model.graph_safe
+        self._portion_heads = {(*p.portion_heads, p.spec.head_dim) for p in model.all_parts() if getattr(p, "portion_heads", None)}
         self.unused_tensors: List[str] = []
         self.stop_token_ids: Tuple[int, ...] = tuple(model.spec.eos_token_ids)
         # a part that will run off its fast path says so once, here, and not at every step
@@ -240,6 +241,11 @@ class Engine:
         bucket_pages = max(1, self.GRAPH_BUCKET_TOKENS // self.page_size)
         return -(-(-(-longest // self.page_size)) // bucket_pages) * bucket_pages
 
+    def _few_columns(self, ctx) -> bool:
+        """Whether some layer's portions of this step run on other blocks where their contexts are known to be short (other steps are
+        bounded by their bucket alone: a bound of its own is a shape of its own, two eager steps and a capture more)."""
+        return any(ops.attention_few_columns(ctx.n_seqs - ctx.n_single, nkv, g, ctx.max_q_len, d) for nkv, g, d in self._portion_heads)
+
     @staticmethod
     def _run_bound(longest: int, bucket_tokens: int, widest: int, least: int = 1) -> int:
         """The tokens that bound one run's launches in a step of portions beside single tokens whose longer run is bounded by
@@ -368,10 +374,10 @@ class Engine:
             # (a portion's keys are not split at up to 2,048: its first two buckets have the same launches)
             ctx.max_kv_single = self._run_bound(longest_single, bucket, widest)
             ctx.max_kv_multi = self._run_bound(longest_multi, bucket, widest, least=2)
-            if longest_multi <= self.GRAPH_SHORT_TOKENS:
+            if longest_multi <= self.GRAPH_SHORT_TOKENS and self._few_columns(ctx):
                 ctx.max_kv_multi = min(self.GRAPH_SHORT_TOKENS, widest)
             key += (ctx.max_kv_single, ctx.max_kv_multi)
-        elif ctx.n_single == 0 and longest <= self.GRAPH_SHORT_TOKENS < pad_pages * self.page_size:
+        elif ctx.n_single == 0 and longest <= self.GRAPH_SHORT_TOKENS < pad_pages * self.page_size and self._few_columns(ctx):
             # (few tokens behind a short context are not worth a split of their keys, which a bucket's bound would have: 40 tokens of
             # two query heads a key head 7.6 us a layer whole, 15.8 split for 1,024)
             ctx.max_kv_len = self.GRAPH_SHORT_TOKENS

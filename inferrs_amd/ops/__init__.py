@@ -544,6 +544,12 @@ ATTN_TILE_WHOLE_UP_TO = 2048   # contexts up to this length are not split
 ATTN_TILE_FEW_UP_TO = 512     # fewer columns than a block has: keys that one walk takes whole
 
 
+def attention_few_columns(n_seqs: int, nkv: int, g: int, max_q_len: int, d: int) -> bool:
+    """Whether portions of so many tokens have fewer columns than a block of the kernel that shares keys between its waves, and run
+    there in one round of blocks where their contexts are short."""
+    return d == 128 and 16 < max_q_len * g < ATTN_TILE_COLS and n_seqs * nkv * -(-max_q_len * g // 64) <= ATTN_TILE_BLOCKS
+
+
 def attention_split(n_seqs: int, nkv: int, g: int, max_q_len: int, max_kv_len: int, d: int = 0) -> Tuple[int, int]:
     """(splits, keys per split) for the matrix-core kernel: the keys are split between waves
     when the batch alone has too few (request, kv head, column block) items to fill the chip."""
@@ -579,7 +585,7 @@ def attention_split(n_seqs: int, nkv: int, g: int, max_q_len: int, max_kv_len: i
                 best, splits = cost, ways
         chunk = -(-max_kv_len // splits)
         return splits, -(-chunk // 64) * 64
-    if d == 128 and cols > 16 and max_kv_len <= ATTN_TILE_FEW_UP_TO and n_seqs * nkv * -(-cols // 64) <= ATTN_TILE_BLOCKS:
+    if max_kv_len <= ATTN_TILE_FEW_UP_TO and attention_few_columns(n_seqs, nkv, g, max_q_len, d):
         # few columns in one round of blocks that share their keys: whole (40 tokens behind 100, two query heads a key head, 12.8 us
         # in two splits of single waves, 7.6 whole; 20 tokens behind 450 12.1 in four, 10.5 whole; 177 sizes 1.06 to 2.39 times as fast)
         return 1, -(-max_kv_len // 64) * 64

@@ -112,6 +112,7 @@ class Attention(Mixer):
         if spec.v_mix not in (None, "first", "mix") or (spec.v_mix and not spec.own_kv):
             raise SpecError(f"attention: v_mix {spec.v_mix!r} is 'first' or 'mix', in a layer with values of its own")
         self.spec = spec
+        self.portion_heads = (spec.n_kv_heads, spec.n_heads // spec.n_kv_heads) if dtype == torch.bfloat16 else None
         named = dict(spec.names or ())
         tensors = {k: tensors[named.get(k, k)] for k in self._tensors(spec) if named.get(k, k) in tensors}
         # rows of the plain layout [q | k | v], heads of one width, go through the kernels made for it; everything else
