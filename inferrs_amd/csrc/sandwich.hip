@@ -162,8 +162,30 @@ extern "C" int ia_sandwich_step(float* x, const void* y1, float s1, const void* 
     return 0;
 }
 
-__device__ __forceinline__ float act_value(float z, int act) {
-    return act == 3 ? 0.5f * z * (1.0f + erff(z * 0.7071067811865476f)) : gate_act(z, act);
+// The exact GELU of a value that is stored in 16 bits: max(z, 0) - |z| / 2 erfc(|z| / sqrt 2), erfc(|z| / sqrt 2) = exp(-z^2 / 2) t P(t),
+// t = 1 / (1 + 0.26 |z|), P a polynomial fitted to exp(z^2 / 2) erfc(|z| / sqrt 2) / t in 64 bits up to |z| = 14 (least squares, reweighted
+// towards the smallest largest relative error: 2.5e-8).  z^2 is exact, no branch, and nothing cancels: of all bfloat16 values those above -4 give
+// the bits of the formula with erff, those below are right where 1 + erff had lost them (a third of the value off between -6 and
+// -4 in the mean).  erff's two branches, which a wave takes both, were what bounded the pass.  An infinity gives what the formula gives.
+__device__ __forceinline__ float gelu_for_bf16(float z) {
+    const float a = fminf(fabsf(z), 64.0f);                  // (beyond: erfc is 0; a product of infinity and 0 would be no number)
+    const float t = __builtin_amdgcn_rcpf(fmaf(0.26f, a, 1.0f));
+    float p = 0.06100985f;
+    p = fmaf(p, t, -0.30565804f);
+    p = fmaf(p, t, 0.50298333f);
+    p = fmaf(p, t, -0.30189878f);
+    p = fmaf(p, t, 0.32189628f);
+    p = fmaf(p, t, 0.10205514f);
+    p = fmaf(p, t, 0.20606056f);
+    p = fmaf(p, t, 0.2060335f);
+    p = fmaf(p, t, 0.20751812f);
+    return fmaf(0.5f, z, 0.5f * fabsf(z)) - 0.5f * a * t * p * __builtin_amdgcn_exp2f(a * a * -0.72134752f);
+}
+template <typename T>
+__device__ __forceinline__ float act_stored(float z, int act) {
+    if (act != 3) return gate_act(z, act);
+    if constexpr (sizeof(T) == 2) return gelu_for_bf16(z);
+    else return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));
 }
 
 // An activation over every element, in place.  act: 1 SiLU, 2 GELU in its tanh form, 3 the exact GELU,
@@ -173,18 +195,19 @@ __global__ void activation_kernel(T* __restrict__ x, long long n, int act) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float z = ld(x + i);
-    st(x + i, act_value(z, act));
+    st(x + i, act_stored<T>(z, act));
 }
 
-// Eight neighbouring bfloat16 values a thread (16-byte accesses), for arrays of a multiple of eight elements.
-__global__ void activation8_kernel(bf16_t* __restrict__ x, long long n8, int act) {
+// Eight neighbouring bfloat16 values a thread (16-byte accesses), for arrays of a multiple of eight elements.  GELU, 1,500 rows of 8,192: 14.2 -> 11.8 us (4.2 TB/s).
+template <int ACT>
+__global__ void activation8_kernel(bf16_t* __restrict__ x, long long n8) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n8) return;
     uint4 q = *reinterpret_cast<const uint4*>(x + 8 * i);
     uint32_t* w = reinterpret_cast<uint32_t*>(&q);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-        w[e] = pack_bf16x2(act_value(__uint_as_float(w[e] << 16), act), act_value(__uint_as_float(w[e] & 0xffff0000u), act));
+        w[e] = pack_bf16x2(act_stored<bf16_t>(__uint_as_float(w[e] << 16), ACT), act_stored<bf16_t>(__uint_as_float(w[e] & 0xffff0000u), ACT));
     *reinterpret_cast<uint4*>(x + 8 * i) = q;
 }
 
@@ -192,7 +215,10 @@ extern "C" int ia_activation(void* x, long long n, int act, int dtype, hipStream
     IA_CHECK(n >= 0 && act >= 1 && act <= 3, "activation: n=%lld act=%d (1 SiLU, 2 GELU tanh, 3 GELU)", n, act);
     if (n == 0) return 0;
     if (dtype != IA_F32 && n % 8 == 0 && ((uintptr_t)x & 15) == 0) {
-        activation8_kernel<<<(unsigned)((n / 8 + 255) / 256), 256, 0, stream>>>((bf16_t*)x, n / 8, act);
+        const unsigned grid = (unsigned)((n / 8 + 255) / 256);
+        if (act == 1) activation8_kernel<1><<<grid, 256, 0, stream>>>((bf16_t*)x, n / 8);
+        else if (act == 2) activation8_kernel<2><<<grid, 256, 0, stream>>>((bf16_t*)x, n / 8);
+        else activation8_kernel<3><<<grid, 256, 0, stream>>>((bf16_t*)x, n / 8);
         IA_LAUNCH_CHECK("activation");
         return 0;
     }

@@ -80,6 +80,23 @@ def test_exact_gelu(dtype):
     np.testing.assert_allclose(got.numpy(), pl.gelu_erf(z.double()).numpy(), rtol=1e-2 if dtype == torch.bfloat16 else 1e-5, atol=2e-3 if dtype == torch.bfloat16 else 1e-6)
 
 
+def test_exact_gelu_of_every_bfloat16_value():
+    """Every value that bfloat16 has, in pieces of eight and one by one: half a unit in the last place from the function in 64 bits (2^-8 of it: eight bits), and
+    1e-5 for the 32-bit steps before (the exponential's argument, up to 86, carries 2^-24 of itself); results under the smallest normal number may
+    be 0."""
+    from inferrs_amd import ops
+    z = torch.arange(-(1 << 15), 1 << 15).to(torch.int16).view(torch.bfloat16)
+    got = ops.activation(dev(z.clone()), ops.state.ACT_GELU).cpu()
+    one = ops.activation(dev(z[1:].clone()), ops.state.ACT_GELU).cpu()
+    assert torch.equal(got[1:].view(torch.int16), one.view(torch.int16))
+    x = z.double()
+    want = x.clamp(min=0) - 0.5 * x.abs() * torch.special.erfc(x.abs() / 2 ** 0.5)
+    finite = x.isfinite()
+    off = (got.double() - want).abs()[finite]
+    assert bool((off <= (2.0 ** -8 + 1e-5) * want.abs()[finite] + 2.0 ** -126).all())
+    assert bool(got[x.isnan() | (x == -float("inf"))].isnan().all()) and bool((got[x == float("inf")] == float("inf")).all())
+
+
 # ---- the softmax with a sink, at a window's edge ------------------------------------------------------
 
 def sink_reference(q, kc, vc, positions, token_seq, table, window, scale):
