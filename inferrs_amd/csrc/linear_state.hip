@@ -795,11 +795,11 @@ __global__ __launch_bounds__(256) void linear_local_mfma_kernel(const ScanArgs a
 // q, k and v are bfloat16 values, so every product q.k is exact there and only its sums are 32-bit, as they were.  What is 32-bit
 // on one side (weighted scores, weighted values, the matrix a chunk starts from) goes in as three bfloat16 numbers that add up to
 // it exactly (eight bits of its 24 each): three products on an instruction that multiplies sixteen times as much a cycle as the
-// 32-bit one.  Errors against 64 bits, 20 sizes: 0.47 to 1.15 of the 32-bit kernels', 0.86 in the mean.  The walk over a chunk comes in two kernels with
+// 32-bit one.  Errors against 64 bits: those of the walk, a quarter more at most, whatever the decays (see `lx_gates`).  The walk over a chunk comes in two kernels with
 // `chunk_states_kernel` between them: the chunk's own matrix U alone, and then every output at once, from the chunk's tokens and from
 // the matrix it starts from, so that outputs are written once and not read again.  What bounded the 32-bit kernels: their instruction
 // (a third of the time) and one operand read of 4 bytes a lane for each of its steps.  us, the three kernels, before and now (1,500
-// tokens): 64 heads of 128 x 64 152 -> 74, 8 of 128 x 256 with a normaliser 98 -> 47, 16 of 64 x 128 58 -> 35; 300 tokens 56 -> 33, 41 -> 24, 28 -> 18.
+// tokens): 64 heads of 128 x 64 152 -> 74, 8 of 128 x 256 with a normaliser 98 -> 48, 16 of 64 x 128 58 -> 36; 300 tokens 56 -> 33, 41 -> 24, 28 -> 18.
 #define LX_LD 72                        // bfloat16 values of a staged row of 64 tokens: 16 rows' 16-byte pieces fall on different banks
 typedef __bf16 ls_bf16x8 __attribute__((ext_vector_type(8)));
 
@@ -829,20 +829,27 @@ __device__ __forceinline__ void lx_split8(const float (&x)[8], uint4 (&part)[3])
     for (int p = 0; p < 3; ++p) part[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
 }
 // A wave's lanes as the chunk's 64 tokens: the sums of the decays' logarithms up to each (g), the input scales (b) and, where `run`
-// is asked for, the products of the decays.
-__device__ __forceinline__ void lx_gates(const ScanArgs& a, int h, int first, int nt, int tt, float& g, float& b, float* run) {
-    g = 0.f;
+// is asked for, the products of the decays.  The sums are 64-bit: what one token weighs for another is the difference of two sums, and a
+// 32-bit sum behind a strong forget no longer holds the mild decays that follow it.  Errors against 64 bits of 33 tokens, 128 x 64, with 32-bit
+// sums / 64-bit ones / by the walk, which multiplies decays: logarithms down to -32 1.4e-6 / 7.6e-8 / 8.6e-8, one of -1,000 among mild
+// ones 1.5e-5 / 1.1e-7 / 9.4e-8, decays of 0 3.6e-4 / 1.1e-7 / 9.0e-8; they cost 0.5 to 1 us of the three kernels' time (64 heads of 128 x 64,
+// 100 tokens 21.4 -> 22.1 us, 1,500 tokens 73.1 -> 74.3).  Powers of a negative constant alternate: b carries the token's sign, its reader
+// multiplies by that of the place it weighs for.
+__device__ __forceinline__ void lx_gates(const ScanArgs& a, int h, int first, int nt, int tt, double& g, float& b, float* run) {
+    g = 0.0;
     b = 0.f;
     float r = 1.f;
     if (tt < nt) {
         const float an = a.log_a[a.a_per_token ? (long long)(first + tt) * a.H + h : h];
-        g = fmaxf(a.a_per_token ? an : logf(an), -1e4f);
+        const float log_an = a.a_per_token ? an : logf(fabsf(an));
+        g = log_an < -1e4f ? -1e4f : log_an;               // (a decay of 0 has a logarithm whose differences stay numbers; what is no number stays none)
         r = a.a_per_token ? expf(an) : an;
         b = a.b != nullptr ? a.b[(long long)(first + tt) * a.H + h] : 1.f;
+        if (!a.a_per_token && an < 0.f && (tt & 1)) b = -b;
     }
 #pragma unroll
     for (int o = 1; o < LC_TOKENS; o <<= 1) {
-        const float before = __shfl_up(g, o, IA_WAVE);
+        const double before = __shfl_up(g, o, IA_WAVE);
         if (tt >= o) g += before;
     }
     if (run == nullptr) return;
@@ -852,6 +859,9 @@ __device__ __forceinline__ void lx_gates(const ScanArgs& a, int h, int first, in
         if (tt >= o) r *= before;
     }
     *run = r;
+}
+__device__ __forceinline__ bool lx_alternates(const ScanArgs& a, int h, int place) {
+    return !a.a_per_token && a.log_a[h] < 0.f && (place & 1);
 }
 
 // U = sum_s exp(G_last - G_s) b_s k_s v_s^T over a chunk, for 64 columns of v: keys and weighted values lie feature by feature in shared
@@ -876,12 +886,17 @@ __global__ __launch_bounds__(256) void linear_chunk_matrix_kernel(const ScanArgs
     for (int i = 0; i < KS; ++i) kp[i] = *(const uint4*)(k + (wave + 4 * i) * 8);
 #pragma unroll
     for (int i = 0; i < 2; ++i) vp[i] = *(const uint4*)(v + (wave + 4 * i) * 8);
-    float g, b;
+    double g;
+    float b;
     lx_gates(a, h, first, nt, lane, g, b, nullptr);
-    const float g_last = __shfl(g, LC_TOKENS - 1, IA_WAVE);
-    const float w = lane < nt ? expf(g_last - g) * b * a.k_scale : 0.f;      // (tokens that the chunk does not have weigh nothing)
+    const double g_last = __shfl(g, LC_TOKENS - 1, IA_WAVE);
+    if (lx_alternates(a, h, nt - 1)) b = -b;
+    const float w = lane < nt ? expf((float)(g_last - g)) * b * a.k_scale : 0.f;      // (tokens that the chunk does not have weigh nothing)
     if (wave == 0) w_s[lane] = w;
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.chunk_a[(long long)blockIdx.z * a.H + h] = expf(g_last);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        const float all = expf((float)g_last);
+        a.chunk_a[(long long)blockIdx.z * a.H + h] = lx_alternates(a, h, nt) ? -all : all;
+    }
 #pragma unroll
     for (int i = 0; i < KS; ++i) {
         const uint32_t word[4] = {kp[i].x, kp[i].y, kp[i].z, kp[i].w};
@@ -931,7 +946,8 @@ __global__ __launch_bounds__(256) void linear_chunk_outputs_kernel(const ScanArg
     __shared__ __attribute__((aligned(16))) uint16_t q_s[LC_TOKENS][32 * KS + 8];
     __shared__ __attribute__((aligned(16))) uint16_t p_s[3][LC_TOKENS][LX_LD];
     __shared__ __attribute__((aligned(16))) uint16_t v_t[64][LX_LD];
-    __shared__ float g_s[LC_TOKENS], b_s[LC_TOKENS], run_s[LC_TOKENS];
+    __shared__ float2 g_s[LC_TOKENS];                      // a 64-bit sum as two 32-bit numbers
+    __shared__ float b_s[LC_TOKENS], run_s[LC_TOKENS];
     const int h = blockIdx.y, j0 = blockIdx.x * 64;
     const int seq = blockIdx.z / a.max_chunks, c = blockIdx.z - seq * a.max_chunks;
     const int first = a.cu_tokens[seq] + c * a.chunk, end = a.cu_tokens[seq + 1];
@@ -964,9 +980,14 @@ __global__ __launch_bounds__(256) void linear_chunk_outputs_kernel(const ScanArg
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
         for (int i = 0; i < 2; ++i) sf[ks][i] = *(const float4*)(start + (long long)(j0 + t_mine) * a.dim + 32 * ks + 8 * g4 + 4 * i);
-    float g, b, run;
+    double g;
+    float b, run;
     lx_gates(a, h, first, nt, lane, g, b, &run);
-    if (wave == 0) { g_s[lane] = g; b_s[lane] = b * a.k_scale * a.q_scale; run_s[lane] = run * a.q_scale; }
+    if (wave == 0) {
+        g_s[lane] = make_float2((float)g, (float)(g - (double)(float)g));
+        b_s[lane] = b * a.k_scale * a.q_scale;
+        run_s[lane] = run * a.q_scale;
+    }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) *(uint4*)&q_s[t_mine][32 * ks + 8 * g4] = qf[ks];
 #pragma unroll
@@ -977,7 +998,8 @@ __global__ __launch_bounds__(256) void linear_chunk_outputs_kernel(const ScanArg
     }
     __syncthreads();
     // ---- weighted scores: lane (token 16 wave + r16) holds keys 32 u + 8 g4 + 4 tt + i
-    const float g_mine = g_s[t_mine];
+    const float2 g_mine = g_s[t_mine];
+    const float sign = lx_alternates(a, h, t_mine) ? -1.f : 1.f;
     float ones = 0.f;                                      // what the column of ones gives
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -991,7 +1013,8 @@ __global__ __launch_bounds__(256) void linear_chunk_outputs_kernel(const ScanArg
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int at = 32 * u + 8 * g4 + 4 * tt + i;
-                score[4 * tt + i] = at <= t_mine && at < nt ? acc[i] * expf(g_mine - g_s[at]) * b_s[at] : 0.f;
+                const float2 g_at = g_s[at];
+                score[4 * tt + i] = at <= t_mine && at < nt ? acc[i] * expf((g_mine.x - g_at.x) + (g_mine.y - g_at.y)) * (sign * b_s[at]) : 0.f;
                 ones += score[4 * tt + i];
             }
         }

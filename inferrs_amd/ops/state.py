@@ -174,9 +174,11 @@ def linear_scan(*, q: torch.Tensor, q_off: int, q_heads: int, k: torch.Tensor, k
     if chunk is None:
         least = SCAN_CHUNKS_FROM
         if (q.dtype == torch.bfloat16 and act == 0 and dim % 32 == 0 and dim <= 128 and vdim % 64 == 0
-                and (q_off | k_off | v_off | q.shape[1] | k.shape[1] | v.shape[1]) % 8 == 0 and (s_off | row) % 4 == 0):
+                and (q_off | k_off | v_off | q.shape[1] | k.shape[1] | v.shape[1]) % 8 == 0 and (s_off | row) % 4 == 0
+                and (q.data_ptr() | k.data_ptr() | v.data_ptr() | state.data_ptr()) % 16 == 0):
             # (chunks of such rows are the bfloat16 matrix cores': one request of 32 tokens 17.7 us by chunks, 19.6 by the walk, 100 tokens
-            # 22 and 51; a request more costs a chunk's matrices: 4 of 32 tokens 27.1 and 27.6, 8 of 16 35 and 26)
+            # 22 and 51; a request more costs a chunk's matrices: 4 of 32 tokens 27.1 and 27.6, 8 of 16 35 and 26.  Any other rows' chunks
+            # weigh with differences of 32-bit sums, which short portions are not given for speed alone)
             least = min(least, 32 + 6 * (n_seqs - 1))
         chunk = SCAN_CHUNK if longest > least else 0
         while chunk and n_seqs * -(-longest // chunk) * heads * (vdim + 1) * dim > SCAN_WORKSPACE_FLOATS:

@@ -411,6 +411,55 @@ def test_chunks_of_bfloat16_numbers_that_add_up(H, qh, dim, vdim, normaliser):
     assert all(new <= 1.25 * old and new < 1e-5 for new, old in zip(*errors)), errors
 
 
+SHORT_DECAYS = {
+    "mild": lambda g, n, H: -0.1 * torch.rand(n, H, generator=g),
+    "down to -2": lambda g, n, H: -2.0 * torch.rand(n, H, generator=g),
+    "down to -32": lambda g, n, H: -32.0 * torch.rand(n, H, generator=g),
+    "one of -1000": lambda g, n, H: torch.where(torch.arange(n)[:, None] == 7, torch.tensor(-1000.0), -0.1 * torch.rand(n, H, generator=g)),
+    "zeros": lambda g, n, H: torch.where(torch.arange(n)[:, None] % 13 == 5, torch.tensor(-float("inf")), -0.1 * torch.rand(n, H, generator=g)),
+    "constants": lambda g, n, H: torch.tensor([0.0, 1.0, 0.97, -0.9])[:H],
+}
+
+
+@pytest.mark.parametrize("dim,vdim,normaliser", [(128, 64, False), (64, 128, True)])
+@pytest.mark.parametrize("decays", list(SHORT_DECAYS))
+def test_short_portions_in_chunks_are_as_exact_as_the_walk(decays, dim, vdim, normaliser):
+    """One request of 33 to 128 tokens goes in chunks of 64 without being asked: no further from 64 bits than the walk, which multiplies
+    decays one by one, whatever these are.  Either way a result carries a few roundings of 2^-24 a token that it remembers, in another
+    order: a quarter more than the walk's error is allowed, and one rounding."""
+    from inferrs_amd import ops
+    H = 4
+    for n in (33, 40, 64, 100, 128):
+        g = torch.Generator().manual_seed(n + dim)
+        vt = vdim + int(normaliser)
+        q, k, v = (torch.randn(n, H * w, generator=g).bfloat16() for w in (dim, dim, vdim))
+        a = SHORT_DECAYS[decays](g, n, H)
+        b = torch.rand(n, H, generator=g) + 0.1
+        start = torch.randn(1, H * vt * dim, generator=g)
+        factor = (a.expand(n, H) if decays == "constants" else a.double().exp()).double()
+        Q, K = (x.double().view(n, H, dim) for x in (q, k))
+        V = torch.cat([v.double().view(n, H, vdim), torch.ones(n, H, 1, dtype=torch.float64)], dim=2)[:, :, :vt]
+        S, want = start.double().view(H, vt, dim).clone(), torch.zeros(n, H, vt, dtype=torch.float64)
+        for t in range(n):
+            S = S * factor[t][:, None, None] + b[t].double()[:, None, None] * V[t][:, :, None] * (K[t] * dim ** -0.5)[:, None, :]
+            want[t] = (S * Q[t][:, None, :]).sum(-1)
+        results = {}
+        for chunk in (None, 64, 0):
+            state = dev(start.clone())
+            gates = dict(decay=dev(a)) if decays == "constants" else dict(log_a=dev(a))
+            out = ops.linear_scan(q=dev(q), q_off=0, q_heads=H, k=dev(k), k_off=0, k_heads=H, v=dev(v), v_off=0, heads=H, dim=dim, vdim=vdim,
+                                  state=state, s_off=0, cu_tokens=dev(torch.tensor([0, n], dtype=torch.int32)),
+                                  state_slots=dev(torch.zeros(1, dtype=torch.int32)), k_scale=dim ** -0.5, normaliser=normaliser,
+                                  max_q_len=n, chunk=chunk, b=dev(b), **gates)
+            outs = out if normaliser else (out,)
+            results[chunk] = [x.cpu() for x in outs] + [state.cpu()]
+        assert all(torch.equal(x, y) for x, y in zip(results[None], results[64])), "the rule does not send this portion to chunks"
+        wants = [want[:, :, :vdim].reshape(n, -1)] + ([want[:, :, vdim]] if normaliser else []) + [S.reshape(1, -1)]
+        for what, new, walk, exact in zip(("outputs",) + ("normaliser",) * normaliser + ("state",), results[None], results[0], wants):
+            e_new, e_walk = (float((x.double() - exact).norm() / exact.norm()) for x in (new, walk))
+            assert e_new <= 1.25 * e_walk + 2 ** -24, (n, what, e_new, e_walk)
+
+
 @pytest.mark.parametrize("where", ["state", "values", "nan"])
 def test_chunks_keep_infinities(where):
     """One infinite entry of the state, one infinite value, one entry that is no number: the chunks on the bfloat16 matrix cores give finite
