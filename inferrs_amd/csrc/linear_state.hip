@@ -753,6 +753,19 @@ __global__ __launch_bounds__(256) void linear_local_mfma_kernel(const ScanArgs a
             for (int c2 = 0; c2 < 2; ++c2) {
                 const int col = j0 + 16 * c2 + r16;
                 if (col >= vt) continue;
+                if (!(fabsf(acc[c2][0]) < INFINITY && fabsf(acc[c2][1]) < INFINITY && fabsf(acc[c2][2]) < INFINITY && fabsf(acc[c2][3]) < INFINITY)) {
+                    // (a value of a later token that is not finite, times its weight of 0: formed again from the tokens up to each alone)
+                    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+                    const int t0 = 16 * wave + 4 * kq;
+                    for (int at = 0; at < t0 + 4; ++at) {
+                        const float value = v_s[at * LL_V_LD + 16 * c2 + r16];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (at <= t0 + r) sum[r] = fmaf(p_s[(t0 + r) * p_ld + at], value, sum[r]);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[c2][r] = sum[r];
+                }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int tt = 16 * wave + 4 * kq + r;
@@ -1066,6 +1079,21 @@ __global__ __launch_bounds__(256) void linear_chunk_outputs_kernel(const ScanArg
 #pragma unroll
             for (int p = 2; p >= 0; --p) own = lx_mfma(vf[u], *(const uint4*)&p_s[p][t][32 * u + 8 * g4], own);
         if (t >= nt) continue;
+        if (!(fabsf(own[0]) < INFINITY && fabsf(own[1]) < INFINITY && fabsf(own[2]) < INFINITY && fabsf(own[3]) < INFINITY)) {
+            // (an infinite value, or one that is no number, of a token behind t is multiplied with that token's weight of 0 above: such
+            // sums are formed again from the tokens up to t, one by one, so that what lies ahead of the value stays as it is; finite sums cost a
+            // comparison: 100 tokens, 64 heads of 128 x 64 22.1 -> 22.3 us)
+            float sum[4] = {0.f, 0.f, 0.f, 0.f};
+            for (int at = 0; at <= t; ++at) {
+                float weight = 0.f;
+#pragma unroll
+                for (int p = 0; p < 3; ++p) weight += __uint_as_float((uint32_t)p_s[p][t][at] << 16);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sum[i] = fmaf(weight, __uint_as_float((uint32_t)v_t[16 * wave + 4 * g4 + i][at] << 16), sum[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) own[i] = sum[i];
+        }
         const float r = run_s[t];
         float o[4];
 #pragma unroll

@@ -491,6 +491,40 @@ def test_chunks_keep_infinities(where):
     assert where == "nan" or got[0][1].isinf().any()
 
 
+@pytest.mark.parametrize("n", [40, 100, 150])
+@pytest.mark.parametrize("where", ["values", "keys", "queries", "state"])
+def test_what_is_not_finite_stays_behind_its_token(where, n):
+    """Infinities and entries that are no numbers: every output and every entry of the state is finite where the walk's is, and then the
+    walk's but for rounding (2e-5 of the largest finite one), tokens ahead of the entry among them."""
+    from inferrs_amd import ops
+    g = torch.Generator().manual_seed(n)
+    H, dim, vdim = 3, 64, 64
+    q, k, v = (torch.randn(n, H * w, generator=g).bfloat16() for w in (dim, dim, vdim))
+    start = torch.randn(1, H * (vdim + 1) * dim, generator=g)
+    inf, nan = float("inf"), float("nan")
+    if where == "values":
+        v[n - 3, 3], v[17, 70], v[32, 69], v[n // 2, 140] = -inf, inf, nan, nan
+    elif where == "keys":
+        k[n - 3, 5], k[20, dim + 7] = inf, nan
+    elif where == "queries":
+        q[n - 3, 5], q[20, dim + 7] = inf, nan
+    else:
+        start[0, 5 * dim + 9], start[0, (vdim + 1 + 8) * dim + 3] = inf, nan
+    got = []
+    for chunk in (None, 0):
+        state = dev(start.clone())
+        out, den = ops.linear_scan(q=dev(q), q_off=0, q_heads=H, k=dev(k), k_off=0, k_heads=H, v=dev(v), v_off=0, heads=H, dim=dim, vdim=vdim,
+                                   state=state, s_off=0, cu_tokens=dev(torch.tensor([0, n], dtype=torch.int32)),
+                                   state_slots=dev(torch.zeros(1, dtype=torch.int32)), skip=dev(torch.zeros(H)), q_scale=0.3, k_scale=0.7,
+                                   normaliser=True, max_q_len=n, chunk=chunk, log_a=dev(torch.full((n, H), -0.01)), b=dev(torch.ones(n, H)))
+        got.append((out.cpu(), den.cpu(), state.cpu()))
+    for new, walk in zip(*got):
+        finite = walk.isfinite()
+        assert torch.equal(new.isfinite(), finite)
+        assert float((new - walk)[finite].abs().max()) <= 2e-5 * float(walk[finite].abs().max())
+    assert not got[0][0].isfinite().all() and got[0][0].isfinite().any()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_gates_of_long_portions_are_the_walk(dtype):
     from inferrs_amd import ops
