@@ -213,6 +213,7 @@ __global__ __launch_bounds__(EG_THREADS) void exp_gates_block_kernel(
     __shared__ float sf[EG_THREADS], si[EG_THREADS], start[EG_THREADS];
     const int seq = blockIdx.x / H, h = blockIdx.x - seq * H;
     const int first = cu_tokens[seq], last = cu_tokens[seq + 1];
+    if (first >= last) return;                                   // (the whole block: no token, and the maximum stays)
     const int per = (last - first + EG_THREADS - 1) / EG_THREADS;
     const int lo = first + threadIdx.x * per < last ? first + threadIdx.x * per : last;
     const int hi = lo + per < last ? lo + per : last;

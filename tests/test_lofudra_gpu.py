@@ -545,6 +545,26 @@ def test_gates_of_long_portions_are_the_walk(dtype):
         assert float((got - want).abs().max()) <= 2e-5 * max(float(want.abs().max()), 1.0)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gates_of_requests_without_tokens(dtype):
+    """A request that brings nothing, ahead of all others, between them and behind them, in the kernel of long portions: nothing of it is
+    read or written, its maximum stays, and the others' results have the bits that they have without it."""
+    from inferrs_amd import ops
+    g = torch.Generator().manual_seed(4)
+    H, lens = 3, [0, 300, 0, 40, 0]
+    proj = dev(4.0 * torch.randn(sum(lens), 2 * H + 5, generator=g), dtype)
+    bi, bf = dev(torch.randn(H, generator=g)), dev(torch.tensor([1.0, 4.0, -2.0]))
+    start = torch.randn(5, H + 2, generator=g)
+    results = []
+    for kept in ([0, 1, 2, 3, 4], [1, 3]):
+        cu = torch.tensor([0] + torch.tensor([lens[i] for i in kept]).cumsum(0).tolist(), dtype=torch.int32)
+        state = dev(start.clone())
+        outs = ops.exp_gates(proj, 2, 2 + H, bi, bf, 7.0, state, 2, dev(cu), dev(torch.tensor(kept, dtype=torch.int32)), max_q_len=300)
+        results.append([o.cpu() for o in outs] + [state.cpu()])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+    assert torch.equal(results[0][-1][[0, 2, 4]], start[[0, 2, 4]])
+
+
 # ---- whole models under every cutting ---------------------------------------------------------------
 
 @pytest.fixture(scope="module")
