@@ -712,27 +712,34 @@ def attention_mfma(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     return out
 
 
-# The decode kernel's counters: zero between calls (the kernel puts them back).  One array a device: calls that
-# share it must follow each other (one stream, or a graph replayed on it), as an engine's steps do.
-_DECODE_COUNTERS: Dict[int, torch.Tensor] = {}
-_DECODE_COUNTERS_OUTGROWN: list = []                # captured graphs may still hold their addresses: never freed
+class DecodeCounters(dict):
+    """The decode kernel's counters, an array a device: zero between calls (the kernel puts them back).  Calls that share them must follow
+    each other (one stream, or a graph replayed on it), as an engine's steps do; every engine holds its own, so that two engines can
+    run on two streams of a device."""
+
+    def __init__(self):
+        super().__init__()
+        self._outgrown: list = []                   # captured graphs may still hold their addresses: kept as long as this is
+
+    def take(self, device: torch.device, needed: int) -> Optional[torch.Tensor]:
+        """At least `needed` of them on `device` (None for none)."""
+        if needed <= 0:
+            return None
+        key = device.index if device.index is not None else torch.cuda.current_device()
+        have = self.get(key)
+        if have is None or have.numel() < needed:
+            if torch.cuda.is_current_stream_capturing():
+                raise KernelError("attention_decode_fused: the counters of the decode kernel cannot be allocated under "
+                                  "graph capture; run a step of this size once before capturing it")
+            if have is not None:
+                self._outgrown.append(have)
+            have = torch.zeros((max(DECODE_COUNTERS_MIN, 2 * needed),), dtype=torch.int32, device=device)
+            self[key] = have
+        return have
+
+
+_DECODE_COUNTERS = DecodeCounters()                 # of calls that bring none
 DECODE_COUNTERS_MIN = 1 << 16
-
-
-def _decode_counters(device: torch.device, needed: int) -> Optional[torch.Tensor]:
-    if needed <= 0:
-        return None
-    key = device.index if device.index is not None else torch.cuda.current_device()
-    have = _DECODE_COUNTERS.get(key)
-    if have is None or have.numel() < needed:
-        if torch.cuda.is_current_stream_capturing():
-            raise KernelError("attention_decode_fused: the counters of the decode kernel cannot be allocated under "
-                              "graph capture; run a step of this size once before capturing it")
-        if have is not None:
-            _DECODE_COUNTERS_OUTGROWN.append(have)
-        have = torch.zeros((max(DECODE_COUNTERS_MIN, 2 * needed),), dtype=torch.int32, device=device)
-        _DECODE_COUNTERS[key] = have
-    return have
 
 
 @functools.lru_cache(maxsize=4096)
@@ -759,13 +766,15 @@ def attention_decode_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: to
                            seqs: Optional[Tuple[int, int]] = None, out: Optional[torch.Tensor] = None,
                            sink: bool = False, mask_chunk: Optional[int] = None, dv: Optional[int] = None,
                            offsets: Optional[Tuple[int, Optional[int], Optional[int]]] = None, rot: Optional[int] = None,
-                           gate_off: Optional[int] = None, gate_per_head: bool = False) -> torch.Tensor:
+                           gate_off: Optional[int] = None, gate_per_head: bool = False,
+                           counters: Optional[DecodeCounters] = None) -> torch.Tensor:
     """Decode steps (one token a request) in one kernel: per-head norm of q and k, rotation, the write
     of the new key and value at `slots` (None: the cache is only read) and the attention over the pages.
     `qkv` [n, (nq + 2 nkv) * d] is the projections' output; request s owns token s.  Returns [n, nq, d].
     Rows of other layouts: values of width `dv`, `offsets` = where the query, key and value heads begin in a row (the last two
     are None where nothing is written), `rot` = the first features of a head that rotate, and `gate_off` = where a row's gate values
-    begin (one a feature of the joined heads, or `gate_per_head`): the output is times their sigmoid."""
+    begin (one a feature of the joined heads, or `gate_per_head`): the output is times their sigmoid.  `counters`: those of the caller's
+    stream (None: one set a device, for callers that use one stream)."""
     _dev(qkv, k_cache, v_cache, positions, cu_tokens, block_table, slots, q_norm_w, k_norm_w, cos, sin, out)
     _i32(positions, "positions"); _i32(cu_tokens, "cu_tokens"); _i32(block_table, "block_table")
     _f32(q_norm_w, "q_norm weight"); _f32(k_norm_w, "k_norm weight"); _f32(cos, "cos"); _f32(sin, "sin")
@@ -818,14 +827,14 @@ def attention_decode_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: to
     lib = library(target)
     ws_floats, n_counters = _decode_sizes(target, n, nq, nkv, splits)
     ws = torch.empty((ws_floats,), dtype=torch.float32, device=qkv.device) if ws_floats else None
-    counters = _decode_counters(qkv.device, n_counters)
+    taken = (_DECODE_COUNTERS if counters is None else counters).take(qkv.device, n_counters)
     _check(lib.ia_attention_mfma_decode_fused(
         _p(out), _p(ws), _p(qkv), _p(k_cache), _p(v_cache), _p(block_table), _p(cu_tokens), _p(positions), _p(slots),
         _p(q_norm_w), _p(k_norm_w), _p(cos), _p(sin), eps, int(add_one), ld_, q_off, k_off or 0, v_off or 0,
         rot if cos is not None else 0, _p(qkv) + 2 * gate_off if gate_off is not None else None, ld_, int(gate_per_head), n, seq_begin,
         n_seqs, seq_begin, n_seqs, max_kv_len, block_table.shape[1], nq, nkv, d, page_size, int(window or 0),
-        scale, splits, chunk, int(bool(sink)), int(mask_chunk or 0), _p(counters),
-        counters.numel() if counters is not None else 0, _stream()), target)
+        scale, splits, chunk, int(bool(sink)), int(mask_chunk or 0), _p(taken),
+        taken.numel() if taken is not None else 0, _stream()), target)
     return out
 
 

@@ -197,7 +197,7 @@ class Attention(Mixer):
                 offsets=(self.q_off, self.k_off, self.v_off), slots=group.slots if writes else None, q_norm_w=self.q_norm_w,
                 k_norm_w=self.k_norm_w, eps=self.norm_eps, add_one=self.norm_add_one, cos=cos, sin=sin, rot=self.position.rot_dim,
                 max_kv_len=ctx.max_kv_len, window=s.window, scale=s.softmax_scale, sink=s.sink, mask_chunk=s.mask_chunk,
-                gate_off=self.g_off, gate_per_head=bool(s.gate and s.gate_per_head))
+                gate_off=self.g_off, gate_per_head=bool(s.gate and s.gate_per_head), counters=getattr(ctx, "decode_counters", None))
             return self._project(ctx, a.view(a.shape[0], H * dv))
         v_with = None
         if s.v_mix is not None:
@@ -240,7 +240,8 @@ class Attention(Mixer):
                     q.dtype, s.head_dim, group.page_size, 0, False, False, s.value_dim):
                 a = ops.attention_decode_fused(q.view(n, -1), *of, nq=q.shape[1], nkv=cache.k.shape[1], d=s.head_dim,
                                                dv=s.value_dim, offsets=(0, None, None), slots=None, q_norm_w=None, k_norm_w=None,
-                                               eps=0.0, add_one=False, cos=None, sin=None, max_kv_len=max_kv, seqs=(0, singles), **common)
+                                               eps=0.0, add_one=False, cos=None, sin=None, max_kv_len=max_kv, seqs=(0, singles),
+                                               counters=getattr(ctx, "decode_counters", None), **common)
             else:
                 a = ops.attention_mfma(q, *of, max_q_len=1, max_kv_len=max_kv, seqs=(0, singles), tokens=(0, singles), **common, **special)
         if singles < ctx.n_seqs:
@@ -312,7 +313,7 @@ class Attention(Mixer):
                 nkv=s.n_kv_heads, d=s.head_dim, slots=group.slots if cache.writable else None,
                 q_norm_w=self.q_norm_w, k_norm_w=self.k_norm_w, eps=self.norm_eps, add_one=self.norm_add_one,
                 cos=cos, sin=sin, rot=self.position.rot_dim, max_kv_len=ctx.max_kv_len, window=s.window, scale=s.softmax_scale,
-                sink=s.sink)
+                sink=s.sink, counters=getattr(ctx, "decode_counters", None))
             return self._project(ctx, a.view(a.shape[0], s.n_heads * s.head_dim))
         q = ops.qk_rope_kv(
             qkv, s.n_heads, s.n_kv_heads, s.head_dim,

@@ -585,3 +585,45 @@ def test_choice_beside_a_gated_product(n, inter, E, gates):
         g, u = rows[:, :inter].double().clamp(max=limit), rows[:, inter:2 * inter].double().clamp(-limit, limit)
         act = g * torch.sigmoid(slope * g) * (u + 1)
         assert float((got[3].cpu().double() - act).abs().max()) <= 2 ** -8 * float(act.abs().max()) * 1.01
+
+
+def test_two_engines_on_two_streams(tmp_path):
+    """Decode steps and steps of single tokens beside a portion, of two engines whose streams run side by side: every engine hands partial
+    results over through counters of its own, and its logits are the bits that it gives alone."""
+    import torch
+    from inferrs_amd import ops
+    from inferrs_amd.engine import Engine, Entry
+    cfg = CONFIGS["D"]
+    folder = str(tmp_path / "d")
+    write_model(folder, cfg, seed=3)
+    prompts = [random_tokens(n, cfg["vocab"], 50 + n) for n in (300, 41, 120)]
+
+    def steps(eng, name):
+        """The steps of one engine, a generator that hands each step's logits out."""
+        yield eng.step([Entry(name + str(i), p, [len(p) - 1]) for i, p in enumerate(prompts)])
+        for j in range(6):
+            yield eng.step([Entry(name + str(i), [(7 * j + i) % cfg["vocab"]], [0]) for i in range(3)])
+        for j in range(3):
+            yield eng.step([Entry(name + str(i), [j + i], [0]) for i in range(2)] + [Entry(name + "2", prompts[1][j:j + 20], [19])])
+
+    def engine():
+        return Engine.from_folder(folder, dtype="bfloat16", page_size=16, num_pages=256, max_seqs=4)
+
+    alone = [[x.clone() for x in logits] for logits in steps(engine(), "s")]
+    shared = {k: v.clone() for k, v in ops._DECODE_COUNTERS.items()}
+    engines = [engine(), engine()]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    runs = [steps(e, f"e{i}") for i, e in enumerate(engines)]
+    got = [[], []]
+    for _ in alone:
+        for i in range(2):
+            with torch.cuda.stream(streams[i]):
+                got[i].append([x.clone() for x in next(runs[i])])
+    torch.cuda.synchronize()
+    for mine in got:
+        for a, b in zip(mine, alone):
+            assert all(torch.equal(x, y) for x, y in zip(a, b))
+    own = [e.builder.decode_counters for e in engines]
+    assert own[0] is not own[1] and all(len(c) == 1 and int(c[0].abs().sum()) == 0 for c in own) and own[0][0].data_ptr() != own[1][0].data_ptr()
+    assert all(torch.equal(ops._DECODE_COUNTERS[k], v) for k, v in shared.items()) and set(shared) == set(ops._DECODE_COUNTERS)
