@@ -629,27 +629,36 @@ def decode_split(n_seqs: int, nkv: int, g: int, max_kv_len: int) -> Tuple[int, i
 
 
 @functools.lru_cache(maxsize=4096)
-def decode_shares(n_seqs: int, nkv: int, g: int, max_kv_len: int) -> Tuple[int, int]:
-    """(splits, keys per split) that a decode step takes: `decode_split`'s, but for other counts where they were faster over contexts of
-    8 to 97 % of the bound up to 1,024 keys and 55 to 97 % of longer ones (a step's bound is a bucket's, and batches of more than eight hold
-    contexts from a third of the longest; in the mean over 8 key/value heads of 2 and 4 query heads and 4 of 4):
-    a round's worth of waves that eight splits leave idle goes to twelve (9 and 10 requests of 8 key heads at 2,048 keys 1.11, 3,072 1.18,
-    8,192 1.21); up to 1,024 keys four splits meet in one block where eight are handed over between two (10 to 16 requests 1.09 to 1.15);
-    blocks of three waves for four where nearly the whole round is taken, at 3,072 keys and more (28 and 32 requests 1.01 to 1.04); one or two
-    requests of 3,072 to 4,096 keys take 48 and 64 splits for 32 (1.05 to 1.13, 1.02 to 1.11), three or four of 3,072 to 4,095 or 8,192 and
-    more 28 (1.10 to 1.15, 1.10)."""
+def decode_shares(n_seqs: int, nkv: int, g: int, max_kv_len: int, d: int = 128, dv: int = 128) -> Tuple[int, int]:
+    """(splits, keys per split) that a decode step takes: `decode_split`'s, but for other counts where they were faster, at keys of `d` and values
+    of `dv` features.  Measured at widths of (64, 64), (128, 128), (128, 64), (192, 192) and (256, 256), 1 to 64 requests of 1 to 8 key heads with 1
+    to 16 query heads, contexts within a bound's last bucket and of 40 to 97 % of it (8 to 97 % of 1,024); speed against `decode_split`'s counts,
+    means at these widths in this order:
+    - a round's worth of waves that eight splits leave idle goes to twelve: 1.11, 1.10, 1.16, 1.15, 1.17, none below 0.98;
+    - up to 1,024 keys four splits meet in one block where eight are handed over between two: 1.11, 1.01, 1.03 (contexts up to 700 keys 1.13 to
+      1.16, longer ones 0.88 to 1.07); 0.93 and 0.96 with wider heads, which keep eight;
+    - 48 splits for 32 of 3,072 to 4,095 keys with up to eight query heads a key head: 1.04, 1.08, 1.11, 1.14; with sixteen 0.95 to 1.03, and 0.92 at
+      256 (what a block hands over is as wide as its query heads are); 64 of 4,096 keys with up to four: 1.02, 1.07, 1.08, 1.14; with more 0.91 to
+      0.98, and 0.86 at 256;
+    - 28 splits for 32, which leave some of the chip's waves out: from 28 pairs of a request and a key head on at 8,192 keys and more 1.03, 1.08, 1.02, 1.05,
+      1.00, with fewer 0.97, 1.00, 0.94, 0.96, 0.94; from 17 on at 3,072 to 4,095 keys 1.02, 1.06, 1.03, 1.04, at 256 0.87 to 1.19.
+    (Blocks of three waves for four: 0.95, 1.00, 0.99, 1.00, 1.01, not taken.)"""
     splits, chunk = decode_split(n_seqs, nkv, g, max_kv_len)
     items = n_seqs * nkv * -(-g // 16)
+    wide = max(d, dv)
     other = splits
     if splits == 8 and 512 < max_kv_len <= 1024:
-        other = 4
+        if wide <= 128:
+            other = 4
     elif splits == 8 and items * 12 <= DECODE_WAVES and max_kv_len >= 2048:
         other = 12
-    elif splits == 4 and items >= 224 and max_kv_len >= 3072:
-        other = 3
-    elif splits == 32 and items <= 16 and 3072 <= max_kv_len <= 4096:
-        other = 64 if max_kv_len == 4096 else 48
-    elif splits == 32 and 16 < items <= 36 and (3072 <= max_kv_len < 4096 or max_kv_len >= 8192):
+    elif splits == 32 and wide < 256 and 3072 <= max_kv_len < 4096 and items > 16:
+        other = 28
+    elif splits == 32 and wide < 256 and 3072 <= max_kv_len < 4096 and g <= 8:
+        other = 48
+    elif splits == 32 and wide < 256 and max_kv_len == 4096 and items <= 16 and g <= 4:
+        other = 64
+    elif splits == 32 and items >= 28 and max_kv_len >= 8192:
         other = 28
     if other == splits:
         return splits, chunk
@@ -820,7 +829,7 @@ def attention_decode_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: to
     elif tuple(out.shape) != (n, nq, dv) or out.dtype != qkv.dtype:
         raise KernelError("attention_decode_fused: `out` must be [n, nq, the values' width] in the dtype of qkv")
     if splits is None:
-        splits, chunk = decode_shares(n_seqs, nkv, nq // nkv, max_kv_len)
+        splits, chunk = decode_shares(n_seqs, nkv, nq // nkv, max_kv_len, d, dv)
     else:
         chunk = -(-(-(-max_kv_len // splits)) // 32) * 32
     target = _build.attn_target(d, dv)

@@ -952,6 +952,43 @@ def test_attention_decode_takes_rows_of_any_layout(nq, nkv, d, dv_, page, window
         assert counters is None or int(counters.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("nq,nkv,d,dv_,window,gate", [
+    (8, 2, 128, 128, None, None), (16, 4, 128, 64, 1500, "feature"), (34, 2, 64, 64, None, "head"), (20, 1, 64, 256, 700, None),
+    (3, 3, 192, 192, None, "feature"), (2, 1, 256, 256, None, None)])
+def test_attention_decode_in_any_count_of_shares(nq, nkv, d, dv_, window, gate):
+    """Counts of shares that are no powers of two: blocks of three waves (3, 9), of one (5, 7), of four (12, 28, 48), merged three to twelve
+    at a time, against the separate kernels with the keys in one share.  The gate's kernel rounds the joined heads before it multiplies them, hence a
+    bound of two roundings to bfloat16 of the largest value."""
+    from inferrs_amd import ops
+    lens, page = [3500, 3073, 1500, 1], 16
+    _, kc, vc, positions, _, table = attention_case(torch.bfloat16, nq, nkv, d, page, lens, [1] * len(lens), 37)
+    vc = randn(kc.shape[0], nkv, dv_, page, dtype=torch.bfloat16, seed=9)
+    n, at = len(lens), nq * d + nkv * (d + dv_)
+    width = at + {None: 0, "feature": nq * dv_, "head": nq}[gate]
+    proj = dev(randn(n, width + -width % 8, dtype=torch.bfloat16, seed=5))
+    qw, kw = (dev(1 + 0.3 * randn(d, dtype=torch.float32, seed=s)) for s in (6, 7))
+    ang = positions.float()[:, None] / 10000.0 ** (torch.arange(0, d, 2, dtype=torch.float32) / d)
+    cos, sin = dev(torch.cos(ang)), dev(torch.sin(ang))
+    slots = dev(torch.tensor([int(table[s, (l - 1) // page]) * page + (l - 1) % page for s, l in enumerate(lens)], dtype=torch.int32))
+    cu, table, positions = dev(torch.arange(n + 1, dtype=torch.int32)), dev(table), dev(positions)
+    k1, v1 = dev(kc), dev(vc)
+    q1 = ops.qk_rope_kv_strided(proj, nq, nkv, d, dv_, q_off=0, k_off=nq * d, v_off=(nq + nkv) * d, q_norm_w=qw, k_norm_w=kw, eps=1e-5,
+                                add_one=False, cos=cos, sin=sin, rot=d, interleaved=False, k_cache=k1, v_cache=v1, slots=slots, page_size=page)
+    want = ops.attention_mfma(q1, k1, v1, positions, cu, table, max_q_len=1, max_kv_len=max(lens), window=window, scale=d ** -0.5,
+                              splits=1).view(n, nq * dv_)
+    if gate:
+        ops.sigmoid_gate(want, proj, at, group=1 if gate == "feature" else dv_)
+    for splits in (3, 5, 7, 9, 12, 28, 48):
+        k2, v2 = dev(kc), dev(vc)
+        got = ops.attention_decode_fused(proj, k2, v2, positions, cu, table, nq=nq, nkv=nkv, d=d, dv=dv_, offsets=(0, nq * d, (nq + nkv) * d),
+                                         slots=slots, q_norm_w=qw, k_norm_w=kw, eps=1e-5, add_one=False, cos=cos, sin=sin, max_kv_len=max(lens),
+                                         window=window, scale=d ** -0.5, splits=splits, gate_off=at if gate else None, gate_per_head=gate == "head")
+        close(got.view(n, -1).float().cpu(), want.float().cpu(), 2 ** -7, f"splits={splits}")
+        assert torch.equal(v2, v1)
+        counters = ops._DECODE_COUNTERS.get(torch.cuda.current_device())
+        assert counters is not None and int(counters.abs().sum()) == 0
+
+
 @pytest.mark.parametrize("nq,nkv,d,page,window", [
     (3, 1, 128, 16, None), (8, 2, 128, 112, 40), (7, 1, 128, 16, None), (8, 1, 128, 32, 95),    # the new key in the first pass over
     (16, 1, 128, 16, None), (17, 1, 64, 48, None), (5, 1, 192, 16, 33), (2, 1, 256, 80, None)])  # the rows, the second, a third, a last of its own

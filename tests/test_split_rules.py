@@ -1,6 +1,6 @@
 """How the attention kernels' keys are split between waves and blocks: the rules are plain functions of a step's sizes,
 so what every kernel launch assumes of them is checked here for many sizes (the kernels refuse what breaks these,
-`csrc/attention_mfma.hip` attention_launch: splits a power of two for the decode kernel, a share that is a multiple of
+`csrc/attention_mfma.hip` attention_launch: blocks of equally many shares for the decode kernel, a share that is a multiple of
 32 keys, of 64 for the tiled kernel, and splits x share covering the longest context)."""
 import itertools
 
@@ -190,10 +190,17 @@ def test_decode_shares_are_whole_blocks_that_cover_the_context(g):
     many waves (up to four, so that more than four shares come in fours), shares of two steps of 32 keys or more."""
     others = set()
     for n_seqs, nkv, kv in itertools.product(range(1, 65), (1, 2, 4, 8), (31, 512, 513, 1024, 2048, 3072, 4095, 4096, 8192, 40960)):
-        base, (splits, chunk) = ops.decode_split(n_seqs, nkv, g, kv), ops.decode_shares(n_seqs, nkv, g, kv)
-        assert chunk % 32 == 0 and splits * chunk >= kv and 1 <= splits <= 128
-        assert splits <= 4 or splits % 4 == 0
-        if (splits, chunk) != base:
-            others.add(splits)
-            assert chunk >= 64 and n_seqs * nkv * -(-g // 16) * splits <= ops.DECODE_WAVES
-    assert others <= {3, 4, 12, 28, 48, 64}
+        base = ops.decode_split(n_seqs, nkv, g, kv)
+        for d, dv in ((64, 64), (128, 64), (128, 128), (192, 192), (256, 256)):
+            splits, chunk = ops.decode_shares(n_seqs, nkv, g, kv, d, dv)
+            assert chunk % 32 == 0 and splits * chunk >= kv and 1 <= splits <= 128
+            assert splits <= 4 or splits % 4 == 0
+            if (splits, chunk) != base:
+                others.add((splits, max(d, dv)))
+                assert chunk >= 64 and n_seqs * nkv * -(-g // 16) * splits <= ops.DECODE_WAVES
+    widths = (64, 128, 192, 256)
+    assert {w for s, w in others if s == 12} == {w for s, w in others if s == 28} == set(widths)
+    assert {w for s, w in others if s == 4} == {64, 128}
+    assert {w for s, w in others if s == 48} == (set(widths[:3]) if g <= 8 else set())
+    assert {w for s, w in others if s == 64} == (set(widths[:3]) if g <= 4 else set())
+    assert {s for s, _ in others} <= {4, 12, 28, 48, 64}
