@@ -665,6 +665,44 @@ def decode_shares(n_seqs: int, nkv: int, g: int, max_kv_len: int, d: int = 128, 
     return other, -(-(-(-max_kv_len // other)) // 32) * 32
 
 
+@functools.lru_cache(maxsize=4096)
+def decode_fused_pays(n_seqs: int, nkv: int, g: int, d: int, dv: int, max_kv_len: int, span: int, *, formed: bool, gated: bool) -> bool:
+    """Whether `attention_decode_fused` is faster than the kernels that it stands for: the norm and rotation, `attention_mfma` with its merge and (`gated`)
+    the gate; or, of queries that are `formed` already, the attention and its merge alone.  `span`: the keys that a token sees at most
+    (a window, a chunk of the mask; 0: all).  What the decode kernel pays for one launch is the hand-over: the last block of a (request, key head)
+    reads all others' partial results past the caches, which the merge's kernel spreads over the chip; and where keys and values are wide, a
+    wave's registers.  Measured at the widths of `decode_shares` and at 700 drawn sizes, (64, 256) among them: 1 to 73 requests of 1 to 8 key heads
+    with 1 to 16 query heads, 512 to 16,384 keys, windows of 128 to 2,048 (times of the separate kernels over this one's, by the floats that one merge
+    reads; a pair is a request and a key head).  Over all of these sizes the choice is 0.2 to 2 % off the faster one in the mean:
+    - layers, widths up to 128: 1.3 to 1.8 in the mean with nothing handed over, 1.2 to 1.5 below 8,192 floats, 1.1 to 1.3 at 8,192; at 16,384 1.07 to
+      1.16 with a gate (fewer than eight pairs 0.87 to 1.16) and 0.94 to 1.01 without, beyond that 0.5 to 0.95.  Without a gate, where a share is
+      as long as a window of 1,024 and more, two waves of a pair have work: up to 127 pairs 0.94 in the mean;
+    - up to 384 features of a key and a value, up to eight query heads a key head: 1.1 to 1.5 up to 4,096 floats, 1.0 to 1.15 with a gate and 0.9 to 1.03
+      without up to 8,192, 0.6 to 1.0 beyond; with more query heads 0.4 to 1.8, 0.7 in the mean.  (256, 256): 0.17 to 1.16, but 1.06 to 1.6 from
+      192 pairs on in one block under windows and up to 1,024 keys;
+    - formed queries: from 64 pairs on 1.2 in the mean, and for 64 features in one block, else 0.86 (0.74 at (64, 256) and (192, 192)).  Under windows
+      shorter than a quarter of the bound from an eighth of the window on: 32 pairs and a window of 128 1.29, 64 and 512 1.02, 128 and 1,024 1.12, 64
+      and 1,024 0.87."""
+    splits, chunk = decode_shares(n_seqs, nkv, g, max_kv_len, d, dv)
+    nq = nkv * g
+    blocks = _decode_sizes(_build.attn_target(d, dv), 1, nq, nkv, splits)[0] // (nq * (dv + 2)) or 1
+    handed = min(g, 16) * dv * blocks if blocks > 1 else 0
+    items = n_seqs * nkv * -(-g // 16)
+    narrow = 0 < 4 * span <= max_kv_len
+    if d + dv > 384:
+        return blocks == 1 and items >= 192 and (0 < span < max_kv_len or (max_kv_len <= 1024 and items <= 256))
+    small = max(d, dv) <= 128
+    if formed:
+        if narrow:
+            return items >= max(32 if small else 64, span // 8)
+        return items >= 64 or (small and d <= 64 and blocks == 1)
+    if not small:
+        return g <= 8 and handed <= (8192 if gated else 4096)
+    if not gated and narrow and 1024 <= span <= chunk and items < 128:
+        return False
+    return handed < 16384 or (gated and handed == 16384 and items >= 8)
+
+
 def attention_mfma(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, positions: torch.Tensor,
                    cu_tokens: torch.Tensor, block_table: torch.Tensor, *, max_q_len: int, max_kv_len: int,
                    window: Optional[int], scale: float, splits: Optional[int] = None,

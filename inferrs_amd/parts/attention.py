@@ -190,7 +190,8 @@ class Attention(Mixer):
         writes = cache.writable and s.own_kv
         if (ctx.max_q_len == 1 and s.v_mix is None and not s.keep_first and s.softcap is None
                 and ops.attention_decode_fused_fits(proj.dtype, d, group.page_size, self.position.rot_dim, self.position.interleaved,
-                                                    cos is not None, dv)):
+                                                    cos is not None, dv)
+                and ops.decode_fused_pays(ctx.n_seqs, G, H // G, d, dv, ctx.max_kv_len, self.span(s), formed=False, gated=bool(s.gate))):
             # decode steps: norm, rotation, cache write, attention and gate in one kernel
             a = ops.attention_decode_fused(
                 proj, cache.k, cache.v, ctx.positions, ctx.cu_tokens, group.block_table, nq=H, nkv=G, d=d, dv=dv,
@@ -220,6 +221,11 @@ class Attention(Mixer):
         return self._project(ctx, joined)
 
     @staticmethod
+    def span(s: AttentionSpec) -> int:
+        """The keys that a token sees at most (0: all)."""
+        return min((k for k in (s.window, s.mask_chunk) if k), default=0)
+
+    @staticmethod
     def attend(s: AttentionSpec, ctx, q, cache, group):
         """The paged attention of the step's queries: the matrix cores where they take the sizes, else the plain kernel."""
         if not ops.attention_mfma_fits(q.dtype, s.head_dim, group.page_size, s.value_dim):
@@ -236,9 +242,12 @@ class Attention(Mixer):
         a = None
         if singles > 0:
             max_kv = ctx.max_kv_single if singles < ctx.n_seqs else ctx.max_kv_len
-            if not s.keep_first and s.softcap is None and ops.attention_decode_fused_fits(
-                    q.dtype, s.head_dim, group.page_size, 0, False, False, s.value_dim):
-                a = ops.attention_decode_fused(q.view(n, -1), *of, nq=q.shape[1], nkv=cache.k.shape[1], d=s.head_dim,
+            nkv = cache.k.shape[1]
+            if (not s.keep_first and s.softcap is None
+                    and ops.attention_decode_fused_fits(q.dtype, s.head_dim, group.page_size, 0, False, False, s.value_dim)
+                    and ops.decode_fused_pays(singles, nkv, q.shape[1] // nkv, s.head_dim, s.value_dim, max_kv, Attention.span(s),
+                                              formed=True, gated=False)):
+                a = ops.attention_decode_fused(q.view(n, -1), *of, nq=q.shape[1], nkv=nkv, d=s.head_dim,
                                                dv=s.value_dim, offsets=(0, None, None), slots=None, q_norm_w=None, k_norm_w=None,
                                                eps=0.0, add_one=False, cos=None, sin=None, max_kv_len=max_kv, seqs=(0, singles),
                                                counters=getattr(ctx, "decode_counters", None), **common)

@@ -204,3 +204,15 @@ def test_decode_shares_are_whole_blocks_that_cover_the_context(g):
     assert {w for s, w in others if s == 48} == (set(widths[:3]) if g <= 8 else set())
     assert {w for s, w in others if s == 64} == (set(widths[:3]) if g <= 4 else set())
     assert {s for s, _ in others} <= {4, 12, 28, 48, 64}
+
+
+@pytest.mark.parametrize("n,nkv,g,d,dv,bound,span,kind,apart,fused", [
+    (8, 4, 4, 128, 64, 2048, 1024, "gated", 15.5, 9.5), (8, 4, 4, 128, 64, 2048, 0, "gated", 16.2, 10.1), (1, 8, 2, 256, 256, 2048, 0, "gated", 17.8, 21.9),
+    (16, 1, 16, 192, 192, 4096, 0, "plain", 22.0, 33.4), (1, 1, 16, 128, 128, 16384, 0, "gated", 16.2, 28.3), (24, 8, 2, 256, 256, 1024, 0, "plain", 43.5, 39.0),
+    (64, 4, 4, 256, 256, 8192, 1024, "plain", 107.4, 69.2), (12, 8, 2, 64, 64, 8192, 1024, "plain", 19.8, 24.9), (24, 8, 2, 128, 128, 8192, 1024, "plain", 38.6, 29.4),
+    (1, 4, 4, 128, 64, 8192, 0, "formed", 8.5, 11.1), (4, 4, 4, 128, 64, 4096, 1024, "formed", 8.8, 10.3), (9, 8, 5, 128, 128, 4096, 0, "formed", 27.4, 22.8),
+    (64, 4, 4, 128, 64, 4096, 1024, "formed", 49.5, 25.1), (12, 8, 5, 128, 128, 8192, 1024, "formed", 22.5, 28.9), (1, 1, 16, 256, 256, 16384, 0, "formed", 15.4, 123.9),
+    (2, 8, 2, 64, 64, 512, 0, "formed", 7.1, 5.5), (16, 2, 8, 128, 128, 1024, 0, "formed", 9.4, 9.7), (32, 2, 8, 128, 128, 1024, 0, "formed", 11.8, 10.5)])
+def test_decode_attention_takes_the_faster_kernels_at_the_measured_points(n, nkv, g, d, dv, bound, span, kind, apart, fused):
+    """The choice between one kernel and several as a layer makes it, against both measured times (us)."""
+    assert ops.decode_fused_pays(n, nkv, g, d, dv, bound, span, formed=kind == "formed", gated=kind == "gated") == (fused < apart)
