@@ -893,6 +893,37 @@ def test_portions_of_few_columns_share_their_keys(nq, nkv, qs, window):
     close(outs[0], outs[1], 2 ** -7, "few columns")
 
 
+@pytest.mark.parametrize("dv_,extra", [
+    (128, dict(mask_chunk=100)), (128, dict(sink=True)), (128, dict(sinks=True, window=50)), (128, dict(window=60, keep_first=5)),
+    (128, dict(window=33, keep_first=40, softcap=3.0)), (128, dict(softcap=5.0)), (64, {}), (64, dict(window=70, softcap=3.0)), (64, dict(mask_chunk=64, sink=True))])
+@pytest.mark.parametrize("nq,nkv,qs", [(16, 8, [9, 60, 1, 17]), (17, 1, [1, 7])])
+def test_portions_of_few_columns_in_every_form(nq, nkv, qs, dv_, extra):
+    """What a token sees and how its scores are formed, and values narrower than keys, in blocks that have fewer columns than they could take: as
+    `test_portions_of_few_columns_share_their_keys`."""
+    from inferrs_amd import ops
+    d, page, extra = 128, 16, dict(extra)
+    lens = [q + c for q, c in zip(qs, (0, 130, 448, 65))]
+    q, kc, vc, positions, token_seq, table = attention_case(torch.bfloat16, nq, nkv, d, page, lens, qs, 31)
+    vc = randn(kc.shape[0], nkv, dv_, page, dtype=torch.bfloat16, seed=9)
+    cu = torch.tensor([0] + torch.tensor(qs).cumsum(0).tolist(), dtype=torch.int32)
+    assert ops.attention_split(len(qs), nkv, nq // nkv, max(qs), max(lens), d)[0] == 1
+    if extra.get("sinks"):
+        extra["sinks"] = dev(randn(nq, dtype=torch.float32, seed=3))
+    lib, outs = ops.library(ops._build.attn_target(d, dv_)), []
+    for tiles in (1, 0):
+        lib.ia_attention_mfma_tiles(tiles)
+        try:
+            outs.append(ops.attention_mfma(dev(q), dev(kc), dev(vc), dev(positions), dev(cu), dev(table), max_q_len=max(qs),
+                                           max_kv_len=max(lens), window=extra.get("window"), scale=d ** -0.5,
+                                           **{k: v for k, v in extra.items() if k != "window"}).float().cpu())
+        finally:
+            lib.ia_attention_mfma_tiles(1)
+    close(outs[0], outs[1], 2 ** -7, "few columns")
+    want = ops.attention_generic(dev(q), dev(kc), dev(vc), dev(positions), dev(token_seq), dev(table), scale=d ** -0.5,
+                                 max_kv_len=max(lens), window=extra.get("window"), **{k: v for k, v in extra.items() if k != "window"})
+    close(outs[0], want.float().cpu(), 2 ** -7, "few columns and the plain kernel")
+
+
 @pytest.mark.parametrize("nq,nkv,d,dv_,page,window,mask_chunk,rot,gate,own", [
     (16, 4, 128, 64, 16, 40, None, 64, "feature", True),       # values narrower than keys, half of a head rotating
     (16, 4, 128, 64, 16, 300, None, 64, "feature", False),     # a layer that reads another's cache: rows [q | g]
