@@ -1810,11 +1810,12 @@ static int attention_launch(void* out, float* workspace, const void* q, const vo
         IA_LAUNCH_CHECK("attention_decode");
         return 0;
     } else if (TILE_FITS && g_tiles && (cols >= 16 * TILE_NBW * TILE_WAVES ? splits == 1 || chunk % TILE_STAGE == 0 :
-                                        splits == 1 && cols > 16 && (cols + 63) / 64 * nkv * n_seqs <= attn_cus())) {
+                                        splits == 1 && cols > 16 && max_kv_len > 32 && (cols + 63) / 64 * nkv * n_seqs <= attn_cus())) {
         // portions of prompts: blocks of four waves that share the keys through shared memory.  Portions of fewer columns than such a
         // block has too, as long as every block has a compute unit of its own: a wave alone walks its keys a step a trip to the memory
         // (a prompt of 40 tokens, two query heads a key head, 9.1 -> 6.0 us a layer, of 20 tokens 8.3 -> 5.5, of 17 behind 100 8.7 -> 6.4; in
-        // a second round of the units the other way round: 64 requests of 9 tokens 5.7 us by single waves, 11.1 by blocks).
+        // a second round of the units the other way round: 64 requests of 9 tokens 5.7 us by single waves, 11.1 by blocks; and up to 32 keys, a wave's one
+        // step, there is nothing to share: 24 tokens of five query heads a key head 5.2 and 6.1).
         // Blocks of 128 columns; of 64 (twice as many, the same bits) where the keys are not split and the blocks of 128
         // would be half a compute unit's worth or less, or, under a causal mask over most of the context, where the
         // blocks' walks differ in length, one a compute unit or less.  Measured, 32 query and 8 key/value heads, whole

@@ -893,6 +893,24 @@ def test_portions_of_few_columns_share_their_keys(nq, nkv, qs, window):
     close(outs[0], outs[1], 2 ** -7, "few columns")
 
 
+@pytest.mark.parametrize("keys", [17, 32, 33, 64])
+def test_portions_of_few_keys(keys):
+    """Either side of where blocks that share their keys begin (up to 32 keys a wave's walk is one step, with nothing to share): the bits of the kernel of
+    single waves up to there, its values beyond."""
+    from inferrs_amd import ops
+    q, kc, vc, positions, _, table = attention_case(torch.bfloat16, 10, 2, 128, 16, [keys, 17], [17, 9], 31)
+    lib, outs = ops.library("attn_d128"), []
+    for tiles in (1, 0):
+        lib.ia_attention_mfma_tiles(tiles)
+        try:
+            outs.append(ops.attention_mfma(dev(q), dev(kc), dev(vc), dev(positions), dev(torch.tensor([0, 17, 26], dtype=torch.int32)), dev(table),
+                                           max_q_len=17, max_kv_len=keys, window=None, scale=128 ** -0.5).cpu())
+        finally:
+            lib.ia_attention_mfma_tiles(1)
+    assert keys > 32 or torch.equal(*outs)
+    close(outs[0].float(), outs[1].float(), 2 ** -7, "few keys")
+
+
 @pytest.mark.parametrize("dv_,extra", [
     (128, dict(mask_chunk=100)), (128, dict(sink=True)), (128, dict(sinks=True, window=50)), (128, dict(window=60, keep_first=5)),
     (128, dict(window=33, keep_first=40, softcap=3.0)), (128, dict(softcap=5.0)), (64, {}), (64, dict(window=70, softcap=3.0)), (64, dict(mask_chunk=64, sink=True))])
