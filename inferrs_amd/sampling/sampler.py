@@ -72,9 +72,9 @@ class Sampler:
             parts.append(pack(f"{rows * n_bias}i", *[int(t) for row in pairs for t, _ in row]))
             parts.append(array("f", [v for row in pairs for _, v in row]).tobytes())
         temperature = [p.temperature for p in params]
-        if min(temperature) < SAMPLING_EPS:
+        if not min(temperature) >= SAMPLING_EPS:                 # (a temperature that is no number hides the ones behind it)
             temperature = [p.draw_temperature(n) for p, n in zip(params, lens)]
-        parts += [array("f", temperature).tobytes(), pack(f"{rows}i", *[p.top_k for p in params]),
+        parts += [array("f", temperature).tobytes(), pack(f"{rows}i", *[int(p.top_k) for p in params]),
                   array("f", [p.top_p for p in params] + [p.min_p for p in params]).tobytes()]
         front = b"".join(parts)
         at = len(front)
@@ -84,7 +84,7 @@ class Sampler:
         # the step of a draw is the number of tokens before it (`sampler.rs:323-325`); rows of temperature 0 draw nothing
         rand_f32_many(seeds, lens, host.data_ptr() + at)
         for i, t in enumerate(temperature):
-            if t < SAMPLING_EPS:
+            if not t >= SAMPLING_EPS:
                 view[at + 4 * i:at + 4 * i + 4] = b"\0\0\0\0"
         view[at + 4 * rows:] = pack(f"{rows}i", *[p.top_logprobs if p.logprobs else -1 for p in params])
         return host.to(self.device, non_blocking=True), width, n_bias, penalized
@@ -113,13 +113,13 @@ class Sampler:
             return ops.argmax(logits).cpu().tolist(), [None] * rows
 
         words, width, n_bias, penalized = self._pack(params, previous, seeds)
-        top_k = [p.top_k for p in params]
+        top_k = [int(p.top_k) for p in params]
         reports = any([p.logprobs for p in params])
         narrow = all_narrow(min(top_k), max(top_k), logits.shape[1])
         # (rows that report entries of a list which top_p or min_p may not end, to within what 32 bits round: one call for all)
         open_rows = [p for p in params if p.top_logprobs > 1 and p.top_p > 0.999 and p.min_p < 1e-6] if reports else ()
         if narrow and open_rows:
-            narrow = ops.sample_is_narrow(open_rows[0].top_k, logits.shape[1], min(p.temperature for p in open_rows), 1.0, 0.0, 2,
+            narrow = ops.sample_is_narrow(int(open_rows[0].top_k), logits.shape[1], min(p.temperature for p in open_rows), 1.0, 0.0, 2,
                                           any(p.logit_bias for p in open_rows))
         if not logits.is_contiguous():
             logits = logits.clone()

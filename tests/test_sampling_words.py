@@ -62,3 +62,19 @@ def test_words_hold_every_rows_values(case):
     for i, (prev, seed) in enumerate(zip(previous, seeds)):
         assert u[i] == (rand_f32(seed, len(prev)) if temperature[i] >= 1e-5 else 0.0)
     assert column(1, np.int32)[:, 0].tolist() == [-1] * rows and at == words.size
+
+
+def test_words_of_parameters_in_other_number_types():
+    """Whole numbers that come as floats or NumPy's, and a temperature that is no number beside rows at 0: every row as alone."""
+    params = [SamplingParams(top_k=50.0), SamplingParams(top_k=np.int64(7), temperature=np.float32(0.5)), SamplingParams(temperature=float("nan")),
+              SamplingParams(temperature=0.0), SamplingParams(temperature=0.0, repetition_penalty=1.0)]
+    previous, seeds = [(1, 2, 3), [4, 5], range(8), [6], [7]], [1, 2, 3, 4, 5]
+    words, width, _, _ = Sampler("cpu")._pack(params, previous, seeds)
+    draw = words.numpy()[-6 * len(params):].reshape(6, -1)
+    assert width == 8 and draw[1].tolist() == [50, 7, 50, 50, 50]
+    for i, (p, prev, seed) in enumerate(zip(params, previous, seeds)):
+        alone = Sampler("cpu")._pack([p], [prev], [seed])[0].numpy()[-6:]
+        assert draw[:, i].tolist() == alone.tolist()
+        t = p.draw_temperature(len(prev))
+        assert np.array_equal(draw[0, i:i + 1].view(np.float32)[0], np.float32(t), equal_nan=True)
+        assert draw[4, i:i + 1].view(np.float32)[0] == (rand_f32(seed, len(prev)) if t >= 1e-5 else 0.0)
