@@ -823,8 +823,9 @@ __device__ __forceinline__ ls_f32x4 lx_mfma(const uint4& x, const uint4& y, cons
 // x = part 0 + part 1 + part 2 exactly, each in the upper half of its word: the leading eight bits, those behind them, the rest
 __device__ __forceinline__ void lx_split(float x, uint32_t (&part)[3]) {
     part[0] = __float_as_uint(x) & 0xffff0000u;
-    // (an infinity less itself is no number: the smaller of that and a bound above every rest keeps the products infinite)
-    const float rest = fminf(x - __uint_as_float(part[0]), 0x1p120f);
+    // (an infinity less itself is no number: the smaller of that and a bound above every rest, with the infinity's sign, keeps the products
+    // infinite, also where the bound's own product overflows)
+    const float rest = copysignf(fminf(fabsf(x) - fabsf(__uint_as_float(part[0])), 0x1p120f), x);
     part[1] = __float_as_uint(rest) & 0xffff0000u;
     part[2] = __float_as_uint(rest - __uint_as_float(part[1]));
 }

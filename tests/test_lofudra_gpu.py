@@ -491,6 +491,34 @@ def test_chunks_keep_infinities(where):
     assert where == "nan" or got[0][1].isinf().any()
 
 
+@pytest.mark.parametrize("where", ["state", "values", "keys"])
+def test_infinities_of_either_sign_beside_large_factors(where):
+    """Infinite entries of both signs, all else positive and of 512: the infinities that the walk gives, with its signs, and no entry that is no number."""
+    from inferrs_amd import ops
+    n, H, dim, vdim, inf = 40, 2, 64, 64, float("inf")
+    q, k, v = (torch.full((n, H * w), 512.0).bfloat16() for w in (dim, dim, vdim))
+    start = torch.ones(1, H * vdim * dim)
+    if where == "state":
+        start[0, 5 * dim + 9], start[0, (vdim + 8) * dim + 3] = inf, -inf
+    elif where == "values":
+        v[7, 3], v[20, vdim + 6] = inf, -inf
+    else:
+        k[7, 3], k[20, dim + 6] = inf, -inf
+    got = []
+    for chunk in (None, 0):
+        state = dev(start.clone())
+        out = ops.linear_scan(q=dev(q), q_off=0, q_heads=H, k=dev(k), k_off=0, k_heads=H, v=dev(v), v_off=0, heads=H, dim=dim, vdim=vdim,
+                              state=state, s_off=0, cu_tokens=dev(torch.tensor([0, n], dtype=torch.int32)),
+                              state_slots=dev(torch.zeros(1, dtype=torch.int32)), max_q_len=n, chunk=chunk, skip=dev(torch.ones(H)),
+                              log_a=dev(torch.full((n, H), -0.01)), b=dev(torch.ones(n, H)))
+        got.append((out.cpu(), state.cpu()))
+    for new, walk in zip(*got):
+        assert not walk.isnan().any() and (walk == inf).any() and (walk == -inf).any()
+        assert torch.equal(new.isinf(), walk.isinf()) and torch.equal(new[walk.isinf()], walk[walk.isinf()])
+        finite = walk.isfinite()
+        assert float((new - walk)[finite].abs().max()) <= 2e-5 * float(walk[finite].abs().max())
+
+
 @pytest.mark.parametrize("n", [40, 100, 150])
 @pytest.mark.parametrize("where", ["values", "keys", "queries", "state"])
 def test_what_is_not_finite_stays_behind_its_token(where, n):
