@@ -482,7 +482,7 @@ __device__ __forceinline__ float column_sum(float x) {
 // features of a head turned, a gate's values behind them (the output is times their sigmoid before it is rounded), no keys at all
 // (a layer that reads another's cache; queries that a kernel before has formed).  16 query heads of 128 beside values of 64 and a gate,
 // 8 requests at 2,000 keys, window 1,024: four kernels of 5.3, 7.8, 4.5 and 4.0 us (norm and rotation, attention, merge, gate), 10.2 in
-// this one, a step of six such layers 657 -> 600 us; the single tokens of a step that also brings a portion, 40 query heads, 9 requests at 3,100
+// this one, a step of six such layers 644 -> 600 us; the single tokens of a step that also brings a portion, 40 query heads, 9 requests at 3,100
 // keys: 28.6 + 4.8 us by the kernel of single waves and its merge, 27.1 here beside nothing else.
 // A wave is mostly alone on its SIMD, so every instruction it executes is four cycles of the step (returning from the kernel early, 16 query
 // and 8 key/value heads, 700 keys, 64 a wave: rows and first keys are there 1.0 us after the start, rows formed 2.0 later, two steps done

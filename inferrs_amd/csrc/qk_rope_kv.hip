@@ -536,14 +536,6 @@ __global__ __launch_bounds__(QKV_THREADS) void qk_rope_kv_bf16_vec_kernel(
                                         pack_bf16x2(v[6], v[7]));
 }
 
-// Steps with prompt portions, where the head size is a power of two and the whole head rotates in
-// halves: the threads of a head (d / 8 of them, neighbours in one wave) walk up to QKV_HEADS heads
-// of one token.  The token's angles and the norm weights are read once for all of them, the heads'
-// rows are all asked for before the first is used, and the sum of squares and the rotation partners
-// go from lane to lane without shared memory.  The sum runs in the order of the kernel above, so
-// that both give the same bits.
-// QKV_HEADS: 8; 2 in steps of few tokens, where threads of eight heads would leave most of the chip without a block (117 tokens
-// of 24 heads: 22 blocks of queries and keys; 8.3 -> 5.2 us, the two splits of their product added up on the way).
 // The sum of a head's lanes, lane by lane from the first on, in all of them.  Sixteen lanes are a row of the vector units' exchanges,
 // which give every lane another's value without a trip through shared memory (the same order, the same bits; 117 tokens of 16 + 16
 // heads 5.2 -> 4.3 us, 459 of 32 + 16 8.9 -> 8.7).
@@ -554,6 +546,14 @@ __device__ __forceinline__ float row_total(float x, float total = 0.f) {
     else return row_total<TPU, J + 1>(x, total + __shfl(x, J, TPU));
 }
 
+// Steps with prompt portions, where the head size is a power of two and the whole head rotates in
+// halves: the threads of a head (d / 8 of them, neighbours in one wave) walk up to QKV_HEADS heads
+// of one token.  The token's angles and the norm weights are read once for all of them, the heads'
+// rows are all asked for before the first is used, and the sum of squares and the rotation partners
+// go from lane to lane without shared memory.  The sum runs in the order of the kernel above, so
+// that both give the same bits.
+// QKV_HEADS: 8; 2 in steps of few tokens, where threads of eight heads would leave most of the chip without a block (117 tokens
+// of 24 heads: 22 blocks of queries and keys; 8.3 -> 5.2 us, the two splits of their product added up on the way).
 template <int TPU, int QKV_HEADS, typename Rows>
 __global__ __launch_bounds__(QKV_THREADS) void qk_rope_kv_bf16_rows_kernel(
     bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache,
