@@ -59,6 +59,7 @@ class StepContext:
     router_logits: Any = None               # (32-bit rows, offset): the logits of the next feed-forward's router, from a product that its matrix joined
     post_rows: Any = None                   # a 32-bit stream's rows once more in the products' precision, where a part has them already (the embedding, a block's last kernel)
     decode_counters: Any = None             # the decode attention's counters (`ops.DecodeCounters`), the step builder's own
+    run_words: Any = None                 # the words of runs of layers (`ops.RunWords`), the step builder's own
     _tables: Dict[Any, Any] = field(default_factory=dict)
 
     @property
@@ -100,6 +101,7 @@ class StepBuilder:
         self._dev: Optional[torch.Tensor] = None
         self._meta = (ctypes.c_int * 16)()
         self.decode_counters = ops.DecodeCounters()     # (an engine's steps follow each other on one stream; two engines' need not)
+        self.run_words = ops.RunWords()
         self.generation = 0                # grows when the device staging buffer moves
 
     def _staging(self, n: int) -> Tuple[torch.Tensor, torch.Tensor, int]:
@@ -185,4 +187,4 @@ class StepBuilder:
             q_lens=[q_given[order[j]] for j in range(s_count)], kv_starts=flat[n + cu].tolist(),
             state_slots_host=flat[slot_off:slot_off + s_count].tolist(),
             max_q_len=meta[5], max_kv_len=meta[6], n_single=meta[7], max_kv_single=meta[8], max_kv_multi=meta[9],
-            decode_counters=self.decode_counters)
+            decode_counters=self.decode_counters, run_words=self.run_words)

@@ -10,6 +10,7 @@ import torch
 from .. import ops
 from ..config.spec import ModelSpec, SpecError
 from ..parts.base import block_class, part_class
+from ..parts.layer_run import LayerRun
 from ..parts.linear import Linear
 from ..parts.norm import build_norm
 from .batch import StepContext
@@ -54,6 +55,7 @@ class DecoderModel:
         self.final_norm = None
         if spec.final_norm is not None:
             self.final_norm = build_norm(spec.final_norm_name, spec.final_norm, tensors, dtype, device, pop=True)
+        self.layer_run = LayerRun.of_model(spec, self.blocks)
 
     @property
     def graph_safe(self) -> bool:
@@ -93,7 +95,12 @@ class DecoderModel:
         if hasattr(first, "enter"):                  # an arrangement whose stream is not the embedding's rows
             x = first.enter(ctx, x)
         pending = None                               # a block's output that is not added to x yet
+        in_run = self.layer_run.length if self.layer_run is not None and self.layer_run.takes(ctx, x, storage) else 0
+        if in_run:                                  # the first layers in one kernel, which leaves nothing to be added
+            x = self.layer_run.forward(ctx, x, storage)
         for stop, e in enumerate(self.spec.schedule):
+            if stop < in_run:
+                continue
             cache = storage.layers.get(self.spec.cache_stop(stop))
             if cache is not None and e.cache_of is not None:
                 cache = cache.reader()

@@ -764,6 +764,8 @@ class DecodeCounters(dict):
     each other (one stream, or a graph replayed on it), as an engine's steps do; every engine holds its own, so that two engines can
     run on two streams of a device."""
 
+    dtype, what = torch.int32, "attention_decode_fused: the counters of the decode kernel"
+
     def __init__(self):
         super().__init__()
         self._outgrown: list = []                   # captured graphs may still hold their addresses: kept as long as this is
@@ -776,11 +778,10 @@ class DecodeCounters(dict):
         have = self.get(key)
         if have is None or have.numel() < needed:
             if torch.cuda.is_current_stream_capturing():
-                raise KernelError("attention_decode_fused: the counters of the decode kernel cannot be allocated under "
-                                  "graph capture; run a step of this size once before capturing it")
+                raise KernelError(f"{self.what} cannot be allocated under graph capture; run a step of this size once before capturing it")
             if have is not None:
                 self._outgrown.append(have)
-            have = torch.zeros((max(DECODE_COUNTERS_MIN, 2 * needed),), dtype=torch.int32, device=device)
+            have = torch.zeros((max(DECODE_COUNTERS_MIN, 2 * needed),), dtype=self.dtype, device=device)
             self[key] = have
         return have
 
@@ -883,6 +884,88 @@ def attention_decode_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: to
         scale, splits, chunk, int(bool(sink)), int(mask_chunk or 0), _p(taken),
         taken.numel() if taken is not None else 0, _stream()), target)
     return out
+
+
+# ---- whole layers of decode steps of few rows ----------------------------------------------------
+
+class RunWords(DecodeCounters):
+    """The words through which the blocks of `layer_run` hand rows on, with its counter; as the decode kernel's counters, an engine's own."""
+    dtype, what = torch.int64, "layer_run: the words of runs of layers"
+
+
+RUN_MAX_ROWS = 8
+RUN_SHARED_BYTES = 160 * 1024 - 64
+
+
+def run_shares(max_kv_len: int) -> Tuple[int, int]:
+    """(shares, keys of a share) of a row's keys in `layer_run`."""
+    chunk = 512 * max(1, -(-max_kv_len // (512 * 32)))
+    return -(-max_kv_len // chunk), chunk
+
+
+def layer_run_fits(rows: int, width: int, ff: int, nq: int, nkv: int, page_size: int) -> bool:
+    """Whether `layer_run` takes steps of these sizes: what a wave loads at once divides the inner widths, and a step's widest rows
+    fit a compute unit's shared memory."""
+    return (1 <= rows <= RUN_MAX_ROWS and page_size == 16 and width % 512 == 0 and width <= 6144 and ff % 512 == 0 and nq % nkv == 0
+            and nq // nkv <= 8 and nq % 4 == 0 and rows * (max(width, ff, nq * 128) * 2 + 384) <= RUN_SHARED_BYTES)
+
+
+def layer_run_pays(rows: int, width: int, ff: int, nq: int, nkv: int, max_kv_len: int) -> bool:
+    """Whether a step of these sizes is faster by `layer_run` than by five kernels a layer.  What it gains is a layer's launches, first bytes and
+    last sums, which weigh less the larger the weights are, the more rows every block fetches for itself and the more keys there are (which the
+    decode attention walks with twice the waves a compute unit).  us a step, five kernels / `layer_run`: 28 layers of the 0.6B shape 8 rows at
+    3,000 keys 1,303 / 1,068, at 8,000 2,035 / 2,086, 3 rows at 14,000 1,634 / 1,492; 16 of the 4B shape 8 rows at 3,000 1,446 / 1,349, at 8,000
+    1,867 / 1,936; 10 of the 8B shape 4 rows at 3,000 1,187 / 1,157, at 8,000 1,306 / 1,366, 6 rows at 700 1,152 / 1,217; 6 of the 14B shape
+    2 rows at 3,000 1,147 / 1,099, 3 rows at 3,000 1,176 / 1,174; 5 of the 32B shape 2 rows at 14,000 1,369 / 1,348."""
+    weights = 2 * (2 * (nq + nkv) * 128 * width + 3 * width * ff)
+    if weights <= 256 << 20:
+        most, keys = 8, 44 << 10
+    elif weights <= 512 << 20:
+        most, keys = 4, 20 << 10
+    else:
+        most, keys = 2, 24 << 10
+    return rows <= most and rows * max_kv_len <= keys
+
+
+def layer_run(x: torch.Tensor, layers: Sequence[Sequence[torch.Tensor]], words: RunWords, positions: torch.Tensor, slots: torch.Tensor,
+                 block_table: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, *, nq: int, nkv: int, ff: int, max_kv_len: int,
+                 eps: Tuple[float, float, float], add_one: Tuple[bool, bool, bool], scale: float) -> torch.Tensor:
+    """A run of whole layers over the stream `x` [rows, width], in place: `layers` holds each layer's [q | k | v], o, [gate; up] and down
+    weights, the norms' weights of the stream (two) and of the heads (q, k), and its arrays of keys and values; `eps` and `add_one` are
+    those of the three kinds of norms.  Row i is the newest token of request i."""
+    _dev(x, positions, slots, block_table, cos, sin)
+    _i32(positions, "positions"); _i32(slots, "slots"); _i32(block_table, "block_table")
+    _f32(cos, "cos"); _f32(sin, "sin")
+    rows, width = x.shape
+    if x.dtype != torch.bfloat16 or not layers:
+        raise KernelError("layer_run: bfloat16 rows and one layer or more")
+    page_size = layers[0][8].shape[2]
+    if not layer_run_fits(rows, width, ff, nq, nkv, page_size):
+        raise KernelError(f"layer_run: {rows} rows of {width}, feed-forward {ff}, {nq} and {nkv} heads, pages of {page_size}")
+    shapes = ([((nq + 2 * nkv) * 128, width), (width, nq * 128), (2 * ff, width), (width, ff)], [width, width, 128, 128])
+    for of in layers:
+        _dev(*of)
+        if any(t.dtype != torch.bfloat16 or tuple(t.shape) != want for t, want in zip(of[:4], shapes[0])):
+            raise KernelError(f"layer_run: weights {[tuple(t.shape) for t in of[:4]]}, expected bfloat16 {shapes[0]}")
+        for t, want in zip(of[4:8], shapes[1]):
+            _f32(t, "norm weight")
+            if t.numel() != want:
+                raise KernelError(f"layer_run: a norm weight of {t.numel()} entries, expected {want}")
+        _check_cache(of[8], of[9], nkv, page_size, 128, x.dtype, "layer_run", 128)
+    if (positions.numel() != rows or slots.numel() != rows or block_table.dim() != 2 or block_table.shape[0] < rows
+            or cos.shape != (rows, 64) or sin.shape != cos.shape or max_kv_len > block_table.shape[1] * page_size):
+        raise KernelError("layer_run: positions, slots, block table and angles do not fit the rows")
+    splits, chunk = run_shares(max_kv_len)
+    lib = library()
+    space = words.take(x.device, int(lib.ia_layer_run_words(rows, width, ff, nq, nkv, splits)))
+    most = lib.ia_layer_run_layers()
+    for lo in range(0, len(layers), most):
+        of = layers[lo:lo + most]
+        table = (ctypes.c_void_p * (10 * len(of)))(*[t.data_ptr() for layer in of for t in layer])
+        _check(lib.ia_layer_run(
+            _p(x), ctypes.addressof(table), len(of), _p(space), space.numel(), _p(positions), _p(slots), _p(block_table), _p(cos), _p(sin), rows,
+            width, ff, nq, nkv, page_size, block_table.shape[1], splits, chunk, *eps, *(int(o) for o in add_one), scale, _stream()))
+    return x
 
 
 # ---- matrix products --------------------------------------------------------------------------
