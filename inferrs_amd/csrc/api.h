@@ -99,6 +99,11 @@ int ia_gemm_wide_dual_fits(int M, int N, int K);
 int ia_gemm_wide_norm_fits(int M, int N, int K);
 int ia_gemm_wide_rope_fits(int M, int N, int K);
 int ia_gemm_wide_plan(int mt, int splits);
+// The whole product, act: 0 none, 1 SiLU, 2 GELU in its tanh form, 3 the exact GELU (N a multiple of 4)
+int ia_gemm_wide_rows_bf16(void* out, const void* x, const void* w, int M, int N, int K, int act, hipStream_t stream);
+// (whether that is faster than the vendor's GEMM, and than that and the activation's kernel)
+int ia_gemm_wide_rows_fits(int M, int N, int K);
+int ia_gemm_wide_act_fits(int M, int N, int K);
 // Large bfloat16 products through the vendor's library, hipBLASLt, called directly (vendor_gemm.hip).  ia_vendor_gemm_init
 // opens the library at `path` (the copy the process already holds) once; ia_vendor_gemm_bf16: out [M, N] = x [M, K] . w [N, K]^T,
 // contiguous, with `workspace_bytes` of device memory for kernels that want some.

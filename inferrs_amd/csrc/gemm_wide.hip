@@ -30,11 +30,14 @@
 // 196 / 184 and 301 / 300; output projection at 256 28 / 25 and 56 / 33, at 1,024 51 / 48 and 76 / 67; gate|up with the activation, 8B
 // shape, at 320 81 / 77, at 700 165 / 135, 14B shape at 900 404 / 300.  A stage's rate over a long k is 1,270 to 1,340 TFLOP/s with
 // 160 to 240 rows a block and 1,140 with 256, at the chip's power limit (with operands of zeros a stage takes a fifth less).
+// Tiles that are shared along k between all compute units, each an equal share of the stages, were slower at every size (gate|up of the 14B
+// shape at 521 rows 209 -> 289): the blocks of a die are then at different places of k and of w, and share nothing in its L2.
 #include <type_traits>
 #include <utility>
 
 #include "common.h"
 #include "api.h"
+#include "activation.h"
 
 typedef __bf16 gw_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float gw_f32x4 __attribute__((ext_vector_type(4)));
@@ -214,27 +217,62 @@ void gemm_wide_kernel(const GemmWideParams p) {
     __builtin_amdgcn_s_waitcnt(GW_WAIT(0));                  // (nothing may still be on its way into shared memory at the end)
 
     // ---- results: the lane holds features 4 g .. + 4 of w tile a for row r of x tile b (N is a multiple of 4)
+    if constexpr (OUT == GW_F32) {
 #pragma unroll
-    for (int b = 0; b < MT; ++b) {
-        const int m = m0 + b * 16 + r;
-        if (m >= p.M) continue;
+        for (int b = 0; b < MT; ++b) {
+            const int m = m0 + b * 16 + r;
+            if (m >= p.M) continue;
 #pragma unroll
-        for (int a = 0; a < (DUAL ? 2 : 4); ++a) {
-            const int n = n0 + (DUAL ? wave * 32 : wave * 64) + a * 16 + 4 * g;
-            if (n >= p.N) continue;
-            gw_f32x4 v = acc[a][b];
-            if constexpr (DUAL) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    // the products are rounded to the storage precision before the activation, as the two-kernel way rounds them
-                    const uint32_t both = pack_bf16x2(v[i], acc[a + 2][b][i]);
-                    v[i] = gate_act(__uint_as_float(both << 16), p.act) * __uint_as_float(both & 0xffff0000u);
-                }
+            for (int a = 0; a < 4; ++a) {
+                const int n = n0 + wave * 64 + a * 16 + 4 * g;
+                if (n < p.N) *(gw_f32x4*)((float*)p.out + ((size_t)split * p.M + m) * p.N + n) = acc[a][b];
             }
-            if constexpr (OUT == GW_F32)
-                *(gw_f32x4*)((float*)p.out + ((size_t)split * p.M + m) * p.N + n) = v;
-            else
-                *(uint2*)((bf16_t*)p.out + (size_t)m * p.N + n) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        }
+    } else {
+        // The tile's rounded rows go through shared memory and out a row of the tile after the other, so that whole lines leave together: from
+        // the accumulators a store writes 32 bytes to each of 16 rows (1,500 rows of 8,512 over k of 2,048 50.9 -> 47.4 us, 16,384 over 4,096
+        // at 1,300 152 -> 147).  16 bytes behind each row, so that a lane's 16 rows fall on different banks.
+        constexpr int PITCH = FEATS * 2 + 16;
+        static_assert(BM * PITCH <= (int)sizeof(lds), "a tile's rows fit the stages' places");
+        __builtin_amdgcn_s_barrier();                        // (every wave has read its last operands, and no load is under way)
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int b = 0; b < MT; ++b) {
+#pragma unroll
+            for (int a = 0; a < (DUAL ? 2 : 4); ++a) {
+                gw_f32x4 v = acc[a][b];
+                if constexpr (DUAL) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        // the products are rounded to the storage precision before the activation, as the two-kernel way rounds them
+                        const uint32_t both = pack_bf16x2(v[i], acc[a + 2][b][i]);
+                        v[i] = gate_act(__uint_as_float(both << 16), p.act) * __uint_as_float(both & 0xffff0000u);
+                    }
+                }
+                *(uint2*)(lds + (b * 16 + r) * PITCH + (wave * (FEATS / 4) + a * 16 + 4 * g) * 2) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+            }
+        }
+        __syncthreads();
+        constexpr int LANES = FEATS / 4;                     // threads of a row, four features each
+        const int at = threadIdx.x % LANES * 4, m_end = min(BM, p.M - m0);
+        if (n0 + at >= p.N) return;
+        // an activation without a gate comes here, over the rounded values: unrolled over the accumulators the exact GELU would be 60 KB of code
+        auto rows = [&](auto act_c) __attribute__((always_inline)) {
+            constexpr int ACT = decltype(act_c)::value;
+            for (int m = threadIdx.x / LANES; m < m_end; m += 256 / LANES) {
+                uint2 q = *(const uint2*)(lds + m * PITCH + at * 2);
+                if constexpr (ACT) {
+                    q.x = pack_bf16x2(act_stored<bf16_t>(__uint_as_float(q.x << 16), ACT), act_stored<bf16_t>(__uint_as_float(q.x & 0xffff0000u), ACT));
+                    q.y = pack_bf16x2(act_stored<bf16_t>(__uint_as_float(q.y << 16), ACT), act_stored<bf16_t>(__uint_as_float(q.y & 0xffff0000u), ACT));
+                }
+                *(uint2*)((bf16_t*)p.out + (size_t)(m0 + m) * p.N + n0 + at) = q;
+            }
+        };
+        if (DUAL || p.act == 0) rows(std::integral_constant<int, 0>());
+        else if constexpr (!DUAL) {
+            if (p.act == 1) rows(std::integral_constant<int, 1>());
+            else if (p.act == 2) rows(std::integral_constant<int, 2>());
+            else rows(std::integral_constant<int, 3>());
         }
     }
 }
@@ -393,4 +431,60 @@ extern "C" int ia_gemm_wide_bf16(void* out, const void* x, const void* w, int M,
     }
     IA_LAUNCH_CHECK("gemm_wide");
     return 0;
+}
+
+// out [M, N] = x . w^T in bfloat16 with an activation over the rounded result (1 SiLU, 2 GELU in its tanh form, 3 the exact GELU; 0 none),
+// k never split.  K a multiple of 64, N of 4, operands 16-byte aligned.
+extern "C" int ia_gemm_wide_rows_bf16(void* out, const void* x, const void* w, int M, int N, int K, int act, hipStream_t stream) {
+    IA_CHECK(M > 0 && N > 0 && K > 0 && K % GW_STAGE_K == 0 && N % 4 == 0, "gemm_wide_rows: bad sizes M=%d N=%d K=%d (K a multiple of %d, N of 4)",
+             M, N, K, GW_STAGE_K);
+    IA_CHECK(act >= 0 && act <= 3, "gemm_wide_rows: unknown activation %d", act);
+    IA_CHECK((((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0, "gemm_wide_rows: operands must be 16-byte aligned");
+    IA_CHECK((long long)GW_BN * K * 2 < (1LL << 32), "gemm_wide_rows: rows of K=%d are too far apart", K);
+    const WidePlan plan = wide_plan(M, N, K, false, false);
+    GemmWideParams p;
+    p.out = out; p.x = (const bf16_t*)x; p.w = (const bf16_t*)w;
+    p.M = M; p.N = N; p.K = K; p.act = act;
+    p.tiles_m = (M + 16 * plan.mt - 1) / (16 * plan.mt);
+    p.tiles_n = (N + GW_BN - 1) / GW_BN;
+    p.stages = plan.stages;
+    const long long blocks = (long long)p.tiles_m * p.tiles_n;
+    IA_CHECK(plan.mt >= 6 && plan.stages > 0 && blocks < (1LL << 31), "gemm_wide_rows: %lld blocks", blocks);
+    switch (plan.mt) {
+#define GW_CASE(MT) case MT: gemm_wide_kernel<MT, GW_BF16><<<(unsigned)blocks, 256, 0, stream>>>(p); break;
+    GW_CASE(6) GW_CASE(7) GW_CASE(8) GW_CASE(9) GW_CASE(10) GW_CASE(11) GW_CASE(12) GW_CASE(13) GW_CASE(14) GW_CASE(15) GW_CASE(16)
+#undef GW_CASE
+    }
+    IA_LAUNCH_CHECK("gemm_wide_rows");
+    return 0;
+}
+
+// What the vendor's GEMM takes for whole rows (us): a round of the chip with blocks of 256 x 256 at 1.49 us a stage where they fill it, less
+// where smaller blocks share the work out, and at least 1.4 rounds beyond one.  Fitted to 150 sizes (150 to 2,048 rows, 2,064 to 16,928
+// features, k 1,024 to 4,096, in graphs that walk more weights than the caches hold): within a tenth for the most part; with features that
+// are no multiple of 256 the library is 1.0 to 1.7 times that slow.
+static double vendor_rows_us(int M, int N, int K) {
+    const double rounds = (double)((M + 255) / 256) * ((N + 255) / 256) / wide_cus();
+    return (rounds <= 1.0 ? 0.38 + 0.6 * rounds : rounds > 1.4 ? rounds : 1.4) * (K / GW_STAGE_K * 1.49 + 3.0);
+}
+
+// Whether a product whose whole rows are wanted goes here instead of to the vendor's GEMM.  us, the vendor's / this: 8,512 features over 2,048,
+// 600 rows 30.6 / 27.1, 1,500 54.3 / 47.4, 2,048 82 / 66; 4,304 over 1,024, 1,000 rows 18.3 / 13.5; 16,928 over 4,096, 1,300 rows 214 /
+// 152; of even ones 8,192 over 2,048, 1,000 rows 35.1 / 32.6, 10,240 over 2,560, 800 rows 51.4 / 45.8.  Not where the library's blocks fill their
+// rounds (8,192 over 2,048, 2,048 rows 50.9 / 61.3).  Of the 105 sizes of 512 rows and more it takes none that loses more than 2 %.  (Two rounds of
+// this kernel over a long k take 7 % longer than its stages add up to: 34,816 over 5,120 at 521 rows 187 / 205.)
+extern "C" int ia_gemm_wide_rows_fits(int M, int N, int K) {
+    if (M < 512 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
+    const WidePlan plan = gw_plan(M, N, K, false, false);
+    const bool one_round = (long long)((M + 16 * plan.mt - 1) / (16 * plan.mt)) * ((N + GW_BN - 1) / GW_BN) <= wide_cus();
+    return plan.cost <= (N % 256 ? 1.2 : one_round ? 1.02 : 0.95) * vendor_rows_us(M, N, K);
+}
+
+// The same with an activation, which costs this kernel a few microseconds at its end (four waves a unit form it: 8,192 features, 1,500 rows,
+// exact GELU, 8) and the other way a kernel (11.4 there).  8,192 over 2,048, 1,500 rows 55.3 / 51.3, 1,000 43.7 / 38.3; 4,096 over 1,024,
+// 2,048 rows 28.9 / 25.1; 16,384 over 4,096, 800 rows 106 / 91.
+extern "C" int ia_gemm_wide_act_fits(int M, int N, int K) {
+    if (M < 512 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
+    const double values = (double)M * N;
+    return gw_plan(M, N, K, false, false).cost + 3.0 + values * 3.5e-7 <= vendor_rows_us(M, N, K) + 2.5 + values * 8e-7;
 }

@@ -1379,6 +1379,31 @@ def gemm_wide_bf16(x: torch.Tensor, w: torch.Tensor, dual: bool = False, partial
     return out
 
 
+def gemm_wide_rows(x: torch.Tensor, w: torch.Tensor, act: int = 0) -> torch.Tensor:
+    """x [m, k] . w[n, k]^T in bfloat16 with an activation of `state.activation` (0: none) over the rounded result (k a multiple of 64, n of 4)."""
+    _dev(x, w)
+    m, k = x.shape
+    n, k2 = w.shape
+    if (k2 != k or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or m < 1 or k % 64 or n % 4
+            or not (x.is_contiguous() and w.is_contiguous())):
+        raise KernelError(f"gemm_wide_rows: x {tuple(x.shape)} {x.dtype} does not fit w {tuple(w.shape)} {w.dtype}")
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    _check(library().ia_gemm_wide_rows_bf16(_p(out), _p(x), _p(w), m, n, k, act, _stream()))
+    return out
+
+
+def activated_linear(x, w: torch.Tensor, act: int) -> torch.Tensor:
+    """An activation of `state.activation` over x . w^T: inside the product where that is faster."""
+    if isinstance(x, torch.Tensor) and _wide_takes("act", x, w):
+        return gemm_wide_rows(x, w, act)
+    return activation(linear(x, w), act)
+
+
+def _wide_takes(rule: str, x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (x.shape[0] > MID_MAX_ROWS and x.dim() == 2 and w.shape[0] % 4 == 0 and _wide_pays(rule, x.shape[0], w.shape[0], x.shape[1])
+            and wide_fits(x, w))
+
+
 @functools.lru_cache(maxsize=4096)
 def _wide_pays(reader: str, m: int, n: int, k: int) -> bool:
     """gemm_wide.hip's rule for `m` rows, `n` features and k ahead of a reader ("norm", "rope", or "dual": [gate; up] of n features
@@ -1425,7 +1450,8 @@ def linear(x, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None, mid: boo
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [m, k] . w[n, k]^T (+ bias [n], in the precision of w).  32-bit: `gemm_tiled` (true 32-bit, fixed order).
     bfloat16: the skinny MFMA kernel for up to SKINNY_MAX_ROWS rows, the vendor's GEMM beyond that (the reference uses
-    cuBLAS for all of them; products that `linear_partials` or `gated_linear` send to gemm_wide.hip do not come here).
+    cuBLAS for all of them) or, from 512 rows on where that is faster, gemm_wide.hip (products that `linear_partials` or `gated_linear`
+    send there do not come here).
     A 32-bit result of bfloat16 operands (logits) comes straight from the skinny kernel's accumulators for those few
     rows; beyond that it is the vendor's bfloat16 result widened, which is what the reference does for every row (its
     logits are computed in the model's precision and cast for sampling, `inferrs/src/sampler.rs:182`).  From
@@ -1463,6 +1489,8 @@ def _linear_no_bias(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, mi
             return gemm_mid_bf16(x, w, torch.float32)
         y = gemm_mid_bf16(x, w, partial=True)
         return y.materialize() if isinstance(y, Partials) else y
+    if out_dtype == torch.bfloat16 and _wide_takes("rows", x, w):
+        return gemm_wide_rows(x, w)
     _dev(x, w)
     if w.shape[1] != k or w.dtype != x.dtype:
         raise KernelError(f"gemm: x {tuple(x.shape)} {x.dtype} does not fit w {tuple(w.shape)} {w.dtype}")

@@ -82,4 +82,4 @@ class DenseMlp(FeedForward):
     def forward(self, ctx, h):
         if hasattr(h, "materialize"):
             h = h.materialize()
-        return self.down(ops.activation(self.up(h), self.ACTIVATIONS[self.spec.activation]))
+        return self.down(ops.activated_linear(h, self.up.weight, self.ACTIVATIONS[self.spec.activation]))

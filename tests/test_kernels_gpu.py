@@ -1555,6 +1555,45 @@ def test_wide_product_in_every_block_shape(m, n, k):
         assert torch.equal(ours, theirs), ways
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 4, 64), (129, 260, 128), (161, 508, 192), (513, 1028, 256), (2047, 772, 640)])
+def test_wide_product_with_an_activation_in_every_block_shape(m, n, k):
+    """Whole rows at sizes that end inside tiles of rows and of features, every number of rows a block: the exact product within its storage's
+    rounding, and every activation with the bits of its own kernel behind the plain product."""
+    from inferrs_amd import ops
+    lib = ops.library()
+    x, w = randn(m, k, dtype=torch.bfloat16, seed=1), randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.3)
+    want, dx, dw = x.double() @ w.double().t(), dev(x), dev(w)
+    try:
+        for mt in range(6, 17):
+            assert lib.ia_gemm_wide_plan(mt, 1) == 0
+            plain = ops.gemm_wide_rows(dx, dw)
+            close(plain, want, 2 ** -8, ("stored", mt))
+            assert torch.equal(plain, ops.gemm_wide_bf16(dx, dw)), mt
+            for act in (1, 2, 3):
+                assert torch.equal(ops.gemm_wide_rows(dx, dw, act), ops.activation(plain.clone(), act)), (mt, act)
+    finally:
+        lib.ia_gemm_wide_plan(0, 0)
+    out = torch.empty((m, n), dtype=torch.bfloat16, device="cuda:0")
+    assert lib.ia_gemm_wide_rows_bf16(out.data_ptr(), dx.data_ptr(), dw.data_ptr(), m, n, k, 4, 0) != 0
+
+
+@pytest.mark.parametrize("m,n,k,own", [(511, 8512, 2048, False), (512, 8512, 2048, True), (1500, 8512, 2048, True), (2048, 8192, 2048, False),
+                                       (2049, 8512, 2048, False)])
+def test_whole_rows_take_the_measured_route(m, n, k, own):
+    """Both sides of the rule give the product, and the product with an activation."""
+    from inferrs_amd import ops
+    x, w = dev(randn(m, k, dtype=torch.bfloat16, seed=1)), dev(randn(n, k, dtype=torch.bfloat16, seed=2, scale=0.05))
+    assert ops._wide_takes("rows", x, w) == own
+    got = ops.linear(x, w)
+    if own:
+        assert torch.equal(got, ops.gemm_wide_rows(x, w))
+    rows = slice(m - 40, m)
+    want = x[rows].double().cpu() @ w.double().cpu().t()
+    close(got[rows], want, 2 ** -8, (m, n, k))
+    # (two roundings of 2^-9 of values that an activation of slope up to 1.13 and then its own rounding follow)
+    close(ops.activated_linear(x, w, 3)[rows], torch.nn.functional.gelu(want), 3 * 2 ** -8, ("gelu", m, n, k))
+
+
 @pytest.mark.parametrize("m,n,k,split", [(512, 1024, 2048, True), (1024, 1024, 2048, None), (160, 2560, 4096, True), (521, 4096, 4096, True),
                                          (160, 4096, 12288, True), (1536, 5120, 17408, False)])
 def test_product_ahead_of_the_streams_norm_takes_the_measured_route(m, n, k, split):
