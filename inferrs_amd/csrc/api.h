@@ -94,6 +94,7 @@ int ia_gemm_skinny_bf16(void* out, const void* x, const void* w, const void* bia
 int ia_gemm_wide_bf16(void* out, const void* x, const void* w, int M, int N, int K, int out_mode, int dual, hipStream_t stream);
 int ia_gemm_wide_splits(int M, int N, int K);
 int ia_gemm_wide_dual_fits(int M, int N, int K);
+int ia_gemm_wide_narrow_fits(int M, int N, int K);
 // (whether that is faster than the vendor's GEMM: for the kernel that adds the product to the stream and norms it, and for the one
 // that norms and turns queries and keys)
 int ia_gemm_wide_norm_fits(int M, int N, int K);

@@ -9,7 +9,7 @@
 // whoever reads them (gemm_mid.hip's readers: the kernel that adds a product to the residual stream and norms it, or
 // ia_sum_partials).  A block's rows of x come in steps of 16, so that 521 rows do not pay for 768 (gw_plan below).
 //
-// A block of four waves, one a SIMD, owns 16 MT rows of x by 256 rows of w and a range of k.  A wave multiplies 64 of the
+// A block of four waves, one a SIMD, owns 16 MT rows of x by 256 rows of w (or 192: ia_gemm_wide_narrow_fits) and a range of k.  A wave multiplies 64 of the
 // rows of w (four MFMA A-operands, v_mfma_f32_16x16x32_bf16) with all of the block's rows of x: MT + 4 operand reads from
 // shared memory for 4 MT products.  Stages of 64 k (whole lines of 128 bytes a row: a load of 1 KiB takes the compute unit's
 // address unit 18 cycles, in rows of 64 bytes 37) go from memory straight into shared memory (global_load_lds), two places
@@ -42,7 +42,8 @@
 typedef __bf16 gw_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float gw_f32x4 __attribute__((ext_vector_type(4)));
 
-#define GW_BN 256                            // rows of w of a block
+#define GW_BN 256                            // rows of w of a block at most
+#define GW_NARROW_MT 21                      // tiles of 16 rows of x of a block of 192 rows of w, at most (its stages fill the shared memory)
 #define GW_STAGE_K 64                        // k of a stage: two steps of the matrix instruction
 #define GW_ROW 128                           // bytes of a staged row
 
@@ -72,17 +73,20 @@ __device__ __forceinline__ void gw_unrolled(std::integer_sequence<int, I...>, Fn
 
 enum { GW_BF16 = 0, GW_F32 = 1, GW_DUAL = 2 };          // what leaves the kernel; GW_F32: a split's sums
 
-template <int MT, int OUT>
+// NA: tiles of 16 rows of w that a wave owns, 4 or (with the activation inside) 3.
+template <int MT, int OUT, int NA = 4>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void gemm_wide_kernel(const GemmWideParams p) {
     constexpr bool DUAL = OUT == GW_DUAL;
     constexpr int BM = 16 * MT;
-    constexpr int XL = (MT + 1) / 2, WL = 8;                 // a wave's loads of 1 KiB (8 rows) for a stage's rows of x and of w
+    constexpr int BN = 64 * NA;                              // rows of w of a block
+    constexpr int XL = (MT + 1) / 2, WL = 2 * NA;               // a wave's loads of 1 KiB (8 rows) for a stage's rows of x and of w
     constexpr int W1 = MT - XL < WL ? MT - XL : WL;          // (an odd MT: the last ones of x fetch a row again into a place nobody reads)
     constexpr uint32_t X_STAGE = XL * 4 * 1024, W_STAGE = WL * 4 * 1024, W_AT = 2 * X_STAGE;
     static_assert(2 * X_STAGE + 3 * W_STAGE <= 160 * 1024, "the stages fit a compute unit's shared memory");
     static_assert(WL - W1 <= MT, "a group has room for a load");
-    constexpr int FEATS = DUAL ? GW_BN / 2 : GW_BN;          // output features of a block
+    static_assert(NA == 4 || (NA == 3 && DUAL), "blocks of 192 rows of w are those of the activation inside");
+    constexpr int FEATS = DUAL ? BN / 2 : BN;                // output features of a block
     __shared__ __attribute__((aligned(1024))) char lds[2 * X_STAGE + 3 * W_STAGE];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -116,8 +120,8 @@ void gemm_wide_kernel(const GemmWideParams p) {
         const int row = 8 * (4 * i + wave) + (lane >> 3);
         int at;
         if (DUAL) {
-            const int q = row & 63, part = q >> 5;           // a wave's 64 rows: 32 of gate, then the same 32 of up
-            at = min((row >> 6) * 32 + (q & 31), p.N - 1 - n0) + part * p.N;
+            // a tile's 16 rows: two of gate and the same two of up in turn, so that a lane's four sums are two pairs
+            at = min((row >> 4) * 8 + ((row >> 2) & 3) * 2 + (row & 1), p.N - 1 - n0) + ((row >> 1) & 1) * p.N;
         } else {
             at = min(row, p.N - 1 - n0);
         }
@@ -139,23 +143,23 @@ void gemm_wide_kernel(const GemmWideParams p) {
         if constexpr (i >= 0 && i < WL) gw_load16(wbase + k, woff[i], lds0 + W_AT + slot + (uint32_t)(4 * i + wave) * 1024);
     };
 
-    gw_f32x4 acc[4][MT];
+    gw_f32x4 acc[NA][MT];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < NA; ++a)
 #pragma unroll
         for (int b = 0; b < MT; ++b) acc[a][b] = (gw_f32x4){0.f, 0.f, 0.f, 0.f};
-    uint4 fw[2][4], fx[2][MT];
+    uint4 fw[2][NA], fx[2][MT];
     // the lane's place in a tile of 16 rows, for the two steps of a stage
     const uint32_t in_tile[2] = {(uint32_t)(r * GW_ROW + ((g ^ ((r >> 1) & 7)) * 16)),
                                  (uint32_t)(r * GW_ROW + (((4 + g) ^ ((r >> 1) & 7)) * 16))};
-    const uint32_t w_rows = W_AT + (uint32_t)(64 * wave) * GW_ROW;
-    // read i of a step's MT + 4 operands: the rows of w first
+    const uint32_t w_rows = W_AT + (uint32_t)(16 * NA * wave) * GW_ROW;
+    // read i of a step's MT + NA operands: the rows of w first
     auto read = [&](uint32_t xslot, uint32_t wslot, int step, auto ic) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
-        if constexpr (i < 4) fw[step][i] = *(const uint4*)(lds + wslot + w_rows + in_tile[step] + i * 16 * GW_ROW);
-        else if constexpr (i < MT + 4) fx[step][i - 4] = *(const uint4*)(lds + xslot + in_tile[step] + (i - 4) * 16 * GW_ROW);
+        if constexpr (i < NA) fw[step][i] = *(const uint4*)(lds + wslot + w_rows + in_tile[step] + i * 16 * GW_ROW);
+        else if constexpr (i < MT + NA) fx[step][i - NA] = *(const uint4*)(lds + xslot + in_tile[step] + (i - NA) * 16 * GW_ROW);
     };
-    // one step: `step`'s operands are multiplied, the other step's are read, two beside each of the first groups of four
+    // one step: `step`'s operands are multiplied, the other step's are read, two beside each of the first groups of NA
     // products, and `load(b)` asks for something beside group b
     auto multiply = [&](auto step_c, uint32_t xslot, uint32_t wslot, auto load) __attribute__((always_inline)) {
         constexpr int step = decltype(step_c)::value;
@@ -165,7 +169,7 @@ void gemm_wide_kernel(const GemmWideParams p) {
             read(xslot, wslot, 1 - step, std::integral_constant<int, 2 * b + 1>());
             load(bc);
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+            for (int a = 0; a < NA; ++a)
                 acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gw_bf16x8, fw[step][a]),
                                                                     __builtin_bit_cast(gw_bf16x8, fx[step][b]), acc[a][b], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
@@ -186,7 +190,7 @@ void gemm_wide_kernel(const GemmWideParams p) {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     uint32_t xs = 0, wh = 0, wn = W_STAGE, wl = 2 * W_STAGE;     // places: this stage's x; w of this stage, the next, the one behind it
-    gw_unrolled(std::make_integer_sequence<int, MT + 4>(), [&](auto i) __attribute__((always_inline)) { read(0, 0, 0, i); });
+    gw_unrolled(std::make_integer_sequence<int, MT + NA>(), [&](auto i) __attribute__((always_inline)) { read(0, 0, 0, i); });
     size_t k_w = k_of(2);
     for (int s = 0; s < stages; ++s) {
         // the stage's first step; the rest of w of stage s + 2 is asked for
@@ -211,7 +215,7 @@ void gemm_wide_kernel(const GemmWideParams p) {
     }
     // (without this the compiler carries half of the accumulators through copies, 3 moves for every two products)
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < NA; ++a)
 #pragma unroll
         for (int b = 0; b < MT; ++b) asm volatile("" : "+a"(acc[a][b]));
     __builtin_amdgcn_s_waitcnt(GW_WAIT(0));                  // (nothing may still be on its way into shared memory at the end)
@@ -256,23 +260,27 @@ void gemm_wide_kernel(const GemmWideParams p) {
 #pragma unroll
         for (int b = 0; b < MT; ++b) {
 #pragma unroll
-            for (int a = 0; a < (DUAL ? 2 : 4); ++a) {
-                gw_f32x4 v = acc[a][b];
+            for (int a = 0; a < NA; ++a) {
+                const gw_f32x4 v = acc[a][b];
+                char* const at = lds + (b * 16 + r) * PITCH + (wave * (FEATS / 4) + (DUAL ? a * 8 + 2 * g : a * 16 + 4 * g)) * 2;
                 if constexpr (DUAL) {
+                    float z[2];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
+                    for (int i = 0; i < 2; ++i) {
                         // the products are rounded to the storage precision before the activation, as the two-kernel way rounds them
-                        const uint32_t both = pack_bf16x2(v[i], acc[a + 2][b][i]);
-                        v[i] = gate_act(__uint_as_float(both << 16), p.act) * __uint_as_float(both & 0xffff0000u);
+                        const uint32_t both = pack_bf16x2(v[i], v[2 + i]);
+                        z[i] = gate_act(__uint_as_float(both << 16), p.act) * __uint_as_float(both & 0xffff0000u);
                     }
+                    *(uint32_t*)at = pack_bf16x2(z[0], z[1]);
+                } else {
+                    *(uint2*)at = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
                 }
-                *(uint2*)(lds + (b * 16 + r) * PITCH + (wave * (FEATS / 4) + a * 16 + 4 * g) * 2) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
             }
         }
         __syncthreads();
         constexpr int LANES = FEATS / 4;                     // threads of a row, four features each
         const int at = threadIdx.x % LANES * 4, m_end = min(BM, p.M - m0);
-        if (n0 + at >= p.N) return;
+        if (n0 + at >= p.N || threadIdx.x >= 256 / LANES * LANES) return;
         // an activation without a gate comes here, over the rounded values: unrolled over the accumulators the exact GELU would be 60 KB of code
         auto rows = [&](auto act_c) __attribute__((always_inline)) {
             constexpr int ACT = decltype(act_c)::value;
@@ -295,8 +303,8 @@ void gemm_wide_kernel(const GemmWideParams p) {
 }
 
 // How a product is shared out: rows of x a block (16 mt), ways k is split, stages of a split.
-struct WidePlan { int mt, splits, stages; double cost; };
-static WidePlan g_wide_forced = {0, 0, 0, 0.0};
+struct WidePlan { int mt, splits, stages; double cost; int na; };
+static WidePlan g_wide_forced = {0, 0, 0, 0.0, 4};
 static int wide_cus() {
     static int cus = 0;
     if (cus == 0) {
@@ -308,38 +316,46 @@ static int wide_cus() {
 // A stage of 64 k, measured with every compute unit at work, rows of 16 mt (us): the memory's latency up to 8, then the matrix
 // pipes at the clock that the chip's power leaves them.
 static const double gw_stage_us[11] = {0.83, 0.89, 0.93, 1.00, 1.05, 1.16, 1.20, 1.32, 1.41, 1.55, 1.89};
-static WidePlan gw_plan(int M, int N, int K, bool dual, bool may_split) {
-    const int cus = wide_cus(), feats = dual ? GW_BN / 2 : GW_BN;
-    WidePlan best = {0, 0, 0, 1e30};
-    const long long tiles_n = (N + feats - 1) / feats;
-    const int stages = K / GW_STAGE_K;
-    for (int mt = 6; mt <= 16; ++mt) {
-        const long long tiles_m = (M + 16 * mt - 1) / (16 * mt);
-        for (int splits = 1; splits <= (may_split && !dual ? 8 : 1); ++splits) {
-            const int each = (stages + splits - 1) / splits;
-            if (splits > 1 && each < 8) break;
-            if ((splits - 1) * each >= stages) continue;
-            const long long rounds = (tiles_m * tiles_n * splits + cus - 1) / cus;
-            // in us: a block's stages, its start and its end, and the splits' sums on their way out and back in
-            const double cost = (double)rounds * (each * gw_stage_us[mt - 6] + 3.0) + (splits > 1 ? 1.0 + 0.42e-6 * splits * M * N * 4.0 : 0.0);
-            if (cost < best.cost) best = {mt, splits, each, cost};
+// Blocks of 192 rows of w: by what their stages took in products of one and two rounds, on the scale of the others.
+static const double gw_narrow_us[16] = {0.75, 0.79, 0.82, 0.88, 0.95, 0.99, 1.08, 1.17, 1.24, 1.38, 1.43, 1.50, 1.57, 1.64, 1.76, 1.83};
+static WidePlan gw_plan(int M, int N, int K, bool dual, bool may_split, bool may_narrow = true) {
+    const int cus = wide_cus(), stages = K / GW_STAGE_K;
+    WidePlan best = {0, 0, 0, 1e30, 4};
+    for (int na = 4; na >= (dual && may_narrow ? 3 : 4); --na) {
+        const int feats = 64 * na / (dual ? 2 : 1);
+        const long long tiles_n = (N + feats - 1) / feats;
+        for (int mt = 6; mt <= (na == 3 ? GW_NARROW_MT : 16); ++mt) {
+            const long long tiles_m = (M + 16 * mt - 1) / (16 * mt);
+            for (int splits = 1; splits <= (may_split && !dual ? 8 : 1); ++splits) {
+                const int each = (stages + splits - 1) / splits;
+                if (splits > 1 && each < 8) break;
+                if ((splits - 1) * each >= stages) continue;
+                const long long rounds = (tiles_m * tiles_n * splits + cus - 1) / cus;
+                // in us: a block's stages, its start and its end, and the splits' sums on their way out and back in
+                const double stage_us = na == 3 ? gw_narrow_us[mt - 6] : gw_stage_us[mt - 6];
+                const double cost = (double)rounds * (each * stage_us + 3.0) + (splits > 1 ? 1.0 + 0.42e-6 * splits * M * N * 4.0 : 0.0);
+                if (cost < best.cost) best = {mt, splits, each, cost, na};
+            }
         }
     }
     return best;
 }
 
-// (a plan for measurements and tests: blocks of 16 mt rows, k split `splits` ways; 0, 0: the plan's own)
+// (a plan for measurements and tests: blocks of 16 mt rows, k split `splits` ways; mt + 32: those of 192 rows of w, for the activation
+// inside; 0, 0: the plan's own)
 extern "C" int ia_gemm_wide_plan(int mt, int splits) {
-    IA_CHECK((mt == 0 && splits == 0) || (mt >= 6 && mt <= 16 && splits >= 1 && splits <= 8),
+    const bool narrow = mt > 32;
+    IA_CHECK((mt == 0 && splits == 0) || (mt >= 6 && mt <= 16 && splits >= 1 && splits <= 8) || (mt >= 38 && mt <= 32 + GW_NARROW_MT && splits == 1),
              "gemm_wide_plan: no blocks of %d rows with %d splits of k", 16 * mt, splits);
-    g_wide_forced = {mt, splits, 0, 0.0};
+    g_wide_forced = {narrow ? mt - 32 : mt, splits, 0, 0.0, narrow ? 3 : 4};
     return 0;
 }
 
 static WidePlan wide_plan(int M, int N, int K, bool dual, bool may_split) {
     WidePlan p = gw_plan(M, N, K, dual, may_split);
-    if (g_wide_forced.mt) {
+    if (g_wide_forced.mt && (dual || g_wide_forced.na == 4)) {
         p.mt = g_wide_forced.mt;
+        p.na = g_wide_forced.na;
         int splits = may_split && !dual ? g_wide_forced.splits : 1;
         const int stages = K / GW_STAGE_K;
         if (splits > stages) splits = stages;
@@ -403,9 +419,10 @@ extern "C" int ia_gemm_wide_rope_fits(int M, int N, int K) {
 // 243, 700 rows 436 / 412, 14B shape, 900 rows 934 / 831, 32B shape, 1,024 rows 1,222 / 1,167; of the 63 points of wide shapes where the
 // rule says yes ten are slower by more than half a percent, 1.2 at most.  It still refuses some that would gain (14B shape, 580 rows
 // 692 / 662, 32B shape, 400 rows 803 / 773).
+// (Said of blocks of 256 rows of w; ia_gemm_wide_narrow_fits says where those of 192 do better than the vendor's.)
 extern "C" int ia_gemm_wide_dual_fits(int M, int N, int K) {
     if (M <= 0 || M > 1024 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4 || ((long long)N + GW_BN) * K * 2 >= (1LL << 32)) return 0;
-    const WidePlan plan = gw_plan(M, N, K, true, false);
+    const WidePlan plan = gw_plan(M, N, K, true, false, false);
     if (!host_bound(M, K)) {
         const long long cus = wide_cus(), tiles_m = (M + 16 * plan.mt - 1) / (16 * plan.mt), tiles_n = (N + GW_BN / 2 - 1) / (GW_BN / 2);
         const long long ours = (tiles_m * tiles_n + cus - 1) / cus * cus;                  // (blocks that this kernel's rounds have room for)
@@ -429,7 +446,7 @@ extern "C" int ia_gemm_wide_bf16(void* out, const void* x, const void* w, int M,
     // (a lane's offset from its block's first row is 32 bits wide)
     IA_CHECK(((dual ? (long long)N : 0) + GW_BN) * K * 2 < (1LL << 32), "gemm_wide: N=%d rows of K=%d are too far apart", N, K);
     const WidePlan plan = wide_plan(M, N, K, dual != 0, out_mode == 2);
-    const int feats = dual ? GW_BN / 2 : GW_BN;
+    const int feats = 64 * plan.na / (dual ? 2 : 1);
     GemmWideParams p;
     p.out = out; p.x = (const bf16_t*)x; p.w = (const bf16_t*)w;
     p.M = M; p.N = N; p.K = K; p.act = dual;
@@ -438,6 +455,16 @@ extern "C" int ia_gemm_wide_bf16(void* out, const void* x, const void* w, int M,
     p.stages = plan.stages;
     const long long blocks = (long long)p.tiles_m * p.tiles_n * plan.splits;
     IA_CHECK(plan.mt >= 6 && plan.stages > 0 && blocks < (1LL << 31), "gemm_wide: %lld blocks", blocks);
+    if (plan.na == 3) {
+        switch (plan.mt) {
+#define GW_CASE(MT) case MT: gemm_wide_kernel<MT, GW_DUAL, 3><<<(unsigned)blocks, 256, 0, stream>>>(p); break;
+        GW_CASE(6) GW_CASE(7) GW_CASE(8) GW_CASE(9) GW_CASE(10) GW_CASE(11) GW_CASE(12) GW_CASE(13) GW_CASE(14) GW_CASE(15) GW_CASE(16)
+        GW_CASE(17) GW_CASE(18) GW_CASE(19) GW_CASE(20) GW_CASE(21)
+#undef GW_CASE
+        }
+        IA_LAUNCH_CHECK("gemm_wide");
+        return 0;
+    }
     switch (plan.mt) {
 #define GW_CASE(MT) \
     case MT: if (dual) gemm_wide_kernel<MT, GW_DUAL><<<(unsigned)blocks, 256, 0, stream>>>(p); \
@@ -504,4 +531,15 @@ extern "C" int ia_gemm_wide_act_fits(int M, int N, int K) {
     if (M < 512 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
     const double values = (double)M * N;
     return gw_plan(M, N, K, false, false).cost + 3.0 + values * 3.5e-7 <= vendor_rows_us(M, N, K) + 2.5 + values * 8e-7;
+}
+
+// Whether a [gate; up] of N features each goes here in blocks of 192 rows of w: widths of 3 x 2^i make whole rounds of them (12,288 features
+// 128 tiles, so that two tiles of up to 336 rows of x are one block for every compute unit, where blocks of 256 x 256 leave a quarter of the chip idle or a
+// second round nearly empty).  us with the activation, the vendor's / blocks of 256 / of 192: 12,288 over 4,096, 200 rows 66 / 65 / 57, 300 76 / 73 /
+// 69, 459 95.6 / 101 / 97.9, 521 133 / 121 / 107, 600 133 / 127 / 117; 17,408 over 5,120, 150 rows 113 / 116 / 98.5, 260 159 / 165 / 122, 330 169 /
+// 181 / 141; 6,144 over 2,048, 400 rows 36.6 / 32.2 / 30.3.
+extern "C" int ia_gemm_wide_narrow_fits(int M, int N, int K) {
+    if (M <= 0 || M > 1024 || N < 2048 || K <= 0 || K % GW_STAGE_K || N % 4 || ((long long)N + GW_BN) * K * 2 >= (1LL << 32)) return 0;
+    const WidePlan plan = gw_plan(M, N, K, true, false);
+    return plan.na == 3 && plan.cost <= 0.97 * (vendor_rows_us(M, 2 * N, K) + 2.5 + (double)M * N * 1.2e-6);
 }

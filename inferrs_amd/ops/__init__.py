@@ -1686,7 +1686,8 @@ def gated_linear(x, w_gate_up: torch.Tensor, activation: str = "silu",
                 and w_gate_up.numel() * w_gate_up.element_size() <= MID_DUAL_MAX_BYTES):
             return gemm_mid_bf16(x, w_gate_up, dual=True, activation=activation)
         if (x.shape[0] > MID_MAX_ROWS and w_gate_up.shape[0] % 8 == 0
-                and _wide_pays("dual", x.shape[0], w_gate_up.shape[0] // 2, x.shape[1]) and wide_fits(x, w_gate_up)):
+                and any(_wide_pays(rule, x.shape[0], w_gate_up.shape[0] // 2, x.shape[1]) for rule in ("dual", "narrow"))
+                and wide_fits(x, w_gate_up)):
             return gemm_wide_bf16(x, w_gate_up, dual=True, activation=activation)
         if even and x.dtype == torch.bfloat16 and skinny_fits(x, w_gate_up) and _own_large(x, w_gate_up):
             return gemm_mfma_bf16(x, w_gate_up, dual=True, activation=activation)

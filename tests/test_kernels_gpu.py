@@ -1594,6 +1594,27 @@ def test_whole_rows_take_the_measured_route(m, n, k, own):
     close(ops.activated_linear(x, w, 3)[rows], torch.nn.functional.gelu(want), 3 * 2 ** -8, ("gelu", m, n, k))
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 4, 64), (129, 100, 128), (337, 196, 192), (600, 1156, 640)])
+def test_wide_product_in_blocks_of_192_rows_of_w(m, n, k):
+    """[gate; up] in every number of rows that such a block takes, at sizes that end inside tiles of rows and of features, against blocks of 256
+    (the same sums in the same order, but for where a block starts its walk of k) and the exact product."""
+    from inferrs_amd import ops
+    lib = ops.library()
+    x, w = randn(m, k, dtype=torch.bfloat16, seed=1), randn(2 * n, k, dtype=torch.bfloat16, seed=2, scale=0.05)
+    gate, up = (x.double() @ w.double().t()).split(n, dim=1)
+    dx, dw = dev(x), dev(w)
+    try:
+        for mt in range(38, 54):
+            assert lib.ia_gemm_wide_plan(mt, 1) == 0
+            for name, act in (("silu", torch.nn.functional.silu), ("gelu_tanh", lambda z: torch.nn.functional.gelu(z, approximate="tanh"))):
+                # (gate, up, and what they give: three roundings of 2^-9)
+                close(ops.gemm_wide_bf16(dx, dw, dual=True, activation=name), act(gate) * up, 3 * 2 ** -8, (name, mt))
+            close(ops.gemm_wide_rows(dx, dw), x.double() @ w.double().t(), 2 ** -8, ("plain", mt))     # (keeps blocks of its own)
+        assert lib.ia_gemm_wide_plan(54, 1) != 0 and lib.ia_gemm_wide_plan(38, 2) != 0
+    finally:
+        lib.ia_gemm_wide_plan(0, 0)
+
+
 @pytest.mark.parametrize("m,n,k,split", [(512, 1024, 2048, True), (1024, 1024, 2048, None), (160, 2560, 4096, True), (521, 4096, 4096, True),
                                          (160, 4096, 12288, True), (1536, 5120, 17408, False)])
 def test_product_ahead_of_the_streams_norm_takes_the_measured_route(m, n, k, split):
