@@ -360,7 +360,7 @@ int ia_fading_scan(void* out, float* state, long long row_floats, long long s_of
                    int chunks, float* workspace, int dtype, hipStream_t stream);
 long long ia_fading_scan_workspace(int n_seqs, int chunks, int H, int dim, int vdim);
 
-// Decode steps of 1 to 4 rows: a run of whole layers (norm, q|k|v, attention, o, norm, gate|up, down; bfloat16, heads of 128, pages
+// Decode steps of 1 to 8 rows: a run of whole layers (norm, q|k|v, attention, o, norm, gate|up, down; bfloat16, heads of 128, pages
 // of 16) in one kernel.  `layers`: ten host pointers a layer (w_qkv, w_o, w_gate_up, w_down, norm 1, norm 2, q norm, k norm, keys,
 // values), ia_layer_run_layers() layers at most.  `words` holds ia_layer_run_words() 64-bit words, zero before their first
 // use and left alone between calls; calls that share them must not overlap.
