@@ -363,12 +363,13 @@ long long ia_fading_scan_workspace(int n_seqs, int chunks, int H, int dim, int v
 // Decode steps of 1 to 8 rows: a run of whole layers (norm, q|k|v, attention, o, norm, gate|up, down; bfloat16, heads of 128, pages
 // of 16) in one kernel.  `layers`: ten host pointers a layer (w_qkv, w_o, w_gate_up, w_down, norm 1, norm 2, q norm, k norm, keys,
 // values), ia_layer_run_layers() layers at most.  `words` holds ia_layer_run_words() 64-bit words, zero before their first
-// use and left alone between calls; calls that share them must not overlap.
+// use and left alone between calls; calls that share them must not overlap.  No row is longer than `max_kv_len` with its new token, which
+// `splits` shares of `chunk` keys hold; a position beyond that is read as the last one inside.
 int ia_layer_run_layers(void);
 long long ia_layer_run_words(int rows, int width, int ff, int nq, int nkv, int splits);
 int ia_layer_run(void* x, const void* layers, int n_layers, long long* words, long long n_words, const int* positions,
                     const int* slots, const int* block_table, const float* cos_t, const float* sin_t, int rows, int width,
-                    int ff, int nq, int nkv, int page_size, int max_pages, int splits, int chunk, float eps1, float eps2,
+                    int ff, int nq, int nkv, int page_size, int max_pages, int max_kv_len, int splits, int chunk, float eps1, float eps2,
                     float eps_qk, int one1, int one2, int one_qk, float scale, hipStream_t stream);
 
 // Built per head size (-DIA_HEAD_DIM) into a library of its own.

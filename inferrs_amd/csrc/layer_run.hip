@@ -60,7 +60,7 @@ struct RunArgs {
     int n_layers, per_layer;
     int b_qkv, b_attn, b_merge, b_o, b_gate_up, b_down;  // blocks of a phase (b_merge 0: keys are not split)
     int s_qkv, s_o, s_gate_up, s_down;                   // log2 of the waves that share a group of weight rows along k
-    int width, ff, nq, nkv, max_pages, splits, chunk;
+    int width, ff, nq, nkv, max_pages, splits, chunk, max_kv;
     float eps1, eps2, eps_qk, scale_log2;
     int one1, one2, one_qk;         // norms weigh with 1 + w
 };
@@ -135,6 +135,10 @@ __device__ __forceinline__ void sum_lanes(float* v) {
         v[i] += wave_lane<0x140>(v[i]);                     // the other eight of sixteen
     }
 }
+
+// The position of a row's newest token, which is the count of its cached keys, inside the bound that the launch is laid out for: beyond it a row
+// would wait for shares of its keys that no block forms, and read pages behind its table's row.
+__device__ __forceinline__ int run_last(const RunArgs& a, int row) { return min(max(a.positions[row], 0), a.max_kv - 1); }
 
 // Features 2 i and 2 i + 1 of the attention of `head` (counted over all rows), from the shares of its row's keys.
 __device__ __forceinline__ uint32_t run_merged(const RunArgs& a, int head, int i, int shares, uint32_t tag) {
@@ -278,7 +282,7 @@ __device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L,
         const bool merges = kind == RUN_O && a.splits > 1 && a.b_merge == 0;
         int shares[R];                                      // of the rows' keys
 #pragma unroll
-        for (int r = 0; r < R; ++r) shares[r] = merges ? a.positions[r] / a.chunk + 1 : 0;
+        for (int r = 0; r < R; ++r) shares[r] = merges ? run_last(a, r) / a.chunk + 1 : 0;
         watch(a.head, merges ? a.part + (size_t)(item % (R * a.nq)) * a.splits * (RUN_HD + 2) : in + (item * 37) % n, tag);
         if (merges) {
             // the shares of every head's keys come together here: few of them, and few blocks that would read them all
@@ -428,7 +432,7 @@ __device__ __forceinline__ void run_attention(const RunArgs& a, const RunLayer& 
     const int r = lane & 15, G = lane >> 4;
     const int g = a.nq / a.nkv;
     const int split = item % a.splits, of = item / a.splits, kvh = of % a.nkv, row = of / a.nkv;
-    const int last = a.positions[row];                      // the new token's own position: as many keys are cached
+    const int last = run_last(a, row);
     const int lo = split * a.chunk;
     if (lo > last) return;
     const bool has_new = last < lo + a.chunk;
@@ -660,7 +664,7 @@ __device__ __forceinline__ void run_attention(const RunArgs& a, const RunLayer& 
 // The shares of a row's keys come together: one key/value head's query heads a block, a thread a pair of features.
 __device__ __forceinline__ void run_merge(const RunArgs& a, int item, uint32_t tag) {
     const int tid = threadIdx.x, g = a.nq / a.nkv;
-    const int shares = a.positions[item / a.nkv] / a.chunk + 1;
+    const int shares = run_last(a, item / a.nkv) / a.chunk + 1;
     watch(a.head, a.part + ((size_t)(item / a.nkv) * a.nq + (item % a.nkv) * g) * a.splits * (RUN_HD + 2), tag);
     if (tid >= g * (RUN_HD / 2)) return;
     const int head = (item / a.nkv) * a.nq + (item % a.nkv) * g + tid / (RUN_HD / 2), i = tid & (RUN_HD / 2 - 1);
@@ -710,15 +714,17 @@ extern "C" int ia_layer_run_layers(void) { return RUN_LAYERS; }
 
 extern "C" int ia_layer_run(void* x, const void* layers, int n_layers, long long* words, long long n_words, const int* positions, const int* slots,
                                const int* block_table, const float* cos_t, const float* sin_t, int rows, int width, int ff, int nq, int nkv,
-                               int page_size, int max_pages, int splits, int chunk, float eps1, float eps2, float eps_qk, int one1, int one2, int one_qk,
+                               int page_size, int max_pages, int max_kv_len, int splits, int chunk, float eps1, float eps2, float eps_qk, int one1, int one2, int one_qk,
                                float scale, hipStream_t stream) {
     IA_CHECK(rows >= 1 && rows <= RUN_ROWS && n_layers >= 1 && n_layers <= RUN_LAYERS, "layer_run: %d rows, %d layers", rows, n_layers);
     IA_CHECK(width > 0 && width % RUN_UNIT == 0 && width <= 6144 && ff > 0 && ff % RUN_UNIT == 0 && nkv > 0 && nq % nkv == 0 && nq % 4 == 0
                  && nq / nkv <= 8 && (nq + 2 * nkv) % 2 == 0,
              "layer_run: width %d, feed-forward %d, %d and %d heads", width, ff, nq, nkv);
-    IA_CHECK(page_size == RUN_PAGE && max_pages >= 1 && splits >= 1 && chunk >= 32 && chunk % 32 == 0
-                 && (long long)splits * chunk >= 1 && n_words >= ia_layer_run_words(rows, width, ff, nq, nkv, splits),
-             "layer_run: pages of %d, %d shares of %d keys, %lld words", page_size, splits, chunk, n_words);
+    IA_CHECK(page_size == RUN_PAGE && max_pages >= 1 && max_kv_len >= 1 && max_kv_len <= (long long)max_pages * RUN_PAGE,
+             "layer_run: %d keys in %d pages of %d", max_kv_len, max_pages, page_size);
+    IA_CHECK(splits >= 1 && chunk >= 32 && chunk % 32 == 0 && (long long)splits * chunk >= max_kv_len
+                 && n_words >= ia_layer_run_words(rows, width, ff, nq, nkv, splits),
+             "layer_run: %d shares of %d keys for %d keys, %lld words", splits, chunk, max_kv_len, n_words);
     RunArgs a = {};
     const void* const* from = (const void* const*)layers;
     for (int i = 0; i < n_layers; ++i, from += 10) {
@@ -749,7 +755,7 @@ extern "C" int ia_layer_run(void* x, const void* layers, int n_layers, long long
     a.b_gate_up = ff / (32 >> a.s_gate_up);
     a.b_down = width / (64 >> a.s_down);
     a.per_layer = a.b_qkv + a.b_attn + a.b_merge + a.b_o + a.b_gate_up + a.b_down;
-    a.width = width; a.ff = ff; a.nq = nq; a.nkv = nkv; a.max_pages = max_pages; a.splits = splits; a.chunk = chunk;
+    a.width = width; a.ff = ff; a.nq = nq; a.nkv = nkv; a.max_pages = max_pages; a.splits = splits; a.chunk = chunk; a.max_kv = max_kv_len;
     a.eps1 = eps1; a.eps2 = eps2; a.eps_qk = eps_qk; a.scale_log2 = scale * 1.4426950408889634f;
     a.one1 = one1; a.one2 = one2; a.one_qk = one_qk;
     const int g = nq / nkv, widest = ff > nq * RUN_HD ? (ff > width ? ff : width) : (nq * RUN_HD > width ? nq * RUN_HD : width);

@@ -953,7 +953,7 @@ def layer_run(x: torch.Tensor, layers: Sequence[Sequence[torch.Tensor]], words: 
                 raise KernelError(f"layer_run: a norm weight of {t.numel()} entries, expected {want}")
         _check_cache(of[8], of[9], nkv, page_size, 128, x.dtype, "layer_run", 128)
     if (positions.numel() != rows or slots.numel() != rows or block_table.dim() != 2 or block_table.shape[0] < rows
-            or cos.shape != (rows, 64) or sin.shape != cos.shape or max_kv_len > block_table.shape[1] * page_size):
+            or cos.shape != (rows, 64) or sin.shape != cos.shape or not 0 < max_kv_len <= block_table.shape[1] * page_size):
         raise KernelError("layer_run: positions, slots, block table and angles do not fit the rows")
     splits, chunk = run_shares(max_kv_len)
     lib = library()
@@ -964,7 +964,7 @@ def layer_run(x: torch.Tensor, layers: Sequence[Sequence[torch.Tensor]], words: 
         table = (ctypes.c_void_p * (10 * len(of)))(*[t.data_ptr() for layer in of for t in layer])
         _check(lib.ia_layer_run(
             _p(x), ctypes.addressof(table), len(of), _p(space), space.numel(), _p(positions), _p(slots), _p(block_table), _p(cos), _p(sin), rows,
-            width, ff, nq, nkv, page_size, block_table.shape[1], splits, chunk, *eps, *(int(o) for o in add_one), scale, _stream()))
+            width, ff, nq, nkv, page_size, block_table.shape[1], max_kv_len, splits, chunk, *eps, *(int(o) for o in add_one), scale, _stream()))
     return x
 
 

@@ -26,6 +26,43 @@ def test_rule_of_the_sizes():
         assert chunk % 32 == 0 and splits * chunk >= keys and splits <= 32 and (splits - 1) * chunk < keys
 
 
+def _run_status(**change):
+    """`ia_layer_run` over addresses that nobody reads unless the checks on the host let them through: (status, message)."""
+    import ctypes
+    lib = ops.library()
+    a = dict(dict(rows=1, width=512, ff=512, nq=4, nkv=4, page_size=16, max_pages=40, max_kv_len=600, splits=2, chunk=512), **change)
+    of = (ctypes.c_void_p * 10)(*[4096] * 10)
+    words = lib.ia_layer_run_words(a["rows"], a["width"], a["ff"], a["nq"], a["nkv"], a["splits"])
+    status = lib.ia_layer_run(4096, ctypes.addressof(of), 1, 4096, words, *[4096] * 5, *a.values(), 1e-6, 1e-6, 1e-6, 0, 0, 0, 0.1, None)
+    return status, lib.ia_last_error().decode()
+
+
+@pytest.mark.parametrize("change", [dict(splits=1), dict(chunk=256), dict(max_kv_len=1025), dict(max_kv_len=0), dict(max_pages=37)])
+def test_bounds_that_do_not_hold_a_row_are_refused(change):
+    """Shares that do not hold the longest row, or pages that do not: such a row would wait for words that no block writes."""
+    status, message = _run_status(**change)
+    assert status == 1 and message.startswith("layer_run: ") and "keys" in message, message
+
+
+@pytest.mark.gpu
+def test_positions_beyond_the_bound_count_as_the_last_inside():
+    """A row longer than the launch is laid out for, and a negative position, read nothing outside their tables and wait for nothing."""
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    layers = _layers(gen, 2, 512, 512, 4, 2, 40)
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    x = torch.empty((2, 512), dtype=torch.bfloat16, device="cuda").normal_(0.0, 1.0, generator=gen)
+    table, cos, sin = torch.arange(80, dtype=torch.int32, device="cuda").view(2, 40) % 40, torch.ones((2, 64), device="cuda"), torch.zeros((2, 64), device="cuda")
+    kw = dict(nq=4, nkv=2, ff=512, max_kv_len=600, eps=(1e-6,) * 3, add_one=(False,) * 3, scale=HD ** -0.5)
+    kept = [(of[8].clone(), of[9].clone()) for of in layers]
+    outs = []
+    for positions in (i32(5000, -7), i32(599, 0)):
+        for of, (k, v) in zip(layers, kept):
+            of[8].copy_(k)
+            of[9].copy_(v)
+        outs.append(ops.layer_run(x.clone(), layers, ops.RunWords(), positions, i32(599, 627), table, cos, sin, **kw))
+    assert torch.equal(*outs) and torch.isfinite(outs[0].float()).all()
+
+
 def _layers(gen, n, width, ff, nq, nkv, pages):
     def draw(*shape, std=0.02, mean=0.0, dtype=torch.bfloat16):
         return torch.empty(shape, dtype=dtype, device="cuda").normal_(mean, std, generator=gen)
