@@ -362,7 +362,7 @@ long long ia_fading_scan_workspace(int n_seqs, int chunks, int H, int dim, int v
 
 // Decode steps of 1 to 8 rows: a run of whole layers (norm, q|k|v, attention, o, norm, gate|up, down; bfloat16, heads of 128, pages
 // of 16) in one kernel.  `layers`: ten host pointers a layer (w_qkv, w_o, w_gate_up, w_down, norm 1, norm 2, q norm, k norm, keys,
-// values), ia_layer_run_layers() layers at most.  `words` holds ia_layer_run_words() 64-bit words, zero before their first
+// values; 16-byte aligned, the norms' weights 8-byte), ia_layer_run_layers() layers at most.  `words` holds ia_layer_run_words() 64-bit words, zero before their first
 // use and left alone between calls; calls that share them must not overlap.  No row is longer than `max_kv_len` with its new token, which
 // `splits` shares of `chunk` keys hold; a position beyond that is read as the last one inside.
 int ia_layer_run_layers(void);

@@ -732,7 +732,12 @@ extern "C" int ia_layer_run(void* x, const void* layers, int n_layers, long long
         L.w_qkv = (const bf16_t*)from[0]; L.w_o = (const bf16_t*)from[1]; L.w_gate_up = (const bf16_t*)from[2]; L.w_down = (const bf16_t*)from[3];
         L.norm1 = (const float*)from[4]; L.norm2 = (const float*)from[5]; L.q_norm = (const float*)from[6]; L.k_norm = (const float*)from[7];
         L.k_cache = (bf16_t*)from[8]; L.v_cache = (bf16_t*)from[9];
+        uintptr_t wide = 0, pairs = 0;                      // what is read 16 bytes at a time, and what 8
+        for (int j = 0; j < 10; ++j) (j >= 4 && j < 8 ? pairs : wide) |= (uintptr_t)from[j];
+        IA_CHECK(wide % 16 == 0 && pairs % 8 == 0, "layer_run: layer %d: weights and caches must be 16-byte aligned, the norms' weights 8-byte", i);
     }
+    IA_CHECK(((uintptr_t)x & 3) == 0 && (((uintptr_t)cos_t | (uintptr_t)sin_t | (uintptr_t)words) & 7) == 0,
+             "layer_run: rows must be 4-byte aligned, angles and words 8-byte");
     a.x = (bf16_t*)x;
     a.head = (uint64_t*)words;
     a.qkv = a.head + RUN_HEAD_WORDS;

@@ -910,6 +910,15 @@ def layer_run_fits(rows: int, width: int, ff: int, nq: int, nkv: int, page_size:
             and nq // nkv <= 8 and nq % 4 == 0 and rows * (max(width, ff, nq * 128) * 2 + 384) <= RUN_SHARED_BYTES)
 
 
+def layer_run_aligned(layers: Sequence[Sequence[torch.Tensor]]) -> bool:
+    """Whether `layer_run` can read these layers' arrays: weights and caches 16 bytes at a time, the norms' weights 8."""
+    wide = pairs = 0
+    for qkv, o, gate_up, down, norm1, norm2, q_norm, k_norm, k, v in layers:
+        wide |= qkv.data_ptr() | o.data_ptr() | gate_up.data_ptr() | down.data_ptr() | k.data_ptr() | v.data_ptr()
+        pairs |= norm1.data_ptr() | norm2.data_ptr() | q_norm.data_ptr() | k_norm.data_ptr()
+    return wide % 16 == 0 and pairs % 8 == 0
+
+
 def layer_run_pays(rows: int, width: int, ff: int, nq: int, nkv: int, max_kv_len: int) -> bool:
     """Whether a step of these sizes is faster by `layer_run` than by five kernels a layer.  What it gains is a layer's launches, first bytes and
     last sums, which weigh less the larger the weights are, the more rows every block fetches for itself and the more keys there are (which the

@@ -63,15 +63,18 @@ class LayerRun:
         s = b.mixer.spec
         sizes = (x.shape[0], s.hidden, b.ffn.spec.intermediate, s.n_heads, s.n_kv_heads)
         return (all(c is not None and c.writable and c.group == caches[0].group for c in caches)
-                and ops.layer_run_fits(*sizes, ctx.groups[caches[0].group].page_size) and ops.layer_run_pays(*sizes, ctx.max_kv_len))
+                and ops.layer_run_fits(*sizes, ctx.groups[caches[0].group].page_size) and ops.layer_run_pays(*sizes, ctx.max_kv_len)
+                and ops.layer_run_aligned(self._layers(caches)))
+
+    def _layers(self, caches) -> List[Tuple[torch.Tensor, ...]]:
+        return [(m.mixer.qkv.weight, m.mixer.o.weight, m.ffn.gate_up.weight, m.ffn.down.weight, m.norm_mixer.weight, m.norm_ffn.weight,
+                 m.mixer.q_norm_w, m.mixer.k_norm_w, c.k, c.v) for m, c in zip(self.blocks, caches)]
 
     def forward(self, ctx, x: torch.Tensor, storage) -> torch.Tensor:
         """The stream after the run, in place."""
         b, caches = self.blocks[0], [storage.layers[s] for s in self.stops]
         a, s, group = b.mixer, b.mixer.spec, ctx.groups[caches[0].group]
         cos, sin = ctx.position_table(a.position)
-        layers = [(m.mixer.qkv.weight, m.mixer.o.weight, m.ffn.gate_up.weight, m.ffn.down.weight, m.norm_mixer.weight, m.norm_ffn.weight,
-                   m.mixer.q_norm_w, m.mixer.k_norm_w, c.k, c.v) for m, c in zip(self.blocks, caches)]
-        return ops.layer_run(x, layers, ctx.run_words, ctx.positions, group.slots, group.block_table, cos, sin, nq=s.n_heads, nkv=s.n_kv_heads,
+        return ops.layer_run(x, self._layers(caches), ctx.run_words, ctx.positions, group.slots, group.block_table, cos, sin, nq=s.n_heads, nkv=s.n_kv_heads,
                                 ff=b.ffn.spec.intermediate, max_kv_len=ctx.max_kv_len, eps=(b.norm_mixer.eps, b.norm_ffn.eps, a.norm_eps),
                                 add_one=(b.norm_mixer.add_one, b.norm_ffn.add_one, a.norm_add_one), scale=s.softmax_scale)

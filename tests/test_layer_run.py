@@ -30,8 +30,9 @@ def _run_status(**change):
     """`ia_layer_run` over addresses that nobody reads unless the checks on the host let them through: (status, message)."""
     import ctypes
     lib = ops.library()
+    at, by = change.pop("off", (0, 0))
     a = dict(dict(rows=1, width=512, ff=512, nq=4, nkv=4, page_size=16, max_pages=40, max_kv_len=600, splits=2, chunk=512), **change)
-    of = (ctypes.c_void_p * 10)(*[4096] * 10)
+    of = (ctypes.c_void_p * 10)(*[4096 + (by if i == at else 0) for i in range(10)])
     words = lib.ia_layer_run_words(a["rows"], a["width"], a["ff"], a["nq"], a["nkv"], a["splits"])
     status = lib.ia_layer_run(4096, ctypes.addressof(of), 1, 4096, words, *[4096] * 5, *a.values(), 1e-6, 1e-6, 1e-6, 0, 0, 0, 0.1, None)
     return status, lib.ia_last_error().decode()
@@ -61,6 +62,42 @@ def test_positions_beyond_the_bound_count_as_the_last_inside():
             of[9].copy_(v)
         outs.append(ops.layer_run(x.clone(), layers, ops.RunWords(), positions, i32(599, 627), table, cos, sin, **kw))
     assert torch.equal(*outs) and torch.isfinite(outs[0].float()).all()
+
+
+def _cpu_run(layers=3, **kw):
+    """A run of layers over tensors on the host, and what `takes` is asked with, for the choices that read no values."""
+    from types import SimpleNamespace as NS
+    from inferrs_amd.cache.storage import LayerCache
+    from inferrs_amd.parts.assemble import generated_tensors
+    from inferrs_amd.parts.base import block_class
+    from inferrs_amd.parts.layer_run import LayerRun
+    spec = _config(num_hidden_layers=layers, **kw).to_spec()
+    tensors = {name: torch.zeros(tuple(t.shape), dtype=torch.bfloat16) for name, t in generated_tensors(spec).items()}
+    blocks = [block_class(layer)(layer, {k: v for k, v in tensors.items() if k in block_class(layer).tensors(layer)}, torch.bfloat16, "cpu") for layer in spec.layers]
+    run = LayerRun.of_model(spec, blocks)
+    nkv = spec.layers[0].mixer.n_kv_heads
+    cache = {i: LayerCache(i, 0, torch.zeros((2, nkv, PAGE, HD), dtype=torch.bfloat16), torch.zeros((2, nkv, HD, PAGE), dtype=torch.bfloat16)) for i in range(layers)}
+    ctx = NS(max_q_len=1, max_kv_len=32, run_words=ops.RunWords(), groups=[NS(page_size=PAGE)])
+    return run, ctx, torch.zeros((1, spec.layers[0].mixer.hidden), dtype=torch.bfloat16), NS(layers=cache)
+
+
+def test_arrays_off_their_alignment_go_through_the_blocks():
+    """A weight or a cache that is a view at an odd offset, which the kernels of the blocks check for, is none of the run's."""
+    run, *step = _cpu_run()
+    m, c = run.blocks[-1], step[2].layers[2]
+    for holder, name in ((m.mixer.qkv, "weight"), (m.mixer.o, "weight"), (m.ffn.gate_up, "weight"), (m.ffn.down, "weight"), (m.norm_mixer, "weight"),
+                         (m.norm_ffn, "weight"), (m.mixer, "q_norm_w"), (m.mixer, "k_norm_w"), (c, "k"), (c, "v")):
+        assert run.takes(*step)
+        t = getattr(holder, name)
+        setattr(holder, name, torch.zeros(t.numel() + 1, dtype=t.dtype)[1:].view(t.shape))      # (two bytes past an aligned address, or four)
+        assert not run.takes(*step), name
+        setattr(holder, name, t)
+
+
+@pytest.mark.parametrize("at,by", [(0, 2), (3, 8), (4, 4), (7, 4), (8, 2), (9, 8)])
+def test_arrays_off_their_alignment_are_refused(at, by):
+    status, message = _run_status(off=(at, by))
+    assert status == 1 and "aligned" in message, message
 
 
 def _layers(gen, n, width, ff, nq, nkv, pages):
