@@ -365,10 +365,12 @@ long long ia_fading_scan_workspace(int n_seqs, int chunks, int H, int dim, int v
 // values; 16-byte aligned, the norms' weights 8-byte), ia_layer_run_layers() layers at most.  `words` holds ia_layer_run_words() 64-bit words, zero before their first
 // use and left alone between calls; calls that share them must not overlap.  No row is longer than `max_kv_len` with its new token, which
 // `splits` shares of `chunk` keys hold; a position beyond that is read as the last one inside.
+// A block that has asked `polls` times for a word gives up: what it waited for counts as no number, and `*given_up` (pinned host
+// memory) becomes 1, which no launch puts back.
 int ia_layer_run_layers(void);
 long long ia_layer_run_words(int rows, int width, int ff, int nq, int nkv, int splits);
-int ia_layer_run(void* x, const void* layers, int n_layers, long long* words, long long n_words, const int* positions,
-                    const int* slots, const int* block_table, const float* cos_t, const float* sin_t, int rows, int width,
+int ia_layer_run(void* x, const void* layers, int n_layers, long long* words, long long n_words, int* given_up, int polls,
+                    const int* positions, const int* slots, const int* block_table, const float* cos_t, const float* sin_t, int rows, int width,
                     int ff, int nq, int nkv, int page_size, int max_pages, int max_kv_len, int splits, int chunk, float eps1, float eps2,
                     float eps_qk, int one1, int one2, int one_qk, float scale, hipStream_t stream);
 

@@ -36,7 +36,6 @@
 #define RUN_ROWS 8
 #define RUN_HEAD_WORDS 32     // words ahead of the regions: the counter, and the mark of a wait that was given up
 #define RUN_PAD 16            // words behind a row in shared memory: the four rows that lanes read side by side begin in other banks
-#define RUN_POLLS (1 << 20)   // reads of a word after which a wait is given up (seconds; no wait of a sound launch comes near)
 #define RUN_NAN 0x7fc07fc0u
 
 typedef __bf16 run_bf2 __attribute__((ext_vector_type(2)));
@@ -54,6 +53,8 @@ struct RunArgs {
     RunLayer layer[RUN_LAYERS];
     bf16_t* x;                      // [rows, width]: the stream, read by the first layer and written by the last
     uint64_t* head;
+    int* given_up;                  // host memory: set where a wait is given up
+    int polls;                      // reads of a word after which that is
     uint64_t *qkv, *part, *attn, *mid, *act, *next;     // regions of words, in the order of a layer's phases
     const int *positions, *slots, *block_table;
     const float *cos_t, *sin_t;     // [rows, 64]
@@ -71,16 +72,21 @@ __device__ __forceinline__ void word_store(uint64_t* p, uint32_t tag, uint32_t d
 }
 __device__ __forceinline__ uint32_t word_tag(uint64_t v) { return (uint32_t)(v >> 32); }
 
-// Whether a wait goes on after its n-th read: not beyond RUN_POLLS, and not once another has been given up.
-__device__ __forceinline__ bool wait_on(uint64_t* head, int n) {
-    if (n >= RUN_POLLS) word_store(head + 16, 1, 0);
-    return (n & 1023) != 1023 || word_load(head + 16) == 0;
+// Whether a wait goes on after its n-th read: not beyond the limit, and not once another has been given up.  What is waited for in vain counts
+// as no number, so that the launch ends, and the host is told: it reads its word where it has waited for the device anyway.
+__device__ __forceinline__ bool wait_on(const RunArgs& a, int n) {
+    if (n >= a.polls) {
+        word_store(a.head + 16, 1, 0);
+        __hip_atomic_store(a.given_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        return false;
+    }
+    return (n & 1023) != 1023 || word_load(a.head + 16) == 0;
 }
 
 // The data of the words at(0) .. at(N - 1), waited for: asked for together until all are there.  (A thread with fewer words names one of
 // them again: loads behind a condition would each be waited for in turn.)
 template <int N, typename AT>
-__device__ __forceinline__ void words_wait(uint64_t* head, uint32_t tag, AT at, uint32_t (&data)[N]) {
+__device__ __forceinline__ void words_wait(const RunArgs& a, uint32_t tag, AT at, uint32_t (&data)[N]) {
     for (int tries = 1;; ++tries) {
         uint64_t v[N];
         bool there = true;
@@ -93,19 +99,19 @@ __device__ __forceinline__ void words_wait(uint64_t* head, uint32_t tag, AT at, 
         }
         if (there) return;
         __builtin_amdgcn_s_sleep(1);
-        if (!wait_on(head, tries)) break;
+        if (!wait_on(a, tries)) break;
     }
 #pragma unroll
     for (int i = 0; i < N; ++i) data[i] = RUN_NAN;
 }
 
 // Held until `at`, one of the words that this block needs, shows the tag: one lane watches, and the others ask once.
-__device__ __forceinline__ void watch(uint64_t* head, const uint64_t* at, uint32_t tag) {
+__device__ __forceinline__ void watch(const RunArgs& a, const uint64_t* at, uint32_t tag) {
     if (threadIdx.x == 0) {
         int n = 0;
         while (word_tag(word_load(at)) != tag) {
             __builtin_amdgcn_s_sleep(2);
-            if (!wait_on(head, ++n)) break;
+            if (!wait_on(a, ++n)) break;
         }
     }
     __syncthreads();
@@ -147,7 +153,7 @@ __device__ __forceinline__ uint32_t run_merged(const RunArgs& a, int head, int i
     float top = -INFINITY, total = 0.f, o0 = 0.f, o1 = 0.f;
     for (int s0 = 0; s0 < shares; s0 += AT_ONCE) {
         uint32_t d[AT_ONCE * 4];
-        words_wait<AT_ONCE * 4>(a.head, tag, [&](int n) __attribute__((always_inline)) {
+        words_wait<AT_ONCE * 4>(a, tag, [&](int n) __attribute__((always_inline)) {
             const int q = n & 3;
             return from + (s0 + (n >> 2) < shares ? s0 + (n >> 2) : shares - 1) * (HD + 2) + (q < 2 ? HD + q : 2 * i + q - 2);
         }, d);
@@ -188,8 +194,8 @@ __device__ __forceinline__ void run_normed_rows(const RunArgs& a, int r0, uint32
 #pragma unroll
         for (int i = 0; i < R * Q; ++i) d[i] = ((const uint32_t*)a.x)[place(i)];
     } else {
-        if (first != nullptr) watch(a.head, first, tag);    // (behind the loads of the weights)
-        words_wait<R * Q>(a.head, tag, [&](int i) __attribute__((always_inline)) { return in + place(i); }, d);
+        if (first != nullptr) watch(a, first, tag);    // (behind the loads of the weights)
+        words_wait<R * Q>(a, tag, [&](int i) __attribute__((always_inline)) { return in + place(i); }, d);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -283,7 +289,7 @@ __device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L,
         int shares[R];                                      // of the rows' keys
 #pragma unroll
         for (int r = 0; r < R; ++r) shares[r] = merges ? run_last(a, r) / a.chunk + 1 : 0;
-        watch(a.head, merges ? a.part + (size_t)(item % (R * a.nq)) * a.splits * (RUN_HD + 2) : in + (item * 37) % n, tag);
+        watch(a, merges ? a.part + (size_t)(item % (R * a.nq)) * a.splits * (RUN_HD + 2) : in + (item * 37) % n, tag);
         if (merges) {
             // the shares of every head's keys come together here: few of them, and few blocks that would read them all
             for (int j = tid; j < n; j += RUN_THREADS) {
@@ -296,7 +302,7 @@ __device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L,
         constexpr int Q = 4;
         for (int j0 = tid; j0 < n; j0 += Q * RUN_THREADS) {
             uint32_t d[Q];
-            words_wait<Q>(a.head, tag, [&](int q) __attribute__((always_inline)) { return in + (j0 + q * RUN_THREADS < n ? j0 + q * RUN_THREADS : j0); }, d);
+            words_wait<Q>(a, tag, [&](int q) __attribute__((always_inline)) { return in + (j0 + q * RUN_THREADS < n ? j0 + q * RUN_THREADS : j0); }, d);
 #pragma unroll
             for (int q = 0; q < Q; ++q)
                 if (j0 + q * RUN_THREADS < n) put(j0 + q * RUN_THREADS, d[q]);
@@ -313,7 +319,7 @@ __device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L,
     uint32_t was[1] = {0};
     if (!normed && r < R) {
         if (kind == RUN_O && layer == 0) was[0] = ((const uint32_t*)a.x)[at];
-        else words_wait<1>(a.head, tag, [&](int) { return old_at; }, was);
+        else words_wait<1>(a, tag, [&](int) { return old_at; }, was);
     }
     __syncthreads();
     float scale = 1.f;
@@ -478,12 +484,12 @@ __device__ __forceinline__ void run_attention(const RunArgs& a, const RunLayer& 
             nw = *(const float2*)((wave < g ? L.q_norm : L.k_norm) + 2 * lane);
             if (a.one_qk) { nw.x += 1.0f; nw.y += 1.0f; }
         }
-        watch(a.head, a.qkv + ((size_t)row * (a.nq + 2 * a.nkv) + kvh * g) * (HD / 2), tag);
+        watch(a, a.qkv + ((size_t)row * (a.nq + 2 * a.nkv) + kvh * g) * (HD / 2), tag);
         if (wave < used) {
             const int head = wave < g ? kvh * g + wave : wave == g ? a.nq + kvh : a.nq + a.nkv + kvh;
             const uint64_t* at = a.qkv + ((size_t)row * (a.nq + 2 * a.nkv) + head) * (HD / 2) + lane;
             uint32_t one[1];
-            words_wait<1>(a.head, tag, [&](int) { return at; }, one);
+            words_wait<1>(a, tag, [&](int) { return at; }, one);
             uint32_t d = one[0];
             if (wave <= g) {                                // (features 2 lane and 2 lane + 1; what they are turned with is 32 lanes away)
                 float x = lo_f32(d), y = hi_f32(d);
@@ -665,7 +671,7 @@ __device__ __forceinline__ void run_attention(const RunArgs& a, const RunLayer& 
 __device__ __forceinline__ void run_merge(const RunArgs& a, int item, uint32_t tag) {
     const int tid = threadIdx.x, g = a.nq / a.nkv;
     const int shares = run_last(a, item / a.nkv) / a.chunk + 1;
-    watch(a.head, a.part + ((size_t)(item / a.nkv) * a.nq + (item % a.nkv) * g) * a.splits * (RUN_HD + 2), tag);
+    watch(a, a.part + ((size_t)(item / a.nkv) * a.nq + (item % a.nkv) * g) * a.splits * (RUN_HD + 2), tag);
     if (tid >= g * (RUN_HD / 2)) return;
     const int head = (item / a.nkv) * a.nq + (item % a.nkv) * g + tid / (RUN_HD / 2), i = tid & (RUN_HD / 2 - 1);
     word_store(a.attn + (size_t)head * (RUN_HD / 2) + i, tag, run_merged(a, head, i, shares, tag));
@@ -712,7 +718,7 @@ extern "C" long long ia_layer_run_words(int rows, int width, int ff, int nq, int
 
 extern "C" int ia_layer_run_layers(void) { return RUN_LAYERS; }
 
-extern "C" int ia_layer_run(void* x, const void* layers, int n_layers, long long* words, long long n_words, const int* positions, const int* slots,
+extern "C" int ia_layer_run(void* x, const void* layers, int n_layers, long long* words, long long n_words, int* given_up, int polls, const int* positions, const int* slots,
                                const int* block_table, const float* cos_t, const float* sin_t, int rows, int width, int ff, int nq, int nkv,
                                int page_size, int max_pages, int max_kv_len, int splits, int chunk, float eps1, float eps2, float eps_qk, int one1, int one2, int one_qk,
                                float scale, hipStream_t stream) {
@@ -725,6 +731,7 @@ extern "C" int ia_layer_run(void* x, const void* layers, int n_layers, long long
     IA_CHECK(splits >= 1 && chunk >= 32 && chunk % 32 == 0 && (long long)splits * chunk >= max_kv_len
                  && n_words >= ia_layer_run_words(rows, width, ff, nq, nkv, splits),
              "layer_run: %d shares of %d keys for %d keys, %lld words", splits, chunk, max_kv_len, n_words);
+    IA_CHECK(given_up != nullptr && polls >= 1, "layer_run: a wait ends after %d reads, and says so in host memory", polls);
     RunArgs a = {};
     const void* const* from = (const void* const*)layers;
     for (int i = 0; i < n_layers; ++i, from += 10) {
@@ -740,6 +747,7 @@ extern "C" int ia_layer_run(void* x, const void* layers, int n_layers, long long
              "layer_run: rows must be 4-byte aligned, angles and words 8-byte");
     a.x = (bf16_t*)x;
     a.head = (uint64_t*)words;
+    a.given_up = given_up; a.polls = polls;
     a.qkv = a.head + RUN_HEAD_WORDS;
     a.part = a.qkv + (size_t)rows * (nq + 2 * nkv) * (RUN_HD / 2);
     a.attn = a.part + (splits > 1 ? (size_t)rows * nq * splits * (RUN_HD + 2) : 0);

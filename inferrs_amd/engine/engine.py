@@ -154,6 +154,11 @@ class Engine:
         return self.cache.length(seq_id)
 
     # ---- the step ---------------------------------------------------------------------------
+    def check(self) -> None:
+        """Raises `ops.KernelError` where a step that the device has ended says that its results are void (`ops.RunWords`).  `step` begins with it
+        and `decode_chain` ends with it; whoever waits for a step's logits by other means can ask before using them."""
+        self.builder.run_words.check()
+
     def step(self, entries: Sequence[Entry], commit: bool = True) -> torch.Tensor:
         """Run one batch; returns float32 logits `[wanted, vocab]` on the device, in the order
         of the entries and of each entry's `want`.  Pages that the entries need beyond what is
@@ -166,6 +171,7 @@ class Engine:
         stepping again."""
         if not entries:
             raise StepError("a step needs at least one entry")
+        self.check()
         vocab = self.spec.vocab_size
         seen = set()
         for e in entries:
@@ -310,7 +316,9 @@ class Engine:
                 self.graph_replays += 1
         finally:
             self._drop_pad_rows()
-        return chosen[:, :n_real].cpu().tolist()
+        tokens = chosen[:, :n_real].cpu().tolist()
+        self.check()
+        return tokens
 
     @staticmethod
     def _decode_key(n_seqs: int, pad_pages: int) -> Tuple[int, ...]:

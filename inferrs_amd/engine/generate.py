@@ -109,6 +109,7 @@ class GenerationLoop:
         drawing = [e.request for e in plan.entries if e.samples]
         tokens, infos = self.sampler.sample_with_logprobs(logits, [r.params for r in drawing],
                                                           [r.tokens for r in drawing], [r.seed for r in drawing])
+        self.engine.check()
         for r, info in zip(drawing, infos):
             if info is not None:
                 # a request that was preempted draws its tokens again while it is recomputed: the same ones

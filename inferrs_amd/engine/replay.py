@@ -55,7 +55,9 @@ def run_trace(engine: Engine, lines: Iterable[str], out_dir: str, reply: IO[str]
         if entries:
             logits = engine.step(entries)
             if logits.shape[0]:
-                logits.cpu().numpy().astype("<f4", copy=False).tofile(os.path.join(out_dir, f"{step}.f32"))
+                rows = logits.cpu()
+                engine.check()
+                rows.numpy().astype("<f4", copy=False).tofile(os.path.join(out_dir, f"{step}.f32"))
         for seq_id in end:
             if engine.has_request(seq_id):
                 engine.end_request(seq_id)

@@ -889,8 +889,30 @@ def attention_decode_fused(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: to
 # ---- whole layers of decode steps of few rows ----------------------------------------------------
 
 class RunWords(DecodeCounters):
-    """The words through which the blocks of `layer_run` hand rows on, with its counter; as the decode kernel's counters, an engine's own."""
+    """The words through which the blocks of `layer_run` hand rows on, with its counter; as the decode kernel's counters, an engine's own.
+    A block that waits for another's words gives up after `polls` reads, so that no launch hangs; the launch's rows, and the keys and values that it
+    caches, are then no numbers.  No wait of a sound launch comes near the limit: `check`, which an engine calls wherever it has waited for the
+    device, makes an error of one that did."""
     dtype, what = torch.int64, "layer_run: the words of runs of layers"
+    POLLS = 1 << 20                                 # (seconds)
+
+    def __init__(self):
+        super().__init__()
+        self.polls = self.POLLS
+        self.given_up: Optional[torch.Tensor] = None        # pinned: the kernel writes it from the device
+
+    def take(self, device: torch.device, needed: int) -> Optional[torch.Tensor]:
+        space = super().take(device, needed)
+        if self.given_up is None:
+            self.given_up = torch.zeros((1,), dtype=torch.int32, pin_memory=True)
+        return space
+
+    def check(self) -> None:
+        """Raises where a launch that has ended gave a wait up, once for all launches since the last check."""
+        if self.given_up is not None and self.given_up.item():
+            self.given_up.zero_()
+            raise KernelError("layer_run: a decode step's blocks waited in vain for each other's rows; the logits of the steps since the last "
+                              "check, and the keys and values that these cached, are void")
 
 
 RUN_MAX_ROWS = 8
@@ -972,7 +994,8 @@ def layer_run(x: torch.Tensor, layers: Sequence[Sequence[torch.Tensor]], words: 
         of = layers[lo:lo + most]
         table = (ctypes.c_void_p * (10 * len(of)))(*[t.data_ptr() for layer in of for t in layer])
         _check(lib.ia_layer_run(
-            _p(x), ctypes.addressof(table), len(of), _p(space), space.numel(), _p(positions), _p(slots), _p(block_table), _p(cos), _p(sin), rows,
+            _p(x), ctypes.addressof(table), len(of), _p(space), space.numel(), _p(words.given_up),
+            words.polls, _p(positions), _p(slots), _p(block_table), _p(cos), _p(sin), rows,
             width, ff, nq, nkv, page_size, block_table.shape[1], max_kv_len, splits, chunk, *eps, *(int(o) for o in add_one), scale, _stream()))
     return x
 

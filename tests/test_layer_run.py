@@ -34,7 +34,7 @@ def _run_status(**change):
     a = dict(dict(rows=1, width=512, ff=512, nq=4, nkv=4, page_size=16, max_pages=40, max_kv_len=600, splits=2, chunk=512), **change)
     of = (ctypes.c_void_p * 10)(*[4096 + (by if i == at else 0) for i in range(10)])
     words = lib.ia_layer_run_words(a["rows"], a["width"], a["ff"], a["nq"], a["nkv"], a["splits"])
-    status = lib.ia_layer_run(4096, ctypes.addressof(of), 1, 4096, words, *[4096] * 5, *a.values(), 1e-6, 1e-6, 1e-6, 0, 0, 0, 0.1, None)
+    status = lib.ia_layer_run(4096, ctypes.addressof(of), 1, 4096, words, 4096, 1, *[4096] * 5, *a.values(), 1e-6, 1e-6, 1e-6, 0, 0, 0, 0.1, None)
     return status, lib.ia_last_error().decode()
 
 
@@ -247,6 +247,86 @@ def test_operands_that_do_not_fit_are_refused():
         ops.layer_run(x.float(), [layer], words, **good)
     with pytest.raises(ops.KernelError):
         ops.layer_run(x, [layer[:3] + (layer[3][:, :256].contiguous(),) + layer[4:]], words, **good)
+
+
+def test_a_wait_given_up_is_an_error_once():
+    words = ops.RunWords()
+    words.check()
+    words.given_up = torch.ones((1,), dtype=torch.int32)
+    with pytest.raises(ops.KernelError, match="waited in vain"):
+        words.check()
+    words.check()
+
+
+@pytest.mark.gpu
+def test_a_wait_given_up_ends_the_launch_and_tells_the_host():
+    """Waits that end after one read: every block ends, the rows are no numbers, the host's word says so, and the next launch is sound."""
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    layers = _layers(gen, 3, 512, 512, 4, 4, 4)
+    x = torch.empty((2, 512), dtype=torch.bfloat16, device="cuda").normal_(0.0, 1.0, generator=gen)
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    args = (i32(5, 20), i32(5, 52), i32(0, 1, 2, 3).view(2, 2), torch.ones((2, 64), device="cuda"), torch.zeros((2, 64), device="cuda"))
+    kw = dict(nq=4, nkv=4, ff=512, max_kv_len=32, eps=(1e-6,) * 3, add_one=(False,) * 3, scale=HD ** -0.5)
+    kept = [(of[8].clone(), of[9].clone()) for of in layers]
+
+    def run(words, polls):
+        for of, (k, v) in zip(layers, kept):
+            of[8].copy_(k)
+            of[9].copy_(v)
+        words.polls = polls
+        out = ops.layer_run(x.clone(), layers, words, *args, **kw)
+        torch.cuda.synchronize()
+        return out
+
+    want, words = run(ops.RunWords(), ops.RunWords.POLLS), ops.RunWords()
+    assert torch.isfinite(want.float()).all()
+    assert torch.isnan(run(words, 1).float()).any()
+    with pytest.raises(ops.KernelError, match="waited in vain"):
+        words.check()
+    for _ in range(2):
+        assert torch.equal(run(words, ops.RunWords.POLLS), want)
+        words.check()
+
+
+@pytest.mark.gpu
+def test_an_engine_raises_where_a_wait_was_given_up():
+    """The step behind the one whose wait was given up raises, and so does the serving loop before it takes a token; both go on from there."""
+    from inferrs_amd.engine import Engine, Entry, GenerationLoop
+    from inferrs_amd.sampling import SamplingParams
+    engines = [Engine.from_random(_config(), seed=3, page_size=16, num_pages=40, max_seqs=2) for _ in range(2)]
+    words = engines[0].builder.run_words
+    prompt = list(range(20))
+    for e in engines:
+        e.step([Entry("a", prompt, [])])
+    words.polls = 1
+    engines[0].step([Entry("a", [7], [0])], commit=False)
+    torch.cuda.synchronize()
+    words.polls = ops.RunWords.POLLS
+    with pytest.raises(ops.KernelError, match="waited in vain"):
+        engines[0].step([Entry("a", [7], [0])], commit=False)
+    got, want = (e.step([Entry("a", [7], [0])]).clone() for e in engines)
+    assert torch.equal(got, want)
+    outputs = []
+    for e, disturbed in zip(engines, (True, False)):
+        e.end_request("a")
+        loop = GenerationLoop(e, max_batch_size=2, decode_run=1)
+        r = loop.add(prompt, SamplingParams.greedy(max_tokens=5, bypass_stop_tokens=True))
+        loop.step()
+        if disturbed:
+            before, sample = list(r.output), loop.sampler.sample_with_logprobs
+
+            def sample_behind_such_a_step(*a):
+                words.given_up.fill_(1)
+                return sample(*a)
+
+            loop.sampler.sample_with_logprobs = sample_behind_such_a_step
+            with pytest.raises(ops.KernelError, match="waited in vain"):
+                loop.step()
+            loop.sampler.sample_with_logprobs = sample
+            assert r.output == before
+        loop.run()
+        outputs.append(list(r.output))
+    assert outputs[0] == outputs[1] and len(outputs[0]) == 5
 
 
 def _config(**kw):
