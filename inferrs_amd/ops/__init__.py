@@ -66,7 +66,7 @@ class KernelTimer:
 
 
 class _Timed:
-    """A kernel library whose entry points report to the active `KernelTimer`, if there is one."""
+    """A kernel library whose entry points that launch something report to the active `KernelTimer`, if there is one."""
     __slots__ = ("_lib", "_short")
 
     def __init__(self, lib: ctypes.CDLL):
@@ -75,9 +75,7 @@ class _Timed:
 
     def __getattr__(self, name):
         fn = getattr(self._lib, name)
-        if KernelTimer.active is None or not name.startswith("ia_") or name.endswith(("_workspace", "_blocks", "_block_rows",
-                                                                                      "_error", "_version", "_capacity", "_top",
-                                                                                      "_splits", "_tune", "_target", "_counters", "_fills", "_fits", "_plan", "_plans")):
+        if KernelTimer.active is None or name not in _LAUNCHING:
             return fn
         timer = KernelTimer.active
         return lambda *args: timer.call(name[3:], fn, *args)
@@ -86,6 +84,7 @@ class _Timed:
 _C_TYPES = {"int": ctypes.c_int, "long long": ctypes.c_longlong, "unsigned long long": ctypes.c_ulonglong,
             "float": ctypes.c_float, "double": ctypes.c_double, "hipStream_t": ctypes.c_void_p, "size_t": ctypes.c_size_t}
 _DECLARATIONS: Dict[str, Tuple[object, list]] = {}
+_LAUNCHING: set = set()                                     # the entry points that take a stream: the others are questions to the host
 
 
 def _declarations() -> Dict[str, Tuple[object, list]]:
@@ -114,6 +113,8 @@ def _declarations() -> Dict[str, Tuple[object, list]]:
         args = [] if params in ("", "void") else [ctype(a) for a in params.split(",")]
         restype = None if result == "void" else (ctypes.c_char_p if "char" in result else _C_TYPES[result])
         _DECLARATIONS[name] = (restype, args)
+        if "hipStream_t" in params:
+            _LAUNCHING.add(name)
     for must in ("ia_last_error", "ia_add_rmsnorm", "ia_gemm_skinny_bf16", "ia_attention_mfma", "ia_sample"):
         if must not in _DECLARATIONS:
             _DECLARATIONS.clear()

@@ -249,6 +249,18 @@ def test_operands_that_do_not_fit_are_refused():
         ops.layer_run(x, [layer[:3] + (layer[3][:, :256].contiguous(),) + layer[4:]], words, **good)
 
 
+def test_questions_to_the_host_are_no_kernel_calls():
+    """The tables of a step's kernels list what launches something: not the run's words and layers, which are asked for at every call."""
+    lib = ops.library()
+    with ops.KernelTimer() as timer:
+        timed = ops.library()
+        for name in ("ia_layer_run_words", "ia_layer_run_layers", "ia_gemm_wide_rows_fits", "ia_attention_mfma_has_fused", "ia_last_error"):
+            if hasattr(lib, name):
+                assert getattr(timed, name) is getattr(lib, name), name
+        assert timed.ia_layer_run is not lib.ia_layer_run and timed.ia_rmsnorm is not lib.ia_rmsnorm
+    assert not timer.records
+
+
 def test_a_wait_given_up_is_an_error_once():
     words = ops.RunWords()
     words.check()
