@@ -942,21 +942,31 @@ def layer_run_aligned(layers: Sequence[Sequence[torch.Tensor]]) -> bool:
     return wide % 16 == 0 and pairs % 8 == 0
 
 
-def layer_run_pays(rows: int, width: int, ff: int, nq: int, nkv: int, max_kv_len: int) -> bool:
-    """Whether a step of these sizes is faster by `layer_run` than by five kernels a layer.  What it gains is a layer's launches, first bytes and
-    last sums, which weigh less the larger the weights are, the more rows every block fetches for itself and the more keys there are (which the
-    decode attention walks with twice the waves a compute unit).  us a step, five kernels / `layer_run`: 28 layers of the 0.6B shape 8 rows at
-    3,000 keys 1,303 / 1,068, at 8,000 2,035 / 2,086, 3 rows at 14,000 1,634 / 1,492; 16 of the 4B shape 8 rows at 3,000 1,446 / 1,349, at 8,000
-    1,867 / 1,936; 10 of the 8B shape 4 rows at 3,000 1,187 / 1,157, at 8,000 1,306 / 1,366, 6 rows at 700 1,152 / 1,217; 6 of the 14B shape
-    2 rows at 3,000 1,147 / 1,099, 3 rows at 3,000 1,176 / 1,174; 5 of the 32B shape 2 rows at 14,000 1,369 / 1,348."""
+def layer_run_pays(rows: int, width: int, ff: int, nq: int, nkv: int, max_kv_len: int, layers: int = 6) -> bool:
+    """Whether a step of these sizes is faster by `layer_run` over a run of `layers` than by five kernels a layer.  What it gains is a layer's launches,
+    first bytes and last sums.  They weigh less the larger the weights are, the more rows every block fetches for itself, and the more bytes of
+    keys and values there are, which the decode attention walks with twice the waves a compute unit.  Of 1,150 sizes of 29 shapes it takes 900,
+    1.3 times as fast in the mean, the worst 0.98 (both ways replayed from graphs in turn; us a layer, five kernels / a run).
+    Rows.  Weights up to 128 MiB: 0.6B shape, 700 keys, 1 row 31 / 15, 8 rows 36 / 23; 1.7B shape, 8 rows 51 / 39.  Up to 256 MiB: 4B shape, 4 rows
+    68 / 57, 6 rows 70 / 64 (one layer 0.87 to 1.03), 8 rows 72 / 69 (1.00 to 1.08 from six layers on, of one to four layers 0.84 to 0.99: a run's
+    first layers gain less than those behind them); with more than 8 key heads attention alone is more blocks than units from 6 rows on (width 2,048, 32 key heads, 5 rows 66 / 62,
+    6 rows 68 / 68, 8 rows 74 / 76); widths of 3,072 and 3,584, of which a wave takes six or seven loads and only four ahead of its wait: 3 rows 60 /
+    58, 4 rows 61 / 67.  Up to 512 MiB: 8B shape 3 rows 91 / 78, 4 rows 92 / 94, 6 rows 95 / 105.  Beyond: 14B shape 2 rows 142 / 126, 32B shape 199 / 184.
+    Keys.  One row: 0.6B shape at 45,000 keys 59 / 50; 32 key heads of width 2,048 at 16,384 0.995 of the speed, at 33,000 1.065, at 45,000 1.05; 40 of
+    width 5,120 at 24,000 1.08.  More: 16 key heads, 4 rows at 8,192 1.08 to 1.11, 5 rows 0.99 to 1.00, 2 rows at 16,384 0.96 to 1.00; 32 key heads,
+    2 rows at 8,192 1.03 to 1.07, 3 rows at 11,000 0.92; 40 of width 5,120, 2 rows at 8,192 1.02, at 12,000 0.97."""
     weights = 2 * (2 * (nq + nkv) * 128 * width + 3 * width * ff)
-    if weights <= 256 << 20:
+    bytes_of_keys = 512 << 10                       # (rows x keys x key heads)
+    if weights <= 128 << 20:
         most, keys = 8, 44 << 10
+    elif weights <= 256 << 20:
+        most, keys = (3 if 6 <= width // 512 < 8 else 4 if layers < 2 else 5 if nkv > 8 else 6 if layers < 6 else 8), 44 << 10
     elif weights <= 512 << 20:
-        most, keys = 4, 20 << 10
+        most, keys = 3, 20 << 10
     else:
-        most, keys = 2, 24 << 10
-    return rows <= most and rows * max_kv_len <= keys
+        most, keys, bytes_of_keys = 2, 24 << 10, 640 << 10
+    return (rows <= most and rows * max_kv_len <= keys
+            and (rows == 1 or (rows * max_kv_len * nkv <= bytes_of_keys and (nkv <= 8 or max_kv_len <= 12 << 10))))
 
 
 def layer_run(x: torch.Tensor, layers: Sequence[Sequence[torch.Tensor]], words: RunWords, positions: torch.Tensor, slots: torch.Tensor,

@@ -63,7 +63,7 @@ class LayerRun:
         s = b.mixer.spec
         sizes = (x.shape[0], s.hidden, b.ffn.spec.intermediate, s.n_heads, s.n_kv_heads)
         return (all(c is not None and c.writable and c.group == caches[0].group for c in caches)
-                and ops.layer_run_fits(*sizes, ctx.groups[caches[0].group].page_size) and ops.layer_run_pays(*sizes, ctx.max_kv_len)
+                and ops.layer_run_fits(*sizes, ctx.groups[caches[0].group].page_size) and ops.layer_run_pays(*sizes, ctx.max_kv_len, self.length)
                 and ops.layer_run_aligned(self._layers(caches)))
 
     def _layers(self, caches) -> List[Tuple[torch.Tensor, ...]]:

@@ -19,8 +19,19 @@ def test_rule_of_the_sizes():
     assert not ops.layer_run_fits(4, 5120, 25600, 64, 8, 16)                 # (four rows of 25,600 are more than a compute unit's shared memory)
     small, mid, large = (1024, 3072, 16, 8), (4096, 12288, 32, 8), (5120, 25600, 64, 8)
     assert ops.layer_run_pays(8, *small, 4096) and not ops.layer_run_pays(8, *small, 8192) and ops.layer_run_pays(1, *small, 40960)
-    assert ops.layer_run_pays(4, *mid, 4096) and not ops.layer_run_pays(4, *mid, 8192) and not ops.layer_run_pays(6, *mid, 1024)
+    # (four rows of the second shape were measured at 0.97 to 0.99 of the speed of five kernels a layer in runs of 10 to 16 layers, three at 1.06 to 1.16)
+    assert ops.layer_run_pays(3, *mid, 4096) and not any(ops.layer_run_pays(4, *mid, keys) for keys in (1024, 4096, 8192)) and not ops.layer_run_pays(6, *mid, 1024)
     assert ops.layer_run_pays(2, *large, 8192) and not ops.layer_run_pays(3, *large, 1024)
+    # weights of up to 256 MiB: by the key heads, the layers of the run, and what a wave takes of the width
+    heads32, width3072, width2560 = (2048, 8192, 32, 32), (3072, 8192, 24, 8), (2560, 9728, 32, 8)
+    assert ops.layer_run_pays(5, *heads32, 2048) and not ops.layer_run_pays(6, *heads32, 1024)
+    assert ops.layer_run_pays(3, *width3072, 4096) and not ops.layer_run_pays(4, *width3072, 1024)
+    assert ops.layer_run_pays(8, *width2560, 4096) and not ops.layer_run_pays(8, *width2560, 1024, 4) and ops.layer_run_pays(6, *width2560, 1024, 4)
+    assert ops.layer_run_pays(4, *width2560, 1024, 1) and not ops.layer_run_pays(6, *width2560, 1024, 1)
+    # the bytes of the keys
+    assert ops.layer_run_pays(1, *heads32, 45056) and ops.layer_run_pays(2, *heads32, 8192) and not ops.layer_run_pays(2, *heads32, 11264)
+    heads16 = (1024, 3072, 16, 16)
+    assert ops.layer_run_pays(4, *heads16, 8192) and not ops.layer_run_pays(5, *heads16, 8192) and not ops.layer_run_pays(2, *heads16, 16384)
     for keys in (1, 511, 512, 513, 16384, 16385, 40960, 131072):
         splits, chunk = ops.run_shares(keys)
         assert chunk % 32 == 0 and splits * chunk >= keys and splits <= 32 and (splits - 1) * chunk < keys
