@@ -214,9 +214,10 @@ def measured_roofs(engine):
     return best, tflops
 
 
-def kernel_breakdown(engine, batch: int, context: int, prefill_tokens: int, vocab: int):
+def kernel_breakdown(engine, batch: int, context: int, prefill_tokens: int, vocab: int, layer_kernels: bool = False):
     """Microseconds by kernel entry point for one decode step (batch, context) and one prefill, each kernel call
-    bracketed by events (eager steps, no graph; an event pair adds a few microseconds to a short kernel)."""
+    bracketed by events (eager steps, no graph; an event pair adds a few microseconds to a short kernel).  `layer_kernels`: layers that
+    a decode step would take whole, in one kernel, go through the kernels of a layer, which are then seen one by one."""
     import torch
     from inferrs_amd import ops
     from inferrs_amd.engine import Entry
@@ -224,7 +225,10 @@ def kernel_breakdown(engine, batch: int, context: int, prefill_tokens: int, voca
     ids = [f"k{i}" for i in range(batch)]
     fill_context(engine, ids, context - 4)
     graphs, engine.use_graphs = engine.use_graphs, False
+    run = engine.model.layer_run
     try:
+        if layer_kernels:
+            engine.model.layer_run = None
         entries = [Entry(sid, [1 + i], [0]) for i, sid in enumerate(ids)]
         engine.step(entries)                                   # once without the timer
         with ops.KernelTimer() as timer:
@@ -241,7 +245,7 @@ def kernel_breakdown(engine, batch: int, context: int, prefill_tokens: int, voca
         out["prefill"] = timer.summary()
         engine.end_request("kp")
     finally:
-        engine.use_graphs = graphs
+        engine.use_graphs, engine.model.layer_run = graphs, run
     return {phase: {name: {"calls": calls, "us": round(us, 1)} for name, (calls, us) in sorted(table.items(), key=lambda kv: -kv[1][1])}
             for phase, table in out.items()}
 
@@ -854,7 +858,8 @@ def main() -> int:
             points[f"prefill_{long_prompt}"] = rec["value"]
             fractions[f"prefill_{long_prompt}_mfma"] = rec["frac"]
             note("per-kernel times of one decode step and one prefill")
-            record["kernels"] = kernel_breakdown(engine, args.batch, args.context, args.prefill_tokens, vocab)
+            # (a model cut to a few layers is how a layer's kernels are looked at one by one; a whole model's table is of its steps as they run)
+            record["kernels"] = kernel_breakdown(engine, args.batch, args.context, args.prefill_tokens, vocab, layer_kernels=args.layers < full_layers)
             # the true 32-bit path at the same layer sizes, four layers of them
             if args.dtype == "bfloat16":
                 f32_layers = min(4, args.layers)

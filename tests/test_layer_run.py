@@ -412,7 +412,7 @@ def test_two_engines_on_two_streams():
 
 
 def test_which_layers_form_a_run():
-    """Layers that differ end a run; a few layers are none, nor are layers of another kind."""
+    """Layers that differ end a run, which one layer makes; layers of another kind are none."""
     from inferrs_amd.parts.assemble import generated_tensors
     from inferrs_amd.parts.layer_run import LayerRun
     from inferrs_amd.parts.base import block_class
@@ -436,5 +436,7 @@ def test_which_layers_form_a_run():
             return dataclasses.replace(spec, layers=type(spec.layers)(layers))
         return change
 
-    assert run_of(_config(), window(3)).length == 3 and run_of(_config(), window(2)) is None and run_of(_config(), window(0)) is None
+    # (runs of one and two layers were none, though measured faster: `LayerRun`)
+    assert [run_of(_config(), window(n)).length for n in (1, 2, 3, 4)] == [1, 2, 3, 4] and run_of(_config(), window(0)) is None
+    assert run_of(_config(num_hidden_layers=1)).length == 1
     assert run_of(_config(head_dim=64)) is None
