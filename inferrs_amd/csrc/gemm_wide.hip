@@ -514,14 +514,19 @@ static double vendor_rows_us(int M, int N, int K) {
 
 // Whether a product whose whole rows are wanted goes here instead of to the vendor's GEMM.  us, the vendor's / this: 8,512 features over 2,048,
 // 600 rows 30.6 / 27.1, 1,500 54.3 / 47.4, 2,048 82 / 66; 4,304 over 1,024, 1,000 rows 18.3 / 13.5; 16,928 over 4,096, 1,300 rows 214 /
-// 152; of even ones 8,192 over 2,048, 1,000 rows 35.1 / 32.6, 10,240 over 2,560, 800 rows 51.4 / 45.8.  Not where the library's blocks fill their
-// rounds (8,192 over 2,048, 2,048 rows 50.9 / 61.3).  Of the 105 sizes of 512 rows and more it takes none that loses more than 2 %.  (Two rounds of
+// 152; of features in whole blocks of 256 10,240 over 2,560, 800 rows 51.4 / 45.8.  Not where the library's blocks fill their
+// rounds (8,192 over 2,048, 2,048 rows 50.9 / 61.3).  Features in whole blocks were measured again inside prompts of the six dense shapes, one product
+// of a layer on either kernel (us a layer): above 1,024 rows 0.6B shape, 1,300 rows, q|k|v 133 / 127, 4B 1,400 rows 384 / 375, 8B 1,536 rows 628 / 617,
+// 14B 1,800 rows 1,219 / 1,203; of 60 points 0.993 to 1.071, 1.010 in the mean.  Up to 1,024 rows a plan has to be ahead clearly, since both sides' times are
+// known to a tenth (4B shape, q|k|v, 800 rows 255.4 / 260.5, 900 rows 289.7 / 293.3), and whole multiples of 1,024 rows, which the library's smaller blocks
+// share out evenly, gain nothing (2,048 rows, o of the 8B shape 0.998 and 1.004, of the 4B shape 0.994 and 0.997).  (Two rounds of
 // this kernel over a long k take 7 % longer than its stages add up to: 34,816 over 5,120 at 521 rows 187 / 205.)
 extern "C" int ia_gemm_wide_rows_fits(int M, int N, int K) {
     if (M < 512 || N <= 0 || K <= 0 || K % GW_STAGE_K || N % 4) return 0;
+    if (N % 256 == 0 && M % 1024 == 0) return 0;
     const WidePlan plan = gw_plan(M, N, K, false, false);
     const bool one_round = (long long)((M + 16 * plan.mt - 1) / (16 * plan.mt)) * ((N + GW_BN - 1) / GW_BN) <= wide_cus();
-    return plan.cost <= (N % 256 ? 1.2 : one_round ? 1.02 : 0.95) * vendor_rows_us(M, N, K);
+    return plan.cost <= (N % 256 ? 1.2 : M <= 1024 ? 0.93 : one_round ? 1.02 : 0.95) * vendor_rows_us(M, N, K);
 }
 
 // The same with an activation, which costs this kernel a few microseconds at its end (four waves a unit form it: 8,192 features, 1,500 rows,

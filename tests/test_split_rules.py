@@ -216,3 +216,11 @@ def test_decode_shares_are_whole_blocks_that_cover_the_context(g):
 def test_decode_attention_takes_the_faster_kernels_at_the_measured_points(n, nkv, g, d, dv, bound, span, kind, apart, fused):
     """The choice between one kernel and several as a layer makes it, against both measured times (us)."""
     assert ops.decode_fused_pays(n, nkv, g, d, dv, bound, span, formed=kind == "formed", gated=kind == "gated") == (fused < apart)
+
+
+@pytest.mark.parametrize("m,n,k,own", [(800, 6144, 2560, 0), (900, 6144, 2560, 0), (800, 10240, 2560, 1), (1400, 6144, 2560, 1), (1300, 4096, 4096, 1),
+                                       (2048, 4096, 4096, 0), (2048, 2560, 4096, 0), (2048, 4096, 1024, 0), (2047, 4096, 4096, 1), (1024, 8512, 2048, 1),
+                                       (2048, 8512, 2048, 1), (511, 8512, 2048, 0)])
+def test_whole_products_stay_with_the_vendor_where_nothing_is_gained(m, n, k, own):
+    """Features in whole blocks of 256: up to 1,024 rows only where the plan is ahead clearly, and no multiples of 1,024 rows; odd ones as before."""
+    assert ops.library().ia_gemm_wide_rows_fits(m, n, k) == own
