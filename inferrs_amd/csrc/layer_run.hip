@@ -53,8 +53,6 @@ struct RunArgs {
     RunLayer layer[RUN_LAYERS];
     bf16_t* x;                      // [rows, width]: the stream, read by the first layer and written by the last
     uint64_t* head;
-    int* given_up;                  // host memory: set where a wait is given up
-    int polls;                      // reads of a word after which that is
     uint64_t *qkv, *part, *attn, *mid, *act, *next;     // regions of words, in the order of a layer's phases
     const int *positions, *slots, *block_table;
     const float *cos_t, *sin_t;     // [rows, 64]
@@ -64,6 +62,8 @@ struct RunArgs {
     int width, ff, nq, nkv, max_pages, splits, chunk, max_kv;
     float eps1, eps2, eps_qk, scale_log2;
     int one1, one2, one_qk;         // norms weigh with 1 + w
+    int polls;                      // reads of a word after which a wait is given up
+    int* given_up;                  // host memory: set where one is
 };
 
 __device__ __forceinline__ uint64_t word_load(const uint64_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -72,46 +72,50 @@ __device__ __forceinline__ void word_store(uint64_t* p, uint32_t tag, uint32_t d
 }
 __device__ __forceinline__ uint32_t word_tag(uint64_t v) { return (uint32_t)(v >> 32); }
 
-// Whether a wait goes on after its n-th read: not beyond the limit, and not once another has been given up.  What is waited for in vain counts
-// as no number, so that the launch ends, and the host is told: it reads its word where it has waited for the device anyway.
-__device__ __forceinline__ bool wait_on(const RunArgs& a, int n) {
-    if (n >= a.polls) {
+// What a block waits for its layer's words with: their tag, and the limit of a wait, which the block reads once, beside its draw (read from the
+// arguments at every wait it cost a step of 28 layers 2 us).
+struct RunWait { uint32_t tag; int polls; };
+
+// Whether a wait goes on that has `left` reads, the one just made among them: not beyond these, and not once another has been given up.  What is
+// waited for in vain counts as no number, so that the launch ends, and the host is told: it reads its word where it has waited for the device
+// anyway.
+__device__ __forceinline__ bool wait_on(const RunArgs& a, int& left) {
+    if (--left <= 0) {
         word_store(a.head + 16, 1, 0);
         __hip_atomic_store(a.given_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        return false;
     }
-    return (n & 1023) != 1023 || word_load(a.head + 16) == 0;
+    return (left & 1023) != 0 || word_load(a.head + 16) == 0;     // (at 0 the mark just set; no way out of its own: the waits' ends stay short)
 }
 
 // The data of the words at(0) .. at(N - 1), waited for: asked for together until all are there.  (A thread with fewer words names one of
 // them again: loads behind a condition would each be waited for in turn.)
 template <int N, typename AT>
-__device__ __forceinline__ void words_wait(const RunArgs& a, uint32_t tag, AT at, uint32_t (&data)[N]) {
-    for (int tries = 1;; ++tries) {
+__device__ __forceinline__ void words_wait(const RunArgs& a, RunWait wait, AT at, uint32_t (&data)[N]) {
+    for (int left = wait.polls;;) {
         uint64_t v[N];
         bool there = true;
 #pragma unroll
         for (int i = 0; i < N; ++i) v[i] = word_load(at(i));
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            there = there && word_tag(v[i]) == tag;
+            there = there && word_tag(v[i]) == wait.tag;
             data[i] = (uint32_t)v[i];
         }
         if (there) return;
         __builtin_amdgcn_s_sleep(1);
-        if (!wait_on(a, tries)) break;
+        if (!wait_on(a, left)) break;
     }
 #pragma unroll
     for (int i = 0; i < N; ++i) data[i] = RUN_NAN;
 }
 
 // Held until `at`, one of the words that this block needs, shows the tag: one lane watches, and the others ask once.
-__device__ __forceinline__ void watch(const RunArgs& a, const uint64_t* at, uint32_t tag) {
+__device__ __forceinline__ void watch(const RunArgs& a, const uint64_t* at, RunWait wait) {
     if (threadIdx.x == 0) {
-        int n = 0;
-        while (word_tag(word_load(at)) != tag) {
+        int left = wait.polls;
+        while (word_tag(word_load(at)) != wait.tag) {
             __builtin_amdgcn_s_sleep(2);
-            if (!wait_on(a, ++n)) break;
+            if (!wait_on(a, left)) break;
         }
     }
     __syncthreads();
@@ -147,13 +151,13 @@ __device__ __forceinline__ void sum_lanes(float* v) {
 __device__ __forceinline__ int run_last(const RunArgs& a, int row) { return min(max(a.positions[row], 0), a.max_kv - 1); }
 
 // Features 2 i and 2 i + 1 of the attention of `head` (counted over all rows), from the shares of its row's keys.
-__device__ __forceinline__ uint32_t run_merged(const RunArgs& a, int head, int i, int shares, uint32_t tag) {
+__device__ __forceinline__ uint32_t run_merged(const RunArgs& a, int head, int i, int shares, RunWait wait) {
     constexpr int HD = RUN_HD, AT_ONCE = 2;
     const uint64_t* from = a.part + (size_t)head * a.splits * (HD + 2);
     float top = -INFINITY, total = 0.f, o0 = 0.f, o1 = 0.f;
     for (int s0 = 0; s0 < shares; s0 += AT_ONCE) {
         uint32_t d[AT_ONCE * 4];
-        words_wait<AT_ONCE * 4>(a, tag, [&](int n) __attribute__((always_inline)) {
+        words_wait<AT_ONCE * 4>(a, wait, [&](int n) __attribute__((always_inline)) {
             const int q = n & 3;
             return from + (s0 + (n >> 2) < shares ? s0 + (n >> 2) : shares - 1) * (HD + 2) + (q < 2 ? HD + q : 2 * i + q - 2);
         }, d);
@@ -177,7 +181,7 @@ __device__ __forceinline__ uint32_t run_merged(const RunArgs& a, int head, int i
 // Rows r0 .. r0 + R - 1 of the stream into shared memory, times the norm's weights and rounded, and every wave's sums of their squares;
 // Q words a thread and row.
 template <int R, int Q>
-__device__ __forceinline__ void run_normed_rows(const RunArgs& a, int r0, uint32_t* xs, float* squares, const float* norm, float one, const uint64_t* in, const uint64_t* first, uint32_t tag, bool plain) {
+__device__ __forceinline__ void run_normed_rows(const RunArgs& a, int r0, uint32_t* xs, float* squares, const float* norm, float one, const uint64_t* in, const uint64_t* first, RunWait wait, bool plain) {
     const int tid = threadIdx.x, pairs = a.width >> 1;
     float2 weight[Q];
 #pragma unroll
@@ -194,8 +198,8 @@ __device__ __forceinline__ void run_normed_rows(const RunArgs& a, int r0, uint32
 #pragma unroll
         for (int i = 0; i < R * Q; ++i) d[i] = ((const uint32_t*)a.x)[place(i)];
     } else {
-        if (first != nullptr) watch(a, first, tag);    // (behind the loads of the weights)
-        words_wait<R * Q>(a, tag, [&](int i) __attribute__((always_inline)) { return in + place(i); }, d);
+        if (first != nullptr) watch(a, first, wait);    // (behind the loads of the weights)
+        words_wait<R * Q>(a, wait, [&](int i) __attribute__((always_inline)) { return in + place(i); }, d);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -215,10 +219,10 @@ __device__ __forceinline__ void run_normed_rows(const RunArgs& a, int r0, uint32
 }
 
 template <int R>
-__device__ __forceinline__ void run_normed_rows(const RunArgs& a, int r0, uint32_t* xs, float* squares, const float* norm, float one, const uint64_t* in, const uint64_t* first, uint32_t tag, bool plain) {
-    if (a.width <= 2 * RUN_THREADS) run_normed_rows<R, 1>(a, r0, xs, squares, norm, one, in, first, tag, plain);
-    else if (a.width <= 4 * RUN_THREADS) run_normed_rows<R, 2>(a, r0, xs, squares, norm, one, in, first, tag, plain);
-    else run_normed_rows<R, 3>(a, r0, xs, squares, norm, one, in, first, tag, plain);
+__device__ __forceinline__ void run_normed_rows(const RunArgs& a, int r0, uint32_t* xs, float* squares, const float* norm, float one, const uint64_t* in, const uint64_t* first, RunWait wait, bool plain) {
+    if (a.width <= 2 * RUN_THREADS) run_normed_rows<R, 1>(a, r0, xs, squares, norm, one, in, first, wait, plain);
+    else if (a.width <= 4 * RUN_THREADS) run_normed_rows<R, 2>(a, r0, xs, squares, norm, one, in, first, wait, plain);
+    else run_normed_rows<R, 3>(a, r0, xs, squares, norm, one, in, first, wait, plain);
 }
 
 enum { RUN_QKV, RUN_O, RUN_GATE_UP, RUN_DOWN };
@@ -231,7 +235,7 @@ enum { RUN_QKV, RUN_O, RUN_GATE_UP, RUN_DOWN };
 // summed at the end; up to four rows cost what one costs, but neighbouring lanes read four rows of memory.  (us a layer, DOT / not, 700
 // keys: 0.6B shape 1 row 14.0 / 14.4, 2 rows 17.2 / 15.8, 4 rows 22.5 / 17.3; 8B shape 1 row 68 / 75, 2 rows 73 / 77.)
 template <int R, bool DOT>
-__device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L, char* mem, int kind, int item, int layer, uint32_t tag) {
+__device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L, char* mem, int kind, int item, int layer, RunWait wait) {
     constexpr int C = (R + 3) / 4;                          // groups of four rows
     const int tid = threadIdx.x, lane = tid & (IA_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / IA_WAVE);
     const int heads_width = a.nq * RUN_HD;
@@ -278,8 +282,8 @@ __device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L,
         const float* norm = kind == RUN_QKV ? L.norm1 : L.norm2;
         const float one = (kind == RUN_QKV ? a.one1 : a.one2) ? 1.0f : 0.0f;
         const uint64_t* in = kind == RUN_QKV ? a.next : a.mid;
-        run_normed_rows<(R < 4 ? R : 4)>(a, 0, xs, squares, norm, one, in, in + (item * 37) % (R * pairs), tag, plain);
-        if constexpr (R > 4) run_normed_rows<R - 4>(a, 4, xs, squares, norm, one, in, nullptr, tag, plain);
+        run_normed_rows<(R < 4 ? R : 4)>(a, 0, xs, squares, norm, one, in, in + (item * 37) % (R * pairs), wait, plain);
+        if constexpr (R > 4) run_normed_rows<R - 4>(a, 4, xs, squares, norm, one, in, nullptr, wait, plain);
     } else {
         const uint64_t* in = kind == RUN_O ? a.attn : a.act;
         const int n = R * pairs;
@@ -289,20 +293,20 @@ __device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L,
         int shares[R];                                      // of the rows' keys
 #pragma unroll
         for (int r = 0; r < R; ++r) shares[r] = merges ? run_last(a, r) / a.chunk + 1 : 0;
-        watch(a, merges ? a.part + (size_t)(item % (R * a.nq)) * a.splits * (RUN_HD + 2) : in + (item * 37) % n, tag);
+        watch(a, merges ? a.part + (size_t)(item % (R * a.nq)) * a.splits * (RUN_HD + 2) : in + (item * 37) % n, wait);
         if (merges) {
             // the shares of every head's keys come together here: few of them, and few blocks that would read them all
             for (int j = tid; j < n; j += RUN_THREADS) {
                 int of = shares[0];
 #pragma unroll
                 for (int r = 1; r < R; ++r) of = j >= r * pairs ? shares[r] : of;
-                put(j, run_merged(a, j >> 6, j & 63, of, tag));
+                put(j, run_merged(a, j >> 6, j & 63, of, wait));
             }
         } else {
         constexpr int Q = 4;
         for (int j0 = tid; j0 < n; j0 += Q * RUN_THREADS) {
             uint32_t d[Q];
-            words_wait<Q>(a, tag, [&](int q) __attribute__((always_inline)) { return in + (j0 + q * RUN_THREADS < n ? j0 + q * RUN_THREADS : j0); }, d);
+            words_wait<Q>(a, wait, [&](int q) __attribute__((always_inline)) { return in + (j0 + q * RUN_THREADS < n ? j0 + q * RUN_THREADS : j0); }, d);
 #pragma unroll
             for (int q = 0; q < Q; ++q)
                 if (j0 + q * RUN_THREADS < n) put(j0 + q * RUN_THREADS, d[q]);
@@ -319,7 +323,7 @@ __device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L,
     uint32_t was[1] = {0};
     if (!normed && r < R) {
         if (kind == RUN_O && layer == 0) was[0] = ((const uint32_t*)a.x)[at];
-        else words_wait<1>(a, tag, [&](int) { return old_at; }, was);
+        else words_wait<1>(a, wait, [&](int) { return old_at; }, was);
     }
     __syncthreads();
     float scale = 1.f;
@@ -414,17 +418,17 @@ __device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L,
     };
     if (kind == RUN_GATE_UP) {
         const float g0 = total(p, 0) * scale, g1 = total(p, 1) * scale, u0 = total(p, 2) * scale, u1 = total(p, 3) * scale;
-        word_store(a.act + r * (a.ff >> 1) + pair, tag, pack_bf16x2(gate_act(g0, IA_ACT_SILU) * u0, gate_act(g1, IA_ACT_SILU) * u1));
+        word_store(a.act + r * (a.ff >> 1) + pair, wait.tag, pack_bf16x2(gate_act(g0, IA_ACT_SILU) * u0, gate_act(g1, IA_ACT_SILU) * u1));
         return;
     }
     const float v0 = total(p >> 1, (p & 1) * 2) * scale, v1 = total(p >> 1, (p & 1) * 2 + 1) * scale;
     if (kind == RUN_QKV) {
-        word_store(a.qkv + r * ((a.nq + 2 * a.nkv) * (RUN_HD / 2)) + pair, tag, pack_bf16x2(v0, v1));
+        word_store(a.qkv + r * ((a.nq + 2 * a.nkv) * (RUN_HD / 2)) + pair, wait.tag, pack_bf16x2(v0, v1));
         return;
     }
     const uint32_t sum = pack_bf16x2(lo_f32(was[0]) + v0, hi_f32(was[0]) + v1);
-    if (kind == RUN_O) word_store(a.mid + at, tag, sum);
-    else if (layer + 1 < a.n_layers) word_store(a.next + at, tag + 1, sum);
+    if (kind == RUN_O) word_store(a.mid + at, wait.tag, sum);
+    else if (layer + 1 < a.n_layers) word_store(a.next + at, wait.tag + 1, sum);
     else ((uint32_t*)a.x)[at] = sum;
 }
 
@@ -432,7 +436,7 @@ __device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L,
 // operands' layouts are those of the decode kernel in attention_mfma.hip: S^T = K Q^T and O^T = V^T P^T, key k0 + 8 G + 4 t + i in
 // row 4 G + i of tile t.  The first step's keys and values are asked for before the wait; the row's heads are normed and turned by a
 // wave each, once for the block; the new key, which is in no page yet, is a step of its own, of a wave that has none where there is one.
-__device__ __forceinline__ void run_attention(const RunArgs& a, const RunLayer& L, char* mem, int item, uint32_t tag) {
+__device__ __forceinline__ void run_attention(const RunArgs& a, const RunLayer& L, char* mem, int item, RunWait wait) {
     constexpr int HD = RUN_HD, KS = HD / 32, DB = HD / 16;
     const int tid = threadIdx.x, lane = tid & (IA_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / IA_WAVE);
     const int r = lane & 15, G = lane >> 4;
@@ -484,12 +488,12 @@ __device__ __forceinline__ void run_attention(const RunArgs& a, const RunLayer& 
             nw = *(const float2*)((wave < g ? L.q_norm : L.k_norm) + 2 * lane);
             if (a.one_qk) { nw.x += 1.0f; nw.y += 1.0f; }
         }
-        watch(a, a.qkv + ((size_t)row * (a.nq + 2 * a.nkv) + kvh * g) * (HD / 2), tag);
+        watch(a, a.qkv + ((size_t)row * (a.nq + 2 * a.nkv) + kvh * g) * (HD / 2), wait);
         if (wave < used) {
             const int head = wave < g ? kvh * g + wave : wave == g ? a.nq + kvh : a.nq + a.nkv + kvh;
             const uint64_t* at = a.qkv + ((size_t)row * (a.nq + 2 * a.nkv) + head) * (HD / 2) + lane;
             uint32_t one[1];
-            words_wait<1>(a, tag, [&](int) { return at; }, one);
+            words_wait<1>(a, wait, [&](int) { return at; }, one);
             uint32_t d = one[0];
             if (wave <= g) {                                // (features 2 lane and 2 lane + 1; what they are turned with is 32 lanes away)
                 float x = lo_f32(d), y = hi_f32(d);
@@ -644,12 +648,12 @@ __device__ __forceinline__ void run_attention(const RunArgs& a, const RunLayer& 
         const size_t head = (size_t)row * a.nq + kvh * g + col;
         if (a.splits == 1) {
             const float inv = 1.0f / total;
-            word_store(a.attn + head * (HD / 2) + i, tag, pack_bf16x2(o0 * inv, o1 * inv));
+            word_store(a.attn + head * (HD / 2) + i, wait.tag, pack_bf16x2(o0 * inv, o1 * inv));
         } else {
             uint64_t* to = a.part + (head * a.splits + split) * (HD + 2);
-            word_store(to + 2 * i, tag, __float_as_uint(o0));
-            word_store(to + 2 * i + 1, tag, __float_as_uint(o1));
-            if (i < 2) word_store(to + HD + i, tag, __float_as_uint(i == 0 ? top : total));
+            word_store(to + 2 * i, wait.tag, __float_as_uint(o0));
+            word_store(to + 2 * i + 1, wait.tag, __float_as_uint(o1));
+            if (i < 2) word_store(to + HD + i, wait.tag, __float_as_uint(i == 0 ? top : total));
         }
     }
     // the new key and value, for the steps to come
@@ -668,13 +672,13 @@ __device__ __forceinline__ void run_attention(const RunArgs& a, const RunLayer& 
 }
 
 // The shares of a row's keys come together: one key/value head's query heads a block, a thread a pair of features.
-__device__ __forceinline__ void run_merge(const RunArgs& a, int item, uint32_t tag) {
+__device__ __forceinline__ void run_merge(const RunArgs& a, int item, RunWait wait) {
     const int tid = threadIdx.x, g = a.nq / a.nkv;
     const int shares = run_last(a, item / a.nkv) / a.chunk + 1;
-    watch(a, a.part + ((size_t)(item / a.nkv) * a.nq + (item % a.nkv) * g) * a.splits * (RUN_HD + 2), tag);
+    watch(a, a.part + ((size_t)(item / a.nkv) * a.nq + (item % a.nkv) * g) * a.splits * (RUN_HD + 2), wait);
     if (tid >= g * (RUN_HD / 2)) return;
     const int head = (item / a.nkv) * a.nq + (item % a.nkv) * g + tid / (RUN_HD / 2), i = tid & (RUN_HD / 2 - 1);
-    word_store(a.attn + (size_t)head * (RUN_HD / 2) + i, tag, run_merged(a, head, i, shares, tag));
+    word_store(a.attn + (size_t)head * (RUN_HD / 2) + i, wait.tag, run_merged(a, head, i, shares, wait));
 }
 
 template <int R, bool DOT>
@@ -682,6 +686,8 @@ __global__ __launch_bounds__(RUN_THREADS) void layer_run_kernel(const RunArgs a)
     extern __shared__ __align__(16) char run_mem[];
     __shared__ uint64_t s_draw;
     if (threadIdx.x == 0) s_draw = __hip_atomic_fetch_add(a.head, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    int polls = a.polls;
+    asm volatile("" : "+s"(polls));                         // (here, and not where it is used)
     __syncthreads();
     const uint64_t drawn = s_draw;
     const uint32_t number = __builtin_amdgcn_readfirstlane((uint32_t)drawn), base = __builtin_amdgcn_readfirstlane((uint32_t)(drawn >> 32));
@@ -690,16 +696,16 @@ __global__ __launch_bounds__(RUN_THREADS) void layer_run_kernel(const RunArgs a)
     if (number == 0 && threadIdx.x == 0) __hip_atomic_store(a.head + 16, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int layer = number / (uint32_t)a.per_layer;
     int item = number - layer * a.per_layer;
-    const uint32_t tag = base + layer + 1;
+    const RunWait wait = {base + layer + 1, polls};
     const RunLayer& L = a.layer[layer];
     int kind;
     if (item < a.b_qkv) kind = RUN_QKV;
-    else if ((item -= a.b_qkv) < a.b_attn) { run_attention(a, L, run_mem, item, tag); return; }
-    else if ((item -= a.b_attn) < a.b_merge) { run_merge(a, item, tag); return; }
+    else if ((item -= a.b_qkv) < a.b_attn) { run_attention(a, L, run_mem, item, wait); return; }
+    else if ((item -= a.b_attn) < a.b_merge) { run_merge(a, item, wait); return; }
     else if ((item -= a.b_merge) < a.b_o) kind = RUN_O;
     else if ((item -= a.b_o) < a.b_gate_up) kind = RUN_GATE_UP;
     else { item -= a.b_gate_up; kind = RUN_DOWN; }
-    run_product<R, DOT>(a, L, run_mem, kind, item, layer, tag);
+    run_product<R, DOT>(a, L, run_mem, kind, item, layer, wait);
 }
 
 // ---- host -----------------------------------------------------------------------------------------------
