@@ -60,6 +60,8 @@ class LayerRun:
         b, caches = self.blocks[0], [storage.layers.get(s) for s in self.stops]
         s = b.mixer.spec
         sizes = (x.shape[0], s.hidden, b.ffn.spec.intermediate, s.n_heads, s.n_kv_heads)
+        if (ops.MID_PRODUCTS != "own" or ops.MID_FROM_ROWS is not None) and x.shape[0] >= ops.mid_from_rows(s.hidden):
+            return False                                 # (a switch says which kernels the products of so many rows take)
         return (all(c is not None and c.writable and c.group == caches[0].group for c in caches)
                 and ops.layer_run_fits(*sizes, ctx.groups[caches[0].group].page_size) and ops.layer_run_pays(*sizes, ctx.max_kv_len, self.length)
                 and ops.layer_run_aligned(self._layers(caches)))

@@ -105,6 +105,18 @@ def test_arrays_off_their_alignment_go_through_the_blocks():
         setattr(holder, name, t)
 
 
+def test_switches_of_the_products_reach_steps_that_the_run_would_take(monkeypatch):
+    """Rows whose products a switch keeps from gemm_mid.hip, or hands to it, go through the blocks, which follow the switch."""
+    run, ctx, x, storage = _cpu_run(hidden_size=2560)
+    step = lambda rows: run.takes(ctx, x[:1].expand(rows, -1), storage)
+    assert step(4) and step(5)
+    monkeypatch.setattr(ops, "MID_PRODUCTS", "library")
+    assert step(4) and not step(5)                   # (`mid_from_rows` of a width that is no power of two)
+    monkeypatch.setattr(ops, "MID_PRODUCTS", "own")
+    monkeypatch.setattr(ops, "MID_FROM_ROWS", 2)
+    assert step(1) and not step(2)
+
+
 @pytest.mark.parametrize("at,by", [(0, 2), (3, 8), (4, 4), (7, 4), (8, 2), (9, 8)])
 def test_arrays_off_their_alignment_are_refused(at, by):
     status, message = _run_status(off=(at, by))
