@@ -241,6 +241,55 @@ def test_layer_run_against_64_bits(case, one):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(512, 1024, 8, 2), (2560, 9728, 32, 8)], ids=["products on the matrix cores", "products by dot products"])
+def test_what_is_no_number_stays_in_its_row(shape):
+    """Infinities and NaN in a row of the stream and in a row's cached keys and values leave the other rows' bits alone; NaN and infinities in slots
+    behind a row's length, and in pages that are nobody's, leave all rows' bits alone."""
+    width, ff, nq, nkv = shape
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    lengths, pages = [70, 33, 517], 48
+    layers = _layers(gen, 2, width, ff, nq, nkv, pages)
+    counts = [length // PAGE + 1 for length in lengths]
+    table = torch.zeros((3, 40), dtype=torch.int32)
+    order = torch.randperm(pages, generator=torch.Generator().manual_seed(2)).to(torch.int32)
+    for r, c in enumerate(counts):
+        table[r, :c] = order[sum(counts[:r]):sum(counts[:r]) + c]
+    x = torch.empty((3, width), dtype=torch.bfloat16, device="cuda").normal_(0.0, 1.0, generator=gen)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    slots = i32([int(table[r, length // PAGE]) * PAGE + length % PAGE for r, length in enumerate(lengths)])
+    cached = torch.zeros((pages, PAGE), dtype=torch.bool)                   # the slots that some row reads, and those of row 1
+    of_row_1 = torch.zeros_like(cached)
+    for r, length in enumerate(lengths):
+        at = torch.arange(length)
+        cached[table[r, at // PAGE].long(), at % PAGE] = True
+        if r == 1:
+            of_row_1[table[r, at // PAGE].long(), at % PAGE] = True
+    kept = [(of[8].clone(), of[9].clone()) for of in layers]
+    kw = dict(nq=nq, nkv=nkv, ff=ff, max_kv_len=640, eps=(1e-6,) * 3, add_one=(False,) * 3, scale=HD ** -0.5)
+
+    def run(x, where=None, what=0.0):
+        for of, (k, v) in zip(layers, kept):
+            of[8].copy_(k)
+            of[9].copy_(v)
+            if where is not None:
+                of[8].masked_fill_(where.cuda()[:, None, :, None], what)
+                of[9].masked_fill_(where.cuda()[:, None, None, :], what)
+        out = ops.layer_run(x.clone(), layers, ops.RunWords(), i32(lengths), slots, table.cuda(), torch.ones((3, 64), device="cuda"), torch.zeros((3, 64), device="cuda"), **kw)
+        at = (slots // PAGE).long(), (slots % PAGE).long()
+        return [out] + [t for of in layers for t in (of[8][at[0], :, at[1]], of[9][at[0], :, :, at[1]])]
+
+    want = run(x)
+    assert all(torch.isfinite(t.float()).all() for t in want)
+    for what in (float("nan"), float("inf"), float("-inf")):
+        assert all(torch.equal(a, b) for a, b in zip(run(x, ~cached, what), want)), what
+        odd = x.clone()
+        odd[1, 5] = what
+        for got in (run(odd), run(x, of_row_1, what)):
+            assert all(torch.equal(a[[0, 2]], b[[0, 2]]) for a, b in zip(got, want)), what
+            assert not torch.isfinite(got[0][1].float()).any(), what
+
+
+@pytest.mark.gpu
 def test_words_are_not_made_under_capture():
     x = torch.zeros((1, 512), dtype=torch.bfloat16, device="cuda")
     gen = torch.Generator(device="cuda").manual_seed(0)
@@ -374,23 +423,53 @@ def _config(**kw):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 3, 8])
-def test_engine_steps_with_and_without(rows):
+def test_engine_steps_with_and_without(rows, monkeypatch):
     """Decode steps behind prompts of several lengths, eager and from graphs, against the same engine without the run of layers: no further
     apart than a few roundings of the last layer's rows."""
     from inferrs_amd.engine import Engine, Entry
     engines = [Engine.from_random(_config(), seed=3, page_size=16, num_pages=400, max_seqs=8) for _ in range(2)]
     assert engines[0].model.layer_run is not None and engines[0].model.layer_run.length == 5
     engines[1].model.layer_run = None
+    calls = []
+    real = ops.layer_run
+    monkeypatch.setattr(ops, "layer_run", lambda x, *a, **k: (calls.append(x.shape[0]), real(x, *a, **k))[1])
     gen = torch.Generator().manual_seed(rows)
     lengths = [5, 600, 33, 511, 512, 1, 64, 15][:rows]
     prompts = [torch.randint(0, 1024, (n,), generator=gen).tolist() for n in lengths]
     for e in engines:
         e.step([Entry(i, p, []) for i, p in enumerate(prompts)])
+    assert not calls                                  # (portions of prompts are no steps of the run's)
     for step in range(6):
         tokens = torch.randint(0, 1024, (rows,), generator=gen).tolist()
         got, want = (e.step([Entry(i, [t], [0]) for i, t in enumerate(tokens)]).clone() for e in engines)
         assert _rel(got, want.double()) < 2.0 ** -9 * math.sqrt(8 * 5)
     assert engines[0].graph_replays > 0
+    assert set(calls) == {rows} and engines[0].builder.run_words and not engines[1].builder.run_words
+
+
+@pytest.mark.gpu
+def test_steps_past_the_rule_go_through_the_blocks(monkeypatch):
+    """Nine rows, a portion beside a single token, and contexts beyond the rule's keys take no run; eight rows of the same engine do."""
+    from inferrs_amd.engine import Engine, Entry
+    e = Engine.from_random(_config(max_position_embeddings=16384), seed=3, page_size=16, num_pages=3200, max_seqs=9, use_graphs=False)
+    calls = []
+    real = ops.layer_run
+    monkeypatch.setattr(ops, "layer_run", lambda x, *a, **k: (calls.append(x.shape[0]), real(x, *a, **k))[1])
+    for i in range(9):
+        e.step([Entry(i, [1, 2, 3], [])])
+    e.step([Entry(i, [4], [0]) for i in range(9)])
+    e.step([Entry(0, [4, 5], [1]), Entry(1, [4], [0])])
+    assert not calls
+    e.step([Entry(i, [4], [0]) for i in range(8)])
+    assert calls == [8]
+    for i in range(4):                                # (3 x 12,000 keys are within the rule's 45,056, 4 x 12,000 are not)
+        more = 11999 - e.cached_length(i)
+        assert e.cache.reserve(i, more)
+        e.cache.commit(i, more)
+    e.step([Entry(i, [4], [0]) for i in range(4)])
+    assert calls == [8]
+    e.step([Entry(i, [4], [0]) for i in range(3)])
+    assert calls == [8, 3]
 
 
 @pytest.mark.gpu
@@ -418,6 +497,8 @@ def test_two_engines_on_two_streams():
 
     torch.cuda.synchronize()
     want = steps(False)
+    words = [list(e.builder.run_words.values()) for e in engines]
+    assert all(len(w) == 1 for w in words) and words[0][0].data_ptr() != words[1][0].data_ptr()
     got = steps(True)
     for a, b in zip(want, got):
         assert all(torch.equal(x, y) for x, y in zip(a, b))
