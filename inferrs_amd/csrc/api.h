@@ -370,9 +370,9 @@ long long ia_fading_scan_workspace(int n_seqs, int chunks, int H, int dim, int v
 int ia_layer_run_layers(void);
 long long ia_layer_run_words(int rows, int width, int ff, int nq, int nkv, int splits);
 int ia_layer_run(void* x, const void* layers, int n_layers, long long* words, long long n_words, int* given_up, int polls,
-                    const int* positions, const int* slots, const int* block_table, const float* cos_t, const float* sin_t, int rows, int width,
-                    int ff, int nq, int nkv, int page_size, int max_pages, int max_kv_len, int splits, int chunk, float eps1, float eps2,
-                    float eps_qk, int one1, int one2, int one_qk, float scale, hipStream_t stream);
+                 const int* positions, const int* slots, const int* block_table, const float* cos_t, const float* sin_t, int rows,
+                 int width, int ff, int nq, int nkv, int page_size, int max_pages, int max_kv_len, int splits, int chunk, float eps1,
+                 float eps2, float eps_qk, int one1, int one2, int one_qk, float scale, hipStream_t stream);
 
 // Built per head size (-DIA_HEAD_DIM) into a library of its own.
 int ia_attention_mfma_head_dim(void);

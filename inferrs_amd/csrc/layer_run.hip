@@ -303,14 +303,14 @@ __device__ __forceinline__ void run_product(const RunArgs& a, const RunLayer& L,
                 put(j, run_merged(a, j >> 6, j & 63, of, wait));
             }
         } else {
-        constexpr int Q = 4;
-        for (int j0 = tid; j0 < n; j0 += Q * RUN_THREADS) {
-            uint32_t d[Q];
-            words_wait<Q>(a, wait, [&](int q) __attribute__((always_inline)) { return in + (j0 + q * RUN_THREADS < n ? j0 + q * RUN_THREADS : j0); }, d);
+            constexpr int Q = 4;
+            for (int j0 = tid; j0 < n; j0 += Q * RUN_THREADS) {
+                uint32_t d[Q];
+                words_wait<Q>(a, wait, [&](int q) __attribute__((always_inline)) { return in + (j0 + q * RUN_THREADS < n ? j0 + q * RUN_THREADS : j0); }, d);
 #pragma unroll
-            for (int q = 0; q < Q; ++q)
-                if (j0 + q * RUN_THREADS < n) put(j0 + q * RUN_THREADS, d[q]);
-        }
+                for (int q = 0; q < Q; ++q)
+                    if (j0 + q * RUN_THREADS < n) put(j0 + q * RUN_THREADS, d[q]);
+            }
         }
     }
     // What the outputs' threads need beside the sums comes while the products are formed: the stream's old values (there before this block's rows
@@ -711,7 +711,7 @@ __global__ __launch_bounds__(RUN_THREADS) void layer_run_kernel(const RunArgs a)
 // ---- host -----------------------------------------------------------------------------------------------
 
 // log2 of the waves that share a group of weight rows: as many as leave a wave `least` loads a weight row.
-static int run_shares(int inner, int least) {
+static int run_waves_log2(int inner, int least) {
     int s = 0;
     while (s < 4 && inner / RUN_UNIT >> (s + 1) >= least) ++s;
     return s;
@@ -724,10 +724,10 @@ extern "C" long long ia_layer_run_words(int rows, int width, int ff, int nq, int
 
 extern "C" int ia_layer_run_layers(void) { return RUN_LAYERS; }
 
-extern "C" int ia_layer_run(void* x, const void* layers, int n_layers, long long* words, long long n_words, int* given_up, int polls, const int* positions, const int* slots,
-                               const int* block_table, const float* cos_t, const float* sin_t, int rows, int width, int ff, int nq, int nkv,
-                               int page_size, int max_pages, int max_kv_len, int splits, int chunk, float eps1, float eps2, float eps_qk, int one1, int one2, int one_qk,
-                               float scale, hipStream_t stream) {
+extern "C" int ia_layer_run(void* x, const void* layers, int n_layers, long long* words, long long n_words, int* given_up, int polls,
+                            const int* positions, const int* slots, const int* block_table, const float* cos_t, const float* sin_t, int rows,
+                            int width, int ff, int nq, int nkv, int page_size, int max_pages, int max_kv_len, int splits, int chunk, float eps1,
+                            float eps2, float eps_qk, int one1, int one2, int one_qk, float scale, hipStream_t stream) {
     IA_CHECK(rows >= 1 && rows <= RUN_ROWS && n_layers >= 1 && n_layers <= RUN_LAYERS, "layer_run: %d rows, %d layers", rows, n_layers);
     IA_CHECK(width > 0 && width % RUN_UNIT == 0 && width <= 6144 && ff > 0 && ff % RUN_UNIT == 0 && nkv > 0 && nq % nkv == 0 && nq % 4 == 0
                  && nq / nkv <= 8 && (nq + 2 * nkv) % 2 == 0,
@@ -764,9 +764,9 @@ extern "C" int ia_layer_run(void* x, const void* layers, int n_layers, long long
     a.n_layers = n_layers;
     const long long weights = 2ll * ((long long)(2 * nq + 2 * nkv) * RUN_HD * width + 3ll * width * ff);
     const int least = weights <= 64ll << 20 ? 2 : weights <= 128ll << 20 ? 3 : weights <= 512ll << 20 ? 4 : 5;
-    a.s_qkv = a.s_gate_up = run_shares(width, least);
-    a.s_o = run_shares(nq * RUN_HD, least);
-    a.s_down = run_shares(ff, least);
+    a.s_qkv = a.s_gate_up = run_waves_log2(width, least);
+    a.s_o = run_waves_log2(nq * RUN_HD, least);
+    a.s_down = run_waves_log2(ff, least);
     a.b_qkv = (nq + 2 * nkv) * RUN_HD / (64 >> a.s_qkv);
     a.b_attn = rows * nkv * splits;
     a.b_o = width / (64 >> a.s_o);

@@ -59,7 +59,7 @@ class StepContext:
     router_logits: Any = None               # (32-bit rows, offset): the logits of the next feed-forward's router, from a product that its matrix joined
     post_rows: Any = None                   # a 32-bit stream's rows once more in the products' precision, where a part has them already (the embedding, a block's last kernel)
     decode_counters: Any = None             # the decode attention's counters (`ops.DecodeCounters`), the step builder's own
-    run_words: Any = None                 # the words of runs of layers (`ops.RunWords`), the step builder's own
+    run_words: Any = None                   # the words of runs of layers (`ops.RunWords`), the step builder's own
     _tables: Dict[Any, Any] = field(default_factory=dict)
 
     @property

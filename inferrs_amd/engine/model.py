@@ -96,7 +96,7 @@ class DecoderModel:
             x = first.enter(ctx, x)
         pending = None                               # a block's output that is not added to x yet
         in_run = self.layer_run.length if self.layer_run is not None and self.layer_run.takes(ctx, x, storage) else 0
-        if in_run:                                  # the first layers in one kernel, which leaves nothing to be added
+        if in_run:                                   # the first layers in one kernel, which leaves nothing to be added
             x = self.layer_run.forward(ctx, x, storage)
         for stop, e in enumerate(self.spec.schedule):
             if stop < in_run:

@@ -970,8 +970,8 @@ def layer_run_pays(rows: int, width: int, ff: int, nq: int, nkv: int, max_kv_len
 
 
 def layer_run(x: torch.Tensor, layers: Sequence[Sequence[torch.Tensor]], words: RunWords, positions: torch.Tensor, slots: torch.Tensor,
-                 block_table: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, *, nq: int, nkv: int, ff: int, max_kv_len: int,
-                 eps: Tuple[float, float, float], add_one: Tuple[bool, bool, bool], scale: float) -> torch.Tensor:
+              block_table: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, *, nq: int, nkv: int, ff: int, max_kv_len: int,
+              eps: Tuple[float, float, float], add_one: Tuple[bool, bool, bool], scale: float) -> torch.Tensor:
     """A run of whole layers over the stream `x` [rows, width], in place: `layers` holds each layer's [q | k | v], o, [gate; up] and down
     weights, the norms' weights of the stream (two) and of the heads (q, k), and its arrays of keys and values; `eps` and `add_one` are
     those of the three kinds of norms.  Row i is the newest token of request i."""
@@ -1005,9 +1005,8 @@ def layer_run(x: torch.Tensor, layers: Sequence[Sequence[torch.Tensor]], words: 
         of = layers[lo:lo + most]
         table = (ctypes.c_void_p * (10 * len(of)))(*[t.data_ptr() for layer in of for t in layer])
         _check(lib.ia_layer_run(
-            _p(x), ctypes.addressof(table), len(of), _p(space), space.numel(), _p(words.given_up),
-            words.polls, _p(positions), _p(slots), _p(block_table), _p(cos), _p(sin), rows,
-            width, ff, nq, nkv, page_size, block_table.shape[1], max_kv_len, splits, chunk, *eps, *(int(o) for o in add_one), scale, _stream()))
+            _p(x), ctypes.addressof(table), len(of), _p(space), space.numel(), _p(words.given_up), words.polls, _p(positions), _p(slots),
+            _p(block_table), _p(cos), _p(sin), rows, width, ff, nq, nkv, page_size, block_table.shape[1], max_kv_len, splits, chunk, *eps, *(int(o) for o in add_one), scale, _stream()))
     return x
 
 

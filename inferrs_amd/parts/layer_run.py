@@ -76,5 +76,5 @@ class LayerRun:
         a, s, group = b.mixer, b.mixer.spec, ctx.groups[caches[0].group]
         cos, sin = ctx.position_table(a.position)
         return ops.layer_run(x, self._layers(caches), ctx.run_words, ctx.positions, group.slots, group.block_table, cos, sin, nq=s.n_heads, nkv=s.n_kv_heads,
-                                ff=b.ffn.spec.intermediate, max_kv_len=ctx.max_kv_len, eps=(b.norm_mixer.eps, b.norm_ffn.eps, a.norm_eps),
-                                add_one=(b.norm_mixer.add_one, b.norm_ffn.add_one, a.norm_add_one), scale=s.softmax_scale)
+                             ff=b.ffn.spec.intermediate, max_kv_len=ctx.max_kv_len, eps=(b.norm_mixer.eps, b.norm_ffn.eps, a.norm_eps),
+                             add_one=(b.norm_mixer.add_one, b.norm_ffn.add_one, a.norm_add_one), scale=s.softmax_scale)
