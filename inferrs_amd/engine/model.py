@@ -95,9 +95,9 @@ class DecoderModel:
         if hasattr(first, "enter"):                  # an arrangement whose stream is not the embedding's rows
             x = first.enter(ctx, x)
         pending = None                               # a block's output that is not added to x yet
-        in_run = self.layer_run.length if self.layer_run is not None and self.layer_run.takes(ctx, x, storage) else 0
-        if in_run:                                   # the first layers in one kernel, which leaves nothing to be added
-            x = self.layer_run.forward(ctx, x, storage)
+        of_run, in_run = self.layer_run.takes(ctx, x, storage) if self.layer_run is not None else None, 0
+        if of_run is not None:                       # the first layers in one kernel, which leaves nothing to be added
+            x, in_run = self.layer_run.forward(ctx, x, of_run, storage), self.layer_run.length
         for stop, e in enumerate(self.spec.schedule):
             if stop < in_run:
                 continue

@@ -900,17 +900,11 @@ class RunWords(DecodeCounters):
     def __init__(self):
         super().__init__()
         self.polls = self.POLLS
-        self.given_up: Optional[torch.Tensor] = None        # pinned: the kernel writes it from the device
-
-    def take(self, device: torch.device, needed: int) -> Optional[torch.Tensor]:
-        space = super().take(device, needed)
-        if self.given_up is None:
-            self.given_up = torch.zeros((1,), dtype=torch.int32, pin_memory=True)
-        return space
+        self.given_up = torch.zeros((1,), dtype=torch.int32, pin_memory=torch.cuda.is_available())      # (the kernel writes it from the device)
 
     def check(self) -> None:
         """Raises where a launch that has ended gave a wait up, once for all launches since the last check."""
-        if self.given_up is not None and self.given_up.item():
+        if self.given_up.item():
             self.given_up.zero_()
             raise KernelError("layer_run: a decode step's blocks waited in vain for each other's rows; the logits of the steps since the last "
                               "check, and the keys and values that these cached, are void")

@@ -53,28 +53,27 @@ class LayerRun:
             stops.append(stop)
         return cls(run, stops) if run else None
 
-    def takes(self, ctx, x: torch.Tensor, storage) -> bool:
-        """Whether this step goes through the kernel: one token a request, few of them, all layers' pages in one table."""
+    def takes(self, ctx, x: torch.Tensor, storage) -> Optional[List[Tuple[torch.Tensor, ...]]]:
+        """The layers' arrays where this step goes through the kernel, else None: one token a request, few of them, all layers' pages in one table."""
         if ctx.max_q_len != 1 or ctx.run_words is None or not (0 < x.shape[0] <= ops.RUN_MAX_ROWS):
-            return False
+            return None
         b, caches = self.blocks[0], [storage.layers.get(s) for s in self.stops]
         s = b.mixer.spec
         sizes = (x.shape[0], s.hidden, b.ffn.spec.intermediate, s.n_heads, s.n_kv_heads)
         if (ops.MID_PRODUCTS != "own" or ops.MID_FROM_ROWS is not None) and x.shape[0] >= ops.mid_from_rows(s.hidden):
-            return False                                 # (a switch says which kernels the products of so many rows take)
-        return (all(c is not None and c.writable and c.group == caches[0].group for c in caches)
-                and ops.layer_run_fits(*sizes, ctx.groups[caches[0].group].page_size) and ops.layer_run_pays(*sizes, ctx.max_kv_len, self.length)
-                and ops.layer_run_aligned(self._layers(caches)))
+            return None                                  # (a switch says which kernels the products of so many rows take)
+        if (not all(c is not None and c.writable and c.group == caches[0].group for c in caches)
+                or not ops.layer_run_fits(*sizes, ctx.groups[caches[0].group].page_size) or not ops.layer_run_pays(*sizes, ctx.max_kv_len, self.length)):
+            return None
+        layers = [(m.mixer.qkv.weight, m.mixer.o.weight, m.ffn.gate_up.weight, m.ffn.down.weight, m.norm_mixer.weight, m.norm_ffn.weight,
+                   m.mixer.q_norm_w, m.mixer.k_norm_w, c.k, c.v) for m, c in zip(self.blocks, caches)]
+        return layers if ops.layer_run_aligned(layers) else None
 
-    def _layers(self, caches) -> List[Tuple[torch.Tensor, ...]]:
-        return [(m.mixer.qkv.weight, m.mixer.o.weight, m.ffn.gate_up.weight, m.ffn.down.weight, m.norm_mixer.weight, m.norm_ffn.weight,
-                 m.mixer.q_norm_w, m.mixer.k_norm_w, c.k, c.v) for m, c in zip(self.blocks, caches)]
-
-    def forward(self, ctx, x: torch.Tensor, storage) -> torch.Tensor:
-        """The stream after the run, in place."""
-        b, caches = self.blocks[0], [storage.layers[s] for s in self.stops]
-        a, s, group = b.mixer, b.mixer.spec, ctx.groups[caches[0].group]
+    def forward(self, ctx, x: torch.Tensor, layers: List[Tuple[torch.Tensor, ...]], storage) -> torch.Tensor:
+        """The stream after the run, in place; `layers` as `takes` has given them."""
+        b = self.blocks[0]
+        a, s, group = b.mixer, b.mixer.spec, ctx.groups[storage.layers[self.stops[0]].group]
         cos, sin = ctx.position_table(a.position)
-        return ops.layer_run(x, self._layers(caches), ctx.run_words, ctx.positions, group.slots, group.block_table, cos, sin, nq=s.n_heads, nkv=s.n_kv_heads,
+        return ops.layer_run(x, layers, ctx.run_words, ctx.positions, group.slots, group.block_table, cos, sin, nq=s.n_heads, nkv=s.n_kv_heads,
                              ff=b.ffn.spec.intermediate, max_kv_len=ctx.max_kv_len, eps=(b.norm_mixer.eps, b.norm_ffn.eps, a.norm_eps),
                              add_one=(b.norm_mixer.add_one, b.norm_ffn.add_one, a.norm_add_one), scale=s.softmax_scale)

@@ -336,7 +336,7 @@ def test_questions_to_the_host_are_no_kernel_calls():
 def test_a_wait_given_up_is_an_error_once():
     words = ops.RunWords()
     words.check()
-    words.given_up = torch.ones((1,), dtype=torch.int32)
+    words.given_up.fill_(1)
     with pytest.raises(ops.KernelError, match="waited in vain"):
         words.check()
     words.check()
