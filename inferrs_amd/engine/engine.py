@@ -168,7 +168,8 @@ class Engine:
         The tensor that a step returns under `use_graphs` may be a captured graph's own output buffer (decode
         steps and steps of up to `GRAPH_MAX_TOKENS` tokens whose shape has been seen before): it holds this
         step's logits until the next step of the same shape overwrites them.  Read or `.clone()` it before
-        stepping again."""
+        stepping again.  Raises `ops.KernelError`, before anything of this step is done, where an earlier step has
+        turned out void (`check`)."""
         if not entries:
             raise StepError("a step needs at least one entry")
         self.check()
